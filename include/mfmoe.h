@@ -197,8 +197,7 @@ int mf_qmm_path(mf_qtensor w, mf_bits bits, const uint16_t* x, const void* y, ui
  * act = bf16(silu(bf16(gate.x)) * bf16(up.x)).  Also the dense SwiGLU MLP of Qwen38ForwardRunner
  * (mlp.encode, :1094) and, for any t, PrefillSharedExpert.encodeBlock (Kernels/Prefill/MoE/
  * PrefillSharedExpert.swift:81-190) / encodeDenseMLPPrefill (Qwen38ForwardRunner.swift:862-913):
- * from 32 rows on the projections run on the matrix cores when d and f are multiples of 128,
- * d <= 7168, the operands are 16-byte aligned and scratch_act holds
+ * from 32 rows on the projections run on the matrix cores when d and f are at least 128, the operands are 16-byte aligned and scratch_act holds
  * mf_shared_expert_scratch_bytes(d, f, t) bytes; otherwise row by row, MF_MAX_TOKENS rows per pair
  * of launches, for which t*f bf16 of scratch suffice (all that t <= MF_MAX_TOKENS ever needs). */
 size_t mf_shared_expert_scratch_bytes(uint32_t d, uint32_t f, uint32_t t);
@@ -565,10 +564,11 @@ mf_status mf_group_pairs_host(const mf_pair* pairs, size_t n_pairs, int query_co
  * (PrefillSharedExpert.swift:81-99, 27-36).  Result per token equals
  * mf_moe_decode_layer on that token within the layer tolerance.
  * Any t >= 1.  The matrix-core path takes 4-bit, 2-bit and ternary experts (with a 4-bit
- * shared expert, if any) with d, f, shared_f multiples of 128 and x, y and every weight
- * tensor 16-byte aligned; every other configuration (other widths, another shared-expert
+ * shared expert, if any) with d, f, shared_f at least 128 and x, y and every weight
+ * tensor 16-byte aligned; every other configuration (a width of 64, another shared-expert
  * format) runs the same rows through the decode launch, MF_MAX_TOKENS at a time, and needs
- * no workspace.  Covers MoEDeepseekV4's pair-major 2-bit prefill
+ * no workspace.  Widths that are no multiples of 128 run that way too when the call brings no
+ * workspace or an unaligned operand (with widths of whole 128s that is an error).  Covers MoEDeepseekV4's pair-major 2-bit prefill
  * (Metal/MoE/moe.metal:1293-1409) with the same call.
  * workspace: device scratch of at least mf_moe_prefill_workspace_bytes(h, t) (0 when the
  * configuration takes the decode launch; workspace may then be null). */
@@ -584,7 +584,7 @@ mf_status mf_moe_prefill_layer(mf_moe* h, mf_stream stream, const mf_moe_layer_w
  * instruction of the matrix-core matmul reads consecutive bytes (inside a sub-tensor: blocks of 32 rows, K
  * group by K group, the 64 half-group pieces of a block and group side by side); tables, offsets and stride
  * are unchanged.  Costs a second pool in HBM (Qwen shape: 453 MB per layer) and buys 4..7 % of a prefill
- * layer.  Needs the matrix-core configuration (mf_moe_prefill_workspace_bytes(h, t) != 0), else
+ * layer.  Needs the matrix-core configuration with widths that are multiples of 128, else
  * MF_ERR_DIMENSION_MISMATCH. */
 mf_status mf_moe_tile_experts(mf_moe* h, mf_stream stream, const void* expert_base, size_t expert_stride,
                               const mf_expert_offsets* offsets, void* tiled);
@@ -611,7 +611,7 @@ mf_status mf_moe_set_prefill_route_rounding(mf_moe* h, int narrow);
  * per dispatch pair; here one launch per projection covers every tile of every expert.  The counts
  * and pairs are checked on the device before they are trusted (sum of counts <= t * top_k, token < t,
  * rank < top_k): a grouping that fails computes nothing and mf_moe_group_status returns
- * MF_ERR_EXPERT_RANGE.  Needs the matrix-core configuration (mf_moe_prefill_workspace_bytes(h, t) != 0),
+ * MF_ERR_EXPERT_RANGE.  Needs the matrix-core configuration with widths that are multiples of 128,
  * else MF_ERR_DIMENSION_MISMATCH; workspace as for mf_moe_prefill_layer.
  *
  * mf_moe_unpermute: PrefillMoE.encodeReduceTokenMajor (Kernels/Prefill/MoE/PrefillMoE.swift:11-38,

@@ -766,9 +766,20 @@ mf_status mf_moe_prefill_layer(mf_moe* h, mf_stream stream, const mf_moe_layer_w
   if (!h || !wts || !x || !y) return MF_ERR_INVALID_ARGUMENT;
   if (t == 0 || t > MF_MAX_ROWS) return MF_ERR_INVALID_ARGUMENT;
   const mf_moe_config& c = h->cfg;
-  if (!mf::prefill_supported(c)) {
-    // 2-bit / ternary experts, or widths the matmul tiles do not divide: the same rows through
-    // the decode launch, MF_MAX_TOKENS at a time (correct for every configuration, not fast)
+  // Widths that are multiples of 64 but not of 128 take the matrix cores when the call brings what they need and
+  // the decode launch otherwise (which needs no workspace and no alignment); whole 128-row widths insist on it.
+  const uint32_t offs = wts->offsets.gate_w | wts->offsets.up_w | wts->offsets.down_w;
+  const bool al = mf::aligned16(wts->expert_base) && wts->expert_stride % 16 == 0 && offs % 16 == 0 &&
+                  mf::aligned16(wts->router_w) && mf::aligned16(x) && mf::aligned16(y) && mf::aligned16(workspace) &&
+                  mf::aligned16(wts->expert_tiled) &&
+                  (!c.shared_f || (mf::aligned16(wts->shared_gate.weights) && mf::aligned16(wts->shared_up.weights) &&
+                                   mf::aligned16(wts->shared_down.weights) &&
+                                   !(wts->w_sg && !wts->w_sg_q8.weights && !mf::aligned16(wts->w_sg))));
+  if (!mf::prefill_supported(c) ||
+      (!mf::prefill_whole_tiles(c) &&
+       (!al || !workspace || wts->expert_tiled || workspace_bytes < mf::prefill_workspace_bytes(c, t)))) {
+    // another shared-expert format, a width of one group, or no workspace: the same rows through the decode
+    // launch, MF_MAX_TOKENS at a time (correct for every configuration, not fast)
     for (uint32_t t0 = 0; t0 < t; t0 += MF_MAX_TOKENS) {
       const uint32_t n = t - t0 < MF_MAX_TOKENS ? t - t0 : MF_MAX_TOKENS;
       const mf_status st = mf_moe_decode_layer(
@@ -781,18 +792,11 @@ mf_status mf_moe_prefill_layer(mf_moe* h, mf_stream stream, const mf_moe_layer_w
   }
   if (!workspace) return MF_ERR_INVALID_ARGUMENT;
   if (workspace_bytes < mf::prefill_workspace_bytes(c, t)) return MF_ERR_SCRATCH_TOO_SMALL;
-  const uint32_t offs = wts->offsets.gate_w | wts->offsets.up_w | wts->offsets.down_w;
-  if ((!wts->router_w && (!out_idx || !out_w)) || !wts->expert_base || !offsets_ok(wts->offsets, c.bits) ||
-      !mf::aligned16(wts->expert_base) || wts->expert_stride % 16 || offs % 16 ||
-      !mf::aligned16(wts->router_w) || !mf::aligned16(x) || !mf::aligned16(y) ||
-      !mf::aligned16(workspace) || !mf::aligned16(wts->expert_tiled))
+  if ((!wts->router_w && (!out_idx || !out_w)) || !wts->expert_base || !offsets_ok(wts->offsets, c.bits) || !al)
     return MF_ERR_INVALID_ARGUMENT;
   if (c.shared_f && (!qtensor_ok(wts->shared_gate, c.shared_bits) ||
                      !qtensor_ok(wts->shared_up, c.shared_bits) ||
-                     !qtensor_ok(wts->shared_down, c.shared_bits) ||
-                     !mf::aligned16(wts->shared_gate.weights) || !mf::aligned16(wts->shared_up.weights) ||
-                     !mf::aligned16(wts->shared_down.weights) ||
-                     (wts->w_sg && !wts->w_sg_q8.weights && !mf::aligned16(wts->w_sg))))
+                     !qtensor_ok(wts->shared_down, c.shared_bits)))
     return MF_ERR_INVALID_ARGUMENT;
   if (c.shared_f && wts->w_sg_q8.weights && !qtensor_ok(wts->w_sg_q8, MF_BITS_8)) return MF_ERR_INVALID_ARGUMENT;
   MF_HIP(h->ctx, mf::launch_prefill_layer(static_cast<hipStream_t>(stream), *h, *wts, x, t, y, workspace,
@@ -808,7 +812,7 @@ mf_status mf_moe_ragged_qmm(mf_moe* h, mf_stream stream, const void* expert_base
     return MF_ERR_INVALID_ARGUMENT;
   if (t == 0 || t > MF_MAX_ROWS) return MF_ERR_QUERY_COUNT;
   const mf_moe_config& c = h->cfg;
-  if (!mf::prefill_supported(c)) return MF_ERR_DIMENSION_MISMATCH;
+  if (!mf::prefill_whole_tiles(c)) return MF_ERR_DIMENSION_MISMATCH;
   if (!workspace) return MF_ERR_INVALID_ARGUMENT;
   if (workspace_bytes < mf::prefill_workspace_bytes(c, t)) return MF_ERR_SCRATCH_TOO_SMALL;
   const uint32_t offs = offsets->gate_w | offsets->up_w | offsets->down_w;
@@ -825,7 +829,7 @@ mf_status mf_moe_tile_experts(mf_moe* h, mf_stream stream, const void* expert_ba
                               const mf_expert_offsets* offsets, void* tiled) {
   if (!h || !expert_base || !offsets || !tiled) return MF_ERR_INVALID_ARGUMENT;
   const mf_moe_config& c = h->cfg;
-  if (!mf::prefill_supported(c)) return MF_ERR_DIMENSION_MISMATCH;
+  if (!mf::prefill_whole_tiles(c)) return MF_ERR_DIMENSION_MISMATCH;
   const uint32_t offs = offsets->gate_w | offsets->up_w | offsets->down_w;
   if (!offsets_ok(*offsets, c.bits) || !mf::aligned16(expert_base) || !mf::aligned16(tiled) || expert_stride % 16 ||
       offs % 16)

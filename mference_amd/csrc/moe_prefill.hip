@@ -1100,7 +1100,7 @@ void qmm_kernel(const QmmLaunch launch) {
   const QmmArgs& a = launch.part[second ? 1 : 0];
   const uint32_t work = (blockIdx.x & 7u) * launch.per_xcd[second ? 1 : 0] + (xcd_slot - (second ? launch.per_xcd[0] : 0u));
   const uint32_t wave_rows = a.pair_rows ? 32u * NPROJ : 32u;  // weight rows of one wave
-  const uint32_t n_slices = a.rows / (kQmmWaves * wave_rows);
+  const uint32_t n_slices = (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
   uint32_t tile_id = work / n_slices, slice = work % n_slices, win = 0;
   if (a.dense_mode) {
     if (work >= a.dense_items) return;
@@ -1163,7 +1163,9 @@ void qmm_kernel(const QmmLaunch launch) {
       Sp[p] = reinterpret_cast<const uint16_t*>(blob + a.s_off[t]);
       Bp[p] = reinterpret_cast<const uint16_t*>(blob + a.b_off[t]);
     }
-    row_base[p] = (slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u);
+    // (a width that is no multiple of the workgroup's rows: the last slice's waves past the end compute the last
+    // 32 rows again and store nothing)
+    row_base[p] = min((slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u), a.rows - 32u);
   }
   const uint32_t ng_ld = a.ng_ld ? a.ng_ld : ng;
   const size_t row_bytes = static_cast<size_t>(ng_ld) * kGB;
@@ -1210,19 +1212,21 @@ void qmm_kernel(const QmmLaunch launch) {
   }
   // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
   const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_q * 16;
-  // K groups travel in pairs (ng is even: kdim is a multiple of 128)
+  // K groups travel in pairs; a contraction of an odd number of groups ends in half a pair (its other half is read
+  // from the last group again and not multiplied)
   // (arrays of a native vector type: arrays of the uint4 struct were kept in scratch memory)
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
   u32x4_t xs[2][2];  // the pair after the one in LDS, on its way there
   u32x4_t x0[2][2];
 #pragma unroll
   for (int gi = 0; gi < 2; ++gi) {
-    x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gi * kGroup);
-    x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gi * kGroup + 8);
+    const uint32_t ga = NG8 ? gi : min(static_cast<uint32_t>(gi), ng - 1), gb = NG8 ? 2u + gi : min(2u + gi, ng - 1);
+    x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup);
+    x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + 8);
     xs[gi][0] = xs[gi][1] = u32x4_t{0, 0, 0, 0};
     if (NG8 || ng > 2) {
-      xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + (2 + gi) * kGroup);
-      xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + (2 + gi) * kGroup + 8);
+      xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup);
+      xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + 8);
     }
   }
   // Scale and bias words of the lane's row and the group sums of its two routes, 8 K groups at a time
@@ -1384,14 +1388,16 @@ void qmm_kernel(const QmmLaunch launch) {
           const uint32_t gx = NG8 ? min(gu + 4, ng - 2) : gu + 4;
 #pragma unroll
           for (int gi = 0; gi < 2; ++gi) {
-            xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + (gx + gi) * kGroup);
-            xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + (gx + gi) * kGroup + 8);
+            const uint32_t gy = NG8 ? gx + gi : min(gx + gi, ng - 1);
+            xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup);
+            xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + 8);
           }
         }
       }
 #pragma unroll
       for (int gi = 0; gi < 2; ++gi) {
         const uint32_t g = gu + gi;
+        if (!NG8 && g >= ng) break;  // the half pair at the end of an odd number of groups
         // ---- matrix core: tmp[token, row] = sum over the group of x * (8 + q/2)
         const uint4* buf = s_x + uu * 1024 + gi * 512;
         uint4 bx[2][4];
@@ -1428,6 +1434,7 @@ void qmm_kernel(const QmmLaunch launch) {
 
   qmm_trace(a, work, 3);
   // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
+  const uint32_t row_raw = (slice * kQmmWaves + wv) * wave_rows;  // past a.rows: this wave has no rows of its own
   if (a.epi == 0) {
     // SwiGLU, narrowed to bf16, transposed through the (now free) x ring so that a lane stores
     // 16 bytes of one token: [token][32 rows] per wave, the rows of a run of 8 in the
@@ -1485,7 +1492,7 @@ void qmm_kernel(const QmmLaunch launch) {
       const uint32_t c = it * 64 + lane, tok = c >> 2, part = c & 3u;
       const uint32_t sl = s_slot[tok];
       const uint4 v = reinterpret_cast<const uint4*>(so)[c];
-      if (sl != 0xFFFFFFFFu)
+      if (sl != 0xFFFFFFFFu && row_raw < a.rows)
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out_base) + static_cast<size_t>(sl) * a.rows + row_base[0] +
                                   part * 8) = v;
     }
@@ -1504,6 +1511,7 @@ void qmm_kernel(const QmmLaunch launch) {
 #pragma unroll
           for (int p = 0; p < NPROJ; ++p) {
             if (p > 0 && !a.pair_rows && !out2_base) break;
+            if (row_raw + (a.pair_rows ? 32u * p : 0u) >= a.rows) break;
             uint8_t* ob = (p > 0 && !a.pair_rows) ? out2_base : out_base;  // the second projection's own buffer
             if (a.epi == 1) reinterpret_cast<float*>(ob)[at + row_base[p] + m] = acc[p][nt][4 * j + i];
             else reinterpret_cast<uint16_t*>(ob)[at + row_base[p] + m] = f_to_bf16(acc[p][nt][4 * j + i]);
@@ -2152,7 +2160,7 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
     QmmArgs& q = launch.part[part];
     q = part ? *b : a;
     const uint32_t slots = part ? b_tile_slots : tile_slots;
-    const uint32_t n_slices = q.rows / (kQmmRows * (q.pair_rows ? nproj : 1));
+    const uint32_t slice_rows = kQmmRows * (q.pair_rows ? nproj : 1), n_slices = (q.rows + slice_rows - 1) / slice_rows;
     if (q.dense_mode) {
       q.dense_tiles = slots;
       q.tile_major = dense_tile_major(q.rows * (q.pair_rows ? 1 : nproj), q.dense_rows, bits);
@@ -2354,7 +2362,7 @@ hipError_t launch_dense_qmm(hipStream_t s, const mf_qtensor& w, int bits, const 
 // (gate and up narrowed first, dequant_int4.metal:240-245), then the down projection.
 bool dense_mlp_takes(const mf_qtensor& gate, const mf_qtensor& up, const mf_qtensor& down, const void* x,
                      const void* y, const void* scratch, uint32_t d, uint32_t f, uint32_t t) {
-  if (d % kQmmRows || f % kQmmRows || t == 0) return false;
+  if (d % kGroup || f % kGroup || d < kQmmRows || f < kQmmRows || t == 0) return false;
   return aligned16(gate.weights) && aligned16(up.weights) && aligned16(down.weights) && aligned16(x) && aligned16(y) &&
          aligned16(scratch) && static_cast<uint64_t>(t) * std::max(d, f) < (1ull << 31);
 }
@@ -2470,11 +2478,19 @@ size_t prefill_workspace_bytes(const mf_moe_config& c, uint32_t t) {
   return prefill_carve(c, t, nullptr).bytes;
 }
 
+// widths of whole 128-row workgroups: the configurations whose calls insist on a workspace (the others fall back to
+// the decode launch without one) and whose pool can be tiled
+bool prefill_whole_tiles(const mf_moe_config& c) {
+  return prefill_supported(c) && c.d % kQmmRows == 0 && c.f % kQmmRows == 0 && c.shared_f % kQmmRows == 0;
+}
+
 bool prefill_supported(const mf_moe_config& c) {
   if (c.bits != MF_BITS_4 && c.bits != MF_BITS_2 && c.bits != MF_BITS_TERNARY) return false;
   if (c.shared_f && c.shared_bits != MF_BITS_4) return false;
   if (c.gate_group_size == 32) return false;  // the matmul's tables hold one entry per 64 weights
-  if (c.d % kQmmRows || c.f % kQmmRows || (c.shared_f % kQmmRows)) return false;
+  // any multiple of the quantization group from 128 on; a width of 64 is one group, which the decode launch serves
+  if (c.d % kGroup || c.f % kGroup || c.shared_f % kGroup) return false;
+  if (c.d < kQmmRows || c.f < kQmmRows || (c.shared_f && c.shared_f < kQmmRows)) return false;
   if (c.d > 8192 || c.f > 8192 || c.shared_f > 8192) return false;
   return true;
 }

@@ -285,6 +285,50 @@ def test_prefill_other_widths_take_the_decode_launch(gpu, oracle):
         assert np.array_equal(y, ops.bf16_bits(yd))
 
 
+@pytest.mark.parametrize("bits,d,f,e,fs,t", [
+    (4, 192, 128, 16, 192, 70),    # an odd number of K groups in front, half a workgroup of rows behind
+    (4, 128, 704, 16, 0, 133),     # eleven groups behind, the last slice of gate / up rows half empty
+    (2, 704, 192, 8, 320, 65),     # 2-bit experts beside a 4-bit shared expert
+    (1, 320, 448, 32, 0, 40),      # ternary
+    (4, 1088, 576, 8, 576, 9),     # one tile, few routes
+])
+def test_prefill_widths_of_whole_groups(gpu, oracle, bits, d, f, e, fs, t):
+    """Widths that are multiples of 64 but not of 128 through the matmuls; without a workspace the same call takes
+    the decode launch and agrees within the layer tolerance."""
+    k = 4
+    root = ROOT_SEED + 0xA280 + d + f
+    layer = oracle.synth_layer(root, d, f, e, k, bits=bits, fs=fs, router_mode=1 if bits == 1 else 0)
+    x = oracle.synth_x(root, t, d)
+    ref_y, ref_idx, ref_w = oracle.moe_layer(layer, x)
+    moe = make_moe(gpu, layer)
+    assert moe.prefill_workspace_bytes(t) > 0
+    wts = to_device_layer(layer)
+    y, idx, w = _run_prefill(moe, wts, x, t, d, k)
+    assert np.array_equal(idx, ref_idx)
+    assert np.array_equal(w.view(np.uint32), ref_w.view(np.uint32))
+    assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref_y), f"bits={bits} d={d} f={f} t={t}")
+    yd = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    moe.encode_prefill_layer(wts, ops.bf16_tensor(x), yd, t, workspace=torch.empty(16, dtype=torch.uint8, device="cuda"))
+    moe.status()
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(yd)), oracle.bf16_to_float(ref_y), "without a workspace")
+
+
+@pytest.mark.parametrize("d,f,t", [(192, 320, 33), (1152, 704, 64), (128, 448, 130)])
+def test_dense_mlp_widths_of_whole_groups(gpu, oracle, d, f, t):
+    """the block form of the dense MLP at widths that are no multiples of 128"""
+    from helpers import to_device_q
+    rng = oracle.Rng.key(ROOT_SEED + 0xA290, f"mlp-{d}-{f}")
+    qs = [oracle.quantize(rng.normal(0.0, 0.02, r * c).reshape(r, c), 4) for r, c in ((f, d), (f, d), (d, f))]
+    xb = oracle.bf16_bits(rng.normal(0.0, 1.0, t * d).reshape(t, d))
+    ref = np.stack([oracle.shared_expert(*qs, xb[i]) for i in range(t)])
+    op = ops.SharedExpertInt4(gpu)
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    scratch = torch.zeros(op.scratch_bytes(d, f, t), dtype=torch.uint8, device="cuda")
+    op.encode(ops.bf16_tensor(xb), *[to_device_q(q) for q in qs], y, scratch, t=t)
+    torch.cuda.synchronize()
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(ref), f"d={d} f={f} t={t}")
+
+
 @pytest.mark.parametrize("d,e,t", [(5120, 32, 40), (5120, 32, 300), (4224, 32, 40), (4224, 48, 290),
                                    (5120, 48, 290)])
 def test_prefill_rows_wider_than_4096(gpu, oracle, d, e, t):
