@@ -10,7 +10,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmfmoe.so")
-SOURCES = ["format.hip", "gemv.hip", "router.hip", "router_family.hip", "moe_decode.hip", "moe_fused.hip",
+SOURCES = ["format.hip", "gemv.hip", "int8_mlp.hip", "router.hip", "router_family.hip", "moe_decode.hip", "moe_fused.hip",
            "moe_prefill.hip", "static_scratch.hip", "api.hip"]
 
 FLAGS = [

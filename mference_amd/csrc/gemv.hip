@@ -929,6 +929,8 @@ hipError_t launch_gemv(hipStream_t s, const mf_qtensor& w, int bits, const uint1
   if (bits == kBits8) {  // one wave per (token, row); any number of token rows
     const uint64_t waves = static_cast<uint64_t>(m) * t;
     if (!waves) return hipSuccess;
+    hipError_t err = hipSuccess;
+    if (launch_q8_gemv(s, w, x, y, m, n, t, out_f32, err)) return err;
     if (waves >= (1ull << 30)) return hipErrorInvalidValue;
     const int al8 = (reinterpret_cast<uintptr_t>(w.weights) % 8 == 0) && n % 8 == 0 && aligned16(x);
     gemv_q8_kernel<<<dim3(static_cast<uint32_t>((waves + 3) / 4)), dim3(256), 0, s>>>(
@@ -1090,6 +1092,8 @@ hipError_t launch_gate_up_act_q8(hipStream_t s, const mf_qtensor& gate, const mf
                                  uint16_t* act, uint32_t f, uint32_t d, uint32_t t, bool silu) {
   const uint64_t waves = static_cast<uint64_t>(f) * t;
   if (!waves) return hipSuccess;
+  hipError_t err = hipSuccess;
+  if (launch_q8_gate_up(s, gate, up, x, act, f, d, t, silu, err)) return err;
   if (waves >= (1ull << 30)) return hipErrorInvalidValue;
   const int al8 = (reinterpret_cast<uintptr_t>(gate.weights) % 8 == 0) && (reinterpret_cast<uintptr_t>(up.weights) % 8 == 0) &&
                   d % 8 == 0 && aligned16(x);

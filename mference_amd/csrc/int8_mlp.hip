@@ -1,0 +1,335 @@
+// 8-bit affine rows beyond the one-wave-per-(token, row) kernels of gemv.hip: a row kernel that requests a whole
+// row before it uses any of it (few token rows, the bits of those kernels), and a matrix-core matmul (many).
+//
+// Replaces shared_int8_gate_up_act_simd and dequant_int8_gemv_simd (Metal/Quant/dequant_int8.metal:66-164).
+#include <algorithm>
+
+#include "mf_device.h"
+#include "mf_internal.h"
+#include "mf_router.h"
+
+#pragma clang fp contract(off)
+
+namespace mf {
+
+struct Q8Args {
+  const uint8_t* W[2];
+  const uint16_t* S[2];
+  const uint16_t* B[2];
+  const uint16_t* x;  // [T, N]
+  void* y;            // one projection: [T, M] bf16 or fp32; two: bf16 activations [T, M]
+  uint32_t M, N, T;
+  int out_f32, silu;
+};
+
+// narrowed gate and up, tanh-GELU or SiLU (int8_gelu_pytorch_tanh and FC_SHARED_INT8_ACT_SILU, dequant_int8.metal:44-57)
+__device__ __forceinline__ uint16_t q8_activation(float g, float u, bool silu) {
+  const float gh = round_bf16(g), uh = round_bf16(u);
+  return f_to_bf16((silu ? mf_silu(gh) : mf_gelu_tanh(gh)) * uh);
+}
+
+// ---- few token rows: one wave per weight row (both projections), in dot_q8_row's order -- chunk c of 8 codes on lane
+// c % 64, sums in ascending order, two fmas per chunk, neighbour-first butterfly -- so a token has the same bits in
+// every kernel of this family.  Bound: a wave's life is one memory round trip plus its arithmetic.  Chunk by chunk
+// (gemv_q8_kernel) a 2816-element row is six round trips in a row; here the codes, tables and the first token's x of
+// the whole row leave together (CPL chunks per lane), and every further token reuses the codes.
+template <int NPROJ, int CPL>
+__global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= a.M) return;
+  const uint32_t chunks = a.N / 8, ng = a.N / kGroup;
+  uint2 q[NPROJ][CPL];
+  uint32_t sr[NPROJ][CPL], br[NPROJ][CPL];
+  uint4 xv[CPL], xn[CPL];
+#pragma unroll
+  for (int i = 0; i < CPL; ++i) {
+    const uint32_t c = min(lane + 64 * i, chunks - 1);  // a chunk past the row repeats the last one and is dropped
+    xv[i] = load_x8<true>(a.x + c * 8);
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) {
+      q[p][i] = *reinterpret_cast<const uint2*>(a.W[p] + static_cast<size_t>(row) * a.N + c * 8);
+      sr[p][i] = a.S[p][static_cast<size_t>(row) * ng + (c >> 3)];
+      br[p][i] = a.B[p][static_cast<size_t>(row) * ng + (c >> 3)];
+    }
+  }
+  issue_fence();
+  for (uint32_t t = 0; t < a.T; ++t) {
+    const uint16_t* nx = a.x + static_cast<size_t>(min(t + 1, a.T - 1)) * a.N;  // (the last token requests itself again)
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) xn[i] = load_x8<true>(nx + min(lane + 64 * i, chunks - 1) * 8);
+    issue_fence();
+    float acc[NPROJ];
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) acc[p] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      if (lane + 64 * i < chunks) {
+        const uint32_t xs[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+        float dot[NPROJ], sum = 0.0f;
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) dot[p] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float x0 = bf16_lo(xs[j]), x1 = bf16_hi(xs[j]);
+          sum = sum + x0;
+          sum = sum + x1;
+#pragma unroll
+          for (int p = 0; p < NPROJ; ++p) {
+            const uint32_t word = (j < 2 ? q[p][i].x : q[p][i].y) >> ((j & 1) * 16);
+            dot[p] = __builtin_fmaf(static_cast<float>(word & 0xFFu), x0, dot[p]);
+            dot[p] = __builtin_fmaf(static_cast<float>((word >> 8) & 0xFFu), x1, dot[p]);
+          }
+        }
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) {
+          acc[p] = __builtin_fmaf(__uint_as_float(sr[p][i] << 16), dot[p], acc[p]);
+          acc[p] = __builtin_fmaf(__uint_as_float(br[p][i] << 16), sum, acc[p]);
+        }
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) acc[p] = wave_sum(acc[p]);
+    if (lane == 0) {
+      const size_t at = static_cast<size_t>(t) * a.M + row;
+      if constexpr (NPROJ == 2) static_cast<uint16_t*>(a.y)[at] = q8_activation(acc[0], acc[1], a.silu != 0);
+      else if (a.out_f32) static_cast<float*>(a.y)[at] = acc[0];
+      else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(acc[0]);
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) xv[i] = xn[i];
+  }
+}
+
+// ---- many token rows, on the bf16 matrix cores.  Codes 0..255 are bf16 numbers as they are, so a K group is
+// sum(q x) from four 32x32x16 products, one fp32 multiply-add with the row's scale, and the biases enter as one more
+// product per two groups: sum(x) of a group as three bf16 terms (all 24 bits) against the bias in three K slots.
+// Tokens are the M side, weight rows the N side: a lane ends with one weight row, its scale is a per-lane scalar.
+//
+// A workgroup is 64 weight rows (of each projection) x 64 NT tokens, waves 2 x 2.  A stage is 128 K values: x rows and
+// code rows come in as whole 128-byte lines, one stage ahead in registers, and are handed out through LDS (16-byte
+// pieces, XOR-swizzled so that 16 lanes reading one piece of 16 rows cover all banks): read straight from memory a
+// lane's 16 bytes of its own row touch 32 lines per load instruction, and the line rate of the L1, not the matrix
+// core, would set the pace.
+template <int NPROJ, int NT>
+__global__ __launch_bounds__(256) void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
+  constexpr uint32_t kTok = 64 * NT;
+  __shared__ uint4 s_x[2][kTok * 16];          // [token][16 pieces of 8 values], piece ^ (token & 15)
+  __shared__ uint4 s_w[2][NPROJ][64 * 8];      // [row][8 pieces of 16 codes], piece ^ ((row >> 1) & 7)
+  __shared__ float s_sum[2][kTok][2];          // sum of x over the stage's two groups
+  // consecutive work items (the token tiles of one row slice) on one XCD: its L2 serves the weight rows' re-reads
+  const uint32_t per = (n_work + 7) / 8, work = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if ((blockIdx.x >> 3) >= per || work >= n_work) return;
+  const uint32_t t0 = (work % n_tiles) * kTok, r0 = (work / n_tiles) * 64;
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m = lane & 31, h = lane >> 5;
+  const uint32_t rb = wv & 1, tb = wv >> 1;
+  const uint32_t ng = a.N / kGroup, n_st = (ng + 1) / 2;
+
+  // staging roles: x -- token t / 4 (+ 64), pieces 4q .. 4q + 3 (half a group); codes -- row t / 8 (+ 32), piece t % 8
+  const uint32_t xt = threadIdx.x >> 2, xq = threadIdx.x & 3, wr = threadIdx.x >> 3, wc = threadIdx.x & 7;
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t xr[NT][4], wreg[NPROJ][2];
+  const uint32_t row = min(r0 + rb * 32 + m, a.M - 1);  // the lane's weight row (past the end: the last one, not stored)
+  uint32_t sc[NPROJ][2], bi[NPROJ];                     // scale words of the stage's groups; the bias of group h of it
+  auto fetch = [&](uint32_t st) __attribute__((always_inline)) {
+    const uint32_t g = 2 * st + (xq >> 1);
+    const bool in = g < ng;  // half a stage behind an odd number of groups: zeros
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt + 64 * n, a.T - 1)) * a.N + (in ? g : ng - 1) * kGroup + (xq & 1) * 32;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        xr[n][i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
+        if (!in) xr[n][i] = u32x4_t{0, 0, 0, 0};
+      }
+    }
+    const uint32_t k0 = min(st * 128 + wc * 16, a.N - 16);  // (codes past the row meet x = 0)
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        wreg[p][i] = *reinterpret_cast<const u32x4_t*>(a.W[p] + static_cast<size_t>(min(r0 + wr + 32 * i, a.M - 1)) * a.N + k0);
+    }
+  };
+  auto fetch_tab = [&](uint32_t st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) {
+      const size_t at = static_cast<size_t>(row) * ng;
+      sc[p][0] = a.S[p][at + min(2 * st, ng - 1)];
+      sc[p][1] = a.S[p][at + min(2 * st + 1, ng - 1)];
+      bi[p] = a.B[p][at + min(2 * st + h, ng - 1)];
+    }
+  };
+  auto put = [&](uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const uint32_t tok = xt + 64 * n;
+      float part = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const u32x4_t v = xr[n][i];
+        reinterpret_cast<u32x4_t*>(s_x[buf])[tok * 16 + ((4 * xq + i) ^ (tok & 15u))] = v;
+        part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
+                ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
+      }
+      part = group_sum(part, 2);
+      if ((xq & 1) == 0) s_sum[buf][tok][xq >> 1] = part;
+    }
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t r = wr + 32 * i;
+        reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = wreg[p][i];
+      }
+  };
+  f32x16_t acc[NPROJ][NT];
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[p][n][r] = 0.0f;
+
+  fetch(0);
+  fetch_tab(0);
+  put(0);
+  if (n_st > 1) fetch(1);
+  for (uint32_t st = 0; st < n_st; ++st) {
+    __syncthreads();  // buffer st & 1 is complete, the other one is no longer read
+    const uint32_t buf = st & 1;
+    uint32_t scv[NPROJ][2], bv[NPROJ];
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) scv[p][0] = sc[p][0], scv[p][1] = sc[p][1], bv[p] = bi[p];
+    if (st + 1 < n_st) {
+      put(buf ^ 1);
+      fetch_tab(st + 1);
+      if (st + 2 < n_st) fetch(st + 2);
+    }
+    // biases: K slots of half h = (hi, mid, lo) of sum(x) over group 2 st + h (a group past the end sums to 0)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const float v = s_sum[buf][(tb * NT + n) * 32 + m][h];
+      const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
+      const float r1 = v - __uint_as_float(hi);
+      const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
+      const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
+      const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) acc[p][n] = mfma_bf16(av, make_uint4(bv[p] | (bv[p] << 16), bv[p], 0, 0), acc[p][n]);
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      uint4 bx[NT][4];
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        const uint32_t tok = (tb * NT + n) * 32 + m;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) bx[n][s] = s_x[buf][tok * 16 + ((8 * g + 4 * h + s) ^ (tok & 15u))];
+      }
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+        const uint32_t r = rb * 32 + m;
+        f32x16_t tmp[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) tmp[n][i] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const uint4 w = s_w[buf][p][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
+          const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {  // eight codes -> eight bf16 numbers (a byte as fp32 has its bits in the upper half)
+            uint32_t o[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t word = ww[2 * u + (k >> 1)] >> (16 * (k & 1));
+              o[k] = __builtin_amdgcn_perm(__float_as_uint(static_cast<float>((word >> 8) & 0xFFu)),
+                                           __float_as_uint(static_cast<float>(word & 0xFFu)), 0x07060302u);
+            }
+            const uint4 ov = make_uint4(o[0], o[1], o[2], o[3]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) tmp[n] = mfma_bf16(bx[n][2 * c + u], ov, tmp[n]);
+          }
+        }
+        const float s = __uint_as_float(scv[p][g] << 16);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[p][n][i] = __builtin_fmaf(s, tmp[n][i], acc[p][n][i]);
+      }
+    }
+  }
+  // the lane holds weight row r0 + 32 rb + m for tokens 8j + 4h + i of each 32-token block
+  const uint32_t out_row = r0 + rb * 32 + m;
+  if (out_row >= a.M) return;
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t tok = t0 + (tb * NT + n) * 32 + 8 * j + 4 * h + i;
+        if (tok >= a.T) continue;
+        const size_t at = static_cast<size_t>(tok) * a.M + out_row;
+        const float v = acc[0][n][4 * j + i];
+        if constexpr (NPROJ == 2) static_cast<uint16_t*>(a.y)[at] = q8_activation(v, acc[NPROJ - 1][n][4 * j + i], a.silu != 0);
+        else if (a.out_f32) static_cast<float*>(a.y)[at] = v;
+        else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(v);
+      }
+}
+
+// Which kernel: from 16 token rows on the matmul (its workgroups take 64 tokens at the price of one), below that the row
+// kernel while a row fits its registers and there are rows enough to cover the chip; false: neither takes the shape.
+template <int NPROJ>
+static bool q8_launch(hipStream_t s, const Q8Args& a, hipError_t& err) {
+  for (int p = 0; p < NPROJ; ++p)
+    if (!aligned16(a.W[p])) return false;
+  if (!aligned16(a.x) || a.N % kGroup) return false;
+  if (a.T >= 16 && a.M >= 64) {
+    // 128 tokens per workgroup once 64 would give every CU more than two workgroups
+    const uint32_t slices = (a.M + 63) / 64;
+    const bool wide = slices * ((a.T + 63) / 64) > 768;
+    const uint32_t tok = wide ? 128 : 64, tiles = (a.T + tok - 1) / tok, n_work = slices * tiles;
+    const dim3 grid((n_work + 7) / 8 * 8), block(256);
+    if (wide) qmm8_kernel<NPROJ, 2><<<grid, block, 0, s>>>(a, tiles, n_work);
+    else qmm8_kernel<NPROJ, 1><<<grid, block, 0, s>>>(a, tiles, n_work);
+    err = hipGetLastError();
+    return true;
+  }
+  if (a.M < 256 || a.N > 8 * 512) return false;
+  const uint32_t cpl = (a.N / 8 + 63) / 64;
+  const dim3 grid((a.M + 3) / 4), block(256);
+#define MF_Q8(C) rows_q8_kernel<NPROJ, C><<<grid, block, 0, s>>>(a)
+  if (cpl <= 2) MF_Q8(2);
+  else if (cpl <= 4) MF_Q8(4);
+  else if (cpl <= 5) MF_Q8(5);
+  else if (cpl <= 6) MF_Q8(6);
+  else MF_Q8(8);
+#undef MF_Q8
+  err = hipGetLastError();
+  return true;
+}
+
+bool launch_q8_gemv(hipStream_t s, const mf_qtensor& w, const uint16_t* x, void* y, uint32_t m, uint32_t n, uint32_t t,
+                    bool out_f32, hipError_t& err) {
+  Q8Args a{};
+  a.W[0] = a.W[1] = static_cast<const uint8_t*>(w.weights);
+  a.S[0] = a.S[1] = w.scales;
+  a.B[0] = a.B[1] = w.biases;
+  a.x = x; a.y = y; a.M = m; a.N = n; a.T = t; a.out_f32 = out_f32 ? 1 : 0;
+  return q8_launch<1>(s, a, err);
+}
+
+bool launch_q8_gate_up(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const uint16_t* x, uint16_t* act,
+                       uint32_t f, uint32_t d, uint32_t t, bool silu, hipError_t& err) {
+  Q8Args a{};
+  a.W[0] = static_cast<const uint8_t*>(gate.weights); a.W[1] = static_cast<const uint8_t*>(up.weights);
+  a.S[0] = gate.scales; a.S[1] = up.scales;
+  a.B[0] = gate.biases; a.B[1] = up.biases;
+  a.x = x; a.y = act; a.M = f; a.N = d; a.T = t; a.silu = silu ? 1 : 0;
+  return q8_launch<2>(s, a, err);
+}
+
+}  // namespace mf

@@ -78,6 +78,11 @@ hipError_t launch_gate_up_act(hipStream_t s, const mf_qtensor& gate, const mf_qt
                               uint32_t t, bool lane_order = false);
 hipError_t launch_gate_up_act_q8(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const uint16_t* x,
                                  uint16_t* act, uint32_t f, uint32_t d, uint32_t t, bool silu);
+// int8_mlp.hip: the same two operations for the shapes its kernels take (false: not this shape, nothing launched)
+bool launch_q8_gemv(hipStream_t s, const mf_qtensor& w, const uint16_t* x, void* y, uint32_t m, uint32_t n, uint32_t t,
+                    bool out_f32, hipError_t& err);
+bool launch_q8_gate_up(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const uint16_t* x, uint16_t* act,
+                       uint32_t f, uint32_t d, uint32_t t, bool silu, hipError_t& err);
 hipError_t launch_residual_rmsnorm(hipStream_t s, uint16_t* hidden, const uint16_t* delta,
                                    const uint16_t* weight, uint16_t* out, uint32_t d, uint32_t t, float eps);
 hipError_t launch_silu_mul(hipStream_t s, const uint16_t* gate, const uint16_t* up, uint16_t* out,

@@ -1058,6 +1058,28 @@ def test_int8_shared_expert(gpu, oracle, d, f, t, silu):
                                      scratch.data_ptr(), t * f * 2) == -2
 
 
+@pytest.mark.parametrize("d,f,t,silu", [(128, 64, 16, False), (192, 128, 65, True), (320, 704, 130, False),
+                                        (2816, 2112, 33, False), (704, 64, 15, True), (4096, 320, 8, False)])
+def test_int8_shared_expert_many_rows(gpu, oracle, d, f, t, silu):
+    """from 16 rows on the 8-bit MLP is a matrix-core matmul (odd numbers of K groups, half slices of rows, ragged
+    token tiles): within the layer tolerance of the checker; below, the checker's bits"""
+    rng = oracle.Rng.key(ROOT_SEED + 0x1E9, f"int8-mlp-{d}-{f}")
+    qs = [oracle.quantize(rng.normal(0.0, 0.03, r * c).reshape(r, c), 8) for r, c in ((f, d), (f, d), (d, f))]
+    xb = oracle.bf16_bits(rng.normal(0.0, 1.0, t * d).reshape(t, d))
+    ref = np.stack([oracle.shared_expert_int8(*qs, xb[i], silu=silu) for i in range(t)])
+    op = ops.SharedExpertInt8(gpu, silu_activation=silu)
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    scratch = torch.zeros((t, f), dtype=torch.bfloat16, device="cuda")
+    op.encode(ops.bf16_tensor(xb), *[to_device_q(q) for q in qs], y, scratch, t=t)
+    torch.cuda.synchronize()
+    if t < 16:
+        assert np.array_equal(ops.bf16_bits(y), ref)
+    else:
+        got, want = (oracle.bf16_to_float(v).astype(np.float64) for v in (ops.bf16_bits(y), ref))
+        assert np.linalg.norm(got - want) <= 1e-3 * np.linalg.norm(want)
+        assert np.abs(got - want).max() <= 2.0 ** -6 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("bits,d,f,e,k,fs,t,with_delta", [
     (4, 2048, 512, 256, 8, 512, 1, True),     # the headline shape's one-token instance
     (4, 2048, 512, 256, 8, 512, 5, False),    # ... its several-rows instance, no delta
