@@ -885,12 +885,8 @@ bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipErr
   if (lds > 156 * 1024 || (n_ks != 4 && n_ks != 16) || (NPROJ == 2 && n_ks != 4)) return false;
   RowsMfmaArgs b = a;
   b.gps = gps;
-  const void* fn = n_ks == 4 ? reinterpret_cast<const void*>(rows_mfma_kernel<NPROJ, 4>)
-                             : reinterpret_cast<const void*>(rows_mfma_kernel<1, 16>);
-  if (lds > 48 * 1024) {
-    err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    if (err != hipSuccess) return true;
-  }
+  err = n_ks == 4 ? allow_lds<rows_mfma_kernel<NPROJ, 4>>(lds, 156 * 1024) : allow_lds<rows_mfma_kernel<1, 16>>(lds, 156 * 1024);
+  if (err != hipSuccess) return true;
   if (n_ks == 4) rows_mfma_kernel<NPROJ, 4><<<dim3(blocks), dim3(256), lds, s>>>(b);
   else rows_mfma_kernel<1, 16><<<dim3(blocks), dim3(1024), lds, s>>>(b);
   err = hipGetLastError();

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/mfmoe.h"
 
 struct mf_ctx {
@@ -51,6 +53,22 @@ namespace mf {
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 inline bool aligned2(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 1u) == 0; }
+
+// Dynamic LDS beyond the 48 KiB default is allowed once per kernel and device, up to `cap` bytes, and not again on every
+// launch (a runtime call of its own).
+template <auto KERNEL>
+hipError_t allow_lds(size_t lds, int cap) {
+  if (lds <= 48 * 1024) return hipSuccess;
+  static std::atomic<uint64_t> done{0};  // bit per device
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (dev < 64 && (done.load(std::memory_order_acquire) & bit)) return hipSuccess;
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, cap);
+  if (e == hipSuccess && dev < 64) done.fetch_or(bit, std::memory_order_release);
+  return e;
+}
 
 // lanes of a wave that share one row of n elements (power of two, <= 64)
 inline uint32_t lanes_per_row_log2(uint32_t n, int elems_per_lane) {

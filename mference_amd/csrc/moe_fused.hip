@@ -1057,14 +1057,9 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   }
 #define MF_FUSED(B, SB, SHAPE)                                                                 \
   do {                                                                                         \
-    auto kern = fused_decode_kernel<B, SB, SHAPE>;                                             \
-    if (lds > 48 * 1024) {                                                                     \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                  \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,           \
-                                         static_cast<int>(lds));                               \
-      if (e != hipSuccess) return e;                                                           \
-    }                                                                                          \
-    kern<<<grid, block, lds, s>>>(a);                                                          \
+    const hipError_t e = allow_lds<fused_decode_kernel<B, SB, SHAPE>>(lds, kFusedLdsLimit);    \
+    if (e != hipSuccess) return e;                                                             \
+    fused_decode_kernel<B, SB, SHAPE><<<grid, block, lds, s>>>(a);                             \
   } while (0)
   // Shape-specialised instances: a layer shape's dimensions as literals with the token rows read from the
   // arguments (Tn), and the one-token launch with T = 1 as a literal as well (T1: it drops the code of the
@@ -1108,14 +1103,9 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   const bool lit = !h.generic_shape;  // shape instances allowed
 #define MF_FUSED_N(B, SB, SHAPE)                                                               \
   do {                                                                                         \
-    auto kern = fused_decode_kernel<B, SB, SHAPE, true>;                                       \
-    if (lds > 48 * 1024) {                                                                     \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),                  \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,           \
-                                         static_cast<int>(lds));                               \
-      if (e != hipSuccess) return e;                                                           \
-    }                                                                                          \
-    kern<<<grid, block, lds, s>>>(a);                                                          \
+    const hipError_t e = allow_lds<fused_decode_kernel<B, SB, SHAPE, true>>(lds, kFusedLdsLimit); \
+    if (e != hipSuccess) return e;                                                             \
+    fused_decode_kernel<B, SB, SHAPE, true><<<grid, block, lds, s>>>(a);                       \
   } while (0)
   if (norm) {  // x made inside the launch: the Qwen shape's instances and the ones that read every dimension
     if (lit && qwen && t == 1 && !c.maple_rounding && no_limit && a.xprep) MF_FUSED_N(kBits4, kBits4, QwenT1);

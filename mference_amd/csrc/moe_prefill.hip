@@ -30,6 +30,7 @@
 
 namespace mf {
 
+constexpr int kMaxLds = 160 * 1024;    // LDS of a CU
 constexpr uint32_t kTileTokens = 64;   // tokens of one expert a workgroup handles
 constexpr uint32_t kQmmWaves = 4;      // waves per workgroup, 32 weight rows each
 constexpr uint32_t kQmmRows = kQmmWaves * 32;
@@ -2005,8 +2006,7 @@ hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint
     const size_t lds = group_one_lds_bytes(t, E);
     uint32_t tpe_log2 = 0;  // threads per row of the bit matrix: as many as 1024 threads give, at most 16
     while (tpe_log2 < 4 && (E << (tpe_log2 + 1)) <= 1024) ++tpe_log2;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(group_one_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGroupOneMaxBytes));
+    const hipError_t e = allow_lds<group_one_kernel>(lds, static_cast<int>(kGroupOneMaxBytes));
     if (e != hipSuccess) return e;
     group_one_kernel<<<dim3(1), dim3(1024), lds, s>>>(idx, w, n_pairs, K, E, tpe_log2, counts, offsets, starts, sorted,
                                                       static_cast<Tile*>(tiles), tile_slots, n_tiles, status);
@@ -2133,11 +2133,8 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
   const size_t lds = static_cast<size_t>(ng) * 8192 + kTileTokens * 4 + kTileTokens * ng * 4;
 #define MF_KRES(B, N)                                                                                  \
   do {                                                                                                 \
-    if (lds > 48 * 1024) {                                                                             \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qmm_kres_kernel<B, N>),         \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-      if (e != hipSuccess) return e;                                                                   \
-    }                                                                                                  \
+    const hipError_t e = allow_lds<qmm_kres_kernel<B, N>>(lds, kMaxLds);                               \
+    if (e != hipSuccess) return e;                                                                     \
     qmm_kres_kernel<B, N><<<grid, block, lds, s>>>(launch);                                            \
   } while (0)
   if (bits == 4) {
@@ -2182,11 +2179,8 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
   if (grid.x == 0) return hipSuccess;
 #define MF_QMM(B, P, G, T)                                                                             \
   do {                                                                                                 \
-    if (lds > 48 * 1024) {                                                                             \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(qmm_kernel<B, P, G, T>),        \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)); \
-      if (e != hipSuccess) return e;                                                                   \
-    }                                                                                                  \
+    const hipError_t e = allow_lds<qmm_kernel<B, P, G, T>>(lds, kMaxLds);                              \
+    if (e != hipSuccess) return e;                                                                     \
     qmm_kernel<B, P, G, T><<<grid, block, lds, s>>>(launch);                                           \
   } while (0)
 #define MF_QMM_G(B, P, G)                                            \
