@@ -76,7 +76,7 @@ def write_shapes_inc(shapes: list[dict]) -> str:
                 f"c.num_experts == {sh['num_experts']} && c.top_k == {sh['top_k']} && c.shared_f == {fs}")
         if fs:
             cond += f" && c.shared_bits == {_MF_BITS[sh['shared_bits']]}"
-        one = f"t == 1 && c.maple_rounding == {maple}u && no_limit && a.xprep"
+        one = f"one && c.maple_rounding == {maple}u && no_limit && a.xprep"
         own.append(f"  else if ({cond} && c.router_mode == {mode}) {{\n"
                    f"    if ({one}) MF_FUSED({b}, {sb}, Gen{i}T1);\n    else MF_FUSED({b}, {sb}, Gen{i}Tn);\n  }}")
         given.append(f"  else if ({cond}) {{\n"

@@ -218,8 +218,13 @@ __device__ __forceinline__ bool full_softmax_probs(const float* lg, float* p, ui
       const bool live = x < e;
       ch[j] = live ? mf_exp(ch[j] - mx) : 0.0f;
       float part = ch[j];
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) part = part + __shfl_xor(part, o, kWave);
+      // xor strides 16, 8, 4, 2, 1 (behind the stride-8 step the values repeat every 8 lanes, so the rotation by 4
+      // is the exchange with lane ^ 4, and so on down)
+      part = part + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(part), 0x401F));
+      part = part + dpp_f<0x128>(part);
+      part = part + dpp_f<0x124>(part);
+      part = part + dpp_f<0x122>(part);
+      part = part + dpp_f<0x121>(part);
       const float lo = readlane_f(part, 0), hi = readlane_f(part, 32);
       if (static_cast<uint32_t>(2 * j) < e / 32) total += lo;
       if (static_cast<uint32_t>(2 * j + 1) < e / 32) total += hi;

@@ -44,6 +44,9 @@
 // than CUs and the kernel needs a whole CU (1024 threads, <= 128 VGPRs).  Waits
 // are bounded: a poll that does not complete within kSpinLimit tries sets the
 // status word, the workgroup writes NaN to the output rows it owns and the grid drains.
+#include <algorithm>
+#include <type_traits>
+
 #include "mf_device.h"
 #include "mf_internal.h"
 #include "mf_router.h"
@@ -148,6 +151,29 @@ __device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, const f
   return xs;
 }
 
+// n / d for n < 2^31 as a multiplication: the dimensions of most instances are launch arguments, a division by one
+// expands to some thirty instructions, and with sixteen waves on a CU an instruction that every wave executes costs 5 ns.
+struct FastDiv {
+  uint32_t m, add, sh;
+};
+__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.m) + (n & f.add)) >> f.sh; }
+static FastDiv make_fastdiv(uint32_t d) {
+  if (d <= 1) return FastDiv{0u, ~0u, 0u};
+  uint32_t s = 1;
+  while (s < 31 && (1u << s) < d) ++s;
+  return FastDiv{static_cast<uint32_t>((1ull << (31 + s)) / d + 1), 0u, s - 1};
+}
+
+// Launch geometry: what follows from the shape and the number of workgroups (uniform, made on the host once per launch)
+struct FusedGeo {
+  uint32_t b_per_wg;   // units (rpw rows of one routed slot) a workgroup takes in stage B
+  uint32_t c_wgs;      // workgroups that share one token's output rows in stage C
+  uint32_t c_units;    // output units of one workgroup: per round (rows form) or in all (units form)
+  uint32_t c_rounds;   // rounds (rows form)
+  uint8_t lpr_d, lpr_f, lpr_sd, lpr_sf;  // log2 of the lanes per row: rows of D and F (routed), of D and Fs (shared)
+  FastDiv E, n_sl, rgf, K, srg, c_wgs_div, rpr;
+};
+
 struct FusedArgs {
   const uint16_t* router_w;
   const uint8_t* expert_base;
@@ -182,6 +208,7 @@ struct FusedArgs {
   int maple;  // MapleMoE's rounding points (mf_moe_config::maple_rounding)
   uint32_t stage_words;  // words of the LDS staging area
   int xprep;             // the routed rows read x from LDS, permuted and summed once per workgroup
+  FusedGeo g;
 };
 
 __device__ __forceinline__ void store_u64_agent(unsigned long long* p, unsigned long long v) {
@@ -238,7 +265,48 @@ constexpr uint32_t static_rows_per_wave(uint32_t n, uint32_t elems_per_lane) {
   return 64u / lanes;
 }
 
-template <int BITS, int SBITS, class S, bool NORM = false>
+// The launch geometry as one function of the shape, for the host (every instance) and at compile time (the one-token
+// instances with literal dimensions, which the launcher picks for kStaticWgs workgroups only).
+constexpr uint32_t kStaticWgs = 256;
+
+// Units of stage B one workgroup takes: an equal share, in whole 64-byte pieces of the exchanged activations (one
+// writer per memory line).
+constexpr uint32_t fused_b_per_wg(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg) {
+  const uint32_t rpw = static_rows_per_wave(d, epl);
+  const uint32_t n = t * k * ((f + rpw - 1) / rpw), piece = rpw < 16 ? 16 / rpw : 1;
+  const uint32_t share = (n + n_wg - 1) / n_wg;
+  return (share + piece - 1) / piece * piece;
+}
+
+// How stage C deals a token's output rows.  Rows form: a unit's K slots on K waves, their values meet in LDS -- all
+// waves work although a workgroup has only a unit or two.  Units form: a wave takes all K slots of a unit one after
+// the other with four rows requested ahead, no meeting -- from three units per workgroup on (large 2-bit layer, one
+// token: 8 units; most shapes at several tokens), while a row is one step of 64 lanes and the slices of the
+// activations are at most one a thread.
+struct FusedSplit {
+  bool by_units;
+  uint32_t wgs, units, rounds;  // workgroups per token; units per workgroup (rows form: and round); rounds
+};
+constexpr FusedSplit fused_split(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg) {
+  const uint32_t rpw = static_rows_per_wave(f, epl), rg = (d + rpw - 1) / rpw, wgs = n_wg / t;
+  const uint32_t share = (rg + wgs - 1) / wgs;
+  const bool by_units = share >= 3 && f <= 64 * epl && k * (f / epl) <= kFusedThreads;
+  const uint32_t per_round = kFusedWaves / k < share ? kFusedWaves / k : share;
+  const uint32_t units = by_units ? share : per_round;
+  return FusedSplit{by_units, wgs, units, by_units ? 1 : (rg + wgs * units - 1) / (wgs * units)};
+}
+
+// stage A: waves that poll for n2 16-byte pieces of tagged logits, and waves that build n slices of x
+__host__ __device__ __forceinline__ uint32_t fused_poll_waves(uint32_t n2) {
+  const uint32_t w = (n2 + kWave - 1) / kWave;
+  return w < 8 ? w : 8;
+}
+__host__ __device__ __forceinline__ uint32_t fused_slice_waves(uint32_t n, uint32_t n_poll) {
+  const uint32_t w = (n + kWave - 1) / kWave;
+  return w < kFusedWaves - n_poll - 4 ? w : kFusedWaves - n_poll - 4;
+}
+
+template <int BITS, int SBITS, class S, bool NORM, bool UNITS>
 __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const FusedArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t D = S::D != kDyn ? S::D : a.D, F = S::F != kDyn ? S::F : a.F;
@@ -268,7 +336,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // the wave index as a scalar: what derives from it (rows, experts, base addresses) is then
   // computed once per wave by the scalar unit instead of per lane
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t G = gridDim.x, wg = blockIdx.x;
+  const uint32_t G = S::kStatic ? kStaticWgs : gridDim.x, wg = blockIdx.x;
+  constexpr FusedSplit kSplit =
+      S::kStatic ? fused_split(Fmt<BITS>::kElemsPer16B, S::D, S::F, S::K, 1, kStaticWgs) : FusedSplit{UNITS, 0, 0, 0};
+  static_assert(!S::kStatic || (S::T == 1 && kSplit.by_units == UNITS), "an instance with every dimension literal has the form of its shape");
   // x slices of the routed rows, built once per workgroup (when a.xprep)
   constexpr uint32_t kEPL = Fmt<BITS>::kElemsPer16B;
   const uint32_t n_sl = D / kEPL;  // slices per token (the last partial slice, if any, is not kept)
@@ -395,9 +466,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // Who does what while the logits are on their way: the top waves poll for them (n_poll waves),
   // the waves below those build the x slices, the bottom waves have the rows of stage A.
   const uint32_t n2 = S::kGiven ? 0 : T * E / 2;  // 16-byte pieces of tagged logits (E % 4 == 0)
-  const uint32_t n_poll = n2 ? ((n2 + kWave - 1) / kWave < 8 ? (n2 + kWave - 1) / kWave : 8) : 0;
-  const uint32_t n_xw = (T * n_sl + kWave - 1) / kWave < kFusedWaves - n_poll - 4
-                            ? (T * n_sl + kWave - 1) / kWave : kFusedWaves - n_poll - 4;
+  const uint32_t n_poll = fused_poll_waves(n2), n_xw = fused_slice_waves(T * n_sl, n_poll);
 
   // ------------------------------------------------------------- stage A
   // Router rows are on the critical path and their logits are gathered by everybody: they go in
@@ -406,7 +475,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // much later; they are dealt one at a time over the waves of the other workgroups (their
   // dot products are vector-ALU work: spread thin, they cost no workgroup more than a row or two).
   {
-    const uint32_t lpr_log2 = Fs ? lanes_per_row_log2_dev(D, Fmt<SBITS>::kElemsPer16B) : 0;
+    const uint32_t lpr_log2 = S::D != kDyn ? lanes_per_row_log2_dev(D, Fmt<SBITS>::kElemsPer16B) : a.g.lpr_sd;
     const uint32_t lpr = 1u << lpr_log2, rpw = 64u >> lpr_log2;
     const uint32_t n_rows_r = S::kGiven ? 0 : E * T;
     const uint32_t n_rc = (n_rows_r + kRouterChunk - 1) / kRouterChunk;
@@ -414,7 +483,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     for (uint32_t ci = wg; ci < n_rc; ci += G) {
       const uint32_t row = ci * kRouterChunk + wv;
       if (wv < kRouterChunk && row < n_rows_r) {
-        const uint32_t tok = row / E, e = row % E;
+        const uint32_t tok = S::E != kDyn ? row / E : fdiv(row, a.g.E), e = row - tok * E;
         float v;
         if (NORM && pre_router && ci == wg) {  // the weights are here already: dot_bf16_row's products in its order
           const uint16_t* xr = xin + static_cast<size_t>(tok) * D;
@@ -447,7 +516,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     }
     const uint32_t skip = n_rc < G ? n_rc : 0;  // workgroups [0, skip) had router rows
     const uint32_t n_gate = (Fs && (a.w_sg || a.gq_w)) ? T : 0;
-    const uint32_t srg = Fs ? (Fs + rpw - 1) / rpw : 0;
+    const uint32_t srg = (Fs + rpw - 1) >> (6 - lpr_log2);
     const uint32_t n_items = n_gate + T * srg;
     const uint32_t Gs = G - skip;
     for (uint32_t item = wg >= skip ? wv * Gs + (wg - skip) : n_items; item < n_items; item += kFusedWaves * Gs) {
@@ -460,9 +529,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
                           (lane == 0 ? static_cast<uint32_t>(f_to_bf16(v)) : 0u) | (epoch_now() << 16));
       } else {
         const uint32_t it = item - n_gate;
-        const uint32_t srg1 = srg ? srg : 1u;  // no shared expert: this branch is never taken
-        const uint32_t tok = it / srg1;
-        const uint32_t row = (it % srg1) * rpw + (lane >> lpr_log2);
+        // (no shared expert: this branch is never taken)
+        const uint32_t tok = S::Fs != kDyn && S::D != kDyn ? (srg ? it / srg : 0u) : fdiv(it, a.g.srg);
+        const uint32_t row = (it - tok * srg) * rpw + (lane >> lpr_log2);
         const uint32_t sub = lane & (lpr - 1);
         const bool ok = row < Fs;
         const size_t r = ok ? row : 0;
@@ -488,7 +557,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     // the x slices of the routed rows
     if (xprep && wv + n_poll + n_xw >= kFusedWaves && wv + n_poll < kFusedWaves) {
       for (uint32_t q = (wv + n_poll + n_xw - kFusedWaves) * kWave + lane; q < T * n_sl; q += n_xw * kWave) {
-        const uint32_t tok = q / n_sl, sl = q % n_sl;
+        const uint32_t tok = S::D != kDyn ? q / n_sl : fdiv(q, a.g.n_sl), sl = q - tok * n_sl;
         store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, sl,
                                load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(tok) * D + sl * kEPL));
       }
@@ -588,72 +657,100 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // Every workgroup takes a run of consecutive units (rpw rows of one routed slot), its waves
   // take them in turn; gate and up sums meet in LDS, the first threads turn them into
   // activations (one exp and one division per thread instead of per wave) and the run leaves as
-  // one contiguous piece.
+  // one contiguous piece.  A wave with several units (or rows of several steps) requests the next
+  // step's codes before it multiplies the present ones.
   {
-    const uint32_t lpr_log2 = lanes_per_row_log2_dev(D, kEPL);
-    const uint32_t lpr = 1u << lpr_log2, rpw = 64u >> lpr_log2;
-    const uint32_t rgf = (F + rpw - 1) / rpw;   // units per (token, slot)
+    const uint32_t lpr_log2 = S::D != kDyn ? lanes_per_row_log2_dev(D, kEPL) : a.g.lpr_d;
+    const uint32_t lpr = 1u << lpr_log2, rpw_log2 = 6 - lpr_log2, rpw = 1u << rpw_log2;
+    const uint32_t rgf = (F + rpw - 1) >> rpw_log2;   // units per (token, slot)
     const uint32_t n_items = T * K * rgf;
-    uint32_t per_wg = (n_items + G - 1) / G;
-    per_wg = (per_wg + kFusedWaves - 1) / kFusedWaves * kFusedWaves;
+    const uint32_t per_wg = S::kStatic ? fused_b_per_wg(kEPL, S::D, S::F, S::K, 1, kStaticWgs) : a.g.b_per_wg;
     const uint32_t first = wg * per_wg;
     const uint32_t last = first + per_wg < n_items ? first + per_wg : n_items;
     float* s_gu = reinterpret_cast<float*>(s_stage);  // (gate sum, up sum) per staged row
     const uint32_t sub = lane & (lpr - 1), rloc = lane >> lpr_log2;
     const uint32_t ng = D / kGroup;
     const size_t rb = static_cast<size_t>(D) * Store<BITS>::kBits / 8;
-    for (uint32_t item = first + wv; item < last; item += kFusedWaves) {
-      const uint32_t pair = item / rgf;
-      const uint32_t row = (item % rgf) * rpw + rloc;
+    const uint32_t steps = (D + lpr * kEPL - 1) / kEPL >> lpr_log2;  // 16-byte steps of a lane along a row
+    auto pair_of = [&](uint32_t item) __attribute__((always_inline)) {
+      return S::F != kDyn && S::D != kDyn ? item / rgf : fdiv(item, a.g.rgf);
+    };
+    struct Step {
+      Chunk<BITS> g, u;
+      uint32_t tok, e0;  // where its x slice lies; ok: the lane has a row and the slot an expert
+      bool ok;
+    };
+    // one step's codes and table entries, without a branch around the loads: a lane without a row (or past the row's
+    // end), or a router sentinel, reads something that exists and its sums stay 0
+    auto fetch = [&](uint32_t item, uint32_t step, Step& c) __attribute__((always_inline)) {
+      const uint32_t pair = pair_of(item);
+      const uint32_t row = ((item - pair * rgf) << rpw_log2) + rloc;
       const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[pair]);
-      // A lane without a row, or a router sentinel, contributes nothing: its sums stay 0.  For 2-bit codes the
-      // loads carry no branch (such a lane reads a row that exists and drops it): 29.4 -> 28.3 us on the large
-      // 2-bit layer; the 4-bit layers lose 2-3 % at several token rows that way and keep the branch.
-      constexpr bool kFreeLoads = BITS == kBits2;
-      const bool ok = row < F && expert < E;
-      const uint32_t ec = expert < E ? expert : 0u, rc = row < F ? row : 0u;
-      float ga = 0.0f, ua = 0.0f;
-      if (kFreeLoads || ok) {
-        const uint8_t* blob = a.expert_base + static_cast<size_t>(ec) * a.expert_stride;
-        const uint8_t* gw = blob + a.off.gate_w + rc * rb;
-        const uint8_t* uw = blob + a.off.up_w + rc * rb;
-        const uint16_t* gs = reinterpret_cast<const uint16_t*>(blob + a.off.gate_s) + static_cast<size_t>(rc) * ng;
-        const uint16_t* gb = reinterpret_cast<const uint16_t*>(blob + a.off.gate_b) + static_cast<size_t>(rc) * ng;
-        const uint16_t* us = reinterpret_cast<const uint16_t*>(blob + a.off.up_s) + static_cast<size_t>(rc) * ng;
-        const uint16_t* ub = reinterpret_cast<const uint16_t*>(blob + a.off.up_b) + static_cast<size_t>(rc) * ng;
-        const uint32_t tok = pair / K;
-        for (uint32_t e0 = sub * kEPL; e0 < D; e0 += lpr * kEPL) {  // the steps of gate_up_partial
-          const Chunk<BITS> gc = load_chunk<BITS>(gw, gs, gb, e0);
-          const Chunk<BITS> uc = load_chunk<BITS>(uw, us, ub, e0);
-          issue_fence();
-          const XSlice<BITS> xs = xprep ? load_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, e0 / kEPL)
-                                          : load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(tok) * D + e0);
-          const float gd = codes_dot<BITS>(gc.codes, xs), ud = codes_dot<BITS>(uc.codes, xs);
-          if (ok) {
-            ga = __builtin_fmaf(gc.s, gd, ga);
-            ga = __builtin_fmaf(gc.b, xs.sum, ga);
-            ua = __builtin_fmaf(uc.s, ud, ua);
-            ua = __builtin_fmaf(uc.b, xs.sum, ua);
-          }
+      c.e0 = (step * lpr + sub) * kEPL;
+      c.ok = row < F && expert < E && c.e0 < D;
+      if (!(c.e0 < D)) c.e0 = 0;
+      c.tok = S::K != kDyn ? pair / K : fdiv(pair, a.g.K);
+      const uint8_t* blob = a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride;
+      const uint32_t rc = row < F ? row : 0u;
+      const size_t tb = static_cast<size_t>(rc) * ng;
+      c.g = load_chunk<BITS>(blob + a.off.gate_w + rc * rb, reinterpret_cast<const uint16_t*>(blob + a.off.gate_s) + tb,
+                             reinterpret_cast<const uint16_t*>(blob + a.off.gate_b) + tb, c.e0);
+      c.u = load_chunk<BITS>(blob + a.off.up_w + rc * rb, reinterpret_cast<const uint16_t*>(blob + a.off.up_s) + tb,
+                             reinterpret_cast<const uint16_t*>(blob + a.off.up_b) + tb, c.e0);
+    };
+    float ga = 0.0f, ua = 0.0f;
+    auto multiply = [&](uint32_t item, uint32_t step, const Step& c) __attribute__((always_inline)) {
+      const XSlice<BITS> xs = xprep ? load_xslice_lds<BITS>(s_xq, s_xsum, c.tok, n_sl, c.e0 / kEPL)
+                                    : load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(c.tok) * D + c.e0);
+      const float gd = codes_dot<BITS>(c.g.codes, xs), ud = codes_dot<BITS>(c.u.codes, xs);
+      if (c.ok) {
+        ga = __builtin_fmaf(c.g.s, gd, ga);
+        ga = __builtin_fmaf(c.g.b, xs.sum, ga);
+        ua = __builtin_fmaf(c.u.s, ud, ua);
+        ua = __builtin_fmaf(c.u.b, xs.sum, ua);
+      }
+      if (step + 1 == steps) {  // the row is complete
+        const float g = group_sum(ga, static_cast<int>(lpr));
+        const float u = group_sum(ua, static_cast<int>(lpr));
+        if (sub == 0) {
+          float* dst = s_gu + 2 * (((item - first) << rpw_log2) + rloc);
+          dst[0] = g;
+          dst[1] = u;
         }
+        ga = ua = 0.0f;
       }
-      const float g = group_sum(ga, static_cast<int>(lpr));
-      const float u = group_sum(ua, static_cast<int>(lpr));
-      if (sub == 0) {
-        float* dst = s_gu + 2 * ((item - first) * rpw + rloc);
-        dst[0] = g;
-        dst[1] = u;
+    };
+    uint32_t item = first + wv, step = 0;
+    if (item < last) {
+      Step cur;
+      fetch(item, 0, cur);
+      for (;;) {
+        uint32_t nitem = item, nstep = step + 1;
+        if (nstep == steps) {
+          nstep = 0;
+          nitem += kFusedWaves;
+        }
+        if (nitem >= last) break;
+        Step nxt;
+        fetch(nitem, nstep, nxt);
+        issue_fence();
+        multiply(item, step, cur);
+        cur = nxt;
+        item = nitem;
+        step = nstep;
       }
+      multiply(item, step, cur);
     }
     __syncthreads();
     // staged row (item - first) * rpw + r is activation (item % rgf) * rpw + r of pair item / rgf
-    const uint32_t n_words = first < last ? (last - first) * rpw : 0;
+    const uint32_t n_words = first < last ? (last - first) << rpw_log2 : 0;
     for (uint32_t i = threadIdx.x; i < n_words; i += kFusedThreads) {
-      const uint32_t item = first + i / rpw, row = (item % rgf) * rpw + i % rpw;
+      const uint32_t it = first + (i >> rpw_log2), pair = pair_of(it);
+      const uint32_t row = ((it - pair * rgf) << rpw_log2) + (i & (rpw - 1));
       // moe.metal:27-34, 528; maple_moe.metal:153-164
       const uint32_t word =
           static_cast<uint32_t>(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) | (tag16 << 16);
-      if (row < F) store_u32_agent(&a.t_acts[static_cast<size_t>(item / rgf) * F + row], word);
+      if (row < F) store_u32_agent(&a.t_acts[static_cast<size_t>(pair) * F + row], word);
     }
   }
   trace_mark(a, 4);
@@ -667,77 +764,90 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   }
 
   // ------------------------------------------------------------- stage C
-  const uint32_t lpr_log2 = lanes_per_row_log2_dev(F, Fmt<BITS>::kElemsPer16B);
-  const uint32_t lpr = 1u << lpr_log2, rpw = 64u >> lpr_log2;
-  const uint32_t rg_per_tok = (D + rpw - 1) / rpw;  // units (groups of rpw output rows) per token
-  const uint32_t ub = kFusedWaves / K;              // units a workgroup handles per round
-  const uint32_t rounds = (rg_per_tok + G * ub - 1) / (G * ub);
-  const uint32_t unit_local = wv / K, slot = wv % K;
-  const uint32_t sub = lane & (lpr - 1);
+  // The workgroups are split among the tokens: c_wgs of them own the output rows of one token, so a workgroup gathers
+  // one token's activations (T tokens' by every workgroup one after the other: T waits, and T times the bytes past
+  // every cache).  A unit is rpw output rows of the token.
+  const uint32_t lpr_log2 = S::F != kDyn ? lanes_per_row_log2_dev(F, Fmt<BITS>::kElemsPer16B) : a.g.lpr_f;
+  const uint32_t lpr = 1u << lpr_log2, rpw_log2 = 6 - lpr_log2, rpw = 1u << rpw_log2;
+  const uint32_t rg_per_tok = (D + rpw - 1) >> rpw_log2;  // units of a token
+  const uint32_t c_wgs = S::kStatic ? kSplit.wgs : a.g.c_wgs;
+  const uint32_t tok = S::T == 1 ? 0u : fdiv(wg, a.g.c_wgs_div), wl = wg - tok * c_wgs;
+  const uint32_t sub = lane & (lpr - 1), rloc = lane >> lpr_log2;
   const uint32_t ng = F / kGroup;
   const size_t rb = static_cast<size_t>(F) * Store<BITS>::kBits / 8;
-  const uint32_t rows_per_round = ub * rpw;
-  // shared-expert down rows: srpw rows per wave step
-  const uint32_t slpr_log2 = Fs ? lanes_per_row_log2_dev(Fs, Fmt<SBITS>::kElemsPer16B) : 0;
-  const uint32_t slpr = 1u << slpr_log2, srpw = 64u >> slpr_log2;
-
-  // Round 0's routed codes of every token after the first are requested while the token before it is
-  // being summed up (a token's turn is otherwise a round trip to HBM longer).  That request has no branch
-  // around it -- a lane without a row reads one that exists and drops it, and the last token requests its
-  // own row again -- so that the products of the token at hand need not wait for it.  A launch that is
-  // compiled for one token has none of this.
-  constexpr bool kOneToken = S::T == 1;
-  auto request_round0 = [&](uint32_t tok, Chunk<BITS>& c) __attribute__((always_inline)) {
-    const uint32_t unit = wg * ub + unit_local;
-    const uint32_t row = unit * rpw + (lane >> lpr_log2);
-    const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[tok * K + slot]);
-    const uint32_t e0 = sub * Fmt<BITS>::kElemsPer16B;
-    const bool live = unit_local < ub && unit < rg_per_tok && row < D && expert < E && e0 < F;
-    const uint32_t ec = expert < E ? expert : 0u, rc = row < D ? row : 0u, e0c = e0 < F ? e0 : 0u;
-    const uint8_t* blob = a.expert_base + static_cast<size_t>(ec) * a.expert_stride;
-    c = load_chunk<BITS>(blob + a.off.down_w + rc * rb,
-                         reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + static_cast<size_t>(rc) * ng,
-                         reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + static_cast<size_t>(rc) * ng, e0c);
-    return live;
+  const uint32_t ub = S::kStatic ? kSplit.units : a.g.c_units;
+  // The output row behind index i of the workgroup's rows (LDS order): rows form -- round by round, ub units each;
+  // units form -- one run of units.
+  const uint32_t rounds = UNITS ? 1u : S::kStatic ? kSplit.rounds : a.g.c_rounds, rows_per_round = ub << rpw_log2;
+  auto row_at = [&](uint32_t i) __attribute__((always_inline)) {
+    if constexpr (UNITS) return (wl * ub << rpw_log2) + i;
+    const uint32_t round = rounds == 1 ? 0u : fdiv(i, a.g.rpr), in_round = i - round * rows_per_round;
+    return ((round * c_wgs + wl) * ub << rpw_log2) + in_round;
   };
-  Chunk<BITS> pre_next{};
-  bool have_next = false;
-  for (uint32_t tok = 0; tok < T; ++tok) {
-    // request round 0's routed codes, then wait for what other workgroups produce
-    // (the first token's request in the same branch-free form: 12.7 -> 12.35 us per Qwen-shaped layer; the
-    // ternary layer, 13.5 us with the request under its conditions, read 14.5 us without them and keeps them)
-    Chunk<BITS> pre = pre_next;
-    bool have_pre = have_next;
-    if (BITS != kBitsTernary && (kOneToken || tok == 0)) {
-      have_pre = request_round0(tok, pre);
-    } else if (kOneToken || tok == 0) {
-      const uint32_t unit = wg * ub + unit_local;
-      if (unit_local < ub && unit < rg_per_tok) {
-        const uint32_t row = unit * rpw + (lane >> lpr_log2);
-        const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[tok * K + slot]);
-        if (row < D && expert < E && sub * Fmt<BITS>::kElemsPer16B < F) {
-          const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-          pre = load_chunk<BITS>(blob + a.off.down_w + row * rb,
-                                 reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng,
-                                 reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng,
-                                 sub * Fmt<BITS>::kElemsPer16B);
-          have_pre = true;
-        }
+  if (tok < T) {
+    // shared-expert down rows: srpw rows per wave step
+    const uint32_t slpr_log2 = !Fs ? 0u : S::Fs != kDyn ? lanes_per_row_log2_dev(Fs, Fmt<SBITS>::kElemsPer16B) : a.g.lpr_sf;
+    const uint32_t slpr = 1u << slpr_log2, srpw = 64u >> slpr_log2;
+
+    // What the router decided is all a down row needs to be requested: the first codes leave before anything is
+    // waited for.  Rows form: slot wv % K of unit wv / K of the first round.  Units form: a wave walks
+    // (unit, slot) pairs, slots fastest; four of them are in flight.
+    constexpr uint32_t kEPLF = Fmt<BITS>::kElemsPer16B;
+    constexpr int kRing = UNITS ? 4 : 1;
+    Chunk<BITS> ring[kRing];
+    const uint32_t e0 = sub * kEPLF;
+    const bool lane_in = e0 < F;
+    const uint32_t e0c = lane_in ? e0 : 0u;
+    // rows form
+    const uint32_t unit_local = S::K != kDyn ? wv / K : fdiv(wv, a.g.K), slot = wv - unit_local * K;
+    // units form: the slots' blobs and weights, a slot per lane
+    uint32_t base_lo = 0, base_hi = 0;
+    float w_lane = 0.0f;
+    uint32_t f_unit = wv, f_slot = 0;               // the next (unit, slot) to request
+    const uint32_t u_first = wl * ub, u_n = u_first < rg_per_tok ? (rg_per_tok - u_first < ub ? rg_per_tok - u_first : ub) : 0;
+    const uint32_t n_mine = UNITS ? (wv < u_n ? (u_n - wv + kFusedWaves - 1) / kFusedWaves : 0u) * K : 0u;
+    auto request = [&](const uint8_t* blob, uint32_t row) __attribute__((always_inline)) {
+      const uint32_t rc = row < D ? row : 0u;
+      return load_chunk<BITS>(blob + a.off.down_w + rc * rb,
+                              reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + static_cast<size_t>(rc) * ng,
+                              reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + static_cast<size_t>(rc) * ng, e0c);
+    };
+    auto fetch_unit = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
+      const uint64_t base = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_hi), f_slot))) << 32) |
+                            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_lo), f_slot));
+      c = request(reinterpret_cast<const uint8_t*>(base), ((u_first + (f_unit < u_n ? f_unit : 0u)) << rpw_log2) + rloc);
+      if (++f_slot == K) {
+        f_slot = 0;
+        f_unit += kFusedWaves;
       }
+    };
+    auto fetch_first = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
+      const uint32_t unit = wl * ub + unit_local;
+      const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[tok * K + slot]);
+      c = request(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride, (unit << rpw_log2) + rloc);
+    };
+    if constexpr (UNITS) {
+      const uint32_t expert = lane < K ? s_idx[tok * K + lane] : E;
+      const uint64_t base = reinterpret_cast<uint64_t>(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride);
+      base_lo = static_cast<uint32_t>(base);
+      base_hi = static_cast<uint32_t>(base >> 32);
+      if (n_mine) {
+#pragma unroll
+        for (int i = 0; i < kRing; ++i) fetch_unit(ring[i]);
+      }
+    } else if (S::kStatic || unit_local < ub) {  // (literal shapes: no branch around the loads)
+      fetch_first(ring[0]);
     }
     // first shared-expert down chunk of this wave, requested before the wait as well
     const uint32_t sng = Fs ? Fs / kGroup : 0;
     const size_t srb = static_cast<size_t>(Fs) * Store<SBITS>::kBits / 8;
-    const uint32_t n_slots = Fs ? rounds * rows_per_round : 0;
+    const uint32_t n_slots = !Fs ? 0u : UNITS ? u_n << rpw_log2 : rounds * rows_per_round;
     const uint32_t ssub = lane & (slpr - 1);
     Chunk<SBITS> spre{};
     bool have_spre = false;
     if (Fs) {
-      const uint32_t i = wv * srpw + (lane >> slpr_log2);
-      const uint32_t round = i / rows_per_round, in_round = i % rows_per_round;
-      const uint32_t unit = (round * G + wg) * ub + in_round / rpw;
-      const uint32_t row = unit * rpw + in_round % rpw;
-      if (i < n_slots && unit < rg_per_tok && row < D && ssub * Fmt<SBITS>::kElemsPer16B < Fs) {
+      const uint32_t i = wv * srpw + (lane >> slpr_log2), row = row_at(i);
+      if (i < n_slots && row < D && ssub * Fmt<SBITS>::kElemsPer16B < Fs) {
         spre = load_chunk<SBITS>(static_cast<const uint8_t*>(a.sd.weights) + row * srb,
                                  a.sd.scales + static_cast<size_t>(row) * sng,
                                  a.sd.biases + static_cast<size_t>(row) * sng,
@@ -788,16 +898,12 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         }
       }
     };
-    // gated shared output h1 of the output rows this workgroup owns for this token; waves
-    // [0, nw) share the rows
+    // gated shared output h1 of the output rows this workgroup owns; waves [0, nw) share the rows
     auto shared_rows = [&](uint32_t nw) __attribute__((always_inline)) {
       const float gate = gated ? bf16_lo(s_sact[Fs / 2]) : 0.0f;
       for (uint32_t s0 = wv * srpw; s0 < n_slots; s0 += nw * srpw) {
-        const uint32_t i = s0 + (lane >> slpr_log2);  // slot of (round, unit_local, row in unit)
-        const uint32_t round = i / rows_per_round, in_round = i % rows_per_round;
-        const uint32_t unit = (round * G + wg) * ub + in_round / rpw;
-        const uint32_t row = unit * rpw + in_round % rpw;
-        const bool ok = i < n_slots && unit < rg_per_tok && row < D;
+        const uint32_t i = s0 + (lane >> slpr_log2), row = row_at(i);
+        const bool ok = i < n_slots && row < D;
         float part = 0.0f;
         if (ok)
           part = row_partial<SBITS>(static_cast<const uint8_t*>(a.sd.weights) + row * srb,
@@ -814,109 +920,131 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       }
     };
     // waves that own shared rows when the rows are dealt one wave step each
-    const uint32_t sh_waves = Fs ? (n_slots + srpw - 1) / srpw : 0;
-    // (the first token only: the later tokens' routed words have arrived as well by then, and one fetch of
-    // everything is a trip past L2 shorter than two behind each other)
-    const bool split = tok == 0 && Fs && sh_waves <= 4 && n_a <= (kFusedWaves - sh_waves) * 8 * kWave;
+    const uint32_t sh_waves = Fs ? (n_slots + srpw - 1) >> (6 - slpr_log2) : 0;
+    const bool split = Fs && sh_waves <= 4 && n_a <= (kFusedWaves - sh_waves) * 8 * kWave;
     if (split) {
       gather(n_a, n_s, 0, kFusedWaves);  // first try succeeds: one round trip
       __syncthreads();
       if (wv < sh_waves) shared_rows(sh_waves);
       else gather(0, n_a, sh_waves, kFusedWaves - sh_waves);
       __syncthreads();
-      if (tok == 0) trace_mark(a, 5);
+      trace_mark(a, 5);
     } else {
       gather(0, n_a + n_s, 0, kFusedWaves);
       __syncthreads();
-      if (tok == 0) trace_mark(a, 5);
+      trace_mark(a, 5);
       if (Fs) shared_rows(kFusedWaves);
     }
 
-    if constexpr (!kOneToken) {
-      have_next = request_round0(tok + 1 < T ? tok + 1 : tok, pre_next);
-      issue_fence();
-    }
-    // When a lane's share of a row is one 16-byte step, its slice of the slot's activations is the same in
-    // every round: it is built once per token (with several rounds of rows that is a third of the round's
-    // vector work).
-    // (2-bit codes only: their slices are the longest to build and their layers the ones with several rounds;
-    // the 4-bit and ternary launches measured slower with the extra path compiled in)
-    const bool one_step = BITS == kBits2 && lpr * Fmt<BITS>::kElemsPer16B >= F && rounds > 1 && unit_local < ub;
-    XSlice<BITS> xs_slot{};
-    if (one_step && sub * Fmt<BITS>::kElemsPer16B < F)
-      xs_slot = load_xslice<BITS, kXAligned>(reinterpret_cast<const uint16_t*>(s_acts) + slot * F +
-                                             sub * Fmt<BITS>::kElemsPer16B);
-    for (uint32_t round = 0; round < rounds; ++round) {
-      const uint32_t unit = (round * G + wg) * ub + unit_local;
-      const bool active = unit_local < ub && unit < rg_per_tok;
-      if (active) {
-        const uint32_t row = unit * rpw + (lane >> lpr_log2);
-        const uint32_t pair = tok * K + slot;
-        const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[pair]);
-        float part = 0.0f;
-        if (row < D && expert < E) {
-          const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-          const uint8_t* wrow = blob + a.off.down_w + row * rb;
-          const uint16_t* srow = reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng;
-          const uint16_t* brow = reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng;
-          if (one_step) {
-            const uint32_t e0 = sub * Fmt<BITS>::kElemsPer16B;
-            if (e0 < F) {  // the one step of row_partial over the slice at hand
-              uint4 codes = pre.codes;
-              float sc = pre.s, bi = pre.b;
-              if (!(have_pre && round == 0)) {
-                codes = load_codes16<true>(wrow + static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
-                load_scale_bias<BITS>(srow, brow, e0, sc, bi);
-              }
-              part = __builtin_fmaf(sc, codes_dot<BITS>(codes, xs_slot), 0.0f);
-              part = __builtin_fmaf(bi, xs_slot.sum, part);
-            }
-          } else {
-            part = row_partial<BITS>(wrow, srow, brow, reinterpret_cast<const uint16_t*>(s_acts) + slot * F, F, sub,
-                                     lpr, have_pre && round == 0, pre);
-          }
+    auto store_row = [&](uint32_t row, float acc, bool failed) __attribute__((always_inline)) {
+      const size_t o = static_cast<size_t>(tok) * D + row;
+      const uint16_t yb = failed ? static_cast<uint16_t>(0x7FC0u) : f_to_bf16(acc);
+      a.y[o] = yb;
+      if (a.hidden && !failed) {  // residual_add_fp16, utility.metal:83-92
+        uint16_t hv = a.hidden[o];
+        if constexpr (NORM) {  // the residual add in front of the norm, made here for good
+          if (a.delta) hv = f_to_bf16(bf16_to_f(hv) + bf16_to_f(a.delta[o]));
         }
-        const float v = group_sum(part, static_cast<int>(lpr));
-        // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first)
-        if (sub == 0) s_v[wv * kWave + (lane >> lpr_log2)] = s_w[pair] * (maple ? round_bf16(v) : v);
+        a.hidden[o] = f_to_bf16(bf16_to_f(hv) + bf16_to_f(yb));
+      }
+    };
+
+    if constexpr (UNITS) {
+      // The lane slices of the activations (permuted pairs and their sum) are the same for every unit: made once, in
+      // place, in the layout of the x slices.  (The launcher takes this form only when they are at most one a thread
+      // and a row is one step.)
+      const uint32_t spl = F / kEPLF, n_asl = K * spl;
+      float* s_asum = reinterpret_cast<float*>(s_stage);
+      {
+        XSlice<BITS> xs{};
+        if (threadIdx.x < n_asl)
+          xs = load_xslice<BITS, kXAligned>(reinterpret_cast<const uint16_t*>(s_acts) + threadIdx.x * kEPLF);
+        __syncthreads();
+        if (threadIdx.x < n_asl) store_xslice_lds<BITS>(reinterpret_cast<uint4*>(s_acts), s_asum, 0, n_asl, threadIdx.x, xs);
       }
       __syncthreads();
-      if (threadIdx.x < rows_per_round) {
-        const uint32_t ul = threadIdx.x / rpw, rr = threadIdx.x % rpw;
-        const uint32_t u2 = (round * G + wg) * ub + ul;
-        const uint32_t row = u2 * rpw + rr;
-        if (u2 < rg_per_tok && row < D) {
-          const size_t o = static_cast<size_t>(tok) * D + row;
-          // the K weighted values first (independent LDS reads: one round of latency, not K),
-          // then the sum in rank order, residual first
-          float vk[MF_MAX_TOPK];
-          bool live[MF_MAX_TOPK];
+      const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
+      const uint32_t my_expert = lane < K ? s_idx[tok * K + lane] : E;
+      w_lane = lane < K ? s_w[tok * K + lane] : 0.0f;
+      const unsigned long long live = __ballot(my_expert < E);
+      uint32_t c_unit = wv, c_slot = 0;  // the (unit, slot) at hand
+      float acc = 0.0f;
+      auto take = [&](const Chunk<BITS>& c) __attribute__((always_inline)) {
+        if (c_slot == 0) acc = Fs ? s_h1[(c_unit << rpw_log2) + rloc] : 0.0f;
+        const XSlice<BITS> xs =
+            load_xslice_lds<BITS>(reinterpret_cast<const uint4*>(s_acts), s_asum, 0, n_asl, c_slot * spl + (lane_in ? sub : 0u));
+        float part = __builtin_fmaf(c.s, codes_dot<BITS>(c.codes, xs), 0.0f);  // the one step of row_partial
+        part = __builtin_fmaf(c.b, xs.sum, part);
+        const float v = group_sum(lane_in ? part : 0.0f, static_cast<int>(lpr));
+        // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first); sums in rank order
+        const float wgt = readlane_f(w_lane, static_cast<int>(c_slot));
+        if ((live >> c_slot) & 1ull) acc = acc + wgt * (maple ? round_bf16(v) : v);
+        if (++c_slot == K) {
+          const uint32_t row = ((u_first + c_unit) << rpw_log2) + rloc;
+          if (sub == 0 && row < D) store_row(row, acc, failed);
+          c_slot = 0;
+          c_unit += kFusedWaves;
+        }
+      };
+      uint32_t n = 0;
+      for (; n + 2 * kRing <= n_mine; n += kRing) {
 #pragma unroll
-          for (uint32_t k = 0; k < MF_MAX_TOPK; ++k) {
-            live[k] = k < K && s_idx[tok * K + (k < K ? k : 0)] < E;
-            vk[k] = s_v[(ul * K + (k < K ? k : 0)) * kWave + rr];
-          }
-          float acc = Fs ? s_h1[round * rows_per_round + threadIdx.x] : 0.0f;
-#pragma unroll
-          for (uint32_t k = 0; k < MF_MAX_TOPK; ++k)
-            if (live[k]) acc = acc + vk[k];
-          const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
-          const uint16_t yb = failed ? static_cast<uint16_t>(0x7FC0u) : f_to_bf16(acc);
-          a.y[o] = yb;
-          if (a.hidden && !failed) {  // residual_add_fp16, utility.metal:83-92
-            uint16_t hv = a.hidden[o];
-            if constexpr (NORM) {  // the residual add in front of the norm, made here for good
-              if (a.delta) hv = f_to_bf16(bf16_to_f(hv) + bf16_to_f(a.delta[o]));
-            }
-            a.hidden[o] = f_to_bf16(bf16_to_f(hv) + bf16_to_f(yb));
-          }
+        for (int i = 0; i < kRing; ++i) {
+          take(ring[i]);
+          fetch_unit(ring[i]);
         }
       }
-      // The next round (or token) overwrites s_v.  Behind the last round nothing is left to protect, and a
-      // barrier there only makes every wave wait for the acknowledgement of the stores of y: the one-token
-      // instances leave it out.  (With the token count an argument the same condition, or a barrier that
-      // waits for LDS operations only, made the launch slower: the large 2-bit layer at 4 rows 92 -> 111 us.)
-      if (!(kOneToken && round + 1 == rounds)) __syncthreads();
+      for (; n < n_mine; ++n) {
+        take(ring[0]);
+        ring[0] = ring[1];
+        ring[1] = ring[2];
+        ring[2] = ring[3];
+        if (n + kRing < n_mine) fetch_unit(ring[3]);
+      }
+    } else {
+      for (uint32_t round = 0; round < rounds; ++round) {
+        const uint32_t unit = (round * c_wgs + wl) * ub + unit_local;
+        if (unit_local < ub && unit < rg_per_tok) {
+          const uint32_t row = (unit << rpw_log2) + rloc;
+          const uint32_t pair = tok * K + slot;
+          const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[pair]);
+          float part = 0.0f;
+          if (row < D && expert < E) {
+            const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
+            part = row_partial<BITS>(blob + a.off.down_w + row * rb,
+                                     reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng,
+                                     reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng,
+                                     reinterpret_cast<const uint16_t*>(s_acts) + slot * F, F, sub, lpr, round == 0, ring[0]);
+          }
+          const float v = group_sum(part, static_cast<int>(lpr));
+          // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first)
+          if (sub == 0) s_v[wv * kWave + rloc] = s_w[pair] * (maple ? round_bf16(v) : v);
+        }
+        __syncthreads();
+        if (threadIdx.x < rows_per_round) {
+          const uint32_t ul = threadIdx.x >> rpw_log2, rr = threadIdx.x & (rpw - 1);
+          const uint32_t row = (((round * c_wgs + wl) * ub + ul) << rpw_log2) + rr;
+          if (row < D) {
+            // the K weighted values first (independent LDS reads: one round of latency, not K),
+            // then the sum in rank order, residual first
+            float vk[MF_MAX_TOPK];
+            bool live[MF_MAX_TOPK];
+#pragma unroll
+            for (uint32_t k = 0; k < MF_MAX_TOPK; ++k) {
+              live[k] = k < K && s_idx[tok * K + (k < K ? k : 0)] < E;
+              vk[k] = s_v[(ul * K + (k < K ? k : 0)) * kWave + rr];
+            }
+            float acc = Fs ? s_h1[round * rows_per_round + threadIdx.x] : 0.0f;
+#pragma unroll
+            for (uint32_t k = 0; k < MF_MAX_TOPK; ++k)
+              if (live[k]) acc = acc + vk[k];
+            store_row(row, acc, *s_fail != 0u);  // a wait gave up: no result, and hidden stays as it is
+          }
+        }
+        // The next round overwrites s_v.  Behind the last round nothing is left to protect, and a barrier there only
+        // makes every wave wait for the acknowledgement of the stores of y.
+        if (round + 1 < rounds) __syncthreads();
+      }
     }
   }
   if constexpr (!S::kGiven) {
@@ -929,15 +1057,44 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   trace_mark(a, 6);
 }
 
+// Host side: how a launch divides its work.
+static uint32_t fused_epl(const mf_moe_config& c) { return c.bits == MF_BITS_4 ? 32 : 64; }
+
+static uint32_t fused_b_per_wg(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
+  return fused_b_per_wg(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
+}
+static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
+  return fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
+}
+
+static FusedGeo fused_geo(const mf_moe_config& c, uint32_t num_cu, uint32_t t, const FusedSplit& sp) {
+  const uint32_t epl = fused_epl(c), sepl = c.shared_bits == MF_BITS_4 ? 32 : 64;
+  FusedGeo g{};
+  g.b_per_wg = fused_b_per_wg(c, num_cu, t);
+  g.c_wgs = sp.wgs;
+  g.c_units = sp.units;
+  g.c_rounds = sp.rounds;
+  g.lpr_d = static_cast<uint8_t>(lanes_per_row_log2_dev(c.d, epl));
+  g.lpr_f = static_cast<uint8_t>(lanes_per_row_log2_dev(c.f, epl));
+  g.lpr_sd = static_cast<uint8_t>(c.shared_f ? lanes_per_row_log2_dev(c.d, sepl) : 0);
+  g.lpr_sf = static_cast<uint8_t>(c.shared_f ? lanes_per_row_log2_dev(c.shared_f, sepl) : 0);
+  const uint32_t rpw_d = 64u >> g.lpr_d, rpw_f = 64u >> g.lpr_f, rpw_sd = 64u >> g.lpr_sd;
+  g.E = make_fastdiv(c.num_experts);
+  g.n_sl = make_fastdiv(c.d / epl);
+  g.rgf = make_fastdiv((c.f + rpw_d - 1) / rpw_d);
+  g.K = make_fastdiv(c.top_k);
+  g.srg = make_fastdiv((c.shared_f + rpw_sd - 1) / rpw_sd);
+  g.c_wgs_div = make_fastdiv(sp.wgs);
+  g.rpr = make_fastdiv(sp.units * rpw_f);
+  return g;
+}
+
 // words of the LDS staging area: a chunk of router logits in stage A, the (gate, up) sums of a
 // workgroup's run of routed rows in stage B
+// (and, in stage C's units form, the sums of the activation slices)
 static uint32_t fused_stage_words(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
-  const uint32_t epl = c.bits == MF_BITS_4 ? 32 : 64;
-  const uint32_t rpw = 64u >> lanes_per_row_log2_dev(c.d, epl);
-  const uint32_t rgf = (c.f + rpw - 1) / rpw;
-  uint32_t per_wg = (t * c.top_k * rgf + num_cu - 1) / num_cu;
-  per_wg = (per_wg + kFusedWaves - 1) / kFusedWaves * kFusedWaves;
-  const uint32_t words = 2 * per_wg * rpw;
+  const uint32_t epl = fused_epl(c), rpw = 64u >> lanes_per_row_log2_dev(c.d, epl);
+  const uint32_t words = std::max(2 * fused_b_per_wg(c, num_cu, t) * rpw, c.top_k * (c.f / epl));
   return words < 64 ? 64 : (words + 3) & ~3u;
 }
 // words of the x slices of the routed rows (permuted pairs + sum per slice)
@@ -972,13 +1129,11 @@ bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void*
                      (c.bits == MF_BITS_TERNARY && (!c.shared_f || c.shared_bits == MF_BITS_4));
   if (!combo || c.d % 8 != 0) return false;
   if (fused_lds_base(c, static_cast<uint32_t>(h.ctx->num_cu), t) > kFusedLdsLimit) return false;
-  {  // rows of one token a workgroup owns must fit the h1 array
-    const uint32_t epl = c.bits == MF_BITS_4 ? 32 : 64;
-    const uint32_t rpw = 64u >> lanes_per_row_log2_dev(c.f, epl);
-    const uint32_t rg = (c.d + rpw - 1) / rpw, ub = kFusedWaves / c.top_k;
-    const uint32_t G = static_cast<uint32_t>(h.ctx->num_cu);
-    const uint32_t rounds = (rg + G * ub - 1) / (G * ub);
-    if (rounds * ub * rpw > kMaxH1) return false;
+  {  // rows of one token a workgroup owns must fit the h1 array, and every token needs a workgroup
+    const uint32_t num_cu = static_cast<uint32_t>(h.ctx->num_cu);
+    if (num_cu < t) return false;
+    const FusedSplit sp = fused_split(c, num_cu, t);
+    if (sp.rounds * sp.units * (64u >> lanes_per_row_log2_dev(c.f, fused_epl(c))) > kMaxH1) return false;
   }
   const uint32_t offs = w.offsets.gate_w | w.offsets.up_w | w.offsets.down_w;
   if (!aligned16(w.expert_base) || w.expert_stride % 16 || offs % 16) return false;
@@ -1004,6 +1159,25 @@ bool fused_norm_supported(const mf_moe& h, const mf_moe_layer_weights& w, const 
   if (!fused_supported(h, w, hidden, y, hidden, t)) return false;  // (x stands in as an aligned pointer)
   const uint32_t num_cu = static_cast<uint32_t>(h.ctx->num_cu);
   return fused_lds_bytes(c, num_cu, t) + 16 + static_cast<size_t>(t) * c.d * 2 <= kFusedLdsLimit;
+}
+
+// One instance in the form (rows or units of stage C) its shape takes; an instance with every dimension literal exists
+// in one form only.
+template <int BITS, int SBITS, class S, bool NORM>
+static hipError_t launch_instance(bool by_units, dim3 grid, dim3 block, size_t lds, hipStream_t s, const FusedArgs& a) {
+  auto go = [&](auto units) {
+    constexpr auto kKernel = fused_decode_kernel<BITS, SBITS, S, NORM, decltype(units)::value>;
+    const hipError_t e = allow_lds<kKernel>(lds, kFusedLdsLimit);
+    if (e != hipSuccess) return e;
+    kKernel<<<grid, block, lds, s>>>(a);
+    return hipGetLastError();
+  };
+  if constexpr (S::kStatic) {
+    return go(std::bool_constant<fused_split(Fmt<BITS>::kElemsPer16B, S::D, S::F, S::K, 1, kStaticWgs).by_units>{});
+  } else {
+    if (by_units) return go(std::true_type{});
+    return go(std::false_type{});
+  }
 }
 
 hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_layer_weights& w,
@@ -1055,12 +1229,11 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
     a.xn_off = static_cast<uint32_t>((lds + 15) & ~size_t(15));
     lds = a.xn_off + static_cast<size_t>(t) * c.d * 2;
   }
-#define MF_FUSED(B, SB, SHAPE)                                                                 \
-  do {                                                                                         \
-    const hipError_t e = allow_lds<fused_decode_kernel<B, SB, SHAPE>>(lds, kFusedLdsLimit);    \
-    if (e != hipSuccess) return e;                                                             \
-    fused_decode_kernel<B, SB, SHAPE><<<grid, block, lds, s>>>(a);                             \
-  } while (0)
+  const FusedSplit sp = fused_split(c, num_cu, t);
+  a.g = fused_geo(c, num_cu, t, sp);
+#define MF_FUSED(B, SB, SHAPE) return launch_instance<B, SB, SHAPE, false>(sp.by_units, grid, block, lds, s, a)
+#define MF_FUSED_N(B, SB, SHAPE) return launch_instance<B, SB, SHAPE, true>(sp.by_units, grid, block, lds, s, a)
+  const bool one = t == 1 && num_cu == kStaticWgs;  // the instances with every dimension literal
   // Shape-specialised instances: a layer shape's dimensions as literals with the token rows read from the
   // arguments (Tn), and the one-token launch with T = 1 as a literal as well (T1: it drops the code of the
   // token loop; Qwen shape 12.3 us against 13.5 us through Tn).  Which literal buys what, Qwen shape, 4
@@ -1101,22 +1274,14 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   const bool qwen_dims = c.bits == MF_BITS_4 && c.shared_bits == MF_BITS_4 && c.d == 2048 && c.f == 512 &&
                          c.num_experts == 256 && c.top_k == 8 && c.shared_f == 512;
   const bool lit = !h.generic_shape;  // shape instances allowed
-#define MF_FUSED_N(B, SB, SHAPE)                                                               \
-  do {                                                                                         \
-    const hipError_t e = allow_lds<fused_decode_kernel<B, SB, SHAPE, true>>(lds, kFusedLdsLimit); \
-    if (e != hipSuccess) return e;                                                             \
-    fused_decode_kernel<B, SB, SHAPE, true><<<grid, block, lds, s>>>(a);                       \
-  } while (0)
   if (norm) {  // x made inside the launch: the Qwen shape's instances and the ones that read every dimension
-    if (lit && qwen && t == 1 && !c.maple_rounding && no_limit && a.xprep) MF_FUSED_N(kBits4, kBits4, QwenT1);
+    if (lit && qwen && one && !c.maple_rounding && no_limit && a.xprep) MF_FUSED_N(kBits4, kBits4, QwenT1);
     else if (lit && qwen) MF_FUSED_N(kBits4, kBits4, QwenTn);
     else if (c.bits == MF_BITS_4) MF_FUSED_N(kBits4, kBits4, RuntimeShape);
     else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits2, RuntimeShape);
     else if (c.bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits4, RuntimeShape);
     else MF_FUSED_N(kBitsTernary, kBits4, RuntimeShape);
-    return hipGetLastError();
   }
-#undef MF_FUSED_N
   if (!w.router_w) {  // caller-given routing
     if (!lit) {
       if (c.bits == MF_BITS_4) MF_FUSED(kBits4, kBits4, Given);
@@ -1124,8 +1289,8 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
       else if (c.bits == MF_BITS_2) MF_FUSED(kBits2, kBits4, Given);
       else MF_FUSED(kBitsTernary, kBits4, Given);
     }
-    else if (big2 && t == 1) MF_FUSED(kBits2, kBits4, Big2T1Given);
-    else if (qwen_dims && t == 1 && !c.maple_rounding && no_limit && a.xprep) MF_FUSED(kBits4, kBits4, QwenT1Given);
+    else if (big2 && one) MF_FUSED(kBits2, kBits4, Big2T1Given);
+    else if (qwen_dims && one && !c.maple_rounding && no_limit && a.xprep) MF_FUSED(kBits4, kBits4, QwenT1Given);
     else if (qwen_dims) MF_FUSED(kBits4, kBits4, QwenTnGiven);
 #define MF_SHAPES_PICK_GIVEN
 #include "fused_shapes.inc"
@@ -1139,14 +1304,14 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
     else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED(kBits2, kBits2, RuntimeShape);
     else if (c.bits == MF_BITS_2) MF_FUSED(kBits2, kBits4, RuntimeShape);
     else MF_FUSED(kBitsTernary, kBits4, RuntimeShape);
-  } else if (qwen && t == 1 && !c.maple_rounding && no_limit && a.xprep) MF_FUSED(kBits4, kBits4, QwenT1);
+  } else if (qwen && one && !c.maple_rounding && no_limit && a.xprep) MF_FUSED(kBits4, kBits4, QwenT1);
   else if (qwen) MF_FUSED(kBits4, kBits4, QwenTn);
-  else if (big2 && t == 1 && !c.maple_rounding && a.xprep) MF_FUSED(kBits2, kBits4, Big2T1);
+  else if (big2 && one && !c.maple_rounding && a.xprep) MF_FUSED(kBits2, kBits4, Big2T1);
   else if (big2) MF_FUSED(kBits2, kBits4, Big2Tn);
-  else if (tern && t == 1 && c.router_mode == MF_ROUTER_FULL_SOFTMAX && c.maple_rounding && no_limit && a.xprep)
+  else if (tern && one && c.router_mode == MF_ROUTER_FULL_SOFTMAX && c.maple_rounding && no_limit && a.xprep)
     MF_FUSED(kBitsTernary, kBits4, TernT1);
   else if (tern) MF_FUSED(kBitsTernary, kBits4, TernTn);
-  else if (maple && t == 1 && c.router_mode == MF_ROUTER_FULL_SOFTMAX && c.maple_rounding && no_limit && a.xprep)
+  else if (maple && one && c.router_mode == MF_ROUTER_FULL_SOFTMAX && c.maple_rounding && no_limit && a.xprep)
     MF_FUSED(kBitsTernary, kBits4, MapleT1);
   else if (maple) MF_FUSED(kBitsTernary, kBits4, MapleTn);
 #define MF_SHAPES_PICK_OWN
@@ -1158,7 +1323,7 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   else if (c.bits == MF_BITS_2) MF_FUSED(kBits2, kBits4, RuntimeShape);
   else MF_FUSED(kBitsTernary, kBits4, RuntimeShape);
 #undef MF_FUSED
-  return hipGetLastError();
+#undef MF_FUSED_N
 }
 
 }  // namespace mf
