@@ -63,9 +63,23 @@ constexpr uint32_t kRankCountLimit = 1u << 18;  // T * E * E up to which the top
 constexpr uint32_t kRankWords = 2048;      // ... and T * E it may have then
 constexpr uint32_t kMaxH1 = 2048;          // output rows of one token a workgroup may own
 
+// A lane's step of a row: codes and the table entries of its group as they come from memory.  The entries become
+// numbers where they are used (scale(), bias()), behind an empty asm statement: converted next to their load they
+// would be waited for there, in front of everything that was to run while they are on their way.
 template <int BITS> struct Chunk {
   uint4 codes;
-  float s, b;
+  uint32_t sraw, braw;
+  __device__ __forceinline__ float scale() const {
+    uint32_t r = sraw;
+    asm volatile("" : "+v"(r));
+    return __uint_as_float(r << 16);
+  }
+  __device__ __forceinline__ float bias() const {
+    if constexpr (BITS == kBitsTernary) return -scale();
+    uint32_t r = braw;
+    asm volatile("" : "+v"(r));
+    return __uint_as_float(r << 16);
+  }
 };
 
 template <int BITS>
@@ -73,7 +87,9 @@ __device__ __forceinline__ Chunk<BITS> load_chunk(const uint8_t* wrow, const uin
                                                   const uint16_t* brow, uint32_t e0) {
   Chunk<BITS> c;
   c.codes = load_codes16<true>(wrow + static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
-  load_scale_bias<BITS>(srow, brow, e0, c.s, c.b);
+  c.sraw = srow[e0 / kGroup];
+  if constexpr (BITS == kBitsTernary) c.braw = 0;
+  else c.braw = brow[e0 / kGroup];
   return c;
 }
 
@@ -89,7 +105,7 @@ __device__ __forceinline__ float row_partial(const uint8_t* wrow, const uint16_t
   for (uint32_t e0 = sub * EPL; e0 < N; e0 += lpr * EPL) {
     // plain scalars, not a struct select: the prefetched chunk must stay in registers
     uint4 codes = first.codes;
-    float s = first.s, b = first.b;
+    float s = first.scale(), b = first.bias();
     if (!(have_first && e0 == sub * EPL)) {
       codes = load_codes16<true>(wrow + static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
       load_scale_bias<BITS>(srow, brow, e0, s, b);
@@ -117,10 +133,10 @@ __device__ __forceinline__ void gate_up_partial(const uint8_t* gw, const uint16_
     issue_fence();
     const XSlice<BITS> xs = make_xslice<BITS>(xr);
     const float gd = codes_dot<BITS>(g.codes, xs), ud = codes_dot<BITS>(u.codes, xs);
-    ga = __builtin_fmaf(g.s, gd, ga);
-    ga = __builtin_fmaf(g.b, xs.sum, ga);
-    ua = __builtin_fmaf(u.s, ud, ua);
-    ua = __builtin_fmaf(u.b, xs.sum, ua);
+    ga = __builtin_fmaf(g.scale(), gd, ga);
+    ga = __builtin_fmaf(g.bias(), xs.sum, ga);
+    ua = __builtin_fmaf(u.scale(), ud, ua);
+    ua = __builtin_fmaf(u.bias(), xs.sum, ua);
   }
 }
 
@@ -173,6 +189,15 @@ struct FusedGeo {
   uint8_t lpr_d, lpr_f, lpr_sd, lpr_sf;  // log2 of the lanes per row: rows of D and F (routed), of D and Fs (shared)
   FastDiv E, n_sl, rgf, K, srg, c_wgs_div, rpr;
 };
+
+// an activation slice out of its raw blocks in that layout
+template <int BITS>
+__device__ __forceinline__ XSlice<BITS> load_act_slice(const uint4* blocks, uint32_t ld, uint32_t sl) {
+  XRaw<BITS> r;
+#pragma unroll
+  for (int q = 0; q < Fmt<BITS>::kElemsPer16B / 8; ++q) r.q[q] = blocks[q * ld + sl];
+  return make_xslice<BITS>(r);
+}
 
 struct FusedArgs {
   const uint16_t* router_w;
@@ -329,7 +354,11 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   float* s_lg = reinterpret_cast<float*>(dyn);                          // [MF_MAX_TOKENS][E]
   uint32_t* s_sact = reinterpret_cast<uint32_t*>(dyn + MF_MAX_TOKENS * E * 4);  // [(Fs+4)/2]
   uint32_t* s_acts = s_sact + (((Fs + 4) / 2 + 3) & ~3u);               // [K*F/2], 16-byte aligned
-  uint32_t* s_stage = s_acts + ((K * F / 2 + 3) & ~3u);                 // chunk staging, a.stage_words
+  // the routed activations as 16-byte blocks in the order of the x slices: block q of slice sl at q * act_ld + sl (an
+  // odd stride: the lanes that write a slice's blocks and those that read one block of many slices both spread over
+  // the banks; row by row the readers' slices lay 64 or 128 bytes apart, four or eight of 16 lanes on one bank)
+  const uint32_t act_ld = (K * F / Fmt<BITS>::kElemsPer16B) | 1u;
+  uint32_t* s_stage = s_acts + Fmt<BITS>::kElemsPer16B / 8 * 4 * act_ld;  // chunk staging, a.stage_words
   const uint32_t sact_stride = Fs + 4;  // words per token in t_sact
 
   const uint32_t lane = threadIdx.x & 63;
@@ -653,6 +682,104 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   }
   trace_mark(a, 3);
 
+  // ------------------------------------------------------------- what stage C will read
+  // The workgroups are split among the tokens: c_wgs of them own the output rows of one token, so a workgroup gathers
+  // one token's activations (T tokens' by every workgroup one after the other: T waits, and T times the bytes past
+  // every cache).  A unit is rpw output rows of the token.
+  const uint32_t lpr_log2 = S::F != kDyn ? lanes_per_row_log2_dev(F, Fmt<BITS>::kElemsPer16B) : a.g.lpr_f;
+  const uint32_t lpr = 1u << lpr_log2, rpw_log2 = 6 - lpr_log2, rpw = 1u << rpw_log2;
+  const uint32_t rg_per_tok = (D + rpw - 1) >> rpw_log2;  // units of a token
+  const uint32_t c_wgs = S::kStatic ? kSplit.wgs : a.g.c_wgs;
+  const uint32_t tok = S::T == 1 ? 0u : fdiv(wg, a.g.c_wgs_div), wl = wg - tok * c_wgs;
+  const uint32_t sub = lane & (lpr - 1), rloc = lane >> lpr_log2;
+  const uint32_t ng = F / kGroup;
+  const size_t rb = static_cast<size_t>(F) * Store<BITS>::kBits / 8;
+  const uint32_t ub = S::kStatic ? kSplit.units : a.g.c_units;
+  // The output row behind index i of the workgroup's rows (LDS order): rows form -- round by round, ub units each;
+  // units form -- one run of units.
+  const uint32_t rounds = UNITS ? 1u : S::kStatic ? kSplit.rounds : a.g.c_rounds, rows_per_round = ub << rpw_log2;
+  auto row_at = [&](uint32_t i) __attribute__((always_inline)) {
+    if constexpr (UNITS) return (wl * ub << rpw_log2) + i;
+    const uint32_t round = rounds == 1 ? 0u : fdiv(i, a.g.rpr), in_round = i - round * rows_per_round;
+    return ((round * c_wgs + wl) * ub << rpw_log2) + in_round;
+  };
+  // shared-expert down rows: srpw rows per wave step
+  const uint32_t slpr_log2 = !Fs ? 0u : S::Fs != kDyn ? lanes_per_row_log2_dev(Fs, Fmt<SBITS>::kElemsPer16B) : a.g.lpr_sf;
+  const uint32_t slpr = 1u << slpr_log2, srpw = 64u >> slpr_log2;
+
+  // What the router decided is all a down row needs to be requested: the first codes leave before anything is
+  // waited for.  Rows form: slot wv % K of unit wv / K of the first round.  Units form: a wave walks
+  // (unit, slot) pairs, slots fastest; four of them are in flight.
+  constexpr uint32_t kEPLF = Fmt<BITS>::kElemsPer16B;
+  constexpr int kRing = UNITS ? 4 : 1;
+  Chunk<BITS> ring[kRing];
+  const uint32_t e0 = sub * kEPLF;
+  const bool lane_in = e0 < F;
+  const uint32_t e0c = lane_in ? e0 : 0u;
+  // rows form
+  const uint32_t unit_local = S::K != kDyn ? wv / K : fdiv(wv, a.g.K), slot = wv - unit_local * K;
+  // units form: the slots' blobs and weights, a slot per lane
+  uint32_t base_lo = 0, base_hi = 0;
+  float w_lane = 0.0f;
+  uint32_t f_unit = wv, f_slot = 0;               // the next (unit, slot) to request
+  const uint32_t u_first = wl * ub, u_n = u_first < rg_per_tok ? (rg_per_tok - u_first < ub ? rg_per_tok - u_first : ub) : 0;
+  const uint32_t n_mine = UNITS ? (wv < u_n ? (u_n - wv + kFusedWaves - 1) / kFusedWaves : 0u) * K : 0u;
+  auto request = [&](const uint8_t* blob, uint32_t row) __attribute__((always_inline)) {
+    const uint32_t rc = row < D ? row : 0u;
+    return load_chunk<BITS>(blob + a.off.down_w + rc * rb,
+                            reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + static_cast<size_t>(rc) * ng,
+                            reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + static_cast<size_t>(rc) * ng, e0c);
+  };
+  auto fetch_unit = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
+    const uint64_t base = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_hi), f_slot))) << 32) |
+                          static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_lo), f_slot));
+    c = request(reinterpret_cast<const uint8_t*>(base), ((u_first + (f_unit < u_n ? f_unit : 0u)) << rpw_log2) + rloc);
+    if (++f_slot == K) {
+      f_slot = 0;
+      f_unit += kFusedWaves;
+    }
+  };
+  auto fetch_first = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
+    const uint32_t unit = wl * ub + unit_local;
+    const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[tok * K + slot]);
+    c = request(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride, (unit << rpw_log2) + rloc);
+  };
+  // first shared-expert down chunk of a wave
+  const uint32_t sng = Fs ? Fs / kGroup : 0;
+  const size_t srb = static_cast<size_t>(Fs) * Store<SBITS>::kBits / 8;
+  const uint32_t n_slots = !Fs ? 0u : UNITS ? u_n << rpw_log2 : rounds * rows_per_round;
+  const uint32_t ssub = lane & (slpr - 1);
+  Chunk<SBITS> spre{};
+  bool have_spre = false;
+  // When the requests go out.  Rows form: behind stage B's first (and mostly only) ones, so that the codes are here when
+  // the activations are and no poll for activations has to wait for them -- a wave's loads return in order (small 4-bit
+  // layer 12.4 -> 11.5 us, ternary layer 12.6 -> 12.3).  Units form: behind stage B, whose own stream of rows they
+  // would sit in (Qwen shape, five tokens: 26.4 us, with the early requests 28.9).
+  auto request_down_rows = [&]() __attribute__((always_inline)) {
+    if constexpr (UNITS) {
+      const uint32_t expert = lane < K ? s_idx[tok * K + lane] : E;
+      const uint64_t base = reinterpret_cast<uint64_t>(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride);
+      base_lo = static_cast<uint32_t>(base);
+      base_hi = static_cast<uint32_t>(base >> 32);
+      if (n_mine) {
+  #pragma unroll
+        for (int i = 0; i < kRing; ++i) fetch_unit(ring[i]);
+      }
+    } else if (S::kStatic || unit_local < ub) {  // (literal shapes: no branch around the loads)
+      fetch_first(ring[0]);
+    }
+    if (Fs) {
+      const uint32_t i = wv * srpw + (lane >> slpr_log2), row = row_at(i);
+      if (i < n_slots && row < D && ssub * Fmt<SBITS>::kElemsPer16B < Fs) {
+        spre = load_chunk<SBITS>(static_cast<const uint8_t*>(a.sd.weights) + row * srb,
+                                 a.sd.scales + static_cast<size_t>(row) * sng,
+                                 a.sd.biases + static_cast<size_t>(row) * sng,
+                                 ssub * Fmt<SBITS>::kElemsPer16B);
+        have_spre = true;
+      }
+    }
+  };
+
   // ------------------------------------------------------------- stage B
   // Every workgroup takes a run of consecutive units (rpw rows of one routed slot), its waves
   // take them in turn; gate and up sums meet in LDS, the first threads turn them into
@@ -704,10 +831,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
                                     : load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(c.tok) * D + c.e0);
       const float gd = codes_dot<BITS>(c.g.codes, xs), ud = codes_dot<BITS>(c.u.codes, xs);
       if (c.ok) {
-        ga = __builtin_fmaf(c.g.s, gd, ga);
-        ga = __builtin_fmaf(c.g.b, xs.sum, ga);
-        ua = __builtin_fmaf(c.u.s, ud, ua);
-        ua = __builtin_fmaf(c.u.b, xs.sum, ua);
+        ga = __builtin_fmaf(c.g.scale(), gd, ga);
+        ga = __builtin_fmaf(c.g.bias(), xs.sum, ga);
+        ua = __builtin_fmaf(c.u.scale(), ud, ua);
+        ua = __builtin_fmaf(c.u.bias(), xs.sum, ua);
       }
       if (step + 1 == steps) {  // the row is complete
         const float g = group_sum(ga, static_cast<int>(lpr));
@@ -721,9 +848,11 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       }
     };
     uint32_t item = first + wv, step = 0;
+    Step cur{};
+    if (S::kStatic || item < last) fetch(item < n_items ? item : 0u, 0, cur);  // (literal shapes: no branch around the loads)
+    if constexpr (!UNITS) request_down_rows();
+    issue_fence();
     if (item < last) {
-      Step cur;
-      fetch(item, 0, cur);
       for (;;) {
         uint32_t nitem = item, nstep = step + 1;
         if (nstep == steps) {
@@ -764,97 +893,8 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   }
 
   // ------------------------------------------------------------- stage C
-  // The workgroups are split among the tokens: c_wgs of them own the output rows of one token, so a workgroup gathers
-  // one token's activations (T tokens' by every workgroup one after the other: T waits, and T times the bytes past
-  // every cache).  A unit is rpw output rows of the token.
-  const uint32_t lpr_log2 = S::F != kDyn ? lanes_per_row_log2_dev(F, Fmt<BITS>::kElemsPer16B) : a.g.lpr_f;
-  const uint32_t lpr = 1u << lpr_log2, rpw_log2 = 6 - lpr_log2, rpw = 1u << rpw_log2;
-  const uint32_t rg_per_tok = (D + rpw - 1) >> rpw_log2;  // units of a token
-  const uint32_t c_wgs = S::kStatic ? kSplit.wgs : a.g.c_wgs;
-  const uint32_t tok = S::T == 1 ? 0u : fdiv(wg, a.g.c_wgs_div), wl = wg - tok * c_wgs;
-  const uint32_t sub = lane & (lpr - 1), rloc = lane >> lpr_log2;
-  const uint32_t ng = F / kGroup;
-  const size_t rb = static_cast<size_t>(F) * Store<BITS>::kBits / 8;
-  const uint32_t ub = S::kStatic ? kSplit.units : a.g.c_units;
-  // The output row behind index i of the workgroup's rows (LDS order): rows form -- round by round, ub units each;
-  // units form -- one run of units.
-  const uint32_t rounds = UNITS ? 1u : S::kStatic ? kSplit.rounds : a.g.c_rounds, rows_per_round = ub << rpw_log2;
-  auto row_at = [&](uint32_t i) __attribute__((always_inline)) {
-    if constexpr (UNITS) return (wl * ub << rpw_log2) + i;
-    const uint32_t round = rounds == 1 ? 0u : fdiv(i, a.g.rpr), in_round = i - round * rows_per_round;
-    return ((round * c_wgs + wl) * ub << rpw_log2) + in_round;
-  };
   if (tok < T) {
-    // shared-expert down rows: srpw rows per wave step
-    const uint32_t slpr_log2 = !Fs ? 0u : S::Fs != kDyn ? lanes_per_row_log2_dev(Fs, Fmt<SBITS>::kElemsPer16B) : a.g.lpr_sf;
-    const uint32_t slpr = 1u << slpr_log2, srpw = 64u >> slpr_log2;
-
-    // What the router decided is all a down row needs to be requested: the first codes leave before anything is
-    // waited for.  Rows form: slot wv % K of unit wv / K of the first round.  Units form: a wave walks
-    // (unit, slot) pairs, slots fastest; four of them are in flight.
-    constexpr uint32_t kEPLF = Fmt<BITS>::kElemsPer16B;
-    constexpr int kRing = UNITS ? 4 : 1;
-    Chunk<BITS> ring[kRing];
-    const uint32_t e0 = sub * kEPLF;
-    const bool lane_in = e0 < F;
-    const uint32_t e0c = lane_in ? e0 : 0u;
-    // rows form
-    const uint32_t unit_local = S::K != kDyn ? wv / K : fdiv(wv, a.g.K), slot = wv - unit_local * K;
-    // units form: the slots' blobs and weights, a slot per lane
-    uint32_t base_lo = 0, base_hi = 0;
-    float w_lane = 0.0f;
-    uint32_t f_unit = wv, f_slot = 0;               // the next (unit, slot) to request
-    const uint32_t u_first = wl * ub, u_n = u_first < rg_per_tok ? (rg_per_tok - u_first < ub ? rg_per_tok - u_first : ub) : 0;
-    const uint32_t n_mine = UNITS ? (wv < u_n ? (u_n - wv + kFusedWaves - 1) / kFusedWaves : 0u) * K : 0u;
-    auto request = [&](const uint8_t* blob, uint32_t row) __attribute__((always_inline)) {
-      const uint32_t rc = row < D ? row : 0u;
-      return load_chunk<BITS>(blob + a.off.down_w + rc * rb,
-                              reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + static_cast<size_t>(rc) * ng,
-                              reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + static_cast<size_t>(rc) * ng, e0c);
-    };
-    auto fetch_unit = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
-      const uint64_t base = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_hi), f_slot))) << 32) |
-                            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_lo), f_slot));
-      c = request(reinterpret_cast<const uint8_t*>(base), ((u_first + (f_unit < u_n ? f_unit : 0u)) << rpw_log2) + rloc);
-      if (++f_slot == K) {
-        f_slot = 0;
-        f_unit += kFusedWaves;
-      }
-    };
-    auto fetch_first = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
-      const uint32_t unit = wl * ub + unit_local;
-      const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[tok * K + slot]);
-      c = request(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride, (unit << rpw_log2) + rloc);
-    };
-    if constexpr (UNITS) {
-      const uint32_t expert = lane < K ? s_idx[tok * K + lane] : E;
-      const uint64_t base = reinterpret_cast<uint64_t>(a.expert_base + static_cast<size_t>(expert < E ? expert : 0u) * a.expert_stride);
-      base_lo = static_cast<uint32_t>(base);
-      base_hi = static_cast<uint32_t>(base >> 32);
-      if (n_mine) {
-#pragma unroll
-        for (int i = 0; i < kRing; ++i) fetch_unit(ring[i]);
-      }
-    } else if (S::kStatic || unit_local < ub) {  // (literal shapes: no branch around the loads)
-      fetch_first(ring[0]);
-    }
-    // first shared-expert down chunk of this wave, requested before the wait as well
-    const uint32_t sng = Fs ? Fs / kGroup : 0;
-    const size_t srb = static_cast<size_t>(Fs) * Store<SBITS>::kBits / 8;
-    const uint32_t n_slots = !Fs ? 0u : UNITS ? u_n << rpw_log2 : rounds * rows_per_round;
-    const uint32_t ssub = lane & (slpr - 1);
-    Chunk<SBITS> spre{};
-    bool have_spre = false;
-    if (Fs) {
-      const uint32_t i = wv * srpw + (lane >> slpr_log2), row = row_at(i);
-      if (i < n_slots && row < D && ssub * Fmt<SBITS>::kElemsPer16B < Fs) {
-        spre = load_chunk<SBITS>(static_cast<const uint8_t*>(a.sd.weights) + row * srb,
-                                 a.sd.scales + static_cast<size_t>(row) * sng,
-                                 a.sd.biases + static_cast<size_t>(row) * sng,
-                                 ssub * Fmt<SBITS>::kElemsPer16B);
-        have_spre = true;
-      }
-    }
+    if constexpr (UNITS) request_down_rows();
     // Gather what other workgroups produced: the routed activations [K*F] and the shared
     // activations (+ gate) [Fs (+4)], 256 words per wave step, two steps in flight.
     // The shared activations were written in stage A, long ago: when the routed words fit the
@@ -886,16 +926,13 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
           }
           __builtin_amdgcn_s_sleep(1);
         }
-        if (in0) {
-          uint32_t* dst = i0 < n_a ? s_acts + i0 / 2 : s_sact + (i0 - n_a) / 2;
-          dst[0] = __builtin_amdgcn_perm(v0.y, v0.x, 0x05040100u);
-          dst[1] = __builtin_amdgcn_perm(v0.w, v0.z, 0x05040100u);
-        }
-        if (in1) {
-          uint32_t* dst = i1 < n_a ? s_acts + i1 / 2 : s_sact + (i1 - n_a) / 2;
-          dst[0] = __builtin_amdgcn_perm(v1.y, v1.x, 0x05040100u);
-          dst[1] = __builtin_amdgcn_perm(v1.w, v1.z, 0x05040100u);
-        }
+        auto put = [&](uint32_t i, const uint4& v) __attribute__((always_inline)) {  // four activations from element i on
+          uint32_t* dst = i < n_a ? s_acts + ((i % kEPLF / 8) * act_ld + i / kEPLF) * 4 + i % 8 / 2 : s_sact + (i - n_a) / 2;
+          *reinterpret_cast<uint2*>(dst) =
+              make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u));
+        };
+        if (in0) put(i0, v0);
+        if (in1) put(i1, v1);
       }
     };
     // gated shared output h1 of the output rows this workgroup owns; waves [0, nw) share the rows
@@ -956,11 +993,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       const uint32_t spl = F / kEPLF, n_asl = K * spl;
       float* s_asum = reinterpret_cast<float*>(s_stage);
       {
-        XSlice<BITS> xs{};
-        if (threadIdx.x < n_asl)
-          xs = load_xslice<BITS, kXAligned>(reinterpret_cast<const uint16_t*>(s_acts) + threadIdx.x * kEPLF);
-        __syncthreads();
-        if (threadIdx.x < n_asl) store_xslice_lds<BITS>(reinterpret_cast<uint4*>(s_acts), s_asum, 0, n_asl, threadIdx.x, xs);
+        if (threadIdx.x < n_asl) {  // a thread reads and writes the blocks of its own slice only
+          uint4* acts4 = reinterpret_cast<uint4*>(s_acts);
+          store_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, threadIdx.x, load_act_slice<BITS>(acts4, act_ld, threadIdx.x));
+        }
       }
       __syncthreads();
       const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
@@ -972,9 +1008,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       auto take = [&](const Chunk<BITS>& c) __attribute__((always_inline)) {
         if (c_slot == 0) acc = Fs ? s_h1[(c_unit << rpw_log2) + rloc] : 0.0f;
         const XSlice<BITS> xs =
-            load_xslice_lds<BITS>(reinterpret_cast<const uint4*>(s_acts), s_asum, 0, n_asl, c_slot * spl + (lane_in ? sub : 0u));
-        float part = __builtin_fmaf(c.s, codes_dot<BITS>(c.codes, xs), 0.0f);  // the one step of row_partial
-        part = __builtin_fmaf(c.b, xs.sum, part);
+            load_xslice_lds<BITS>(reinterpret_cast<const uint4*>(s_acts), s_asum, 0, act_ld, c_slot * spl + (lane_in ? sub : 0u));
+        float part = __builtin_fmaf(c.scale(), codes_dot<BITS>(c.codes, xs), 0.0f);  // the one step of row_partial
+        part = __builtin_fmaf(c.bias(), xs.sum, part);
         const float v = group_sum(lane_in ? part : 0.0f, static_cast<int>(lpr));
         // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first); sums in rank order
         const float wgt = readlane_f(w_lane, static_cast<int>(c_slot));
@@ -1011,10 +1047,16 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
           float part = 0.0f;
           if (row < D && expert < E) {
             const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-            part = row_partial<BITS>(blob + a.off.down_w + row * rb,
-                                     reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng,
-                                     reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng,
-                                     reinterpret_cast<const uint16_t*>(s_acts) + slot * F, F, sub, lpr, round == 0, ring[0]);
+            const uint8_t* wrow = blob + a.off.down_w + row * rb;
+            const uint16_t* srow = reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng;
+            const uint16_t* brow = reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng;
+            for (uint32_t e = e0; e < F; e += lpr * kEPLF) {  // the steps of row_partial
+              Chunk<BITS> c = ring[0];
+              if (!(round == 0 && e == e0)) c = load_chunk<BITS>(wrow, srow, brow, e);
+              const XSlice<BITS> xs = load_act_slice<BITS>(reinterpret_cast<const uint4*>(s_acts), act_ld, (slot * F + e) / kEPLF);
+              part = __builtin_fmaf(c.scale(), codes_dot<BITS>(c.codes, xs), part);
+              part = __builtin_fmaf(c.bias(), xs.sum, part);
+            }
           }
           const float v = group_sum(part, static_cast<int>(lpr));
           // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first)
@@ -1104,7 +1146,8 @@ static uint32_t fused_xprep_words(const mf_moe_config& c, uint32_t t) {
 }
 static size_t fused_lds_base(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
   const size_t sact_words = ((c.shared_f + 4) / 2 + 3) & ~size_t(3);
-  const size_t acts_words = (static_cast<size_t>(c.top_k) * c.f / 2 + 3) & ~size_t(3);
+  const uint32_t epl = fused_epl(c);
+  const size_t acts_words = static_cast<size_t>(epl / 8 * 4) * ((c.top_k * c.f / epl) | 1u);
   return 1024 + 4096 + kMaxH1 * 4 + kRankWords * 4 + static_cast<size_t>(MF_MAX_TOKENS) * c.num_experts * 4 +
          4 * (sact_words + acts_words + fused_stage_words(c, num_cu, t));
 }
