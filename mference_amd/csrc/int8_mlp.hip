@@ -33,6 +33,8 @@ __device__ __forceinline__ uint16_t q8_activation(float g, float u, bool silu) {
 // every kernel of this family.  Bound: a wave's life is one memory round trip plus its arithmetic.  Chunk by chunk
 // (gemv_q8_kernel) a 2816-element row is six round trips in a row; here the codes, tables and the first token's x of
 // the whole row leave together (CPL chunks per lane), and every further token reuses the codes.
+// (The codes become numbers inside the token loop: kept as fp32 they take 180 registers for a gate / up pair of 2816,
+// two waves to a SIMD, and 2112 rows are then a full round of waves plus a little.)
 template <int NPROJ, int CPL>
 __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
   const uint32_t lane = threadIdx.x & 63;
@@ -59,6 +61,10 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 #pragma unroll
     for (int i = 0; i < CPL; ++i) xn[i] = load_x8<true>(nx + min(lane + 64 * i, chunks - 1) * 8);
     issue_fence();
+#pragma unroll
+    for (int i = 0; i < CPL; ++i)
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) asm volatile("" : "+v"(q[p][i].x), "+v"(q[p][i].y));
     float acc[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) acc[p] = 0.0f;
@@ -111,22 +117,31 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // pieces, XOR-swizzled so that 16 lanes reading one piece of 16 rows cover all banks): read straight from memory a
 // lane's 16 bytes of its own row touch 32 lines per load instruction, and the line rate of the L1, not the matrix
 // core, would set the pace.
-template <int NPROJ, int NT>
-__global__ __launch_bounds__(256) void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
+// KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
+// meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
+// loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens: gate/up 47.6 -> 37.9 us, down 23.8 -> 20.0).
+template <int NPROJ, int NT, int KS>
+__global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   constexpr uint32_t kTok = 64 * NT;
-  __shared__ uint4 s_x[2][kTok * 16];          // [token][16 pieces of 8 values], piece ^ (token & 15)
-  __shared__ uint4 s_w[2][NPROJ][64 * 8];      // [row][8 pieces of 16 codes], piece ^ ((row >> 1) & 7)
-  __shared__ float s_sum[2][kTok][2];          // sum of x over the stage's two groups
+  __shared__ uint4 s_x_all[KS][2][kTok * 16];      // [token][16 pieces of 8 values], piece ^ (token & 15)
+  __shared__ uint4 s_w_all[KS][2][NPROJ][64 * 8];  // [row][8 pieces of 16 codes], piece ^ ((row >> 1) & 7)
+  __shared__ float s_sum_all[KS][2][kTok][2];      // sum of x over the stage's two groups
+  const uint32_t tid = threadIdx.x & 255u, kh = KS == 1 ? 0u : threadIdx.x >> 8;
+  auto& s_x = s_x_all[kh];
+  auto& s_w = s_w_all[kh];
+  auto& s_sum = s_sum_all[kh];
   // consecutive work items (the token tiles of one row slice) on one XCD: its L2 serves the weight rows' re-reads
   const uint32_t per = (n_work + 7) / 8, work = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per || work >= n_work) return;
   const uint32_t t0 = (work % n_tiles) * kTok, r0 = (work / n_tiles) * 64;
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, m = lane & 31, h = lane >> 5;
+  const uint32_t lane = tid & 63, wv = tid >> 6, m = lane & 31, h = lane >> 5;
   const uint32_t rb = wv & 1, tb = wv >> 1;
   const uint32_t ng = a.N / kGroup, n_st = (ng + 1) / 2;
+  const uint32_t n_walk = (n_st + KS - 1) / KS, st0 = kh * n_walk, st1 = min(n_st, st0 + n_walk);  // this set's stages
 
   // staging roles: x -- token t / 4 (+ 64), pieces 4q .. 4q + 3 (half a group); codes -- row t / 8 (+ 32), piece t % 8
-  const uint32_t xt = threadIdx.x >> 2, xq = threadIdx.x & 3, wr = threadIdx.x >> 3, wc = threadIdx.x & 7;
+  // (whole 256-byte token rows per 16 threads measured slower: 40.4 against 37.9 us, four row addresses a thread)
+  const uint32_t xt = tid >> 2, xq = tid & 3, wr = tid >> 3, wc = tid & 7;
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
   u32x4_t xr[NT][4], wreg[NPROJ][2];
   const uint32_t row = min(r0 + rb * 32 + m, a.M - 1);  // the lane's weight row (past the end: the last one, not stored)
@@ -191,20 +206,23 @@ __global__ __launch_bounds__(256) void qmm8_kernel(const Q8Args a, uint32_t n_ti
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[p][n][r] = 0.0f;
 
-  fetch(0);
-  fetch_tab(0);
-  put(0);
-  if (n_st > 1) fetch(1);
-  for (uint32_t st = 0; st < n_st; ++st) {
-    __syncthreads();  // buffer st & 1 is complete, the other one is no longer read
-    const uint32_t buf = st & 1;
+  if (st0 < st1) {
+    fetch(st0);
+    fetch_tab(st0);
+    put(0);
+    if (st0 + 1 < st1) fetch(st0 + 1);
+  }
+  for (uint32_t i_st = 0; i_st < n_walk; ++i_st) {
+    __syncthreads();  // buffer i_st & 1 is complete, the other one is no longer read
+    const uint32_t st = st0 + i_st, buf = i_st & 1;
+    if (st >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
     uint32_t scv[NPROJ][2], bv[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) scv[p][0] = sc[p][0], scv[p][1] = sc[p][1], bv[p] = bi[p];
-    if (st + 1 < n_st) {
+    if (st + 1 < st1) {
       put(buf ^ 1);
       fetch_tab(st + 1);
-      if (st + 2 < n_st) fetch(st + 2);
+      if (st + 2 < st1) fetch(st + 2);
     }
     // biases: K slots of half h = (hi, mid, lo) of sum(x) over group 2 st + h (a group past the end sums to 0)
 #pragma unroll
@@ -261,6 +279,27 @@ __global__ __launch_bounds__(256) void qmm8_kernel(const Q8Args a, uint32_t n_ti
       }
     }
   }
+  if constexpr (KS == 2) {  // the second set's sums to the first, over the x buffers
+    static_assert(sizeof(s_x_all) >= 4u * 64 * NPROJ * NT * 16 * sizeof(float), "the sums fit the x buffers");
+    float* s_acc = reinterpret_cast<float*>(&s_x_all[0][0][0]);
+    __syncthreads();
+    if (kh == 1) {
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s_acc[((p * NT + n) * 16 + i) * 256 + tid] = acc[p][n][i];
+    }
+    __syncthreads();
+    if (kh == 1) return;
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[p][n][i] = acc[p][n][i] + s_acc[((p * NT + n) * 16 + i) * 256 + tid];
+  }
   // the lane holds weight row r0 + 32 rb + m for tokens 8j + 4h + i of each 32-token block
   const uint32_t out_row = r0 + rb * 32 + m;
   if (out_row >= a.M) return;
@@ -292,9 +331,12 @@ static bool q8_launch(hipStream_t s, const Q8Args& a, hipError_t& err) {
     const uint32_t slices = (a.M + 63) / 64;
     const bool wide = slices * ((a.T + 63) / 64) > 768;
     const uint32_t tok = wide ? 128 : 64, tiles = (a.T + tok - 1) / tok, n_work = slices * tiles;
-    const dim3 grid((n_work + 7) / 8 * 8), block(256);
-    if (wide) qmm8_kernel<NPROJ, 2><<<grid, block, 0, s>>>(a, tiles, n_work);
-    else qmm8_kernel<NPROJ, 1><<<grid, block, 0, s>>>(a, tiles, n_work);
+    const dim3 grid((n_work + 7) / 8 * 8);
+#define MF_QMM8(NT, KS) qmm8_kernel<NPROJ, NT, KS><<<grid, dim3(256 * KS), 0, s>>>(a, tiles, n_work)
+    if (wide) MF_QMM8(2, 1);
+    else if (n_work > 256) MF_QMM8(1, 1);
+    else MF_QMM8(1, 2);
+#undef MF_QMM8
     err = hipGetLastError();
     return true;
   }

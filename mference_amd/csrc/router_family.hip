@@ -17,7 +17,9 @@ namespace {
 // One wave per (token, expert) row of router_gemv_gemma4_body (moe.metal:102-139).  8-wide chunks
 // are dealt to the 64 lanes; a chunk lies inside one group of 64, its sum q*x' and sum x' are built
 // in ascending order from 0 and enter the lane's accumulator as fma(s, dot, acc), fma(b, sum, acc);
-// x' = x * effective_scale is exact in fp32 for bf16 factors.
+// x' = x * effective_scale is exact in fp32 for bf16 factors.  A lane's first CPL chunks are requested together
+// (a row of 2816 is six chunks a lane: six trips to memory one after the other took 2 us of a one-token call).
+template <int CPL>
 __global__ __launch_bounds__(256) void router_logits_int8_kernel(
     const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ x,
@@ -32,64 +34,70 @@ __global__ __launch_bounds__(256) void router_logits_int8_kernel(
   const uint16_t* b_row = biases + static_cast<size_t>(row) * (d / MF_GROUP_SIZE);
   const uint16_t* x_row = x + static_cast<size_t>(tok) * x_stride;
   float acc = 0.0f;
-  for (uint32_t c = lane; c < d / 8; c += kWave) {
-    uint32_t q[2];
-    uint4 xv, ev;
-    if (aligned) {
-      const uint2 qq = *reinterpret_cast<const uint2*>(q_row + c * 8);
-      q[0] = qq.x; q[1] = qq.y;
-      xv = load_x8<true>(x_row + c * 8);
-      ev = load_x8<true>(eff + c * 8);
-    } else {
-      const uint8_t* p = q_row + c * 8;
-      q[0] = p[0] | (p[1] << 8) | (p[2] << 16) | (static_cast<uint32_t>(p[3]) << 24);
-      q[1] = p[4] | (p[5] << 8) | (p[6] << 16) | (static_cast<uint32_t>(p[7]) << 24);
-      xv = load_x8<false>(x_row + c * 8);
-      ev = load_x8<false>(eff + c * 8);
-    }
-    const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w}, es[4] = {ev.x, ev.y, ev.z, ev.w};
-    float dot = 0.0f, sum = 0.0f;
+  for (uint32_t c0 = lane; c0 < d / 8; c0 += CPL * kWave) {
+    uint2 q[CPL];
+    uint4 xv[CPL], ev[CPL];
+    uint32_t sv[CPL], bv[CPL];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float x0 = bf16_lo(xs[j]) * bf16_lo(es[j]);
-      const float x1 = bf16_hi(xs[j]) * bf16_hi(es[j]);
-      const uint32_t word = q[j >> 1] >> ((j & 1) * 16);
-      dot = __builtin_fmaf(static_cast<float>(word & 0xFFu), x0, dot);
-      sum = sum + x0;
-      dot = __builtin_fmaf(static_cast<float>((word >> 8) & 0xFFu), x1, dot);
-      sum = sum + x1;
+    for (int i = 0; i < CPL; ++i) {
+      const uint32_t c = min(c0 + i * kWave, d / 8 - 1);  // past the row: the last chunk again, dropped below
+      if (aligned) {
+        q[i] = *reinterpret_cast<const uint2*>(q_row + c * 8);
+        xv[i] = load_x8<true>(x_row + c * 8);
+        ev[i] = load_x8<true>(eff + c * 8);
+      } else {
+        q[i] = make_uint2(load_u32_bytes(q_row + c * 8), load_u32_bytes(q_row + c * 8 + 4));
+        xv[i] = load_x8<false>(x_row + c * 8);
+        ev[i] = load_x8<false>(eff + c * 8);
+      }
+      sv[i] = s_row[c * 8 / MF_GROUP_SIZE];
+      bv[i] = b_row[c * 8 / MF_GROUP_SIZE];
     }
-    const uint32_t g = c * 8 / MF_GROUP_SIZE;
-    acc = __builtin_fmaf(bf16_to_f(s_row[g]), dot, acc);
-    acc = __builtin_fmaf(bf16_to_f(b_row[g]), sum, acc);
+    issue_fence();
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+      if (c0 + i * kWave >= d / 8) break;
+      const uint32_t xs[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, es[4] = {ev[i].x, ev[i].y, ev[i].z, ev[i].w};
+      float dot = 0.0f, sum = 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float x0 = bf16_lo(xs[j]) * bf16_lo(es[j]);
+        const float x1 = bf16_hi(xs[j]) * bf16_hi(es[j]);
+        const uint32_t word = (j < 2 ? q[i].x : q[i].y) >> ((j & 1) * 16);
+        dot = __builtin_fmaf(static_cast<float>(word & 0xFFu), x0, dot);
+        sum = sum + x0;
+        dot = __builtin_fmaf(static_cast<float>((word >> 8) & 0xFFu), x1, dot);
+        sum = sum + x1;
+      }
+      acc = __builtin_fmaf(__uint_as_float(sv[i] << 16), dot, acc);
+      acc = __builtin_fmaf(__uint_as_float(bv[i] << 16), sum, acc);
+    }
   }
   acc = wave_sum(acc);
   if (lane == 0) logits[static_cast<size_t>(tok) * e + row] = acc;
 }
 
-// The same rows for many tokens, bit-exact with the kernel above: a wave keeps R expert rows in
-// registers (lane l holds the chunks l, l+64, ... of each row as floats, with their group's scale and
-// bias) together with effective_scale, and streams token rows past them; sum x' of a chunk is the
-// same for every row and is built once per token.  Needs 16-byte aligned x and effective_scale, 8-byte
-// aligned code rows.
+// The same rows for many tokens, bit-exact with the kernel above.  A wave keeps R expert rows in registers (lane l
+// holds the chunks l, l+64, ... of each row as floats, with their group's scale and bias); the workgroup's threads make
+// x' and the chunk sums of one token ahead, once for all its rows, in LDS (two buffers).  Bound by vector
+// instructions: with x' made by every wave for its two rows it was 150 a row and token, here 90 (128 rows of 2816,
+// 300 tokens: 29.6 -> 18.3 us).  Needs 16-byte aligned x and effective_scale, 8-byte aligned code rows.
 template <int CPL, int R>
 __global__ __launch_bounds__(256) void router_logits_int8_tiled_kernel(
     const uint8_t* __restrict__ codes, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint16_t* __restrict__ x,
     const uint16_t* __restrict__ eff, uint32_t e, uint32_t d, uint32_t t, uint32_t x_stride,
     float* __restrict__ logits, uint32_t tokens_per_block) {
+  constexpr uint32_t kChunks = 64 * CPL, kMine = (kChunks + 255) / 256;
+  __shared__ float4 s_x[2][2][kChunks];  // [buffer][half of the chunk][chunk]
+  __shared__ float s_sum[2][kChunks];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint32_t row0 = (blockIdx.x * 4 + wv) * R;
-  if (row0 >= e) return;
+  const uint32_t row0 = (blockIdx.x * 4 + wv) * R;  // (a wave without a row still helps with x')
   const uint32_t chunks = d / 8, groups = d / MF_GROUP_SIZE;
-  float qf[R][CPL][8], sf[R][CPL], bf[R][CPL], ef[CPL][8];
+  float qf[R][CPL][8], sf[R][CPL], bf[R][CPL];
 #pragma unroll
   for (int c = 0; c < CPL; ++c) {
     const uint32_t ci = lane + 64 * c;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (ci < chunks) v = load_x8<true>(eff + ci * 8);
-    ef[c][0] = bf16_lo(v.x); ef[c][1] = bf16_hi(v.x); ef[c][2] = bf16_lo(v.y); ef[c][3] = bf16_hi(v.y);
-    ef[c][4] = bf16_lo(v.z); ef[c][5] = bf16_hi(v.z); ef[c][6] = bf16_lo(v.w); ef[c][7] = bf16_hi(v.w);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const bool live = ci < chunks && row0 + r < e;
@@ -104,38 +112,65 @@ __global__ __launch_bounds__(256) void router_logits_int8_tiled_kernel(
   }
   const uint32_t t0 = blockIdx.y * tokens_per_block;
   const uint32_t t1 = min(t, t0 + tokens_per_block);
+  uint4 ev[kMine], xv[kMine];
+  auto fetch = [&](uint32_t tok) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < kMine; ++i)
+      xv[i] = load_x8<true>(x + static_cast<size_t>(min(tok, t - 1)) * x_stride + min(threadIdx.x + 256 * i, chunks - 1) * 8);
+  };
+  auto put = [&](uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (uint32_t i = 0; i < kMine; ++i) {
+      const uint32_t ci = threadIdx.x + 256 * i;
+      if (ci < kChunks) {
+        const uint32_t xw[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, ew[4] = {ev[i].x, ev[i].y, ev[i].z, ev[i].w};
+        float p[8], sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          p[2 * j] = bf16_lo(xw[j]) * bf16_lo(ew[j]);
+          p[2 * j + 1] = bf16_hi(xw[j]) * bf16_hi(ew[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum = sum + p[j];
+        s_x[buf][0][ci] = make_float4(p[0], p[1], p[2], p[3]);
+        s_x[buf][1][ci] = make_float4(p[4], p[5], p[6], p[7]);
+        s_sum[buf][ci] = sum;
+      }
+    }
+  };
+#pragma unroll
+  for (uint32_t i = 0; i < kMine; ++i) ev[i] = load_x8<true>(eff + min(threadIdx.x + 256 * i, chunks - 1) * 8);
+  fetch(t0);
+  put(0);
+  fetch(t0 + 1);
   for (uint32_t tok = t0; tok < t1; ++tok) {
-    const uint16_t* xt = x + static_cast<size_t>(tok) * x_stride;
-    float xs[CPL][8], sum[CPL];
+    __syncthreads();  // this token's buffer is complete, the other one is no longer read
+    const uint32_t buf = (tok - t0) & 1;
+    put(buf ^ 1);
+    fetch(tok + 2);
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0f;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       const uint32_t ci = lane + 64 * c;
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (ci < chunks) v = load_x8<true>(xt + ci * 8);
-      const float xv[8] = {bf16_lo(v.x), bf16_hi(v.x), bf16_lo(v.y), bf16_hi(v.y),
-                           bf16_lo(v.z), bf16_hi(v.z), bf16_lo(v.w), bf16_hi(v.w)};
-      sum[c] = 0.0f;
+      const float4 a = s_x[buf][0][ci], b = s_x[buf][1][ci];
+      const float sum = s_sum[buf][ci], xs[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      if (ci < chunks) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        xs[c][j] = xv[j] * ef[c][j];
-        sum[c] = sum[c] + xs[c][j];
+        for (int r = 0; r < R; ++r) {
+          float dot = 0.0f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) dot = __builtin_fmaf(qf[r][c][j], xs[j], dot);
+          acc[r] = __builtin_fmaf(sf[r][c], dot, acc[r]);
+          acc[r] = __builtin_fmaf(bf[r][c], sum, acc[r]);
+        }
       }
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      float acc = 0.0f;
-#pragma unroll
-      for (int c = 0; c < CPL; ++c) {
-        if (lane + 64 * c < chunks) {
-          float dot = 0.0f;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) dot = __builtin_fmaf(qf[r][c][j], xs[c][j], dot);
-          acc = __builtin_fmaf(sf[r][c], dot, acc);
-          acc = __builtin_fmaf(bf[r][c], sum[c], acc);
-        }
-      }
-      acc = wave_sum(acc);
-      if (lane == 0 && row0 + r < e) logits[static_cast<size_t>(tok) * e + row0 + r] = acc;
+      const float v = wave_sum(acc[r]);
+      if (lane == 0 && row0 + r < e) logits[static_cast<size_t>(tok) * e + row0 + r] = v;
     }
   }
 }
@@ -169,43 +204,62 @@ __device__ __forceinline__ float ordered_sum(float v, uint32_t n) {
   return sum;
 }
 
-// One wave per token.
-template <int FAMILY>
-__global__ __launch_bounds__(64) void family_select_kernel(FamilyArgs a) {
+// One wave per token selects.  A few tokens are all latency: there a workgroup of four waves takes a token, an expert
+// per thread and no loop over them (four trips to memory one after the other otherwise: 5.4 -> 3.7 us for 256
+// experts), and what the tail needs of the picked experts -- raw score, scale -- is kept in LDS instead of fetched
+// again by index.
+template <int FAMILY, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void family_select_kernel(FamilyArgs a) {
   __shared__ float s_sel[MF_MAX_EXPERTS];
+  __shared__ float s_raw[MF_MAX_EXPERTS];
   __shared__ uint32_t s_idx[MF_MAX_TOPK];
   __shared__ float s_w[MF_MAX_TOPK];
-  const uint32_t lane = threadIdx.x, tok = blockIdx.x, k = a.k;
+  const uint32_t lane = threadIdx.x & 63, tok = blockIdx.x, k = a.k;
+  constexpr uint32_t kThreads = 64 * WAVES;
+  auto settle = [&]() {  // what the token's threads wrote to LDS is there
+    if constexpr (WAVES > 1) __syncthreads();
+    else lds_settle();
+  };
   const float* lg = a.logits + static_cast<size_t>(tok) * (a.e + a.n_shared);
   uint32_t* idx = a.idx + static_cast<size_t>(tok) * k;
   float* w = a.w + static_cast<size_t>(tok) * k;
 
   if constexpr (FAMILY == kScaledSoftmax) {
     // router_topk_select_k8 (moe.metal:190-240): softmax over the selected, times per_expert_scale
-    topk_select_fast(lg, a.e, k, s_idx, s_w, lane);
+    for (uint32_t x = threadIdx.x; x < a.e; x += kThreads) {
+      s_sel[x] = lg[x];
+      s_raw[x] = bf16_to_f(a.expert_scale[x]);
+    }
+    settle();
+    if (threadIdx.x >= kWave) return;
+    topk_select_fast(s_sel, a.e, k, s_idx, s_w, lane);
     lds_settle();
     if (lane < k) {
       const uint32_t my = s_idx[lane];
       idx[lane] = my;
-      w[lane] = s_w[lane] * bf16_to_f(a.expert_scale[my]);
+      w[lane] = s_w[lane] * s_raw[my];
     }
     return;
   }
 
   uint32_t my = 0;
+  float raw = 0.0f;  // the picked expert's raw score (sqrtsoftplus) or logit (Inkling)
   if constexpr (FAMILY == kHash) {
     if (lane < k) my = a.given[static_cast<size_t>(tok) * k + lane];
   } else {
-    for (uint32_t x = lane; x < a.e; x += kWave) {
-      const float l = lg[x];
-      s_sel[x] = (FAMILY == kSqrtSoftplus ? mf_sqrtsoftplus(l) : 1.0f / (1.0f + mf_exp(-l))) + a.bias[x];
+    for (uint32_t x = threadIdx.x; x < a.e; x += kThreads) {
+      const float l = lg[x], b = a.bias[x], sp = FAMILY == kSqrtSoftplus ? mf_sqrtsoftplus(l) : l;
+      s_raw[x] = sp;
+      s_sel[x] = (FAMILY == kSqrtSoftplus ? sp : 1.0f / (1.0f + mf_exp(-l))) + b;
     }
-    lds_settle();
+    settle();
+    if (threadIdx.x >= kWave) return;
     topk_select_indices(s_sel, a.e, k, s_idx, lane);
     lds_settle();
     if (lane < k) {
       my = s_idx[lane];
       idx[lane] = my;
+      raw = s_raw[my];
     }
   }
 
@@ -215,7 +269,7 @@ __global__ __launch_bounds__(64) void family_select_kernel(FamilyArgs a) {
     const uint32_t total = k + a.n_shared;
     float lp = -__builtin_inff();
     if (lane < total) {
-      const float x = lane < k ? lg[my] : lg[a.e + (lane - k)];
+      const float x = lane < k ? raw : lg[a.e + (lane - k)];
       lp = (x < 0.0f ? x : 0.0f) - mf_log_1to2(1.0f + mf_exp(-__builtin_fabsf(x)));
     }
     const float mx = wave_max(lp);
@@ -227,7 +281,7 @@ __global__ __launch_bounds__(64) void family_select_kernel(FamilyArgs a) {
   } else {
     // moe.metal:773-785 / :855-865: raw sqrtsoftplus scores of the chosen experts, renormalised.
     // An expert index past the table (possible only for given indices) weighs nothing.
-    const float raw = (lane < k && my < a.e) ? mf_sqrtsoftplus(lg[my]) : 0.0f;
+    if constexpr (FAMILY == kHash) raw = (lane < k && my < a.e) ? mf_sqrtsoftplus(lg[my]) : 0.0f;
     const float inv = a.route_scale / (ordered_sum(raw, k) + 1e-20f);
     if (lane < k) w[lane] = raw * inv;
   }
@@ -236,7 +290,9 @@ __global__ __launch_bounds__(64) void family_select_kernel(FamilyArgs a) {
 template <int FAMILY>
 hipError_t launch_family(hipStream_t s, const FamilyArgs& a, uint32_t t) {
   if (!t) return hipSuccess;
-  family_select_kernel<FAMILY><<<dim3(t), dim3(64), 0, s>>>(a);
+  // (given indices have nothing to select; from 512 tokens on the chip is full with a wave each)
+  if (FAMILY != kHash && t < 512) family_select_kernel<FAMILY, 4><<<dim3(t), dim3(256), 0, s>>>(a);
+  else family_select_kernel<FAMILY, 1><<<dim3(t), dim3(64), 0, s>>>(a);
   return hipGetLastError();
 }
 
@@ -251,7 +307,8 @@ hipError_t launch_router_logits_int8(hipStream_t s, const uint8_t* codes, const 
                  x_stride % 8 == 0 && d % 8 == 0;
   const uint32_t cpl = (d / 8 + 63) / 64;
   if (al && t >= 16 && cpl <= 8) {  // many tokens: rows stay in registers
-    const uint32_t tpb = std::max(1u, std::min(64u, t / 64));
+    // about 600 workgroups of 8 rows (two to a CU), at least 4 tokens to a row load
+    const uint32_t tpb = std::max(4u, std::min(64u, t * ((e + 7) / 8) / 600));
 #define MF_R8(CPL, R)                                                                                \
   router_logits_int8_tiled_kernel<CPL, R><<<dim3((e + 4 * R - 1) / (4 * R), (t + tpb - 1) / tpb), dim3(256), 0, \
                                             s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits, tpb)
@@ -262,8 +319,13 @@ hipError_t launch_router_logits_int8(hipStream_t s, const uint8_t* codes, const 
 #undef MF_R8
     return hipGetLastError();
   }
-  router_logits_int8_kernel<<<dim3((waves + 3) / 4), dim3(256), 0, s>>>(codes, scales, biases, x, eff, e, d, t,
-                                                                       x_stride, logits, al);
+#define MF_R8(CPL)                                                                                                  \
+  router_logits_int8_kernel<CPL><<<dim3((waves + 3) / 4), dim3(256), 0, s>>>(codes, scales, biases, x, eff, e, d, t, \
+                                                                            x_stride, logits, al)
+  if (cpl <= 2) MF_R8(2);
+  else if (cpl <= 4) MF_R8(4);
+  else MF_R8(6);
+#undef MF_R8
   return hipGetLastError();
 }
 

@@ -1059,7 +1059,8 @@ def test_int8_shared_expert(gpu, oracle, d, f, t, silu):
 
 
 @pytest.mark.parametrize("d,f,t,silu", [(128, 64, 16, False), (192, 128, 65, True), (320, 704, 130, False),
-                                        (2816, 2112, 33, False), (704, 64, 15, True), (4096, 320, 8, False)])
+                                        (2816, 2112, 33, False), (704, 64, 15, True), (4096, 320, 8, False),
+                                        (128, 2112, 530, False), (192, 2112, 1601, True), (3136, 128, 70, False)])
 def test_int8_shared_expert_many_rows(gpu, oracle, d, f, t, silu):
     """from 16 rows on the 8-bit MLP is a matrix-core matmul (odd numbers of K groups, half slices of rows, ragged
     token tiles): within the layer tolerance of the checker; below, the checker's bits"""
