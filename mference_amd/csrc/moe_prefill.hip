@@ -1060,6 +1060,22 @@ __device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint3
   if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
 }
 
+// 16 bytes from any address the element type allows (global memory takes unaligned vector loads)
+__device__ __forceinline__ uint4 load_16_bytes(const void* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+// eight bf16 numbers without the first n (0..7); zeros follow
+__device__ __forceinline__ uint4 drop_bf16(uint4 v, uint32_t n) {
+  if (n & 4u) v = make_uint4(v.z, v.w, 0, 0);
+  if (n & 2u) v = make_uint4(v.y, v.z, v.w, 0);
+  if (n & 1u)
+    v = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                   __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+  return v;
+}
+
 // silu with the hardware exp2 / reciprocal (1 ulp each): the result is narrowed to bf16 right after
 __device__ __forceinline__ float fast_silu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
@@ -1085,23 +1101,15 @@ struct QmmLaunch {
   uint32_t per_xcd[2];  // work items of each part on one XCD (grid = 8 * their sum)
 };
 
+// NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
+// of groups and rows.
 template <int BITS, int NPROJ, bool NG8, bool TAB16>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
-void qmm_kernel(const QmmLaunch launch) {
+__device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_t* smem) {
   constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t m = lane & 31, h = lane >> 5;
-  // Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of
-  // one tile share its x rows, the tiles of one expert share its weights) are laid on ONE XCD so
-  // that its L2 serves the re-reads.  The tile list is laid out by group_scan_kernel so that every
-  // eighth of it holds an eighth of the live tiles.
-  const uint32_t xcd_slot = blockIdx.x >> 3;
-  const bool second = xcd_slot >= launch.per_xcd[0];
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  const uint32_t work = (blockIdx.x & 7u) * launch.per_xcd[second ? 1 : 0] + (xcd_slot - (second ? launch.per_xcd[0] : 0u));
   const uint32_t wave_rows = a.pair_rows ? 32u * NPROJ : 32u;  // weight rows of one wave
-  const uint32_t n_slices = (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
+  const uint32_t n_slices = NG8 ? a.rows / (kQmmWaves * wave_rows) : (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
   uint32_t tile_id = work / n_slices, slice = work % n_slices, win = 0;
   if (a.dense_mode) {
     if (work >= a.dense_items) return;
@@ -1166,7 +1174,8 @@ void qmm_kernel(const QmmLaunch launch) {
     }
     // (a width that is no multiple of the workgroup's rows: the last slice's waves past the end compute the last
     // 32 rows again and store nothing)
-    row_base[p] = min((slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u), a.rows - 32u);
+    row_base[p] = (slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u);
+    if (!NG8) row_base[p] = min(row_base[p], a.rows - 32u);
   }
   const uint32_t ng_ld = a.ng_ld ? a.ng_ld : ng;
   const size_t row_bytes = static_cast<size_t>(ng_ld) * kGB;
@@ -1241,6 +1250,35 @@ void qmm_kernel(const QmmLaunch launch) {
     TabStep t;
     const uint32_t gl = g0 + 8 * h;
     const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
+    if (!NG8 && ng >= 8) {  // whole 16-byte loads at any group; in the last step they end at the row's end and are moved down
+      const uint32_t gb = min(gc, ng - 8), sh = gc - gb;
+      const bool last = g0 + 16 > ng;  // (uniform)
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+        const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gb;
+        t.B[p] = load_16_bytes(Bp[p] + at);
+        t.S[p] = load_16_bytes(Sp[p] + at);
+        if (last) {
+          t.B[p] = drop_bf16(t.B[p], sh);
+          t.S[p] = drop_bf16(t.S[p], sh);
+        }
+      }
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const float* sp = a.sumx + static_cast<size_t>(xrow[nt]) * ng_ld + g_off + gb;
+        const uint4 s0 = load_16_bytes(sp), s1 = load_16_bytes(sp + 4);
+        const uint32_t w[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t.sx[nt][e] = __uint_as_float(w[e]);
+        if (last) {
+#pragma unroll
+          for (int bit = 4; bit >= 1; bit /= 2)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t.sx[nt][e] = (sh & bit) ? (e + bit < 8 ? t.sx[nt][(e + bit) & 7] : 0.0f) : t.sx[nt][e];
+        }
+      }
+      return t;
+    }
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
       const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gc;
@@ -1493,7 +1531,7 @@ void qmm_kernel(const QmmLaunch launch) {
       const uint32_t c = it * 64 + lane, tok = c >> 2, part = c & 3u;
       const uint32_t sl = s_slot[tok];
       const uint4 v = reinterpret_cast<const uint4*>(so)[c];
-      if (sl != 0xFFFFFFFFu && row_raw < a.rows)
+      if (sl != 0xFFFFFFFFu && (NG8 || row_raw < a.rows))
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out_base) + static_cast<size_t>(sl) * a.rows + row_base[0] +
                                   part * 8) = v;
     }
@@ -1512,7 +1550,7 @@ void qmm_kernel(const QmmLaunch launch) {
 #pragma unroll
           for (int p = 0; p < NPROJ; ++p) {
             if (p > 0 && !a.pair_rows && !out2_base) break;
-            if (row_raw + (a.pair_rows ? 32u * p : 0u) >= a.rows) break;
+            if (!NG8 && row_raw + (a.pair_rows ? 32u * p : 0u) >= a.rows) break;
             uint8_t* ob = (p > 0 && !a.pair_rows) ? out2_base : out_base;  // the second projection's own buffer
             if (a.epi == 1) reinterpret_cast<float*>(ob)[at + row_base[p] + m] = acc[p][nt][4 * j + i];
             else reinterpret_cast<uint16_t*>(ob)[at + row_base[p] + m] = f_to_bf16(acc[p][nt][4 * j + i]);
@@ -1522,6 +1560,39 @@ void qmm_kernel(const QmmLaunch launch) {
     }
   }
   qmm_trace(a, work, 4);
+}
+
+// Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of
+// one tile share its x rows, the tiles of one expert share its weights) are laid on ONE XCD so
+// that its L2 serves the re-reads.  The tile list is laid out by group_scan_kernel so that every
+// eighth of it holds an eighth of the live tiles.
+__device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool& second) {
+  const uint32_t xcd_slot = blockIdx.x >> 3;
+  second = xcd_slot >= per_xcd[0];
+  return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
+}
+
+template <int BITS, int NPROJ, bool NG8, bool TAB16>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
+void qmm_kernel(const QmmLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  qmm_item<BITS, NPROJ, NG8, TAB16>(launch.part[second ? 1 : 0], work, smem);
+}
+
+// 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
+// expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
+// tokens: 53 + 33 beside 388 + 207).
+template <int NPROJ, bool NG8, bool TAB16>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
+void qmm_mixed_kernel(const QmmLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  if (a.dense_mode) qmm_item<4, NPROJ, NG8, TAB16>(a, work, smem);
+  else qmm_item<2, NPROJ, NG8, TAB16>(a, work, smem);
 }
 
 // ---- the same product for a short contraction (K <= 512: the down projections) ----
@@ -1552,19 +1623,12 @@ template <int NG> __device__ __forceinline__ uint4 load_groups_bf16(const uint16
 }
 
 template <int BITS, int NG>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void qmm_kres_kernel(const KresLaunch launch) {
+__device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, uint32_t n_walk, uint8_t* smem) {
   static_assert(NG == 2 || NG == 4 || NG == 8, "K is 128, 256 or 512");
   constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
   constexpr int kRing = NG < 4 ? NG : 4;  // code registers in flight per projection
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t m = lane & 31, h = lane >> 5;
-  const uint32_t xcd_slot = blockIdx.x >> 3;
-  const bool second = xcd_slot >= launch.per_xcd[0];
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  const uint32_t work = (blockIdx.x & 7u) * launch.per_xcd[second ? 1 : 0] + (xcd_slot - (second ? launch.per_xcd[0] : 0u));
-  const uint32_t n_walk = launch.slices[second ? 1 : 0];
   const uint32_t items_per_tile = a.rows / (256u * n_walk);
   uint32_t tile_id = work / items_per_tile, slice0 = (work % items_per_tile) * n_walk;
   if (a.dense_mode) {
@@ -1825,6 +1889,26 @@ void qmm_kres_kernel(const KresLaunch launch) {
   if (count > 32) tile_body(std::integral_constant<int, 2>{});
   else tile_body(std::integral_constant<int, 1>{});
   qmm_trace(a, work, 4);
+}
+
+template <int BITS, int NG>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void qmm_kres_kernel(const KresLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  qmm_kres_item<BITS, NG>(launch.part[second ? 1 : 0], work, launch.slices[second ? 1 : 0], smem);
+}
+
+template <int NG>  // as qmm_mixed_kernel
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void qmm_kres_mixed_kernel(const KresLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  if (a.dense_mode) qmm_kres_item<4, NG>(a, work, walk, smem);
+  else qmm_kres_item<2, NG>(a, work, walk, smem);
 }
 
 // y[t,d] = bf16(h1[t,d] + sum_r w[t,r] * partial[t*K+r, d]), residual first, rank
@@ -2105,7 +2189,9 @@ bool kres_takes(const QmmArgs& q, size_t out_rows) {
   return aligned16(q.expert_base) && q.expert_stride % 16 == 0 && (q.w_off[0] | q.s_off[0] | q.b_off[0]) % 16 == 0;
 }
 
-// bits: 4, or 2 for 2-bit and ternary codes (both problems of one launch have the same width)
+// bits: 4, 2 (2-bit and ternary codes), or kMixedBits: the routed problem 2-bit, the dense one 4-bit
+constexpr int kMixedBits = 24;
+static int part_bits(int bits, const QmmArgs& q) { return bits != kMixedBits ? bits : q.dense_mode ? 4 : 2; }
 hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t tile_slots, const QmmArgs* b,
                            uint32_t b_tile_slots) {
   KresLaunch launch{};
@@ -2120,7 +2206,7 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
     launch.slices[part] = walk;
     if (q.dense_mode) {
       q.dense_tiles = slots;
-      q.tile_major = dense_tile_major(q.rows, q.dense_rows, bits);
+      q.tile_major = dense_tile_major(q.rows, q.dense_rows, part_bits(bits, q));
       q.dense_items = slots * (n_slices / walk);
       launch.per_xcd[part] = dense_per_xcd(q.dense_items);
     } else {
@@ -2131,17 +2217,20 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
   if (grid.x == 0) return hipSuccess;
   const uint32_t ng = a.kdim / kGroup;
   const size_t lds = static_cast<size_t>(ng) * 8192 + kTileTokens * 4 + kTileTokens * ng * 4;
-#define MF_KRES(B, N)                                                                                  \
+#define MF_KRES_L(...)                                                                                 \
   do {                                                                                                 \
-    const hipError_t e = allow_lds<qmm_kres_kernel<B, N>>(lds, kMaxLds);                               \
+    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
     if (e != hipSuccess) return e;                                                                     \
-    qmm_kres_kernel<B, N><<<grid, block, lds, s>>>(launch);                                            \
+    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
   } while (0)
-  if (bits == 4) {
-    if (ng == 8) MF_KRES(4, 8); else if (ng == 4) MF_KRES(4, 4); else MF_KRES(4, 2);
-  } else {
-    if (ng == 8) MF_KRES(2, 8); else if (ng == 4) MF_KRES(2, 4); else MF_KRES(2, 2);
-  }
+#define MF_KRES(N)                                                                                     \
+  do {                                                                                                 \
+    if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<N>);                                       \
+    else if (bits == 4) MF_KRES_L(qmm_kres_kernel<4, N>);                                              \
+    else MF_KRES_L(qmm_kres_kernel<2, N>);                                                             \
+  } while (0)
+  if (ng == 8) MF_KRES(8); else if (ng == 4) MF_KRES(4); else MF_KRES(2);
+#undef MF_KRES_L
 #undef MF_KRES
   return hipGetLastError();
 }
@@ -2160,7 +2249,7 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
     const uint32_t slice_rows = kQmmRows * (q.pair_rows ? nproj : 1), n_slices = (q.rows + slice_rows - 1) / slice_rows;
     if (q.dense_mode) {
       q.dense_tiles = slots;
-      q.tile_major = dense_tile_major(q.rows * (q.pair_rows ? 1 : nproj), q.dense_rows, bits);
+      q.tile_major = dense_tile_major(q.rows * (q.pair_rows ? 1 : nproj), q.dense_rows, part_bits(bits, q));
       q.dense_items = slots * n_slices * std::max(1u, q.n_win);
       launch.per_xcd[part] = dense_per_xcd(q.dense_items);
     } else {
@@ -2172,30 +2261,32 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
         : aligned16(q.expert_base) && q.expert_stride % 16 == 0 &&
               (q.s_off[0] | q.b_off[0] | q.s_off[1] | q.b_off[1]) % 16 == 0;
     tab16 = tab16 || qmm_tab16(q.kdim, nproj);  // with windows: kdim is the longest window
-    ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0;
+    ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0 && q.rows % slice_rows == 0;
   }
   for (int part = 0; part < (b ? 2 : 1); ++part) lds = std::max(lds, qmm_lds_bytes(launch.part[part].kdim, nproj, tab16));
   const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
   if (grid.x == 0) return hipSuccess;
-#define MF_QMM(B, P, G, T)                                                                             \
+#define MF_QMM_L(...)                                                                                  \
   do {                                                                                                 \
-    const hipError_t e = allow_lds<qmm_kernel<B, P, G, T>>(lds, kMaxLds);                              \
+    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
     if (e != hipSuccess) return e;                                                                     \
-    qmm_kernel<B, P, G, T><<<grid, block, lds, s>>>(launch);                                           \
+    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
   } while (0)
-#define MF_QMM_G(B, P, G)                                            \
-  do {                                                               \
-    if (tab16) MF_QMM(B, P, G, true); else MF_QMM(B, P, G, false);   \
+#define MF_QMM(P, G, T)                                                                                \
+  do {                                                                                                 \
+    if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<P, G, T>);                                       \
+    else if (bits == 4) MF_QMM_L(qmm_kernel<4, P, G, T>);                                              \
+    else MF_QMM_L(qmm_kernel<2, P, G, T>);                                                             \
   } while (0)
-#define MF_QMM_B(B)                                                        \
-  do {                                                                     \
-    if (nproj == 2) { if (ng8) MF_QMM_G(B, 2, true); else MF_QMM_G(B, 2, false); } \
-    else { if (ng8) MF_QMM_G(B, 1, true); else MF_QMM_G(B, 1, false); }    \
+#define MF_QMM_G(P, G)                                         \
+  do {                                                         \
+    if (tab16) MF_QMM(P, G, true); else MF_QMM(P, G, false);   \
   } while (0)
-  if (bits == 4) MF_QMM_B(4); else MF_QMM_B(2);
-#undef MF_QMM_B
+  if (nproj == 2) { if (ng8) MF_QMM_G(2, true); else MF_QMM_G(2, false); }
+  else { if (ng8) MF_QMM_G(1, true); else MF_QMM_G(1, false); }
 #undef MF_QMM_G
 #undef MF_QMM
+#undef MF_QMM_L
   return hipGetLastError();
 }
 
@@ -2602,9 +2693,9 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   const bool ternary = c.bits == MF_BITS_TERNARY;
   q.ternary = ternary;
   q.maple = static_cast<int>(c.maple_rounding);
-  // the (4-bit) shared expert rides in the routed launches when the routed experts are 4-bit too;
-  // otherwise its matmuls are launches of their own
-  const bool shared_rides = c.shared_f && code_bits == 4;
+  // the (4-bit) shared expert rides in the routed launches of the same phase
+  const bool shared_rides = c.shared_f != 0;
+  const int launch_bits = c.shared_f && code_bits != 4 ? kMixedBits : code_bits;
   if (h.trace && h.trace_bytes >= 64) {  // stage stamps of the routed gate/up matmul
     q.trace = h.trace;
     q.trace_items = static_cast<uint32_t>(std::min<size_t>(h.trace_bytes / 64, 1u << 30));
@@ -2627,9 +2718,8 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // (Qwen shape, layer: 2048 tokens 280.5 -> 274.5 us, 1024 tokens 191 -> 187 us, 4096 tokens 506 -> 503 us;
   // at 16 384 tokens they are better last, 1763 against 1776 us, where they fill the holes of the last round).
   const bool dense_first = shared_rides && pairs <= 32768;
-  if (dense_first) MF_TRY(launch_qmm(s, code_bits, d, 2, dense_tiles, &q, max_tiles));
-  else MF_TRY(launch_qmm(s, code_bits, q, 2, max_tiles, shared_rides ? &d : nullptr, dense_tiles));
-  if (c.shared_f && !shared_rides) MF_TRY(launch_qmm(s, 4, d, 2, dense_tiles, nullptr, 0));
+  if (dense_first) MF_TRY(launch_qmm(s, launch_bits, d, 2, dense_tiles, &q, max_tiles));
+  else MF_TRY(launch_qmm(s, launch_bits, q, 2, max_tiles, shared_rides ? &d : nullptr, dense_tiles));
   // phase 2: routed down -> fp32 partials [token*K+rank, D]; shared down -> hs [token, D]
   q.w_off[0] = w.offsets.down_w; q.s_off[0] = w.offsets.down_s; q.b_off[0] = ternary ? w.offsets.down_s : w.offsets.down_b;
   q.w_off[1] = q.s_off[1] = q.b_off[1] = 0;
@@ -2652,27 +2742,22 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   {
     // group sums of the activation rows for qmm_kernel (qmm_kres_kernel sums the rows it stages itself);
     // routes past the last tile's count were never written: only pairs rows exist, all written
-    const bool q_ring = !(kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim)));
-    const bool d_ring = c.shared_f && !(kres_d && (!shared_rides || (kres_q && d.kdim == q.kdim)));
+    const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
+    const bool q_ring = !kres_both, d_ring = shared_rides && !kres_both;
     if (q_ring || d_ring)
       MF_TRY(launch_prep_rows(s, q_ring ? ws.acts : nullptr, nullptr, ws.sum_acts, q_ring ? pairs * c.f : 0,
                               d_ring ? ws.sact : nullptr, nullptr, ws.sum_sact,
                               d_ring ? static_cast<size_t>(t) * c.shared_f : 0));
   }
-  if (shared_rides) {
-    if (kres_q && kres_d && d.kdim == q.kdim) {
-      if (dense_first) MF_TRY(launch_qmm_kres(s, 4, d, dense_tiles, &q, max_tiles));
-      else MF_TRY(launch_qmm_kres(s, 4, q, max_tiles, &d, dense_tiles));
-    } else if (dense_first) MF_TRY(launch_qmm(s, 4, d, q.pair_rows ? 2 : 1, dense_tiles, &q, max_tiles));
-    else MF_TRY(launch_qmm(s, 4, q, q.pair_rows ? 2 : 1, max_tiles, &d, dense_tiles));
-  } else {
+  const int down_proj = q.pair_rows ? 2 : 1;
+  if (!shared_rides) {
     if (kres_q) MF_TRY(launch_qmm_kres(s, code_bits, q, max_tiles, nullptr, 0));
-    else MF_TRY(launch_qmm(s, code_bits, q, q.pair_rows ? 2 : 1, max_tiles, nullptr, 0));
-    if (c.shared_f) {
-      if (kres_d) MF_TRY(launch_qmm_kres(s, 4, d, dense_tiles, nullptr, 0));
-      else MF_TRY(launch_qmm(s, 4, d, d.pair_rows ? 2 : 1, dense_tiles, nullptr, 0));
-    }
-  }
+    else MF_TRY(launch_qmm(s, code_bits, q, down_proj, max_tiles, nullptr, 0));
+  } else if (kres_q && kres_d && d.kdim == q.kdim) {
+    if (dense_first) MF_TRY(launch_qmm_kres(s, launch_bits, d, dense_tiles, &q, max_tiles));
+    else MF_TRY(launch_qmm_kres(s, launch_bits, q, max_tiles, &d, dense_tiles));
+  } else if (dense_first) MF_TRY(launch_qmm(s, launch_bits, d, down_proj, dense_tiles, &q, max_tiles));
+  else MF_TRY(launch_qmm(s, launch_bits, q, down_proj, max_tiles, &d, dense_tiles));
   if (ragged) return hipSuccess;  // the per-route results are the caller's: mf_moe_unpermute reduces them
   const uint16_t* hs = nullptr;
   const uint16_t* gate = nullptr;
