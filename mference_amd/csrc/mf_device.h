@@ -366,38 +366,85 @@ __device__ __forceinline__ void expand_q2(uint32_t w, uint4& a, uint4& b) {
 // What the quantized matmuls need to know about a code width: a lane's share of one 64-wide group
 // of its weight row is half the group -- 16 bytes of 4-bit codes or 8 bytes of 2-bit codes (ternary
 // weights are 2-bit codes) -- and it becomes four MFMA operands of 8 bf16 numbers offset + q * step.
-template <int BITS> struct QmmCodes;
-template <> struct QmmCodes<4> {
+//
+// Codes travel in pairs of groups.  Lane l = m + 32 h multiplies half h of row m of a 32-row block.  Asked for that
+// way, from rows as they are, a load instruction touches 32 rows, 32 memory lines, for 1 KB (4-bit) or 512 B (2-bit),
+// and the L1's line rate is a large part of what short batches cost.  So a lane asks for other bytes and
+// the pair is put in order in registers (settle): 4-bit, two loads of 16 rows x 64 bytes (rows 0..15, then 16..31; the
+// 16 lanes q of a quarter-wave take half q / 2 of group q % 2) and one row swap per register pair; 2-bit, one
+// load of 32 rows x 32 bytes (the lanes of half h take group h) and one half-wave swap per register pair.
+// SWAPPED = false (4-bit only): the lane asks for what it multiplies.  That is the better form for a tiled pool
+// (tile_codes_kernel), where those bytes lie side by side and the swaps (2 of 66 vector instructions per group and
+// row block) would buy nothing.  (Layers from the pool as loaded, in us, one piece per row -> this: Qwen shape, 93 tokens
+// 89.9 -> 83.4; dense MLP 5120 x 17408, 150 rows, two of them 345 -> 337.  Qwen shape, 2048 tokens, tiled: 251 without
+// the swaps, 254 with them.)
+template <int BITS, bool SWAPPED = true> struct QmmCodes;
+template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
   static constexpr uint32_t kGroupBytes = 32;     // one group of one row
   static constexpr uint32_t kNegOffsetAdd = 0x02000200u;  // exponent + 4: 16 * scale (offset 8 at step 1/2)
   static constexpr float kScaleMul = 2.0f;        // codes enter as 8 + q/2
-  uint32_t w[4];
-  __device__ __forceinline__ void load(const uint8_t* p) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  uint32_t w[8];  // group 0: w[0..3], group 1: w[4..7]
+  // which group of the pair the lane asks for first; its place in 32 rows as they are and in a tiled block; how far
+  // behind the second load is
+  static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return SWAPPED ? (lane >> 4) & 1u : 0u; }
+  static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool tiled) {
+    if (!SWAPPED) return tiled ? lane * 16u : (lane & 31u) * row_bytes + (lane >> 5) * 16u;
+    return tiled ? lane_group(lane) * 1024u + (lane >> 5) * 512u + (lane & 15u) * 16u
+                 : (lane & 15u) * row_bytes + lane_group(lane) * 32u + (lane >> 5) * 16u;
+  }
+  static __device__ __forceinline__ size_t second(size_t row_bytes, bool tiled) {
+    if (!SWAPPED) return tiled ? 1024u : 32u;
+    return tiled ? 256u : 16u * row_bytes;
+  }
+  // the part of the pair whose registers are free once group i of the pair before has been multiplied
+  __device__ __forceinline__ void load(int i, const uint8_t* p, size_t behind) {
+    const uint4 v = *reinterpret_cast<const uint4*>(i ? p + behind : p);
+    w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
+  }
+  __device__ __forceinline__ void settle() {
+    if (!SWAPPED) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto r = __builtin_amdgcn_permlane16_swap(w[i], w[4 + i], false, false);
+      w[i] = r[0]; w[4 + i] = r[1];
+    }
   }
 };
-template <> struct QmmCodes<2> {
+template <> struct QmmCodes<2, true> {
   static constexpr uint32_t kGroupBytes = 16;
   static constexpr uint32_t kNegOffsetAdd = 0x01000100u;  // exponent + 2: 4 * scale (offset 4 at step 1)
   static constexpr float kScaleMul = 1.0f;        // codes enter as 4 + q
-  uint32_t w[2];
-  __device__ __forceinline__ void load(const uint8_t* p) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    w[0] = v.x; w[1] = v.y;
+  uint32_t w[4];  // group 0: w[0..1], group 1: w[2..3]
+  static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return lane >> 5; }
+  static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool tiled) {
+    return tiled ? lane * 16u : (lane & 31u) * row_bytes + lane_group(lane) * 16u;
+  }
+  static __device__ __forceinline__ size_t second(size_t, bool) { return 0; }
+  __device__ __forceinline__ void load(int i, const uint8_t* p, size_t) {
+    if (i == 0) return;
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  }
+  __device__ __forceinline__ void settle() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const auto r = __builtin_amdgcn_permlane32_swap(w[i], w[2 + i], false, false);
+      w[i] = r[0]; w[2 + i] = r[1];
+    }
   }
 };
 
 // tmp[token block] += x * codes over one group: 8 MFMAs; `after(s)` runs once both token blocks have
 // issued theirs on operand s (the caller may then overwrite bx[.][s])
 // (NTA = 1: only the first token block holds routes, the second is left alone)
-template <int BITS, int NTA = 2, typename After>
-__device__ __forceinline__ void group_products(const QmmCodes<BITS>& c, const uint4 (&bx)[2][4], f32x16_t (&tmp)[2],
+// (g: which group of the settled pair)
+template <int BITS, int NTA = 2, bool SWAPPED, typename After>
+__device__ __forceinline__ void group_products(const QmmCodes<BITS, SWAPPED>& c, int g, const uint4 (&bx)[2][4], f32x16_t (&tmp)[2],
                                                After after) {
   if constexpr (BITS == 4) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const uint4 av = expand_q4(c.w[s]);
+      const uint4 av = expand_q4(c.w[4 * g + s]);
       tmp[0] = mfma_bf16(bx[0][s], av, tmp[0]);
       if constexpr (NTA > 1) tmp[1] = mfma_bf16(bx[1][s], av, tmp[1]);
       after(s);
@@ -406,7 +453,7 @@ __device__ __forceinline__ void group_products(const QmmCodes<BITS>& c, const ui
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       uint4 a, b;
-      expand_q2(c.w[j], a, b);
+      expand_q2(c.w[2 * g + j], a, b);
       tmp[0] = mfma_bf16(bx[0][2 * j], a, tmp[0]);
       if constexpr (NTA > 1) tmp[1] = mfma_bf16(bx[1][2 * j], a, tmp[1]);
       after(2 * j);

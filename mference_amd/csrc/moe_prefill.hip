@@ -874,29 +874,25 @@ __global__ __launch_bounds__(MF_MAX_EXPERTS) void group_place_kernel(const uint3
 }
 
 // ---- the expert pool in the matmul's order
-// A lane of the matmul reads half a K group of ONE weight row per load (16 bytes of 4-bit codes, 8 of 2-bit):
-// row by row that is 32 rows, 32 memory lines, per load instruction, and the L1's line rate is a large part
-// of what a work item costs (Qwen shape, 2048 tokens: layer 273 -> 255 us with the loads below).  In the
-// tiled pool every sub-tensor keeps its place in the blob and its size; inside it, the pieces of the 32 rows
-// of a block for one K group sit side by side in lane order: piece (row block rb, group g, lane l = m + 32 h)
-// = row 32 rb + m, bytes [g * GB + h * GB / 2, + GB / 2) of the row, GB = 32 (4-bit) or 16 (2-bit, ternary)
-// bytes per group.  A load instruction then reads 1 KB (512 B) of consecutive bytes.  Scale and bias tables
+// Row by row a load instruction of the matmul touches 16 (4-bit) or 32 (2-bit) weight rows, a memory line each, and
+// the L1's line rate is a part of what a work item costs.  In the
+// tiled pool every sub-tensor keeps its place in the blob and its size; inside it, the 16-byte pieces of the 32 rows
+// of a block sit side by side, so that a load instruction reads whole runs of consecutive bytes.  4-bit: one run of 1 KB per
+// K group, piece l = m + 32 h = half h of the group of row 32 rb + m.  2-bit, ternary: one run of 1 KB per two
+// groups, piece l = group h of the two of row 32 rb + m.  Scale and bias tables
 // stay row by row.  One thread per piece; sub-tensor w of every expert in one launch.
 __global__ __launch_bounds__(256) void tile_codes_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                                          size_t expert_stride, uint32_t w_off, uint32_t rows,
                                                          uint32_t ng, uint32_t group_bytes) {
-  const uint32_t half = group_bytes / 2;
-  const uint64_t pieces = static_cast<uint64_t>(rows) * ng * 2;
+  const uint32_t row_pieces = ng * group_bytes / 16;  // even: K is a multiple of 128
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= pieces) return;
-  const uint32_t l = static_cast<uint32_t>(i & 63u), m = l & 31u, h = l >> 5;
-  const uint64_t bg = i >> 6;  // rb * ng + g
-  const uint32_t g = static_cast<uint32_t>(bg % ng), rb = static_cast<uint32_t>(bg / ng);
+  if (i >= static_cast<uint64_t>(rows) * row_pieces) return;
+  const uint32_t m = static_cast<uint32_t>(i & 31u), h = static_cast<uint32_t>(i >> 5) & 1u;
+  const uint64_t run = i >> 6;
+  const uint32_t r = static_cast<uint32_t>(run % (row_pieces / 2)), rb = static_cast<uint32_t>(run / (row_pieces / 2));
   const size_t base = static_cast<size_t>(blockIdx.y) * expert_stride + w_off;
-  const uint8_t* from = src + base + (static_cast<size_t>(32u * rb + m) * ng + g) * group_bytes + h * half;
-  uint8_t* to = dst + base + i * half;
-  if (half == 16) *reinterpret_cast<uint4*>(to) = *reinterpret_cast<const uint4*>(from);
-  else *reinterpret_cast<uint2*>(to) = *reinterpret_cast<const uint2*>(from);
+  const uint8_t* from = src + base + (static_cast<size_t>(32u * rb + m) * row_pieces + 2 * r + h) * 16;
+  *reinterpret_cast<uint4*>(dst + base + i * 16) = *reinterpret_cast<const uint4*>(from);
 }
 
 // dst = the pool `src` (E blobs, expert_stride apart) with the three code sub-tensors of every blob tiled
@@ -907,7 +903,7 @@ hipError_t launch_tile_experts(hipStream_t s, const mf_moe_config& c, const void
   const uint32_t gb = c.bits == MF_BITS_4 ? 32u : 16u;
   const struct { uint32_t off, rows, k; } parts[3] = {{off.gate_w, c.f, c.d}, {off.up_w, c.f, c.d}, {off.down_w, c.d, c.f}};
   for (const auto& p : parts) {
-    const uint64_t pieces = static_cast<uint64_t>(p.rows) * (p.k / kGroup) * 2;
+    const uint64_t pieces = static_cast<uint64_t>(p.rows) * (p.k / kGroup) * gb / 16;
     tile_codes_kernel<<<dim3(static_cast<uint32_t>((pieces + 255) / 256), c.num_experts), dim3(256), 0, s>>>(
         static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), expert_stride, p.off, p.rows, p.k / kGroup, gb);
     e = hipGetLastError();
@@ -1103,7 +1099,7 @@ struct QmmLaunch {
 
 // NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
 // of groups and rows.
-template <int BITS, int NPROJ, bool NG8, bool TAB16>
+template <int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
 __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_t* smem) {
   constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1200,16 +1196,25 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     }
   }
   const uint8_t* wrow[NPROJ];
+  using Codes = QmmCodes<BITS, SWAPPED>;
   const uint32_t gstride = a.tiled ? 32u * kGB : kGB;  // bytes from a group's codes to the next group's
-  QmmCodes<BITS> cur[NPROJ][4];
+  const size_t second = Codes::second(row_bytes, a.tiled);
+  const uint32_t last_pair = (ng - 1) & ~1u;
+  // (the last pair of an odd number of groups is half a pair: the lanes that would ask for its second group ask for the first)
+  const uint32_t odd_back = !NG8 && (ng & 1u) ? Codes::lane_group(lane) * gstride : 0u;
+  auto pair_at = [&](uint32_t g) -> size_t {  // g: the pair's first group; past the end: the last pair again
+    const uint32_t gc = min(g, last_pair);
+    return static_cast<size_t>(gc) * gstride - (!NG8 && gc == last_pair ? odd_back : 0u);
+  };
+  Codes cur[NPROJ][2];
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p) {
-    // row by row: the lane's half group of its row, groups kGB apart.  Tiled: the 32 rows' pieces of a group are
-    // one run of 64 x kGB / 2 bytes in lane order (one load instruction reads 1 KB of consecutive bytes)
-    wrow[p] = a.tiled ? Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride + lane * (kGB / 2)
-                      : Wp[p] + (row_base[p] + m) * row_bytes + static_cast<size_t>(g_off) * gstride + h * (kGB / 2);
+    wrow[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride +
+              Codes::lane_offset(lane, row_bytes, a.tiled);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) cur[p][u].load(wrow[p] + min(static_cast<uint32_t>(u), ng - 1) * gstride);
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow[p] + pair_at(2 * u), second);
   }
   __builtin_amdgcn_sched_barrier(0);  // (keeps the look at the routes behind the code loads)
   if (!a.dense_mode) {
@@ -1454,10 +1459,11 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-          group_products<BITS, NTA>(cur[p][2 * uu + gi], bx, tmp, [](int) {});
-          // the register that held this group's codes takes those of the group four ahead
-          // (past the end the last group is read again: no branch inside the unrolled body)
-          cur[p][2 * uu + gi].load(wrow[p] + min(g + 4, ng - 1) * gstride);
+          if (gi == 0) cur[p][uu].settle();
+          group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
+          // the registers that held this group's codes take their part of the pair two ahead
+          // (past the end the last pair is read again: no branch inside the unrolled body)
+          cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
 #pragma unroll
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -1572,13 +1578,13 @@ __device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool&
   return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
 }
 
-template <int BITS, int NPROJ, bool NG8, bool TAB16>
+template <int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
 void qmm_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
-  qmm_item<BITS, NPROJ, NG8, TAB16>(launch.part[second ? 1 : 0], work, smem);
+  qmm_item<BITS, NPROJ, NG8, TAB16, SWAPPED>(launch.part[second ? 1 : 0], work, smem);
 }
 
 // 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
@@ -1591,8 +1597,8 @@ void qmm_mixed_kernel(const QmmLaunch launch) {
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_item<4, NPROJ, NG8, TAB16>(a, work, smem);
-  else qmm_item<2, NPROJ, NG8, TAB16>(a, work, smem);
+  if (a.dense_mode) qmm_item<4, NPROJ, NG8, TAB16, true>(a, work, smem);
+  else qmm_item<2, NPROJ, NG8, TAB16, true>(a, work, smem);
 }
 
 // ---- the same product for a short contraction (K <= 512: the down projections) ----
@@ -1622,11 +1628,12 @@ template <int NG> __device__ __forceinline__ uint4 load_groups_bf16(const uint16
   }
 }
 
-template <int BITS, int NG>
+template <int BITS, int NG, bool SWAPPED>
 __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, uint32_t n_walk, uint8_t* smem) {
   static_assert(NG == 2 || NG == 4 || NG == 8, "K is 128, 256 or 512");
   constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
-  constexpr int kRing = NG < 4 ? NG : 4;  // code registers in flight per projection
+  using Codes = QmmCodes<BITS, SWAPPED>;
+  constexpr int kRing = NG < 4 ? 1 : 2;  // pairs of groups in flight per projection
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t m = lane & 31, h = lane >> 5;
   const uint32_t items_per_tile = a.rows / (256u * n_walk);
@@ -1673,18 +1680,20 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   constexpr uint32_t kRowBytes = NG * kGB;
   // the lane's weight row of block p of slice w: row0 + 256 w + 32 p
   const uint32_t row0 = (slice0 * kQmmWaves + wv) * 64 + m;
-  const uint32_t gstride = a.tiled ? 32u * kGB : kGB;
-  const uint8_t* wrow = a.tiled ? W + static_cast<size_t>(row0 - m) * kRowBytes + lane * (kGB / 2)
-                                : W + static_cast<size_t>(row0) * kRowBytes + h * (kGB / 2);
+  const uint32_t pair_stride = a.tiled ? 64u * kGB : 2u * kGB;
+  const size_t second = Codes::second(kRowBytes, a.tiled);
+  const uint8_t* wrow = W + static_cast<size_t>(row0 - m) * kRowBytes + Codes::lane_offset(lane, kRowBytes, a.tiled);
   const uint16_t* srow = Sp + static_cast<size_t>(row0) * NG;
   const uint16_t* brow = Bp + static_cast<size_t>(row0) * NG;
 
   // ---- everything issued back to back: codes of the first slice, its scale / bias words, the x tile
-  QmmCodes<BITS> cur[2][kRing];
+  Codes cur[2][kRing];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int u = 0; u < kRing; ++u) cur[p][u].load(wrow + p * 32 * kRowBytes + u * gstride);
+    for (int u = 0; u < kRing; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride, second);
   uint4 nS[2], nB[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -1823,16 +1832,19 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-        group_products<BITS, NTA>(cur[p][g % kRing], bx, tmp, [&](int s) {
+        constexpr int kPairs = NG / 2;
+        Codes& codes = cur[p][(g / 2) % kRing];
+        if (g % 2 == 0) codes.settle();
+        group_products<BITS, NTA>(codes, g % 2, bx, tmp, [&](int s) {
           if (p == 1) {  // both row blocks have read x slot s of this group
             bx[0][s] = nbuf[((0 * 4 + s) * 2 + h) * 32 + rd_col[s]];
             if (NTA > 1) bx[1][s] = nbuf[((1 * 4 + s) * 2 + h) * 32 + rd_col[s]];
           }
         });
-        // the register takes the codes kRing groups on: of this slice, or of the next one
-        const int ahead = g + kRing;
-        cur[p][g % kRing].load(ahead < NG ? wrow + p * 32 * kRowBytes + ahead * gstride
-                                          : wnext + p * 32 * kRowBytes + (ahead - NG) * gstride);
+        // the registers take the codes kRing pairs on: of this slice, or of the next one
+        const int ahead = g / 2 + kRing;
+        codes.load(g % 2, ahead < kPairs ? wrow + p * 32 * kRowBytes + ahead * pair_stride
+                                         : wnext + p * 32 * kRowBytes + (ahead - kPairs) * pair_stride, second);
 #pragma unroll
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -1891,13 +1903,13 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   qmm_trace(a, work, 4);
 }
 
-template <int BITS, int NG>
+template <int BITS, int NG, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void qmm_kres_kernel(const KresLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
-  qmm_kres_item<BITS, NG>(launch.part[second ? 1 : 0], work, launch.slices[second ? 1 : 0], smem);
+  qmm_kres_item<BITS, NG, SWAPPED>(launch.part[second ? 1 : 0], work, launch.slices[second ? 1 : 0], smem);
 }
 
 template <int NG>  // as qmm_mixed_kernel
@@ -1907,8 +1919,8 @@ void qmm_kres_mixed_kernel(const KresLaunch launch) {
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_kres_item<4, NG>(a, work, walk, smem);
-  else qmm_kres_item<2, NG>(a, work, walk, smem);
+  if (a.dense_mode) qmm_kres_item<4, NG, true>(a, work, walk, smem);
+  else qmm_kres_item<2, NG, true>(a, work, walk, smem);
 }
 
 // y[t,d] = bf16(h1[t,d] + sum_r w[t,r] * partial[t*K+r, d]), residual first, rank
@@ -2195,6 +2207,7 @@ static int part_bits(int bits, const QmmArgs& q) { return bits != kMixedBits ? b
 hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t tile_slots, const QmmArgs* b,
                            uint32_t b_tile_slots) {
   KresLaunch launch{};
+  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
   for (int part = 0; part < (b ? 2 : 1); ++part) {
     QmmArgs& q = launch.part[part];
     q = part ? *b : a;
@@ -2226,8 +2239,9 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
 #define MF_KRES(N)                                                                                     \
   do {                                                                                                 \
     if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<N>);                                       \
-    else if (bits == 4) MF_KRES_L(qmm_kres_kernel<4, N>);                                              \
-    else MF_KRES_L(qmm_kres_kernel<2, N>);                                                             \
+    else if (bits == 4 && tiled) MF_KRES_L(qmm_kres_kernel<4, N, false>);                              \
+    else if (bits == 4) MF_KRES_L(qmm_kres_kernel<4, N, true>);                                        \
+    else MF_KRES_L(qmm_kres_kernel<2, N, true>);                                                       \
   } while (0)
   if (ng == 8) MF_KRES(8); else if (ng == 4) MF_KRES(4); else MF_KRES(2);
 #undef MF_KRES_L
@@ -2240,6 +2254,7 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
 hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t tile_slots, const QmmArgs* b,
                       uint32_t b_tile_slots) {
   QmmLaunch launch{};
+  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
   size_t lds = 0;
   bool ng8 = true, tab16 = false;
   for (int part = 0; part < (b ? 2 : 1); ++part) {
@@ -2275,8 +2290,9 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
 #define MF_QMM(P, G, T)                                                                                \
   do {                                                                                                 \
     if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<P, G, T>);                                       \
-    else if (bits == 4) MF_QMM_L(qmm_kernel<4, P, G, T>);                                              \
-    else MF_QMM_L(qmm_kernel<2, P, G, T>);                                                             \
+    else if (bits == 4 && G && tiled) MF_QMM_L(qmm_kernel<4, P, G, T, !(G)>);                          \
+    else if (bits == 4) MF_QMM_L(qmm_kernel<4, P, G, T, true>);                                        \
+    else MF_QMM_L(qmm_kernel<2, P, G, T, true>);                                                       \
   } while (0)
 #define MF_QMM_G(P, G)                                         \
   do {                                                         \
