@@ -373,9 +373,9 @@ __device__ __forceinline__ void expand_q2(uint32_t w, uint4& a, uint4& b) {
 // the pair is put in order in registers (settle): 4-bit, two loads of 16 rows x 64 bytes (rows 0..15, then 16..31; the
 // 16 lanes q of a quarter-wave take half q / 2 of group q % 2) and one row swap per register pair; 2-bit, one
 // load of 32 rows x 32 bytes (the lanes of half h take group h) and one half-wave swap per register pair.
-// SWAPPED = false (4-bit only): the lane asks for what it multiplies.  That is the better form for a tiled pool
+// SWAPPED = false: the lane asks for what it multiplies.  That is the better form for a tiled pool
 // (tile_codes_kernel), where those bytes lie side by side and the swaps (2 of 66 vector instructions per group and
-// row block) would buy nothing.  (Layers from the pool as loaded, in us, one piece per row -> this: Qwen shape, 93 tokens
+// row block; 4 of 55 of 2-bit codes and a tile of at most 32 routes) would buy nothing.  (Layers from the pool as loaded, in us, one piece per row -> this: Qwen shape, 93 tokens
 // 89.9 -> 83.4; dense MLP 5120 x 17408, 150 rows, two of them 345 -> 337.  Qwen shape, 2048 tokens, tiled: 251 without
 // the swaps, 254 with them.)
 template <int BITS, bool SWAPPED = true> struct QmmCodes;
@@ -388,13 +388,12 @@ template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
   // behind the second load is
   static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return SWAPPED ? (lane >> 4) & 1u : 0u; }
   static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool tiled) {
-    if (!SWAPPED) return tiled ? lane * 16u : (lane & 31u) * row_bytes + (lane >> 5) * 16u;
-    return tiled ? lane_group(lane) * 1024u + (lane >> 5) * 512u + (lane & 15u) * 16u
-                 : (lane & 15u) * row_bytes + lane_group(lane) * 32u + (lane >> 5) * 16u;
+    if (SWAPPED) return (lane & 15u) * row_bytes + lane_group(lane) * 32u + (lane >> 5) * 16u;
+    return tiled ? lane * 16u : (lane & 31u) * row_bytes + (lane >> 5) * 16u;
   }
   static __device__ __forceinline__ size_t second(size_t row_bytes, bool tiled) {
-    if (!SWAPPED) return tiled ? 1024u : 32u;
-    return tiled ? 256u : 16u * row_bytes;
+    if (SWAPPED) return 16u * row_bytes;
+    return tiled ? 1024u : 32u;
   }
   // the part of the pair whose registers are free once group i of the pair before has been multiplied
   __device__ __forceinline__ void load(int i, const uint8_t* p, size_t behind) {
@@ -410,14 +409,14 @@ template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
     }
   }
 };
-template <> struct QmmCodes<2, true> {
+template <bool SWAPPED> struct QmmCodes<2, SWAPPED> {  // (SWAPPED = false: only tiled)
   static constexpr uint32_t kGroupBytes = 16;
   static constexpr uint32_t kNegOffsetAdd = 0x01000100u;  // exponent + 2: 4 * scale (offset 4 at step 1)
   static constexpr float kScaleMul = 1.0f;        // codes enter as 4 + q
   uint32_t w[4];  // group 0: w[0..1], group 1: w[2..3]
-  static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return lane >> 5; }
-  static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool tiled) {
-    return tiled ? lane * 16u : (lane & 31u) * row_bytes + lane_group(lane) * 16u;
+  static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return SWAPPED ? lane >> 5 : 0u; }
+  static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool) {
+    return SWAPPED ? (lane & 31u) * row_bytes + lane_group(lane) * 16u : lane * 16u;
   }
   static __device__ __forceinline__ size_t second(size_t, bool) { return 0; }
   __device__ __forceinline__ void load(int i, const uint8_t* p, size_t) {
@@ -426,6 +425,7 @@ template <> struct QmmCodes<2, true> {
     w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
   }
   __device__ __forceinline__ void settle() {
+    if (!SWAPPED) return;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const auto r = __builtin_amdgcn_permlane32_swap(w[i], w[2 + i], false, false);

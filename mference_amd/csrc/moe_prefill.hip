@@ -877,22 +877,29 @@ __global__ __launch_bounds__(MF_MAX_EXPERTS) void group_place_kernel(const uint3
 // Row by row a load instruction of the matmul touches 16 (4-bit) or 32 (2-bit) weight rows, a memory line each, and
 // the L1's line rate is a part of what a work item costs.  In the
 // tiled pool every sub-tensor keeps its place in the blob and its size; inside it, the 16-byte pieces of the 32 rows
-// of a block sit side by side, so that a load instruction reads whole runs of consecutive bytes.  4-bit: one run of 1 KB per
-// K group, piece l = m + 32 h = half h of the group of row 32 rb + m.  2-bit, ternary: one run of 1 KB per two
-// groups, piece l = group h of the two of row 32 rb + m.  Scale and bias tables
+// of a block sit side by side, so that a load instruction reads whole runs of consecutive bytes, every lane what it
+// multiplies.  4-bit: one run of 1 KB per K group, piece l = m + 32 h = half h of the group of row 32 rb + m.
+// 2-bit, ternary: one run of 1 KB per two groups, piece l = half h of both groups of that row.  Scale and bias tables
 // stay row by row.  One thread per piece; sub-tensor w of every expert in one launch.
 __global__ __launch_bounds__(256) void tile_codes_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                                          size_t expert_stride, uint32_t w_off, uint32_t rows,
                                                          uint32_t ng, uint32_t group_bytes) {
-  const uint32_t row_pieces = ng * group_bytes / 16;  // even: K is a multiple of 128
+  const uint32_t row_bytes = ng * group_bytes, runs = row_bytes / 32;  // (K is a multiple of 128)
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= static_cast<uint64_t>(rows) * row_pieces) return;
+  if (i >= static_cast<uint64_t>(rows) * (row_bytes / 16)) return;
   const uint32_t m = static_cast<uint32_t>(i & 31u), h = static_cast<uint32_t>(i >> 5) & 1u;
   const uint64_t run = i >> 6;
-  const uint32_t r = static_cast<uint32_t>(run % (row_pieces / 2)), rb = static_cast<uint32_t>(run / (row_pieces / 2));
+  const uint32_t r = static_cast<uint32_t>(run % runs), rb = static_cast<uint32_t>(run / runs);
   const size_t base = static_cast<size_t>(blockIdx.y) * expert_stride + w_off;
-  const uint8_t* from = src + base + (static_cast<size_t>(32u * rb + m) * row_pieces + 2 * r + h) * 16;
-  *reinterpret_cast<uint4*>(dst + base + i * 16) = *reinterpret_cast<const uint4*>(from);
+  const uint8_t* from = src + base + static_cast<size_t>(32u * rb + m) * row_bytes + r * 32;
+  uint4 v;
+  if (group_bytes == 32) {
+    v = *reinterpret_cast<const uint4*>(from + h * 16);
+  } else {
+    const uint2 a = *reinterpret_cast<const uint2*>(from + h * 8), b = *reinterpret_cast<const uint2*>(from + 16 + h * 8);
+    v = make_uint4(a.x, a.y, b.x, b.y);
+  }
+  *reinterpret_cast<uint4*>(dst + base + i * 16) = v;
 }
 
 // dst = the pool `src` (E blobs, expert_stride apart) with the three code sub-tensors of every blob tiled
@@ -1410,6 +1417,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   // from HBM); x rows come from L2 in pairs of groups, one pair in registers behind
   // the pair in the LDS stage that is not being read.
 
+  Codes now[NPROJ];
   for (uint32_t g0 = 0; g0 < ng; g0 += 4) {
 #pragma unroll
     for (int uu = 0; uu < 2; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
@@ -1459,11 +1467,18 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-          if (gi == 0) cur[p][uu].settle();
-          group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
+          if (gi == 0) {
+            if constexpr (BITS == 2) {  // (all four registers of the pair are one load: it leaves at once, from a copy)
+              now[p] = cur[p][uu];
+              cur[p][uu].load(1, wrow[p] + pair_at(gu + 4), second);
+              now[p].settle();
+            } else cur[p][uu].settle();
+          }
+          if constexpr (BITS == 2) group_products<BITS, NTA>(now[p], gi, bx, tmp, [](int) {});
+          else group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
           // the registers that held this group's codes take their part of the pair two ahead
           // (past the end the last pair is read again: no branch inside the unrolled body)
-          cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
+          if constexpr (BITS != 2) cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
 #pragma unroll
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -1584,13 +1599,20 @@ void qmm_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
-  qmm_item<BITS, NPROJ, NG8, TAB16, SWAPPED>(launch.part[second ? 1 : 0], work, smem);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  if constexpr (BITS == 2 && !SWAPPED) {  // (a dense problem beside a tiled pool lies row by row)
+    if (a.dense_mode) {
+      qmm_item<BITS, NPROJ, NG8, TAB16, true>(a, work, smem);
+      return;
+    }
+  }
+  qmm_item<BITS, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
 }
 
 // 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
 // expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
 // tokens: 53 + 33 beside 388 + 207).
-template <int NPROJ, bool NG8, bool TAB16>
+template <int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
 void qmm_mixed_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -1598,7 +1620,7 @@ void qmm_mixed_kernel(const QmmLaunch launch) {
   const uint32_t work = qmm_work(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
   if (a.dense_mode) qmm_item<4, NPROJ, NG8, TAB16, true>(a, work, smem);
-  else qmm_item<2, NPROJ, NG8, TAB16, true>(a, work, smem);
+  else qmm_item<2, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
 }
 
 // ---- the same product for a short contraction (K <= 512: the down projections) ----
@@ -1820,6 +1842,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
         for (int s = 0; s < 4; ++s) bx[nt][s] = s_x[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
     }
+    Codes now[2];
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       const uint4* nbuf = s_x + ((g + 1) % NG) * 512;  // after the last group: group 0 again, for the next slice
@@ -1834,17 +1857,24 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
           for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
         constexpr int kPairs = NG / 2;
         Codes& codes = cur[p][(g / 2) % kRing];
-        if (g % 2 == 0) codes.settle();
-        group_products<BITS, NTA>(codes, g % 2, bx, tmp, [&](int s) {
+        const int ahead = g / 2 + kRing;
+        const uint8_t* next_pair = ahead < kPairs ? wrow + p * 32 * kRowBytes + ahead * pair_stride
+                                                  : wnext + p * 32 * kRowBytes + (ahead - kPairs) * pair_stride;
+        if (g % 2 == 0) {
+          if constexpr (BITS == 2) {
+            now[p] = codes;
+            codes.load(1, next_pair, second);
+            now[p].settle();
+          } else codes.settle();
+        }
+        group_products<BITS, NTA>(BITS == 2 ? now[p] : codes, g % 2, bx, tmp, [&](int s) {
           if (p == 1) {  // both row blocks have read x slot s of this group
             bx[0][s] = nbuf[((0 * 4 + s) * 2 + h) * 32 + rd_col[s]];
             if (NTA > 1) bx[1][s] = nbuf[((1 * 4 + s) * 2 + h) * 32 + rd_col[s]];
           }
         });
         // the registers take the codes kRing pairs on: of this slice, or of the next one
-        const int ahead = g / 2 + kRing;
-        codes.load(g % 2, ahead < kPairs ? wrow + p * 32 * kRowBytes + ahead * pair_stride
-                                         : wnext + p * 32 * kRowBytes + (ahead - kPairs) * pair_stride, second);
+        if constexpr (BITS != 2) codes.load(g % 2, next_pair, second);
 #pragma unroll
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -1909,10 +1939,18 @@ void qmm_kres_kernel(const KresLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
-  qmm_kres_item<BITS, NG, SWAPPED>(launch.part[second ? 1 : 0], work, launch.slices[second ? 1 : 0], smem);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  const uint32_t walk = launch.slices[second ? 1 : 0];
+  if constexpr (BITS == 2 && !SWAPPED) {
+    if (a.dense_mode) {
+      qmm_kres_item<BITS, NG, true>(a, work, walk, smem);
+      return;
+    }
+  }
+  qmm_kres_item<BITS, NG, SWAPPED>(a, work, walk, smem);
 }
 
-template <int NG>  // as qmm_mixed_kernel
+template <int NG, bool SWAPPED>  // as qmm_mixed_kernel
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void qmm_kres_mixed_kernel(const KresLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -1920,7 +1958,7 @@ void qmm_kres_mixed_kernel(const KresLaunch launch) {
   const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
   const QmmArgs& a = launch.part[second ? 1 : 0];
   if (a.dense_mode) qmm_kres_item<4, NG, true>(a, work, walk, smem);
-  else qmm_kres_item<2, NG, true>(a, work, walk, smem);
+  else qmm_kres_item<2, NG, SWAPPED>(a, work, walk, smem);
 }
 
 // y[t,d] = bf16(h1[t,d] + sum_r w[t,r] * partial[t*K+r, d]), residual first, rank
@@ -2238,9 +2276,11 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
   } while (0)
 #define MF_KRES(N)                                                                                     \
   do {                                                                                                 \
-    if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<N>);                                       \
+    if (bits == kMixedBits && tiled) MF_KRES_L(qmm_kres_mixed_kernel<N, false>);                       \
+    else if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<N, true>);                            \
     else if (bits == 4 && tiled) MF_KRES_L(qmm_kres_kernel<4, N, false>);                              \
     else if (bits == 4) MF_KRES_L(qmm_kres_kernel<4, N, true>);                                        \
+    else if (tiled) MF_KRES_L(qmm_kres_kernel<2, N, false>);                                           \
     else MF_KRES_L(qmm_kres_kernel<2, N, true>);                                                       \
   } while (0)
   if (ng == 8) MF_KRES(8); else if (ng == 4) MF_KRES(4); else MF_KRES(2);
@@ -2289,9 +2329,11 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
   } while (0)
 #define MF_QMM(P, G, T)                                                                                \
   do {                                                                                                 \
-    if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<P, G, T>);                                       \
-    else if (bits == 4 && G && tiled) MF_QMM_L(qmm_kernel<4, P, G, T, !(G)>);                          \
+    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<P, G, T, false>);                       \
+    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<P, G, T, true>);                            \
+    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<4, P, G, T, false>);                              \
     else if (bits == 4) MF_QMM_L(qmm_kernel<4, P, G, T, true>);                                        \
+    else if (tiled) MF_QMM_L(qmm_kernel<2, P, G, T, false>);                                           \
     else MF_QMM_L(qmm_kernel<2, P, G, T, true>);                                                       \
   } while (0)
 #define MF_QMM_G(P, G)                                         \
