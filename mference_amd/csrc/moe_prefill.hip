@@ -1185,7 +1185,10 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 
   // ---- everything the tile needs that depends only on the tile: issued back to back.
   // Routes past `count` read the tile's last route instead (finite data, results discarded).
-  const uint32_t st_i = threadIdx.x >> 2, st_q = threadIdx.x & 3;  // staging: token i, K values 16q..16q+15
+  // staging: a thread takes two runs of 8 K values of one token in every group, or one of a tile of at most 32 routes
+  const bool few = NPROJ == 2 && count <= 32;
+  const uint32_t st_i = few ? threadIdx.x >> 3 : threadIdx.x >> 2;
+  const uint32_t st_c0 = few ? threadIdx.x & 7 : (threadIdx.x & 3) * 2, st_c1 = few ? st_c0 : st_c0 + 1;
   const uint32_t st_pair = pair_start + min(st_i, count - 1);
   const uint32_t ti_pair[2] = {pair_start + min(m, count - 1), pair_start + min(32 + m, count - 1)};
   uint32_t st_row = st_pair, xrow[2] = {ti_pair[0], ti_pair[1]};
@@ -1233,7 +1236,8 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
   }
   // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
-  const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_q * 16;
+  const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_c0 * 8;
+  const uint32_t st_2nd = (st_c1 - st_c0) * 8;
   // K groups travel in pairs; a contraction of an odd number of groups ends in half a pair (its other half is read
   // from the last group again and not multiplied)
   // (arrays of a native vector type: arrays of the uint4 struct were kept in scratch memory)
@@ -1244,11 +1248,11 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   for (int gi = 0; gi < 2; ++gi) {
     const uint32_t ga = NG8 ? gi : min(static_cast<uint32_t>(gi), ng - 1), gb = NG8 ? 2u + gi : min(2u + gi, ng - 1);
     x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup);
-    x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + 8);
+    x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + st_2nd);
     xs[gi][0] = xs[gi][1] = u32x4_t{0, 0, 0, 0};
     if (NG8 || ng > 2) {
       xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup);
-      xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + 8);
+      xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + st_2nd);
     }
   }
   // Scale and bias words of the lane's row and the group sums of its two routes, 8 K groups at a time
@@ -1334,9 +1338,10 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   // offset * sum(x) the matrix core accumulated with the codes, so it has to be exact.
   // A tile of at most 32 routes fills only the first token block: the second block's matrix
   // instructions and scale multiplies are left out (NTA = 1); its accumulators stay zero and its
-  // output slots are empty.
-  auto tile_body = [&](auto nta_c) {
-  constexpr int NTA = decltype(nta_c)::value;
+  // output slots are empty.  Of a tile of at most 8 routes (most tiles of a short prompt) a lane's first four results are all
+  // there is: only those are scaled (RES), 4 of 16 multiply-adds per group and row block.
+  auto tile_body = [&](auto nta_c, auto res_c) {
+  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
   for (uint32_t g0 = 0; g0 < ng; g0 += 16) {
     const TabStep t = tab_cur;
     tab_cur = tab_fetch(g0 + 16 < ng ? g0 + 16 : g0);  // past the end: the same step again, unused
@@ -1398,7 +1403,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   qmm_trace(a, work, 2);
 
   // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
-  const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = 2 * st_q, c1 = c0 + 1;
+  const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
   // inside a 32-token block the column is rotated by 4 * ((s >> 1) + 2h): the four lanes that
   // stage one token then hit four different bank groups
   const uint32_t st_rot = 4 * ((c0 & 3) >> 1) + 8 * (c0 >> 2);
@@ -1410,7 +1415,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
   for (int gi = 0; gi < 2; ++gi) {
     *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot0) = x0[gi][0];
-    *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot1) = x0[gi][1];
+    if (NTA > 1) *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot1) = x0[gi][1];
   }
 
   // Weight codes run four K groups ahead in a ring of registers (the expert's bytes come
@@ -1434,7 +1439,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
         for (int gi = 0; gi < 2; ++gi) {
           *reinterpret_cast<u32x4_t*>(wbuf + gi * 512 + st_slot0) = xs[gi][0];
-          *reinterpret_cast<u32x4_t*>(wbuf + gi * 512 + st_slot1) = xs[gi][1];
+          if (NTA > 1) *reinterpret_cast<u32x4_t*>(wbuf + gi * 512 + st_slot1) = xs[gi][1];
         }
         if (NG8 || gu + 4 < ng) {
           const uint32_t gx = NG8 ? min(gu + 4, ng - 2) : gu + 4;
@@ -1442,7 +1447,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           for (int gi = 0; gi < 2; ++gi) {
             const uint32_t gy = NG8 ? gx + gi : min(gx + gi, ng - 1);
             xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup);
-            xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + 8);
+            if (NTA > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + st_2nd);
           }
         }
       }
@@ -1482,15 +1487,18 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
+            for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
         }
       }
     }
   }
   };  // tile_body
   // (the one-projection form keeps to its budget of 168 registers, three waves per SIMD, with one body only)
-  if (NPROJ == 1 || count > 32) tile_body(std::integral_constant<int, 2>{});
-  else tile_body(std::integral_constant<int, 1>{});
+  using two = std::integral_constant<int, 2>;
+  using one = std::integral_constant<int, 1>;
+  if (NPROJ == 1 || count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
+  else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
+  else tile_body(one{}, std::integral_constant<int, 4>{});
 
   qmm_trace(a, work, 3);
   // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
@@ -1515,6 +1523,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
         if (nt == 1 && count <= 32) break;  // no route in the second block: its slots are empty
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+          if (j == 1 && count <= 8) break;
           uint32_t bits[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -1562,6 +1571,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
       if (nt == 1 && count <= 32) break;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
+        if (j == 1 && count <= 8) break;
         const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
         const uint32_t slot[4] = {sl.x, sl.y, sl.z, sl.w};
 #pragma unroll
@@ -1776,8 +1786,9 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   // groups again, multiplied by the biases for h = 0 and by -offset * scale for h = 1.
   // A tile of at most 32 routes fills only the first route block (NTA = 1): the second block, whose routes
   // would all repeat the last route, is left out of the products, the scale multiplies and the stores.
-  auto tile_body = [&](auto nta_c) {
-  constexpr int NTA = decltype(nta_c)::value;
+  // (RES = 4 for a tile of at most 8 routes: as in qmm_item)
+  auto tile_body = [&](auto nta_c, auto res_c) {
+  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
   uint4 b_term[2][3];
 #pragma unroll
   for (int nt = 0; nt < NTA; ++nt) {
@@ -1878,7 +1889,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
+          for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
         // the sums are wanted here, not after the last group: without this the compiler keeps every
         // group's products and adds them up at the end of the slice, out of scratch memory
         if constexpr (NTA > 1) asm volatile("" : "+v"(acc[p][0]), "+v"(acc[p][1]));
@@ -1896,7 +1907,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
       for (int nt = 0; nt < NTA; ++nt) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < RES / 4; ++j) {
           const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
           const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
 #pragma unroll
@@ -1913,7 +1924,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
       for (int nt = 0; nt < NTA; ++nt) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < RES / 4; ++j) {
           const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
           const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
 #pragma unroll
@@ -1928,8 +1939,11 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
     wrow = wnext;
   }
   };  // tile_body
-  if (count > 32) tile_body(std::integral_constant<int, 2>{});
-  else tile_body(std::integral_constant<int, 1>{});
+  using two = std::integral_constant<int, 2>;
+  using one = std::integral_constant<int, 1>;
+  if (count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
+  else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
+  else tile_body(one{}, std::integral_constant<int, 4>{});
   qmm_trace(a, work, 4);
 }
 
