@@ -197,9 +197,10 @@ int mf_qmm_path(mf_qtensor w, mf_bits bits, const uint16_t* x, const void* y, ui
  * act = bf16(silu(bf16(gate.x)) * bf16(up.x)).  Also the dense SwiGLU MLP of Qwen38ForwardRunner
  * (mlp.encode, :1094) and, for any t, PrefillSharedExpert.encodeBlock (Kernels/Prefill/MoE/
  * PrefillSharedExpert.swift:81-190) / encodeDenseMLPPrefill (Qwen38ForwardRunner.swift:862-913):
- * from 32 rows on the projections run on the matrix cores when d and f are at least 128, the operands are 16-byte aligned and scratch_act holds
- * mf_shared_expert_scratch_bytes(d, f, t) bytes; otherwise row by row, MF_MAX_TOKENS rows per pair
- * of launches, for which t*f bf16 of scratch suffice (all that t <= MF_MAX_TOKENS ever needs). */
+ * beyond MF_MAX_TOKENS rows (small 4-bit shapes: from 16 rows on) the projections run on the matrix cores when d and f
+ * are at least 128, the operands are 16-byte aligned and scratch_act holds mf_shared_expert_scratch_bytes(d, f, t)
+ * bytes; otherwise row by row, MF_MAX_TOKENS rows per pair of launches, for which t*f bf16 of scratch suffice (all
+ * that t <= MF_MAX_TOKENS ever needs). */
 size_t mf_shared_expert_scratch_bytes(uint32_t d, uint32_t f, uint32_t t);
 mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_qtensor gate,
                            mf_qtensor up, mf_qtensor down, mf_bits bits, uint32_t d, uint32_t f,
@@ -212,7 +213,8 @@ mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_
  * Metal/Quant/dequant_int8.metal:110-164): both narrowed to 16 bits, act[f] = narrow(a(gate) * up) with
  * a = the tanh form of GELU (int8_gelu_pytorch_tanh, :44-49) or, silu_activation != 0, SiLU
  * (FC_SHARED_INT8_ACT_SILU, :51-57); then y[d] = narrow(down . act) (dequant_int8_gemv_simd, :66-107).
- * Any t; scratch_act holds t*f bf16.  tanh is built on this library's exp (as every exp on this path). */
+ * Any t; scratch_act holds t*f bf16.  From 16 rows on the products run on the matrix cores (codes and x exact, fp32
+ * sums in their order; below, in the lane order of mf_gemv).  tanh is built on this library's exp (as every exp on this path). */
 mf_status mf_shared_expert_int8(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_qtensor gate,
                                 mf_qtensor up, mf_qtensor down, uint32_t d, uint32_t f, uint32_t t,
                                 int silu_activation, uint16_t* y, uint16_t* scratch_act,

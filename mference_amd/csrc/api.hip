@@ -190,9 +190,13 @@ mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_
   if (scratch_act_bytes < static_cast<size_t>(t) * f * sizeof(uint16_t))
     return MF_ERR_SCRATCH_TOO_SMALL;
   auto s = static_cast<hipStream_t>(stream);
-  // PrefillSharedExpert.encodeBlock (PrefillSharedExpert.swift:114-172): from 32 rows on the projections
-  // go through the matrix-core matmul when the shape allows and the scratch holds its staging rows
-  if (t >= 32 && mf::dense_mlp_takes(gate, up, down, x, y, scratch_act, d, f, t) &&
+  // PrefillSharedExpert.encodeBlock (PrefillSharedExpert.swift:114-172): beyond MF_MAX_TOKENS rows the projections
+  // go through the matrix-core matmul when the shape allows and the scratch holds its staging rows.  Row by row the
+  // weights are read once per 8 rows (2-bit: per row); a small 4-bit MLP of few rows is still faster that way
+  // (us, row by row / matmul: 1024 x 2048, 9 rows 26 / 28, 16 rows 34 / 28; 2048 x 8192, 9 rows 63 / 37;
+  // 5120 x 17408, 9 rows 121 / 77, 31 rows 329 / 81, 2-bit 1522 / 72)
+  const bool few = bits == MF_BITS_4 && t < 16 && static_cast<uint64_t>(t) * d * f < (64ull << 20);
+  if (t > MF_MAX_TOKENS && !few && mf::dense_mlp_takes(gate, up, down, x, y, scratch_act, d, f, t) &&
       scratch_act_bytes >= mf::dense_mlp_scratch_bytes(d, f, t)) {
     MF_HIP(ctx, mf::launch_dense_mlp(s, gate, up, down, bits, x, y, d, f, t, scratch_act));
     return MF_OK;

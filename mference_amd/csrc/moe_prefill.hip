@@ -2388,19 +2388,36 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(const float* __restr
   else static_cast<uint16_t*>(y)[i] = f_to_bf16(acc);
 }
 
-// windows of a contraction of length k
-static uint32_t dense_windows(uint32_t k, uint32_t max_groups = kDenseWindow) {
-  return std::max(1u, (k / kGroup + max_groups - 1) / max_groups);
+// Windows of a contraction of length k for m rows of n results.  At least as many as the scale tables ask for; more where
+// the work items (64 rows of x, 128 or 256 weight rows, one window) would leave the chip idle or its last round nearly
+// empty.  Two items share a CU; an item costs about 3.6 us per 8 groups and 4.7 for its set-up, the
+// windows' sums their bytes and a launch (fitted to n = 5120, k = 17408, m = 32 .. 512: the choice is the best
+// or within 2 % of it; m = 32, 5 -> 12 windows, 101 -> 87 us for the MLP; m = 150, 5 -> 7, 172 -> 158; m = 512, 5 -> 6, 401 -> 389).
+static uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k) {
+  constexpr uint32_t kSlots = 2 * 256;
+  const uint32_t ng = k / kGroup, steps = (ng + 7) / 8;
+  const uint32_t slice_rows = n % (2 * kQmmRows) == 0 ? 2 * kQmmRows : kQmmRows;
+  const uint64_t items = static_cast<uint64_t>((m + kTileTokens - 1) / kTileTokens) * ((n + slice_rows - 1) / slice_rows);
+  const uint32_t lo = std::max(1u, (ng + kDenseWindow - 1) / kDenseWindow), hi = std::max(lo, ng / 8);
+  uint32_t best = lo;
+  double best_us = 0.0;
+  for (uint32_t w = lo; w <= hi; ++w) {
+    const double rounds = static_cast<double>((items * w + kSlots - 1) / kSlots);
+    double us = rounds * (3.6 * ((steps + w - 1) / w) + 4.7);
+    if (w > 1) us += 4.0 + static_cast<double>(w) * m * n * 8.0 / 5.0e6;
+    if (w == lo || us < best_us) { best = w; best_us = us; }
+  }
+  return best;
 }
 
 // bytes of fp32 window results a projection of n rows over m tokens needs (0: one window, written directly)
 static size_t dense_parts_bytes(uint32_t m, uint32_t n, uint32_t k) {
-  const uint32_t n_win = dense_windows(k);
+  const uint32_t n_win = dense_windows(m, n, k);
   return n_win > 1 ? up256(sizeof(float) * static_cast<size_t>(m) * n) * n_win : 0;
 }
 // ... and of the gate / up pair of an MLP (both projections of a work item: kQmmRows rows each)
 static uint32_t dense_gate_up_windows(uint32_t d) {
-  return dense_windows(d, kDenseFusedMax);
+  return std::max(1u, (d / kGroup + kDenseFusedMax - 1) / kDenseFusedMax);
 }
 static size_t dense_gate_up_parts_bytes(uint32_t t, uint32_t f, uint32_t d) {
   const uint32_t n_win = dense_gate_up_windows(d);
@@ -2469,7 +2486,7 @@ size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
 // x_prepared: rows already in the matmul's order with their group sums in sumx (x is then ignored)
 static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, const uint16_t* xp, const float* sumx,
                                 void* y, uint32_t m, uint32_t n, uint32_t k, bool out_f32, void* parts) {
-  const uint32_t ng = k / kGroup, n_win = dense_windows(k);
+  const uint32_t ng = k / kGroup, n_win = dense_windows(m, n, k);
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
   QmmArgs d{};
   d.dense_mode = 1; d.dense_rows = m; d.top_k = 1;

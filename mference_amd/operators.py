@@ -250,7 +250,7 @@ class SharedExpertInt4:
 
     @staticmethod
     def scratch_bytes(d: int, f: int, t: int) -> int:
-        """bytes of scratch the call can use for t rows (the matrix-core path from 32 rows on)"""
+        """bytes of scratch the call can use for t rows (the matrix-core path beyond 8 rows)"""
         return int(_capi.lib().mf_shared_expert_scratch_bytes(d, f, t))
 
     def encode_static(self, x: torch.Tensor, gate: QuantizedTensor, up: QuantizedTensor,
