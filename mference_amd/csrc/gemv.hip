@@ -517,8 +517,11 @@ __device__ __forceinline__ f32x4_t mfma_quad(uint2 a, uint2 b, f32x4_t c) {
 
 constexpr uint32_t kQuadMaxWaves = 8;
 
-template <int NPROJ, int ITS>
+// BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group -- and its codes enter as 4 + q.
+template <int BITS, int NPROJ, int ITS>
 __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const RowsQuadArgs a) {
+  using chunk_t = std::conditional_t<BITS == kBits4, uint4, uint2>;
+  constexpr uint32_t kScaleStep = BITS == kBits4 ? 0x0200u : 0x0100u;  // bf16 exponent of the offset: 16 or 4
   // partial sums [buffer][projection][wave][16-lane row][weight row][token]
   __shared__ __attribute__((aligned(16))) float s_part[2][NPROJ][kQuadMaxWaves][4][4][4];
   // scale / bias pieces [wave][ring slot][(table, row, piece)][8 groups]
@@ -526,7 +529,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   const uint32_t lane = threadIdx.x & 63, wsub = threadIdx.x >> 6, wpr = blockDim.x >> 6;
   const uint32_t b = lane >> 2, c = lane & 3;
   const uint32_t n_chunks = a.N / 32, ng = a.N / kGroup, n_sets = a.M / 4;
-  const size_t row_bytes = static_cast<size_t>(a.N) / 2;
+  const size_t row_bytes = static_cast<size_t>(a.N) * BITS / 8;
 
   // chunk of every slot of this lane: (wsub * ITS + j) * 16 + b
   uint32_t chc[ITS];
@@ -544,7 +547,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   // piece goes to the wave's own LDS area when that stage ends, and a lane picks the two values of
   // each slot from there (LDS reads cost no vector-memory issue slot,
   // which is what limits this kernel).
-  uint4 cw[2][ITS];
+  chunk_t cw[2][ITS];
   // (lanes past 8 * ITS fetch and store a copy nobody reads: no branch around the load)
   const uint32_t tb_lane = lane % (8 * ITS);
   const uint32_t tb_bias = tb_lane / (4 * ITS), tb_row = (tb_lane / ITS) & 3u, tb_piece = tb_lane % ITS;
@@ -553,7 +556,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   uint16_t* my_tab = &s_tab[wsub][0][0];
   auto fetch = [&](int buf, int j, uint32_t set, int p) __attribute__((always_inline)) {
     const size_t row = static_cast<size_t>(set) * 4 + c;
-    cw[buf][j] = *reinterpret_cast<const uint4*>(a.W[p] + row * row_bytes + static_cast<size_t>(chc[j]) * 16);
+    cw[buf][j] = *reinterpret_cast<const chunk_t*>(a.W[p] + row * row_bytes + static_cast<size_t>(chc[j]) * sizeof(chunk_t));
   };
   auto fetch_tables = [&](uint32_t set, int p) __attribute__((always_inline)) {
     return *reinterpret_cast<const uint4*>((tb_bias ? a.B[p] : a.S[p]) + (static_cast<size_t>(set) * 4 + tb_row) * ng +
@@ -569,19 +572,32 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
     uint4 tbn = make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < ITS; ++j) {
-      const uint32_t w[4] = {cw[buf][j].x, cw[buf][j].y, cw[buf][j].z, cw[buf][j].w};
       f32x4_t tmp = {0.0f, 0.0f, 0.0f, 0.0f};
+      if constexpr (BITS == kBits4) {
+        const uint32_t w[4] = {cw[buf][j].x, cw[buf][j].y, cw[buf][j].z, cw[buf][j].w};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint4 e = expand_q4(w[i]);
-        tmp = mfma_quad(xa[j][2 * i], make_uint2(e.x, e.y), tmp);
-        tmp = mfma_quad(xa[j][2 * i + 1], make_uint2(e.z, e.w), tmp);
+        for (int i = 0; i < 4; ++i) {
+          const uint4 e = expand_q4(w[i]);
+          tmp = mfma_quad(xa[j][2 * i], make_uint2(e.x, e.y), tmp);
+          tmp = mfma_quad(xa[j][2 * i + 1], make_uint2(e.z, e.w), tmp);
+        }
+      } else {
+        const uint32_t w[2] = {cw[buf][j].x, cw[buf][j].y};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          uint4 e, f;
+          expand_q2(w[i], e, f);
+          tmp = mfma_quad(xa[j][4 * i], make_uint2(e.x, e.y), tmp);
+          tmp = mfma_quad(xa[j][4 * i + 1], make_uint2(e.z, e.w), tmp);
+          tmp = mfma_quad(xa[j][4 * i + 2], make_uint2(f.x, f.y), tmp);
+          tmp = mfma_quad(xa[j][4 * i + 3], make_uint2(f.z, f.w), tmp);
+        }
       }
       const uint32_t sb = tab[((c * ITS) + j) * 8 + (b >> 1)], bb = tab[(((4 + c) * ITS) + j) * 8 + (b >> 1)];
-      const uint32_t ms = ((sb + 0x0200u) ^ 0x8000u) & 0xFFFFu;  // -16 s: exponent + 4, sign flipped
+      const uint32_t ms = ((sb + kScaleStep) ^ 0x8000u) & 0xFFFFu;  // -16 s (-4 s): exponent + 4 (2), sign flipped
       acc = mfma_quad(sx[j], make_uint2(bb | (bb << 16), bb), acc);
       acc = mfma_quad(sx[j], make_uint2(ms | (ms << 16), ms), acc);
-      const float s2 = 2.0f * __uint_as_float(sb << 16);
+      const float s2 = (BITS == kBits4 ? 2.0f : 1.0f) * __uint_as_float(sb << 16);
       fetch(buf, j, refill, p);
       if (j == 0) tbn = fetch_tables(refill, p);
 #pragma unroll
@@ -896,7 +912,7 @@ bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipErr
 // The quad kernel takes 4-bit matrices with at least 1024 rows (a multiple of 4) and up to 4
 // token rows when the 32-element chunks of a row split over (waves, ITS slots of 16 chunks)
 // with little waste.
-template <int NPROJ>
+template <int BITS, int NPROJ>
 bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipError_t& err) {
   if (a.N % (8 * kGroup) || a.T < 1 || a.T > 4 || a.M < 1024 || a.M % 4) return false;
   const uint32_t chunks = a.N / 32;
@@ -911,11 +927,34 @@ bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipErr
   const uint32_t n_sets = a.M / 4;
   const uint32_t grid = std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / best_wpr));
   const dim3 block(best_wpr * 64);
-  if (best_its == 4) rows_quad_kernel<NPROJ, 4><<<dim3(grid), block, 0, s>>>(a);
-  else if (best_its == 5) rows_quad_kernel<NPROJ, 5><<<dim3(grid), block, 0, s>>>(a);
-  else rows_quad_kernel<NPROJ, 6><<<dim3(grid), block, 0, s>>>(a);
+  if (best_its == 4) rows_quad_kernel<BITS, NPROJ, 4><<<dim3(grid), block, 0, s>>>(a);
+  else if (best_its == 5) rows_quad_kernel<BITS, NPROJ, 5><<<dim3(grid), block, 0, s>>>(a);
+  else rows_quad_kernel<BITS, NPROJ, 6><<<dim3(grid), block, 0, s>>>(a);
   err = hipGetLastError();
   return true;
+}
+
+// Up to four token rows in one launch.  Five to eight: two launches, rows 0..3 and the
+// rest.  The quad kernel runs the same instructions for a token whatever rides along, so every row
+// keeps the bits of a single-token call (MultiXKernelParityTests.swift:50-77); the weights stream
+// twice.  (y rows are M elements apart, 2 or 4 bytes each: 16-byte aligned since M % 4 == 0.)
+template <int NPROJ>
+bool rows_quad_any(hipStream_t s, int bits, const RowsQuadArgs& a, hipError_t& err) {
+  if (a.T > 8) return false;
+  // one row of 2-bit weights that rows_stream_kernel takes in one step of a wave is faster there
+  // (6656 x 2048, two projections: 13 us against 17; 5120 x 17408: 59 us for the MLP there, 38 here)
+  if (bits == kBits2 && a.T == 1 && a.N <= 4096) return false;
+  for (uint32_t t0 = 0; t0 < a.T; t0 += 4) {
+    RowsQuadArgs q = a;
+    q.T = std::min(a.T - t0, 4u);
+    q.x = a.x + static_cast<size_t>(t0) * a.N;
+    q.y = static_cast<uint8_t*>(a.y) + static_cast<size_t>(t0) * a.M * (a.out_f32 ? 4 : 2);
+    const bool took = bits == kBits4 ? rows_quad_try<kBits4, NPROJ>(s, q, device_cu_count(), err)
+                                     : rows_quad_try<kBits2, NPROJ>(s, q, device_cu_count(), err);
+    if (!took) return false;  // (the shape decides: the first launch is refused or none is)
+    if (err != hipSuccess) return true;
+  }
+  return a.T > 0;
 }
 
 }  // namespace
@@ -934,32 +973,18 @@ hipError_t launch_gemv(hipStream_t s, const mf_qtensor& w, int bits, const uint1
     return hipGetLastError();
   }
   const bool al = aligned16(w.weights) && aligned16(x);
+  if (!lane_order && al && (bits == kBits4 || bits == kBits2) && aligned16(w.scales) && aligned16(w.biases)) {
+    RowsQuadArgs qa{};
+    qa.W[0] = static_cast<const uint8_t*>(w.weights); qa.S[0] = w.scales; qa.B[0] = w.biases;
+    qa.x = x; qa.y = y; qa.M = m; qa.N = n; qa.T = t; qa.out_f32 = out_f32 ? 1 : 0;
+    hipError_t err = hipSuccess;
+    if (rows_quad_any<1>(s, bits, qa, err)) return err;
+  }
   if (!lane_order && al && bits == kBits4 && aligned16(w.scales) && aligned16(w.biases)) {
     RowsMfmaArgs ma{};
     ma.W[0] = static_cast<const uint8_t*>(w.weights); ma.S[0] = w.scales; ma.B[0] = w.biases;
     ma.x = x; ma.y = y; ma.M = m; ma.N = n; ma.T = t; ma.out_f32 = out_f32 ? 1 : 0;
     hipError_t err = hipSuccess;
-    RowsQuadArgs qa{};
-    qa.W[0] = ma.W[0]; qa.S[0] = ma.S[0]; qa.B[0] = ma.B[0];
-    qa.x = x; qa.y = y; qa.M = m; qa.N = n; qa.T = t; qa.out_f32 = ma.out_f32;
-    if (rows_quad_try<1>(s, qa, device_cu_count(), err)) return err;
-    // Five to eight token rows of a matrix the quad kernel takes: two launches, rows 0..3 and the
-    // rest.  The quad kernel runs the same instructions for a token whatever rides along, so every row
-    // keeps the bits of a single-token call (MultiXKernelParityTests.swift:50-77); the weights stream
-    // twice.  (y rows are m elements apart, 2 or 4 bytes each: 16-byte aligned since m % 4 == 0 and t > 4
-    // only reaches here with m >= 1024.)
-    if (t > 4 && t <= 8) {
-      RowsQuadArgs q0 = qa, q1 = qa;
-      q0.T = 4;
-      q1.T = t - 4;
-      q1.x = x + static_cast<size_t>(4) * n;
-      q1.y = static_cast<uint8_t*>(y) + static_cast<size_t>(4) * m * (out_f32 ? 4 : 2);
-      if (rows_quad_try<1>(s, q0, device_cu_count(), err)) {
-        if (err != hipSuccess) return err;
-        if (rows_quad_try<1>(s, q1, device_cu_count(), err)) return err;
-        return hipErrorUnknown;  // (not reached: the second launch has the shape of the first)
-      }
-    }
     if (rows_mfma_try<1>(s, ma, device_cu_count(), err)) return err;
   }
   if (!lane_order && al && (bits == kBits4 || bits == kBits2)) {
@@ -989,29 +1014,21 @@ hipError_t launch_gate_up_act(hipStream_t s, const mf_qtensor& gate, const mf_qt
                               int bits, const uint16_t* x, uint16_t* act, uint32_t f, uint32_t d,
                               uint32_t t, bool lane_order) {
   const bool al = aligned16(gate.weights) && aligned16(up.weights) && aligned16(x);
-  if (!lane_order && al && bits == kBits4 && aligned16(gate.scales) && aligned16(gate.biases) && aligned16(up.scales) &&
-      aligned16(up.biases)) {
+  const bool tables = aligned16(gate.scales) && aligned16(gate.biases) && aligned16(up.scales) && aligned16(up.biases);
+  if (!lane_order && al && tables && (bits == kBits4 || bits == kBits2)) {
+    RowsQuadArgs qa{};
+    qa.W[0] = static_cast<const uint8_t*>(gate.weights); qa.S[0] = gate.scales; qa.B[0] = gate.biases;
+    qa.W[1] = static_cast<const uint8_t*>(up.weights); qa.S[1] = up.scales; qa.B[1] = up.biases;
+    qa.x = x; qa.y = act; qa.M = f; qa.N = d; qa.T = t;
+    hipError_t err = hipSuccess;
+    if (rows_quad_any<2>(s, bits, qa, err)) return err;
+  }
+  if (!lane_order && al && tables && bits == kBits4) {
     RowsMfmaArgs ma{};
     ma.W[0] = static_cast<const uint8_t*>(gate.weights); ma.S[0] = gate.scales; ma.B[0] = gate.biases;
     ma.W[1] = static_cast<const uint8_t*>(up.weights); ma.S[1] = up.scales; ma.B[1] = up.biases;
     ma.x = x; ma.y = act; ma.M = f; ma.N = d; ma.T = t;
     hipError_t err = hipSuccess;
-    RowsQuadArgs qa{};
-    for (int p = 0; p < 2; ++p) { qa.W[p] = ma.W[p]; qa.S[p] = ma.S[p]; qa.B[p] = ma.B[p]; }
-    qa.x = x; qa.y = act; qa.M = f; qa.N = d; qa.T = t;
-    if (rows_quad_try<2>(s, qa, device_cu_count(), err)) return err;
-    if (t > 4 && t <= 8) {  // as in launch_gemv: rows 0..3, then the rest, same bits as single-token calls
-      RowsQuadArgs q0 = qa, q1 = qa;
-      q0.T = 4;
-      q1.T = t - 4;
-      q1.x = x + static_cast<size_t>(4) * d;
-      q1.y = act + static_cast<size_t>(4) * f;
-      if (rows_quad_try<2>(s, q0, device_cu_count(), err)) {
-        if (err != hipSuccess) return err;
-        if (rows_quad_try<2>(s, q1, device_cu_count(), err)) return err;
-        return hipErrorUnknown;
-      }
-    }
     if (rows_mfma_try<2>(s, ma, device_cu_count(), err)) return err;
   }
   if (!lane_order && al && (bits == kBits4 || bits == kBits2)) {
