@@ -518,7 +518,8 @@ __device__ __forceinline__ f32x4_t mfma_quad(uint2 a, uint2 b, f32x4_t c) {
 constexpr uint32_t kQuadMaxWaves = 8;
 
 // BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group -- and its codes enter as 4 + q.
-template <int BITS, int NPROJ, int ITS>
+// ANY: K is any multiple of 64; otherwise of 512, so that the table pieces are whole and aligned.
+template <int BITS, int NPROJ, int ITS, bool ANY>
 __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const RowsQuadArgs a) {
   using chunk_t = std::conditional_t<BITS == kBits4, uint4, uint2>;
   constexpr uint32_t kScaleStep = BITS == kBits4 ? 0x0200u : 0x0100u;  // bf16 exponent of the offset: 16 or 4
@@ -552,15 +553,17 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   const uint32_t tb_lane = lane % (8 * ITS);
   const uint32_t tb_bias = tb_lane / (4 * ITS), tb_row = (tb_lane / ITS) & 3u, tb_piece = tb_lane % ITS;
   const uint32_t tb_g = (wsub * ITS + tb_piece) * 8;
-  const uint32_t tb_group = tb_g < ng ? tb_g : 0u;  // a piece past the row is never used: read piece 0
+  // a piece past the row is never used: read piece 0.  ANY: the row's last piece ends with the row and is moved down
+  const uint32_t tb_group = tb_g >= ng ? 0u : ANY ? min(tb_g, ng - 8u) : tb_g;
+  const uint32_t tb_drop = ANY && tb_g < ng ? tb_g - tb_group : 0u;
   uint16_t* my_tab = &s_tab[wsub][0][0];
   auto fetch = [&](int buf, int j, uint32_t set, int p) __attribute__((always_inline)) {
     const size_t row = static_cast<size_t>(set) * 4 + c;
     cw[buf][j] = *reinterpret_cast<const chunk_t*>(a.W[p] + row * row_bytes + static_cast<size_t>(chc[j]) * sizeof(chunk_t));
   };
   auto fetch_tables = [&](uint32_t set, int p) __attribute__((always_inline)) {
-    return *reinterpret_cast<const uint4*>((tb_bias ? a.B[p] : a.S[p]) + (static_cast<size_t>(set) * 4 + tb_row) * ng +
-                                           tb_group);
+    const uint16_t* piece = (tb_bias ? a.B[p] : a.S[p]) + (static_cast<size_t>(set) * 4 + tb_row) * ng + tb_group;
+    return ANY ? load_16_bytes(piece) : *reinterpret_cast<const uint4*>(piece);
   };
   // the wave's part of D[token, row] for one row set; then the four blocks of each 16-lane row
   // are added and lanes 0..3 of the row leave [weight row][token] in LDS.  `refill` is the row
@@ -605,7 +608,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
     }
     // every read of this ring slot's tables is issued: the refill stage's pieces take their place
     __builtin_amdgcn_wave_barrier();
-    *reinterpret_cast<uint4*>(tab + lane * 8) = tbn;
+    *reinterpret_cast<uint4*>(tab + lane * 8) = ANY ? drop_bf16(tbn, tb_drop) : tbn;
     float v[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -677,8 +680,8 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
     sx[j] = make_uint2((hi >> 16) | mid, lo >> 16);  // K slots: hi, mid, lo, 0
   }
 
-  *reinterpret_cast<uint4*>(my_tab + lane * 8) = t0;
-  *reinterpret_cast<uint4*>(my_tab + 64 * 8 + lane * 8) = t1;
+  *reinterpret_cast<uint4*>(my_tab + lane * 8) = ANY ? drop_bf16(t0, tb_drop) : t0;
+  *reinterpret_cast<uint4*>(my_tab + 64 * 8 + lane * 8) = ANY ? drop_bf16(t1, tb_drop) : t1;
   if constexpr (NPROJ == 2) {
     for (; set < n_sets; set += G) {
       const uint32_t nxt = min(set + G, last);
@@ -909,27 +912,43 @@ bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipErr
   return true;
 }
 
-// The quad kernel takes 4-bit matrices with at least 1024 rows (a multiple of 4) and up to 4
-// token rows when the 32-element chunks of a row split over (waves, ITS slots of 16 chunks)
-// with little waste.
+// The quad kernel takes 4-bit and 2-bit matrices with at least 1024 rows (a multiple of 4) and up to 4
+// token rows.  The 32-element chunks of a row split over (waves, ITS slots of 16 chunks).  K a multiple of 512 that splits
+// with little waste: any number of rows.  `any_k`: any other K, the split that costs the fewest
+// slots, a stage of a wave counted as one more.
 template <int BITS, int NPROJ>
-bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipError_t& err) {
-  if (a.N % (8 * kGroup) || a.T < 1 || a.T > 4 || a.M < 1024 || a.M % 4) return false;
+bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, bool any_k, uint32_t num_cu, hipError_t& err) {
+  if (a.N % kGroup || a.N < 8 * kGroup || a.T < 1 || a.T > 4 || a.M < 1024 || a.M % 4) return false;
   const uint32_t chunks = a.N / 32;
-  uint32_t best_its = 0, best_wpr = 0, best_waste = ~0u;
-  for (uint32_t its = 6; its >= 4; --its) {
-    const uint32_t wpr = (chunks + 16 * its - 1) / (16 * its);
-    if (wpr > kQuadMaxWaves) continue;
-    const uint32_t waste = 16 * its * wpr - chunks;
-    if (waste < best_waste) { best_waste = waste; best_its = its; best_wpr = wpr; }
+  uint32_t its = 0, wpr = 0, waste = ~0u;
+  for (uint32_t i = 6; i >= 4; --i) {
+    const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
+    if (w > kQuadMaxWaves) continue;
+    if (16 * i * w - chunks < waste) { waste = 16 * i * w - chunks; its = i; wpr = w; }
   }
-  if (!best_its || best_waste * 10 > chunks) return false;
+  const bool fits = a.N % (8 * kGroup) == 0 && its && waste * 10 <= chunks;
+  if (!fits) {
+    if (!any_k) return false;
+    uint32_t cost = ~0u;
+    for (uint32_t i = 6; i >= 2; --i) {
+      const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
+      if (w <= kQuadMaxWaves && w * (i + 1) < cost) { cost = w * (i + 1); its = i; wpr = w; }
+    }
+    if (cost == ~0u) return false;
+  }
   const uint32_t n_sets = a.M / 4;
-  const uint32_t grid = std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / best_wpr));
-  const dim3 block(best_wpr * 64);
-  if (best_its == 4) rows_quad_kernel<BITS, NPROJ, 4><<<dim3(grid), block, 0, s>>>(a);
-  else if (best_its == 5) rows_quad_kernel<BITS, NPROJ, 5><<<dim3(grid), block, 0, s>>>(a);
-  else rows_quad_kernel<BITS, NPROJ, 6><<<dim3(grid), block, 0, s>>>(a);
+  const dim3 grid(std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / wpr))), block(wpr * 64);
+  if (fits) {
+    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, false><<<grid, block, 0, s>>>(a);
+    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, false><<<grid, block, 0, s>>>(a);
+    else rows_quad_kernel<BITS, NPROJ, 6, false><<<grid, block, 0, s>>>(a);
+  } else {
+    if (its == 2) rows_quad_kernel<BITS, NPROJ, 2, true><<<grid, block, 0, s>>>(a);
+    else if (its == 3) rows_quad_kernel<BITS, NPROJ, 3, true><<<grid, block, 0, s>>>(a);
+    else if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, 0, s>>>(a);
+    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, true><<<grid, block, 0, s>>>(a);
+    else rows_quad_kernel<BITS, NPROJ, 6, true><<<grid, block, 0, s>>>(a);
+  }
   err = hipGetLastError();
   return true;
 }
@@ -941,16 +960,29 @@ bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipErr
 template <int NPROJ>
 bool rows_quad_any(hipStream_t s, int bits, const RowsQuadArgs& a, hipError_t& err) {
   if (a.T > 8) return false;
-  // one row of 2-bit weights that rows_stream_kernel takes in one step of a wave is faster there
-  // (6656 x 2048, two projections: 13 us against 17; 5120 x 17408: 59 us for the MLP there, 38 here)
-  if (bits == kBits2 && a.T == 1 && a.N <= 4096) return false;
+  const bool two = bits == kBits2;
+  // One row of 2-bit weights that rows_stream_kernel takes in one step of a wave is faster there
+  // (6656 x 2048, two projections: 13 us against 17; 5120 x 17408: 59 us for the MLP there, 38 here).
+  const uint32_t step = two ? 4096 : 2048, steps = (a.N + step - 1) / step;
+  if (two && a.T == 1 && steps == 1) return false;
+  // Where a K that is no multiple of 512, or splits badly, goes (us per MLP, other kernels / this one):
+  // one row: where a step of rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3;
+  // 3840 x 7680, a sixteenth empty: 22.2 / 22.9); two to four (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25;
+  // 2048 x 6656: 23.5 / 21.7); more: where the weights outweigh two launches (five rows, 2816 x 4096: 29.5 / 31.5;
+  // 3328 x 8192: 46.5 / 42.8; 2-bit, 1088 x 2112: 18.9 / 19.9, 1984 x 5056: 33.6 / 28.0).  Small matrices stay with the
+  // kernels whose rows have the bits of single-token calls for every number of rows.
+  const uint64_t weights = static_cast<uint64_t>(a.M) * a.N * NPROJ;
+  const bool wide = weights >= (two ? 8ull : 24ull) * 1000000;
+  const bool any_k = a.T == 1 ? wide && a.N * 5ull < steps * static_cast<uint64_t>(step) * 4
+                   : a.T <= 4 ? weights >= 4000000
+                              : wide;
   for (uint32_t t0 = 0; t0 < a.T; t0 += 4) {
     RowsQuadArgs q = a;
     q.T = std::min(a.T - t0, 4u);
     q.x = a.x + static_cast<size_t>(t0) * a.N;
     q.y = static_cast<uint8_t*>(a.y) + static_cast<size_t>(t0) * a.M * (a.out_f32 ? 4 : 2);
-    const bool took = bits == kBits4 ? rows_quad_try<kBits4, NPROJ>(s, q, device_cu_count(), err)
-                                     : rows_quad_try<kBits2, NPROJ>(s, q, device_cu_count(), err);
+    const bool took = bits == kBits4 ? rows_quad_try<kBits4, NPROJ>(s, q, any_k, device_cu_count(), err)
+                                     : rows_quad_try<kBits2, NPROJ>(s, q, any_k, device_cu_count(), err);
     if (!took) return false;  // (the shape decides: the first launch is refused or none is)
     if (err != hipSuccess) return true;
   }

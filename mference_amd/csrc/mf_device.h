@@ -464,6 +464,22 @@ __device__ __forceinline__ void group_products(const QmmCodes<BITS, SWAPPED>& c,
   }
 }
 
+// 16 bytes from any address the element type allows (global memory takes unaligned vector loads)
+__device__ __forceinline__ uint4 load_16_bytes(const void* p) {
+  uint4 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+// eight bf16 numbers without the first n (0..7); zeros follow
+__device__ __forceinline__ uint4 drop_bf16(uint4 v, uint32_t n) {
+  if (n & 4u) v = make_uint4(v.z, v.w, 0, 0);
+  if (n & 2u) v = make_uint4(v.y, v.z, v.w, 0);
+  if (n & 1u)
+    v = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                   __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+  return v;
+}
+
 // 8 bf16 from p, of which only the first `avail` exist (the rest read as 0)
 __device__ __forceinline__ uint4 load_bf16x8_guarded(const uint16_t* p, uint32_t avail) {
   if (avail >= 8) return load_x8<false>(p);

@@ -1063,22 +1063,6 @@ __device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint3
   if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
 }
 
-// 16 bytes from any address the element type allows (global memory takes unaligned vector loads)
-__device__ __forceinline__ uint4 load_16_bytes(const void* p) {
-  uint4 v;
-  __builtin_memcpy(&v, p, 16);
-  return v;
-}
-// eight bf16 numbers without the first n (0..7); zeros follow
-__device__ __forceinline__ uint4 drop_bf16(uint4 v, uint32_t n) {
-  if (n & 4u) v = make_uint4(v.z, v.w, 0, 0);
-  if (n & 2u) v = make_uint4(v.y, v.z, v.w, 0);
-  if (n & 1u)
-    v = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
-                   __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
-  return v;
-}
-
 // silu with the hardware exp2 / reciprocal (1 ulp each): the result is narrowed to bf16 right after
 __device__ __forceinline__ float fast_silu(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));

@@ -171,6 +171,35 @@ def test_gemv_quad_rows_kernel(gpu, oracle, m, n, t):
     assert np.array_equal(y2.cpu().numpy().view(np.uint32), got.view(np.uint32))
 
 
+@pytest.mark.parametrize("bits,m,n,t", [
+    (4, 7936, 512, 2), (2, 7040, 576, 3),     # the fewest groups; one more than a table piece
+    (4, 1280, 3136, 4), (2, 1284, 3136, 2),   # a last piece of one group
+    (4, 1024, 6656, 3), (2, 1100, 7616, 4),   # ragged last slots; seven groups in the last piece
+    (2, 1024, 8256, 8), (4, 3072, 8128, 7),   # two launches
+    (4, 7680, 3136, 1), (2, 1792, 4672, 1),
+])
+def test_gemv_quad_rows_kernel_at_any_k(gpu, oracle, bits, m, n, t):
+    """the quad kernel where K does not split evenly, 4-bit and 2-bit; up to four rows of a call keep the bits
+    of a two-row call"""
+    rng = oracle.Rng.key(0xF6, f"quad-any-{bits}-{m}-{n}-{t}")
+    q = oracle.quantize(rng.uniform_fill(-1.0, 1.0, m * n).reshape(m, n), bits)
+    x = oracle.bf16_bits(rng.uniform_fill(-1.0, 1.0, t * n).reshape(t, n))
+    ref = oracle.gemv_multix(q, x)
+    xd = ops.bf16_tensor(x)
+    g = ops.DequantInt4GEMVMultiX(gpu)
+    dq = to_device_q(q)
+    y = torch.full((t, m), 7.0, dtype=torch.float32, device="cuda")
+    g.encode(dq, xd, y, m, n, t, output_float32=True)
+    _sync()
+    got = y.cpu().numpy()
+    assert np.abs(got - ref).max() / max(np.abs(ref).max(), 1e-6) < 2e-5
+    if 2 <= t <= 4:
+        y2 = torch.zeros((2, m), dtype=torch.float32, device="cuda")
+        g.encode(dq, xd[t - 2:].contiguous(), y2, m, n, 2, output_float32=True)
+        _sync()
+        assert np.array_equal(y2.cpu().numpy().view(np.uint32), got[t - 2:].view(np.uint32))
+
+
 @pytest.mark.parametrize("d,f,t", [(2048, 1024, 1), (5120, 1536, 4)])
 def test_shared_expert_streaming_rows_kernel(gpu, oracle, d, f, t):
     """dense SwiGLU MLP wide enough for the streaming gate/up and down kernels"""
