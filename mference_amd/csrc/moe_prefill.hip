@@ -1388,14 +1388,13 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 
   // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
   const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
-  // inside a 32-token block the column is rotated by 4 * ((s >> 1) + 2h): the four lanes that
-  // stage one token then hit four different bank groups
-  const uint32_t st_rot = 4 * ((c0 & 3) >> 1) + 8 * (c0 >> 2);
-  const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + st_rot) & 31);
-  const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + st_rot) & 31);
+  // inside a 32-token block the column is rotated by 2 * (s + 4h): the 16 lanes that store together -- four runs
+  // of four tokens, or eight of two -- hit sixteen different bank groups
+  const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + 2 * c0) & 31);
+  const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + 2 * c1) & 31);
   uint32_t rd_col[4];
 #pragma unroll
-  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 4 * (sidx >> 1) + 8 * h) & 31;
+  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 2 * sidx + 8 * h) & 31;
 #pragma unroll
   for (int gi = 0; gi < 2; ++gi) {
     *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot0) = x0[gi][0];
