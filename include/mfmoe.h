@@ -175,10 +175,12 @@ mf_status mf_residual_rmsnorm(mf_ctx* ctx, mf_stream stream, uint16_t* hidden, c
  * [m, k], y bf16 [m, n] (fp32 when out_f32 != 0), k a multiple of 64, any m and n.  With n and k
  * multiples of 128, 16-byte aligned w.weights / x / y and a 16-byte aligned workspace of at least
  * mf_qmm_workspace_bytes(m, n, k) the call runs on the matrix cores (codes expanded to exact bf16 in
- * registers, one fp32 scale multiply per 64-wide K group -- the kernel of mf_moe_prefill_layer; a K
- * beyond 4096 is cut into windows whose fp32 results are added in order); every other shape,
- * alignment or workspace runs row by row through the kernels of mf_gemv, bit-identical to
- * mf_gemv.  Where the reference returns .unavailable (bad sizes or offsets) the call returns a
+ * registers, one fp32 scale multiply per 64-wide K group -- the kernel of mf_moe_prefill_layer; K may
+ * be cut into windows whose fp32 results are added in order, as many as n, k and the number of 64-row
+ * tiles of m ask for, never the size of the workspace: a row has the same bits in every block of that
+ * many tiles, and may differ in the last place of the fp32 sum in a block of another number); every other
+ * shape, alignment or workspace runs row by row through the kernels of mf_gemv, bit-identical to
+ * mf_gemv.  A workspace of mf_qmm_workspace_bytes(m, n, k) bytes serves every smaller m of the same n and k too.  Where the reference returns .unavailable (bad sizes or offsets) the call returns a
  * negative status and launches nothing.  Replaces the 4-bit, 2-bit and ternary projections alike. */
 size_t mf_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k);
 mf_status mf_qmm(mf_ctx* ctx, mf_stream stream, mf_qtensor w, mf_bits bits, const uint16_t* x, void* y, uint32_t m,
@@ -199,7 +201,7 @@ int mf_qmm_path(mf_qtensor w, mf_bits bits, const uint16_t* x, const void* y, ui
  * PrefillSharedExpert.swift:81-190) / encodeDenseMLPPrefill (Qwen38ForwardRunner.swift:862-913):
  * beyond MF_MAX_TOKENS rows (small 4-bit shapes: from 16 rows on) the projections run on the matrix cores when d and f
  * are at least 128, the operands are 16-byte aligned and scratch_act holds mf_shared_expert_scratch_bytes(d, f, t)
- * bytes; otherwise row by row, MF_MAX_TOKENS rows per pair of launches, for which t*f bf16 of scratch suffice (all
+ * bytes (which serve every smaller t of the same d and f too; K windows and the bits of a row as for mf_qmm); otherwise row by row, MF_MAX_TOKENS rows per pair of launches, for which t*f bf16 of scratch suffice (all
  * that t <= MF_MAX_TOKENS ever needs). */
 size_t mf_shared_expert_scratch_bytes(uint32_t d, uint32_t f, uint32_t t);
 mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_qtensor gate,

@@ -197,7 +197,7 @@ mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_
   // 5120 x 17408, 9 rows 121 / 77, 31 rows 329 / 81, 2-bit 1522 / 72)
   const bool few = bits == MF_BITS_4 && t < 16 && static_cast<uint64_t>(t) * d * f < (64ull << 20);
   if (t > MF_MAX_TOKENS && !few && mf::dense_mlp_takes(gate, up, down, x, y, scratch_act, d, f, t) &&
-      scratch_act_bytes >= mf::dense_mlp_scratch_bytes(d, f, t)) {
+      scratch_act_bytes >= mf::dense_mlp_needs(d, f, t)) {
     MF_HIP(ctx, mf::launch_dense_mlp(s, gate, up, down, bits, x, y, d, f, t, scratch_act));
     return MF_OK;
   }
@@ -247,7 +247,7 @@ static int qmm_path(mf_qtensor w, mf_bits bits, const uint16_t* x, const void* y
   if (m == 0 || n == 0 || k == 0 || k % MF_GROUP_SIZE != 0 || m > MF_MAX_ROWS) return MF_ERR_DIMENSION_MISMATCH;
   if (!qtensor_ok(w, bits) || !mf::aligned2(x) || !mf::aligned2(y)) return MF_ERR_INVALID_ARGUMENT;
   if (workspace && mf::aligned16(workspace) && mf::dense_qmm_takes(w, bits, x, y, m, n, k) &&
-      workspace_bytes >= mf::dense_qmm_workspace_bytes(m, n, k))
+      workspace_bytes >= mf::dense_qmm_needs(m, n, k))
     return MF_QMM_PATH_MATRIX_CORE;
   return MF_QMM_PATH_ROWS;
 }

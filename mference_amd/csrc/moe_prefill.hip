@@ -2376,27 +2376,46 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(const float* __restr
 // empty.  Two items share a CU; an item costs about 3.6 us per 8 groups and 4.7 for its set-up, the
 // windows' sums their bytes and a launch (fitted to n = 5120, k = 17408, m = 32 .. 512: the choice is the best
 // or within 2 % of it; m = 32, 5 -> 12 windows, 101 -> 87 us for the MLP; m = 150, 5 -> 7, 172 -> 158; m = 512, 5 -> 6, 401 -> 389).
-static uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k) {
-  constexpr uint32_t kSlots = 2 * 256;
-  const uint32_t ng = k / kGroup, steps = (ng + 7) / 8;
+// The choice follows the number of 64-row tiles, not m: a row's sums come out the same in every block of that many tiles.
+// From kWholeRounds rounds of the fewest windows on an emptier last round is no longer worth the windows' bytes.
+constexpr uint32_t kWindowSlots = 2 * 256, kWholeRounds = 8;
+static uint32_t dense_tile_items(uint32_t n) {
   const uint32_t slice_rows = n % (2 * kQmmRows) == 0 ? 2 * kQmmRows : kQmmRows;
-  const uint64_t items = static_cast<uint64_t>((m + kTileTokens - 1) / kTileTokens) * ((n + slice_rows - 1) / slice_rows);
-  const uint32_t lo = std::max(1u, (ng + kDenseWindow - 1) / kDenseWindow), hi = std::max(lo, ng / 8);
+  return (n + slice_rows - 1) / slice_rows;
+}
+static uint32_t dense_fewest_windows(uint32_t k) { return std::max(1u, (k / kGroup + kDenseWindow - 1) / kDenseWindow); }
+static uint32_t dense_windows_of_tiles(uint32_t tiles, uint32_t n, uint32_t k) {
+  const uint32_t ng = k / kGroup, steps = (ng + 7) / 8;
+  const uint64_t items = static_cast<uint64_t>(tiles) * dense_tile_items(n);
+  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, ng / 8);
+  if (items * lo >= kWholeRounds * kWindowSlots) return lo;
   uint32_t best = lo;
   double best_us = 0.0;
   for (uint32_t w = lo; w <= hi; ++w) {
-    const double rounds = static_cast<double>((items * w + kSlots - 1) / kSlots);
+    const double rounds = static_cast<double>((items * w + kWindowSlots - 1) / kWindowSlots);
     double us = rounds * (3.6 * ((steps + w - 1) / w) + 4.7);
-    if (w > 1) us += 4.0 + static_cast<double>(w) * m * n * 8.0 / 5.0e6;
+    if (w > 1) us += 4.0 + static_cast<double>(w) * tiles * kTileTokens * n * 8.0 / 5.0e6;
     if (w == lo || us < best_us) { best = w; best_us = us; }
   }
   return best;
+}
+static uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k) {
+  return dense_windows_of_tiles((m + kTileTokens - 1) / kTileTokens, n, k);
 }
 
 // bytes of fp32 window results a projection of n rows over m tokens needs (0: one window, written directly)
 static size_t dense_parts_bytes(uint32_t m, uint32_t n, uint32_t k) {
   const uint32_t n_win = dense_windows(m, n, k);
   return n_win > 1 ? up256(sizeof(float) * static_cast<size_t>(m) * n) * n_win : 0;
+}
+// ... and the most any call of up to m tokens needs: fewer tiles can take more windows, so the bytes of a single call do
+// not grow with its rows (5120 x 17408: 37.4 MB for 128 rows, 24.5 for 129).  Only tile counts below kWholeRounds differ.
+static size_t dense_parts_bytes_up_to(uint32_t m, uint32_t n, uint32_t k) {
+  size_t most = dense_parts_bytes(m, n, k);
+  const uint64_t row = static_cast<uint64_t>(dense_tile_items(n)) * dense_fewest_windows(k);
+  const uint32_t tiles = static_cast<uint32_t>(std::min<uint64_t>((m - 1) / kTileTokens, kWholeRounds * kWindowSlots / row + 1));
+  for (uint32_t i = 1; i <= tiles; ++i) most = std::max(most, dense_parts_bytes(i * kTileTokens, n, k));
+  return most;
 }
 // ... and of the gate / up pair of an MLP (both projections of a work item: kQmmRows rows each)
 static uint32_t dense_gate_up_windows(uint32_t d) {
@@ -2461,9 +2480,12 @@ bool dense_qmm_takes(const mf_qtensor& w, int bits, const void* x, const void* y
   return true;
 }
 
+static size_t dense_qmm_rows_bytes(uint32_t m, uint32_t k) {
+  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup));
+}
+size_t dense_qmm_needs(uint32_t m, uint32_t n, uint32_t k) { return dense_qmm_rows_bytes(m, k) + dense_parts_bytes(m, n, k); }
 size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
-  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup)) +
-         dense_parts_bytes(m, n, k);
+  return dense_qmm_rows_bytes(m, k) + dense_parts_bytes_up_to(m, n, k);
 }
 
 // x_prepared: rows already in the matmul's order with their group sums in sumx (x is then ignored)
@@ -2524,10 +2546,16 @@ bool dense_mlp_takes(const mf_qtensor& gate, const mf_qtensor& up, const mf_qten
          aligned16(scratch) && static_cast<uint64_t>(t) * std::max(d, f) < (1ull << 31);
 }
 
-size_t dense_mlp_scratch_bytes(uint32_t d, uint32_t f, uint32_t t) {
+static size_t dense_mlp_rows_bytes(uint32_t d, uint32_t f, uint32_t t) {
   return up256(sizeof(uint16_t) * static_cast<size_t>(t) * f) + up256(sizeof(uint16_t) * static_cast<size_t>(t) * d) +
-         up256(sizeof(float) * static_cast<size_t>(t) * (d / kGroup)) + up256(sizeof(float) * static_cast<size_t>(t) * (f / kGroup)) +
-         std::max(dense_parts_bytes(t, d, f), dense_gate_up_parts_bytes(t, f, d));  // (the two uses follow one another)
+         up256(sizeof(float) * static_cast<size_t>(t) * (d / kGroup)) + up256(sizeof(float) * static_cast<size_t>(t) * (f / kGroup));
+}
+// (the window results of gate / up and of down follow one another in the same place)
+size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t) {
+  return dense_mlp_rows_bytes(d, f, t) + std::max(dense_parts_bytes(t, d, f), dense_gate_up_parts_bytes(t, f, d));
+}
+size_t dense_mlp_scratch_bytes(uint32_t d, uint32_t f, uint32_t t) {
+  return dense_mlp_rows_bytes(d, f, t) + std::max(dense_parts_bytes_up_to(t, d, f), dense_gate_up_parts_bytes(t, f, d));
 }
 
 hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const mf_qtensor& down,

@@ -241,3 +241,19 @@ def test_repacked_ternary_layout_is_the_file_layout(d, f):
         a, b = ops.expert_blob_layout(d, f, bits, 16384), ops.expert_blob_layout(d, f, bits, 16384, repacked=True)
         assert (a[1], a[2]) == (b[1], b[2])
         assert all(getattr(a[0], n) == getattr(b[0], n) for n, _ in a[0]._fields_)
+
+
+@pytest.mark.parametrize("n,k", [(5120, 17408), (2048, 8192), (1152, 3200), (128, 128), (384, 12800)])
+def test_a_workspace_for_many_rows_serves_every_smaller_block(n, k):
+    """sizes never fall as rows are added, and a buffer sized for the most rows keeps every smaller block on the matrix
+    cores (the K windows of a block depend on its rows, so the bytes of a single call do not grow with them)"""
+    lib = _capi.lib()
+    w = _capi.QTensor(4096, 4096, 4096)  # addresses are only looked at: mf_qmm_path launches nothing
+    qmm = [lib.mf_qmm_workspace_bytes(m, n, k) for m in range(1, 701)]
+    mlp = [lib.mf_shared_expert_scratch_bytes(n, k, t) for t in range(1, 701)]
+    assert qmm == sorted(qmm) and mlp == sorted(mlp)
+    for most in (65, 129, 330, 600, 700, 5000):
+        have = lib.mf_qmm_workspace_bytes(most, n, k)
+        for m in range(1, min(most, 700) + 1):
+            assert lib.mf_qmm_path(w, 4, 4096, 4096, m, n, k, 4096, have) == 1, (most, m)
+        assert lib.mf_qmm_path(w, 4, 4096, 4096, most, n, k, 4096, 256) == 2

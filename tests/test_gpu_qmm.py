@@ -166,3 +166,25 @@ def test_shared_expert_block_form(gpu, oracle, d, f, t):
     _close_or_one_step(oracle, ops.bf16_bits(y_rows), ref, "row by row")
     for i in range(0, t, 7):
         assert torch.equal(y_rows[i], y_one[i])
+
+
+@pytest.mark.parametrize("d,f,most,rows", [(384, 12800, 385, (9, 300, 384)), (2560, 2048, 416, (16, 100, 415)), (2048, 8192, 140, (64, 90, 137))])
+def test_mlp_block_in_a_scratch_sized_for_more_rows(gpu, oracle, d, f, most, rows):
+    """one scratch buffer, sized for the largest block, gives every smaller block the bits of a buffer of its own size"""
+    rng = oracle.Rng.key(0xB10C, f"mlp-scratch-{d}-{f}")
+    qs = [to_device_q(oracle.quantize(rng.normal(0.0, 0.02, r * c).reshape(r, c), 4)) for r, c in ((f, d), (f, d), (d, f))]
+    op = ops.SharedExpertInt4(gpu)
+    most_bytes = op.scratch_bytes(d, f, most)
+    for t in rows:
+        x = ops.bf16_tensor(oracle.bf16_bits(rng.normal(0.0, 1.0, t * d).reshape(t, d)))
+        got = []
+        # guard bytes behind each buffer: a call stays inside what it was given
+        for own in (True, False):
+            size = op.scratch_bytes(d, f, t) if own else most_bytes
+            buf = torch.full((size + 256,), 0xA5, dtype=torch.uint8, device="cuda")
+            y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+            op.encode(x, *qs, y, buf[:size], t=t)
+            torch.cuda.synchronize()
+            assert bool((buf[size:] == 0xA5).all())
+            got.append(ops.bf16_bits(y))
+        assert np.array_equal(got[0], got[1]), t
