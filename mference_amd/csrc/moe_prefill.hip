@@ -1586,6 +1586,8 @@ __device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool&
   return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
 }
 
+// (Both parts of a launch read their codes in the form SWAPPED names; without it 2-bit codes have to be tiled.  The dense
+// problem beside 2-bit experts is 4-bit and goes through qmm_mixed_kernel: the launchers refuse a 2-bit one beside a tiled pool.)
 template <int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
 void qmm_kernel(const QmmLaunch launch) {
@@ -1593,12 +1595,6 @@ void qmm_kernel(const QmmLaunch launch) {
   bool second;
   const uint32_t work = qmm_work(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if constexpr (BITS == 2 && !SWAPPED) {  // (a dense problem beside a tiled pool lies row by row)
-    if (a.dense_mode) {
-      qmm_item<BITS, NPROJ, NG8, TAB16, true>(a, work, smem);
-      return;
-    }
-  }
   qmm_item<BITS, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
 }
 
@@ -1938,12 +1934,6 @@ void qmm_kres_kernel(const KresLaunch launch) {
   const uint32_t work = qmm_work(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
   const uint32_t walk = launch.slices[second ? 1 : 0];
-  if constexpr (BITS == 2 && !SWAPPED) {
-    if (a.dense_mode) {
-      qmm_kres_item<BITS, NG, true>(a, work, walk, smem);
-      return;
-    }
-  }
   qmm_kres_item<BITS, NG, SWAPPED>(a, work, walk, smem);
 }
 
@@ -2243,6 +2233,7 @@ hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t t
                            uint32_t b_tile_slots) {
   KresLaunch launch{};
   const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
+  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
   for (int part = 0; part < (b ? 2 : 1); ++part) {
     QmmArgs& q = launch.part[part];
     q = part ? *b : a;
@@ -2292,6 +2283,7 @@ hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t ti
                       uint32_t b_tile_slots) {
   QmmLaunch launch{};
   const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
+  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
   size_t lds = 0;
   bool ng8 = true, tab16 = false;
   for (int part = 0; part < (b ? 2 : 1); ++part) {
