@@ -138,7 +138,11 @@ mf_status mf_dequantize(mf_ctx* ctx, mf_stream stream, mf_qtensor q, size_t rows
  * DequantInt4GEMVMultiX.encode (Kernels/Quant/DequantInt4GEMVMultiX.swift:48-82)
  * for 1 < t <= 8, MapleTernaryGEMV.encode (Kernels/Quant/MapleTernaryGEMV.swift:
  * 29-45) for ternary.  x bf16 [t, n], y [t, m] bf16 or fp32 (out_f32 != 0,
- * the _f32out kernels).  Each weight row is read once for all t tokens.
+ * the _f32out kernels).  Each weight row is read once for up to 4 tokens.
+ * A token's result does not depend on the tokens beside it, bit for bit (MultiXKernelParityTests.swift:50-77), except
+ * where a long K is split among waves by the number of tokens: 4-bit matrices of n > 4096, or of n a multiple of 256 with
+ * 16384 rows and more, and gate / up pairs of 2-bit matrices of n > 4096 -- each unless n is a multiple of 512 that divides
+ * evenly.  There a token agrees with its single call within 2e-6 of the result's norm.
  * Two storages of ternary weights exist in the reference.  Routed experts pack four 2-bit codes
  * per byte with a scale table only (RepackPlanner.swift:560-651): MF_BITS_TERNARY.  The resident
  * projections MapleTernaryGEMV reads keep the same codes widened to nibbles, with a scale (alpha)

@@ -844,22 +844,31 @@ uint32_t device_cu_count() {
   return static_cast<uint32_t>(cached[dev]);
 }
 
+// waves that share a row in rows_stream_kernel (1, 2 or 4) and the 16-byte steps each takes; 0: not a shape of it
 template <int BITS, int NPROJ>
-bool rows_stream_try(hipStream_t s, const RowsArgs& in, uint32_t t, uint32_t num_cu, hipError_t& err) {
+uint32_t rows_stream_split(uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu, uint32_t& its) {
   constexpr int EPL = Fmt<BITS>::kElemsPer16B;
-  if (in.N % kGroup || in.N < 64 * EPL || (t != 1 && t != 2 && t != 4) || in.M < 1024) return false;
-  const uint32_t steps = (in.N + 64 * EPL - 1) / (64 * EPL);  // 16-byte steps of one wave along a row
+  if (n % kGroup || n < 64 * EPL || (t != 1 && t != 2 && t != 4) || m < 1024) return 0;
+  const uint32_t steps = (n + 64 * EPL - 1) / (64 * EPL);  // 16-byte steps of one wave along a row
   // x slices live in registers for the whole launch: T x its x (pairs + sum).  A 2-bit slice is 33
   // registers, and with two projections in flight the 9-step and the 4-token 3-step instances spill.
   constexpr bool wide_slices = BITS == kBits2 && NPROJ == 2;
   const uint32_t max_its = t == 1 ? (wide_slices ? 3 : 9) : (wide_slices && t == 4 ? 1 : 3);
-  if (BITS == kBitsTernary) return false;
+  if (BITS == kBitsTernary) return 0;
   uint32_t wpr = 1;
   while (wpr < 4 && (steps + wpr - 1) / wpr > max_its) wpr *= 2;
   // few rows and long rows: split the rows so that every wave still walks a useful number of them
-  while (wpr < 4 && in.M / wpr < num_cu * 8 * 4 && (steps + wpr - 1) / wpr > 2) wpr *= 2;
-  const uint32_t its = (steps + wpr - 1) / wpr;
-  if (its > max_its) return false;
+  while (wpr < 4 && m / wpr < num_cu * 8 * 4 && (steps + wpr - 1) / wpr > 2) wpr *= 2;
+  its = (steps + wpr - 1) / wpr;
+  return its > max_its ? 0 : wpr;
+}
+
+template <int BITS, int NPROJ>
+bool rows_stream_try(hipStream_t s, const RowsArgs& in, uint32_t t, uint32_t num_cu, hipError_t& err) {
+  constexpr bool wide_slices = BITS == kBits2 && NPROJ == 2;
+  uint32_t its = 0;
+  const uint32_t wpr = rows_stream_split<BITS, NPROJ>(in.M, in.N, t, num_cu, its);
+  if (!wpr) return false;
   RowsArgs a = in;
   a.wpr = wpr;
   const uint32_t rows_per_wg = 4 / wpr;
@@ -887,21 +896,28 @@ bool rows_stream_try(hipStream_t s, const RowsArgs& in, uint32_t t, uint32_t num
 // 256 (so that the per-wave group ranges start on 8-byte boundaries of the scale table), up to 8
 // token rows, when the x rows of one workgroup fit LDS.
 template <int NPROJ>
-bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipError_t& err) {
-  const uint32_t ng = a.N / kGroup;
+bool rows_mfma_split(uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu, uint32_t& n_ks, uint32_t& gps, size_t& lds) {
+  const uint32_t ng = n / kGroup;
   // one or two token rows stream faster through rows_stream_kernel (1 KB contiguous per load
   // instruction against 32-byte pieces of 32 rows here); from three rows on the dot products
   // outweigh that
-  if (a.N % (4 * kGroup) || a.N < 2048 || a.T < 3 || a.T > 8 || a.M < 1024) return false;
-  const uint32_t blocks = (a.M + 31) / 32;
+  if (n % (4 * kGroup) || n < 2048 || t < 3 || t > 8 || m < 1024) return false;
+  const uint32_t blocks = (m + 31) / 32;
   // enough waves to fill the chip: 4 K-splits when there are many row blocks, 16 when few
-  uint32_t n_ks = blocks * 4 >= num_cu * 8 ? 4 : 16;
+  n_ks = blocks * 4 >= num_cu * 8 ? 4 : 16;
   while (n_ks > 4 && ng / n_ks < 4) n_ks /= 2;
-  uint32_t gps = (ng + n_ks - 1) / n_ks;
+  gps = (ng + n_ks - 1) / n_ks;
   gps = (gps + 3) / 4 * 4;  // multiples of 4 groups per wave
-  const size_t lds = std::max<size_t>(static_cast<size_t>(n_ks) * gps * (8 * a.T * 16 + a.T * 4),
-                                      static_cast<size_t>(n_ks) * NPROJ * 8 * 32 * 4);
-  if (lds > 156 * 1024 || (n_ks != 4 && n_ks != 16) || (NPROJ == 2 && n_ks != 4)) return false;
+  lds = std::max<size_t>(static_cast<size_t>(n_ks) * gps * (8 * t * 16 + t * 4), static_cast<size_t>(n_ks) * NPROJ * 8 * 32 * 4);
+  return lds <= 156 * 1024 && (n_ks == 4 || n_ks == 16) && (NPROJ == 1 || n_ks == 4);
+}
+
+template <int NPROJ>
+bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipError_t& err) {
+  uint32_t n_ks = 0, gps = 0;
+  size_t lds = 0;
+  if (!rows_mfma_split<NPROJ>(a.M, a.N, a.T, num_cu, n_ks, gps, lds)) return false;
+  const uint32_t blocks = (a.M + 31) / 32;
   RowsMfmaArgs b = a;
   b.gps = gps;
   err = n_ks == 4 ? allow_lds<rows_mfma_kernel<NPROJ, 4>>(lds, 156 * 1024) : allow_lds<rows_mfma_kernel<1, 16>>(lds, 156 * 1024);
@@ -912,81 +928,104 @@ bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipErr
   return true;
 }
 
-// The quad kernel takes 4-bit and 2-bit matrices with at least 1024 rows (a multiple of 4) and up to 4
-// token rows.  The 32-element chunks of a row split over (waves, ITS slots of 16 chunks).  K a multiple of 512 that splits
-// with little waste: any number of rows.  `any_k`: any other K, the split that costs the fewest
-// slots, a stage of a wave counted as one more.
-template <int BITS, int NPROJ>
-bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, bool any_k, uint32_t num_cu, hipError_t& err) {
-  if (a.N % kGroup || a.N < 8 * kGroup || a.T < 1 || a.T > 4 || a.M < 1024 || a.M % 4) return false;
-  const uint32_t chunks = a.N / 32;
-  uint32_t its = 0, wpr = 0, waste = ~0u;
+// The quad kernel takes 4-bit and 2-bit matrices with at least 1024 rows (a multiple of 4), a K of at least 2048 and up to
+// 4 token rows.  The 32-element chunks of a row split over (waves, ITS slots of 16 chunks).  EVEN: K is a multiple of 512
+// and splits with little waste.  ANY: any other K, the split that costs the fewest slots, a stage of a wave counted as
+// one more.
+enum class QuadFit { kNone, kEven, kAny };
+QuadFit rows_quad_split(uint32_t m, uint32_t n, uint32_t& its, uint32_t& wpr) {
+  if (n % kGroup || n < 2048 || m < 1024 || m % 4) return QuadFit::kNone;
+  const uint32_t chunks = n / 32;
+  uint32_t waste = ~0u;
+  its = wpr = 0;
   for (uint32_t i = 6; i >= 4; --i) {
     const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
     if (w > kQuadMaxWaves) continue;
     if (16 * i * w - chunks < waste) { waste = 16 * i * w - chunks; its = i; wpr = w; }
   }
-  const bool fits = a.N % (8 * kGroup) == 0 && its && waste * 10 <= chunks;
-  if (!fits) {
-    if (!any_k) return false;
-    uint32_t cost = ~0u;
-    for (uint32_t i = 6; i >= 2; --i) {
-      const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
-      if (w <= kQuadMaxWaves && w * (i + 1) < cost) { cost = w * (i + 1); its = i; wpr = w; }
-    }
-    if (cost == ~0u) return false;
+  if (n % (8 * kGroup) == 0 && its && waste * 10 <= chunks) return QuadFit::kEven;
+  uint32_t cost = ~0u;
+  for (uint32_t i = 6; i >= 4; --i) {
+    const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
+    if (w <= kQuadMaxWaves && w * (i + 1) < cost) { cost = w * (i + 1); its = i; wpr = w; }
   }
+  return cost == ~0u ? QuadFit::kNone : QuadFit::kAny;
+}
+
+template <int BITS, int NPROJ>
+hipError_t launch_rows_quad(hipStream_t s, const RowsQuadArgs& a, QuadFit fit, uint32_t its, uint32_t wpr, uint32_t num_cu) {
   const uint32_t n_sets = a.M / 4;
   const dim3 grid(std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / wpr))), block(wpr * 64);
-  if (fits) {
+  if (fit == QuadFit::kEven) {
     if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, false><<<grid, block, 0, s>>>(a);
     else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, false><<<grid, block, 0, s>>>(a);
     else rows_quad_kernel<BITS, NPROJ, 6, false><<<grid, block, 0, s>>>(a);
   } else {
-    if (its == 2) rows_quad_kernel<BITS, NPROJ, 2, true><<<grid, block, 0, s>>>(a);
-    else if (its == 3) rows_quad_kernel<BITS, NPROJ, 3, true><<<grid, block, 0, s>>>(a);
-    else if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, 0, s>>>(a);
+    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, 0, s>>>(a);
     else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, true><<<grid, block, 0, s>>>(a);
     else rows_quad_kernel<BITS, NPROJ, 6, true><<<grid, block, 0, s>>>(a);
   }
-  err = hipGetLastError();
+  return hipGetLastError();
+}
+
+// Whether the other kernels add every row of such a matrix in gemv_kernel's order, for 1 to 8 token rows alike: a row of
+// rows_stream_kernel in one wave's hands keeps that order, one split over waves or on rows_mfma_kernel does not.
+template <int BITS, int NPROJ>
+bool rows_lane_ordered(uint32_t m, uint32_t n, uint32_t num_cu) {
+  uint32_t a = 0, b = 0;
+  size_t lds = 0;
+  for (uint32_t t = 1; t <= 8; ++t) {
+    if (rows_stream_split<BITS, NPROJ>(m, n, t, num_cu, a) > 1) return false;
+    if (BITS == kBits4 && rows_mfma_split<NPROJ>(m, n, t, num_cu, a, b, lds)) return false;
+  }
   return true;
+}
+
+// Whether t token rows of the matrix go to the quad kernel.  A draft's verification and the plain step it stands for
+// have to agree: where the other kernels give a row the same bits for every number of token rows, the quad kernel takes
+// all numbers or none, by what one row costs (us, other kernels / this one, one row; four rows):
+//   4-bit of K below 2048, none (17408 x 1536: 7.3 / 8.3; 18.6 / 9.6), 4-bit above, from 36 M weights on
+//   (17408 x 2112: 11.6 / 10.6; 31.8 / 12.7; gate / up 6656 x 3136: 12.4 / 11.5, 6656 x 2112: 11.5 / 12.5);
+//   2-bit of K up to 4096, only long and many rows (17408 x 3136: 15.7 / 11.0; 52.9 / 12.4; gate / up 6656 x 3136:
+//   9.5 / 10.7; 28.9 / 12.0; 4096 is one whole step of rows_stream_kernel: 17408 rows 10.1 / 12.4), 2-bit above, from
+//   8 M weights on (6656 x 6592: 14.7 / 10.6; 34.0 / 12.1; 1024 x 6592: 4.9 / 5.1).
+// Elsewhere the number of token rows decides (us per MLP, other kernels / this one): one row, where a step of
+// rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3; 3840 x 7680, a
+// sixteenth empty: 22.2 / 22.9); two to four (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25; 2048 x 6656:
+// 23.5 / 21.7); more: where the weights outweigh two launches (five rows, 2816 x 4096: 29.5 / 31.5; 3328 x 8192:
+// 46.5 / 42.8; 2-bit, 1088 x 2112: 18.9 / 19.9, 1984 x 5056: 33.6 / 28.0).
+template <int BITS, int NPROJ>
+bool rows_quad_takes(QuadFit fit, uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu) {
+  constexpr bool two = BITS == kBits2;
+  constexpr uint32_t step = two ? 4096 : 2048;  // K values of one step of a wave in rows_stream_kernel
+  const uint64_t weights = static_cast<uint64_t>(m) * n * NPROJ;
+  if (fit == QuadFit::kNone) return false;
+  if (two && n <= step) return n >= 2560 && n < step && weights >= 24000000ull * NPROJ * NPROJ;
+  if (fit == QuadFit::kEven) return true;
+  if (rows_lane_ordered<BITS, NPROJ>(m, n, num_cu)) return n >= step && weights >= (two ? 8ull : 36ull) * 1000000;
+  const uint32_t steps = (n + step - 1) / step;
+  const bool wide = weights >= (two ? 8ull : 24ull) * 1000000;
+  return t == 1 ? wide && n * 5ull < steps * static_cast<uint64_t>(step) * 4 : t <= 4 ? weights >= 4000000 : wide;
 }
 
 // Up to four token rows in one launch.  Five to eight: two launches, rows 0..3 and the
 // rest.  The quad kernel runs the same instructions for a token whatever rides along, so every row
 // keeps the bits of a single-token call (MultiXKernelParityTests.swift:50-77); the weights stream
 // twice.  (y rows are M elements apart, 2 or 4 bytes each: 16-byte aligned since M % 4 == 0.)
-template <int NPROJ>
-bool rows_quad_any(hipStream_t s, int bits, const RowsQuadArgs& a, hipError_t& err) {
-  if (a.T > 8) return false;
-  const bool two = bits == kBits2;
-  // One row of 2-bit weights that rows_stream_kernel takes in one step of a wave is faster there
-  // (6656 x 2048, two projections: 13 us against 17; 5120 x 17408: 59 us for the MLP there, 38 here).
-  const uint32_t step = two ? 4096 : 2048, steps = (a.N + step - 1) / step;
-  if (two && a.T == 1 && steps == 1) return false;
-  // Where a K that is no multiple of 512, or splits badly, goes (us per MLP, other kernels / this one):
-  // one row: where a step of rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3;
-  // 3840 x 7680, a sixteenth empty: 22.2 / 22.9); two to four (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25;
-  // 2048 x 6656: 23.5 / 21.7); more: where the weights outweigh two launches (five rows, 2816 x 4096: 29.5 / 31.5;
-  // 3328 x 8192: 46.5 / 42.8; 2-bit, 1088 x 2112: 18.9 / 19.9, 1984 x 5056: 33.6 / 28.0).  Small matrices stay with the
-  // kernels whose rows have the bits of single-token calls for every number of rows.
-  const uint64_t weights = static_cast<uint64_t>(a.M) * a.N * NPROJ;
-  const bool wide = weights >= (two ? 8ull : 24ull) * 1000000;
-  const bool any_k = a.T == 1 ? wide && a.N * 5ull < steps * static_cast<uint64_t>(step) * 4
-                   : a.T <= 4 ? weights >= 4000000
-                              : wide;
-  for (uint32_t t0 = 0; t0 < a.T; t0 += 4) {
+template <int BITS, int NPROJ>
+bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipError_t& err) {
+  if (a.T < 1 || a.T > 8) return false;
+  uint32_t its = 0, wpr = 0;
+  const QuadFit fit = rows_quad_split(a.M, a.N, its, wpr);
+  if (!rows_quad_takes<BITS, NPROJ>(fit, a.M, a.N, a.T, num_cu)) return false;
+  for (uint32_t t0 = 0; t0 < a.T && err == hipSuccess; t0 += 4) {
     RowsQuadArgs q = a;
     q.T = std::min(a.T - t0, 4u);
     q.x = a.x + static_cast<size_t>(t0) * a.N;
     q.y = static_cast<uint8_t*>(a.y) + static_cast<size_t>(t0) * a.M * (a.out_f32 ? 4 : 2);
-    const bool took = bits == kBits4 ? rows_quad_try<kBits4, NPROJ>(s, q, any_k, device_cu_count(), err)
-                                     : rows_quad_try<kBits2, NPROJ>(s, q, any_k, device_cu_count(), err);
-    if (!took) return false;  // (the shape decides: the first launch is refused or none is)
-    if (err != hipSuccess) return true;
+    err = launch_rows_quad<BITS, NPROJ>(s, q, fit, its, wpr, num_cu);
   }
-  return a.T > 0;
+  return true;
 }
 
 }  // namespace
@@ -1010,7 +1049,9 @@ hipError_t launch_gemv(hipStream_t s, const mf_qtensor& w, int bits, const uint1
     qa.W[0] = static_cast<const uint8_t*>(w.weights); qa.S[0] = w.scales; qa.B[0] = w.biases;
     qa.x = x; qa.y = y; qa.M = m; qa.N = n; qa.T = t; qa.out_f32 = out_f32 ? 1 : 0;
     hipError_t err = hipSuccess;
-    if (rows_quad_any<1>(s, bits, qa, err)) return err;
+    if (bits == kBits4 ? rows_quad_try<kBits4, 1>(s, qa, device_cu_count(), err)
+                       : rows_quad_try<kBits2, 1>(s, qa, device_cu_count(), err))
+      return err;
   }
   if (!lane_order && al && bits == kBits4 && aligned16(w.scales) && aligned16(w.biases)) {
     RowsMfmaArgs ma{};
@@ -1053,7 +1094,9 @@ hipError_t launch_gate_up_act(hipStream_t s, const mf_qtensor& gate, const mf_qt
     qa.W[1] = static_cast<const uint8_t*>(up.weights); qa.S[1] = up.scales; qa.B[1] = up.biases;
     qa.x = x; qa.y = act; qa.M = f; qa.N = d; qa.T = t;
     hipError_t err = hipSuccess;
-    if (rows_quad_any<2>(s, bits, qa, err)) return err;
+    if (bits == kBits4 ? rows_quad_try<kBits4, 2>(s, qa, device_cu_count(), err)
+                       : rows_quad_try<kBits2, 2>(s, qa, device_cu_count(), err))
+      return err;
   }
   if (!lane_order && al && tables && bits == kBits4) {
     RowsMfmaArgs ma{};

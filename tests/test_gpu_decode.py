@@ -200,6 +200,48 @@ def test_gemv_quad_rows_kernel_at_any_k(gpu, oracle, bits, m, n, t):
         assert np.array_equal(y2.cpu().numpy().view(np.uint32), got[t - 2:].view(np.uint32))
 
 
+@pytest.mark.parametrize("bits,m,n", [
+    (4, 3136, 1984), (4, 12288, 1536),      # 4-bit, K below a wave's step: the vector kernels
+    (4, 7680, 3136), (4, 11520, 3136),      # ... above, below and above the quad kernel's 36 M weights; one group in the last piece
+    (4, 16384, 2240), (4, 1024, 2816), (4, 9216, 4672),
+    (2, 4096, 2048), (2, 9408, 2560), (2, 9344, 2560), (2, 6656, 4032), (2, 2816, 4096),  # 2-bit, one step or less
+    (2, 1216, 6592), (2, 1152, 6592), (2, 2816, 5120), (2, 1024, 8128),                   # ... more
+])
+def test_a_row_has_the_same_bits_in_every_call(gpu, bits, m, n):
+    """MultiXKernelParityTests.swift:50-77, bit for bit: a row alone and among up to eight, as one projection and as a
+    gate / up pair, at both sides of the lines between the row kernels"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m * n + bits)
+    tables = lambda sign: (sign * torch.rand(m * (n // 64), generator=gen, device="cuda") * 0.02).to(torch.bfloat16)
+    qs = [ops.QuantizedTensor(torch.randint(0, 256, (m * n * bits // 8,), dtype=torch.uint8, generator=gen, device="cuda"),
+                              tables(1), tables(-8 if bits == 4 else -2), bits, m, n) for _ in range(2)]
+    down = ops.QuantizedTensor(qs[0].packed, qs[0].scales, qs[0].biases, bits, n, m)
+    x = torch.randn(8, n, generator=gen, device="cuda").to(torch.bfloat16)
+    g, mlp = ops.DequantInt4GEMVMultiX(gpu), ops.SharedExpertInt4(gpu)
+
+    def call(t, row):
+        y = torch.zeros((t, m), dtype=torch.float32, device="cuda")
+        act = torch.zeros((t, m), dtype=torch.bfloat16, device="cuda")
+        out = torch.zeros((t, n), dtype=torch.bfloat16, device="cuda")
+        xs = x[row:row + t].contiguous()
+        g.encode(qs[0], xs, y, m, n, t, output_float32=True)
+        mlp.encode(xs, qs[0], qs[1], down, out, act, t=t)
+        return y.view(torch.int32), act.view(torch.int16)
+
+    ones = [call(1, i) for i in range(8)]
+    w = (qs[0].packed.view(m, -1, 1) >> torch.arange(0, 8, bits, device="cuda")) & (2 ** bits - 1)
+    w = w.view(m, n // 64, 64).double() * qs[0].scales.view(m, -1, 1).double() + qs[0].biases.view(m, -1, 1).double()
+    want = x.double() @ w.view(m, n).T
+    got = torch.cat([o[0] for o in ones]).view(torch.float32).double()
+    assert torch.linalg.norm(got - want) <= 2e-6 * torch.linalg.norm(want)
+    for t in range(2, 9):
+        y, act = call(t, 0)
+        for i in range(t):
+            assert torch.equal(y[i:i + 1], ones[i][0]), (t, i)
+            if (bits, n > 4096) != (2, True) or n % 512 == 0:  # (2-bit pairs of a longer K may split four rows over waves)
+                assert torch.equal(act[i:i + 1], ones[i][1]), (t, i)
+
+
 @pytest.mark.parametrize("d,f,t", [(2048, 1024, 1), (5120, 1536, 4)])
 def test_shared_expert_streaming_rows_kernel(gpu, oracle, d, f, t):
     """dense SwiGLU MLP wide enough for the streaming gate/up and down kernels"""
