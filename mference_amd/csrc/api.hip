@@ -779,10 +779,18 @@ mf_status mf_moe_prefill_layer(mf_moe* h, mf_stream stream, const mf_moe_layer_w
                   (!c.shared_f || (mf::aligned16(wts->shared_gate.weights) && mf::aligned16(wts->shared_up.weights) &&
                                    mf::aligned16(wts->shared_down.weights) &&
                                    !(wts->w_sg && !wts->w_sg_q8.weights && !mf::aligned16(wts->w_sg))));
+  // ... and up to one decode launch of rows always: six dependent launches do not pay there (us, decode / matmul:
+  // 2816 x 704, 128 experts, top 8: 1 row 18.5 / 56, 8 rows 58 / 98; 1088 x 576, 64 experts, top 4: 1 row 15 / 41,
+  // 8 rows 32 / 47).  Two of them where the routes rarely share an expert and no shared expert is read again (the first
+  // layer: 9 rows 78 / 99, 16 rows 113 / 135, 17 rows 132 / 137; 2-bit codes cost the decode launch more, 1472 x 1408,
+  // 92 experts, top 7: 12 rows 97 / 91).
+  const bool few = t <= MF_MAX_TOKENS ||
+                   (t <= 2 * MF_MAX_TOKENS && !c.shared_f && c.bits != MF_BITS_2 && t * c.top_k <= c.num_experts &&
+                    h->fused && mf::fused_supported(*h, *wts, x, y, nullptr, MF_MAX_TOKENS));
   if (!mf::prefill_supported(c) ||
       (!mf::prefill_whole_tiles(c) &&
-       (!al || !workspace || wts->expert_tiled || workspace_bytes < mf::prefill_workspace_bytes(c, t)))) {
-    // another shared-expert format, a width of one group, or no workspace: the same rows through the decode
+       (few || !al || !workspace || wts->expert_tiled || workspace_bytes < mf::prefill_workspace_bytes(c, t)))) {
+    // another shared-expert format, a width of one group, few rows or no workspace: the same rows through the decode
     // launch, MF_MAX_TOKENS at a time (correct for every configuration, not fast)
     for (uint32_t t0 = 0; t0 < t; t0 += MF_MAX_TOKENS) {
       const uint32_t n = t - t0 < MF_MAX_TOKENS ? t - t0 : MF_MAX_TOKENS;

@@ -313,6 +313,31 @@ def test_prefill_widths_of_whole_groups(gpu, oracle, bits, d, f, e, fs, t):
     assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(yd)), oracle.bf16_to_float(ref_y), "without a workspace")
 
 
+@pytest.mark.parametrize("bits,e,fs,t,decode", [
+    (4, 32, 0, 1, True), (4, 16, 192, 8, True), (2, 16, 0, 5, True),   # one decode launch of rows
+    (4, 32, 0, 16, True), (1, 32, 0, 9, True),                        # two, at most a route per expert
+    (4, 32, 0, 17, False), (4, 16, 0, 9, False), (2, 32, 0, 9, False), (4, 32, 192, 9, False),
+])
+def test_prefill_of_few_rows_takes_the_decode_launch(gpu, oracle, bits, e, fs, t, decode):
+    """at widths that 128 does not divide, up to the number of rows the decode launch is faster for: its bits, with a
+    workspace or without"""
+    d, f, k = 320, 192, 2
+    root = ROOT_SEED + 0xA2A0 + e
+    layer = oracle.synth_layer(root, d, f, e, k, bits=bits, fs=fs, router_mode=1 if bits == 1 else 0)
+    x = oracle.synth_x(root, t, d)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    y, idx, w = _run_prefill(moe, wts, x, t, d, k)
+    yd = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    xd = ops.bf16_tensor(x)
+    for t0 in range(0, t, 8):
+        moe.encode_decode_layer(wts, xd[t0:t0 + 8], yd[t0:t0 + 8], t=min(8, t - t0))
+    moe.status()
+    assert np.array_equal(y, ops.bf16_bits(yd)) == decode
+    ref_y, ref_idx, ref_w = oracle.moe_layer(layer, x)
+    assert np.array_equal(idx, ref_idx)
+    assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref_y), f"bits={bits} t={t}")
+
+
 @pytest.mark.parametrize("d,f,t", [(192, 320, 33), (1152, 704, 64), (128, 448, 130)])
 def test_dense_mlp_widths_of_whole_groups(gpu, oracle, d, f, t):
     """the block form of the dense MLP at widths that are no multiples of 128"""
