@@ -2831,21 +2831,31 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
     d.pair_rows = q.pair_rows;
   }
   const bool kres_q = kres_takes(q, pairs), kres_d = c.shared_f && kres_takes(d, t);
+  // Both parts in one launch of one kernel: the resident one when it takes both (their K has to be the same), else the
+  // ring.  Routed experts the resident kernel takes beside a shared expert of another width get it in a launch of their
+  // own once its gain outweighs the shared expert's launch, whose few items are then alone on the chip (layer, us, one
+  // launch / two, same bits: 4096 x 256, shared 512, top 6: 40 tokens 98 / 93, 2048 tokens 369 / 296; 2048 x 128, shared
+  // 512, top 8: 150 tokens 72 / 74, 300 tokens 87 / 85, 2048 tokens 176 / 143; 2048 x 512, shared 1024, top 8: 300 tokens
+  // 102 / 111, 777 tokens 155 / 155, 2048 tokens 274 / 262; routed 1024 or 2048 beside a resident shared expert: one
+  // launch always, 375 / 385).
+  const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
+  const bool apart = shared_rides && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
   {
     // group sums of the activation rows for qmm_kernel (qmm_kres_kernel sums the rows it stages itself);
     // routes past the last tile's count were never written: only pairs rows exist, all written
-    const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
-    const bool q_ring = !kres_both, d_ring = shared_rides && !kres_both;
+    const bool q_ring = !kres_both && !apart, d_ring = shared_rides && (apart ? !kres_d : !kres_both);
     if (q_ring || d_ring)
       MF_TRY(launch_prep_rows(s, q_ring ? ws.acts : nullptr, nullptr, ws.sum_acts, q_ring ? pairs * c.f : 0,
                               d_ring ? ws.sact : nullptr, nullptr, ws.sum_sact,
                               d_ring ? static_cast<size_t>(t) * c.shared_f : 0));
   }
   const int down_proj = q.pair_rows ? 2 : 1;
-  if (!shared_rides) {
+  if (!shared_rides || apart) {
     if (kres_q) MF_TRY(launch_qmm_kres(s, code_bits, q, max_tiles, nullptr, 0));
     else MF_TRY(launch_qmm(s, code_bits, q, down_proj, max_tiles, nullptr, 0));
-  } else if (kres_q && kres_d && d.kdim == q.kdim) {
+    if (apart && kres_d) MF_TRY(launch_qmm_kres(s, 4, d, dense_tiles, nullptr, 0));
+    else if (apart) MF_TRY(launch_qmm(s, 4, d, down_proj, dense_tiles, nullptr, 0));
+  } else if (kres_both) {
     if (dense_first) MF_TRY(launch_qmm_kres(s, launch_bits, d, dense_tiles, &q, max_tiles));
     else MF_TRY(launch_qmm_kres(s, launch_bits, q, max_tiles, &d, dense_tiles));
   } else if (dense_first) MF_TRY(launch_qmm(s, launch_bits, d, down_proj, dense_tiles, &q, max_tiles));

@@ -122,6 +122,11 @@ def _run_prefill(moe, wts, x, t, d, k):
     (2, 512, 256, 32, 6, 256, 200, 0, 7.0),    # top-6 + SwiGLU clamp (moe.metal:902-1195)
     (2, 1024, 512, 16, 6, 0, 133, 0, 0.0),     # K a multiple of 512 (whole-table vector loads), no shared expert
     (2, 384, 384, 16, 2, 128, 45, 0, 0.0),     # neither down projection has K of 128, 256 or 512
+    # routed experts of the resident kernel beside a shared expert of another width: one launch below 1024 routes, two from
+    # there on (8192 beside a shared expert wider than 512), the shared expert resident itself or not
+    (2, 256, 128, 16, 8, 256, 127, 0, 0.0), (2, 256, 128, 16, 8, 256, 128, 0, 0.0),
+    (1, 512, 256, 32, 8, 512, 150, 1, 0.0), (4, 512, 256, 16, 8, 384, 150, 0, 0.0),
+    (2, 512, 512, 16, 8, 640, 140, 0, 0.0), (2, 256, 128, 16, 8, 640, 1030, 0, 0.0),
     # ternary experts, scale-only tables, full-softmax router (maple_moe.metal:62-265)
     (1, 256, 128, 32, 8, 0, 131, 1, 0.0),
     (1, 512, 256, 32, 4, 0, 64, 1, 0.0),
