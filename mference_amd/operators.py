@@ -10,8 +10,8 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
-from operator import is_ as _is
 from typing import Optional, Sequence
+from weakref import ref as _ref
 
 import numpy as np
 import torch
@@ -366,20 +366,22 @@ class MoELayerWeights:
         return t if q is None else t + (q.packed, q.scales, q.biases)
 
     def c(self) -> _capi.LayerWeights:
-        """The C struct of the layer.  It is kept between calls: it is the same while the same tensors are named and
-        lie where they lay (a field, or a tensor's storage, may be replaced at any time)."""
+        """The C struct of the layer.  It is kept between calls and is the same while every tensor named lies where it lay
+        and the pools keep their shape (a field, or a tensor's storage, may be replaced at any time).  No tensor is held for
+        it: one that the layer no longer names is the caller's to free, and an address is not trusted beyond its tensor."""
         now = self._tensors()
+        key = [0 if t is None else t.data_ptr() for t in now]
+        key += self.experts.stride()
+        if self.experts_tiled is not None:
+            key += (*self.experts.shape, *self.experts_tiled.shape, self.experts_tiled.stride(0))
+        key.append(bytes(self.offsets))
         kept = self.__dict__.get("_kept")
-        if kept is not None:
-            was, where, offsets, stride, struct = kept
-            if (len(was) == len(now) and all(map(_is, was, now)) and offsets is self.offsets and
-                    [t.data_ptr() for t in now if t is not None] == where and self.experts.stride(0) == stride and
-                    struct.offsets_bytes == bytes(offsets)):
-                return struct
+        if kept is not None and kept[0] == key:
+            return kept[1]
         struct = self._build()
-        struct.offsets_bytes = bytes(self.offsets)
-        self.__dict__["_kept"] = (now, [t.data_ptr() for t in now if t is not None], self.offsets,
-                                  self.experts.stride(0), struct)
+        kept = [key, struct]
+        kept.append([_ref(t, lambda _, k=kept: k.__setitem__(0, None)) for t in now if t is not None])
+        self.__dict__["_kept"] = kept
         return struct
 
     def __getstate__(self):  # a copy makes its own C struct

@@ -1199,3 +1199,40 @@ def test_decode_layer_with_the_norm_in_front(gpu, oracle, bits, d, f, e, k, fs, 
     assert np.array_equal(ops.bf16_bits(xn), x_ref)
     assert np.array_equal(idx.cpu().numpy().astype(np.uint32), ref_idx)
     assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(ref_y), "normed layer")
+
+
+def test_a_layer_holds_no_tensor_it_does_not_name(gpu, oracle):
+    """a pool taken out of a layer is freed at once, also between calls; what the next call reads is what the layer
+    names then, and a tiled copy of another shape is refused wherever it lies"""
+    import gc
+    import weakref
+    layer = oracle.synth_layer(ROOT_SEED + 0x3E1, 256, 128, 16, 4, bits=4, fs=128)
+    moe, lw = make_moe(gpu, layer), to_device_layer(layer)
+    x = ops.bf16_tensor(oracle.synth_x(ROOT_SEED + 0x3E1, 2, 256))
+
+    def run():
+        y = torch.zeros((2, 256), dtype=torch.bfloat16, device="cuda")
+        moe.encode_decode_layer(lw, x, y, t=2)
+        moe.status()
+        return ops.bf16_bits(y)
+
+    lw.experts_tiled = moe.tile_experts(lw.experts, lw.offsets)
+    first = run()
+    gone, at = weakref.ref(lw.experts_tiled), lw.experts_tiled.data_ptr()
+    lw.experts_tiled = None
+    gc.collect()
+    assert gone() is None
+    lw.experts_tiled = torch.zeros((15, lw.experts.shape[1]), dtype=torch.uint8, device="cuda")  # (may lie where the other lay)
+    with pytest.raises(ops.MfError):
+        run()
+    lw.experts_tiled = None
+    assert np.array_equal(run(), first)
+    old = weakref.ref(lw.experts)
+    lw.experts = lw.experts.clone()
+    gc.collect()
+    assert old() is None and np.array_equal(run(), first)
+    lw.shared[0].packed = torch.zeros_like(lw.shared[0].packed)
+    assert not np.array_equal(run(), first)
+    lw.experts = lw.experts.cpu()
+    with pytest.raises(ValueError):
+        run()
