@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
     for (int n = 0; n < NT; ++n) {
       const float v = s_sum[buf][(tb * NT + n) * 32 + m][h];
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
-      const float r1 = v - __uint_as_float(hi);
+      const float r1 = __builtin_isinf(v) ? 0.0f : v - __uint_as_float(hi);  // (an infinite sum has no rest: inf - inf would be NaN)
       const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
       const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
       const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);

@@ -1152,6 +1152,63 @@ def test_int8_shared_expert_many_rows(gpu, oracle, d, f, t, silu):
         assert np.abs(got - want).max() <= 2.0 ** -6 * np.abs(want).max()
 
 
+def _wild_rows(gen, t, n):
+    """t rows of finite numbers and the same rows with an infinity of either sign and a NaN in three of them"""
+    x = torch.randn(t, n, generator=gen, device="cuda").to(torch.bfloat16)
+    wild = x.clone()
+    wild[1, n // 2], wild[t // 2, 5], wild[t - 1, n - 1] = float("inf"), float("-inf"), float("nan")
+    return x, wild, [1, t // 2, t - 1]
+
+
+@pytest.mark.parametrize("t", [16, 70])
+@pytest.mark.parametrize("d,f", [(192, 128), (704, 320)])
+def test_int8_matmul_passes_infinities_on(gpu, d, f, t):
+    """rows with infinities and NaN through the 8-bit matmul: the values the row kernels give (weights above zero, so an
+    infinity stays one), and no other row is touched"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + t)
+    def q(rows, n):
+        table = lambda: (0.01 + 0.01 * torch.rand(rows, n // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+        return ops.QuantizedTensor(torch.randint(1, 256, (rows, n), dtype=torch.uint8, generator=gen, device="cuda"), table(), table(), 8, rows, n)
+    qs = [q(f, d), q(f, d), q(d, f)]
+    x, wild, at = _wild_rows(gen, t, d)
+    op = ops.SharedExpertInt8(gpu)
+
+    def run(rows, step):
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        act = torch.zeros((t, f), dtype=torch.bfloat16, device="cuda")
+        for t0 in range(0, t, step):
+            op.encode(rows[t0:t0 + step], *qs, y[t0:t0 + step], act[t0:t0 + step], t=min(step, t - t0))
+        return torch.cat([act, y], 1)
+
+    finite, got, want = run(x, t), run(wild, t), run(wild, 8)
+    others = [i for i in range(t) if i not in at]
+    assert torch.equal(got[others].view(torch.int16), finite[others].view(torch.int16))
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.isinf(got[1]).all() and torch.isnan(got[t - 1]).all()
+    assert torch.equal(torch.sign(got[1].float()), torch.sign(want[1].float()))
+
+
+@pytest.mark.parametrize("bits,m,n,t", [(4, 1024, 5120, 3), (4, 11520, 3136, 8), (2, 9408, 2560, 4), (2, 1216, 6592, 7)])
+def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
+    """an infinity or a NaN makes its own token's results NaN (the code offset is taken out as inf - inf, as in every row
+    kernel of these formats) and leaves the other tokens' bits alone"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n + t)
+    table = lambda s: (s * (0.01 + 0.01 * torch.rand(m, n // 64, generator=gen, device="cuda"))).to(torch.bfloat16)
+    q = ops.QuantizedTensor(torch.randint(0, 256, (m, n * bits // 8), dtype=torch.uint8, generator=gen, device="cuda"), table(1), table(-4), bits, m, n)
+    x, wild, at = _wild_rows(gen, t, n)
+    g = ops.DequantInt4GEMVMultiX(gpu)
+    out = []
+    for rows in (x, wild):
+        y = torch.zeros((t, m), dtype=torch.float32, device="cuda")
+        g.encode(q, rows, y, m, n, t, output_float32=True)
+        out.append(y)
+    others = [i for i in range(t) if i not in at]
+    assert torch.equal(out[0][others].view(torch.int32), out[1][others].view(torch.int32))
+    assert torch.isnan(out[1][at]).all() and torch.isfinite(out[0]).all()
+
+
 @pytest.mark.parametrize("bits,d,f,e,k,fs,t,with_delta", [
     (4, 2048, 512, 256, 8, 512, 1, True),     # the headline shape's one-token instance
     (4, 2048, 512, 256, 8, 512, 5, False),    # ... its several-rows instance, no delta
