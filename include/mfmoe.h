@@ -220,7 +220,7 @@ mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_
  * a = the tanh form of GELU (int8_gelu_pytorch_tanh, :44-49) or, silu_activation != 0, SiLU
  * (FC_SHARED_INT8_ACT_SILU, :51-57); then y[d] = narrow(down . act) (dequant_int8_gemv_simd, :66-107).
  * Any t; scratch_act holds t*f bf16.  From 16 rows on the products run on the matrix cores (codes and x exact, fp32
- * sums in their order; below, in the lane order of mf_gemv).  tanh is built on this library's exp (as every exp on this path). */
+ * sums in their order, K in one run or in two halves by the number of 64-row tiles; below, in the lane order of mf_gemv).  tanh is built on this library's exp (as every exp on this path). */
 mf_status mf_shared_expert_int8(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_qtensor gate,
                                 mf_qtensor up, mf_qtensor down, uint32_t d, uint32_t f, uint32_t t,
                                 int silu_activation, uint16_t* y, uint16_t* scratch_act,

@@ -829,22 +829,9 @@ hipError_t gate_up_dispatch_t(hipStream_t s, const mf_qtensor& g, const mf_qtens
   return hipGetLastError();
 }
 
-// Picks the streaming kernel when the shape fits one of its instantiations:
-// 16-byte aligned operands, N a multiple of the group, T in {1, 2, 4}, and a
-// (wpr, ITS) split with T * ITS x-slices small enough to stay in registers.
-uint32_t device_cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return static_cast<uint32_t>(cached[dev]);
-}
-
-// waves that share a row in rows_stream_kernel (1, 2 or 4) and the 16-byte steps each takes; 0: not a shape of it
+// The streaming kernel takes a shape that fits one of its instantiations: N a multiple of the group, T in {1, 2, 4},
+// and a (wpr, ITS) split with T * ITS x-slices small enough to stay in registers.  Returns wpr, the waves that share a
+// row (1, 2 or 4), and the 16-byte steps each takes; 0: not a shape of it.
 template <int BITS, int NPROJ>
 uint32_t rows_stream_split(uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu, uint32_t& its) {
   constexpr int EPL = Fmt<BITS>::kElemsPer16B;

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // product per two groups: sum(x) of a group as three bf16 terms (all 24 bits) against the bias in three K slots.
 // Tokens are the M side, weight rows the N side: a lane ends with one weight row, its scale is a per-lane scalar.
 //
-// A workgroup is 64 weight rows (of each projection) x 64 NT tokens, waves 2 x 2.  A stage is 128 K values: x rows and
+// A workgroup is 64 weight rows (of each projection) x 64 tokens, waves 2 x 2.  A stage is 128 K values: x rows and
 // code rows come in as whole 128-byte lines, one stage ahead in registers, and are handed out through LDS (16-byte
 // pieces, XOR-swizzled so that 16 lanes reading one piece of 16 rows cover all banks): read straight from memory a
 // lane's 16 bytes of its own row touch 32 lines per load instruction, and the line rate of the L1, not the matrix
@@ -120,9 +120,11 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
 // meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
 // loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens: gate/up 47.6 -> 37.9 us, down 23.8 -> 20.0).
-template <int NPROJ, int NT, int KS>
+// (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
+// against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
+template <int NPROJ, int KS>
 __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
-  constexpr uint32_t kTok = 64 * NT;
+  constexpr uint32_t kTok = 64;
   __shared__ uint4 s_x_all[KS][2][kTok * 16];      // [token][16 pieces of 8 values], piece ^ (token & 15)
   __shared__ uint4 s_w_all[KS][2][NPROJ][64 * 8];  // [row][8 pieces of 16 codes], piece ^ ((row >> 1) & 7)
   __shared__ float s_sum_all[KS][2][kTok][2];      // sum of x over the stage's two groups
@@ -139,24 +141,21 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
   const uint32_t ng = a.N / kGroup, n_st = (ng + 1) / 2;
   const uint32_t n_walk = (n_st + KS - 1) / KS, st0 = kh * n_walk, st1 = min(n_st, st0 + n_walk);  // this set's stages
 
-  // staging roles: x -- token t / 4 (+ 64), pieces 4q .. 4q + 3 (half a group); codes -- row t / 8 (+ 32), piece t % 8
+  // staging roles: x -- token t / 4, pieces 4q .. 4q + 3 (half a group); codes -- row t / 8 (+ 32), piece t % 8
   // (whole 256-byte token rows per 16 threads measured slower: 40.4 against 37.9 us, four row addresses a thread)
   const uint32_t xt = tid >> 2, xq = tid & 3, wr = tid >> 3, wc = tid & 7;
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-  u32x4_t xr[NT][4], wreg[NPROJ][2];
+  u32x4_t xr[4], wreg[NPROJ][2];
   const uint32_t row = min(r0 + rb * 32 + m, a.M - 1);  // the lane's weight row (past the end: the last one, not stored)
   uint32_t sc[NPROJ][2], bi[NPROJ];                     // scale words of the stage's groups; the bias of group h of it
   auto fetch = [&](uint32_t st) __attribute__((always_inline)) {
     const uint32_t g = 2 * st + (xq >> 1);
     const bool in = g < ng;  // half a stage behind an odd number of groups: zeros
+    const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt, a.T - 1)) * a.N + (in ? g : ng - 1) * kGroup + (xq & 1) * 32;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt + 64 * n, a.T - 1)) * a.N + (in ? g : ng - 1) * kGroup + (xq & 1) * 32;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        xr[n][i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
-        if (!in) xr[n][i] = u32x4_t{0, 0, 0, 0};
-      }
+    for (int i = 0; i < 4; ++i) {
+      xr[i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
+      if (!in) xr[i] = u32x4_t{0, 0, 0, 0};
     }
     const uint32_t k0 = min(st * 128 + wc * 16, a.N - 16);  // (codes past the row meet x = 0)
 #pragma unroll
@@ -176,20 +175,16 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
     }
   };
   auto put = [&](uint32_t buf) __attribute__((always_inline)) {
+    float part = 0.0f;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const uint32_t tok = xt + 64 * n;
-      float part = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const u32x4_t v = xr[n][i];
-        reinterpret_cast<u32x4_t*>(s_x[buf])[tok * 16 + ((4 * xq + i) ^ (tok & 15u))] = v;
-        part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
-                ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
-      }
-      part = group_sum(part, 2);
-      if ((xq & 1) == 0) s_sum[buf][tok][xq >> 1] = part;
+    for (int i = 0; i < 4; ++i) {
+      const u32x4_t v = xr[i];
+      reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] = v;
+      part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
+              ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
     }
+    part = group_sum(part, 2);
+    if ((xq & 1) == 0) s_sum[buf][xt][xq >> 1] = part;
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
@@ -198,13 +193,12 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
         reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = wreg[p][i];
       }
   };
-  f32x16_t acc[NPROJ][NT];
+  f32x16_t acc[NPROJ];
+  const uint32_t tok_m = tb * 32 + m;  // the token whose x operands this lane reads
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[p][n][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[p][r] = 0.0f;
 
   if (st0 < st1) {
     fetch(st0);
@@ -225,34 +219,27 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
       if (st + 2 < st1) fetch(st + 2);
     }
     // biases: K slots of half h = (hi, mid, lo) of sum(x) over group 2 st + h (a group past the end sums to 0)
-#pragma unroll
-    for (int n = 0; n < NT; ++n) {
-      const float v = s_sum[buf][(tb * NT + n) * 32 + m][h];
+    {
+      const float v = s_sum[buf][tok_m][h];
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
       const float r1 = __builtin_isinf(v) ? 0.0f : v - __uint_as_float(hi);  // (an infinite sum has no rest: inf - inf would be NaN)
       const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
       const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
       const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p) acc[p][n] = mfma_bf16(av, make_uint4(bv[p] | (bv[p] << 16), bv[p], 0, 0), acc[p][n]);
+      for (int p = 0; p < NPROJ; ++p) acc[p] = mfma_bf16(av, make_uint4(bv[p] | (bv[p] << 16), bv[p], 0, 0), acc[p]);
     }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
-      uint4 bx[NT][4];
+      uint4 bx[4];
 #pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const uint32_t tok = (tb * NT + n) * 32 + m;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) bx[n][s] = s_x[buf][tok * 16 + ((8 * g + 4 * h + s) ^ (tok & 15u))];
-      }
+      for (int s = 0; s < 4; ++s) bx[s] = s_x[buf][tok_m * 16 + ((8 * g + 4 * h + s) ^ (tok_m & 15u))];
 #pragma unroll
       for (int p = 0; p < NPROJ; ++p) {
         const uint32_t r = rb * 32 + m;
-        f32x16_t tmp[NT];
+        f32x16_t tmp;
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) tmp[n][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) tmp[i] = 0.0f;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const uint4 w = s_w[buf][p][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
@@ -266,57 +253,47 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
               o[k] = __builtin_amdgcn_perm(__float_as_uint(static_cast<float>((word >> 8) & 0xFFu)),
                                            __float_as_uint(static_cast<float>(word & 0xFFu)), 0x07060302u);
             }
-            const uint4 ov = make_uint4(o[0], o[1], o[2], o[3]);
-#pragma unroll
-            for (int n = 0; n < NT; ++n) tmp[n] = mfma_bf16(bx[n][2 * c + u], ov, tmp[n]);
+            tmp = mfma_bf16(bx[2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp);
           }
         }
         const float s = __uint_as_float(scv[p][g] << 16);
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) acc[p][n][i] = __builtin_fmaf(s, tmp[n][i], acc[p][n][i]);
+        for (int i = 0; i < 16; ++i) acc[p][i] = __builtin_fmaf(s, tmp[i], acc[p][i]);
       }
     }
   }
   if constexpr (KS == 2) {  // the second set's sums to the first, over the x buffers
-    static_assert(sizeof(s_x_all) >= 4u * 64 * NPROJ * NT * 16 * sizeof(float), "the sums fit the x buffers");
+    static_assert(sizeof(s_x_all) >= 4u * 64 * NPROJ * 16 * sizeof(float), "the sums fit the x buffers");
     float* s_acc = reinterpret_cast<float*>(&s_x_all[0][0][0]);
     __syncthreads();
     if (kh == 1) {
 #pragma unroll
       for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s_acc[((p * NT + n) * 16 + i) * 256 + tid] = acc[p][n][i];
+        for (int i = 0; i < 16; ++i) s_acc[(p * 16 + i) * 256 + tid] = acc[p][i];
     }
     __syncthreads();
     if (kh == 1) return;
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[p][n][i] = acc[p][n][i] + s_acc[((p * NT + n) * 16 + i) * 256 + tid];
+      for (int i = 0; i < 16; ++i) acc[p][i] = acc[p][i] + s_acc[(p * 16 + i) * 256 + tid];
   }
   // the lane holds weight row r0 + 32 rb + m for tokens 8j + 4h + i of each 32-token block
   const uint32_t out_row = r0 + rb * 32 + m;
   if (out_row >= a.M) return;
 #pragma unroll
-  for (int n = 0; n < NT; ++n)
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t tok = t0 + (tb * NT + n) * 32 + 8 * j + 4 * h + i;
-        if (tok >= a.T) continue;
-        const size_t at = static_cast<size_t>(tok) * a.M + out_row;
-        const float v = acc[0][n][4 * j + i];
-        if constexpr (NPROJ == 2) static_cast<uint16_t*>(a.y)[at] = q8_activation(v, acc[NPROJ - 1][n][4 * j + i], a.silu != 0);
-        else if (a.out_f32) static_cast<float*>(a.y)[at] = v;
-        else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(v);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t tok = t0 + tb * 32 + 8 * j + 4 * h + i;
+      if (tok >= a.T) continue;
+      const size_t at = static_cast<size_t>(tok) * a.M + out_row;
+      const float v = acc[0][4 * j + i];
+      if constexpr (NPROJ == 2) static_cast<uint16_t*>(a.y)[at] = q8_activation(v, acc[NPROJ - 1][4 * j + i], a.silu != 0);
+      else if (a.out_f32) static_cast<float*>(a.y)[at] = v;
+      else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(v);
+    }
 }
 
 // Which kernel: from 16 token rows on the matmul (its workgroups take 64 tokens at the price of one), below that the row
@@ -327,16 +304,12 @@ static bool q8_launch(hipStream_t s, const Q8Args& a, hipError_t& err) {
     if (!aligned16(a.W[p])) return false;
   if (!aligned16(a.x) || a.N % kGroup) return false;
   if (a.T >= 16 && a.M >= 64) {
-    // 128 tokens per workgroup once 64 would give every CU more than two workgroups
-    const uint32_t slices = (a.M + 63) / 64;
-    const bool wide = slices * ((a.T + 63) / 64) > 768;
-    const uint32_t tok = wide ? 128 : 64, tiles = (a.T + tok - 1) / tok, n_work = slices * tiles;
+    // K halved among two sets of waves while there is at most a workgroup per CU (2816 x 2112: 420 rows 69 us with, 75
+    // without; 512 rows, 264 and 352 workgroups on 256 CUs, 101 and 88)
+    const uint32_t tiles = (a.T + 63) / 64, n_work = (a.M + 63) / 64 * tiles;
     const dim3 grid((n_work + 7) / 8 * 8);
-#define MF_QMM8(NT, KS) qmm8_kernel<NPROJ, NT, KS><<<grid, dim3(256 * KS), 0, s>>>(a, tiles, n_work)
-    if (wide) MF_QMM8(2, 1);
-    else if (n_work > 256) MF_QMM8(1, 1);
-    else MF_QMM8(1, 2);
-#undef MF_QMM8
+    if (n_work > device_cu_count()) qmm8_kernel<NPROJ, 1><<<grid, dim3(256), 0, s>>>(a, tiles, n_work);
+    else qmm8_kernel<NPROJ, 2><<<grid, dim3(512), 0, s>>>(a, tiles, n_work);
     err = hipGetLastError();
     return true;
   }

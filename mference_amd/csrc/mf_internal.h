@@ -70,6 +70,20 @@ hipError_t allow_lds(size_t lds, int cap) {
   return e;
 }
 
+// compute units of the current device (256 where there is none to ask); asked once per device
+inline uint32_t device_cu_count() {
+  static std::atomic<uint32_t> known[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  uint32_t n = known[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    int got = 0;
+    n = hipDeviceGetAttribute(&got, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && got > 0 ? static_cast<uint32_t>(got) : 256u;
+    known[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 // lanes of a wave that share one row of n elements (power of two, <= 64)
 inline uint32_t lanes_per_row_log2(uint32_t n, int elems_per_lane) {
   uint32_t need = (n + elems_per_lane - 1) / elems_per_lane;
