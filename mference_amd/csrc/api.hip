@@ -193,13 +193,15 @@ mf_status mf_shared_expert(mf_ctx* ctx, mf_stream stream, const uint16_t* x, mf_
   // PrefillSharedExpert.encodeBlock (PrefillSharedExpert.swift:114-172): beyond MF_MAX_TOKENS rows the projections
   // go through the matrix-core matmul when the shape allows and the scratch holds its staging rows.  Row by row the
   // weights are read once per 8 rows (2-bit: per row); a small 4-bit MLP of few rows is still faster that way
-  // (us, row by row / matmul: 1024 x 2048, 9 rows 26 / 28, 16 rows 34 / 28; 2048 x 8192, 9 rows 63 / 37;
-  // 5120 x 17408, 9 rows 121 / 77, 31 rows 329 / 81, 2-bit 1522 / 72)
+  // (us, row by row / matmul: 1024 x 2048, 9 rows 24 / 26, 16 rows 34 / 28; 2048 x 8192, 9 rows 66 / 40;
+  // 5120 x 17408, 9 rows 129 / 75, 31 rows 335 / 78, 2-bit 323 / 73)
   const bool few = bits == MF_BITS_4 && t < 16 && static_cast<uint64_t>(t) * d * f < (64ull << 20);
-  if (t > MF_MAX_TOKENS && !few && mf::dense_mlp_takes(gate, up, down, x, y, scratch_act, d, f, t) &&
-      scratch_act_bytes >= mf::dense_mlp_needs(d, f, t)) {
-    MF_HIP(ctx, mf::launch_dense_mlp(s, gate, up, down, bits, x, y, d, f, t, scratch_act));
-    return MF_OK;
+  if (t > MF_MAX_TOKENS && !few && mf::dense_mlp_takes(gate, up, down, x, y, scratch_act, d, f, t)) {
+    const uint32_t windows = mf::dense_windows(t, d, f);
+    if (scratch_act_bytes >= mf::dense_mlp_needs(d, f, t, windows)) {
+      MF_HIP(ctx, mf::launch_dense_mlp(s, gate, up, down, bits, x, y, d, f, t, windows, scratch_act));
+      return MF_OK;
+    }
   }
   // row by row otherwise (PrefillSharedExpert.swift:174-190), MF_MAX_TOKENS rows per pair of launches
   for (uint32_t t0 = 0; t0 < t; t0 += MF_MAX_TOKENS) {

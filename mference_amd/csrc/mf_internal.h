@@ -209,10 +209,13 @@ hipError_t launch_dense_qmm(hipStream_t s, const mf_qtensor& w, int bits, const 
                             uint32_t n, uint32_t k, bool out_f32, void* workspace);
 bool dense_mlp_takes(const mf_qtensor& gate, const mf_qtensor& up, const mf_qtensor& down, const void* x,
                      const void* y, const void* scratch, uint32_t d, uint32_t f, uint32_t t);
-size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t);
+// K windows of a projection; an MLP's down projection gets its from the caller, who has asked for the size with them
+uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k);
+size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows);
 size_t dense_mlp_scratch_bytes(uint32_t d, uint32_t f, uint32_t t);
 hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const mf_qtensor& down,
-                            int bits, const uint16_t* x, uint16_t* y, uint32_t d, uint32_t f, uint32_t t, void* scratch);
+                            int bits, const uint16_t* x, uint16_t* y, uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows,
+                            void* scratch);
 hipError_t launch_prefill_router(hipStream_t s, const uint16_t* W, const uint16_t* x, uint32_t E,
                                  uint32_t D, uint32_t T, uint32_t x_stride, float* logits);
 }  // namespace mf

@@ -20,7 +20,9 @@
 // (Metal/Prefill/prefill.metal:748-820), prefill_moe_reduce_token_major
 // (:631-652) and the staged-affine tensor-core QMM
 // mpp_prefill_affine_threadgroup_f16 (Metal/TensorCore/tensorops.metal:13-105).
+#include <algorithm>
 #include <type_traits>
+#include <vector>
 
 #include "mf_device.h"
 #include "mf_internal.h"
@@ -2365,48 +2367,71 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(const float* __restr
 
 // Windows of a contraction of length k for m rows of n results.  At least as many as the scale tables ask for; more where
 // the work items (64 rows of x, 128 or 256 weight rows, one window) would leave the chip idle or its last round nearly
-// empty.  Two items share a CU; an item costs about 3.6 us per 8 groups and 4.7 for its set-up, the
-// windows' sums their bytes and a launch (fitted to n = 5120, k = 17408, m = 32 .. 512: the choice is the best
-// or within 2 % of it; m = 32, 5 -> 12 windows, 101 -> 87 us for the MLP; m = 150, 5 -> 7, 172 -> 158; m = 512, 5 -> 6, 401 -> 389).
+// empty.  A round is two items a CU, whose time follows the longest window: 4 us per 8 groups and 1.5; a last round of at
+// most one item a CU has the CU to itself, 3 us per 8 groups and 1 less.  The windows' sums cost their bytes, written and read at 8 TB/s,
+// and 2 us.  (Fitted to 13 shapes, n 1024 .. 5120, k 1024 .. 17408, 9 .. 2048 rows, every count of windows timed: 0.5 % from
+// the best on average, 10 % at worst; the fewest windows 35 % and 126 %.  us for the projection, fewest / chosen:
+// 5120 x 17408, 9 rows 38.2 / 28.2 (5, 9 windows), 150 rows 79.1 / 65.5 (7), 512 rows 164 / 149 (6); 1152 x 3200, 32 rows
+// 31.8 / 16.5 (1, 6); 2048 x 8192, 64 rows 54.1 / 26.1 (2, 16); 4096 x 14336, 32 rows 39.2 / 25.8 (4, 15).)
 // The choice follows the number of 64-row tiles, not m: a row's sums come out the same in every block of that many tiles.
 // From kWholeRounds rounds of the fewest windows on an emptier last round is no longer worth the windows' bytes.
-constexpr uint32_t kWindowSlots = 2 * 256, kWholeRounds = 8;
+constexpr uint32_t kWholeRounds = 8;
 static uint32_t dense_tile_items(uint32_t n) {
   const uint32_t slice_rows = n % (2 * kQmmRows) == 0 ? 2 * kQmmRows : kQmmRows;
   return (n + slice_rows - 1) / slice_rows;
 }
 static uint32_t dense_fewest_windows(uint32_t k) { return std::max(1u, (k / kGroup + kDenseWindow - 1) / kDenseWindow); }
-static uint32_t dense_windows_of_tiles(uint32_t tiles, uint32_t n, uint32_t k) {
-  const uint32_t ng = k / kGroup, steps = (ng + 7) / 8;
+// (as the differences of dense_window_start, which steps by ng / n_win, without a division a window)
+static uint32_t dense_longest_window(uint32_t ng, uint32_t n_win) {
+  const uint32_t whole = ng / n_win, part = ng % n_win;
+  uint32_t longest = 0, at = 0, over = 0, start = 0;
+  for (uint32_t w = 1; w < n_win; ++w) {
+    at += whole;
+    over += part;
+    if (over >= n_win) { over -= n_win; ++at; }
+    longest = std::max(longest, (at & ~7u) - start);
+    start = at & ~7u;
+  }
+  return std::max(longest, ng - start);
+}
+// longest(w): groups of the longest of w windows
+template <typename Longest>
+static uint32_t dense_windows_of_tiles(uint32_t tiles, uint32_t n, uint32_t k, Longest longest) {
+  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, k / kGroup / 8), num_cu = device_cu_count();
   const uint64_t items = static_cast<uint64_t>(tiles) * dense_tile_items(n);
-  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, ng / 8);
-  if (items * lo >= kWholeRounds * kWindowSlots) return lo;
+  if (items * lo >= kWholeRounds * 2ull * num_cu) return lo;
   uint32_t best = lo;
   double best_us = 0.0;
   for (uint32_t w = lo; w <= hi; ++w) {
-    const double rounds = static_cast<double>((items * w + kWindowSlots - 1) / kWindowSlots);
-    double us = rounds * (3.6 * ((steps + w - 1) / w) + 4.7);
-    if (w > 1) us += 4.0 + static_cast<double>(w) * tiles * kTileTokens * n * 8.0 / 5.0e6;
+    const double steps = longest(w) / 8.0;
+    const uint32_t all = static_cast<uint32_t>(items) * w, rounds = all / (2 * num_cu), rest = all % (2 * num_cu);
+    double us = (rounds + (rest > num_cu)) * (4.0 * steps + 1.5);
+    if (rest > 0 && rest <= num_cu) us += 3.0 * steps - 1.0;
+    if (w > 1) us += 2.0 + static_cast<double>(w) * tiles * kTileTokens * n * 8.0 / 8.0e6;
     if (w == lo || us < best_us) { best = w; best_us = us; }
   }
   return best;
 }
-static uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k) {
-  return dense_windows_of_tiles((m + kTileTokens - 1) / kTileTokens, n, k);
+uint32_t dense_windows(uint32_t m, uint32_t n, uint32_t k) {
+  return dense_windows_of_tiles((m + kTileTokens - 1) / kTileTokens, n, k, [&](uint32_t w) { return dense_longest_window(k / kGroup, w); });
 }
 
 // bytes of fp32 window results a projection of n rows over m tokens needs (0: one window, written directly)
-static size_t dense_parts_bytes(uint32_t m, uint32_t n, uint32_t k) {
-  const uint32_t n_win = dense_windows(m, n, k);
+static size_t dense_parts_bytes(uint32_t m, uint32_t n, uint32_t n_win) {
   return n_win > 1 ? up256(sizeof(float) * static_cast<size_t>(m) * n) * n_win : 0;
 }
 // ... and the most any call of up to m tokens needs: fewer tiles can take more windows, so the bytes of a single call do
-// not grow with its rows (5120 x 17408: 37.4 MB for 128 rows, 24.5 for 129).  Only tile counts below kWholeRounds differ.
+// not grow with its rows (5120 x 17408: 27.5 MB of results for 192 rows, 24.6 for 200).  Only tile counts below kWholeRounds differ.
 static size_t dense_parts_bytes_up_to(uint32_t m, uint32_t n, uint32_t k) {
-  size_t most = dense_parts_bytes(m, n, k);
-  const uint64_t row = static_cast<uint64_t>(dense_tile_items(n)) * dense_fewest_windows(k);
-  const uint32_t tiles = static_cast<uint32_t>(std::min<uint64_t>((m - 1) / kTileTokens, kWholeRounds * kWindowSlots / row + 1));
-  for (uint32_t i = 1; i <= tiles; ++i) most = std::max(most, dense_parts_bytes(i * kTileTokens, n, k));
+  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, k / kGroup / 8);
+  std::vector<uint32_t> longest(hi + 1);
+  for (uint32_t w = lo; w <= hi; ++w) longest[w] = dense_longest_window(k / kGroup, w);
+  const auto of_tiles = [&](uint32_t tiles) { return dense_windows_of_tiles(tiles, n, k, [&](uint32_t w) { return longest[w]; }); };
+  size_t most = dense_parts_bytes(m, n, of_tiles((m + kTileTokens - 1) / kTileTokens));
+  const uint64_t row = static_cast<uint64_t>(dense_tile_items(n)) * lo;
+  const uint32_t tiles = static_cast<uint32_t>(std::min<uint64_t>((m - 1) / kTileTokens, kWholeRounds * 2ull * device_cu_count() / row + 1));
+  for (uint32_t i = tiles; i > 0 && dense_parts_bytes(i * kTileTokens, n, hi) > most; --i)
+    most = std::max(most, dense_parts_bytes(i * kTileTokens, n, of_tiles(i)));
   return most;
 }
 // ... and of the gate / up pair of an MLP (both projections of a work item: kQmmRows rows each)
@@ -2475,15 +2500,15 @@ bool dense_qmm_takes(const mf_qtensor& w, int bits, const void* x, const void* y
 static size_t dense_qmm_rows_bytes(uint32_t m, uint32_t k) {
   return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup));
 }
-size_t dense_qmm_needs(uint32_t m, uint32_t n, uint32_t k) { return dense_qmm_rows_bytes(m, k) + dense_parts_bytes(m, n, k); }
+size_t dense_qmm_needs(uint32_t m, uint32_t n, uint32_t k) { return dense_qmm_rows_bytes(m, k) + dense_parts_bytes(m, n, dense_windows(m, n, k)); }
 size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
   return dense_qmm_rows_bytes(m, k) + dense_parts_bytes_up_to(m, n, k);
 }
 
 // x_prepared: rows already in the matmul's order with their group sums in sumx (x is then ignored)
 static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, const uint16_t* xp, const float* sumx,
-                                void* y, uint32_t m, uint32_t n, uint32_t k, bool out_f32, void* parts) {
-  const uint32_t ng = k / kGroup, n_win = dense_windows(m, n, k);
+                                void* y, uint32_t m, uint32_t n, uint32_t k, uint32_t n_win, bool out_f32, void* parts) {
+  const uint32_t ng = k / kGroup;
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
   QmmArgs d{};
   d.dense_mode = 1; d.dense_rows = m; d.top_k = 1;
@@ -2500,10 +2525,7 @@ static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, co
   if (n_win == 1) {
     d.kdim = k; d.epi = out_f32 ? 1 : 2; d.out = y;
   } else {  // all windows in one launch, each writing fp32 into its own buffer
-    uint32_t longest = 0;
-    for (uint32_t wdx = 0; wdx < n_win; ++wdx)
-      longest = std::max(longest, dense_window_start(ng, n_win, wdx + 1) - dense_window_start(ng, n_win, wdx));
-    d.kdim = longest * kGroup; d.n_win = n_win; d.out_win_stride = part_stride; d.epi = 1; d.out = parts;
+    d.kdim = dense_longest_window(ng, n_win) * kGroup; d.n_win = n_win; d.out_win_stride = part_stride; d.epi = 1; d.out = parts;
   }
   {
     const hipError_t e = launch_qmm(s, code_bits, d, d.pair_rows ? 2 : 1, tiles, nullptr, 0);
@@ -2526,7 +2548,7 @@ hipError_t launch_dense_qmm(hipStream_t s, const mf_qtensor& w, int bits, const 
   void* parts = reinterpret_cast<uint8_t*>(sumx) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup));
   const hipError_t e = launch_prep_rows(s, x, xp, sumx, static_cast<size_t>(m) * k);
   if (e != hipSuccess) return e;
-  return dense_project(s, w, bits, xp, sumx, y, m, n, k, out_f32, parts);
+  return dense_project(s, w, bits, xp, sumx, y, m, n, k, dense_windows(m, n, k), out_f32, parts);
 }
 
 // The block form of the shared expert / dense SwiGLU MLP: gate and up in one launch with the SwiGLU epilogue
@@ -2543,15 +2565,16 @@ static size_t dense_mlp_rows_bytes(uint32_t d, uint32_t f, uint32_t t) {
          up256(sizeof(float) * static_cast<size_t>(t) * (d / kGroup)) + up256(sizeof(float) * static_cast<size_t>(t) * (f / kGroup));
 }
 // (the window results of gate / up and of down follow one another in the same place)
-size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t) {
-  return dense_mlp_rows_bytes(d, f, t) + std::max(dense_parts_bytes(t, d, f), dense_gate_up_parts_bytes(t, f, d));
+size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows) {
+  return dense_mlp_rows_bytes(d, f, t) + std::max(dense_parts_bytes(t, d, down_windows), dense_gate_up_parts_bytes(t, f, d));
 }
 size_t dense_mlp_scratch_bytes(uint32_t d, uint32_t f, uint32_t t) {
   return dense_mlp_rows_bytes(d, f, t) + std::max(dense_parts_bytes_up_to(t, d, f), dense_gate_up_parts_bytes(t, f, d));
 }
 
 hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qtensor& up, const mf_qtensor& down,
-                            int bits, const uint16_t* x, uint16_t* y, uint32_t d, uint32_t f, uint32_t t, void* scratch) {
+                            int bits, const uint16_t* x, uint16_t* y, uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows,
+                            void* scratch) {
   uint8_t* base = static_cast<uint8_t*>(scratch);
   uint16_t* act = reinterpret_cast<uint16_t*>(base);
   base += up256(sizeof(uint16_t) * static_cast<size_t>(t) * f);
@@ -2581,10 +2604,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     const size_t part_stride = up256(sizeof(float) * static_cast<size_t>(t) * f) / sizeof(float);
     float* pg = reinterpret_cast<float*>(base);
     float* pu = pg + part_stride * gu_win;
-    uint32_t longest = 0;
-    for (uint32_t wdx = 0; wdx < gu_win; ++wdx)
-      longest = std::max(longest, dense_window_start(ng, gu_win, wdx + 1) - dense_window_start(ng, gu_win, wdx));
-    q.ng_ld = ng; q.kdim = longest * kGroup; q.n_win = gu_win; q.out_win_stride = part_stride;
+    q.ng_ld = ng; q.kdim = dense_longest_window(ng, gu_win) * kGroup; q.n_win = gu_win; q.out_win_stride = part_stride;
     q.epi = 1; q.out = pg; q.out2 = pu;
     e = launch_qmm(s, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
     if (e != hipSuccess) return e;
@@ -2599,7 +2619,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     e = launch_prep_rows(s, act, nullptr, sum_act, static_cast<size_t>(t) * f);  // the activations are in matmul order already
     if (e != hipSuccess) return e;
   }
-  return dense_project(s, down, bits, act, sum_act, y, t, d, f, false, base);
+  return dense_project(s, down, bits, act, sum_act, y, t, d, f, down_windows, false, base);
 }
 
 // entries of the tile list: every live expert may end in a partial tile; a multiple of 8

@@ -54,6 +54,7 @@ def _offset_tensor(arr, offset_bytes):
     (17, 35, 128, True, (13, 2, 6)),                    # the reference's four cases (:191-205)
     (64, 128, 128, True, (0, 0, 0)), (96, 256, 2048, False, (0, 0, 0)), (33, 384, 4352, False, (0, 0, 0)),
     (130, 128, 8320, True, (0, 0, 0)),                  # matrix-core path: one window, two, three
+    (9, 128, 2176, True, (0, 0, 0)), (40, 1152, 3200, False, (0, 0, 0)), (65, 256, 1152, True, (0, 0, 0)),  # windows of uneven length
 ])
 def test_qmm_matches_reference_test_inputs(gpu, oracle, m, n, k, adversarial, offsets):
     q, xb = _reference_inputs(oracle, m, n, k, adversarial)
