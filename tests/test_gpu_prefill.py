@@ -117,7 +117,7 @@ def _run_prefill(moe, wts, x, t, d, k):
     (4, 2048, 512, 256, 8, 512, 96, 0, 0.0),   # the headline layer shape
     (4, 512, 256, 16, 4, 128, 90, 0, 0.0),     # shared width != routed width: the two down projections differ in K
     (4, 256, 384, 16, 4, 384, 67, 0, 0.0),     # K of the down projection not 128, 256 or 512
-    # 2-bit routed experts with a 4-bit shared expert (the shared matmuls are launches of their own)
+    # 2-bit routed experts with a 4-bit shared expert (both in one launch per phase)
     (2, 256, 128, 16, 4, 128, 70, 0, 0.0),
     (2, 512, 256, 32, 6, 256, 200, 0, 7.0),    # top-6 + SwiGLU clamp (moe.metal:902-1195)
     (2, 1024, 512, 16, 6, 0, 133, 0, 0.0),     # K a multiple of 512 (whole-table vector loads), no shared expert
@@ -194,7 +194,7 @@ def test_skewed_qwen_prefill_against_the_checker(gpu, oracle, t):
 @pytest.mark.parametrize("bits,d,f,e,k,fs,t,mode", [
     (4, 512, 256, 32, 8, 256, 1100, 0),    # 8800 routes, the shared expert rides along
     (4, 1024, 128, 16, 8, 0, 1031, 0),     # few experts: long runs, an odd tile out at the end of every run
-    (2, 512, 256, 16, 6, 128, 1500, 0),    # 2-bit codes; the 4-bit shared expert is a launch of its own
+    (2, 512, 256, 16, 6, 128, 1500, 0),    # 2-bit codes beside a 4-bit shared expert
     (1, 512, 128, 32, 8, 0, 1030, 1),      # ternary rows, full-softmax router
     (4, 128, 128, 100, 3, 0, 3000, 0),     # 94 chunks of 32 tokens (two per wave of the selecting launch), 3 routes each
     (4, 128, 128, 24, 1, 128, 8500, 0),    # 133 chunks of 64 tokens, one route per token

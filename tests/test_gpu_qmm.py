@@ -189,3 +189,50 @@ def test_mlp_block_in_a_scratch_sized_for_more_rows(gpu, oracle, d, f, most, row
             assert bool((buf[size:] == 0xA5).all())
             got.append(ops.bf16_bits(y))
         assert np.array_equal(got[0], got[1]), t
+
+
+@pytest.mark.parametrize("bits", [4, 2, 1])
+@pytest.mark.parametrize("d,f,t", [(256, 192, 9), (1152, 640, 16), (192, 3200, 31), (320, 448, 20)])
+def test_mlp_block_of_few_rows(gpu, oracle, bits, d, f, t):
+    """9 to 31 rows of the dense MLP (4-bit: row by row up to 15 rows of these sizes; else the matmul), every format"""
+    rng = oracle.Rng.key(0xF03, f"mlp-few-{bits}-{d}-{f}")
+    def weights(r, c):
+        if bits != 1:
+            return oracle.quantize(rng.normal(0.0, 0.02, r * c).reshape(r, c), bits)
+        codes = np.digitize(rng.uniform_fill(0.0, 1.0, r * c), (0.25, 0.75)).astype(np.uint8).reshape(r, c)
+        scales = oracle.bf16_bits((np.abs(rng.normal(0.0, 0.02, r * c // 64)) + 1e-3).astype(np.float32).reshape(r, c // 64))
+        return oracle.QTensor(oracle.pack_codes(codes, 1), scales, None, 1, r, c)
+    qs = [weights(f, d), weights(f, d), weights(d, f)]
+    xb = oracle.bf16_bits(rng.normal(0.0, 1.0, t * d).reshape(t, d))
+    ref = np.stack([oracle.shared_expert(*qs, xb[i]) for i in range(t)])
+    op = ops.SharedExpertInt4(gpu)
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    scratch = torch.zeros(op.scratch_bytes(d, f, t), dtype=torch.uint8, device="cuda")
+    op.encode(ops.bf16_tensor(xb), *[to_device_q(q) for q in qs], y, scratch, t=t)
+    torch.cuda.synchronize()
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(ref), f"bits={bits} d={d} f={f} t={t}")
+
+
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("d,f,t", [(1152, 640, 20), (256, 3200, 70)])
+def test_mlp_block_keeps_infinities_to_their_row(gpu, bits, d, f, t):
+    """rows with an infinity or a NaN come out NaN (the code offset is taken out as inf - inf, as in the row kernels) and
+    leave every other row's bits alone"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + t + bits)
+    def q(rows, n):
+        table = lambda s: (s * (0.01 + 0.01 * torch.rand(rows, n // 64, generator=gen, device="cuda"))).to(torch.bfloat16)
+        return ops.QuantizedTensor(torch.randint(0, 256, (rows, n * bits // 8), dtype=torch.uint8, generator=gen, device="cuda"), table(1), table(-2), bits, rows, n)
+    qs = [q(f, d), q(f, d), q(d, f)]
+    x = torch.randn(t, d, generator=gen, device="cuda").to(torch.bfloat16)
+    wild, at = x.clone(), [1, t // 2, t - 1]
+    wild[1, d // 2], wild[t // 2, 5], wild[t - 1, d - 1] = float("inf"), float("-inf"), float("nan")
+    op = ops.SharedExpertInt4(gpu)
+    out = []
+    for rows in (x, wild):
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        op.encode(rows, *qs, y, torch.zeros(op.scratch_bytes(d, f, t), dtype=torch.uint8, device="cuda"), t=t)
+        out.append(y)
+    others = [i for i in range(t) if i not in at]
+    assert torch.equal(out[0][others].view(torch.int16), out[1][others].view(torch.int16))
+    assert torch.isnan(out[1][at]).all() and torch.isfinite(out[0]).all()
