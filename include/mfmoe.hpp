@@ -206,7 +206,7 @@ class SharedExpertInt4 {
     check(mf_shared_expert(ctx_, commandBuffer, x, gate, up, down, bits_, d, f, tokens, y, scratchAct,
                            scratchActBytes), ctx_);
   }
-  // scratch the block form (PrefillSharedExpert.encodeBlock, from 32 rows on) can use
+  // scratch the block form (PrefillSharedExpert.encodeBlock, beyond MF_MAX_TOKENS rows) can use; serves fewer rows too
   static size_t scratchBytes(uint32_t d, uint32_t f, uint32_t tokens) { return mf_shared_expert_scratch_bytes(d, f, tokens); }
   // the same operator without a scratch argument and without device allocation (the activations go
   // through a device array inside the library; tokens * f <= MF_STATIC_ACT_ELEMS, calls must not overlap)

@@ -7,10 +7,12 @@
 //      -> every workgroup gathers the logits and selects the top-k itself (cheap and
 //         deterministic: rank counting over the logits in LDS, all waves)
 //   B  routed gate/up/activation rows of the K selected experts of every token
-//   C  per token: the shared expert's down rows of this workgroup's output rows
-//      (-> gated h1, kept in LDS), then the routed down rows: K waves take the K
-//      slots of one group of output rows, weight them, and one thread per row
-//      adds them to h1 in rank order.
+//   C  the workgroups are split among the tokens, each owns output rows of one: the
+//      shared expert's down rows of those rows (-> gated h1, kept in LDS), then the
+//      routed down rows.  With one or two units of rows per workgroup K waves take the
+//      K slots of a unit, weight them, and one thread per row adds them to h1 in rank
+//      order; with three and more a wave takes all K slots of its units one after the
+//      other, four rows requested ahead.
 //
 // Workgroups exchange three small vectors through HBM: logits, shared
 // activations, routed activations.  There is no grid barrier.  Every exchanged

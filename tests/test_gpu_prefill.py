@@ -343,6 +343,25 @@ def test_prefill_of_few_rows_takes_the_decode_launch(gpu, oracle, bits, e, fs, t
     assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref_y), f"bits={bits} t={t}")
 
 
+@pytest.mark.parametrize("bits", [4, 2, 1])
+def test_tiled_pool_has_the_documented_order(gpu, oracle, bits):
+    """mf_moe_tile_experts byte for byte: per block of 32 rows, runs of 64 pieces of 16 bytes, piece m + 32 h for row m --
+    4-bit: a run per K group, half h of it; 2-bit, ternary: a run per two groups, half h of each; the rest unchanged"""
+    layer = oracle.synth_layer(ROOT_SEED + 0xA2B0, 256, 128, 8 if bits != 1 else 32, 4, bits=bits, fs=0, router_mode=1 if bits == 1 else 0)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    got = moe.tile_experts(wts.experts, wts.offsets).cpu().numpy()
+    want = wts.experts.cpu().numpy().copy()
+    for at, rows, cols in ((wts.offsets.gate_w, 128, 256), (wts.offsets.up_w, 128, 256), (wts.offsets.down_w, 256, 128)):
+        size = rows * cols * (4 if bits == 4 else 2) // 8
+        codes = want[:, at:at + size].reshape(-1, rows // 32, 32, size // rows)  # [expert, block, m, bytes of the row]
+        if bits == 4:
+            t = codes.reshape(*codes.shape[:3], -1, 2, 16).transpose(0, 1, 3, 4, 2, 5)           # group, h, m
+        else:
+            t = codes.reshape(*codes.shape[:3], -1, 2, 2, 8).transpose(0, 1, 3, 5, 2, 4, 6)      # pair, h, m, group of the pair
+        want[:, at:at + size] = t.reshape(want.shape[0], size)
+    assert np.array_equal(got, want)
+
+
 @pytest.mark.parametrize("d,f,t", [(192, 320, 33), (1152, 704, 64), (128, 448, 130)])
 def test_dense_mlp_widths_of_whole_groups(gpu, oracle, d, f, t):
     """the block form of the dense MLP at widths that are no multiples of 128"""

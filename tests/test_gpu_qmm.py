@@ -139,7 +139,7 @@ def _close_or_one_step(oracle, got_bits, ref_bits, what):
 # that meet in the SwiGLU combine pass)
 @pytest.mark.parametrize("d,f,t", [(2048, 512, 40), (1024, 1536, 128), (5120, 1536, 33), (7680, 256, 70)])
 def test_shared_expert_block_form(gpu, oracle, d, f, t):
-    """PrefillSharedExpert.encodeBlock: t >= 32 rows through the matrix cores == the checker's shared
+    """PrefillSharedExpert.encodeBlock: many rows through the matrix cores == the oracle's shared
     expert row by row within the layer tolerance; with only t*f of scratch the call goes row by row and
     gives the bits of t calls with one row each."""
     rng = oracle.Rng.key(0xB10C, f"block-{d}-{f}-{t}")
