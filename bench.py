@@ -10,7 +10,7 @@ own weights, so every layer streams its expert bytes from HBM (40 x 453 MB of
 resident experts, far beyond the 256 MB Infinity Cache).
 
 Prints ONE JSON line: metric, value, unit, timing fields, `roofline` (dominant kernel against
-the HBM or matrix-core peak) and `cpu_baseline` (the CPU checker timed on a bounded sample).
+the HBM or matrix-core peak) and `cpu_baseline` (the CPU oracle timed on a bounded sample).
 """
 from __future__ import annotations
 
@@ -166,7 +166,7 @@ def measure_prefill(ctx, w, layer, device, tokens=(128, 512, 2048), steps=100, w
     """Ragged prefill of one layer of the same shape: T tokens, top-k routing from skewed
     logits (router weights plus a per-expert bias ~ N(0, 1.5), carried by a constant-one last
     feature of x and the last column of the router, so expert loads are uneven and some
-    experts get no token).  Parity at the smallest T against the per-token CPU checker."""
+    experts get no token).  Parity at the smallest T against the per-token CPU oracle."""
     import numpy as np
     import torch
     from mference_amd import operators as ops
@@ -205,7 +205,7 @@ def measure_prefill(ctx, w, layer, device, tokens=(128, 512, 2048), steps=100, w
         run = {"tokens": t}
         if t == min(tokens):
             host = layer_to_host(lw, w)
-            n_par = t if qwen else min(t, 16)   # the large layers: the first 16 rows (the checker is a CPU loop)
+            n_par = t if qwen else min(t, 16)   # the large layers: the first 16 rows (the oracle is a CPU loop)
             ref_y, ref_idx, _ = O.moe_layer(host, ops.bf16_bits(x[:n_par].contiguous()))
             got = O.bf16_to_float(ops.bf16_bits(y[:n_par].contiguous())).astype(np.float64)
             ref = O.bf16_to_float(ref_y).astype(np.float64)
@@ -284,7 +284,7 @@ def measure_prefill(ctx, w, layer, device, tokens=(128, 512, 2048), steps=100, w
 
 
 def _omp_threads(n):
-    """thread count of the CPU checker's OpenMP loops (libgomp of this process); None = leave"""
+    """thread count of the CPU oracle's OpenMP loops (libgomp of this process); None = leave"""
     import ctypes
     try:
         gomp = ctypes.CDLL("libgomp.so.1")
@@ -298,7 +298,7 @@ def _omp_threads(n):
 
 def bench_single_expert(args, device) -> int:
     """One SwiGLU expert FFN at batch 1 (hidden 2048, intermediate 512, 4-bit g64): the shared-expert
-    operator on one expert's projections, `layers` distinct experts in rotation; beside it the CPU checker
+    operator on one expert's projections, `layers` distinct experts in rotation; beside it the CPU oracle
     (a restatement of the reference's CPU path) single-threaded and on all cores."""
     import numpy as np
     import torch
@@ -421,21 +421,21 @@ def bench_dense_mlp(args, device) -> int:
         for l in range(L):
             mlp.encode(x, sets[l][0], sets[l][1], sets[l][2], y[l], scratch, t=t)
 
-    # parity of set 0 against the CPU checker
+    # parity of set 0 against the CPU oracle
     import numpy as np
     from oracle import mf_oracle as O
     def hq(q):
         return O.QTensor(q.packed.cpu().numpy(), ops.bf16_bits(q.scales), ops.bf16_bits(q.biases), 4, q.rows, q.n)
     step()
     torch.cuda.synchronize()
-    rows = list(range(t)) if t <= 8 else sorted({0, 1, t // 2, t - 1})  # the checker takes ~1 s per row
+    rows = list(range(t)) if t <= 8 else sorted({0, 1, t // 2, t - 1})  # the oracle takes ~1 s per row
     h0 = [hq(q) for q in sets[0]]
     t_cpu = time.perf_counter()
     ref = np.stack([O.shared_expert(h0[0], h0[1], h0[2], ops.bf16_bits(x[i])) for i in rows])
     cpu_us_per_row = (time.perf_counter() - t_cpu) / len(rows) * 1e6
     cores = int(os.environ.get("OMP_NUM_THREADS") or min(16, os.cpu_count() or 1))
     cpu_baseline = {"value": round(cpu_us_per_row * t, 1), "unit": "us", "cores": cores, "kind": "port",
-                    "sample": f"{len(rows)} token rows of weight set 0 through the CPU checker, scaled to {t} rows"}
+                    "sample": f"{len(rows)} token rows of weight set 0 through the CPU oracle, scaled to {t} rows"}
     got = O.bf16_to_float(ops.bf16_bits(y[0][rows])).astype(np.float64)
     reff = O.bf16_to_float(ref).astype(np.float64)
     parity = dict(max_abs=float(np.abs(got - reff).max()),
@@ -566,7 +566,7 @@ def measure_given_routing(ctx, device, layers=16, replays=50):
 def bench_family_routers(args, device) -> int:
     """The four family routers at their reference shapes, T = 1 (decode) and T = 2048 (prefill): µs per
     call from HIP-graph replays, the decode call against the HBM roofline of its router bytes, and the
-    routing of row 0 against the CPU checker bit for bit.  `sets` distinct weight sets rotate at T = 1."""
+    routing of row 0 against the CPU oracle bit for bit.  `sets` distinct weight sets rotate at T = 1."""
     import numpy as np
     import torch
     from mference_amd import operators as ops
@@ -764,9 +764,9 @@ def phase_trace(ctx, w, stack, moes, device, with_norm=False) -> int:
 
 
 OTHER_CONFIGS = [
-    # (key, BASELINE.json configuration, extra arguments of this script)
+    # (key, number of the configuration, extra arguments of this script)
     ("single_expert_ffn_T1", 0, ["--workload", "single-expert", "--steps", "20", "--warmup", "5"]),
-    # the headline layer at the token count of an MTP verification step (not a BASELINE row of its own)
+    # the headline layer at the token count of an MTP verification step (no configuration of its own)
     ("qwen_layer_T4", 1, ["--tokens", "4", "--steps", "100", "--warmup", "10"]),
     ("large_2bit_layer_T1", 3, ["--workload", "dsv4-2bit", "--steps", "100", "--warmup", "10"]),
     ("large_2bit_layer_T4", 3, ["--workload", "dsv4-2bit", "--tokens", "4", "--steps", "100", "--warmup", "10"]),
@@ -777,10 +777,10 @@ OTHER_CONFIGS = [
 
 
 def measure_other_configs(cpu_seconds: float, budget_s: float = 400.0) -> dict:
-    """The remaining BASELINE.json configurations, each measured by this script in a child process of its
+    """The remaining configurations, each measured by this script in a child process of its
     own (one GPU, one after the other, after the headline's timed region) and reduced to a few fields:
-    time, algorithmic bytes, achieved rate and fraction of the HBM peak, parity against the CPU checker
-    and the checker's own time."""
+    time, algorithmic bytes, achieved rate and fraction of the HBM peak, parity against the CPU oracle
+    and the oracle's own time."""
     import subprocess
     out, t_start = {}, time.perf_counter()
     for key, cfg, extra in OTHER_CONFIGS:
@@ -827,7 +827,7 @@ def main() -> int:
     ap.add_argument("--cpu-seconds", type=float, default=12.0)
     ap.add_argument("--no-prefill", action="store_true", help="skip the ragged prefill section")
     ap.add_argument("--no-other-configs", action="store_true",
-                    help="skip the short runs of the other BASELINE configurations that the default run appends")
+                    help="skip the short runs of the other configurations that the default run appends")
     ap.add_argument("--with-norm", action="store_true",
                     help="with --phase-trace: the launch that makes x itself (mf_moe_decode_layer_normed)")
     ap.add_argument("--no-side-runs", action="store_true",
@@ -899,7 +899,7 @@ def main() -> int:
         for l in range(L):
             moes[l].encode_decode_layer(stack[l], xs[l], ys[l], t=w["t"])
 
-    # ---- parity of layer 0 at full size against the CPU checker
+    # ---- parity of layer 0 at full size against the CPU oracle
     from oracle import mf_oracle as O
     host0 = layer_to_host(stack[0], w)
     host0.router_mode = 1 if w["bits"] == 1 else 0
@@ -1049,7 +1049,7 @@ def main() -> int:
     if not args.no_prefill:
         out["prefill"] = measure_prefill(ctx, w, stack[0], device, use_graph=not args.no_graph)
     if not args.no_cpu_baseline:
-        # the CPU checker (a restatement of the reference's CPU path: bulk
+        # the CPU oracle (a restatement of the reference's CPU path: bulk
         # dequantize each row, scalar fp32 dot, experts in slot order) timed on
         # layer 0 for about cpu-seconds of work
         cores = int(os.environ.get("OMP_NUM_THREADS") or min(16, os.cpu_count() or 1))

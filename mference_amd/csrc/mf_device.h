@@ -47,7 +47,7 @@ __device__ __forceinline__ float round_bf16(float x) { return bf16_to_f(f_to_bf1
 
 // ------------------------------------------------------------------- exp
 
-// Deterministic exp: the same sequence of IEEE operations as the CPU checker,
+// Deterministic exp: the same sequence of IEEE operations as the CPU oracle,
 // so routing weights agree bit for bit.  Results below e^-86 are 0.
 __device__ __forceinline__ float mf_exp(float x) {
   if (x != x) return x;
@@ -70,7 +70,7 @@ __device__ __forceinline__ float mf_exp(float x) {
 }
 
 // log(t) for 1 <= t <= 2 (t = 1 + exp(-|x|) in the routers): 2*atanh((t-1)/(t+1)), odd series
-// through s^15; the same IEEE sequence as the CPU checker.
+// through s^15; the same IEEE sequence as the CPU oracle.
 __device__ __forceinline__ float mf_log_1to2(float t) {
   const float s = (t - 1.0f) / (t + 1.0f);
   const float z = s * s;
@@ -97,7 +97,7 @@ __device__ __forceinline__ float mf_silu(float x) { return x / (1.0f + mf_exp(-x
 
 // int8_gelu_pytorch_tanh (Metal/Quant/dequant_int8.metal:44-49): 0.5 x (1 + tanh(c (x + 0.044715 x^3))), the
 // argument clamped to +-20; tanh(z) = 1 - 2 / (exp(2 z) + 1) on this build's exp, the same IEEE sequence as the
-// CPU checker.
+// CPU oracle.
 __device__ __forceinline__ float mf_gelu_tanh(float x) {
   const float x3 = x * x * x;
   float inner = 0.7978845608028654f * (x + 0.044715f * x3);

@@ -1,6 +1,6 @@
 // Router device functions shared by the stand-alone router kernels and the
 // fused decode layer: the fixed-order bf16 row dot and the one-wave top-k
-// selectors.  Both are bit-exact against the CPU checker.
+// selectors.  Both are bit-exact against the CPU oracle.
 #pragma once
 
 #include "mf_device.h"

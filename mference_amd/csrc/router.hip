@@ -1,5 +1,5 @@
 // Router: bf16 GEMV to fp32 logits and the top-k selectors.  Both are
-// bit-exact against the CPU checker: the logit summation order is fixed (see
+// bit-exact against the CPU oracle: the logit summation order is fixed (see
 // dot_bf16_row) and exp/divide are IEEE sequences shared with it.
 #include "mf_device.h"
 #include "mf_internal.h"

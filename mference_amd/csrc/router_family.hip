@@ -1,6 +1,6 @@
 // Family-specific routers: DeepSeek-V4 sqrtsoftplus selection and hash weighting, the Inkling
 // sigmoid router with shared sinks, and Gemma's 8-bit affine router rows with per-expert scales.
-// All share the tie rule of the plain top-k selector and are bit-exact against the CPU checker:
+// All share the tie rule of the plain top-k selector and are bit-exact against the CPU oracle:
 // exp, log and the summation orders are fixed IEEE sequences, divide and sqrt are correctly rounded.
 #include "mf_device.h"
 #include "mf_internal.h"

@@ -1,7 +1,7 @@
 /*
  * mf_oracle.c — CPU restatement of Mference's MoE expert hot path.
  *
- * TEST INFRASTRUCTURE ONLY: the checker for the HIP kernels.  Nothing in the
+ * TEST INFRASTRUCTURE ONLY: the oracle for the HIP kernels.  Nothing in the
  * product library links, loads or calls this file.
  *
  * Build: gcc -O3 -march=native -ffp-contract=off -fopenmp (see Makefile).

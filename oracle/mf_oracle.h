@@ -1,7 +1,7 @@
 /*
  * mf_oracle — CPU restatement of Mference's MoE expert hot path.
  *
- * TEST INFRASTRUCTURE ONLY.  This library is the checker for the HIP kernels:
+ * TEST INFRASTRUCTURE ONLY.  This library is the oracle for the HIP kernels:
  * only the test-suite, the smoke check and the benchmark's cpu_baseline leg may
  * load it.  The product library (libmfmoe) never links or calls it.
  *

@@ -1,7 +1,7 @@
 // Drives libmfmoe through the C++ mirror of the reference's operator classes
-// (include/mfmoe.hpp) and checks the results against the CPU checker, the way the reference's
+// (include/mfmoe.hpp) and checks the results against the CPU oracle, the way the reference's
 // own XCTest cases drive its Swift operators: SeedTree-seeded inputs, one small layer,
-// decode == per-token checker, ragged prefill == per-token checker, family routers bit for bit,
+// decode == per-token oracle, ragged prefill == per-token oracle, family routers bit for bit,
 // grouping KATs and errors.
 //
 //   mirror_test cpu   grouping KATs and error cases only (no GPU needed)
@@ -72,7 +72,7 @@ static void test_grouping() {
   EXPECT(routes.groups.size() == 3 && routes.tiles.size() == 2, "groups %zu tiles %zu", routes.groups.size(),
          routes.tiles.size());
   EXPECT(routes.maxPairsPerExpert() == 3 && routes.maxPairsPerTile() == 5, "max pairs");
-  // the same result as the checker's restatement
+  // the same result as the oracle's restatement
   std::vector<mfo_pair> op(6), os(6);
   mfo_make_pairs(idx, wb, 3, 2, op.data());
   std::vector<uint32_t> oo(4), oc(4);
@@ -310,7 +310,7 @@ static void test_layer() {
 
 // ---------------------------------------------------------------- family routers (GPU)
 // The DeepSeek-V4 selector and the Inkling router through the mirror classes, bit for bit against
-// the checker on seeded inputs.
+// the oracle on seeded inputs.
 static void test_family_routers(const mf::MetalContext& ctx) {
   const uint32_t e = 64, shared = 2, d = 256, t = 3, k = 6;
   mfo_rng rng = mfo_seed_tree_key(0x4D464D4F0000FA40ull, "family");

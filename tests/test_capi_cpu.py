@@ -201,7 +201,7 @@ def test_struct_layouts_of_header_and_ctypes_mirror_agree(tmp_path):
 
 @pytest.mark.parametrize("d,f,bits", [(2048, 512, 4), (4096, 2048, 2), (2048, 1024, 1), (128, 64, 4)])
 def test_expert_blob_layout_matches_checker(d, f, bits):
-    """mf_expert_blob_layout (the product's own helper) against the checker's restatement of the
+    """mf_expert_blob_layout (the product's own helper) against the oracle's restatement of the
     repacker's blob order; the Qwen expert is 1 769 472 bytes = 108 pages of 16 KiB exactly."""
     from mference_amd import operators as ops
     from oracle import mf_oracle as O

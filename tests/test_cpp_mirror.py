@@ -1,6 +1,6 @@
 """The C++ mirror of the reference's operator classes (include/mfmoe.hpp), driven by a C++
 program that reads like the reference's own operator tests: grouping KATs and thrown errors on
-the CPU, one layer (decode, two-phase, ragged prefill) against the CPU checker on the GPU."""
+the CPU, one layer (decode, two-phase, ragged prefill) against the CPU oracle on the GPU."""
 import os
 import subprocess
 

@@ -526,7 +526,7 @@ def test_routed_phases_over_slots_named_directly(gpu, oracle, bits, t):
     _sync()
     assert np.array_equal(ops.bf16_bits(acts1), ops.bf16_bits(acts0))
     assert np.array_equal(ops.bf16_bits(y1), ops.bf16_bits(y0))
-    # ... and, directly, the checker's layer (no shared expert, no residual: y = sum of the weighted routes)
+    # ... and, directly, the oracle's layer (no shared expert, no residual: y = sum of the weighted routes)
     assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y1)), oracle.bf16_to_float(ref_y), f"slots bits={bits}")
     # a slab that starts 2 bytes into its allocation (all the reference promises) takes the byte-wise kernels
     raw = torch.zeros(slab.numel() + 32, dtype=torch.uint8, device="cuda")
@@ -646,7 +646,7 @@ def test_qwen_shape_specialised_launch(gpu, oracle, t):
 def test_qwen_shape_with_other_flags(gpu, oracle, limit, maple):
     """the Qwen-shaped layer with a SwiGLU clamp or Maple rounding: the one-token instance has "no clamp, no
     Maple rounding" as literals, so these calls take the instance that reads the flags from the arguments --
-    one token row and three, against the checker and against the chain of launches"""
+    one token row and three, against the oracle and against the chain of launches"""
     import bench
     w = dict(bench.QWEN)
     stack = bench.build_stack(gpu, w, 1, torch.device("cuda", 0))
@@ -680,7 +680,7 @@ def test_other_shape_specialised_launches(gpu, oracle, workload, t):
     """the large 2-bit layer (D 4096, F 2048, E 256, K 6, 4-bit shared 2048) and the ternary layer
     (D 2048, F 1024, E 64, K 8, full-softmax router) at full size take their own shape-specialised fused
     kernels (one for a single token row, one for any other count); weights drawn and quantized on the GPU as bench.py does,
-    checked against the CPU checker and against the chain of separate launches"""
+    checked against the CPU oracle and against the chain of separate launches"""
     import bench
     w = dict(bench.WORKLOADS[workload])
     stack = bench.build_stack(gpu, w, 1, torch.device("cuda", 0))
@@ -711,7 +711,7 @@ def test_other_shape_specialised_launches(gpu, oracle, workload, t):
 
 def test_dense_mlp_full_size(gpu, oracle):
     """hidden 5120, intermediate 17408, 4 token rows (the dense-MLP configuration of bench.py):
-    weights drawn and quantized on the GPU, every row against the CPU checker; rows of the
+    weights drawn and quantized on the GPU, every row against the CPU oracle; rows of the
     4-token call equal the single-token calls bit for bit"""
     d, f, t = 5120, 17408, 4
     dev = torch.device("cuda", 0)
@@ -750,7 +750,7 @@ def test_dense_mlp_full_size(gpu, oracle):
 @pytest.mark.parametrize("bits,d,f,e,k,t", [(1, 256, 128, 32, 8, 1), (1, 512, 256, 64, 8, 3), (4, 256, 128, 32, 4, 2)])
 def test_decode_layer_with_maple_rounding(gpu, oracle, bits, d, f, e, k, t):
     """MapleMoE's rounding points (bf16-stepped activation clamped at 7, bf16 down outputs before
-    the routing weights; maple_moe.metal:153-164, 243-264) against the CPU checker, fused launch
+    the routing weights; maple_moe.metal:153-164, 243-264) against the CPU oracle, fused launch
     and launch chain bit for bit, and different from the same layer without the flag"""
     root = ROOT_SEED + 0x9A00 + bits + d
     layer = oracle.synth_layer(root, d, f, e, k, bits=bits, router_mode=1, sigma=0.1, maple_rounding=True)
@@ -783,7 +783,7 @@ def test_decode_layer_with_maple_rounding(gpu, oracle, bits, d, f, e, k, t):
 def test_residual_rmsnorm_matches_oracle(gpu, oracle, d, t, with_delta):
     """hidden += delta, then RMSNorm with a bf16 weight, one launch (rmsnorm.metal:30-92,
     utility.metal:83-92): the updated hidden bit for bit; the normalised rows within one bf16 step
-    of the checker (it sums the squares in double, the kernel in fp32 in lane order) and equal on
+    of the oracle (it sums the squares in double, the kernel in fp32 in lane order) and equal on
     all but a few elements"""
     r = oracle.Rng.key(ROOT_SEED + 0x9B00 + d, "rms")
     hb = oracle.bf16_bits(r.normal(0.0, 1.5, t * d).reshape(t, d))
@@ -805,7 +805,7 @@ def test_residual_rmsnorm_matches_oracle(gpu, oracle, d, t, with_delta):
 @pytest.mark.parametrize("count", [1, 63, 512, 4099])
 def test_silu_mul_matches_oracle(gpu, oracle, count):
     """silu_mul_fp16 (utility.metal:21-33): out = narrow(silu(gate) * up), one rounding, bit for bit
-    against the checker's silu on every element (incl. large |gate|, zeros and negative zero)."""
+    against the oracle's silu on every element (incl. large |gate|, zeros and negative zero)."""
     rng = oracle.Rng.key(0x51, f"silu-mul-{count}")
     g = rng.normal(0.0, 3.0, count).astype(np.float32)
     u = rng.normal(0.0, 2.0, count).astype(np.float32)
@@ -886,9 +886,9 @@ def test_nibble_widened_ternary_gemv_exact_bits(gpu, oracle):
 def test_single_expert_ffn_at_full_size(gpu, oracle):
     """One SwiGLU expert FFN at batch 1, hidden 2048 / intermediate 512, weights N(0, 0.02) quantized
     4-bit g64, x ~ N(0, 1) (the CPU-runnable configuration): as the shared-expert operator
-    (gate and up narrowed before the activation, dequant_int4.metal:240-245) against the checker's
+    (gate and up narrowed before the activation, dequant_int4.metal:240-245) against the oracle's
     shared expert, and as a routed expert through the two phases with K = 1, weight 1, no residual
-    (gate and up kept fp32, moe.metal:526-528, 1262-1270) against the checker's phase functions."""
+    (gate and up kept fp32, moe.metal:526-528, 1262-1270) against the oracle's phase functions."""
     d, f = 2048, 512
     rng = oracle.Rng.key(ROOT_SEED + 0x000, "single-expert")
     gq = oracle.quantize(rng.normal(0.0, 0.02, f * d).reshape(f, d), 4)
@@ -932,7 +932,7 @@ def test_fused_topk_on_non_finite_logits(gpu, oracle, e):
     """top-k softmax router (mode 0) on logits that are NaN, +inf, -inf, mostly -inf (fewer finite ones than
     routes) or all equal: NaN counts as -inf and is never picked, ranks nobody wins keep index 0 (the serial
     selector of moe.metal:190-240).  The fused launch -- threshold prefilter, its fallback to a rank count over
-    all experts when more than 64 candidates tie, and the rank count itself -- gives the indices of the checker
+    all experts when more than 64 candidates tie, and the rank count itself -- gives the indices of the oracle
     and the indices AND weight bits of the chain of launches, for the four rows in one call and one at a time."""
     d, f, k, t = 2 * e, 64, 8, 4
     root = ROOT_SEED + 0x9A0 + e
@@ -987,7 +987,7 @@ def test_fused_topk_on_non_finite_logits(gpu, oracle, e):
 @pytest.mark.parametrize("m,n,t", [(1, 2048, 1), (1, 2048, 8), (64, 64, 3), (65, 192, 2), (130, 2816, 1), (8, 5120, 8)])
 def test_int8_gemv(gpu, oracle, m, n, t):
     """8-bit affine rows (DequantInt8GEMV.encode, Kernels/Quant/DequantInt8GEMV.swift:53; dequant_int8_gemv_simd,
-    dequant_int8.metal:66-107): the value of every (token, row) has the bits of the checker's lane-order row dot
+    dequant_int8.metal:66-107): the value of every (token, row) has the bits of the oracle's lane-order row dot
     (x unscaled), agrees with the reference's CPU path (bulk dequantize, scalar dot) to fp32 summation order, and
     does not depend on how many token rows ride along; weights two bytes into their allocation take the
     byte-wise loads."""
@@ -1027,7 +1027,7 @@ def test_int8_gemv(gpu, oracle, m, n, t):
 def test_layer_with_int8_scalar_gate(gpu, oracle, d, f, e, k, fs, t):
     """The scalar shared gate as the reference's model files store it -- an 8-bit affine row
     (RealForwardRunner.swift:2925-2941): the fused launch and the chain of launches give the same bits, the
-    layer agrees with the checker, and so does the ragged prefill call on the same weights."""
+    layer agrees with the oracle, and so does the ragged prefill call on the same weights."""
     root = ROOT_SEED + 0x8A7E + d + t
     layer = oracle.synth_layer(root, d, f, e, k, bits=4, fs=fs)
     gate_row = oracle.Rng.key(root, "w_sg.q8").normal(0.0, 0.05, d).reshape(1, d)
@@ -1070,7 +1070,7 @@ def test_layer_with_int8_scalar_gate(gpu, oracle, d, f, e, k, fs, t):
 def test_listed_shape_instance_at_full_size(gpu, oracle, t):
     """A layer shape that is no benchmark shape -- Gemma 4's (hidden 2816, 128 experts of 704, top-8;
     ArchConfig.gemma4_26B_A4B, ModelTypes.swift:376-398) -- listed in fused_shapes.json: the build holds
-    instances of the fused launch with its dimensions as literals.  At full size against the checker, and the
+    instances of the fused launch with its dimensions as literals.  At full size against the oracle, and the
     same bits as the instance that reads every dimension from its arguments and as the chain of launches;
     with the routing given by the caller too (Gemma routes through its 8-bit router)."""
     d, f, e, k = 2816, 704, 128, 8
@@ -1108,7 +1108,7 @@ def test_listed_shape_instance_at_full_size(gpu, oracle, t):
 @pytest.mark.parametrize("d,f,t,silu", [(256, 128, 1, False), (2816, 2112, 3, False), (512, 1024, 9, True)])
 def test_int8_shared_expert(gpu, oracle, d, f, t, silu):
     """SharedExpertInt8.encode (SharedExpertInt8.swift:78-181): 8-bit gate / up rows in one launch with the tanh
-    GELU (or SiLU), 8-bit down rows -- the checker's bits (the lane order and the activation are defined)."""
+    GELU (or SiLU), 8-bit down rows -- the oracle's bits (the lane order and the activation are defined)."""
     rng = oracle.Rng.key(ROOT_SEED + 0x1E8, f"int8-mlp-{d}-{f}")
     gq = oracle.quantize(rng.normal(0.0, 0.03, f * d).reshape(f, d), 8)
     uq = oracle.quantize(rng.normal(0.0, 0.03, f * d).reshape(f, d), 8)
@@ -1134,7 +1134,7 @@ def test_int8_shared_expert(gpu, oracle, d, f, t, silu):
                                         (128, 2112, 530, False), (192, 2112, 1601, True), (3136, 128, 70, False)])
 def test_int8_shared_expert_many_rows(gpu, oracle, d, f, t, silu):
     """from 16 rows on the 8-bit MLP is a matrix-core matmul (odd numbers of K groups, half slices of rows, ragged
-    token tiles): within the layer tolerance of the checker; below, the checker's bits"""
+    token tiles): within the layer tolerance of the oracle; below, the oracle's bits"""
     rng = oracle.Rng.key(ROOT_SEED + 0x1E9, f"int8-mlp-{d}-{f}")
     qs = [oracle.quantize(rng.normal(0.0, 0.03, r * c).reshape(r, c), 8) for r, c in ((f, d), (f, d), (d, f))]
     xb = oracle.bf16_bits(rng.normal(0.0, 1.0, t * d).reshape(t, d))
@@ -1220,7 +1220,7 @@ def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
 def test_decode_layer_with_the_norm_in_front(gpu, oracle, bits, d, f, e, k, fs, t, with_delta):
     """mf_moe_decode_layer_normed: hidden += delta, x = RMSNorm(hidden) * w, y = layer(x), hidden += y in one
     call -- the bits of mf_residual_rmsnorm followed by mf_moe_decode_layer (also with the fused launch off),
-    and the checker's composition of the two."""
+    and the oracle's composition of the two."""
     root = ROOT_SEED + 0x4042 + d + t
     layer = oracle.synth_layer(root, d, f, e, k, bits=bits, fs=fs, router_mode=1 if bits == 1 else 0,
                                maple_rounding=bits == 1)
@@ -1250,7 +1250,7 @@ def test_decode_layer_with_the_norm_in_front(gpu, oracle, bits, d, f, e, k, fs, 
         assert torch.equal(y, y_ref), f"y, fused={fused}"
         assert torch.equal(h, h_ref), f"hidden, fused={fused}"
     moe.set_fused(1)
-    # the checker: norm, layer, residual add
+    # the oracle: norm, layer, residual add
     h1, x_ref = oracle.residual_rmsnorm(hb, wb, 1e-6, delta_bits=db)
     ref_y, ref_idx, ref_w = oracle.moe_layer(layer, x_ref)
     assert np.array_equal(ops.bf16_bits(xn), x_ref)

@@ -84,7 +84,7 @@ def test_router_logits_sweep(gpu, oracle, seed):
     """drawn (experts, width, tokens) across the batched router's kernels: the register-tiled one (up to 256
     tokens, widths that are no multiple of 512), the matrix-core walk as a loop (1536, 2560, 3072) and unrolled
     (1024, 2048, 4096), expert counts that leave rows over after the blocks of 32 (100, 258) -- logits bit for
-    bit against the one-row order of the checker on sampled tokens, and the selection on top of them"""
+    bit against the one-row order of the oracle on sampled tokens, and the selection on top of them"""
     rng0 = np.random.default_rng(0x60A7 + seed)
     e = int(rng0.choice([32, 64, 100, 128, 256, 258, 512]))
     d = int(rng0.choice([512, 1024, 1536, 2048, 2560, 3072, 4096]))
@@ -320,7 +320,7 @@ def test_row_counts_beyond_the_limit_are_refused(gpu):
 
 def test_sqrtsoftplus_routing_feeds_the_two_phase_layer(gpu, oracle):
     """a 2-bit layer routed by the DeepSeek-V4 selector: router -> phase 1 -> phase 2 through the ABI
-    against the checker's composition of the same parts"""
+    against the oracle's composition of the same parts"""
     d, f, e, k, t = 512, 256, 32, 6, 2
     root = ROOT_SEED + 0x4D5
     layer = oracle.synth_layer(root, d, f, e, k, bits=2, fs=0)

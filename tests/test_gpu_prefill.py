@@ -168,7 +168,7 @@ def _skewed_qwen_layer(oracle):
 
 @pytest.mark.parametrize("t", [128, 512, 2048])
 def test_skewed_qwen_prefill_against_the_checker(gpu, oracle, t):
-    """The headline prefill configuration at its three token counts, directly against the per-token checker:
+    """The headline prefill configuration at its three token counts, directly against the per-token oracle:
     routing indices and weights bit for bit on every row, the layer output within tolerance on 64 sampled rows
     (the busiest expert takes most tokens here, so full 64-route tiles, ragged tails and experts without
     tokens all occur in one call)."""
@@ -202,7 +202,7 @@ def test_skewed_qwen_prefill_against_the_checker(gpu, oracle, t):
 ])
 def test_prefill_long_batches_against_the_per_token_oracle(gpu, oracle, bits, d, f, e, k, fs, t, mode):
     """More than a thousand tokens on small layers (long runs per expert, many full tiles, an odd tile at
-    the end of every run), checked directly against the per-token checker: routing bit-exact, sampled rows
+    the end of every run), checked directly against the per-token oracle: routing bit-exact, sampled rows
     within the layer tolerance; and the rows do not depend on their neighbours (the first 300 tokens alone
     give the same bits).  Beyond 8192 routes the layer call selects and groups its routes in two launches
     of its own (chunks of up to 64 tokens, an expert's routes of a chunk as a 64-bit word); the 300-token
@@ -404,7 +404,7 @@ def test_prefill_rows_wider_than_4096(gpu, oracle, d, e, t):
 def test_prefill_other_formats_full_size(gpu, oracle, workload, t):
     """the large 2-bit layer (D 4096, F 2048, E 256, K 6, 4-bit shared 2048) and the ternary layer
     (D 2048, F 1024, E 64, K 8, full-softmax router) at full size through the matrix-core path:
-    routing against the CPU checker for every token, sampled rows against the CPU checker and
+    routing against the CPU oracle for every token, sampled rows against the CPU oracle and
     against the decode launch of the same token; a second call gives the same bits"""
     import bench
     w = dict(bench.WORKLOADS[workload])

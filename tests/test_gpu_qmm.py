@@ -1,5 +1,5 @@
 """The dense projection of many rows (mf_qmm = MPPPrefillInt4QMM.encode) and the block form of the
-shared expert / dense MLP (mf_shared_expert beyond 8 rows), against the CPU checker and against the
+shared expert / dense MLP (mf_shared_expert beyond 8 rows), against the CPU oracle and against the
 closed-form inputs and tolerances of the reference's own test (MPPPrefillInt4QMMTests.swift)."""
 import numpy as np
 import pytest
@@ -84,7 +84,7 @@ def test_qmm_matches_reference_test_inputs(gpu, oracle, m, n, k, adversarial, of
 
 @pytest.mark.parametrize("bits,m,n,k", [(4, 70, 256, 512), (2, 64, 128, 1024), (1, 40, 256, 256), (4, 9, 64, 192)])
 def test_qmm_matches_gemv_oracle(gpu, oracle, bits, m, n, k):
-    """random weights, every format; fp32 and bf16 outputs against the checker's GEMV row by row"""
+    """random weights, every format; fp32 and bf16 outputs against the oracle's GEMV row by row"""
     rng = oracle.Rng.key(0x0A11, f"qmm-{bits}-{m}-{n}-{k}")
     if bits == 1:
         codes = (rng.uniform_fill(0.0, 4.0, n * k).astype(np.int64) // 1).clip(0, 3)

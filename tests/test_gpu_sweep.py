@@ -1,6 +1,6 @@
 """Seeded sweeps over shapes nobody picked by hand: the decode call (fused launch and chain of
 launches) and the prefill call against the per-token CPU oracle, and the stand-alone dense projection and
-shared-expert MLP against the checker's rows.  Shapes are drawn from what
+shared-expert MLP against the oracle's rows.  Shapes are drawn from what
 mf_moe_create accepts (widths in multiples of the group size, up to 8 routes per token), so the sweep
 crosses the boundaries between the specialised kernels and their fall-backs: widths that are and are not
 multiples of 128 or 512, expert counts that are no multiple of 32, tiles that are empty, partial and full."""
@@ -82,9 +82,9 @@ def test_prefill_sweep(gpu, oracle, seed):
 @pytest.mark.parametrize("seed", range(8))
 def test_prefill_long_sweep(gpu, oracle, seed):
     """the same draw with 2200 to 4400 tokens (beyond 8192 routes the layer call selects and groups its
-    routes chunk by chunk): routing bit-exact on every row, 48 sampled rows against the per-token checker"""
+    routes chunk by chunk): routing bit-exact on every row, 48 sampled rows against the per-token oracle"""
     bits, d, f, e, k, fs, _, mode, limit = _draw(0xF1A0 + seed, prefill=True)
-    d, f = min(d, 512), min(f, 256)   # the checker walks every sampled row's experts in numpy
+    d, f = min(d, 512), min(f, 256)   # the oracle walks every sampled row's experts in numpy
     t = int(np.random.default_rng(0xF1A1 + seed).integers(2200, 4400))
     root = ROOT_SEED + 0xBC00 + seed
     layer = oracle.synth_layer(root, d, f, e, k, bits=bits, fs=min(fs, f), router_mode=mode, swiglu_limit=limit)
@@ -130,7 +130,7 @@ def test_qmm_sweep(gpu, oracle, seed):
 @pytest.mark.parametrize("seed", range(12))
 def test_shared_expert_sweep(gpu, oracle, seed):
     """the shared expert / dense MLP over drawn (d, f, t): the GEMV kernels up to 8 rows, the matrix cores
-    beyond, against the checker row by row"""
+    beyond, against the oracle row by row"""
     from helpers import to_device_q
     rng0 = np.random.default_rng(0x5E50 + seed)
     d = int(rng0.choice([128, 256, 512, 1024, 2048]))

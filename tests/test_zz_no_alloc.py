@@ -44,7 +44,7 @@ def _run_both(gpu, oracle, label, d, f, t, bits=4):
     torch.cuda.synchronize()
     got, want = ops.bf16_bits(y), ops.bf16_bits(y_ref)
     assert np.array_equal(got, want), f"{label}: {(got != want).sum()} of {got.size} outputs differ"
-    # and the existing entry point agrees with the CPU checker on this case
+    # and the existing entry point agrees with the CPU oracle on this case
     ref = np.stack([oracle.shared_expert(gq, uq, dq, x[i]) for i in range(t)])
     err = np.abs(oracle.bf16_to_float(want).astype(np.float64) - oracle.bf16_to_float(ref).astype(np.float64)).max()
     assert err <= 2e-2, (label, err)
