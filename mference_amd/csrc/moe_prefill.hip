@@ -2381,6 +2381,8 @@ static uint32_t dense_tile_items(uint32_t n) {
   return (n + slice_rows - 1) / slice_rows;
 }
 static uint32_t dense_fewest_windows(uint32_t k) { return std::max(1u, (k / kGroup + kDenseWindow - 1) / kDenseWindow); }
+// (none of the shapes timed wanted more than 25; the bound keeps the search short for any k)
+static uint32_t dense_most_windows(uint32_t k) { return std::max(dense_fewest_windows(k), std::min(k / kGroup / 8, 64u)); }
 // (as the differences of dense_window_start, which steps by ng / n_win, without a division a window)
 static uint32_t dense_longest_window(uint32_t ng, uint32_t n_win) {
   const uint32_t whole = ng / n_win, part = ng % n_win;
@@ -2397,7 +2399,7 @@ static uint32_t dense_longest_window(uint32_t ng, uint32_t n_win) {
 // longest(w): groups of the longest of w windows
 template <typename Longest>
 static uint32_t dense_windows_of_tiles(uint32_t tiles, uint32_t n, uint32_t k, Longest longest) {
-  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, k / kGroup / 8), num_cu = device_cu_count();
+  const uint32_t lo = dense_fewest_windows(k), hi = dense_most_windows(k), num_cu = device_cu_count();
   const uint64_t items = static_cast<uint64_t>(tiles) * dense_tile_items(n);
   if (items * lo >= kWholeRounds * 2ull * num_cu) return lo;
   uint32_t best = lo;
@@ -2423,7 +2425,7 @@ static size_t dense_parts_bytes(uint32_t m, uint32_t n, uint32_t n_win) {
 // ... and the most any call of up to m tokens needs: fewer tiles can take more windows, so the bytes of a single call do
 // not grow with its rows (5120 x 17408: 27.5 MB of results for 192 rows, 24.6 for 200).  Only tile counts below kWholeRounds differ.
 static size_t dense_parts_bytes_up_to(uint32_t m, uint32_t n, uint32_t k) {
-  const uint32_t lo = dense_fewest_windows(k), hi = std::max(lo, k / kGroup / 8);
+  const uint32_t lo = dense_fewest_windows(k), hi = dense_most_windows(k);
   std::vector<uint32_t> longest(hi + 1);
   for (uint32_t w = lo; w <= hi; ++w) longest[w] = dense_longest_window(k / kGroup, w);
   const auto of_tiles = [&](uint32_t tiles) { return dense_windows_of_tiles(tiles, n, k, [&](uint32_t w) { return longest[w]; }); };

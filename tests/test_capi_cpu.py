@@ -243,7 +243,7 @@ def test_repacked_ternary_layout_is_the_file_layout(d, f):
         assert all(getattr(a[0], n) == getattr(b[0], n) for n, _ in a[0]._fields_)
 
 
-@pytest.mark.parametrize("n,k", [(5120, 17408), (2048, 8192), (1152, 3200), (128, 128), (384, 12800)])
+@pytest.mark.parametrize("n,k", [(5120, 17408), (2048, 8192), (1152, 3200), (128, 128), (384, 12800), (256, 1 << 20)])
 def test_a_workspace_for_many_rows_serves_every_smaller_block(n, k):
     """sizes never fall as rows are added, and a buffer sized for the most rows keeps every smaller block on the matrix
     cores (the K windows of a block depend on its rows, so the bytes of a single call do not grow with them)"""
