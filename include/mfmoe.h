@@ -576,8 +576,9 @@ mf_status mf_group_pairs_host(const mf_pair* pairs, size_t n_pairs, int query_co
  * tensor 16-byte aligned; every other configuration (a width of 64, another shared-expert
  * format) runs the same rows through the decode launch, MF_MAX_TOKENS at a time, and needs
  * no workspace.  Widths that are no multiples of 128 run that way too for up to MF_MAX_TOKENS rows (twice as many
- * where few routes share an expert), and when the call brings no workspace or an unaligned operand (with widths of whole 128s that is an error).  Covers MoEDeepseekV4's pair-major 2-bit prefill
- * (Metal/MoE/moe.metal:1293-1409) with the same call.
+ * where few routes share an expert), and when the call brings no workspace or an unaligned operand (with widths of
+ * whole 128s that is an error); what mf_moe_decode_layer asks of the caller holds for these calls.  Covers
+ * MoEDeepseekV4's pair-major 2-bit prefill (Metal/MoE/moe.metal:1293-1409) with the same call.
  * workspace: device scratch of at least mf_moe_prefill_workspace_bytes(h, t) (0 when the
  * configuration takes the decode launch; workspace may then be null). */
 size_t mf_moe_prefill_workspace_bytes(const mf_moe* h, uint32_t t);

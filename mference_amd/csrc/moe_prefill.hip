@@ -2859,7 +2859,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // launch / two, same bits: 4096 x 256, shared 512, top 6: 40 tokens 98 / 93, 2048 tokens 369 / 296; 2048 x 128, shared
   // 512, top 8: 150 tokens 72 / 74, 300 tokens 87 / 85, 2048 tokens 176 / 143; 2048 x 512, shared 1024, top 8: 300 tokens
   // 102 / 111, 777 tokens 155 / 155, 2048 tokens 274 / 262; routed 1024 or 2048 beside a resident shared expert: one
-  // launch always, 375 / 385).
+  // launch always, 375 / 385; 4-bit experts alike, 4096 x 256, 2048 tokens 362 / 297).
   const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
   const bool apart = shared_rides && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
   {
