@@ -516,6 +516,9 @@ __device__ __forceinline__ f32x4_t mfma_quad(uint2 a, uint2 b, f32x4_t c) {
 }
 
 constexpr uint32_t kQuadMaxWaves = 8;
+// LDS of one wave: table pieces of two stages, partial sums of two buffers
+constexpr uint32_t kQuadTabBytes = 2 * 64 * 8 * sizeof(uint16_t);
+__host__ __device__ constexpr uint32_t quad_wave_bytes(int nproj) { return kQuadTabBytes + 2u * nproj * 4 * 4 * 4 * sizeof(float); }
 
 // BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group -- and its codes enter as 4 + q.
 // ANY: K is any multiple of 64; otherwise of 512, so that the table pieces are whole and aligned.
@@ -523,12 +526,17 @@ template <int BITS, int NPROJ, int ITS, bool ANY>
 __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const RowsQuadArgs a) {
   using chunk_t = std::conditional_t<BITS == kBits4, uint4, uint2>;
   constexpr uint32_t kScaleStep = BITS == kBits4 ? 0x0200u : 0x0100u;  // bf16 exponent of the offset: 16 or 4
-  // partial sums [buffer][projection][wave][16-lane row][weight row][token]
-  __shared__ __attribute__((aligned(16))) float s_part[2][NPROJ][kQuadMaxWaves][4][4][4];
-  // scale / bias pieces [wave][ring slot][(table, row, piece)][8 groups]
-  __shared__ __attribute__((aligned(16))) uint16_t s_tab[kQuadMaxWaves][2][64 * 8];
+  // LDS, sized for the waves there are (a workgroup of one wave that held room for eight left six to a CU: gate / up of
+  // 2-bit 6656 x 2048, one row, 10.8 -> 8.5 us; 4-bit 17408 x 2112 19.1 -> 14.7).  Per wave, so that no address depends on
+  // their number: scale / bias pieces [ring slot][(table, row, piece)][8 groups], partial sums
+  // [buffer][projection][16-lane row][weight row][token]
+  constexpr uint32_t kWaveFloats = quad_wave_bytes(NPROJ) / sizeof(float), kTabFloats = kQuadTabBytes / sizeof(float);
+  extern __shared__ __attribute__((aligned(16))) float s_quad[];
   const uint32_t lane = threadIdx.x & 63, wsub = threadIdx.x >> 6, wpr = blockDim.x >> 6;
   const uint32_t b = lane >> 2, c = lane & 3;
+  auto part_of = [&](uint32_t w, uint32_t pb, int p, uint32_t r, uint32_t row) __attribute__((always_inline)) {
+    return s_quad + w * kWaveFloats + kTabFloats + (((pb * NPROJ + p) * 4 + r) * 4 + row) * 4;
+  };
   const uint32_t n_chunks = a.N / 32, ng = a.N / kGroup, n_sets = a.M / 4;
   const size_t row_bytes = static_cast<size_t>(a.N) * BITS / 8;
 
@@ -556,7 +564,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   // a piece past the row is never used: read piece 0.  ANY: the row's last piece ends with the row and is moved down
   const uint32_t tb_group = tb_g >= ng ? 0u : ANY ? min(tb_g, ng - 8u) : tb_g;
   const uint32_t tb_drop = ANY && tb_g < ng ? tb_g - tb_group : 0u;
-  uint16_t* my_tab = &s_tab[wsub][0][0];
+  uint16_t* my_tab = reinterpret_cast<uint16_t*>(s_quad + wsub * kWaveFloats);
   auto fetch = [&](int buf, int j, uint32_t set, int p) __attribute__((always_inline)) {
     const size_t row = static_cast<size_t>(set) * 4 + c;
     cw[buf][j] = *reinterpret_cast<const chunk_t*>(a.W[p] + row * row_bytes + static_cast<size_t>(chc[j]) * sizeof(chunk_t));
@@ -616,7 +624,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
       v[t] = v[t] + dpp_f<0x128>(v[t]);      // + lane - 8
     }
     if ((lane & 12u) == 0)
-      *reinterpret_cast<float4*>(&s_part[pb][p][wsub][lane >> 4][c][0]) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(part_of(wsub, pb, p, lane >> 4, c)) = make_float4(v[0], v[1], v[2], v[3]);
   };
   // threads 0..15: (weight row, token) totals in wave then row order
   auto combine = [&](uint32_t set, uint32_t pb) __attribute__((always_inline)) {
@@ -628,7 +636,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
       v[p] = 0.0f;
       for (uint32_t w = 0; w < wpr; ++w)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[p] = v[p] + s_part[pb][p][w][r][cc][t];
+        for (int r = 0; r < 4; ++r) v[p] = v[p] + part_of(w, pb, p, r, cc)[t];
     }
     if (t >= a.T) return;
     const size_t at = static_cast<size_t>(t) * a.M + set * 4 + cc;
@@ -915,13 +923,13 @@ bool rows_mfma_try(hipStream_t s, const RowsMfmaArgs& a, uint32_t num_cu, hipErr
   return true;
 }
 
-// The quad kernel takes 4-bit and 2-bit matrices with at least 1024 rows (a multiple of 4), a K of at least 2048 and up to
+// The quad kernel takes 4-bit and 2-bit matrices with at least 1024 rows (a multiple of 4), a K of at least 1024 and up to
 // 4 token rows.  The 32-element chunks of a row split over (waves, ITS slots of 16 chunks).  EVEN: K is a multiple of 512
 // and splits with little waste.  ANY: any other K, the split that costs the fewest slots, a stage of a wave counted as
 // one more.
 enum class QuadFit { kNone, kEven, kAny };
 QuadFit rows_quad_split(uint32_t m, uint32_t n, uint32_t& its, uint32_t& wpr) {
-  if (n % kGroup || n < 2048 || m < 1024 || m % 4) return QuadFit::kNone;
+  if (n % kGroup || n < 1024 || m < 1024 || m % 4) return QuadFit::kNone;
   const uint32_t chunks = n / 32;
   uint32_t waste = ~0u;
   its = wpr = 0;
@@ -932,7 +940,7 @@ QuadFit rows_quad_split(uint32_t m, uint32_t n, uint32_t& its, uint32_t& wpr) {
   }
   if (n % (8 * kGroup) == 0 && its && waste * 10 <= chunks) return QuadFit::kEven;
   uint32_t cost = ~0u;
-  for (uint32_t i = 6; i >= 4; --i) {
+  for (uint32_t i = 6; i >= 2; --i) {
     const uint32_t w = (chunks + 16 * i - 1) / (16 * i);
     if (w <= kQuadMaxWaves && w * (i + 1) < cost) { cost = w * (i + 1); its = i; wpr = w; }
   }
@@ -943,14 +951,17 @@ template <int BITS, int NPROJ>
 hipError_t launch_rows_quad(hipStream_t s, const RowsQuadArgs& a, QuadFit fit, uint32_t its, uint32_t wpr, uint32_t num_cu) {
   const uint32_t n_sets = a.M / 4;
   const dim3 grid(std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / wpr))), block(wpr * 64);
+  const uint32_t lds = wpr * quad_wave_bytes(NPROJ);
   if (fit == QuadFit::kEven) {
-    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, false><<<grid, block, 0, s>>>(a);
-    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, false><<<grid, block, 0, s>>>(a);
-    else rows_quad_kernel<BITS, NPROJ, 6, false><<<grid, block, 0, s>>>(a);
+    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, false><<<grid, block, lds, s>>>(a);
+    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, false><<<grid, block, lds, s>>>(a);
+    else rows_quad_kernel<BITS, NPROJ, 6, false><<<grid, block, lds, s>>>(a);
   } else {
-    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, 0, s>>>(a);
-    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, true><<<grid, block, 0, s>>>(a);
-    else rows_quad_kernel<BITS, NPROJ, 6, true><<<grid, block, 0, s>>>(a);
+    if (its == 2) rows_quad_kernel<BITS, NPROJ, 2, true><<<grid, block, lds, s>>>(a);
+    else if (its == 3) rows_quad_kernel<BITS, NPROJ, 3, true><<<grid, block, lds, s>>>(a);
+    else if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, lds, s>>>(a);
+    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, true><<<grid, block, lds, s>>>(a);
+    else rows_quad_kernel<BITS, NPROJ, 6, true><<<grid, block, lds, s>>>(a);
   }
   return hipGetLastError();
 }
@@ -970,12 +981,16 @@ bool rows_lane_ordered(uint32_t m, uint32_t n, uint32_t num_cu) {
 
 // Whether t token rows of the matrix go to the quad kernel.  A draft's verification and the plain step it stands for
 // have to agree: where the other kernels give a row the same bits for every number of token rows, the quad kernel takes
-// all numbers or none, by what one row costs (us, other kernels / this one, one row; four rows):
-//   4-bit of K below 2048, none (17408 x 1536: 7.3 / 8.3; 18.6 / 9.6), 4-bit above, from 36 M weights on
-//   (17408 x 2112: 11.6 / 10.6; 31.8 / 12.7; gate / up 6656 x 3136: 12.4 / 11.5, 6656 x 2112: 11.5 / 12.5);
-//   2-bit of K up to 4096, only long and many rows (17408 x 3136: 15.7 / 11.0; 52.9 / 12.4; gate / up 6656 x 3136:
-//   9.5 / 10.7; 28.9 / 12.0; 4096 is one whole step of rows_stream_kernel: 17408 rows 10.1 / 12.4), 2-bit above, from
-//   8 M weights on (6656 x 6592: 14.7 / 10.6; 34.0 / 12.1; 1024 x 6592: 4.9 / 5.1).
+// all numbers or none.  The lines are where what four rows gain is more than what one row loses, the one row's share
+// counted twice (us, other kernels / this one; one row; four rows):
+//   4-bit of K below 2048, gate / up from 36 rows a CU on (9216 x 1536: 7.6 / 9.0; 19.9 / 10.1; 5120 x 1536: 5.4 / 7.2;
+//   13.7 / 8.2; one projection, 9216 x 1536: 4.9 / 6.8; 12.1 / 8.4);
+//   4-bit above, from 8 M weights a projection on (4096 x 3136: 6.5 / 7.0; 13.3 / 8.5, gate / up 9.4 / 8.8; 20.3 / 10.3;
+//   9216 x 3008: 8.0 / 9.7; 21.1 / 12.5; 2048 x 3136: 4.5 / 5.7; 10.7 / 6.3, and eight 10.5 / 12.1);
+//   2-bit of K up to 4096, from 16 rows a CU on (5120 x 1024: 3.7 / 4.4; 9.7 / 5.0; 4096 x 2560: 5.0 / 6.4; 13.5 / 7.9,
+//   gate / up 6.2 / 7.4; 19.9 / 8.7; 17408 x 4096: 10.1 / 12.2; 21.2 / 14.5, and eight 124 / 27; 2048 x 3136: 3.7 / 5.4;
+//   8.7 / 6.1);
+//   2-bit above, from 8 M weights on (6656 x 6592: 14.7 / 10.6; 34.0 / 12.1; 1024 x 6592: 4.9 / 5.1).
 // Elsewhere the number of token rows decides (us per MLP, other kernels / this one): one row, where a step of
 // rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3; 3840 x 7680, a
 // sixteenth empty: 22.2 / 22.9); two to four (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25; 2048 x 6656:
@@ -987,9 +1002,10 @@ bool rows_quad_takes(QuadFit fit, uint32_t m, uint32_t n, uint32_t t, uint32_t n
   constexpr uint32_t step = two ? 4096 : 2048;  // K values of one step of a wave in rows_stream_kernel
   const uint64_t weights = static_cast<uint64_t>(m) * n * NPROJ;
   if (fit == QuadFit::kNone) return false;
-  if (two && n <= step) return n >= 2560 && n < step && weights >= 24000000ull * NPROJ * NPROJ;
+  if (two && n <= step) return m >= 16 * num_cu;
+  if (!two && n < step) return NPROJ == 2 && m >= 36 * num_cu;
   if (fit == QuadFit::kEven) return true;
-  if (rows_lane_ordered<BITS, NPROJ>(m, n, num_cu)) return n >= step && weights >= (two ? 8ull : 36ull) * 1000000;
+  if (rows_lane_ordered<BITS, NPROJ>(m, n, num_cu)) return weights >= (two ? 8ull : 8ull * NPROJ) * 1000000;
   const uint32_t steps = (n + step - 1) / step;
   const bool wide = weights >= (two ? 8ull : 24ull) * 1000000;
   return t == 1 ? wide && n * 5ull < steps * static_cast<uint64_t>(step) * 4 : t <= 4 ? weights >= 4000000 : wide;

@@ -201,10 +201,10 @@ def test_gemv_quad_rows_kernel_at_any_k(gpu, oracle, bits, m, n, t):
 
 
 @pytest.mark.parametrize("bits,m,n", [
-    (4, 3136, 1984), (4, 12288, 1536),      # 4-bit, K below a wave's step: the vector kernels
-    (4, 7680, 3136), (4, 11520, 3136),      # ... above, below and above the quad kernel's 36 M weights; one group in the last piece
-    (4, 16384, 2240), (4, 1024, 2816), (4, 9216, 4672),
-    (2, 4096, 2048), (2, 9408, 2560), (2, 9344, 2560), (2, 6656, 4032), (2, 2816, 4096),  # 2-bit, one step or less
+    (4, 3136, 1984), (4, 9152, 1536), (4, 9216, 1536), (4, 12288, 1088),  # 4-bit, K below a wave's step: the vector kernels; pairs of many rows
+    (4, 2496, 3136), (4, 2560, 3136),       # ... above, below and above 8 M weights; one group in the last piece
+    (4, 7680, 3136), (4, 18432, 2240), (4, 1024, 2816), (4, 9216, 4672),
+    (2, 4096, 1024), (2, 5120, 1088), (2, 4160, 1536), (2, 4032, 2048), (2, 4096, 2048), (2, 4096, 2112), (2, 9152, 2560), (2, 6656, 4032), (2, 2816, 4096), (2, 4160, 4096),  # 2-bit, one step or less
     (2, 1216, 6592), (2, 1152, 6592), (2, 2816, 5120), (2, 1024, 8128),                   # ... more
 ])
 def test_a_row_has_the_same_bits_in_every_call(gpu, bits, m, n):
@@ -1189,7 +1189,7 @@ def test_int8_matmul_passes_infinities_on(gpu, d, f, t):
     assert torch.equal(torch.sign(got[1].float()), torch.sign(want[1].float()))
 
 
-@pytest.mark.parametrize("bits,m,n,t", [(4, 1024, 5120, 3), (4, 11520, 3136, 8), (2, 9408, 2560, 4), (2, 1216, 6592, 7)])
+@pytest.mark.parametrize("bits,m,n,t", [(4, 1024, 5120, 3), (4, 12800, 3136, 8), (2, 9408, 2560, 4), (2, 1216, 6592, 7)])
 def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
     """an infinity or a NaN makes its own token's results NaN (the code offset is taken out as inf - inf, as in every row
     kernel of these formats) and leaves the other tokens' bits alone"""
