@@ -363,9 +363,51 @@ __device__ __forceinline__ void expand_q2(uint32_t w, uint4& a, uint4& b) {
                  and_or(v >> 7, 0x00600060u, kMagic4), and_or(v >> 9, 0x00600060u, kMagic4));
 }
 
+// ---- codes as bf16 subnormals: the operands of the quantized matmuls
+//
+// A bf16 number with a zero exponent field is its mantissa times 2^-133, one with exponent 1 is (128 + mantissa) times
+// 2^-133: the low byte u of a 16-bit word whose upper byte is zero IS the number u * 2^-133, and the matrix cores (and
+// v_dot2_f32_bf16) read it as that.  A code needs no magic or-ed in: its field is masked in place, at the top of the byte -- a 4-bit code
+// in bits 4..7 is q * 2^-129, a 2-bit code in bits 6..7 is q * 2^-127 -- and nothing has to be taken off the sums afterwards.
+// Measured against the numbers 8 + q/2 (4 + q) that a mask-and-or gives: an and takes 1.5 ns of a SIMD, an and-or 3.0; one K
+// group of 64 with its operands in registers, two row blocks, two waves a SIMD: 357 -> 323 ns for two token
+// blocks, 243 -> 198 for one, 222 -> 180 for one of at most 8 tokens; and a group's sum is 4 to 5 times nearer to its 64-bit value
+// (relative rms 3.3e-8 -> 0.7e-8 on Gaussian rows, 7.9e-8 -> 1.8e-8 on SwiGLU outputs, 2.1e-7 -> 0.6e-7 beside an outlier of 1000).
+// (Fields left where they are, at the bottom of the byte, would save half of the shifts: 292 / 167 / 147 ns.  The matrix core
+// aligns products by the operands' exponents, though, and the small ones then lose bits: 1.1e-7 on SwiGLU outputs.)
+// The rows that meet such codes are kept times 2^64 (kRowScale), so that products stay in the range of ordinary fp32
+// numbers; the group's scale takes the powers of two back.  Rows hold magnitudes up to 2^64 (beyond: infinity), and a sum keeps
+// all 24 bits down to 2^-61.  (The norm in front of a layer squares its rows in fp32, which ends at 2^64 as well.)
+constexpr float kRowScale = 0x1p64f, kRowUnscale = 0x1p-64f;
+
+// the upper halves of two fp32 numbers, (lo, hi) in the lower and the upper half
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+// eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and at its scale; their sum in *sum (unscaled)
+__device__ __forceinline__ uint4 matmul_row8(const uint4& v, float* sum) {
+  const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
+  const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
+  *sum = ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
+  return make_uint4(upper_halves(x0 * kRowScale, x4 * kRowScale), upper_halves(x1 * kRowScale, x5 * kRowScale),
+                    upper_halves(x2 * kRowScale, x6 * kRowScale), upper_halves(x3 * kRowScale, x7 * kRowScale));
+}
+
+// one packed word of 4-bit codes -> MFMA operand: pairs (q0,q4),(q1,q5),(q2,q6),(q3,q7)
+__device__ __forceinline__ uint4 subnormal_q4(uint32_t w) {
+  return make_uint4((w << 4) & 0x00F000F0u, w & 0x00F000F0u, (w >> 4) & 0x00F000F0u, (w >> 8) & 0x00F000F0u);
+}
+// one packed word of sixteen 2-bit codes -> two MFMA operands in the same pairing: the byte swap (B0, B2, B1, B3) puts
+// code r and code r + 4 sixteen bits apart, and likewise 8 + r and 12 + r
+__device__ __forceinline__ void subnormal_q2(uint32_t w, uint4& a, uint4& b) {
+  const uint32_t v = __builtin_amdgcn_perm(w, w, 0x03010200u);
+  a = make_uint4((v << 6) & 0x00C000C0u, (v << 4) & 0x00C000C0u, (v << 2) & 0x00C000C0u, v & 0x00C000C0u);
+  b = make_uint4((v >> 2) & 0x00C000C0u, (v >> 4) & 0x00C000C0u, (v >> 6) & 0x00C000C0u, (v >> 8) & 0x00C000C0u);
+}
+
 // What the quantized matmuls need to know about a code width: a lane's share of one 64-wide group
 // of its weight row is half the group -- 16 bytes of 4-bit codes or 8 bytes of 2-bit codes (ternary
-// weights are 2-bit codes) -- and it becomes four MFMA operands of 8 bf16 numbers offset + q * step.
+// weights are 2-bit codes) -- and it becomes four MFMA operands of 8 bf16 numbers.
 //
 // Codes travel in pairs of groups.  Lane l = m + 32 h multiplies half h of row m of a 32-row block.  Asked for that
 // way, from rows as they are, a load instruction touches 32 rows, 32 memory lines, for 1 KB (4-bit) or 512 B (2-bit),
@@ -381,8 +423,7 @@ __device__ __forceinline__ void expand_q2(uint32_t w, uint4& a, uint4& b) {
 template <int BITS, bool SWAPPED = true> struct QmmCodes;
 template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
   static constexpr uint32_t kGroupBytes = 32;     // one group of one row
-  static constexpr uint32_t kNegOffsetAdd = 0x02000200u;  // exponent + 4: 16 * scale (offset 8 at step 1/2)
-  static constexpr float kScaleMul = 2.0f;        // codes enter as 8 + q/2
+  static constexpr float kScaleMul = 0x1p65f;     // q * 2^-129 meets x * 2^64
   uint32_t w[8];  // group 0: w[0..3], group 1: w[4..7]
   // which group of the pair the lane asks for first; its place in 32 rows as they are and in a tiled block; how far
   // behind the second load is
@@ -411,8 +452,7 @@ template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
 };
 template <bool SWAPPED> struct QmmCodes<2, SWAPPED> {  // (SWAPPED = false: only tiled)
   static constexpr uint32_t kGroupBytes = 16;
-  static constexpr uint32_t kNegOffsetAdd = 0x01000100u;  // exponent + 2: 4 * scale (offset 4 at step 1)
-  static constexpr float kScaleMul = 1.0f;        // codes enter as 4 + q
+  static constexpr float kScaleMul = 0x1p63f;     // q * 2^-127 meets x * 2^64
   uint32_t w[4];  // group 0: w[0..1], group 1: w[2..3]
   static __device__ __forceinline__ uint32_t lane_group(uint32_t lane) { return SWAPPED ? lane >> 5 : 0u; }
   static __device__ __forceinline__ size_t lane_offset(uint32_t lane, size_t row_bytes, bool) {
@@ -444,7 +484,7 @@ __device__ __forceinline__ void group_products(const QmmCodes<BITS, SWAPPED>& c,
   if constexpr (BITS == 4) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const uint4 av = expand_q4(c.w[4 * g + s]);
+      const uint4 av = subnormal_q4(c.w[4 * g + s]);
       tmp[0] = mfma_bf16(bx[0][s], av, tmp[0]);
       if constexpr (NTA > 1) tmp[1] = mfma_bf16(bx[1][s], av, tmp[1]);
       after(s);
@@ -453,7 +493,7 @@ __device__ __forceinline__ void group_products(const QmmCodes<BITS, SWAPPED>& c,
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       uint4 a, b;
-      expand_q2(c.w[2 * g + j], a, b);
+      subnormal_q2(c.w[2 * g + j], a, b);
       tmp[0] = mfma_bf16(bx[0][2 * j], a, tmp[0]);
       if constexpr (NTA > 1) tmp[1] = mfma_bf16(bx[1][2 * j], a, tmp[1]);
       after(2 * j);

@@ -2,18 +2,17 @@
 // (token, expert) routes, and the tokens-sorted-by-expert quantized matmul on
 // the bf16 matrix cores.
 //
-// The matmul keeps the 4-bit codes EXACT: a lane's packed uint32 (8 codes of
-// one weight row) is masked straight into four bf16 pairs 8 + q/2
-// (0x4100 | q << 3), which is a matrix-core operand as it stands -- no LDS
+// The matmul keeps the codes EXACT: a lane's packed uint32 is masked into bf16 subnormals (a 4-bit code in bits 4..7 of a
+// 16-bit half is the number q * 2^-129, mf_device.h), which are a matrix-core operand as they stand -- no LDS
 // staging of weights.  x rows are pre-permuted once per call to the same
-// (j, j+4) pairing and staged through LDS per 64-wide K group.  Per K group the
-// matrix core yields sum((8 + q/2) * x) (bf16 x bf16 products are exact in
-// fp32), and the group's bf16 scale is applied in fp32: acc += 2s * tmp -- the
+// (j, j+4) pairing, times 2^64, and staged through LDS per 64-wide K group.  Per K group the
+// matrix core yields 2^-65 sum(q * x) (bf16 x bf16 products are exact in
+// fp32), and the group's bf16 scale is applied in fp32: acc += 2^65 s * tmp -- the
 // reference's own factoring s*sum(q*x) + b*sum(x)
 // (Metal/Quant/dequant_int4.metal:14-17), so no weight is ever rounded to bf16
 // (rounding q*s+b to bf16 would cost ~1.6e-3 relative error per weight, above
-// the layer tolerance).  The b*sum(x) and -16*s*sum(x) terms are two more small
-// matmuls over the group index (operands: the bf16 bias / scale tables, exact,
+// the layer tolerance).  The b*sum(x) term is one more small
+// matmul over the group index (operands: the bf16 bias table, exact,
 // and sum(x) split into three bf16 terms, exact).
 //
 // Replaces prefill_grouped_routed_moe_batched_{phase1,down}
@@ -924,9 +923,9 @@ hipError_t launch_tile_experts(hipStream_t s, const mf_moe_config& c, const void
 // --------------------------------------------------------------- the matmul
 
 // Activation rows as the matmul wants them: inside every run of 8 K values the
-// order is (0,4,1,5,2,6,3,7) -- the pairing a packed code word expands to --
-// and the fp32 sum of every 64-wide K group is kept beside them.  One lane per
-// run of 8; `dst` may be null when `src` is already in that order.
+// order is (0,4,1,5,2,6,3,7) -- the pairing a packed code word expands to --, every value is times kRowScale,
+// and the fp32 sum of every 64-wide K group (of the values as they were) is kept beside them.  One lane per
+// run of 8; `dst` is null when `src` is already in that form.
 struct PrepArgs {  // up to two row sets per launch: the second starts at workgroup `blocks0`
   const uint16_t* src[2];
   uint16_t* dst[2];
@@ -944,15 +943,12 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const PrepArgs a) {
   const uint32_t c = (blockIdx.x - (part ? a.blocks0 : 0u)) * blockDim.x + threadIdx.x;
   uint4 v = make_uint4(0, 0, 0, 0);
   if (c < chunks) v = *reinterpret_cast<const uint4*>(src + static_cast<size_t>(c) * 8);
-  float sum = ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
-              ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
+  float sum;
+  const uint4 row = matmul_row8(v, &sum);
   sum = group_sum(sum, 8);
   if (c >= chunks) return;
-  if (dst)
-    *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) =
-        make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
-                   __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));
-  if ((c & 7) == 0) sums[c >> 3] = sum;
+  if (dst) *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) = row;
+  if ((c & 7) == 0) sums[c >> 3] = dst ? sum : sum * kRowUnscale;
 }
 
 // The same for the layer's input rows and, in the same pass, the scalar shared gate's logit
@@ -973,13 +969,11 @@ __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint
       v = *reinterpret_cast<const uint4*>(xr + static_cast<size_t>(c) * 8);
       if (w_sg) wv = *reinterpret_cast<const uint4*>(w_sg + static_cast<size_t>(c) * 8);
     }
-    float sum = ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
-                ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
+    float sum;
+    const uint4 prepared = matmul_row8(v, &sum);
     sum = group_sum(sum, 8);
     if (live) {
-      *reinterpret_cast<uint4*>(xp + (base + c) * 8) =
-          make_uint4(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u), __builtin_amdgcn_perm(v.z, v.x, 0x07060302u),
-                     __builtin_amdgcn_perm(v.w, v.y, 0x05040100u), __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));
+      *reinterpret_cast<uint4*>(xp + (base + c) * 8) = prepared;
       if ((c & 7) == 0) sums[(base + c) >> 3] = sum;
       acc = __builtin_fmaf(bf16_lo(wv.x), bf16_lo(v.x), acc);
       acc = __builtin_fmaf(bf16_hi(wv.x), bf16_hi(v.x), acc);
@@ -1136,8 +1130,8 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   }
 
   uint4* s_x = reinterpret_cast<uint4*>(smem);                      // 2 stages x 2 groups x 512 uint4
-  // The scale of every (row, group): fp32, or (TAB16, long contractions) a bf16 number -- 2 * scale for 4-bit
-  // codes is one (exponent + 1), so the upper half of the fp32 product is all of it.  That is half the LDS,
+  // The scale of every (row, group): fp32, or (TAB16, long contractions) a bf16 number -- a power of two times a bf16
+  // scale is one, so the upper half of the fp32 product is all of it.  That is half the LDS,
   // which lets two workgroups share a CU up to 112 K groups (K = 7168), for one more instruction per read.
   using tab_t = std::conditional_t<TAB16, uint16_t, float>;
   tab_t* s_scale = reinterpret_cast<tab_t*>(smem + kQmmXBytes);  // [NPROJ][4][ng][32]
@@ -1316,12 +1310,9 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
 
-  // ---- per step: scale / code step (4-bit codes enter as 8 + q/2: 2 * scale; 2-bit codes as 4 + q: scale)
-  // of the wave's rows into the [g][row] fp32 table, and the bias and offset terms:
-  // acc[token, row] += sumx[token, g] * B[row, g] + sumx[token, g] * (-offset S[row, g]), offset 16 or 4.
-  // -offset * S is formed in place (exponent + 4 or + 2, sign flipped: exact; a zero scale becomes 2^-123 / 2^-125).
-  // sumx enters as three bf16 terms, which hold all 24 bits: the -offset * S * sumx term cancels the
-  // offset * sum(x) the matrix core accumulated with the codes, so it has to be exact.
+  // ---- per step: the scales of the wave's rows, times the powers of two that codes and rows carry, into the
+  // [g][row] table, and the bias term: acc[token, row] += sumx[token, g] * B[row, g].
+  // sumx enters as three bf16 terms, which hold all 24 bits.
   // A tile of at most 32 routes fills only the first token block: the second block's matrix
   // instructions and scale multiplies are left out (NTA = 1); its accumulators stay zero and its
   // output slots are empty.  Of a tile of at most 8 routes (most tiles of a short prompt) a lane's first four results are all
@@ -1333,7 +1324,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     tab_cur = tab_fetch(g0 + 16 < ng ? g0 + 16 : g0);  // past the end: the same step again, unused
     const uint32_t gl = g0 + 8 * h;
     const bool have = gl < ng;
-    uint4 ab[NPROJ], as[NPROJ];
+    uint4 ab[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
       tab_t* tab = s_scale + (p * kQmmWaves + wv) * ng * 32;
@@ -1347,14 +1338,11 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
         if (have && (NG8 || gl + 2 * i < ng)) tab[(gl + 2 * i) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_lo(pr[i]));
         if (have && (NG8 || gl + 2 * i + 1 < ng)) tab[(gl + 2 * i + 1) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_hi(pr[i]));
       }
-      constexpr uint32_t kAdd = QmmCodes<BITS>::kNegOffsetAdd;
       // ternary rows store no biases: the bias is -scale (the table pointer is the scale table then)
       ab[p] = a.ternary ? make_uint4(t.B[p].x ^ 0x80008000u, t.B[p].y ^ 0x80008000u, t.B[p].z ^ 0x80008000u,
                                      t.B[p].w ^ 0x80008000u)
                         : t.B[p];
-      as[p] = make_uint4((t.S[p].x + kAdd) ^ 0x80008000u, (t.S[p].y + kAdd) ^ 0x80008000u,
-                         (t.S[p].z + kAdd) ^ 0x80008000u, (t.S[p].w + kAdd) ^ 0x80008000u);
-      if (!have) ab[p] = as[p] = make_uint4(0, 0, 0, 0);
+      if (!have) ab[p] = make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int nt = 0; nt < NTA; ++nt) {
@@ -1378,11 +1366,8 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
       for (int p = 0; p < NPROJ; ++p) {
         acc[p][nt] = mfma_bf16(b_hi, ab[p], acc[p][nt]);
-        acc[p][nt] = mfma_bf16(b_hi, as[p], acc[p][nt]);
         acc[p][nt] = mfma_bf16(b_mid, ab[p], acc[p][nt]);
-        acc[p][nt] = mfma_bf16(b_mid, as[p], acc[p][nt]);
         acc[p][nt] = mfma_bf16(b_lo, ab[p], acc[p][nt]);
-        acc[p][nt] = mfma_bf16(b_lo, as[p], acc[p][nt]);
       }
     }
   }
@@ -1440,7 +1425,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
       for (int gi = 0; gi < 2; ++gi) {
         const uint32_t g = gu + gi;
         if (!NG8 && g >= ng) break;  // the half pair at the end of an odd number of groups
-        // ---- matrix core: tmp[token, row] = sum over the group of x * (8 + q/2)
+        // ---- matrix core: tmp[token, row] = sum over the group of x * q, times the powers of two kScaleMul takes back
         const uint4* buf = s_x + uu * 1024 + gi * 512;
         uint4 bx[2][4];
 #pragma unroll
@@ -1489,7 +1474,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
   const uint32_t row_raw = (slice * kQmmWaves + wv) * wave_rows;  // past a.rows: this wave has no rows of its own
   if (a.epi == 0) {
-    // SwiGLU, narrowed to bf16, transposed through the (now free) x ring so that a lane stores
+    // SwiGLU, narrowed to bf16 (at the scale of the matmul's rows, kRowScale), transposed through the (now free) x ring so that a lane stores
     // 16 bytes of one token: [token][32 rows] per wave, the rows of a run of 8 in the
     // (0,4,1,5,2,6,3,7) order phase 2 reads, i.e. rows r and r + 4 share a 32-bit word.
     __syncthreads();  // every wave is past its last read of the ring
@@ -1514,13 +1499,13 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           for (int i = 0; i < 4; ++i) {
             float gv = acc[0][nt][4 * j + i], uv = acc[NPROJ - 1][nt][4 * j + i];
             if constexpr (kMaple) {  // maple_moe.metal:153-164
-              bits[i] = f_to_bf16(maple_swiglu(gv, uv));
+              bits[i] = f_to_bf16(maple_swiglu(gv, uv) * kRowScale);
             } else {
               const float gr = round_bf16(gv), ur = round_bf16(uv);
               const float g0 = narrow ? gr : gv, u0 = narrow ? ur : uv;
               gv = clamp ? fminf(g0, a.limit) : g0;  // (selects, so that a NaN stays one without a clamp)
               uv = clamp ? fminf(fmaxf(u0, -a.limit), a.limit) : u0;
-              bits[i] = f_to_bf16(fast_silu(gv) * uv);
+              bits[i] = f_to_bf16(fast_silu(gv) * uv * kRowScale);
             }
           }
           // lanes m and m ^ 4 trade halves: the lower lane ends with tokens i = 0, 1 of both rows,
@@ -1754,7 +1739,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
                 ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
       }
       part = group_sum(part, 4);
-      if (st_q == 0) s_sum[st_i * NG + g] = part;
+      if (st_q == 0) s_sum[st_i * NG + g] = part * kRowUnscale;
     }
   }
   uint32_t rd_col[4];
@@ -1764,13 +1749,13 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   qmm_trace(a, work, 2);
   // sum(x) of a group as three bf16 terms (all 24 bits), see qmm_kernel.  Both halves of the wave hold
   // the sums of groups 0..7 of the lane's two routes: K slots 8h..8h+7 of the bias product are those
-  // groups again, multiplied by the biases for h = 0 and by -offset * scale for h = 1.
+  // groups again, the first terms for h = 0 and the second ones for h = 1, then the third for h = 0 -- two products instead of three.
   // A tile of at most 32 routes fills only the first route block (NTA = 1): the second block, whose routes
   // would all repeat the last route, is left out of the products, the scale multiplies and the stores.
   // (RES = 4 for a tile of at most 8 routes: as in qmm_item)
   auto tile_body = [&](auto nta_c, auto res_c) {
   constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
-  uint4 b_term[2][3];
+  uint4 b_term[2][2];
 #pragma unroll
   for (int nt = 0; nt < NTA; ++nt) {
     float sx[8];
@@ -1785,28 +1770,27 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
       mid[e] = __float_as_uint(r1) & 0xFFFF0000u;
       lo[e] = __float_as_uint(r1 - __uint_as_float(mid[e]));
     }
-    b_term[nt][0] = make_uint4((hi[0] >> 16) | hi[1], (hi[2] >> 16) | hi[3], (hi[4] >> 16) | hi[5], (hi[6] >> 16) | hi[7]);
-    b_term[nt][1] = make_uint4((mid[0] >> 16) | mid[1], (mid[2] >> 16) | mid[3], (mid[4] >> 16) | mid[5],
-                               (mid[6] >> 16) | mid[7]);
-    b_term[nt][2] = make_uint4(__builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u), __builtin_amdgcn_perm(lo[3], lo[2], 0x07060302u),
+    uint32_t first[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) first[e] = h ? mid[e] : hi[e];
+    b_term[nt][0] = make_uint4((first[0] >> 16) | first[1], (first[2] >> 16) | first[3], (first[4] >> 16) | first[5],
+                               (first[6] >> 16) | first[7]);
+    b_term[nt][1] = make_uint4(__builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u), __builtin_amdgcn_perm(lo[3], lo[2], 0x07060302u),
                                __builtin_amdgcn_perm(lo[5], lo[4], 0x07060302u), __builtin_amdgcn_perm(lo[7], lo[6], 0x07060302u));
+    if (h) b_term[nt][1] = make_uint4(0, 0, 0, 0);
   }
 
   for (uint32_t w = 0; w < n_walk; ++w) {
     const uint32_t step = w + 1 < n_walk ? 1u : 0u;  // the last slice requests itself again: no branch around loads
     const uint8_t* wnext = wrow + static_cast<size_t>(step) * 256 * kRowBytes;
-    // scale words of this slice; bias operand: the biases for K slots 0..7, -offset * scale for K slots
-    // 8..15 (formed in place: exponent + 4 or + 2, sign flipped -- exact; a zero scale becomes 2^-123 / 2^-125);
+    // scale words of this slice; bias operand: the biases, for both halves;
     // ternary rows store no biases: theirs is -scale (the bias pointer is the scale table then)
     uint4 Sv[2], bop[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      constexpr uint32_t kAdd = QmmCodes<BITS>::kNegOffsetAdd;
       Sv[p] = nS[p];
-      const uint4 neg = make_uint4((nS[p].x + kAdd) ^ 0x80008000u, (nS[p].y + kAdd) ^ 0x80008000u,
-                                   (nS[p].z + kAdd) ^ 0x80008000u, (nS[p].w + kAdd) ^ 0x80008000u);
       const uint32_t flip = a.ternary ? 0x80008000u : 0u;
-      bop[p] = h ? neg : make_uint4(nB[p].x ^ flip, nB[p].y ^ flip, nB[p].z ^ flip, nB[p].w ^ flip);
+      bop[p] = make_uint4(nB[p].x ^ flip, nB[p].y ^ flip, nB[p].z ^ flip, nB[p].w ^ flip);
     }
     f32x16_t acc[2][2];
 #pragma unroll
@@ -1816,7 +1800,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
 #pragma unroll
-        for (int term = 0; term < 3; ++term) acc[p][nt] = mfma_bf16(b_term[nt][term], bop[p], acc[p][nt]);
+        for (int term = 0; term < 2; ++term) acc[p][nt] = mfma_bf16(b_term[nt][term], bop[p], acc[p][nt]);
       }
     // the next slice's scale / bias words (the registers are free again)
     srow += step * 256 * NG;
@@ -2481,8 +2465,8 @@ __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* 
       gr = fminf(gr, limit);
       ur = fminf(fmaxf(ur, -limit), limit);
     }
-    a[i] = f_to_bf16(fast_silu(gr) * ur);
-    v[i] = bf16_to_f(static_cast<uint16_t>(a[i]));
+    a[i] = f_to_bf16(fast_silu(gr) * ur * kRowScale);
+    v[i] = bf16_to_f(static_cast<uint16_t>(a[i])) * kRowUnscale;
   }
   float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
   sum = group_sum(sum, 8);

@@ -108,6 +108,38 @@ def test_qmm_matches_gemv_oracle(gpu, oracle, bits, m, n, k):
                        f"qmm bf16 bits={bits}")
 
 
+@pytest.mark.parametrize("bits,m,n,k", [(4, 9, 128, 128), (4, 70, 256, 1152), (2, 33, 128, 896), (1, 64, 256, 512)])
+def test_qmm_of_large_and_small_rows(gpu, bits, m, n, k):
+    """rows times a power of two give the results times it, bit for bit, from 2^-48 to 2^48 (the matmul keeps rows at a
+    scale of its own), one row holds an outlier, and every result lies within the bound of an fp32 sum from its 64-bit value"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m + n + k + bits)
+    per = 4 if bits == 4 else 2
+    codes = torch.randint(0, 3 if bits == 1 else 2 ** per, (n, k), generator=gen, device="cuda", dtype=torch.int32)
+    parts = codes.view(n, k * per // 8, 8 // per)
+    packed = sum(parts[..., i] << (per * i) for i in range(8 // per)).to(torch.uint8)
+    scales = (0.01 + 0.01 * torch.rand(n, k // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+    biases = -scales if bits == 1 else (-0.1 * torch.rand(n, k // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+    q = ops.QuantizedTensor(packed.contiguous(), scales, biases, bits, n, k)
+    x = torch.randn(m, k, generator=gen, device="cuda")
+    x[m // 2, k // 3] *= 1000
+    x = x.to(torch.bfloat16)
+    op = ops.MPPPrefillInt4QMM(gpu)
+    out = []
+    for shift in (0, 48, -48):
+        y = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        assert op.encode(q, (x.double() * 2.0 ** shift).to(torch.bfloat16), y, m, n, k) == _expected_path(n, k, 0)
+        out.append(y.double() * 2.0 ** -shift)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    groups, x, codes, scales, biases = k // 64, x.cpu(), codes.cpu(), scales.cpu(), biases.cpu()
+    xg, qg = x.double().view(m, groups, 64), codes.double().view(n, groups, 64)
+    terms = scales.double().T[:, None, :] * torch.einsum("mgk,ngk->gmn", xg, qg)
+    bias = biases.double().T[:, None, :] * xg.sum(2).T[:, :, None]
+    sizes = scales.double().T[:, None, :] * torch.einsum("mgk,ngk->gmn", xg.abs(), qg) + bias.abs()
+    # a product sum of 64 and its bias term, then `groups` additions, each within 2^-24 of what it adds up (Higham, 4.2)
+    assert ((out[0].cpu() - (terms + bias).sum(0)).abs() <= (groups + 8) * 2.0 ** -24 * sizes.sum(0)).all()
+
+
 def test_qmm_unavailable_for_bad_arguments(gpu, oracle):
     """MPPPrefillInt4QMM.swift:43-55: a K that is no multiple of the group, empty sizes, odd table offsets"""
     q, xb = _reference_inputs(oracle, 8, 32, 64, False)
@@ -216,7 +248,7 @@ def test_mlp_block_of_few_rows(gpu, oracle, bits, d, f, t):
 @pytest.mark.parametrize("bits", [4, 2])
 @pytest.mark.parametrize("d,f,t", [(1152, 640, 20), (256, 3200, 70)])
 def test_mlp_block_keeps_infinities_to_their_row(gpu, bits, d, f, t):
-    """rows with an infinity or a NaN come out NaN (the code offset is taken out as inf - inf, as in the row kernels) and
+    """rows with an infinity or a NaN come out NaN (an infinity meets codes of zero, and biases below zero) and
     leave every other row's bits alone"""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(d + t + bits)
