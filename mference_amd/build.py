@@ -11,7 +11,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmfmoe.so")
 SOURCES = ["format.hip", "gemv.hip", "int8_mlp.hip", "router.hip", "router_family.hip", "moe_decode.hip", "moe_fused.hip",
-           "moe_prefill.hip", "static_scratch.hip", "api.hip"]
+           "moe_prefill.hip", "qmm_ring.hip", "qmm_resident.hip", "qmm_tile32.hip", "static_scratch.hip", "api.hip"]
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -117,7 +117,7 @@ def build(verbose: bool = False, only: list[str] | None = None) -> str:
         if unknown:
             raise ValueError(f"not a source of the library: {unknown}")
     todo = [(s, o) for s, o in zip(SOURCES, objs) if only is None or s in only or not os.path.exists(o)]
-    jobs = min(8, max(1, (os.cpu_count() or 2) // 2))
+    jobs = min(8, max(1, (os.cpu_count() or 2) * 3 // 4))
     with ThreadPoolExecutor(jobs) as pool:
         list(pool.map(lambda so: _run([hipcc, *FLAGS, "-c", "-o", so[1], os.path.join(CSRC, so[0])], verbose), todo))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs], verbose)

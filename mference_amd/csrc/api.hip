@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "mf_internal.h"
+#include "mf_qmm.h"
 
 namespace {
 
@@ -738,7 +739,7 @@ mf_status mf_moe_group(mf_moe* h, mf_stream stream, const uint32_t* idx, const f
   auto s = static_cast<hipStream_t>(stream);
   if (t == 0) {  // queryCount == 0 is valid (PrefillMoEGrouping.swift:99-104): no pairs, every expert empty
     MF_HIP(h->ctx, mf::launch_group(s, nullptr, nullptr, 0, h->cfg.top_k, h->cfg.num_experts, expert_counts,
-                                    expert_offsets, h->ws.group_tmp + 512, nullptr, nullptr, 0, nullptr,
+                                    expert_offsets, h->ws.group_tmp + 512, nullptr, {},
                                     h->ws.group_tmp + 3 * 512, h->ws.group_tmp + 2048));
     return MF_OK;
   }
@@ -747,7 +748,7 @@ mf_status mf_moe_group(mf_moe* h, mf_stream stream, const uint32_t* idx, const f
   uint32_t* starts = h->ws.group_tmp + 512;
   uint32_t* status = h->ws.group_tmp + 3 * 512;
   MF_HIP(h->ctx, mf::launch_group(s, idx, w, t, h->cfg.top_k, h->cfg.num_experts, expert_counts,
-                                  expert_offsets, starts, sorted_pairs, nullptr, 0, nullptr, status,
+                                  expert_offsets, starts, sorted_pairs, {}, status,
                                   h->ws.group_tmp + 2048));
   return MF_OK;
 }

@@ -95,6 +95,11 @@ __device__ __forceinline__ float mf_sqrtsoftplus(float x) {
 // moe.metal:79-84
 __device__ __forceinline__ float mf_silu(float x) { return x / (1.0f + mf_exp(-x)); }
 
+// silu with the hardware exp2 / reciprocal (1 ulp each): the result is narrowed to bf16 right after
+__device__ __forceinline__ float fast_silu(float x) {
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+}
+
 // int8_gelu_pytorch_tanh (Metal/Quant/dequant_int8.metal:44-49): 0.5 x (1 + tanh(c (x + 0.044715 x^3))), the
 // argument clamped to +-20; tanh(z) = 1 - 2 / (exp(2 z) + 1) on this build's exp, the same IEEE sequence as the
 // CPU oracle.
@@ -391,6 +396,23 @@ __device__ __forceinline__ uint4 matmul_row8(const uint4& v, float* sum) {
   *sum = ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
   return make_uint4(upper_halves(x0 * kRowScale, x4 * kRowScale), upper_halves(x1 * kRowScale, x5 * kRowScale),
                     upper_halves(x2 * kRowScale, x6 * kRowScale), upper_halves(x3 * kRowScale, x7 * kRowScale));
+}
+
+// The fp32 sums of a row's groups of 64 values, as the matmuls read them for the bias term: three bf16 numbers each, which
+// hold all 24 bits.  Per eight groups the eight first parts, then the second, then the third ones (48 bytes); groups past the
+// row's last one are zeros.
+__host__ __device__ __forceinline__ size_t group_sum_words(uint32_t ng) { return static_cast<size_t>((ng + 7) / 8) * 24; }
+// sum of group g of ng; `row` = where the row's sums start
+__device__ __forceinline__ void store_group_sum(uint16_t* row, uint32_t g, uint32_t ng, float sum) {
+  const uint32_t hi = __float_as_uint(sum) & 0xFFFF0000u;
+  const float r1 = sum - __uint_as_float(hi);
+  const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u, lo = __float_as_uint(r1 - __uint_as_float(mid));
+  uint16_t* at = row + g / 8 * 24 + g % 8;
+  at[0] = static_cast<uint16_t>(hi >> 16);
+  at[8] = static_cast<uint16_t>(mid >> 16);
+  at[16] = static_cast<uint16_t>(lo >> 16);
+  if (g + 1 == ng)
+    for (uint32_t j = 1; (g + j) % 8; ++j) at[j] = at[8 + j] = at[16 + j] = 0;
 }
 
 // one packed word of 4-bit codes -> MFMA operand: pairs (q0,q4),(q1,q5),(q2,q6),(q3,q7)

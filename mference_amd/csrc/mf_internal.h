@@ -182,9 +182,10 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
 
 // moe_prefill.hip
 namespace mf {
+struct TileLists;  // mf_qmm.h
 hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint32_t t, uint32_t K,
                         uint32_t E, uint32_t* counts, uint32_t* offsets, uint32_t* starts,
-                        mf_pair* sorted, void* tiles, uint32_t tile_slots, uint32_t* n_tiles,
+                        mf_pair* sorted, const TileLists& tiles,
                         uint32_t* status, uint32_t* chunk_hist);
 size_t group_scratch_words();
 size_t prefill_workspace_bytes(const mf_moe_config& c, uint32_t t);

@@ -1,0 +1,1021 @@
+// The quantized matmuls of the prefill path: device code and launches, for tiles of 64 and of 32 routes.  Instantiated by
+// qmm_ring.hip, qmm_resident.hip and qmm_tile32.hip (a source each, so that they compile side by side).
+#pragma once
+
+#include <algorithm>
+#include <type_traits>
+
+#include "mf_qmm.h"
+
+#pragma clang fp contract(off)
+
+namespace mf {
+
+// x tile ring: 2 stages of 2 K groups
+__host__ __device__ constexpr uint32_t qmm_x_bytes(uint32_t tile) { return 2 * 2 * tile * 8 * 16; }
+// waves a SIMD (workgroups a CU) that the kernels' registers are budgeted for
+__host__ __device__ constexpr int qmm_waves(uint32_t tile, int nproj) { return tile == kSmallTile || nproj == 1 ? 3 : 2; }
+
+__device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint32_t k) {
+  if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
+}
+
+// One workgroup: a tile of TT (64 or 32) routes of one expert x 128 weight rows (4 waves x 32) x
+// NPROJ projections, the whole K.  The matrix core computes the TRANSPOSED
+// product: the A operand is the x tile (tokens are the rows), the B operand is
+// the expanded codes, so a lane ends up holding ONE weight row (its column
+// m = lane % 32) for 16 tokens of each 32-token block, and the per-group scale
+// is one scalar per lane.  Tiles of 64: with two row blocks per wave two waves per SIMD stay
+// resident (the register budget of 256 keeps the matrix-core results in ordinary
+// registers, where the scale multiply reads them directly); with one row block the
+// kernel fits 168 registers and three waves stay resident.  Tiles of 32 fit 168 registers in both forms: the table words
+// are not requested a step ahead, units are kept apart in the loop, and a handful of values waits in scratch memory while a
+// loop runs (none inside it).  What that buys: 2816 x 704, 128 experts, 300 tokens, gate / up 70 -> 66 us and down
+// 70 -> 47 us under the tracer; Qwen shape, 93 tokens, gate / up 38.5 -> 31.7.
+// LDS (dynamic): x tile ring, 2 stages x 2 K groups x [TT / 32 nt][4 s][2 h][32 n] x 16 B,
+// scale tables [NPROJ][4 waves][ng][32 rows] fp32 or bf16, out slots [TT] u32.
+// One launch can carry two independent problems of the same instantiation (the routed experts
+// and the shared expert of the same phase): the second problem's work items follow the first's
+// on every XCD, so they fill the slots the first problem's last round leaves empty instead of
+// running as a launch of their own that covers a quarter of the chip.
+struct QmmLaunch {
+  QmmArgs part[2];
+  uint32_t per_xcd[2];  // work items of each part on one XCD (grid = 8 * their sum)
+};
+
+// NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
+// of groups and rows.
+template <int TT, int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
+__device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_t* smem) {
+  constexpr int NT = TT / 32;             // token blocks of a tile
+  constexpr uint32_t kXGroup = TT * 8;    // 16-byte pieces of one K group of the x tile
+  constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const uint32_t m = lane & 31, h = lane >> 5;
+  const uint32_t wave_rows = a.pair_rows ? 32u * NPROJ : 32u;  // weight rows of one wave
+  const uint32_t n_slices = NG8 ? a.rows / (kQmmWaves * wave_rows) : (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
+  uint32_t tile_id = work / n_slices, slice = work % n_slices, win = 0;
+  if (a.dense_mode) {
+    if (work >= a.dense_items) return;
+    const uint32_t inner = a.tile_major ? n_slices : a.dense_tiles, outer = a.tile_major ? a.dense_tiles : n_slices;
+    const uint32_t lo = work % inner, rest = work / inner, hi = rest % outer;
+    tile_id = a.tile_major ? hi : lo;
+    slice = a.tile_major ? lo : hi;
+    win = rest / outer;
+    if (tile_id >= a.dense_tiles) return;
+  }
+  uint32_t ng = a.kdim / kGroup, g_off = a.g_off;
+  uint8_t* out_base = static_cast<uint8_t*>(a.out);
+  uint8_t* out2_base = static_cast<uint8_t*>(a.out2);
+  if (a.n_win > 1) {  // this work item's window of the contraction
+    g_off = dense_window_start(a.ng_ld, a.n_win, win);
+    ng = dense_window_start(a.ng_ld, a.n_win, win + 1) - g_off;
+    out_base += win * a.out_win_stride * sizeof(float);
+    if (out2_base) out2_base += win * a.out_win_stride * sizeof(float);
+  }
+  qmm_trace(a, work, 0);
+
+  uint32_t expert = 0, pair_start, count;
+  if (a.dense_mode) {
+    pair_start = tile_id * TT;
+    count = min(static_cast<uint32_t>(TT), a.dense_rows - pair_start);
+  } else {
+    // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
+    // fetched in a second round trip)
+    const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
+    const Tile t{tv.x, tv.y, tv.z, tv.w};
+    if (t.count == 0) return;
+    expert = t.expert;
+    pair_start = t.pair_start;
+    count = t.count;
+  }
+
+  uint4* s_x = reinterpret_cast<uint4*>(smem);                      // 2 stages x 2 groups x kXGroup uint4
+  // The scale of every (row, group): fp32, or (TAB16, long contractions) a bf16 number -- a power of two times a bf16
+  // scale is one, so the upper half of the fp32 product is all of it.  That is half the LDS,
+  // which lets two workgroups share a CU up to 112 K groups (K = 7168), for one more instruction per read.
+  using tab_t = std::conditional_t<TAB16, uint16_t, float>;
+  tab_t* s_scale = reinterpret_cast<tab_t*>(smem + qmm_x_bytes(TT));  // [NPROJ][4][ng][32]
+  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT) + ((NPROJ * kQmmWaves * ng * 32 * sizeof(tab_t) + 15) & ~15u));
+
+  // weight pointers of this workgroup's projections
+  const uint8_t* Wp[NPROJ];
+  const uint16_t* Sp[NPROJ];
+  const uint16_t* Bp[NPROJ];
+  uint32_t row_base[NPROJ];  // first weight row of each of this wave's 32-row blocks
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p) {
+    const int t = a.pair_rows ? 0 : p;
+    if (a.dense_mode) {
+      Wp[p] = static_cast<const uint8_t*>(a.dense[t].weights);
+      Sp[p] = a.dense[t].scales;
+      Bp[p] = a.dense[t].biases;
+    } else {
+      const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
+      Wp[p] = blob + a.w_off[t];
+      Sp[p] = reinterpret_cast<const uint16_t*>(blob + a.s_off[t]);
+      Bp[p] = reinterpret_cast<const uint16_t*>(blob + a.b_off[t]);
+    }
+    // (a width that is no multiple of the workgroup's rows: the last slice's waves past the end compute the last
+    // 32 rows again and store nothing)
+    row_base[p] = (slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u);
+    if (!NG8) row_base[p] = min(row_base[p], a.rows - 32u);
+  }
+  const uint32_t ng_ld = a.ng_ld ? a.ng_ld : ng;
+  const size_t row_bytes = static_cast<size_t>(ng_ld) * kGB;
+
+  // ---- everything the tile needs that depends only on the tile: issued back to back.
+  // Routes past `count` read the tile's last route instead (finite data, results discarded).
+  // staging: a thread takes two runs of 8 K values of one token in every group, or one of a tile of at most 32 routes
+  const bool few = NT == 1 || (NPROJ == 2 && count <= 32);
+  const uint32_t st_i = few ? threadIdx.x >> 3 : threadIdx.x >> 2;
+  const uint32_t st_c0 = few ? threadIdx.x & 7 : (threadIdx.x & 3) * 2, st_c1 = few ? st_c0 : st_c0 + 1;
+  const uint32_t st_pair = pair_start + min(st_i, count - 1);
+  uint32_t st_row = st_pair, xrow[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) xrow[nt] = pair_start + min(32 * nt + m, count - 1);
+  uint32_t slot = pair_start + min(threadIdx.x & 63u, count - 1);
+  // the routes' records are requested here and looked at behind the code loads below, which do not depend on
+  // them: the first codes are then on their way one memory round trip earlier
+  mf_pair pr{};
+  uint32_t tok_st = 0, tok[NT] = {};
+  if (!a.dense_mode) {
+    pr = a.sorted[slot];
+    if (a.gather) {
+      tok_st = a.sorted[st_pair].token;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) tok[nt] = a.sorted[xrow[nt]].token;
+    }
+  }
+  const uint8_t* wrow[NPROJ];
+  using Codes = QmmCodes<BITS, SWAPPED>;
+  const uint32_t gstride = a.tiled ? 32u * kGB : kGB;  // bytes from a group's codes to the next group's
+  const size_t second = Codes::second(row_bytes, a.tiled);
+  const uint32_t last_pair = (ng - 1) & ~1u;
+  // (the last pair of an odd number of groups is half a pair: the lanes that would ask for its second group ask for the first)
+  const uint32_t odd_back = !NG8 && (ng & 1u) ? Codes::lane_group(lane) * gstride : 0u;
+  auto pair_at = [&](uint32_t g) -> size_t {  // g: the pair's first group; past the end: the last pair again
+    const uint32_t gc = min(g, last_pair);
+    return static_cast<size_t>(gc) * gstride - (!NG8 && gc == last_pair ? odd_back : 0u);
+  };
+  Codes cur[NPROJ][2];
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p) {
+    wrow[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride +
+              Codes::lane_offset(lane, row_bytes, a.tiled);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow[p] + pair_at(2 * u), second);
+  }
+  __builtin_amdgcn_sched_barrier(0);  // (keeps the look at the routes behind the code loads)
+  if (!a.dense_mode) {
+    if (a.gather) {
+      st_row = tok_st;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) xrow[nt] = tok[nt];
+    }
+    if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
+  }
+  // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
+  const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_c0 * 8;
+  const uint32_t st_2nd = (st_c1 - st_c0) * 8;
+  // K groups travel in pairs; a contraction of an odd number of groups ends in half a pair (its other half is read
+  // from the last group again and not multiplied)
+  // (arrays of a native vector type: arrays of the uint4 struct were kept in scratch memory)
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t xs[2][2];  // the pair after the one in LDS, on its way there
+  u32x4_t x0[2][2];
+#pragma unroll
+  for (int gi = 0; gi < 2; ++gi) {
+    const uint32_t ga = NG8 ? gi : min(static_cast<uint32_t>(gi), ng - 1), gb = NG8 ? 2u + gi : min(2u + gi, ng - 1);
+    x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup);
+    if (NT > 1) x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + st_2nd);
+    xs[gi][0] = xs[gi][1] = u32x4_t{0, 0, 0, 0};
+    if (NG8 || ng > 2) {
+      xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup);
+      if (NT > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + st_2nd);
+    }
+  }
+  // Scale and bias words of the lane's row and the group sums of its two routes, 8 K groups at a time
+  // (groups gl = g0 + 8h .. gl + 7 for g0 = 0, 16, ...); the loads of the first step leave now, with the
+  // codes and the x rows, the loads of every later step one step ahead of their use.
+  auto sums_fetch = [&](int nt, uint32_t gc, uint4 (&sum)[3]) {
+    const uint16_t* sp = a.sumx + xrow[nt] * group_sum_words(ng_ld) + (g_off + gc) / 8 * 24;
+#pragma unroll
+    for (int part = 0; part < 3; ++part) sum[part] = *reinterpret_cast<const uint4*>(sp + 8 * part);
+  };
+  struct TabStep {
+    uint4 S[NPROJ], B[NPROJ];
+    uint4 sum[3];  // of the first token block (the second block's are requested at the top of their step: registers)
+  };
+  auto tab_fetch = [&](uint32_t g0) {
+    TabStep t;
+    const uint32_t gl = g0 + 8 * h;
+    const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
+    sums_fetch(0, gc, t.sum);
+    if (!NG8 && ng >= 8) {  // whole 16-byte loads at any group; in the last step they end at the row's end and are moved down
+      const uint32_t gb = min(gc, ng - 8), sh = gc - gb;
+      const bool last = g0 + 16 > ng;  // (uniform)
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+        const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gb;
+        t.B[p] = load_16_bytes(Bp[p] + at);
+        t.S[p] = load_16_bytes(Sp[p] + at);
+        if (last) {
+          t.B[p] = drop_bf16(t.B[p], sh);
+          t.S[p] = drop_bf16(t.S[p], sh);
+        }
+      }
+      return t;
+    }
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) {
+      const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gc;
+      t.B[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Bp[p] + at) : load_x8<false>(Bp[p] + at))
+                   : load_bf16x8_guarded(Bp[p] + at, ng - gc);
+      t.S[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Sp[p] + at) : load_x8<false>(Sp[p] + at))
+                   : load_bf16x8_guarded(Sp[p] + at, ng - gc);
+    }
+    return t;
+  };
+  TabStep tab_cur;
+  if constexpr (NT > 1) tab_cur = tab_fetch(0);
+  qmm_trace(a, work, 1);
+
+  if (threadIdx.x < TT) s_slot[threadIdx.x] = threadIdx.x < count ? slot : 0xFFFFFFFFu;
+
+  f32x16_t acc[NPROJ][NT];
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
+
+  // ---- per step: the scales of the wave's rows, times the powers of two that codes and rows carry, into the
+  // [g][row] table, and the bias term: acc[token, row] += sumx[token, g] * B[row, g].
+  // A tile of at most 32 routes fills only the first token block: the second block's matrix
+  // instructions and scale multiplies are left out (NTA = 1); its accumulators stay zero and its
+  // output slots are empty.  Of a tile of at most 8 routes (most tiles of a short prompt) a lane's first four results are all
+  // there is: only those are scaled (RES), 4 of 16 multiply-adds per group and row block.
+  auto tile_body = [&](auto nta_c, auto res_c) {
+  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
+  for (uint32_t g0 = 0; g0 < ng; g0 += 16) {
+    TabStep t;
+    if constexpr (NT > 1) {
+      t = tab_cur;
+      tab_cur = tab_fetch(g0 + 16 < ng ? g0 + 16 : g0);  // past the end: the same step again, unused
+    } else {
+      t = tab_fetch(g0);  // (three waves a SIMD hide its round trip, and their registers do not hold a second step)
+    }
+    const uint32_t gl = g0 + 8 * h;
+    const bool have = gl < ng;
+    uint4 sum[NTA][3];
+#pragma unroll
+    for (int part = 0; part < 3; ++part) sum[0][part] = t.sum[part];
+    if constexpr (NTA > 1) sums_fetch(1, have ? gl : 0, sum[1]);
+    uint4 ab[NPROJ];
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p) {
+      tab_t* tab = s_scale + (p * kQmmWaves + wv) * ng * 32;
+      auto entry = [](float v) -> tab_t {
+        if constexpr (TAB16) return static_cast<uint16_t>(__float_as_uint(v) >> 16);
+        else return v;
+      };
+      const uint32_t pr[4] = {t.S[p].x, t.S[p].y, t.S[p].z, t.S[p].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (have && (NG8 || gl + 2 * i < ng)) tab[(gl + 2 * i) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_lo(pr[i]));
+        if (have && (NG8 || gl + 2 * i + 1 < ng)) tab[(gl + 2 * i + 1) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_hi(pr[i]));
+      }
+      // ternary rows store no biases: the bias is -scale (the table pointer is the scale table then)
+      ab[p] = a.ternary ? make_uint4(t.B[p].x ^ 0x80008000u, t.B[p].y ^ 0x80008000u, t.B[p].z ^ 0x80008000u,
+                                     t.B[p].w ^ 0x80008000u)
+                        : t.B[p];
+      if (!have) ab[p] = make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int nt = 0; nt < NTA; ++nt) {
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+#pragma unroll
+        for (int part = 0; part < 3; ++part) acc[p][nt] = mfma_bf16(sum[nt][part], ab[p], acc[p][nt]);
+      }
+    }
+  }
+  qmm_trace(a, work, 2);
+
+  // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
+  const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
+  // inside a 32-token block the column is rotated by 2 * (s + 4h): the 16 lanes that store together -- four runs
+  // of four tokens, or eight of two -- hit sixteen different bank groups
+  const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + 2 * c0) & 31);
+  const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + 2 * c1) & 31);
+  uint32_t rd_col[4];
+#pragma unroll
+  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 2 * sidx + 8 * h) & 31;
+#pragma unroll
+  for (int gi = 0; gi < 2; ++gi) {
+    *reinterpret_cast<u32x4_t*>(s_x + gi * kXGroup + st_slot0) = x0[gi][0];
+    if (NTA > 1) *reinterpret_cast<u32x4_t*>(s_x + gi * kXGroup + st_slot1) = x0[gi][1];
+  }
+
+  // Weight codes run four K groups ahead in a ring of registers (the expert's bytes come
+  // from HBM); x rows come from L2 in pairs of groups, one pair in registers behind
+  // the pair in the LDS stage that is not being read.
+
+  Codes now[NPROJ];
+  for (uint32_t g0 = 0; g0 < ng; g0 += 4) {
+#pragma unroll
+    for (int uu = 0; uu < 2; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
+      const uint32_t gu = g0 + 2 * uu;
+      if (!NG8 && gu >= ng) break;
+      __syncthreads();  // stage uu is complete, stage uu ^ 1 is no longer read
+      // ---- the next pair into the other stage, fetch the pair after it into the freed registers.
+      // With whole steps of 8 groups the body has no branch (past the end the last pair is fetched
+      // again and the write goes to the stage nobody reads any more): every pass issues the same
+      // loads in the same order, so a wait for the codes of this pass never covers the x rows
+      // requested a moment before it.
+      if (NG8 || gu + 2 < ng) {
+        uint4* wbuf = s_x + (uu ^ 1) * 2 * kXGroup;
+#pragma unroll
+        for (int gi = 0; gi < 2; ++gi) {
+          *reinterpret_cast<u32x4_t*>(wbuf + gi * kXGroup + st_slot0) = xs[gi][0];
+          if (NTA > 1) *reinterpret_cast<u32x4_t*>(wbuf + gi * kXGroup + st_slot1) = xs[gi][1];
+        }
+        if (NG8 || gu + 4 < ng) {
+          const uint32_t gx = NG8 ? min(gu + 4, ng - 2) : gu + 4;
+#pragma unroll
+          for (int gi = 0; gi < 2; ++gi) {
+            const uint32_t gy = NG8 ? gx + gi : min(gx + gi, ng - 1);
+            xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup);
+            if (NTA > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + st_2nd);
+          }
+        }
+      }
+#pragma unroll
+      for (int gi = 0; gi < 2; ++gi) {
+        const uint32_t g = gu + gi;
+        if (!NG8 && g >= ng) break;  // the half pair at the end of an odd number of groups
+        // ---- matrix core: tmp[token, row] = sum over the group of x * q, times the powers of two kScaleMul takes back
+        const uint4* buf = s_x + (2 * uu + gi) * kXGroup;
+        uint4 bx[2][4];
+#pragma unroll
+        for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) bx[nt][s] = buf[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) {
+          float sc;
+          if constexpr (TAB16) sc = bf16_to_f(s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m]);
+          else sc = s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m];
+          f32x16_t tmp[2];
+#pragma unroll
+          for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
+          if (gi == 0) {
+            if constexpr (BITS == 2) {  // (all four registers of the pair are one load: it leaves at once, from a copy)
+              now[p] = cur[p][uu];
+              cur[p][uu].load(1, wrow[p] + pair_at(gu + 4), second);
+              now[p].settle();
+            } else cur[p][uu].settle();
+          }
+          if constexpr (BITS == 2) group_products<BITS, NTA>(now[p], gi, bx, tmp, [](int) {});
+          else group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
+          // the registers that held this group's codes take their part of the pair two ahead
+          // (past the end the last pair is read again: no branch inside the unrolled body)
+          if constexpr (BITS != 2) cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
+#pragma unroll
+          for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+            for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
+          if constexpr (NT == 1) __builtin_amdgcn_sched_barrier(0);  // one unit at a time: the registers of three waves
+        }
+      }
+    }
+  }
+  // (results that do not exist: not kept through the loop)
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+    for (int r = RES; r < 16; ++r) acc[p][0][r] = 0.0f;
+  };  // tile_body
+  // (the one-projection form keeps to its budget of 168 registers, three waves per SIMD, with one body only)
+  using two = std::integral_constant<int, 2>;
+  using one = std::integral_constant<int, 1>;
+  if constexpr (NT > 1) {
+    if (NPROJ == 1 || count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
+    else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
+    else tile_body(one{}, std::integral_constant<int, 4>{});
+  } else {
+    if (count > 16) tile_body(one{}, std::integral_constant<int, 16>{});
+    else if (count > 8) tile_body(one{}, std::integral_constant<int, 8>{});
+    else tile_body(one{}, std::integral_constant<int, 4>{});
+  }
+
+  qmm_trace(a, work, 3);
+  // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
+  const uint32_t row_raw = (slice * kQmmWaves + wv) * wave_rows;  // past a.rows: this wave has no rows of its own
+  if (a.epi == 0) {
+    // SwiGLU, narrowed to bf16 (at the scale of the matmul's rows, kRowScale), transposed through the (now free) x ring so that a lane stores
+    // 16 bytes of one token: [token][32 rows] per wave, the rows of a run of 8 in the
+    // (0,4,1,5,2,6,3,7) order phase 2 reads, i.e. rows r and r + 4 share a 32-bit word.
+    __syncthreads();  // every wave is past its last read of the ring
+    uint32_t* so = reinterpret_cast<uint32_t*>(s_x) + wv * (TT * 16);
+    const bool upper = (m >> 2) & 1u;
+    const uint32_t dw = ((m & ~7u) >> 1) + (m & 3u);  // word of the row pair (r, r + 4)
+    // The activation's variants are chosen outside the element loops (one uniform branch: Maple's or the
+    // ordinary one) and, for the ordinary one, by selects -- narrowed or not, clamped or not -- so that the
+    // 64 exponentials and reciprocals of a lane are one block of code the compiler can interleave (with
+    // the three tests inside the loops every element was a block of its own).
+    const bool clamp = a.limit > 0.0f, narrow = a.narrow != 0;
+    auto swiglu_block = [&](auto maple_tag) __attribute__((always_inline)) {
+      constexpr bool kMaple = decltype(maple_tag)::value;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        if (nt == 1 && count <= 32) break;  // no route in the second block: its slots are empty
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (j == 1 && count <= 8) break;
+          if (NT == 1 && j == 2 && count <= 16) break;
+          uint32_t bits[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float gv = acc[0][nt][4 * j + i], uv = acc[NPROJ - 1][nt][4 * j + i];
+            if constexpr (kMaple) {  // maple_moe.metal:153-164
+              bits[i] = f_to_bf16(maple_swiglu(gv, uv) * kRowScale);
+            } else {
+              const float gr = round_bf16(gv), ur = round_bf16(uv);
+              const float g0 = narrow ? gr : gv, u0 = narrow ? ur : uv;
+              gv = clamp ? fminf(g0, a.limit) : g0;  // (selects, so that a NaN stays one without a clamp)
+              uv = clamp ? fminf(fmaxf(u0, -a.limit), a.limit) : u0;
+              bits[i] = f_to_bf16(fast_silu(gv) * uv * kRowScale);
+            }
+          }
+          // lanes m and m ^ 4 trade halves: the lower lane ends with tokens i = 0, 1 of both rows,
+          // the upper lane with tokens i = 2, 3
+          const uint32_t t01 = bits[0] | (bits[1] << 16), t23 = bits[2] | (bits[3] << 16);
+          const uint32_t keep = upper ? t23 : t01;
+          const uint32_t got = static_cast<uint32_t>(
+              __builtin_amdgcn_ds_swizzle(static_cast<int>(upper ? t01 : t23), 0x101F));  // lane ^ 4
+          const uint32_t lo_row = upper ? got : keep, hi_row = upper ? keep : got;
+          const uint32_t tok = nt * 32 + 8 * j + 4 * h + (upper ? 2u : 0u);
+          so[tok * 16 + dw] = __builtin_amdgcn_perm(hi_row, lo_row, 0x05040100u);
+          so[(tok + 1) * 16 + dw] = __builtin_amdgcn_perm(hi_row, lo_row, 0x07060302u);
+        }
+      }
+    };
+    if (a.maple) swiglu_block(std::true_type{});
+    else swiglu_block(std::false_type{});
+    __syncthreads();
+    // the sums of the slice's two groups: two waves' rows each, four threads a (token, group), 16 values of every thread
+    {
+      const uint32_t ng_out = a.rows / kGroup, part = threadIdx.x & 3u;
+#pragma unroll
+      for (int it = 0; it < TT / 32; ++it) {
+        if (it == 1 && count <= 32) break;
+        const uint32_t task = it * 64 + (threadIdx.x >> 2), tok = task >> 1, gi = task & 1u, g = slice * 2 + gi;
+        const uint32_t* half = reinterpret_cast<const uint32_t*>(s_x) + (2 * gi + (part >> 1)) * (TT * 16) + tok * 16 + (part & 1u) * 8;
+        const uint4 v0 = *reinterpret_cast<const uint4*>(half), v1 = *reinterpret_cast<const uint4*>(half + 4);
+        float sum = (((bf16_lo(v0.x) + bf16_hi(v0.x)) + (bf16_lo(v0.y) + bf16_hi(v0.y))) +
+                     ((bf16_lo(v0.z) + bf16_hi(v0.z)) + (bf16_lo(v0.w) + bf16_hi(v0.w)))) +
+                    (((bf16_lo(v1.x) + bf16_hi(v1.x)) + (bf16_lo(v1.y) + bf16_hi(v1.y))) +
+                     ((bf16_lo(v1.z) + bf16_hi(v1.z)) + (bf16_lo(v1.w) + bf16_hi(v1.w))));
+        sum = group_sum(sum, 4);
+        const uint32_t sl = s_slot[tok];
+        if (part == 0 && sl != 0xFFFFFFFFu && g < ng_out)
+          store_group_sum(a.out_sums + sl * group_sum_words(ng_out), g, ng_out, sum * kRowUnscale);
+      }
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+    for (int it = 0; it < TT / 16; ++it) {
+      if (it == 2 && count <= 32) break;
+      const uint32_t c = it * 64 + lane, tok = c >> 2, part = c & 3u;
+      const uint32_t sl = s_slot[tok];
+      const uint4 v = reinterpret_cast<const uint4*>(so)[c];
+      if (sl != 0xFFFFFFFFu && (NG8 || row_raw < a.rows))
+        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out_base) + static_cast<size_t>(sl) * a.rows + row_base[0] +
+                                  part * 8) = v;
+    }
+  } else {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      if (nt == 1 && count <= 32) break;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j == 1 && count <= 8) break;
+        if (NT == 1 && j == 2 && count <= 16) break;
+        const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
+        const uint32_t slot[4] = {sl.x, sl.y, sl.z, sl.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (slot[i] == 0xFFFFFFFFu) continue;
+          const size_t at = static_cast<size_t>(slot[i]) * a.rows;
+#pragma unroll
+          for (int p = 0; p < NPROJ; ++p) {
+            if (p > 0 && !a.pair_rows && !out2_base) break;
+            if (!NG8 && row_raw + (a.pair_rows ? 32u * p : 0u) >= a.rows) break;
+            uint8_t* ob = (p > 0 && !a.pair_rows) ? out2_base : out_base;  // the second projection's own buffer
+            if (a.epi == 1) reinterpret_cast<float*>(ob)[at + row_base[p] + m] = acc[p][nt][4 * j + i];
+            else reinterpret_cast<uint16_t*>(ob)[at + row_base[p] + m] = f_to_bf16(acc[p][nt][4 * j + i]);
+          }
+        }
+      }
+    }
+  }
+  qmm_trace(a, work, 4);
+}
+
+// Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of
+// one tile share its x rows, the tiles of one expert share its weights) are laid on ONE XCD so
+// that its L2 serves the re-reads.  The tile list is laid out by group_scan_kernel so that every
+// eighth of it holds an eighth of the live tiles.
+__device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool& second) {
+  const uint32_t xcd_slot = blockIdx.x >> 3;
+  second = xcd_slot >= per_xcd[0];
+  return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
+}
+
+// (Both parts of a launch read their codes in the form SWAPPED names; without it 2-bit codes have to be tiled.  The dense
+// problem beside 2-bit experts is 4-bit and goes through qmm_mixed_kernel: the launchers refuse a 2-bit one beside a tiled pool.)
+template <int TT, int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
+void qmm_kernel(const QmmLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  qmm_item<TT, BITS, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
+}
+
+// 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
+// expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
+// tokens: 53 + 33 beside 388 + 207).
+template <int TT, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
+void qmm_mixed_kernel(const QmmLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  if (a.dense_mode) qmm_item<TT, 4, NPROJ, NG8, TAB16, true>(a, work, smem);
+  else qmm_item<TT, 2, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
+}
+
+// ---- the same product for a short contraction (K <= 512: the down projections) ----
+// With K this short the x tile of a workgroup (64 routes x K bf16 <= 64 KB) stays in LDS whole, so a
+// workgroup stages it once and then walks over `slices` consecutive 256-row slices of the weight matrix
+// without any further workgroup barrier: the waves run free, each wave's next-slice codes and scale / bias
+// words are requested while it still multiplies the current slice, and the stores of a finished slice
+// drain while the next one starts.  (qmm_kernel re-stages x through a two-stage ring for every 128 or 256
+// rows, four barriers per 8 groups, and pays its set-up -- tile, routes, tables, 3 us -- per slice.)
+// A wave owns two consecutive 32-row blocks (64 rows).  Routes past the tile's count repeat the tile's
+// last route in every respect, its output slot included: they store the same values to the same place,
+// and no store needs a branch.
+struct KresLaunch {
+  QmmArgs part[2];
+  uint32_t per_xcd[2];   // work items of each part on one XCD (grid = 8 * their sum)
+  uint32_t slices[2];    // 256-row slices one work item walks (divides rows / 256)
+};
+
+// the columns by which run c of 8 values is turned in the x tile
+template <int TT> __device__ __forceinline__ uint32_t kres_turn(uint32_t c) { return TT == 32 ? 2 * c : 4 * ((c & 3) >> 1) + 8 * (c >> 2); }
+
+template <int NG> __device__ __forceinline__ uint4 load_groups_bf16(const uint16_t* p) {  // NG bf16, zero-padded to 8
+  if constexpr (NG >= 8) {
+    return *reinterpret_cast<const uint4*>(p);
+  } else if constexpr (NG == 4) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    return make_uint4(v.x, v.y, 0, 0);
+  } else {
+    return make_uint4(*reinterpret_cast<const uint32_t*>(p), 0, 0, 0);
+  }
+}
+
+template <int TT, int BITS, int NG, bool SWAPPED>
+__device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, uint32_t n_walk, uint8_t* smem) {
+  static_assert(NG == 2 || NG == 4 || NG == 8, "K is 128, 256 or 512");
+  constexpr int NT = TT / 32;           // token blocks of a tile
+  constexpr uint32_t kXGroup = TT * 8;  // 16-byte pieces of one K group of the x tile
+  constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
+  using Codes = QmmCodes<BITS, SWAPPED>;
+  constexpr int kRing = NG < 4 || TT == 32 ? 1 : 2;  // pairs of groups in flight per row block
+  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const uint32_t m = lane & 31, h = lane >> 5;
+  const uint32_t items_per_tile = a.rows / (256u * n_walk);
+  uint32_t tile_id = work / items_per_tile, slice0 = (work % items_per_tile) * n_walk;
+  if (a.dense_mode) {
+    if (work >= a.dense_items) return;
+    tile_id = a.tile_major ? work / items_per_tile : work % a.dense_tiles;
+    slice0 = (a.tile_major ? work % items_per_tile : work / a.dense_tiles) * n_walk;
+    if (tile_id >= a.dense_tiles) return;
+  }
+  qmm_trace(a, work, 0);
+
+  uint32_t expert = 0, pair_start, count;
+  if (a.dense_mode) {
+    pair_start = tile_id * TT;
+    count = min(static_cast<uint32_t>(TT), a.dense_rows - pair_start);
+  } else {
+    // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
+    // fetched in a second round trip)
+    const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
+    const Tile t{tv.x, tv.y, tv.z, tv.w};
+    if (t.count == 0) return;
+    expert = t.expert;
+    pair_start = t.pair_start;
+    count = t.count;
+  }
+  uint4* s_x = reinterpret_cast<uint4*>(smem);                                  // [NG groups][kXGroup]
+  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + NG * kXGroup * 16);     // [TT]
+
+  const uint8_t* W;
+  const uint16_t* Sp;
+  const uint16_t* Bp;
+  if (a.dense_mode) {
+    W = static_cast<const uint8_t*>(a.dense[0].weights);
+    Sp = a.dense[0].scales;
+    Bp = a.dense[0].biases;
+  } else {
+    const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
+    W = blob + a.w_off[0];
+    Sp = reinterpret_cast<const uint16_t*>(blob + a.s_off[0]);
+    Bp = reinterpret_cast<const uint16_t*>(blob + a.b_off[0]);
+  }
+  constexpr uint32_t kRowBytes = NG * kGB;
+  // the lane's weight row of block p of slice w: row0 + 256 w + 32 p
+  const uint32_t row0 = (slice0 * kQmmWaves + wv) * 64 + m;
+  const uint32_t pair_stride = a.tiled ? 64u * kGB : 2u * kGB;
+  const size_t second = Codes::second(kRowBytes, a.tiled);
+  const uint8_t* wrow = W + static_cast<size_t>(row0 - m) * kRowBytes + Codes::lane_offset(lane, kRowBytes, a.tiled);
+  const uint16_t* srow = Sp + static_cast<size_t>(row0) * NG;
+  const uint16_t* brow = Bp + static_cast<size_t>(row0) * NG;
+
+  // ---- everything issued back to back: codes of the first slice, its scale / bias words, the x tile
+  Codes cur[2][kRing];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int u = 0; u < kRing; ++u)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride, second);
+  uint4 nS[2], nB[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    nS[p] = load_groups_bf16<NG>(srow + p * 32 * NG);
+    nB[p] = load_groups_bf16<NG>(brow + p * 32 * NG);
+  }
+  // staging: 256 / TT threads a route, kPieces neighbouring runs of 8 values of every group each
+  constexpr int kPieces = TT / 32, kPerRoute = 256 / TT;
+  const uint32_t st_i = threadIdx.x / kPerRoute, st_q = threadIdx.x % kPerRoute;
+  const uint16_t* st_src = a.x + static_cast<size_t>(pair_start + min(st_i, count - 1)) * a.x_stride + st_q * 8 * kPieces;
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t xv[kPieces * NG];
+#pragma unroll
+  for (int g = 0; g < kPieces * NG; ++g)
+    xv[g] = *reinterpret_cast<const u32x4_t*>(st_src + (g / kPieces) * kGroup + (g % kPieces) * 8);
+  uint4 b_term[NT][2];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const uint16_t* sp = a.sumx + static_cast<size_t>(pair_start + min(32 * nt + m, count - 1)) * group_sum_words(NG);
+    b_term[nt][0] = *reinterpret_cast<const uint4*>(sp + 8 * h);
+    b_term[nt][1] = *reinterpret_cast<const uint4*>(sp + 16);
+    if (h) b_term[nt][1] = make_uint4(0, 0, 0, 0);
+  }
+  uint32_t slot = 0;
+  if (threadIdx.x < TT) {
+    const uint32_t pi = pair_start + min(threadIdx.x, count - 1);
+    slot = pi;
+    if (!a.dense_mode && (a.epi == 1 || a.epi == 3)) {
+      const mf_pair pr = a.sorted[pi];
+      slot = pr.token * a.top_k + pr.rank;
+    }
+  }
+  qmm_trace(a, work, 1);
+
+  // ---- x tile into LDS (the layout qmm_kernel's ring uses for one group, NG times)
+  {
+    // (the 16 lanes that store together hold four runs of 8 of four routes each, or eight of two: the column is rotated so
+    // that they hit different bank groups)
+    const uint32_t st_nt = st_i >> 5, st_n = st_i & 31;
+    uint32_t st_slot[kPieces];
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+      const uint32_t c = kPieces * st_q + u;
+      st_slot[u] = ((st_nt * 4 + (c & 3)) * 2 + (c >> 2)) * 32 + ((st_n + kres_turn<TT>(c)) & 31);
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u) *reinterpret_cast<u32x4_t*>(s_x + g * kXGroup + st_slot[u]) = xv[kPieces * g + u];
+    if (threadIdx.x < TT) s_slot[threadIdx.x] = slot;
+  }
+  uint32_t rd_col[4];
+#pragma unroll
+  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + kres_turn<TT>(sidx + 4 * h)) & 31;
+  __syncthreads();  // the only workgroup barrier: from here on the waves run on their own
+  qmm_trace(a, work, 2);
+  // The sums of the lane's routes: K slots 8h..8h+7 of the bias product are groups 0..7 twice, the first parts for
+  // h = 0 and the second ones for h = 1, then the third for h = 0 -- two products instead of three.
+  // A tile of at most 32 routes fills only the first route block (NTA = 1): the second block, whose routes
+  // would all repeat the last route, is left out of the products, the scale multiplies and the stores.
+  // (RES = 4 for a tile of at most 8 routes: as in qmm_item)
+  auto tile_body = [&](auto nta_c, auto res_c) {
+  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
+  for (uint32_t w = 0; w < n_walk; ++w) {
+    const uint32_t step = w + 1 < n_walk ? 1u : 0u;  // the last slice requests itself again: no branch around loads
+    const uint8_t* wnext = wrow + static_cast<size_t>(step) * 256 * kRowBytes;
+    // scale words of this slice; bias operand: the biases, for both halves;
+    // ternary rows store no biases: theirs is -scale (the bias pointer is the scale table then)
+    uint4 Sv[2], bop[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      Sv[p] = nS[p];
+      const uint32_t flip = a.ternary ? 0x80008000u : 0u;
+      bop[p] = make_uint4(nB[p].x ^ flip, nB[p].y ^ flip, nB[p].z ^ flip, nB[p].w ^ flip);
+    }
+    f32x16_t acc[2][NT];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int nt = 0; nt < NTA; ++nt) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
+#pragma unroll
+        for (int term = 0; term < 2; ++term) acc[p][nt] = mfma_bf16(b_term[nt][term], bop[p], acc[p][nt]);
+      }
+    // the next slice's scale / bias words (the registers are free again)
+    srow += step * 256 * NG;
+    brow += step * 256 * NG;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      nS[p] = load_groups_bf16<NG>(srow + p * 32 * NG);
+      nB[p] = load_groups_bf16<NG>(brow + p * 32 * NG);
+    }
+    // x of a group comes out of LDS one group ahead, into the registers the matrix core has just read
+    uint4 bx[2][4];
+    if (w == 0) {
+#pragma unroll
+      for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) bx[nt][s] = s_x[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
+    }
+    Codes now[2];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const uint4* nbuf = s_x + ((g + 1) % NG) * kXGroup;  // after the last group: group 0 again, for the next slice
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const uint32_t sw[4] = {Sv[p].x, Sv[p].y, Sv[p].z, Sv[p].w};
+        const float sc = QmmCodes<BITS>::kScaleMul * ((g & 1) ? bf16_hi(sw[g >> 1]) : bf16_lo(sw[g >> 1]));
+        f32x16_t tmp[2];
+#pragma unroll
+        for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
+        constexpr int kPairs = NG / 2;
+        Codes& codes = cur[p][(g / 2) % kRing];
+        const int ahead = g / 2 + kRing;
+        const uint8_t* next_pair = ahead < kPairs ? wrow + p * 32 * kRowBytes + ahead * pair_stride
+                                                  : wnext + p * 32 * kRowBytes + (ahead - kPairs) * pair_stride;
+        if (g % 2 == 0) {
+          if constexpr (BITS == 2) {
+            now[p] = codes;
+            codes.load(1, next_pair, second);
+            now[p].settle();
+          } else codes.settle();
+        }
+        group_products<BITS, NTA>(BITS == 2 ? now[p] : codes, g % 2, bx, tmp, [&](int s) {
+          if (p == 1) {  // both row blocks have read x slot s of this group
+            bx[0][s] = nbuf[((0 * 4 + s) * 2 + h) * 32 + rd_col[s]];
+            if (NTA > 1) bx[1][s] = nbuf[((1 * 4 + s) * 2 + h) * 32 + rd_col[s]];
+          }
+        });
+        // the registers take the codes kRing pairs on: of this slice, or of the next one
+        if constexpr (BITS != 2) codes.load(g % 2, next_pair, second);
+#pragma unroll
+        for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+          for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
+        // the sums are wanted here, not after the last group: without this the compiler keeps every
+        // group's products and adds them up at the end of the slice, out of scratch memory
+        if constexpr (NTA > 1) asm volatile("" : "+v"(acc[p][0]), "+v"(acc[p][NT - 1]));
+        else asm volatile("" : "+v"(acc[p][0]));
+        __builtin_amdgcn_sched_barrier(0);  // one unit at a time: hoisted loads would cost more registers than exist
+      }
+    }
+    if (w + 1 == n_walk) qmm_trace(a, work, 3);
+    // ---- stores: the lane holds rows row + 32 p for routes 8j + 4h + i of each 32-route block
+    const uint32_t row = row0 + w * 256;
+    // byte offsets fit 32 bits (the launcher checks): one multiply-add per route, the base stays scalar
+    if (a.epi == 1) {
+      uint8_t* out = static_cast<uint8_t*>(a.out);
+      const uint32_t pitch = a.rows * 4, col = row * 4;
+#pragma unroll
+      for (int nt = 0; nt < NTA; ++nt) {
+#pragma unroll
+        for (int j = 0; j < RES / 4; ++j) {
+          const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
+          const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            float* o = reinterpret_cast<float*>(out + (sl4[i] * pitch + col));
+            o[0] = acc[0][nt][4 * j + i];
+            o[32] = acc[1][nt][4 * j + i];
+          }
+        }
+      }
+    } else {
+      uint8_t* out = static_cast<uint8_t*>(a.out);
+      const uint32_t pitch = a.rows * 2, col = row * 2;
+#pragma unroll
+      for (int nt = 0; nt < NTA; ++nt) {
+#pragma unroll
+        for (int j = 0; j < RES / 4; ++j) {
+          const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
+          const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            uint16_t* o = reinterpret_cast<uint16_t*>(out + (sl4[i] * pitch + col));
+            o[0] = f_to_bf16(acc[0][nt][4 * j + i]);
+            o[32] = f_to_bf16(acc[1][nt][4 * j + i]);
+          }
+        }
+      }
+    }
+    wrow = wnext;
+  }
+  };  // tile_body
+  using two = std::integral_constant<int, 2>;
+  using one = std::integral_constant<int, 1>;
+  if constexpr (NT > 1) {
+    if (count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
+    else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
+    else tile_body(one{}, std::integral_constant<int, 4>{});
+  } else {
+    if (count > 16) tile_body(one{}, std::integral_constant<int, 16>{});
+    else if (count > 8) tile_body(one{}, std::integral_constant<int, 8>{});
+    else tile_body(one{}, std::integral_constant<int, 4>{});
+  }
+  qmm_trace(a, work, 4);
+}
+
+template <int TT, int BITS, int NG, bool SWAPPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, 2), qmm_waves(TT, 2))))
+void qmm_kres_kernel(const KresLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  const uint32_t walk = launch.slices[second ? 1 : 0];
+  qmm_kres_item<TT, BITS, NG, SWAPPED>(a, work, walk, smem);
+}
+
+template <int TT, int NG, bool SWAPPED>  // as qmm_mixed_kernel
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, 2), qmm_waves(TT, 2))))
+void qmm_kres_mixed_kernel(const KresLaunch launch) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  bool second;
+  const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
+  const QmmArgs& a = launch.part[second ? 1 : 0];
+  if (a.dense_mode) qmm_kres_item<TT, 4, NG, true>(a, work, walk, smem);
+  else qmm_kres_item<TT, 2, NG, SWAPPED>(a, work, walk, smem);
+}
+
+// ------------------------------------------------------------------ launches
+
+inline size_t qmm_lds_bytes(uint32_t tile, uint32_t kdim, int nproj, bool tab16) {
+  const uint32_t ng = kdim / kGroup;
+  return qmm_x_bytes(tile) + ((static_cast<size_t>(nproj) * kQmmWaves * ng * 32 * (tab16 ? 2 : 4) + 15) & ~static_cast<size_t>(15)) +
+         tile * 4;
+}
+// the scale tables as bf16 where fp32 tables would leave a CU (160 KB of LDS) room for one workgroup only
+inline bool qmm_tab16(uint32_t tile, uint32_t kdim, int nproj) {
+  return static_cast<size_t>(qmm_waves(tile, nproj)) * qmm_lds_bytes(tile, kdim, nproj, false) > kMaxLds;
+}
+
+// Work items of a dense problem that one XCD gets: an eighth, but at least 4 while there are any -- a handful
+// of items (the shared expert beside the routed experts of a short batch) runs faster on few XCDs, whose L2
+// serves the x rows and weight rows they share, than spread one to an XCD (Qwen shape, 128 tokens: layer 81 us
+// against 89 us).
+inline uint32_t dense_per_xcd(uint32_t items) { return std::max((items + 7) / 8, std::min(items, 4u)); }
+// Whether an XCD should own tiles (and stream all weight rows) or row slices (and stream all of x): whichever
+// streams fewer bytes.  code_bits: 4 or 2.
+inline int dense_tile_major(uint32_t rows, uint32_t x_rows, int code_bits) {
+  return static_cast<uint64_t>(rows) * code_bits <= static_cast<uint64_t>(x_rows) * 16;
+}
+
+template <int TT>
+hipError_t launch_kres_tiles(hipStream_t s, int bits, const QmmArgs& a, uint32_t tile_slots, const QmmArgs* b,
+                             uint32_t b_tile_slots) {
+  KresLaunch launch{};
+  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
+  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
+  for (int part = 0; part < (b ? 2 : 1); ++part) {
+    QmmArgs& q = launch.part[part];
+    q = part ? *b : a;
+    const uint32_t slots = part ? b_tile_slots : tile_slots;
+    const uint32_t n_slices = q.rows / 256;
+    // two slices per work item halve the set-up per slice and still leave several rounds of work items
+    // (Qwen shape, 2048 tokens, whole layer: 331 us with one slice, 325 with two, 330 with four, 334 with eight)
+    const uint32_t walk = n_slices % 2 == 0 ? 2 : 1;
+    launch.slices[part] = walk;
+    if (q.dense_mode) {
+      q.dense_tiles = slots;
+      q.tile_major = dense_tile_major(q.rows, q.dense_rows, part_bits(bits, q));
+      q.dense_items = slots * (n_slices / walk);
+      launch.per_xcd[part] = dense_per_xcd(q.dense_items);
+    } else {
+      launch.per_xcd[part] = slots / 8 * (n_slices / walk);
+    }
+  }
+  const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
+  if (grid.x == 0) return hipSuccess;
+  const uint32_t ng = a.kdim / kGroup;
+  const size_t lds = static_cast<size_t>(ng) * TT * 128 + TT * 4;
+#define MF_KRES_L(...)                                                                                 \
+  do {                                                                                                 \
+    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
+    if (e != hipSuccess) return e;                                                                     \
+    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
+  } while (0)
+#define MF_KRES(N)                                                                                     \
+  do {                                                                                                 \
+    if (bits == kMixedBits && tiled) MF_KRES_L(qmm_kres_mixed_kernel<TT, N, false>);                       \
+    else if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<TT, N, true>);                            \
+    else if (bits == 4 && tiled) MF_KRES_L(qmm_kres_kernel<TT, 4, N, false>);                              \
+    else if (bits == 4) MF_KRES_L(qmm_kres_kernel<TT, 4, N, true>);                                        \
+    else if (tiled) MF_KRES_L(qmm_kres_kernel<TT, 2, N, false>);                                           \
+    else MF_KRES_L(qmm_kres_kernel<TT, 2, N, true>);                                                       \
+  } while (0)
+  if (ng == 8) MF_KRES(8); else if (ng == 4) MF_KRES(4); else MF_KRES(2);
+#undef MF_KRES_L
+#undef MF_KRES
+  return hipGetLastError();
+}
+
+template <int TT>
+hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj, uint32_t tile_slots, const QmmArgs* b,
+                            uint32_t b_tile_slots) {
+  QmmLaunch launch{};
+  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
+  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
+  size_t lds = 0;
+  bool ng8 = true, tab16 = false;
+  for (int part = 0; part < (b ? 2 : 1); ++part) {
+    QmmArgs& q = launch.part[part];
+    q = part ? *b : a;
+    const uint32_t slots = part ? b_tile_slots : tile_slots;
+    const uint32_t slice_rows = kQmmRows * (q.pair_rows ? nproj : 1), n_slices = (q.rows + slice_rows - 1) / slice_rows;
+    if (q.dense_mode) {
+      q.dense_tiles = slots;
+      q.tile_major = dense_tile_major(q.rows * (q.pair_rows ? 1 : nproj), q.dense_rows, part_bits(bits, q));
+      q.dense_items = slots * n_slices * std::max(1u, q.n_win);
+      launch.per_xcd[part] = dense_per_xcd(q.dense_items);
+    } else {
+      launch.per_xcd[part] = slots / 8 * n_slices;
+    }
+    q.tab_aligned = q.dense_mode
+        ? aligned16(q.dense[0].scales) && aligned16(q.dense[0].biases) && aligned16(q.dense[1].scales) &&
+              aligned16(q.dense[1].biases)
+        : aligned16(q.expert_base) && q.expert_stride % 16 == 0 &&
+              (q.s_off[0] | q.b_off[0] | q.s_off[1] | q.b_off[1]) % 16 == 0;
+    tab16 = tab16 || qmm_tab16(TT, q.kdim, nproj);  // with windows: kdim is the longest window
+    ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0 && q.rows % slice_rows == 0;
+  }
+  for (int part = 0; part < (b ? 2 : 1); ++part) lds = std::max(lds, qmm_lds_bytes(TT, launch.part[part].kdim, nproj, tab16));
+  const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
+  if (grid.x == 0) return hipSuccess;
+#define MF_QMM_L(...)                                                                                  \
+  do {                                                                                                 \
+    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
+    if (e != hipSuccess) return e;                                                                     \
+    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
+  } while (0)
+#define MF_QMM(P, G, T)                                                                                \
+  do {                                                                                                 \
+    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<TT, P, G, T, false>);                       \
+    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<TT, P, G, T, true>);                            \
+    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<TT, 4, P, G, T, false>);                              \
+    else if (bits == 4) MF_QMM_L(qmm_kernel<TT, 4, P, G, T, true>);                                        \
+    else if (tiled) MF_QMM_L(qmm_kernel<TT, 2, P, G, T, false>);                                           \
+    else MF_QMM_L(qmm_kernel<TT, 2, P, G, T, true>);                                                       \
+  } while (0)
+#define MF_QMM_G(P, G)                                         \
+  do {                                                         \
+    if (tab16) MF_QMM(P, G, true); else MF_QMM(P, G, false);   \
+  } while (0)
+  if (nproj == 2) { if (ng8) MF_QMM_G(2, true); else MF_QMM_G(2, false); }
+  else { if (ng8) MF_QMM_G(1, true); else MF_QMM_G(1, false); }
+#undef MF_QMM_G
+#undef MF_QMM
+#undef MF_QMM_L
+  return hipGetLastError();
+}
+
+
+
+}  // namespace mf

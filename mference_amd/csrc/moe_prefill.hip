@@ -25,21 +25,12 @@
 
 #include "mf_device.h"
 #include "mf_internal.h"
+#include "mf_qmm.h"
 #include "mf_router.h"
 
 #pragma clang fp contract(off)
 
 namespace mf {
-
-constexpr int kMaxLds = 160 * 1024;    // LDS of a CU
-constexpr uint32_t kTileTokens = 64;   // tokens of one expert a workgroup handles
-constexpr uint32_t kQmmWaves = 4;      // waves per workgroup, 32 weight rows each
-constexpr uint32_t kQmmRows = kQmmWaves * 32;
-constexpr uint32_t kQmmXBytes = 2 * 2 * 512 * 16;  // x tile ring: 2 stages of 2 K groups
-
-struct Tile {
-  uint32_t expert, pair_start, count, pad;
-};
 
 // ------------------------------------------------------------------ router
 
@@ -60,12 +51,12 @@ struct RouterTail {
   uint16_t* xp;          // null: none of this
   uint32_t router_cols;  // workgroup columns that compute logits; the columns behind them prepare x
   const uint16_t* w_sg;  // null: no scalar gate
-  float* sums;
+  uint16_t* sums;
   uint16_t* gate;
 };
 
 __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ x, uint16_t* __restrict__ xp,
-                                           float* __restrict__ sums, const uint16_t* __restrict__ w_sg,
+                                           uint16_t* __restrict__ sums, const uint16_t* __restrict__ w_sg,
                                            uint16_t* __restrict__ gate, uint32_t row, uint32_t d, uint32_t lane);
 
 template <int CPL, int R>
@@ -421,82 +412,91 @@ __global__ __launch_bounds__(256) void group_count_kernel(const uint32_t* __rest
 
 // From every expert's count (thread e holds c; threads past MF_MAX_EXPERTS only keep the barriers
 // company): counts, offsets (0xFFFFFFFF for an empty expert), the start of every expert's run and
-// the tile list of the matmul (runs of kTileTokens routes).
+// the tile lists of the matmuls.
 __device__ __forceinline__ void group_layout(uint32_t c, uint32_t E, uint32_t* __restrict__ counts,
                                              uint32_t* __restrict__ offsets, uint32_t* __restrict__ starts,
-                                             Tile* __restrict__ tiles, uint32_t tile_slots,
-                                             uint32_t* __restrict__ n_tiles, uint32_t* s_cnt, uint32_t* s_tile,
+                                             const TileLists& tiles, uint32_t* s_cnt,
                                              bool publish = true) {
   const uint32_t e = threadIdx.x;
   const bool act = e < MF_MAX_EXPERTS;
-  if (!publish) tiles = nullptr, n_tiles = nullptr;  // the scans only (s_cnt, s_tile): another workgroup writes
   if (publish && e < E) counts[e] = c;
-  // inclusive scans of the counts and of the tile counts over the MF_MAX_EXPERTS entries: inside a wave
-  // by shuffles, the eight wave totals through the last slots of the two arrays' neighbours
-  __shared__ uint32_t s_wave_cnt[MF_MAX_EXPERTS / 64], s_wave_tile[MF_MAX_EXPERTS / 64];
-  uint32_t run_c = act ? c : 0u, run_t = act ? (c + kTileTokens - 1) / kTileTokens : 0u;
+  // inclusive scans of the counts and of the two lists' tile counts over the MF_MAX_EXPERTS entries: inside a
+  // wave by shuffles, the eight wave totals through the last slots of the two arrays' neighbours
+  __shared__ uint32_t s_wave_cnt[MF_MAX_EXPERTS / 64], s_wave_tile[2][MF_MAX_EXPERTS / 64], s_total[2];
+  uint32_t run_c = act ? c : 0u, mine[2] = {}, run_t[2];
+#pragma unroll
+  for (int l = 0; l < 2; ++l) {
+    if (publish && act && tiles.list[l]) mine[l] = (c + tiles.tokens[l] - 1) / tiles.tokens[l];
+    run_t[l] = mine[l];
+  }
   const uint32_t lane = e & 63u;
   for (uint32_t o = 1; o < 64; o <<= 1) {
     const uint32_t a = static_cast<uint32_t>(__shfl_up(static_cast<int>(run_c), o, 64));
-    const uint32_t b = static_cast<uint32_t>(__shfl_up(static_cast<int>(run_t), o, 64));
+    const uint32_t b0 = static_cast<uint32_t>(__shfl_up(static_cast<int>(run_t[0]), o, 64));
+    const uint32_t b1 = static_cast<uint32_t>(__shfl_up(static_cast<int>(run_t[1]), o, 64));
     if (lane >= o) {
       run_c += a;
-      run_t += b;
+      run_t[0] += b0;
+      run_t[1] += b1;
     }
   }
   if (act && lane == 63) {
     s_wave_cnt[e >> 6] = run_c;
-    s_wave_tile[e >> 6] = run_t;
+    s_wave_tile[0][e >> 6] = run_t[0];
+    s_wave_tile[1][e >> 6] = run_t[1];
   }
   __syncthreads();
   if (act) {
     for (uint32_t v = 0; v < (e >> 6); ++v) {
       run_c += s_wave_cnt[v];
-      run_t += s_wave_tile[v];
+      run_t[0] += s_wave_tile[0][v];
+      run_t[1] += s_wave_tile[1][v];
     }
     s_cnt[e] = run_c;
-    s_tile[e] = run_t;
+  }
+  if (e == MF_MAX_EXPERTS - 1) {
+    s_total[0] = run_t[0];
+    s_total[1] = run_t[1];
+  }
+  // A list has `slots` entries (a multiple of 8).  The matmul sends the workgroups of
+  // slot range k * slots/8 .. to XCD k, so every eighth of the list gets an eighth of the
+  // live tiles, in expert order; the rest of each eighth stays empty (count 0).
+  if (publish) {
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+      if (tiles.list[l])
+        for (uint32_t i = e; i < tiles.slots[l]; i += blockDim.x) tiles.list[l][i] = Tile{0, 0, 0, 0};
   }
   __syncthreads();
-  // The tile list has tile_slots entries (a multiple of 8).  The matmul sends the workgroups of
-  // slot range k * tile_slots/8 .. to XCD k, so every eighth of the list gets an eighth of the
-  // live tiles, in expert order; the rest of each eighth stays empty (count 0).
-  if (tiles) {
-    for (uint32_t i = e; i < tile_slots; i += blockDim.x) tiles[i] = Tile{0, 0, 0, 0};
-    __syncthreads();
-  }
   if (publish && e < E) {
-    const uint32_t start = s_cnt[e] - c;
+    const uint32_t start = run_c - c;
     starts[e] = start;
     offsets[e] = c ? start : 0xFFFFFFFFu;
-    if (tiles) {
-      const uint32_t total = s_tile[MF_MAX_EXPERTS - 1], per_live = (total + 7) / 8, per_slot = tile_slots / 8;
-      const uint32_t nt = (c + kTileTokens - 1) / kTileTokens, t0 = s_tile[e] - nt;
-      for (uint32_t j = 0; j < nt; ++j) {
-        const uint32_t id = t0 + j;
-        tiles[(id / per_live) * per_slot + id % per_live] =
-            Tile{e, start + j * kTileTokens, min(kTileTokens, c - j * kTileTokens), 0};
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+      if (!tiles.list[l]) continue;
+      const uint32_t per_live = (s_total[l] + 7) / 8, per_slot = tiles.slots[l] / 8, tokens = tiles.tokens[l];
+      for (uint32_t j = 0; j < mine[l]; ++j) {
+        const uint32_t id = run_t[l] - mine[l] + j;
+        tiles.list[l][(id / per_live) * per_slot + id % per_live] = Tile{e, start + j * tokens, min(tokens, c - j * tokens), 0};
       }
     }
   }
-  if (n_tiles && e == MF_MAX_EXPERTS - 1) *n_tiles = s_tile[e];
 }
 
 // counts, offsets (0xFFFFFFFF for an empty expert), the start of every expert's
 // run, chunk_hist turned into each chunk's first position inside its expert's
-// run, and the tile list of the matmul (runs of kTileTokens routes).
+// run, and the tile lists of the matmuls.
 __global__ __launch_bounds__(512) void group_scan_kernel(uint32_t* __restrict__ chunk_hist,
                                                          uint32_t n_chunks, uint32_t E,
                                                          uint32_t* __restrict__ counts,
                                                          uint32_t* __restrict__ offsets,
                                                          uint32_t* __restrict__ starts,
-                                                         Tile* __restrict__ tiles,
-                                                         uint32_t tile_slots,
-                                                         uint32_t* __restrict__ n_tiles,
+                                                         const TileLists tiles,
                                                          const uint32_t* __restrict__ chunk_bad,
                                                          uint32_t* __restrict__ status,
                                                          int drop_if_bad = 0) {
-  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_tile[MF_MAX_EXPERTS];
+  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS];
   const uint32_t e = threadIdx.x;
   // status word: 2 when any chunk met an expert index out of range (n_chunks <= blockDim)
   const int any_bad = __syncthreads_or(e < n_chunks && chunk_bad[e] ? 1 : 0);
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(512) void group_scan_kernel(uint32_t* __restrict__ 
       c += v;
     }
   }
-  group_layout(c, E, counts, offsets, starts, tiles, tile_slots, n_tiles, s_cnt, s_tile);
+  group_layout(c, E, counts, offsets, starts, tiles, s_cnt);
 }
 
 __global__ __launch_bounds__(256) void group_emit_kernel(const uint32_t* __restrict__ idx,
@@ -586,9 +586,8 @@ __device__ __forceinline__ void group_serial(const uint32_t* __restrict__ idx, c
                                              uint32_t n_pairs, uint32_t K, uint32_t E,
                                              uint32_t* __restrict__ counts, uint32_t* __restrict__ offsets,
                                              uint32_t* __restrict__ starts, mf_pair* __restrict__ sorted,
-                                             Tile* __restrict__ tiles, uint32_t tile_slots,
-                                             uint32_t* __restrict__ n_tiles, uint32_t* s_hist_flat,
-                                             uint32_t* s_cnt, uint32_t* s_tile) {
+                                             const TileLists tiles, uint32_t* s_hist_flat,
+                                             uint32_t* s_cnt) {
   uint32_t (*s_hist)[MF_MAX_EXPERTS] = reinterpret_cast<uint32_t (*)[MF_MAX_EXPERTS]>(s_hist_flat);
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   __syncthreads();
@@ -610,7 +609,7 @@ __device__ __forceinline__ void group_serial(const uint32_t* __restrict__ idx, c
       c += n;
     }
   }
-  group_layout(c, E, counts, offsets, starts, tiles, tile_slots, n_tiles, s_cnt, s_tile);
+  group_layout(c, E, counts, offsets, starts, tiles, s_cnt);
   __syncthreads();
   // s_cnt holds the inclusive scan: an expert's run starts at s_cnt[e - 1]; the waves' bases are
   // relative to that start
@@ -671,11 +670,10 @@ __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restr
                                                          uint32_t* __restrict__ counts,
                                                          uint32_t* __restrict__ offsets,
                                                          uint32_t* __restrict__ starts,
-                                                         mf_pair* __restrict__ sorted, Tile* __restrict__ tiles,
-                                                         uint32_t tile_slots, uint32_t* __restrict__ n_tiles,
+                                                         mf_pair* __restrict__ sorted, const TileLists tiles,
                                                          uint32_t* __restrict__ status) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_tile[MF_MAX_EXPERTS];
+  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_row[MF_MAX_EXPERTS];
   const uint32_t T = n_pairs / K, W = group_one_row_words(T);
   uint32_t* bm = reinterpret_cast<uint32_t*>(smem);                 // [E][W] bits: token t of row e
   uint16_t* pref = reinterpret_cast<uint16_t*>(smem + static_cast<size_t>(E) * W * 4);  // [E][W] set bits before word
@@ -709,8 +707,8 @@ __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restr
   const int any_dup = __syncthreads_or(dup ? 1 : 0);
   if (threadIdx.x == 0) *status = any_bad ? 2u : 0u;
   if (any_dup) {
-    group_serial(idx, w, n_pairs, K, E, counts, offsets, starts, sorted, tiles, tile_slots, n_tiles,
-                 reinterpret_cast<uint32_t*>(smem), s_cnt, s_tile);
+    group_serial(idx, w, n_pairs, K, E, counts, offsets, starts, sorted, tiles,
+                 reinterpret_cast<uint32_t*>(smem), s_cnt);
     return;
   }
   // prefix counts of every row: 2^tpe_log2 threads per row, each a run of words
@@ -733,12 +731,12 @@ __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restr
       pref[row * W + j] = static_cast<uint16_t>(c);
       c += __popc(bm[row * W + j]);
     }
-    if (part == 0) s_tile[row] = row_total;  // parked for the layout step below
+    if (part == 0) s_row[row] = row_total;  // parked for the layout step below
   }
   __syncthreads();
-  const uint32_t c = threadIdx.x < E ? s_tile[threadIdx.x] : 0u;
+  const uint32_t c = threadIdx.x < E ? s_row[threadIdx.x] : 0u;
   __syncthreads();
-  group_layout(c, E, counts, offsets, starts, tiles, tile_slots, n_tiles, s_cnt, s_tile);
+  group_layout(c, E, counts, offsets, starts, tiles, s_cnt);
   __syncthreads();
 #pragma unroll
   for (uint32_t u = 0; u < kMine; ++u) {
@@ -822,10 +820,9 @@ __global__ __launch_bounds__(MF_MAX_EXPERTS) void group_place_kernel(const uint3
                                                                     uint32_t* __restrict__ offsets,
                                                                     uint32_t* __restrict__ starts,
                                                                     mf_pair* __restrict__ sorted,
-                                                                    Tile* __restrict__ tiles, uint32_t tile_slots,
-                                                                    uint32_t* __restrict__ n_tiles,
+                                                                    const TileLists tiles,
                                                                     uint32_t* __restrict__ status) {
-  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_tile[MF_MAX_EXPERTS], s_base[MF_MAX_EXPERTS];
+  __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_base[MF_MAX_EXPERTS];
   __shared__ unsigned long long s_mine[MF_MAX_EXPERTS];
   const uint32_t e = threadIdx.x, me = blockIdx.x;
   const bool first = me == 0;
@@ -860,7 +857,7 @@ __global__ __launch_bounds__(MF_MAX_EXPERTS) void group_place_kernel(const uint3
   }
   const int any_bad = __syncthreads_or(e < n_chunks && chunk_bad[e] ? 1 : 0);  // n_chunks <= blockDim
   if (first && e == 0) *status = any_bad ? 2u : 0u;
-  group_layout(c, E, counts, offsets, starts, tiles, tile_slots, n_tiles, s_cnt, s_tile, first);
+  group_layout(c, E, counts, offsets, starts, tiles, s_cnt, first);
   if (e < E) s_base[e] = s_cnt[e] - c + before;  // s_cnt is the inclusive scan of the counts
   __syncthreads();
   if (ex < E) {
@@ -925,30 +922,19 @@ hipError_t launch_tile_experts(hipStream_t s, const mf_moe_config& c, const void
 // Activation rows as the matmul wants them: inside every run of 8 K values the
 // order is (0,4,1,5,2,6,3,7) -- the pairing a packed code word expands to --, every value is times kRowScale,
 // and the fp32 sum of every 64-wide K group (of the values as they were) is kept beside them.  One lane per
-// run of 8; `dst` is null when `src` is already in that form.
-struct PrepArgs {  // up to two row sets per launch: the second starts at workgroup `blocks0`
-  const uint16_t* src[2];
-  uint16_t* dst[2];
-  float* sums[2];
-  uint32_t chunks[2];
-  uint32_t blocks0;
-};
-
-__global__ __launch_bounds__(256) void prep_rows_kernel(const PrepArgs a) {
-  const int part = blockIdx.x >= a.blocks0 ? 1 : 0;
-  const uint16_t* src = a.src[part];
-  uint16_t* dst = a.dst[part];
-  float* sums = a.sums[part];
-  const uint32_t chunks = a.chunks[part];
-  const uint32_t c = (blockIdx.x - (part ? a.blocks0 : 0u)) * blockDim.x + threadIdx.x;
+// run of 8.
+__global__ __launch_bounds__(256) void prep_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
+                                                        uint16_t* __restrict__ sums, uint32_t chunks, uint32_t ng) {
+  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
   uint4 v = make_uint4(0, 0, 0, 0);
   if (c < chunks) v = *reinterpret_cast<const uint4*>(src + static_cast<size_t>(c) * 8);
   float sum;
   const uint4 row = matmul_row8(v, &sum);
   sum = group_sum(sum, 8);
   if (c >= chunks) return;
-  if (dst) *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) = row;
-  if ((c & 7) == 0) sums[c >> 3] = dst ? sum : sum * kRowUnscale;
+  *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) = row;
+  const uint32_t g = c >> 3, r = g / ng;
+  if ((c & 7) == 0) store_group_sum(sums + r * group_sum_words(ng), g - r * ng, ng, sum);
 }
 
 // The same for the layer's input rows and, in the same pass, the scalar shared gate's logit
@@ -956,7 +942,7 @@ __global__ __launch_bounds__(256) void prep_rows_kernel(const PrepArgs a) {
 // order (dot_bf16_row: lane l takes the chunks l, l+64, ... of a row, neighbour-first butterfly), so
 // the gate has the bits of the stand-alone router-row launch it replaces.  One wave per row.
 __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint16_t* __restrict__ xp,
-                                           float* __restrict__ sums, const uint16_t* __restrict__ w_sg,
+                                           uint16_t* __restrict__ sums, const uint16_t* __restrict__ w_sg,
                                            uint16_t* __restrict__ gate, uint32_t row, uint32_t d, uint32_t lane) {
   const uint32_t chunks = d / 8;  // a multiple of 8: the 8 lanes of a K group are live together
   const size_t base = static_cast<size_t>(row) * chunks;
@@ -974,7 +960,7 @@ __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint
     sum = group_sum(sum, 8);
     if (live) {
       *reinterpret_cast<uint4*>(xp + (base + c) * 8) = prepared;
-      if ((c & 7) == 0) sums[(base + c) >> 3] = sum;
+      if ((c & 7) == 0) store_group_sum(sums + row * group_sum_words(chunks / 8), c >> 3, chunks / 8, sum);
       acc = __builtin_fmaf(bf16_lo(wv.x), bf16_lo(v.x), acc);
       acc = __builtin_fmaf(bf16_hi(wv.x), bf16_hi(v.x), acc);
       acc = __builtin_fmaf(bf16_lo(wv.y), bf16_lo(v.y), acc);
@@ -990,948 +976,12 @@ __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint
 }
 
 __global__ __launch_bounds__(256) void prep_x_gate_kernel(const uint16_t* __restrict__ x,
-                                                          uint16_t* __restrict__ xp, float* __restrict__ sums,
+                                                          uint16_t* __restrict__ xp, uint16_t* __restrict__ sums,
                                                           const uint16_t* __restrict__ w_sg,
                                                           uint16_t* __restrict__ gate, uint32_t t, uint32_t d) {
   const uint32_t lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= t) return;
   prep_x_row(x + static_cast<size_t>(row) * d, xp, sums, w_sg, gate, row, d, lane);
-}
-
-struct QmmArgs {
-  // weights: routed = blobs of the expert pool, dense = one projection set
-  const uint8_t* expert_base;
-  size_t expert_stride;
-  uint32_t w_off[2], s_off[2], b_off[2];
-  mf_qtensor dense[2];
-  int pair_rows;        // 1: the NPROJ blocks of a wave are consecutive 32-row blocks of projection 0
-  int tiled;            // 1: the routed experts' codes are in the matmul's own order (tile_codes_kernel), not row by row
-  int dense_mode;       // 1: the "expert" is dense[], tiles are runs of consecutive rows
-  uint32_t dense_rows;  // number of x rows in dense mode
-  // activations: rows of kdim bf16 in prep_rows_kernel order + their group sums [row, kdim/64]
-  const uint16_t* x;
-  const float* sumx;
-  uint32_t x_stride;
-  int gather;           // 1: x row = sorted[pair].token, 0: x row = pair index
-  const mf_pair* sorted;
-  const Tile* tiles;
-  const uint32_t* n_tiles;
-  uint32_t rows, kdim;  // weight rows (output width) and contraction length
-  // a launch may take a window of the contraction (long K is cut into windows whose fp32 results are
-  // added afterwards): rows of weights, tables and group sums are ng_ld groups apart (0: kdim / 64)
-  // and the window starts at group g_off (a multiple of 8)
-  uint32_t ng_ld, g_off;
-  // several windows in one launch (dense mode): window w covers the groups from
-  // dense_window_start(ng_ld, n_win, w) on and writes its fp32 result out_win_stride elements behind the
-  // previous window's
-  uint32_t n_win;
-  size_t out_win_stride;
-  // epilogue
-  int epi;              // 0 swiglu -> bf16 [pair, rows] in prep order; 1 fp32 [token*K+rank, rows]; 2 bf16 [pair, rows];
-                        // 3 bf16 [token*K+rank, rows]
-  int narrow;           // shared-expert rounding points (dequant_int4.metal:240-245)
-  int tab_aligned;      // scale / bias rows start on 16-byte boundaries (set by the launcher)
-  int ternary;          // 2-bit codes {0,1,2} with bias = -scale: b_off / dense[].biases name the SCALE table
-  int maple;            // MapleMoE's bf16-stepped activation in the SwiGLU epilogue
-  void* out;
-  void* out2;           // epi 1 / 2 with two projections that are not row blocks of one: where projection 1 goes (null: dropped)
-  uint32_t top_k;
-  float limit;
-  // dense mode: number of 64-row tiles and of work items; every XCD gets an eighth of the items however few
-  // tiles there are.  With few tiles (tile_major = 0: x is small, the weights are not) work item w is tile
-  // w % dense_tiles of row slice (w / dense_tiles) % slices: the items that read the same weight rows follow
-  // one another (same XCD, same moment).  With many tiles (tile_major = 1) the slices of one tile follow one
-  // another and an XCD's L2 holds the x rows of the few tiles it works on.  The window is w / (tiles * slices).
-  uint32_t dense_tiles, dense_items;
-  int tile_major;
-  // optional stage stamps: 8 per work item, 100 MHz clock
-  unsigned long long* trace;
-  uint32_t trace_items;
-};
-
-// first K group of window wdx when ng groups are cut into n_win windows (multiples of 8 groups)
-__host__ __device__ __forceinline__ uint32_t dense_window_start(uint32_t ng, uint32_t n_win, uint32_t wdx) {
-  if (wdx >= n_win) return ng;
-  return static_cast<uint32_t>(static_cast<uint64_t>(ng) * wdx / n_win) & ~7u;
-}
-
-__device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint32_t k) {
-  if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
-}
-
-// silu with the hardware exp2 / reciprocal (1 ulp each): the result is narrowed to bf16 right after
-__device__ __forceinline__ float fast_silu(float x) {
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
-}
-
-// One workgroup: 64 routes of one expert x 128 weight rows (4 waves x 32) x
-// NPROJ projections, the whole K.  The matrix core computes the TRANSPOSED
-// product: the A operand is the x tile (tokens are the rows), the B operand is
-// the expanded codes, so a lane ends up holding ONE weight row (its column
-// m = lane % 32) for 16 tokens of each 32-token block, and the per-group scale
-// is one scalar per lane.  With two row blocks per wave two waves per SIMD stay
-// resident (the register budget of 256 keeps the matrix-core results in ordinary
-// registers, where the scale multiply reads them directly); with one row block the
-// kernel fits 168 registers and three waves stay resident.
-// LDS (dynamic): x tile ring, 2 stages x 2 K groups x [2 nt][4 s][2 h][32 n] x 16 B,
-// scale tables [NPROJ][4 waves][ng][32 rows] fp32, out slots [64] u32.
-// One launch can carry two independent problems of the same instantiation (the routed experts
-// and the shared expert of the same phase): the second problem's work items follow the first's
-// on every XCD, so they fill the slots the first problem's last round leaves empty instead of
-// running as a launch of their own that covers a quarter of the chip.
-struct QmmLaunch {
-  QmmArgs part[2];
-  uint32_t per_xcd[2];  // work items of each part on one XCD (grid = 8 * their sum)
-};
-
-// NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
-// of groups and rows.
-template <int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
-__device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_t* smem) {
-  constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint32_t m = lane & 31, h = lane >> 5;
-  const uint32_t wave_rows = a.pair_rows ? 32u * NPROJ : 32u;  // weight rows of one wave
-  const uint32_t n_slices = NG8 ? a.rows / (kQmmWaves * wave_rows) : (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
-  uint32_t tile_id = work / n_slices, slice = work % n_slices, win = 0;
-  if (a.dense_mode) {
-    if (work >= a.dense_items) return;
-    const uint32_t inner = a.tile_major ? n_slices : a.dense_tiles, outer = a.tile_major ? a.dense_tiles : n_slices;
-    const uint32_t lo = work % inner, rest = work / inner, hi = rest % outer;
-    tile_id = a.tile_major ? hi : lo;
-    slice = a.tile_major ? lo : hi;
-    win = rest / outer;
-    if (tile_id >= a.dense_tiles) return;
-  }
-  uint32_t ng = a.kdim / kGroup, g_off = a.g_off;
-  uint8_t* out_base = static_cast<uint8_t*>(a.out);
-  uint8_t* out2_base = static_cast<uint8_t*>(a.out2);
-  if (a.n_win > 1) {  // this work item's window of the contraction
-    g_off = dense_window_start(a.ng_ld, a.n_win, win);
-    ng = dense_window_start(a.ng_ld, a.n_win, win + 1) - g_off;
-    out_base += win * a.out_win_stride * sizeof(float);
-    if (out2_base) out2_base += win * a.out_win_stride * sizeof(float);
-  }
-  qmm_trace(a, work, 0);
-
-  uint32_t expert = 0, pair_start, count;
-  if (a.dense_mode) {
-    pair_start = tile_id * kTileTokens;
-    count = min(kTileTokens, a.dense_rows - pair_start);
-  } else {
-    // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
-    // fetched in a second round trip)
-    const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
-    const Tile t{tv.x, tv.y, tv.z, tv.w};
-    if (t.count == 0) return;
-    expert = t.expert;
-    pair_start = t.pair_start;
-    count = t.count;
-  }
-
-  uint4* s_x = reinterpret_cast<uint4*>(smem);                      // 2 stages x 2 groups x 512 uint4
-  // The scale of every (row, group): fp32, or (TAB16, long contractions) a bf16 number -- a power of two times a bf16
-  // scale is one, so the upper half of the fp32 product is all of it.  That is half the LDS,
-  // which lets two workgroups share a CU up to 112 K groups (K = 7168), for one more instruction per read.
-  using tab_t = std::conditional_t<TAB16, uint16_t, float>;
-  tab_t* s_scale = reinterpret_cast<tab_t*>(smem + kQmmXBytes);  // [NPROJ][4][ng][32]
-  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + kQmmXBytes + ((NPROJ * kQmmWaves * ng * 32 * sizeof(tab_t) + 15) & ~15u));
-
-  // weight pointers of this workgroup's projections
-  const uint8_t* Wp[NPROJ];
-  const uint16_t* Sp[NPROJ];
-  const uint16_t* Bp[NPROJ];
-  uint32_t row_base[NPROJ];  // first weight row of each of this wave's 32-row blocks
-#pragma unroll
-  for (int p = 0; p < NPROJ; ++p) {
-    const int t = a.pair_rows ? 0 : p;
-    if (a.dense_mode) {
-      Wp[p] = static_cast<const uint8_t*>(a.dense[t].weights);
-      Sp[p] = a.dense[t].scales;
-      Bp[p] = a.dense[t].biases;
-    } else {
-      const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-      Wp[p] = blob + a.w_off[t];
-      Sp[p] = reinterpret_cast<const uint16_t*>(blob + a.s_off[t]);
-      Bp[p] = reinterpret_cast<const uint16_t*>(blob + a.b_off[t]);
-    }
-    // (a width that is no multiple of the workgroup's rows: the last slice's waves past the end compute the last
-    // 32 rows again and store nothing)
-    row_base[p] = (slice * kQmmWaves + wv) * wave_rows + (a.pair_rows ? 32u * p : 0u);
-    if (!NG8) row_base[p] = min(row_base[p], a.rows - 32u);
-  }
-  const uint32_t ng_ld = a.ng_ld ? a.ng_ld : ng;
-  const size_t row_bytes = static_cast<size_t>(ng_ld) * kGB;
-
-  // ---- everything the tile needs that depends only on the tile: issued back to back.
-  // Routes past `count` read the tile's last route instead (finite data, results discarded).
-  // staging: a thread takes two runs of 8 K values of one token in every group, or one of a tile of at most 32 routes
-  const bool few = NPROJ == 2 && count <= 32;
-  const uint32_t st_i = few ? threadIdx.x >> 3 : threadIdx.x >> 2;
-  const uint32_t st_c0 = few ? threadIdx.x & 7 : (threadIdx.x & 3) * 2, st_c1 = few ? st_c0 : st_c0 + 1;
-  const uint32_t st_pair = pair_start + min(st_i, count - 1);
-  const uint32_t ti_pair[2] = {pair_start + min(m, count - 1), pair_start + min(32 + m, count - 1)};
-  uint32_t st_row = st_pair, xrow[2] = {ti_pair[0], ti_pair[1]};
-  uint32_t slot = pair_start + min(threadIdx.x & 63u, count - 1);
-  // the routes' records are requested here and looked at behind the code loads below, which do not depend on
-  // them: the first codes are then on their way one memory round trip earlier
-  mf_pair pr{};
-  uint32_t tok_st = 0, tok_0 = 0, tok_1 = 0;
-  if (!a.dense_mode) {
-    pr = a.sorted[slot];
-    if (a.gather) {
-      tok_st = a.sorted[st_pair].token;
-      tok_0 = a.sorted[ti_pair[0]].token;
-      tok_1 = a.sorted[ti_pair[1]].token;
-    }
-  }
-  const uint8_t* wrow[NPROJ];
-  using Codes = QmmCodes<BITS, SWAPPED>;
-  const uint32_t gstride = a.tiled ? 32u * kGB : kGB;  // bytes from a group's codes to the next group's
-  const size_t second = Codes::second(row_bytes, a.tiled);
-  const uint32_t last_pair = (ng - 1) & ~1u;
-  // (the last pair of an odd number of groups is half a pair: the lanes that would ask for its second group ask for the first)
-  const uint32_t odd_back = !NG8 && (ng & 1u) ? Codes::lane_group(lane) * gstride : 0u;
-  auto pair_at = [&](uint32_t g) -> size_t {  // g: the pair's first group; past the end: the last pair again
-    const uint32_t gc = min(g, last_pair);
-    return static_cast<size_t>(gc) * gstride - (!NG8 && gc == last_pair ? odd_back : 0u);
-  };
-  Codes cur[NPROJ][2];
-#pragma unroll
-  for (int p = 0; p < NPROJ; ++p) {
-    wrow[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride +
-              Codes::lane_offset(lane, row_bytes, a.tiled);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow[p] + pair_at(2 * u), second);
-  }
-  __builtin_amdgcn_sched_barrier(0);  // (keeps the look at the routes behind the code loads)
-  if (!a.dense_mode) {
-    if (a.gather) {
-      st_row = tok_st;
-      xrow[0] = tok_0;
-      xrow[1] = tok_1;
-    }
-    if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
-  }
-  // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
-  const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_c0 * 8;
-  const uint32_t st_2nd = (st_c1 - st_c0) * 8;
-  // K groups travel in pairs; a contraction of an odd number of groups ends in half a pair (its other half is read
-  // from the last group again and not multiplied)
-  // (arrays of a native vector type: arrays of the uint4 struct were kept in scratch memory)
-  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-  u32x4_t xs[2][2];  // the pair after the one in LDS, on its way there
-  u32x4_t x0[2][2];
-#pragma unroll
-  for (int gi = 0; gi < 2; ++gi) {
-    const uint32_t ga = NG8 ? gi : min(static_cast<uint32_t>(gi), ng - 1), gb = NG8 ? 2u + gi : min(2u + gi, ng - 1);
-    x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup);
-    x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + st_2nd);
-    xs[gi][0] = xs[gi][1] = u32x4_t{0, 0, 0, 0};
-    if (NG8 || ng > 2) {
-      xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup);
-      xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + st_2nd);
-    }
-  }
-  // Scale and bias words of the lane's row and the group sums of its two routes, 8 K groups at a time
-  // (groups gl = g0 + 8h .. gl + 7 for g0 = 0, 16, ...); the loads of the first step leave now, with the
-  // codes and the x rows, the loads of every later step one step ahead of their use.
-  struct TabStep {
-    uint4 S[NPROJ], B[NPROJ];
-    float sx[2][8];
-  };
-  auto tab_fetch = [&](uint32_t g0) {
-    TabStep t;
-    const uint32_t gl = g0 + 8 * h;
-    const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
-    if (!NG8 && ng >= 8) {  // whole 16-byte loads at any group; in the last step they end at the row's end and are moved down
-      const uint32_t gb = min(gc, ng - 8), sh = gc - gb;
-      const bool last = g0 + 16 > ng;  // (uniform)
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gb;
-        t.B[p] = load_16_bytes(Bp[p] + at);
-        t.S[p] = load_16_bytes(Sp[p] + at);
-        if (last) {
-          t.B[p] = drop_bf16(t.B[p], sh);
-          t.S[p] = drop_bf16(t.S[p], sh);
-        }
-      }
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        const float* sp = a.sumx + static_cast<size_t>(xrow[nt]) * ng_ld + g_off + gb;
-        const uint4 s0 = load_16_bytes(sp), s1 = load_16_bytes(sp + 4);
-        const uint32_t w[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t.sx[nt][e] = __uint_as_float(w[e]);
-        if (last) {
-#pragma unroll
-          for (int bit = 4; bit >= 1; bit /= 2)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) t.sx[nt][e] = (sh & bit) ? (e + bit < 8 ? t.sx[nt][(e + bit) & 7] : 0.0f) : t.sx[nt][e];
-        }
-      }
-      return t;
-    }
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p) {
-      const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gc;
-      t.B[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Bp[p] + at) : load_x8<false>(Bp[p] + at))
-                   : load_bf16x8_guarded(Bp[p] + at, ng - gc);
-      t.S[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Sp[p] + at) : load_x8<false>(Sp[p] + at))
-                   : load_bf16x8_guarded(Sp[p] + at, ng - gc);
-    }
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const float* sp = a.sumx + static_cast<size_t>(xrow[nt]) * ng_ld + g_off + gc;
-      if (NG8) {
-        const float4 s0 = *reinterpret_cast<const float4*>(sp), s1 = *reinterpret_cast<const float4*>(sp + 4);
-        t.sx[nt][0] = s0.x; t.sx[nt][1] = s0.y; t.sx[nt][2] = s0.z; t.sx[nt][3] = s0.w;
-        t.sx[nt][4] = s1.x; t.sx[nt][5] = s1.y; t.sx[nt][6] = s1.z; t.sx[nt][7] = s1.w;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t.sx[nt][e] = gc + e < ng ? sp[e] : 0.0f;
-      }
-    }
-    return t;
-  };
-  TabStep tab_cur = tab_fetch(0);
-  qmm_trace(a, work, 1);
-
-  if (threadIdx.x < kTileTokens) s_slot[threadIdx.x] = threadIdx.x < count ? slot : 0xFFFFFFFFu;
-
-  f32x16_t acc[NPROJ][2];
-#pragma unroll
-  for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
-
-  // ---- per step: the scales of the wave's rows, times the powers of two that codes and rows carry, into the
-  // [g][row] table, and the bias term: acc[token, row] += sumx[token, g] * B[row, g].
-  // sumx enters as three bf16 terms, which hold all 24 bits.
-  // A tile of at most 32 routes fills only the first token block: the second block's matrix
-  // instructions and scale multiplies are left out (NTA = 1); its accumulators stay zero and its
-  // output slots are empty.  Of a tile of at most 8 routes (most tiles of a short prompt) a lane's first four results are all
-  // there is: only those are scaled (RES), 4 of 16 multiply-adds per group and row block.
-  auto tile_body = [&](auto nta_c, auto res_c) {
-  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
-  for (uint32_t g0 = 0; g0 < ng; g0 += 16) {
-    const TabStep t = tab_cur;
-    tab_cur = tab_fetch(g0 + 16 < ng ? g0 + 16 : g0);  // past the end: the same step again, unused
-    const uint32_t gl = g0 + 8 * h;
-    const bool have = gl < ng;
-    uint4 ab[NPROJ];
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p) {
-      tab_t* tab = s_scale + (p * kQmmWaves + wv) * ng * 32;
-      auto entry = [](float v) -> tab_t {
-        if constexpr (TAB16) return static_cast<uint16_t>(__float_as_uint(v) >> 16);
-        else return v;
-      };
-      const uint32_t pr[4] = {t.S[p].x, t.S[p].y, t.S[p].z, t.S[p].w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (have && (NG8 || gl + 2 * i < ng)) tab[(gl + 2 * i) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_lo(pr[i]));
-        if (have && (NG8 || gl + 2 * i + 1 < ng)) tab[(gl + 2 * i + 1) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_hi(pr[i]));
-      }
-      // ternary rows store no biases: the bias is -scale (the table pointer is the scale table then)
-      ab[p] = a.ternary ? make_uint4(t.B[p].x ^ 0x80008000u, t.B[p].y ^ 0x80008000u, t.B[p].z ^ 0x80008000u,
-                                     t.B[p].w ^ 0x80008000u)
-                        : t.B[p];
-      if (!have) ab[p] = make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int nt = 0; nt < NTA; ++nt) {
-      uint32_t hi[8], mid[8], lo[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float v = t.sx[nt][e];
-        hi[e] = __float_as_uint(v) & 0xFFFF0000u;
-        const float r1 = v - __uint_as_float(hi[e]);
-        mid[e] = __float_as_uint(r1) & 0xFFFF0000u;
-        lo[e] = __float_as_uint(r1 - __uint_as_float(mid[e]));
-      }
-      const uint4 b_hi = make_uint4((hi[0] >> 16) | hi[1], (hi[2] >> 16) | hi[3], (hi[4] >> 16) | hi[5],
-                                    (hi[6] >> 16) | hi[7]);
-      const uint4 b_mid = make_uint4((mid[0] >> 16) | mid[1], (mid[2] >> 16) | mid[3], (mid[4] >> 16) | mid[5],
-                                     (mid[6] >> 16) | mid[7]);
-      const uint4 b_lo = make_uint4(__builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u),
-                                    __builtin_amdgcn_perm(lo[3], lo[2], 0x07060302u),
-                                    __builtin_amdgcn_perm(lo[5], lo[4], 0x07060302u),
-                                    __builtin_amdgcn_perm(lo[7], lo[6], 0x07060302u));
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        acc[p][nt] = mfma_bf16(b_hi, ab[p], acc[p][nt]);
-        acc[p][nt] = mfma_bf16(b_mid, ab[p], acc[p][nt]);
-        acc[p][nt] = mfma_bf16(b_lo, ab[p], acc[p][nt]);
-      }
-    }
-  }
-  qmm_trace(a, work, 2);
-
-  // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
-  const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
-  // inside a 32-token block the column is rotated by 2 * (s + 4h): the 16 lanes that store together -- four runs
-  // of four tokens, or eight of two -- hit sixteen different bank groups
-  const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + 2 * c0) & 31);
-  const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + 2 * c1) & 31);
-  uint32_t rd_col[4];
-#pragma unroll
-  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 2 * sidx + 8 * h) & 31;
-#pragma unroll
-  for (int gi = 0; gi < 2; ++gi) {
-    *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot0) = x0[gi][0];
-    if (NTA > 1) *reinterpret_cast<u32x4_t*>(s_x + gi * 512 + st_slot1) = x0[gi][1];
-  }
-
-  // Weight codes run four K groups ahead in a ring of registers (the expert's bytes come
-  // from HBM); x rows come from L2 in pairs of groups, one pair in registers behind
-  // the pair in the LDS stage that is not being read.
-
-  Codes now[NPROJ];
-  for (uint32_t g0 = 0; g0 < ng; g0 += 4) {
-#pragma unroll
-    for (int uu = 0; uu < 2; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
-      const uint32_t gu = g0 + 2 * uu;
-      if (!NG8 && gu >= ng) break;
-      __syncthreads();  // stage uu is complete, stage uu ^ 1 is no longer read
-      // ---- the next pair into the other stage, fetch the pair after it into the freed registers.
-      // With whole steps of 8 groups the body has no branch (past the end the last pair is fetched
-      // again and the write goes to the stage nobody reads any more): every pass issues the same
-      // loads in the same order, so a wait for the codes of this pass never covers the x rows
-      // requested a moment before it.
-      if (NG8 || gu + 2 < ng) {
-        uint4* wbuf = s_x + (uu ^ 1) * 1024;
-#pragma unroll
-        for (int gi = 0; gi < 2; ++gi) {
-          *reinterpret_cast<u32x4_t*>(wbuf + gi * 512 + st_slot0) = xs[gi][0];
-          if (NTA > 1) *reinterpret_cast<u32x4_t*>(wbuf + gi * 512 + st_slot1) = xs[gi][1];
-        }
-        if (NG8 || gu + 4 < ng) {
-          const uint32_t gx = NG8 ? min(gu + 4, ng - 2) : gu + 4;
-#pragma unroll
-          for (int gi = 0; gi < 2; ++gi) {
-            const uint32_t gy = NG8 ? gx + gi : min(gx + gi, ng - 1);
-            xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup);
-            if (NTA > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + st_2nd);
-          }
-        }
-      }
-#pragma unroll
-      for (int gi = 0; gi < 2; ++gi) {
-        const uint32_t g = gu + gi;
-        if (!NG8 && g >= ng) break;  // the half pair at the end of an odd number of groups
-        // ---- matrix core: tmp[token, row] = sum over the group of x * q, times the powers of two kScaleMul takes back
-        const uint4* buf = s_x + uu * 1024 + gi * 512;
-        uint4 bx[2][4];
-#pragma unroll
-        for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-          for (int s = 0; s < 4; ++s) bx[nt][s] = buf[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
-#pragma unroll
-        for (int p = 0; p < NPROJ; ++p) {
-          float sc;
-          if constexpr (TAB16) sc = bf16_to_f(s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m]);
-          else sc = s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m];
-          f32x16_t tmp[2];
-#pragma unroll
-          for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-          if (gi == 0) {
-            if constexpr (BITS == 2) {  // (all four registers of the pair are one load: it leaves at once, from a copy)
-              now[p] = cur[p][uu];
-              cur[p][uu].load(1, wrow[p] + pair_at(gu + 4), second);
-              now[p].settle();
-            } else cur[p][uu].settle();
-          }
-          if constexpr (BITS == 2) group_products<BITS, NTA>(now[p], gi, bx, tmp, [](int) {});
-          else group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
-          // the registers that held this group's codes take their part of the pair two ahead
-          // (past the end the last pair is read again: no branch inside the unrolled body)
-          if constexpr (BITS != 2) cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
-#pragma unroll
-          for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-            for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
-        }
-      }
-    }
-  }
-  };  // tile_body
-  // (the one-projection form keeps to its budget of 168 registers, three waves per SIMD, with one body only)
-  using two = std::integral_constant<int, 2>;
-  using one = std::integral_constant<int, 1>;
-  if (NPROJ == 1 || count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
-  else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
-  else tile_body(one{}, std::integral_constant<int, 4>{});
-
-  qmm_trace(a, work, 3);
-  // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
-  const uint32_t row_raw = (slice * kQmmWaves + wv) * wave_rows;  // past a.rows: this wave has no rows of its own
-  if (a.epi == 0) {
-    // SwiGLU, narrowed to bf16 (at the scale of the matmul's rows, kRowScale), transposed through the (now free) x ring so that a lane stores
-    // 16 bytes of one token: [token][32 rows] per wave, the rows of a run of 8 in the
-    // (0,4,1,5,2,6,3,7) order phase 2 reads, i.e. rows r and r + 4 share a 32-bit word.
-    __syncthreads();  // every wave is past its last read of the ring
-    uint32_t* so = reinterpret_cast<uint32_t*>(s_x) + wv * 1024;
-    const bool upper = (m >> 2) & 1u;
-    const uint32_t dw = ((m & ~7u) >> 1) + (m & 3u);  // word of the row pair (r, r + 4)
-    // The activation's variants are chosen outside the element loops (one uniform branch: Maple's or the
-    // ordinary one) and, for the ordinary one, by selects -- narrowed or not, clamped or not -- so that the
-    // 64 exponentials and reciprocals of a lane are one block of code the compiler can interleave (with
-    // the three tests inside the loops every element was a block of its own).
-    const bool clamp = a.limit > 0.0f, narrow = a.narrow != 0;
-    auto swiglu_block = [&](auto maple_tag) __attribute__((always_inline)) {
-      constexpr bool kMaple = decltype(maple_tag)::value;
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt) {
-        if (nt == 1 && count <= 32) break;  // no route in the second block: its slots are empty
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (j == 1 && count <= 8) break;
-          uint32_t bits[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float gv = acc[0][nt][4 * j + i], uv = acc[NPROJ - 1][nt][4 * j + i];
-            if constexpr (kMaple) {  // maple_moe.metal:153-164
-              bits[i] = f_to_bf16(maple_swiglu(gv, uv) * kRowScale);
-            } else {
-              const float gr = round_bf16(gv), ur = round_bf16(uv);
-              const float g0 = narrow ? gr : gv, u0 = narrow ? ur : uv;
-              gv = clamp ? fminf(g0, a.limit) : g0;  // (selects, so that a NaN stays one without a clamp)
-              uv = clamp ? fminf(fmaxf(u0, -a.limit), a.limit) : u0;
-              bits[i] = f_to_bf16(fast_silu(gv) * uv * kRowScale);
-            }
-          }
-          // lanes m and m ^ 4 trade halves: the lower lane ends with tokens i = 0, 1 of both rows,
-          // the upper lane with tokens i = 2, 3
-          const uint32_t t01 = bits[0] | (bits[1] << 16), t23 = bits[2] | (bits[3] << 16);
-          const uint32_t keep = upper ? t23 : t01;
-          const uint32_t got = static_cast<uint32_t>(
-              __builtin_amdgcn_ds_swizzle(static_cast<int>(upper ? t01 : t23), 0x101F));  // lane ^ 4
-          const uint32_t lo_row = upper ? got : keep, hi_row = upper ? keep : got;
-          const uint32_t tok = nt * 32 + 8 * j + 4 * h + (upper ? 2u : 0u);
-          so[tok * 16 + dw] = __builtin_amdgcn_perm(hi_row, lo_row, 0x05040100u);
-          so[(tok + 1) * 16 + dw] = __builtin_amdgcn_perm(hi_row, lo_row, 0x07060302u);
-        }
-      }
-    };
-    if (a.maple) swiglu_block(std::true_type{});
-    else swiglu_block(std::false_type{});
-    __builtin_amdgcn_wave_barrier();  // the wave reads back only what it wrote itself
-    const uint32_t lane = threadIdx.x & 63u;
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      if (it == 2 && count <= 32) break;
-      const uint32_t c = it * 64 + lane, tok = c >> 2, part = c & 3u;
-      const uint32_t sl = s_slot[tok];
-      const uint4 v = reinterpret_cast<const uint4*>(so)[c];
-      if (sl != 0xFFFFFFFFu && (NG8 || row_raw < a.rows))
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out_base) + static_cast<size_t>(sl) * a.rows + row_base[0] +
-                                  part * 8) = v;
-    }
-  } else {
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      if (nt == 1 && count <= 32) break;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j == 1 && count <= 8) break;
-        const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
-        const uint32_t slot[4] = {sl.x, sl.y, sl.z, sl.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (slot[i] == 0xFFFFFFFFu) continue;
-          const size_t at = static_cast<size_t>(slot[i]) * a.rows;
-#pragma unroll
-          for (int p = 0; p < NPROJ; ++p) {
-            if (p > 0 && !a.pair_rows && !out2_base) break;
-            if (!NG8 && row_raw + (a.pair_rows ? 32u * p : 0u) >= a.rows) break;
-            uint8_t* ob = (p > 0 && !a.pair_rows) ? out2_base : out_base;  // the second projection's own buffer
-            if (a.epi == 1) reinterpret_cast<float*>(ob)[at + row_base[p] + m] = acc[p][nt][4 * j + i];
-            else reinterpret_cast<uint16_t*>(ob)[at + row_base[p] + m] = f_to_bf16(acc[p][nt][4 * j + i]);
-          }
-        }
-      }
-    }
-  }
-  qmm_trace(a, work, 4);
-}
-
-// Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of
-// one tile share its x rows, the tiles of one expert share its weights) are laid on ONE XCD so
-// that its L2 serves the re-reads.  The tile list is laid out by group_scan_kernel so that every
-// eighth of it holds an eighth of the live tiles.
-__device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool& second) {
-  const uint32_t xcd_slot = blockIdx.x >> 3;
-  second = xcd_slot >= per_xcd[0];
-  return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
-}
-
-// (Both parts of a launch read their codes in the form SWAPPED names; without it 2-bit codes have to be tiled.  The dense
-// problem beside 2-bit experts is 4-bit and goes through qmm_mixed_kernel: the launchers refuse a 2-bit one beside a tiled pool.)
-template <int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
-void qmm_kernel(const QmmLaunch launch) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  qmm_item<BITS, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
-}
-
-// 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
-// expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
-// tokens: 53 + 33 beside 388 + 207).
-template <int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NPROJ == 1 ? 3 : 2, NPROJ == 1 ? 3 : 2)))
-void qmm_mixed_kernel(const QmmLaunch launch) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_item<4, NPROJ, NG8, TAB16, true>(a, work, smem);
-  else qmm_item<2, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
-}
-
-// ---- the same product for a short contraction (K <= 512: the down projections) ----
-// With K this short the x tile of a workgroup (64 routes x K bf16 <= 64 KB) stays in LDS whole, so a
-// workgroup stages it once and then walks over `slices` consecutive 256-row slices of the weight matrix
-// without any further workgroup barrier: the waves run free, each wave's next-slice codes and scale / bias
-// words are requested while it still multiplies the current slice, and the stores of a finished slice
-// drain while the next one starts.  (qmm_kernel re-stages x through a two-stage ring for every 128 or 256
-// rows, four barriers per 8 groups, and pays its set-up -- tile, routes, tables, 3 us -- per slice.)
-// A wave owns two consecutive 32-row blocks (64 rows).  Routes past the tile's count repeat the tile's
-// last route in every respect, its output slot included: they store the same values to the same place,
-// and no store needs a branch.
-struct KresLaunch {
-  QmmArgs part[2];
-  uint32_t per_xcd[2];   // work items of each part on one XCD (grid = 8 * their sum)
-  uint32_t slices[2];    // 256-row slices one work item walks (divides rows / 256)
-};
-
-template <int NG> __device__ __forceinline__ uint4 load_groups_bf16(const uint16_t* p) {  // NG bf16, zero-padded to 8
-  if constexpr (NG >= 8) {
-    return *reinterpret_cast<const uint4*>(p);
-  } else if constexpr (NG == 4) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    return make_uint4(v.x, v.y, 0, 0);
-  } else {
-    return make_uint4(*reinterpret_cast<const uint32_t*>(p), 0, 0, 0);
-  }
-}
-
-template <int BITS, int NG, bool SWAPPED>
-__device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, uint32_t n_walk, uint8_t* smem) {
-  static_assert(NG == 2 || NG == 4 || NG == 8, "K is 128, 256 or 512");
-  constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
-  using Codes = QmmCodes<BITS, SWAPPED>;
-  constexpr int kRing = NG < 4 ? 1 : 2;  // pairs of groups in flight per projection
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const uint32_t m = lane & 31, h = lane >> 5;
-  const uint32_t items_per_tile = a.rows / (256u * n_walk);
-  uint32_t tile_id = work / items_per_tile, slice0 = (work % items_per_tile) * n_walk;
-  if (a.dense_mode) {
-    if (work >= a.dense_items) return;
-    tile_id = a.tile_major ? work / items_per_tile : work % a.dense_tiles;
-    slice0 = (a.tile_major ? work % items_per_tile : work / a.dense_tiles) * n_walk;
-    if (tile_id >= a.dense_tiles) return;
-  }
-  qmm_trace(a, work, 0);
-
-  uint32_t expert = 0, pair_start, count;
-  if (a.dense_mode) {
-    pair_start = tile_id * kTileTokens;
-    count = min(kTileTokens, a.dense_rows - pair_start);
-  } else {
-    // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
-    // fetched in a second round trip)
-    const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
-    const Tile t{tv.x, tv.y, tv.z, tv.w};
-    if (t.count == 0) return;
-    expert = t.expert;
-    pair_start = t.pair_start;
-    count = t.count;
-  }
-  uint4* s_x = reinterpret_cast<uint4*>(smem);                       // [NG groups][512]
-  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + NG * 8192);  // [64]
-  float* s_sum = reinterpret_cast<float*>(smem + NG * 8192 + kTileTokens * 4);  // [64 routes][NG]
-
-  const uint8_t* W;
-  const uint16_t* Sp;
-  const uint16_t* Bp;
-  if (a.dense_mode) {
-    W = static_cast<const uint8_t*>(a.dense[0].weights);
-    Sp = a.dense[0].scales;
-    Bp = a.dense[0].biases;
-  } else {
-    const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-    W = blob + a.w_off[0];
-    Sp = reinterpret_cast<const uint16_t*>(blob + a.s_off[0]);
-    Bp = reinterpret_cast<const uint16_t*>(blob + a.b_off[0]);
-  }
-  constexpr uint32_t kRowBytes = NG * kGB;
-  // the lane's weight row of block p of slice w: row0 + 256 w + 32 p
-  const uint32_t row0 = (slice0 * kQmmWaves + wv) * 64 + m;
-  const uint32_t pair_stride = a.tiled ? 64u * kGB : 2u * kGB;
-  const size_t second = Codes::second(kRowBytes, a.tiled);
-  const uint8_t* wrow = W + static_cast<size_t>(row0 - m) * kRowBytes + Codes::lane_offset(lane, kRowBytes, a.tiled);
-  const uint16_t* srow = Sp + static_cast<size_t>(row0) * NG;
-  const uint16_t* brow = Bp + static_cast<size_t>(row0) * NG;
-
-  // ---- everything issued back to back: codes of the first slice, its scale / bias words, the x tile
-  Codes cur[2][kRing];
-#pragma unroll
-  for (int p = 0; p < 2; ++p)
-#pragma unroll
-    for (int u = 0; u < kRing; ++u)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride, second);
-  uint4 nS[2], nB[2];
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    nS[p] = load_groups_bf16<NG>(srow + p * 32 * NG);
-    nB[p] = load_groups_bf16<NG>(brow + p * 32 * NG);
-  }
-  const uint32_t st_i = threadIdx.x >> 2, st_q = threadIdx.x & 3;  // staging: route i, K values 16q..16q+15 of a group
-  const uint16_t* st_src = a.x + static_cast<size_t>(pair_start + min(st_i, count - 1)) * a.x_stride + st_q * 16;
-  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-  u32x4_t xv[2 * NG];
-#pragma unroll
-  for (int g = 0; g < 2 * NG; ++g) xv[g] = *reinterpret_cast<const u32x4_t*>(st_src + (g >> 1) * kGroup + (g & 1) * 8);
-  uint32_t slot = 0;
-  if (threadIdx.x < kTileTokens) {
-    const uint32_t pi = pair_start + min(threadIdx.x, count - 1);
-    slot = pi;
-    if (!a.dense_mode && (a.epi == 1 || a.epi == 3)) {
-      const mf_pair pr = a.sorted[pi];
-      slot = pr.token * a.top_k + pr.rank;
-    }
-  }
-  qmm_trace(a, work, 1);
-
-  // ---- x tile into LDS (the layout qmm_kernel's ring uses for one group, NG times)
-  {
-    const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = 2 * st_q, c1 = c0 + 1;
-    const uint32_t st_rot = 4 * ((c0 & 3) >> 1) + 8 * (c0 >> 2);
-    const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + st_rot) & 31);
-    const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + st_rot) & 31);
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      *reinterpret_cast<u32x4_t*>(s_x + g * 512 + st_slot0) = xv[2 * g];
-      *reinterpret_cast<u32x4_t*>(s_x + g * 512 + st_slot1) = xv[2 * g + 1];
-    }
-    if (threadIdx.x < kTileTokens) s_slot[threadIdx.x] = slot;
-    // the fp32 sum of every 64-wide group of every route, for the bias and offset terms: the four
-    // threads that stage a route each hold 16 of a group's values
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      float part = 0.0f;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const u32x4_t v = xv[2 * g + u];
-        part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
-                ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
-      }
-      part = group_sum(part, 4);
-      if (st_q == 0) s_sum[st_i * NG + g] = part * kRowUnscale;
-    }
-  }
-  uint32_t rd_col[4];
-#pragma unroll
-  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 4 * (sidx >> 1) + 8 * h) & 31;
-  __syncthreads();  // the only workgroup barrier: from here on the waves run on their own
-  qmm_trace(a, work, 2);
-  // sum(x) of a group as three bf16 terms (all 24 bits), see qmm_kernel.  Both halves of the wave hold
-  // the sums of groups 0..7 of the lane's two routes: K slots 8h..8h+7 of the bias product are those
-  // groups again, the first terms for h = 0 and the second ones for h = 1, then the third for h = 0 -- two products instead of three.
-  // A tile of at most 32 routes fills only the first route block (NTA = 1): the second block, whose routes
-  // would all repeat the last route, is left out of the products, the scale multiplies and the stores.
-  // (RES = 4 for a tile of at most 8 routes: as in qmm_item)
-  auto tile_body = [&](auto nta_c, auto res_c) {
-  constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
-  uint4 b_term[2][2];
-#pragma unroll
-  for (int nt = 0; nt < NTA; ++nt) {
-    float sx[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) sx[e] = e < NG ? s_sum[(nt * 32 + m) * NG + e] : 0.0f;
-    uint32_t hi[8], mid[8], lo[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float v = sx[e];
-      hi[e] = __float_as_uint(v) & 0xFFFF0000u;
-      const float r1 = v - __uint_as_float(hi[e]);
-      mid[e] = __float_as_uint(r1) & 0xFFFF0000u;
-      lo[e] = __float_as_uint(r1 - __uint_as_float(mid[e]));
-    }
-    uint32_t first[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) first[e] = h ? mid[e] : hi[e];
-    b_term[nt][0] = make_uint4((first[0] >> 16) | first[1], (first[2] >> 16) | first[3], (first[4] >> 16) | first[5],
-                               (first[6] >> 16) | first[7]);
-    b_term[nt][1] = make_uint4(__builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u), __builtin_amdgcn_perm(lo[3], lo[2], 0x07060302u),
-                               __builtin_amdgcn_perm(lo[5], lo[4], 0x07060302u), __builtin_amdgcn_perm(lo[7], lo[6], 0x07060302u));
-    if (h) b_term[nt][1] = make_uint4(0, 0, 0, 0);
-  }
-
-  for (uint32_t w = 0; w < n_walk; ++w) {
-    const uint32_t step = w + 1 < n_walk ? 1u : 0u;  // the last slice requests itself again: no branch around loads
-    const uint8_t* wnext = wrow + static_cast<size_t>(step) * 256 * kRowBytes;
-    // scale words of this slice; bias operand: the biases, for both halves;
-    // ternary rows store no biases: theirs is -scale (the bias pointer is the scale table then)
-    uint4 Sv[2], bop[2];
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      Sv[p] = nS[p];
-      const uint32_t flip = a.ternary ? 0x80008000u : 0u;
-      bop[p] = make_uint4(nB[p].x ^ flip, nB[p].y ^ flip, nB[p].z ^ flip, nB[p].w ^ flip);
-    }
-    f32x16_t acc[2][2];
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int nt = 0; nt < NTA; ++nt) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
-#pragma unroll
-        for (int term = 0; term < 2; ++term) acc[p][nt] = mfma_bf16(b_term[nt][term], bop[p], acc[p][nt]);
-      }
-    // the next slice's scale / bias words (the registers are free again)
-    srow += step * 256 * NG;
-    brow += step * 256 * NG;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      nS[p] = load_groups_bf16<NG>(srow + p * 32 * NG);
-      nB[p] = load_groups_bf16<NG>(brow + p * 32 * NG);
-    }
-    // x of a group comes out of LDS one group ahead, into the registers the matrix core has just read
-    uint4 bx[2][4];
-    if (w == 0) {
-#pragma unroll
-      for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) bx[nt][s] = s_x[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
-    }
-    Codes now[2];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      const uint4* nbuf = s_x + ((g + 1) % NG) * 512;  // after the last group: group 0 again, for the next slice
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const uint32_t sw[4] = {Sv[p].x, Sv[p].y, Sv[p].z, Sv[p].w};
-        const float sc = QmmCodes<BITS>::kScaleMul * ((g & 1) ? bf16_hi(sw[g >> 1]) : bf16_lo(sw[g >> 1]));
-        f32x16_t tmp[2];
-#pragma unroll
-        for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-        constexpr int kPairs = NG / 2;
-        Codes& codes = cur[p][(g / 2) % kRing];
-        const int ahead = g / 2 + kRing;
-        const uint8_t* next_pair = ahead < kPairs ? wrow + p * 32 * kRowBytes + ahead * pair_stride
-                                                  : wnext + p * 32 * kRowBytes + (ahead - kPairs) * pair_stride;
-        if (g % 2 == 0) {
-          if constexpr (BITS == 2) {
-            now[p] = codes;
-            codes.load(1, next_pair, second);
-            now[p].settle();
-          } else codes.settle();
-        }
-        group_products<BITS, NTA>(BITS == 2 ? now[p] : codes, g % 2, bx, tmp, [&](int s) {
-          if (p == 1) {  // both row blocks have read x slot s of this group
-            bx[0][s] = nbuf[((0 * 4 + s) * 2 + h) * 32 + rd_col[s]];
-            if (NTA > 1) bx[1][s] = nbuf[((1 * 4 + s) * 2 + h) * 32 + rd_col[s]];
-          }
-        });
-        // the registers take the codes kRing pairs on: of this slice, or of the next one
-        if constexpr (BITS != 2) codes.load(g % 2, next_pair, second);
-#pragma unroll
-        for (int nt = 0; nt < NTA; ++nt)
-#pragma unroll
-          for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
-        // the sums are wanted here, not after the last group: without this the compiler keeps every
-        // group's products and adds them up at the end of the slice, out of scratch memory
-        if constexpr (NTA > 1) asm volatile("" : "+v"(acc[p][0]), "+v"(acc[p][1]));
-        else asm volatile("" : "+v"(acc[p][0]));
-        __builtin_amdgcn_sched_barrier(0);  // one unit at a time: hoisted loads would cost more registers than exist
-      }
-    }
-    if (w + 1 == n_walk) qmm_trace(a, work, 3);
-    // ---- stores: the lane holds rows row + 32 p for routes 8j + 4h + i of each 32-route block
-    const uint32_t row = row0 + w * 256;
-    // byte offsets fit 32 bits (the launcher checks): one multiply-add per route, the base stays scalar
-    if (a.epi == 1) {
-      uint8_t* out = static_cast<uint8_t*>(a.out);
-      const uint32_t pitch = a.rows * 4, col = row * 4;
-#pragma unroll
-      for (int nt = 0; nt < NTA; ++nt) {
-#pragma unroll
-        for (int j = 0; j < RES / 4; ++j) {
-          const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
-          const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float* o = reinterpret_cast<float*>(out + (sl4[i] * pitch + col));
-            o[0] = acc[0][nt][4 * j + i];
-            o[32] = acc[1][nt][4 * j + i];
-          }
-        }
-      }
-    } else {
-      uint8_t* out = static_cast<uint8_t*>(a.out);
-      const uint32_t pitch = a.rows * 2, col = row * 2;
-#pragma unroll
-      for (int nt = 0; nt < NTA; ++nt) {
-#pragma unroll
-        for (int j = 0; j < RES / 4; ++j) {
-          const uint4 sl = *reinterpret_cast<const uint4*>(s_slot + nt * 32 + 8 * j + 4 * h);
-          const uint32_t sl4[4] = {sl.x, sl.y, sl.z, sl.w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            uint16_t* o = reinterpret_cast<uint16_t*>(out + (sl4[i] * pitch + col));
-            o[0] = f_to_bf16(acc[0][nt][4 * j + i]);
-            o[32] = f_to_bf16(acc[1][nt][4 * j + i]);
-          }
-        }
-      }
-    }
-    wrow = wnext;
-  }
-  };  // tile_body
-  using two = std::integral_constant<int, 2>;
-  using one = std::integral_constant<int, 1>;
-  if (count > 32) tile_body(two{}, std::integral_constant<int, 16>{});
-  else if (count > 8) tile_body(one{}, std::integral_constant<int, 16>{});
-  else tile_body(one{}, std::integral_constant<int, 4>{});
-  qmm_trace(a, work, 4);
-}
-
-template <int BITS, int NG, bool SWAPPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void qmm_kres_kernel(const KresLaunch launch) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  const uint32_t walk = launch.slices[second ? 1 : 0];
-  qmm_kres_item<BITS, NG, SWAPPED>(a, work, walk, smem);
-}
-
-template <int NG, bool SWAPPED>  // as qmm_mixed_kernel
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void qmm_kres_mixed_kernel(const KresLaunch launch) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
-  const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_kres_item<4, NG, true>(a, work, walk, smem);
-  else qmm_kres_item<2, NG, SWAPPED>(a, work, walk, smem);
 }
 
 // y[t,d] = bf16(h1[t,d] + sum_r w[t,r] * partial[t*K+r, d]), residual first, rank
@@ -2106,7 +1156,7 @@ hipError_t launch_prefill_router(hipStream_t s, const uint16_t* W, const uint16_
 
 hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint32_t t, uint32_t K,
                         uint32_t E, uint32_t* counts, uint32_t* offsets, uint32_t* starts,
-                        mf_pair* sorted, void* tiles, uint32_t tile_slots, uint32_t* n_tiles,
+                        mf_pair* sorted, const TileLists& tiles,
                         uint32_t* status, uint32_t* chunk_hist) {
   const uint32_t n_pairs = t * K;
   if (n_pairs && n_pairs <= kGroupOnePairs && group_one_lds_bytes(t, E) <= kGroupOneMaxBytes) {
@@ -2116,12 +1166,12 @@ hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint
     const hipError_t e = allow_lds<group_one_kernel>(lds, static_cast<int>(kGroupOneMaxBytes));
     if (e != hipSuccess) return e;
     group_one_kernel<<<dim3(1), dim3(1024), lds, s>>>(idx, w, n_pairs, K, E, tpe_log2, counts, offsets, starts, sorted,
-                                                      static_cast<Tile*>(tiles), tile_slots, n_tiles, status);
+                                                      tiles, status);
     return hipGetLastError();
   }
   if (n_pairs == 0) {  // no routes: the scan over no chunks writes empty experts and a clean status word
     group_scan_kernel<<<dim3(1), dim3(MF_MAX_EXPERTS), 0, s>>>(chunk_hist, 0, E, counts, offsets, starts,
-                                                               static_cast<Tile*>(tiles), tile_slots, n_tiles,
+                                                               tiles,
                                                                chunk_hist, status);
     return hipGetLastError();
   }
@@ -2132,7 +1182,7 @@ hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint
   uint32_t* chunk_bad = chunk_hist + static_cast<size_t>(kGroupChunks) * MF_MAX_EXPERTS;
   group_count_kernel<<<dim3(n_chunks), dim3(256), 0, s>>>(idx, n_pairs, E, chunk_pairs, chunk_hist, chunk_bad);
   group_scan_kernel<<<dim3(1), dim3(MF_MAX_EXPERTS), 0, s>>>(chunk_hist, n_chunks, E, counts, offsets, starts,
-                                                             static_cast<Tile*>(tiles), tile_slots, n_tiles,
+                                                             tiles,
                                                              chunk_bad, status);
   group_emit_kernel<<<dim3(n_chunks), dim3(256), 0, s>>>(idx, w, n_pairs, K, E, chunk_pairs, chunk_hist, starts,
                                                          sorted);
@@ -2152,7 +1202,7 @@ bool topk_group_takes(uint32_t t) { return t != 0 && t <= kGroupChunks * kChunkT
 
 hipError_t launch_topk_group(hipStream_t s, const float* logits, uint32_t t, uint32_t K, uint32_t E, int mode,
                              uint32_t* idx, float* w, uint32_t* counts, uint32_t* offsets, uint32_t* starts,
-                             mf_pair* sorted, void* tiles, uint32_t tile_slots, uint32_t* n_tiles, uint32_t* status,
+                             mf_pair* sorted, const TileLists& tiles, uint32_t* status,
                              uint32_t* group_tmp) {
   // a token per wave while that gives at most 128 chunks, then longer chunks, then more of them
   uint32_t chunk_tokens = ((t + 127) / 128 + kSelectWaves - 1) / kSelectWaves * kSelectWaves;
@@ -2165,41 +1215,28 @@ hipError_t launch_topk_group(hipStream_t s, const float* logits, uint32_t t, uin
                                                                        cnt, bad);
   group_place_kernel<<<dim3(n_chunks), dim3(MF_MAX_EXPERTS), 0, s>>>(idx, w, t, K, E, chunk_tokens, n_chunks, bits, cnt,
                                                                     bad, counts, offsets, starts, sorted,
-                                                                    static_cast<Tile*>(tiles), tile_slots, n_tiles,
+                                                                    tiles,
                                                                     status);
   return hipGetLastError();
 }
 
-size_t qmm_lds_bytes(uint32_t kdim, int nproj, bool tab16) {
-  const uint32_t ng = kdim / kGroup;
-  return kQmmXBytes + ((static_cast<size_t>(nproj) * kQmmWaves * ng * 32 * (tab16 ? 2 : 4) + 15) & ~static_cast<size_t>(15)) +
-         kTileTokens * 4;
-}
-// the scale tables as bf16 where fp32 tables would leave a CU (160 KB of LDS) room for one workgroup only
-bool qmm_tab16(uint32_t kdim, int nproj) { return 2 * qmm_lds_bytes(kdim, nproj, false) > 160 * 1024; }
-
-hipError_t launch_prep_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, float* sums, size_t elems,
-                            const uint16_t* src1 = nullptr, uint16_t* dst1 = nullptr, float* sums1 = nullptr,
-                            size_t elems1 = 0) {
-  PrepArgs a{};
-  a.src[0] = src; a.dst[0] = dst; a.sums[0] = sums; a.chunks[0] = static_cast<uint32_t>(elems / 8);
-  a.src[1] = src1; a.dst[1] = dst1; a.sums[1] = sums1; a.chunks[1] = static_cast<uint32_t>(elems1 / 8);
-  a.blocks0 = (a.chunks[0] + 255) / 256;
-  const uint32_t blocks = a.blocks0 + (a.chunks[1] + 255) / 256;
+// `rows` rows of k values
+hipError_t launch_prep_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, uint16_t* sums, uint32_t rows, uint32_t k) {
+  const uint32_t chunks = static_cast<uint32_t>(static_cast<size_t>(rows) * k / 8), blocks = (chunks + 255) / 256;
   if (!blocks) return hipSuccess;
-  prep_rows_kernel<<<dim3(blocks), dim3(256), 0, s>>>(a);
+  prep_rows_kernel<<<dim3(blocks), dim3(256), 0, s>>>(src, dst, sums, chunks, k / kGroup);
   return hipGetLastError();
 }
 
-// Work items of a dense problem that one XCD gets: an eighth, but at least 4 while there are any -- a handful
-// of items (the shared expert beside the routed experts of a short batch) runs faster on few XCDs, whose L2
-// serves the x rows and weight rows they share, than spread one to an XCD (Qwen shape, 128 tokens: layer 81 us
-// against 89 us).
-static uint32_t dense_per_xcd(uint32_t items) { return std::max((items + 7) / 8, std::min(items, 4u)); }
-// Whether an XCD should own tiles (and stream all weight rows) or row slices (and stream all of x): whichever
-// streams fewer bytes.  code_bits: 4 or 2.
-static int dense_tile_major(uint32_t rows, uint32_t x_rows, int code_bits) {
-  return static_cast<uint64_t>(rows) * code_bits <= static_cast<uint64_t>(x_rows) * 16;
+static hipError_t launch_qmm(hipStream_t s, uint32_t tile, int bits, const QmmArgs& a, int nproj, uint32_t tile_slots,
+                             const QmmArgs* b, uint32_t b_tile_slots) {
+  return tile == kSmallTile ? launch_qmm_tiles<kSmallTile>(s, bits, a, nproj, tile_slots, b, b_tile_slots)
+                            : launch_qmm_tiles<kTileTokens>(s, bits, a, nproj, tile_slots, b, b_tile_slots);
+}
+static hipError_t launch_qmm_kres(hipStream_t s, uint32_t tile, int bits, const QmmArgs& a, uint32_t tile_slots,
+                                  const QmmArgs* b, uint32_t b_tile_slots) {
+  return tile == kSmallTile ? launch_kres_tiles<kSmallTile>(s, bits, a, tile_slots, b, b_tile_slots)
+                            : launch_kres_tiles<kTileTokens>(s, bits, a, tile_slots, b, b_tile_slots);
 }
 
 // Whether qmm_kres_kernel takes the problem: a down-projection epilogue, K of 128, 256 or 512, whole
@@ -2210,117 +1247,6 @@ bool kres_takes(const QmmArgs& q, size_t out_rows) {
   if (static_cast<uint64_t>(out_rows) * q.rows * 4 >= (1ull << 32)) return false;  // 32-bit store offsets
   if (q.dense_mode) return aligned16(q.dense[0].scales) && aligned16(q.dense[0].biases) && aligned16(q.dense[0].weights);
   return aligned16(q.expert_base) && q.expert_stride % 16 == 0 && (q.w_off[0] | q.s_off[0] | q.b_off[0]) % 16 == 0;
-}
-
-// bits: 4, 2 (2-bit and ternary codes), or kMixedBits: the routed problem 2-bit, the dense one 4-bit
-constexpr int kMixedBits = 24;
-static int part_bits(int bits, const QmmArgs& q) { return bits != kMixedBits ? bits : q.dense_mode ? 4 : 2; }
-hipError_t launch_qmm_kres(hipStream_t s, int bits, const QmmArgs& a, uint32_t tile_slots, const QmmArgs* b,
-                           uint32_t b_tile_slots) {
-  KresLaunch launch{};
-  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
-  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
-  for (int part = 0; part < (b ? 2 : 1); ++part) {
-    QmmArgs& q = launch.part[part];
-    q = part ? *b : a;
-    const uint32_t slots = part ? b_tile_slots : tile_slots;
-    const uint32_t n_slices = q.rows / 256;
-    // two slices per work item halve the set-up per slice and still leave several rounds of work items
-    // (Qwen shape, 2048 tokens, whole layer: 331 us with one slice, 325 with two, 330 with four, 334 with eight)
-    const uint32_t walk = n_slices % 2 == 0 ? 2 : 1;
-    launch.slices[part] = walk;
-    if (q.dense_mode) {
-      q.dense_tiles = slots;
-      q.tile_major = dense_tile_major(q.rows, q.dense_rows, part_bits(bits, q));
-      q.dense_items = slots * (n_slices / walk);
-      launch.per_xcd[part] = dense_per_xcd(q.dense_items);
-    } else {
-      launch.per_xcd[part] = slots / 8 * (n_slices / walk);
-    }
-  }
-  const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
-  if (grid.x == 0) return hipSuccess;
-  const uint32_t ng = a.kdim / kGroup;
-  const size_t lds = static_cast<size_t>(ng) * 8192 + kTileTokens * 4 + kTileTokens * ng * 4;
-#define MF_KRES_L(...)                                                                                 \
-  do {                                                                                                 \
-    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
-    if (e != hipSuccess) return e;                                                                     \
-    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
-  } while (0)
-#define MF_KRES(N)                                                                                     \
-  do {                                                                                                 \
-    if (bits == kMixedBits && tiled) MF_KRES_L(qmm_kres_mixed_kernel<N, false>);                       \
-    else if (bits == kMixedBits) MF_KRES_L(qmm_kres_mixed_kernel<N, true>);                            \
-    else if (bits == 4 && tiled) MF_KRES_L(qmm_kres_kernel<4, N, false>);                              \
-    else if (bits == 4) MF_KRES_L(qmm_kres_kernel<4, N, true>);                                        \
-    else if (tiled) MF_KRES_L(qmm_kres_kernel<2, N, false>);                                           \
-    else MF_KRES_L(qmm_kres_kernel<2, N, true>);                                                       \
-  } while (0)
-  if (ng == 8) MF_KRES(8); else if (ng == 4) MF_KRES(4); else MF_KRES(2);
-#undef MF_KRES_L
-#undef MF_KRES
-  return hipGetLastError();
-}
-
-// tile_slots: entries of the tile list (routed; a multiple of 8) or number of 64-row tiles (dense).
-// `b` (optional) is a second problem for the same instantiation, run behind `a` in the same launch.
-hipError_t launch_qmm(hipStream_t s, int bits, QmmArgs a, int nproj, uint32_t tile_slots, const QmmArgs* b,
-                      uint32_t b_tile_slots) {
-  QmmLaunch launch{};
-  const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
-  if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
-  size_t lds = 0;
-  bool ng8 = true, tab16 = false;
-  for (int part = 0; part < (b ? 2 : 1); ++part) {
-    QmmArgs& q = launch.part[part];
-    q = part ? *b : a;
-    const uint32_t slots = part ? b_tile_slots : tile_slots;
-    const uint32_t slice_rows = kQmmRows * (q.pair_rows ? nproj : 1), n_slices = (q.rows + slice_rows - 1) / slice_rows;
-    if (q.dense_mode) {
-      q.dense_tiles = slots;
-      q.tile_major = dense_tile_major(q.rows * (q.pair_rows ? 1 : nproj), q.dense_rows, part_bits(bits, q));
-      q.dense_items = slots * n_slices * std::max(1u, q.n_win);
-      launch.per_xcd[part] = dense_per_xcd(q.dense_items);
-    } else {
-      launch.per_xcd[part] = slots / 8 * n_slices;
-    }
-    q.tab_aligned = q.dense_mode
-        ? aligned16(q.dense[0].scales) && aligned16(q.dense[0].biases) && aligned16(q.dense[1].scales) &&
-              aligned16(q.dense[1].biases)
-        : aligned16(q.expert_base) && q.expert_stride % 16 == 0 &&
-              (q.s_off[0] | q.b_off[0] | q.s_off[1] | q.b_off[1]) % 16 == 0;
-    tab16 = tab16 || qmm_tab16(q.kdim, nproj);  // with windows: kdim is the longest window
-    ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0 && q.rows % slice_rows == 0;
-  }
-  for (int part = 0; part < (b ? 2 : 1); ++part) lds = std::max(lds, qmm_lds_bytes(launch.part[part].kdim, nproj, tab16));
-  const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
-  if (grid.x == 0) return hipSuccess;
-#define MF_QMM_L(...)                                                                                  \
-  do {                                                                                                 \
-    const hipError_t e = allow_lds<__VA_ARGS__>(lds, kMaxLds);                                         \
-    if (e != hipSuccess) return e;                                                                     \
-    __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
-  } while (0)
-#define MF_QMM(P, G, T)                                                                                \
-  do {                                                                                                 \
-    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<P, G, T, false>);                       \
-    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<P, G, T, true>);                            \
-    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<4, P, G, T, false>);                              \
-    else if (bits == 4) MF_QMM_L(qmm_kernel<4, P, G, T, true>);                                        \
-    else if (tiled) MF_QMM_L(qmm_kernel<2, P, G, T, false>);                                           \
-    else MF_QMM_L(qmm_kernel<2, P, G, T, true>);                                                       \
-  } while (0)
-#define MF_QMM_G(P, G)                                         \
-  do {                                                         \
-    if (tab16) MF_QMM(P, G, true); else MF_QMM(P, G, false);   \
-  } while (0)
-  if (nproj == 2) { if (ng8) MF_QMM_G(2, true); else MF_QMM_G(2, false); }
-  else { if (ng8) MF_QMM_G(1, true); else MF_QMM_G(1, false); }
-#undef MF_QMM_G
-#undef MF_QMM
-#undef MF_QMM_L
-  return hipGetLastError();
 }
 
 namespace {
@@ -2435,8 +1361,8 @@ static size_t dense_gate_up_parts_bytes(uint32_t t, uint32_t f, uint32_t d) {
 // one-window launch and prep_rows_kernel produce together.  One thread per run of 8.
 __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* __restrict__ pg, const float* __restrict__ pu,
                                                                    uint32_t n_parts, size_t part_stride,
-                                                                   uint16_t* __restrict__ act, float* __restrict__ sums,
-                                                                   size_t chunks, float limit) {
+                                                                   uint16_t* __restrict__ act, uint16_t* __restrict__ sums,
+                                                                   size_t chunks, uint32_t ng, float limit) {
   const size_t c = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   float g[8], u[8];
 #pragma unroll
@@ -2473,7 +1399,8 @@ __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* 
   if (c >= chunks) return;
   *reinterpret_cast<uint4*>(act + c * 8) = make_uint4(a[0] | (a[4] << 16), a[1] | (a[5] << 16), a[2] | (a[6] << 16),
                                                       a[3] | (a[7] << 16));
-  if ((c & 7) == 0) sums[c >> 3] = sum;
+  const size_t grp = c >> 3, r = grp / ng;
+  if ((c & 7) == 0) store_group_sum(sums + r * group_sum_words(ng), static_cast<uint32_t>(grp - r * ng), ng, sum);
 }
 
 bool dense_qmm_takes(const mf_qtensor& w, int bits, const void* x, const void* y, uint32_t m, uint32_t n, uint32_t k) {
@@ -2483,8 +1410,10 @@ bool dense_qmm_takes(const mf_qtensor& w, int bits, const void* x, const void* y
   return true;
 }
 
+// bytes of the group sums of `rows` rows of k values
+static size_t sums_bytes(size_t rows, uint32_t k) { return sizeof(uint16_t) * rows * group_sum_words(k / kGroup); }
 static size_t dense_qmm_rows_bytes(uint32_t m, uint32_t k) {
-  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup));
+  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sums_bytes(m, k));
 }
 size_t dense_qmm_needs(uint32_t m, uint32_t n, uint32_t k) { return dense_qmm_rows_bytes(m, k) + dense_parts_bytes(m, n, dense_windows(m, n, k)); }
 size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
@@ -2492,7 +1421,7 @@ size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
 }
 
 // x_prepared: rows already in the matmul's order with their group sums in sumx (x is then ignored)
-static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, const uint16_t* xp, const float* sumx,
+static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, const uint16_t* xp, const uint16_t* sumx,
                                 void* y, uint32_t m, uint32_t n, uint32_t k, uint32_t n_win, bool out_f32, void* parts) {
   const uint32_t ng = k / kGroup;
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
@@ -2514,7 +1443,7 @@ static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, co
     d.kdim = dense_longest_window(ng, n_win) * kGroup; d.n_win = n_win; d.out_win_stride = part_stride; d.epi = 1; d.out = parts;
   }
   {
-    const hipError_t e = launch_qmm(s, code_bits, d, d.pair_rows ? 2 : 1, tiles, nullptr, 0);
+    const hipError_t e = launch_qmm(s, kTileTokens, code_bits, d, d.pair_rows ? 2 : 1, tiles, nullptr, 0);
     if (e != hipSuccess) return e;
   }
   if (n_win > 1) {
@@ -2530,9 +1459,9 @@ hipError_t launch_dense_qmm(hipStream_t s, const mf_qtensor& w, int bits, const 
                             uint32_t n, uint32_t k, bool out_f32, void* workspace) {
   uint8_t* base = static_cast<uint8_t*>(workspace);
   uint16_t* xp = reinterpret_cast<uint16_t*>(base);
-  float* sumx = reinterpret_cast<float*>(base + up256(sizeof(uint16_t) * static_cast<size_t>(m) * k));
-  void* parts = reinterpret_cast<uint8_t*>(sumx) + up256(sizeof(float) * static_cast<size_t>(m) * (k / kGroup));
-  const hipError_t e = launch_prep_rows(s, x, xp, sumx, static_cast<size_t>(m) * k);
+  uint16_t* sumx = reinterpret_cast<uint16_t*>(base + up256(sizeof(uint16_t) * static_cast<size_t>(m) * k));
+  void* parts = reinterpret_cast<uint8_t*>(sumx) + up256(sums_bytes(m, k));
+  const hipError_t e = launch_prep_rows(s, x, xp, sumx, m, k);
   if (e != hipSuccess) return e;
   return dense_project(s, w, bits, xp, sumx, y, m, n, k, dense_windows(m, n, k), out_f32, parts);
 }
@@ -2548,7 +1477,7 @@ bool dense_mlp_takes(const mf_qtensor& gate, const mf_qtensor& up, const mf_qten
 
 static size_t dense_mlp_rows_bytes(uint32_t d, uint32_t f, uint32_t t) {
   return up256(sizeof(uint16_t) * static_cast<size_t>(t) * f) + up256(sizeof(uint16_t) * static_cast<size_t>(t) * d) +
-         up256(sizeof(float) * static_cast<size_t>(t) * (d / kGroup)) + up256(sizeof(float) * static_cast<size_t>(t) * (f / kGroup));
+         up256(sums_bytes(t, d)) + up256(sums_bytes(t, f));
 }
 // (the window results of gate / up and of down follow one another in the same place)
 size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows) {
@@ -2566,11 +1495,11 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
   base += up256(sizeof(uint16_t) * static_cast<size_t>(t) * f);
   uint16_t* xp = reinterpret_cast<uint16_t*>(base);
   base += up256(sizeof(uint16_t) * static_cast<size_t>(t) * d);
-  float* sumx = reinterpret_cast<float*>(base);
-  base += up256(sizeof(float) * static_cast<size_t>(t) * (d / kGroup));
-  float* sum_act = reinterpret_cast<float*>(base);
-  base += up256(sizeof(float) * static_cast<size_t>(t) * (f / kGroup));
-  hipError_t e = launch_prep_rows(s, x, xp, sumx, static_cast<size_t>(t) * d);
+  uint16_t* sumx = reinterpret_cast<uint16_t*>(base);
+  base += up256(sums_bytes(t, d));
+  uint16_t* sum_act = reinterpret_cast<uint16_t*>(base);
+  base += up256(sums_bytes(t, f));
+  hipError_t e = launch_prep_rows(s, x, xp, sumx, t, d);
   if (e != hipSuccess) return e;
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
   QmmArgs q{};
@@ -2581,7 +1510,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     q.dense[0].biases = gate.scales;
     q.dense[1].biases = up.scales;
   }
-  q.x = xp; q.sumx = sumx; q.x_stride = d; q.rows = f; q.kdim = d; q.epi = 0; q.out = act;
+  q.x = xp; q.sumx = sumx; q.x_stride = d; q.rows = f; q.kdim = d; q.epi = 0; q.out = act; q.out_sums = sum_act;
   const uint32_t gu_win = dense_gate_up_windows(d);
   if (gu_win > 1) {
     // few rows (or a K too long for one launch's scale tables): the contraction in windows, both projections as
@@ -2592,35 +1521,52 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     float* pu = pg + part_stride * gu_win;
     q.ng_ld = ng; q.kdim = dense_longest_window(ng, gu_win) * kGroup; q.n_win = gu_win; q.out_win_stride = part_stride;
     q.epi = 1; q.out = pg; q.out2 = pu;
-    e = launch_qmm(s, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
+    e = launch_qmm(s, kTileTokens, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
     if (e != hipSuccess) return e;
     const size_t chunks = static_cast<size_t>(t) * f / 8;
     dense_swiglu_combine_kernel<<<dim3(static_cast<uint32_t>((chunks + 255) / 256)), dim3(256), 0, s>>>(
-        pg, pu, gu_win, part_stride, act, sum_act, chunks, 0.0f);
+        pg, pu, gu_win, part_stride, act, sum_act, chunks, f / kGroup, 0.0f);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else {
-    e = launch_qmm(s, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
-    if (e != hipSuccess) return e;
-    e = launch_prep_rows(s, act, nullptr, sum_act, static_cast<size_t>(t) * f);  // the activations are in matmul order already
+    e = launch_qmm(s, kTileTokens, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
     if (e != hipSuccess) return e;
   }
   return dense_project(s, down, bits, act, sum_act, y, t, d, f, down_windows, false, base);
 }
 
+// Routes of a tile of the layer call's two matmuls.  A tile of 32 leaves registers and LDS for three workgroups a CU where one
+// of 64 leaves them for two, and wastes less where few tokens meet an expert; past 32 routes an expert (on average, over the
+// layer's experts) more and more tiles of 64 are full, and expand a weight for 64 tokens at a time.  2-bit codes without a
+// 4-bit shared expert beside them are read and expanded faster: past 128.  Layer call, tiles of 64 / 32, us: 256 4-bit experts
+// 2048 x 512, shared 512: 93 tokens 81.4 / 73.8, 256 95.3 / 88.7, 512 118.6 / 117.8, 2048 243 / 262; 128 experts of
+// 2816 x 704: 300 tokens 235 / 210, 500 302 / 299, 800 358 / 377; 256 2-bit experts of 4096 x 2048, shared 2048: 200 tokens
+// 347 / 322, 777 647 / 623, 2048 1194 / 1224; 64 ternary experts of 2048 x 1024: 400 tokens 136 / 111, 1600 267 / 259, 2048 310 / 312.
+// The resident kernel on 4-bit rows of 512 keeps tiles of 64: its three workgroups a CU have half the codes in flight each
+// (400 tokens, 2048 x 512: 24.1 / 30.0 us; 93 tokens 20.6 / 20.3).
+struct PrefillTiles { uint32_t up, down; };
+static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t) {
+  const bool two_bit = c.bits != MF_BITS_4 && !c.shared_f;
+  const uint64_t few = static_cast<uint64_t>(two_bit ? 128 : 32) * c.num_experts;
+  PrefillTiles p;
+  p.up = static_cast<uint64_t>(t) * c.top_k <= few ? kSmallTile : kTileTokens;
+  p.down = c.bits == MF_BITS_4 && c.f == 512 ? kTileTokens : p.up;
+  return p;
+}
+
 // entries of the tile list: every live expert may end in a partial tile; a multiple of 8
-uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t) {
+uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t, uint32_t tile) {
   const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const size_t n = std::min<size_t>(c.num_experts, pairs) + pairs / kTileTokens + 1;
+  const size_t n = std::min<size_t>(c.num_experts, pairs) + pairs / tile + 1;
   return static_cast<uint32_t>((n + 7) / 8 * 8);
 }
 
 // workspace carve-up of one prefill layer call
 struct PrefillWs {
   float* logits; uint32_t* idx; float* w; uint32_t* counts; uint32_t* offsets; uint32_t* starts;
-  uint32_t* n_tiles; uint32_t* status; Tile* tiles; mf_pair* sorted; uint16_t* acts; float* partials;
+  uint32_t* status; Tile* tiles[2]; mf_pair* sorted; uint16_t* acts; float* partials;
   uint16_t* sact; uint16_t* hs; uint16_t* gate;
-  uint16_t* xp; float* sum_x; float* sum_acts; float* sum_sact;
+  uint16_t* xp; uint16_t* sum_x; uint16_t* sum_acts; uint16_t* sum_sact;
   size_t bytes;
 };
 
@@ -2633,16 +1579,15 @@ PrefillWs prefill_carve(const mf_moe_config& c, uint32_t t, void* base) {
     return static_cast<void*>(base ? at : nullptr);
   };
   const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const size_t max_tiles = prefill_tile_slots(c, t);
+  const size_t max_tiles = prefill_tile_slots(c, t, kSmallTile);  // (of either tile: bytes that grow with t)
   p.logits = static_cast<float*>(take(sizeof(float) * t * c.num_experts));
   p.idx = static_cast<uint32_t*>(take(sizeof(uint32_t) * pairs));
   p.w = static_cast<float*>(take(sizeof(float) * pairs));
   p.counts = static_cast<uint32_t*>(take(sizeof(uint32_t) * MF_MAX_EXPERTS));
   p.offsets = static_cast<uint32_t*>(take(sizeof(uint32_t) * MF_MAX_EXPERTS));
   p.starts = static_cast<uint32_t*>(take(sizeof(uint32_t) * MF_MAX_EXPERTS));
-  p.n_tiles = static_cast<uint32_t*>(take(256));
-  p.status = p.n_tiles ? p.n_tiles + 1 : nullptr;
-  p.tiles = static_cast<Tile*>(take(sizeof(Tile) * max_tiles));
+  p.status = static_cast<uint32_t*>(take(256));
+  for (Tile*& list : p.tiles) list = static_cast<Tile*>(take(sizeof(Tile) * max_tiles));
   p.sorted = static_cast<mf_pair*>(take(sizeof(mf_pair) * pairs));
   p.acts = static_cast<uint16_t*>(take(sizeof(uint16_t) * pairs * c.f));
   p.partials = static_cast<float*>(take(sizeof(float) * pairs * c.d));
@@ -2650,9 +1595,9 @@ PrefillWs prefill_carve(const mf_moe_config& c, uint32_t t, void* base) {
   p.hs = static_cast<uint16_t*>(take(sizeof(uint16_t) * static_cast<size_t>(t) * c.d));
   p.gate = static_cast<uint16_t*>(take(sizeof(uint16_t) * t));
   p.xp = static_cast<uint16_t*>(take(sizeof(uint16_t) * static_cast<size_t>(t) * c.d));
-  p.sum_x = static_cast<float*>(take(sizeof(float) * static_cast<size_t>(t) * (c.d / kGroup)));
-  p.sum_acts = static_cast<float*>(take(sizeof(float) * pairs * (c.f / kGroup)));
-  p.sum_sact = static_cast<float*>(take(sizeof(float) * static_cast<size_t>(t) * (std::max<uint32_t>(c.shared_f, 64) / kGroup)));
+  p.sum_x = static_cast<uint16_t*>(take(sums_bytes(t, c.d)));
+  p.sum_acts = static_cast<uint16_t*>(take(sums_bytes(pairs, c.f)));
+  p.sum_sact = static_cast<uint16_t*>(take(sums_bytes(t, std::max<uint32_t>(c.shared_f, 64))));
   p.bytes = pos;
   return p;
 }
@@ -2723,7 +1668,9 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   hipError_t e;
 #define MF_TRY(call) do { e = (call); if (e != hipSuccess) return e; } while (0)
   const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const uint32_t max_tiles = prefill_tile_slots(c, t);
+  const PrefillTiles tile = prefill_tiles(c, t);
+  TileLists lists{{ws.tiles[0], tile.down != tile.up ? ws.tiles[1] : nullptr},
+                  {prefill_tile_slots(c, t, tile.up), prefill_tile_slots(c, t, tile.down)}, {tile.up, tile.down}};
   bool x_prepared = false, fused_group = false;
   if (ragged) {
     // the caller's grouping: its per-expert counts are a one-chunk histogram for the scan that lays
@@ -2737,7 +1684,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
                                                                            t, c.top_k, bad);
     MF_TRY(hipGetLastError());
     group_scan_kernel<<<dim3(1), dim3(MF_MAX_EXPERTS), 0, s>>>(hist, 1, c.num_experts, ws.counts, ws.offsets, ws.starts,
-                                                               ws.tiles, max_tiles, ws.n_tiles, bad, ws.status, 1);
+                                                               lists, bad, ws.status, 1);
     MF_TRY(hipGetLastError());
     ws.sorted = const_cast<mf_pair*>(ragged->sorted);
     ws.partials = ragged->partials;
@@ -2753,13 +1700,13 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
       fused_group = topk_group_takes(t) && pairs > kGroupOnePairs;
       if (fused_group)
         MF_TRY(launch_topk_group(s, ws.logits, t, c.top_k, c.num_experts, c.router_mode, ws.idx, ws.w, ws.counts,
-                                 ws.offsets, ws.starts, ws.sorted, ws.tiles, max_tiles, ws.n_tiles, ws.status,
+                                 ws.offsets, ws.starts, ws.sorted, lists, ws.status,
                                  h.ws.group_tmp));
       else MF_TRY(launch_topk(s, ws.logits, c.num_experts, c.top_k, t, c.router_mode, ws.idx, ws.w));
     }
     if (!fused_group)
       MF_TRY(launch_group(s, ws.idx, ws.w, t, c.top_k, c.num_experts, ws.counts, ws.offsets, ws.starts,
-                          ws.sorted, ws.tiles, max_tiles, ws.n_tiles, ws.status, h.ws.group_tmp + 2048));
+                          ws.sorted, lists, ws.status, h.ws.group_tmp + 2048));
   }
 
   const bool gate_q8 = c.shared_f && w.w_sg_q8.weights;
@@ -2770,7 +1717,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
     prep_x_gate_kernel<<<dim3((t + 3) / 4), dim3(256), 0, s>>>(x, ws.xp, ws.sum_x, w.w_sg, ws.gate, t, c.d);
     MF_TRY(hipGetLastError());
   } else {
-    MF_TRY(launch_prep_rows(s, x, ws.xp, ws.sum_x, static_cast<size_t>(t) * c.d));
+    MF_TRY(launch_prep_rows(s, x, ws.xp, ws.sum_x, t, c.d));
   }
   // the scalar gate stored as an 8-bit row (RealForwardRunner.swift:2925-2941): one wave per token, the
   // bits of mf_gemv(MF_BITS_8) -- and of the decode launch
@@ -2782,8 +1729,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   q.tiled = w.expert_tiled != nullptr;
   q.expert_stride = w.expert_stride;
   q.sorted = ws.sorted;
-  q.tiles = ws.tiles;
-  q.n_tiles = ws.n_tiles;
+  q.tiles = lists.list[0];
   q.top_k = c.top_k;
   q.limit = c.swiglu_limit;
   // ternary experts are 2-bit codes whose bias is -scale: the kernels take the scale table as bias table
@@ -2800,24 +1746,26 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   }
   // The shared expert's two matmuls ride in the routed launches of the same phase.
   QmmArgs d{};
-  const uint32_t dense_tiles = c.shared_f ? (t + kTileTokens - 1) / kTileTokens : 0;
+  const uint32_t dense_up = c.shared_f ? (t + tile.up - 1) / tile.up : 0, dense_down = c.shared_f ? (t + tile.down - 1) / tile.down : 0;
   if (c.shared_f) {
     d.dense_mode = 1; d.dense_rows = t; d.top_k = c.top_k; d.narrow = 1;
     d.dense[0] = w.shared_gate; d.dense[1] = w.shared_up;
     d.x = ws.xp; d.sumx = ws.sum_x; d.x_stride = c.d; d.rows = c.shared_f; d.kdim = c.d; d.epi = 0; d.out = ws.sact;
+    d.out_sums = ws.sum_sact;
   }
   // phase 1: routed gate/up -> acts [pair, F]; shared gate/up -> sact [token, Fs]
   q.w_off[0] = w.offsets.gate_w; q.s_off[0] = w.offsets.gate_s; q.b_off[0] = ternary ? w.offsets.gate_s : w.offsets.gate_b;
   q.w_off[1] = w.offsets.up_w; q.s_off[1] = w.offsets.up_s; q.b_off[1] = ternary ? w.offsets.up_s : w.offsets.up_b;
   q.x = ws.xp; q.sumx = ws.sum_x; q.x_stride = c.d; q.gather = 1; q.rows = c.f; q.kdim = c.d; q.epi = 0;
   q.out = ws.acts;
+  q.out_sums = ws.sum_acts;
   // The shared expert's work items (whole 64-row tiles, the longest of the launch) go first: a short batch
   // leaves workgroup slots over, and up to about 4096 tokens the launch ends sooner with them out of the way
   // (Qwen shape, layer: 2048 tokens 280.5 -> 274.5 us, 1024 tokens 191 -> 187 us, 4096 tokens 506 -> 503 us;
   // at 16 384 tokens they are better last, 1763 against 1776 us, where they fill the holes of the last round).
   const bool dense_first = shared_rides && pairs <= 32768;
-  if (dense_first) MF_TRY(launch_qmm(s, launch_bits, d, 2, dense_tiles, &q, max_tiles));
-  else MF_TRY(launch_qmm(s, launch_bits, q, 2, max_tiles, shared_rides ? &d : nullptr, dense_tiles));
+  if (dense_first) MF_TRY(launch_qmm(s, tile.up, launch_bits, d, 2, dense_up, &q, lists.slots[0]));
+  else MF_TRY(launch_qmm(s, tile.up, launch_bits, q, 2, lists.slots[0], shared_rides ? &d : nullptr, dense_up));
   // phase 2: routed down -> fp32 partials [token*K+rank, D]; shared down -> hs [token, D]
   q.w_off[0] = w.offsets.down_w; q.s_off[0] = w.offsets.down_s; q.b_off[0] = ternary ? w.offsets.down_s : w.offsets.down_b;
   q.w_off[1] = q.s_off[1] = q.b_off[1] = 0;
@@ -2826,6 +1774,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // reference's prefill keeps 16-bit per-route results, prefill.metal:817-819, 644-651): half the bytes
   // written here and read by the reduce.  The caller's buffer of a ragged call stays fp32.
   const bool narrow_routes = !ragged && (c.maple_rounding || h.narrow_routes);
+  if (lists.list[1]) q.tiles = lists.list[1];
   q.x = ws.acts; q.sumx = ws.sum_acts; q.x_stride = c.f; q.gather = 0; q.rows = c.d; q.kdim = c.f;
   q.epi = narrow_routes ? 3 : 1; q.out = ws.partials;
   q.limit = 0.0f;
@@ -2846,26 +1795,17 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // launch always, 375 / 385; 4-bit experts alike, 4096 x 256, 2048 tokens 362 / 297).
   const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
   const bool apart = shared_rides && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
-  {
-    // group sums of the activation rows for qmm_kernel (qmm_kres_kernel sums the rows it stages itself);
-    // routes past the last tile's count were never written: only pairs rows exist, all written
-    const bool q_ring = !kres_both && !apart, d_ring = shared_rides && (apart ? !kres_d : !kres_both);
-    if (q_ring || d_ring)
-      MF_TRY(launch_prep_rows(s, q_ring ? ws.acts : nullptr, nullptr, ws.sum_acts, q_ring ? pairs * c.f : 0,
-                              d_ring ? ws.sact : nullptr, nullptr, ws.sum_sact,
-                              d_ring ? static_cast<size_t>(t) * c.shared_f : 0));
-  }
   const int down_proj = q.pair_rows ? 2 : 1;
   if (!shared_rides || apart) {
-    if (kres_q) MF_TRY(launch_qmm_kres(s, code_bits, q, max_tiles, nullptr, 0));
-    else MF_TRY(launch_qmm(s, code_bits, q, down_proj, max_tiles, nullptr, 0));
-    if (apart && kres_d) MF_TRY(launch_qmm_kres(s, 4, d, dense_tiles, nullptr, 0));
-    else if (apart) MF_TRY(launch_qmm(s, 4, d, down_proj, dense_tiles, nullptr, 0));
+    if (kres_q) MF_TRY(launch_qmm_kres(s, tile.down, code_bits, q, lists.slots[1], nullptr, 0));
+    else MF_TRY(launch_qmm(s, tile.down, code_bits, q, down_proj, lists.slots[1], nullptr, 0));
+    if (apart && kres_d) MF_TRY(launch_qmm_kres(s, tile.down, 4, d, dense_down, nullptr, 0));
+    else if (apart) MF_TRY(launch_qmm(s, tile.down, 4, d, down_proj, dense_down, nullptr, 0));
   } else if (kres_both) {
-    if (dense_first) MF_TRY(launch_qmm_kres(s, launch_bits, d, dense_tiles, &q, max_tiles));
-    else MF_TRY(launch_qmm_kres(s, launch_bits, q, max_tiles, &d, dense_tiles));
-  } else if (dense_first) MF_TRY(launch_qmm(s, launch_bits, d, down_proj, dense_tiles, &q, max_tiles));
-  else MF_TRY(launch_qmm(s, launch_bits, q, down_proj, max_tiles, &d, dense_tiles));
+    if (dense_first) MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, d, dense_down, &q, lists.slots[1]));
+    else MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, q, lists.slots[1], &d, dense_down));
+  } else if (dense_first) MF_TRY(launch_qmm(s, tile.down, launch_bits, d, down_proj, dense_down, &q, lists.slots[1]));
+  else MF_TRY(launch_qmm(s, tile.down, launch_bits, q, down_proj, lists.slots[1], &d, dense_down));
   if (ragged) return hipSuccess;  // the per-route results are the caller's: mf_moe_unpermute reduces them
   const uint16_t* hs = nullptr;
   const uint16_t* gate = nullptr;

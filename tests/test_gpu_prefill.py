@@ -343,6 +343,49 @@ def test_prefill_of_few_rows_takes_the_decode_launch(gpu, oracle, bits, e, fs, t
     assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref_y), f"bits={bits} t={t}")
 
 
+# loads of the experts that rank 0 and rank 1 of the tokens name: one route, the rows of a lane's results (8, 16) and of a
+# tile (32, 64) on both sides, several tiles; and so few experts that tiles of 64 are taken
+_FILLS = {"few": (16, [1, 8, 9, 16, 17, 32, 33], [4, 7, 15, 24, 31, 35]), "many": (4, [33, 64, 65, 138], [])}
+
+
+@pytest.mark.parametrize("fill", ["few", "many"])
+@pytest.mark.parametrize("bits,d,f,fs,tiled", [
+    (4, 256, 128, 0, True), (4, 256, 512, 512, False), (4, 192, 320, 128, False), (4, 640, 1024, 0, True), (2, 256, 256, 128, True),
+    (2, 384, 704, 0, False), (1, 512, 512, 0, True), (2, 1088, 192, 320, False),
+])
+def test_prefill_tiles_of_every_fill(gpu, oracle, fill, bits, d, f, fs, tiled):
+    """a caller's routing with chosen loads: the matmuls agree with the decode launch row by row, and a token's row does
+    not change when the tokens are handed over in another order"""
+    e, first, second = _FILLS[fill]
+    t, k = sum(first), 2 if second else 1
+    layer = oracle.synth_layer(ROOT_SEED + 0xA2C0 + d + f, d, f, e, k, bits=bits, fs=fs)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    wts.router_w = None
+    named = [np.repeat(np.arange(len(first)), first)] + ([np.repeat(len(first) + np.arange(len(second)), second)] if second else [])
+    rng = np.random.default_rng(d + f)
+    idx = np.stack([rng.permutation(n) for n in named], axis=1).astype(np.int32)
+    w = rng.random((t, k), dtype=np.float32)
+    x = oracle.synth_x(ROOT_SEED + d, t, d)
+    if tiled:
+        wts.experts_tiled = moe.tile_experts(wts.experts, wts.offsets)
+    def run(order):
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        moe.encode_prefill_layer(wts, ops.bf16_tensor(x[order]), y, t, out_indices=torch.from_numpy(idx[order]).cuda(),
+                                 out_weights=torch.from_numpy(w[order]).cuda())
+        torch.cuda.synchronize()
+        return ops.bf16_bits(y)
+    y = run(np.arange(t))
+    rows = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    for t0 in range(0, t, 8):
+        n = min(8, t - t0)
+        moe.encode_decode_layer(wts, ops.bf16_tensor(x[t0:t0 + n]), rows[t0:t0 + n], t=n, out_indices=torch.from_numpy(idx[t0:t0 + n]).cuda(),
+                                out_weights=torch.from_numpy(w[t0:t0 + n]).cuda())
+    moe.status()
+    assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ops.bf16_bits(rows)), f"bits={bits} d={d} f={f} {fill}")
+    order = rng.permutation(t)
+    assert np.array_equal(run(order), y[order])
+
+
 @pytest.mark.parametrize("bits", [4, 2, 1])
 def test_tiled_pool_has_the_documented_order(gpu, oracle, bits):
     """mf_moe_tile_experts byte for byte: per block of 32 rows, runs of 64 pieces of 16 bytes, piece m + 32 h for row m --
