@@ -107,23 +107,33 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
   }
 }
 
-// ---- many token rows, on the bf16 matrix cores.  Codes 0..255 are bf16 numbers as they are, so a K group is
+// ---- many token rows, on the bf16 matrix cores.  A code byte in the low half of a 16-bit word is the bf16 number
+// q * 2^-133 (the subnormals, mf_device.h), so an operand is a mask, or a shift and a mask, of a packed word; rows meet it times
+// 2^64 and in the order the masks leave the codes in, and the scale takes the powers of two back.  A K group is
 // sum(q x) from four 32x32x16 products, one fp32 multiply-add with the row's scale, and the biases enter as one more
 // product per two groups: sum(x) of a group as three bf16 terms (all 24 bits) against the bias in three K slots.
 // Tokens are the M side, weight rows the N side: a lane ends with one weight row, its scale is a per-lane scalar.
 //
 // A workgroup is 64 weight rows (of each projection) x 64 tokens, waves 2 x 2.  A stage is 128 K values: x rows and
-// code rows come in as whole 128-byte lines, one stage ahead in registers, and are handed out through LDS (16-byte
+// code rows come in as whole 128-byte lines, three stages ahead of their use (two sets of registers and an LDS buffer: a stage's
+// arithmetic is 0.5 us, a round trip to memory 1 to 2), and are handed out through LDS (16-byte
 // pieces, XOR-swizzled so that 16 lanes reading one piece of 16 rows cover all banks): read straight from memory a
 // lane's 16 bytes of its own row touch 32 lines per load instruction, and the line rate of the L1, not the matrix
-// core, would set the pace.
+// core, would set the pace.  Scales and biases come 8 groups (four stages) to a load.
 // KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
 // meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
 // loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens: gate/up 47.6 -> 37.9 us, down 23.8 -> 20.0).
+// The whole MLP of 2816 x 2112, us, with codes converted one by one and a stage requested one ahead / now: 16 rows 47.5 / 44.2,
+// 300 54.3 / 50.3, 600 89 / 76, 2048 223 / 203; 704 x 8192, 16 rows 66.4 / 57.4, 300 93 / 84.
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
-template <int NPROJ, int KS>
-__global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
+constexpr float kByteScale = 0x1p69f;  // q * 2^-133 meets x * 2^64
+
+// LONG: a set walks more than three stages; a short walk is a plain loop (instructions that run once cost their fetch:
+// 128 x 192, 16 rows 12.8 us with the long form, 11.6 with this one; 10.1 before stages were requested three ahead).
+template <int NPROJ, int KS, bool LONG>
+__global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   constexpr uint32_t kTok = 64;
   __shared__ uint4 s_x_all[KS][2][kTok * 16];      // [token][16 pieces of 8 values], piece ^ (token & 15)
   __shared__ uint4 s_w_all[KS][2][NPROJ][64 * 8];  // [row][8 pieces of 16 codes], piece ^ ((row >> 1) & 7)
@@ -145,43 +155,56 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
   // (whole 256-byte token rows per 16 threads measured slower: 40.4 against 37.9 us, four row addresses a thread)
   const uint32_t xt = tid >> 2, xq = tid & 3, wr = tid >> 3, wc = tid & 7;
   typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-  u32x4_t xr[4], wreg[NPROJ][2];
+  u32x4_t xr[2][4], wreg[2][NPROJ][2];                  // stage st waits in set st & 1 (counted from st0)
   const uint32_t row = min(r0 + rb * 32 + m, a.M - 1);  // the lane's weight row (past the end: the last one, not stored)
-  uint32_t sc[NPROJ][2], bi[NPROJ];                     // scale words of the stage's groups; the bias of group h of it
-  auto fetch = [&](uint32_t st) __attribute__((always_inline)) {
+  auto fetch = [&](uint32_t st, u32x4_t (&xs)[4], u32x4_t (&ws)[NPROJ][2]) __attribute__((always_inline)) {
     const uint32_t g = 2 * st + (xq >> 1);
-    const bool in = g < ng;  // half a stage behind an odd number of groups: zeros
+    const bool in = g < ng && st < st1;  // half a stage behind an odd number of groups, stages past this set's last: zeros
     const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt, a.T - 1)) * a.N + (in ? g : ng - 1) * kGroup + (xq & 1) * 32;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      xr[i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
-      if (!in) xr[i] = u32x4_t{0, 0, 0, 0};
+      xs[i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
+      if (!in) xs[i] = u32x4_t{0, 0, 0, 0};
     }
-    const uint32_t k0 = min(st * 128 + wc * 16, a.N - 16);  // (codes past the row meet x = 0)
+    const uint32_t k0 = min(st * 128 + wc * 16, a.N - 16);  // (codes past the row, or of a stage past the last, meet x = 0)
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        wreg[p][i] = *reinterpret_cast<const u32x4_t*>(a.W[p] + static_cast<size_t>(min(r0 + wr + 32 * i, a.M - 1)) * a.N + k0);
+        ws[p][i] = *reinterpret_cast<const u32x4_t*>(a.W[p] + static_cast<size_t>(min(r0 + wr + 32 * i, a.M - 1)) * a.N + k0);
     }
   };
-  auto fetch_tab = [&](uint32_t st) __attribute__((always_inline)) {
+  // scales and biases of the eight groups from g (a group of the row) on; groups past the row's last one are zeros
+  struct Tab { uint4 S[NPROJ], B[NPROJ]; };
+  auto fetch_tab = [&](uint32_t g) __attribute__((always_inline)) {
+    Tab t;
+    // (a load past the row's last group reads on into the next row, the table's last loads end with the table: what is not the row's is taken off)
+    const uint32_t at = row * ng + g, base = min(at, a.M * ng - 8);
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
-      const size_t at = static_cast<size_t>(row) * ng;
-      sc[p][0] = a.S[p][at + min(2 * st, ng - 1)];
-      sc[p][1] = a.S[p][at + min(2 * st + 1, ng - 1)];
-      bi[p] = a.B[p][at + min(2 * st + h, ng - 1)];
+      t.S[p] = drop_bf16(load_16_bytes(a.S[p] + base), at - base);
+      t.B[p] = drop_bf16(load_16_bytes(a.B[p] + base), at - base);
+      if (g + 8 > ng) {
+        uint32_t keep[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) keep[i] = g + 2 * i + 1 < ng ? 0xFFFFFFFFu : g + 2 * i < ng ? 0xFFFFu : 0u;
+        t.S[p] = make_uint4(t.S[p].x & keep[0], t.S[p].y & keep[1], t.S[p].z & keep[2], t.S[p].w & keep[3]);
+        t.B[p] = make_uint4(t.B[p].x & keep[0], t.B[p].y & keep[1], t.B[p].z & keep[2], t.B[p].w & keep[3]);
+      }
     }
+    return t;
   };
-  auto put = [&](uint32_t buf) __attribute__((always_inline)) {
+  auto put = [&](uint32_t buf, const u32x4_t (&xs)[4], const u32x4_t (&ws)[NPROJ][2]) __attribute__((always_inline)) {
     float part = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const u32x4_t v = xr[i];
-      reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] = v;
-      part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
-              ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
+      const u32x4_t v = xs[i];
+      const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
+      const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
+      part += ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
+      reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] =
+          u32x4_t{upper_halves(x0 * kRowScale, x2 * kRowScale), upper_halves(x1 * kRowScale, x3 * kRowScale),
+                  upper_halves(x4 * kRowScale, x6 * kRowScale), upper_halves(x5 * kRowScale, x7 * kRowScale)};
     }
     part = group_sum(part, 2);
     if ((xq & 1) == 0) s_sum[buf][xt][xq >> 1] = part;
@@ -190,7 +213,7 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const uint32_t r = wr + 32 * i;
-        reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = wreg[p][i];
+        reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = ws[p][i];
       }
   };
   f32x16_t acc[NPROJ];
@@ -200,25 +223,9 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[p][r] = 0.0f;
 
-  if (st0 < st1) {
-    fetch(st0);
-    fetch_tab(st0);
-    put(0);
-    if (st0 + 1 < st1) fetch(st0 + 1);
-  }
-  for (uint32_t i_st = 0; i_st < n_walk; ++i_st) {
-    __syncthreads();  // buffer i_st & 1 is complete, the other one is no longer read
-    const uint32_t st = st0 + i_st, buf = i_st & 1;
-    if (st >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
-    uint32_t scv[NPROJ][2], bv[NPROJ];
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p) scv[p][0] = sc[p][0], scv[p][1] = sc[p][1], bv[p] = bi[p];
-    if (st + 1 < st1) {
-      put(buf ^ 1);
-      fetch_tab(st + 1);
-      if (st + 2 < st1) fetch(st + 2);
-    }
-    // biases: K slots of half h = (hi, mid, lo) of sum(x) over group 2 st + h (a group past the end sums to 0)
+  // one stage out of LDS; sw, bw: the words of the scales and biases of its two groups
+  auto multiply = [&](uint32_t buf, const uint32_t (&sw)[NPROJ], const uint32_t (&bw)[NPROJ]) __attribute__((always_inline)) {
+    // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0)
     {
       const float v = s_sum[buf][tok_m][h];
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
@@ -227,7 +234,10 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
       const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
       const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p) acc[p] = mfma_bf16(av, make_uint4(bv[p] | (bv[p] << 16), bv[p], 0, 0), acc[p]);
+      for (int p = 0; p < NPROJ; ++p) {
+        const uint32_t b = h ? bw[p] >> 16 : bw[p] & 0xFFFFu;
+        acc[p] = mfma_bf16(av, make_uint4(b | (b << 16), b, 0, 0), acc[p]);
+      }
     }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
@@ -243,23 +253,61 @@ __global__ __launch_bounds__(256 * KS) void qmm8_kernel(const Q8Args a, uint32_t
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const uint4 w = s_w[buf][p][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
-          const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {  // eight codes -> eight bf16 numbers (a byte as fp32 has its bits in the upper half)
-            uint32_t o[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const uint32_t word = ww[2 * u + (k >> 1)] >> (16 * (k & 1));
-              o[k] = __builtin_amdgcn_perm(__float_as_uint(static_cast<float>((word >> 8) & 0xFFu)),
-                                           __float_as_uint(static_cast<float>(word & 0xFFu)), 0x07060302u);
-            }
-            tmp = mfma_bf16(bx[2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp);
-          }
+          constexpr uint32_t kMask = 0x00FF00FFu;
+          tmp = mfma_bf16(bx[2 * c], make_uint4(w.x & kMask, (w.x >> 8) & kMask, w.y & kMask, (w.y >> 8) & kMask), tmp);
+          tmp = mfma_bf16(bx[2 * c + 1], make_uint4(w.z & kMask, (w.z >> 8) & kMask, w.w & kMask, (w.w >> 8) & kMask), tmp);
         }
-        const float s = __uint_as_float(scv[p][g] << 16);
+        const float s = kByteScale * (g ? bf16_hi(sw[p]) : bf16_lo(sw[p]));
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[p][i] = __builtin_fmaf(s, tmp[i], acc[p][i]);
       }
+    }
+  };
+  if constexpr (LONG) {
+    // (no branch around a request: a wait for one stage's registers would cover the later stages' as well)
+    fetch(st0, xr[0], wreg[0]);
+    Tab next = fetch_tab(min(2 * st0, ng - 1));
+    fetch(st0 + 1, xr[1], wreg[1]);
+    put(0, xr[0], wreg[0]);
+    fetch(st0 + 2, xr[0], wreg[0]);
+    for (uint32_t i0 = 0; i0 < n_walk; i0 += 4) {
+      const Tab tab = next;
+      next = fetch_tab(min(2 * (st0 + i0 + 4), ng - 1));
+#pragma unroll
+      for (int u4 = 0; u4 < 4; ++u4) {  // stage i0 + u4, in buffer u4 & 1
+        if (i0 + u4 >= n_walk) break;
+        __syncthreads();  // its buffer is complete, the other one is no longer read
+        const int buf = u4 & 1, other = buf ^ 1;
+        if (i0 + u4 + 1 < n_walk) put(other, xr[other], wreg[other]);
+        fetch(st0 + i0 + u4 + 3, xr[other], wreg[other]);
+        uint32_t sw[NPROJ], bw[NPROJ];
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) {
+          const uint32_t s4[4] = {tab.S[p].x, tab.S[p].y, tab.S[p].z, tab.S[p].w}, b4[4] = {tab.B[p].x, tab.B[p].y, tab.B[p].z, tab.B[p].w};
+          sw[p] = s4[u4];
+          bw[p] = b4[u4];
+        }
+        multiply(buf, sw, bw);
+      }
+    }
+  } else {
+    fetch(st0, xr[0], wreg[0]);
+    Tab tab = fetch_tab(min(2 * st0, ng - 1));
+    put(0, xr[0], wreg[0]);
+#pragma unroll 1
+    for (uint32_t i = 0; i < n_walk; ++i) {
+      __syncthreads();
+      if (i + 1 < n_walk) fetch(st0 + i + 1, xr[0], wreg[0]);
+      uint32_t sw[NPROJ], bw[NPROJ];
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+        sw[p] = tab.S[p].x;
+        bw[p] = tab.B[p].x;
+        tab.S[p] = make_uint4(tab.S[p].y, tab.S[p].z, tab.S[p].w, 0);
+        tab.B[p] = make_uint4(tab.B[p].y, tab.B[p].z, tab.B[p].w, 0);
+      }
+      multiply(i & 1u, sw, bw);
+      if (i + 1 < n_walk) put((i + 1) & 1u, xr[0], wreg[0]);
     }
   }
   if constexpr (KS == 2) {  // the second set's sums to the first, over the x buffers
@@ -308,8 +356,12 @@ static bool q8_launch(hipStream_t s, const Q8Args& a, hipError_t& err) {
     // without; 512 rows, 264 and 352 workgroups on 256 CUs, 101 and 88)
     const uint32_t tiles = (a.T + 63) / 64, n_work = (a.M + 63) / 64 * tiles;
     const dim3 grid((n_work + 7) / 8 * 8);
-    if (n_work > device_cu_count()) qmm8_kernel<NPROJ, 1><<<grid, dim3(256), 0, s>>>(a, tiles, n_work);
-    else qmm8_kernel<NPROJ, 2><<<grid, dim3(512), 0, s>>>(a, tiles, n_work);
+    const bool halved = n_work <= device_cu_count();
+    const uint32_t stages = (a.N / kGroup + 1) / 2, walk = halved ? (stages + 1) / 2 : stages;
+    if (!halved && walk > 3) qmm8_kernel<NPROJ, 1, true><<<grid, dim3(256), 0, s>>>(a, tiles, n_work);
+    else if (!halved) qmm8_kernel<NPROJ, 1, false><<<grid, dim3(256), 0, s>>>(a, tiles, n_work);
+    else if (walk > 3) qmm8_kernel<NPROJ, 2, true><<<grid, dim3(512), 0, s>>>(a, tiles, n_work);
+    else qmm8_kernel<NPROJ, 2, false><<<grid, dim3(512), 0, s>>>(a, tiles, n_work);
     err = hipGetLastError();
     return true;
   }
