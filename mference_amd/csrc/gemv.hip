@@ -483,27 +483,34 @@ __global__ __launch_bounds__(KS * 64) void rows_mfma_kernel(const RowsMfmaArgs a
   }
 }
 
-// Quad form for 1..4 token rows of a wide 4-bit matrix.  v_mfma_f32_4x4x4_16b_bf16 multiplies
+// Quad form for 1..8 token rows of a wide 4-bit or 2-bit matrix.  v_mfma_f32_4x4x4_16b_bf16 multiplies
 // sixteen independent 4x4x4 blocks, one per quad of lanes.  Block b takes the K positions of the
 // 16-byte code chunks b, b + 16, ... of a row, so the lanes of a wave read 4 weight rows x 256
 // contiguous bytes per load, and the x values a lane meets never change: they stay in registers
-// as the A operand (lane (b, r) holds token r), pre-ordered for the code pairing of expand_q4,
-// next to their per-chunk sums.  The B operand is the chunk's codes of weight row c = lane % 4 as
-// the bf16 numbers 8 + q/2, so the result D[token, row] puts ONE weight row in a lane (its four
+// as the A operand (lane (b, r) holds token r), in the order and at the scale of
+// matmul_row8, next to their per-chunk sums.  The B operand is the chunk's codes of weight row c = lane % 4 as bf16
+// subnormals (mf_device.h), so the result D[token, row] puts ONE weight row in a lane (its four
 // token sums in four registers) and the group's scale is a per-lane scalar:
-//   acc[t] += 2 s * (sum x (8 + q/2))            4 fma per chunk
-//   acc[t] += b * sum(x) - 16 s * sum(x)         two more matrix instructions per chunk (sum(x) as
+//   acc[t] += 2^65 s * (sum x q)                 4 fma per chunk
+//   acc[t] += b * sum(x)                         one more matrix instruction per chunk (sum(x) as
 //                                                three bf16 terms: exact products)
-// Every token count 1..4 runs the same instructions on its own A rows: a token's result does
-// not depend on how many tokens ride along.  The waves of a workgroup split the chunks of a row
+// Every token count runs the same instructions on its own A rows: a token's result does
+// not depend on how many tokens ride along; rows 4.. are workgroups of their own (blockIdx.y), which meet those of rows 0..3 in
+// the L2.  The waves of a workgroup split the chunks of a row
 // set (4 rows); partial sums meet in LDS in a fixed order.
+//
+// Bound by how long a stage waits for its loads: codes are requested two stages ahead into the registers that the stage has just
+// read (an empty scheduling barrier keeps every request there: left alone the compiler gathers them behind the last product), a
+// stage's table pieces two stages ahead into registers and to LDS one stage ahead -- written in the stage that requested
+// them they made it wait out a whole round trip -- and a request is a scalar base and a constant offset per lane.  4-bit MLP of 5120 x 17408,
+// one / four rows: 43.4 / 47.3 -> 39.5 / 43.5 us; 2-bit 40.8 / 45.2 -> 35.3 / 40.1; 4-bit 4096 x 12800 30.5 / 33.2 -> 26.6 / 29.4.
 struct RowsQuadArgs {
   const uint8_t* W[2];
   const uint16_t* S[2];
   const uint16_t* B[2];
   const uint16_t* x;   // [T, N]
   void* y;             // NPROJ 1: [T, M] bf16 or fp32; NPROJ 2: act [T, M] bf16
-  uint32_t M, N, T;    // M % 4 == 0, N % 64 == 0, T <= 4
+  uint32_t M, N, T;    // M % 4 == 0, N % 64 == 0, T <= 4 gridDim.y
   int out_f32;
 };
 
@@ -520,12 +527,16 @@ constexpr uint32_t kQuadMaxWaves = 8;
 constexpr uint32_t kQuadTabBytes = 2 * 64 * 8 * sizeof(uint16_t);
 __host__ __device__ constexpr uint32_t quad_wave_bytes(int nproj) { return kQuadTabBytes + 2u * nproj * 4 * 4 * 4 * sizeof(float); }
 
-// BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group -- and its codes enter as 4 + q.
+// BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group.
 // ANY: K is any multiple of 64; otherwise of 512, so that the table pieces are whole and aligned.
 template <int BITS, int NPROJ, int ITS, bool ANY>
-__global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const RowsQuadArgs a) {
+__global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadArgs a) {
+  // this workgroup's four token rows
+  a.x += 4 * static_cast<size_t>(blockIdx.y) * a.N;
+  a.y = static_cast<uint8_t*>(a.y) + 4 * static_cast<size_t>(blockIdx.y) * a.M * (a.out_f32 ? 4 : 2);
+  a.T = min(a.T - 4 * blockIdx.y, 4u);
   using chunk_t = std::conditional_t<BITS == kBits4, uint4, uint2>;
-  constexpr uint32_t kScaleStep = BITS == kBits4 ? 0x0200u : 0x0100u;  // bf16 exponent of the offset: 16 or 4
+  constexpr float kScaleMul = BITS == kBits4 ? 0x1p65f : 0x1p63f;  // q * 2^-129 or q * 2^-127 meets x * 2^64
   // LDS, sized for the waves there are (a workgroup of one wave that held room for eight left six to a CU: gate / up of
   // 2-bit 6656 x 2048, one row, 10.8 -> 8.5 us; 4-bit 17408 x 2112 19.1 -> 14.7).  Per wave, so that no address depends on
   // their number: scale / bias pieces [ring slot][(table, row, piece)][8 groups], partial sums
@@ -540,12 +551,14 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   const uint32_t n_chunks = a.N / 32, ng = a.N / kGroup, n_sets = a.M / 4;
   const size_t row_bytes = static_cast<size_t>(a.N) * BITS / 8;
 
-  // chunk of every slot of this lane: (wsub * ITS + j) * 16 + b
-  uint32_t chc[ITS];
+  // byte offset, within a set of four rows, of every slot of this lane: row c, chunk (wsub * ITS + j) * 16 + b
+  // (a set's address is the same for all lanes: a request is this offset against a scalar base, no vector arithmetic)
+  uint32_t slot_at[ITS];
   uint2 xa[ITS][8], sx[ITS];  // this lane's x operands and chunk sums (filled below)
 #pragma unroll
   for (int j = 0; j < ITS; ++j)
-    chc[j] = min((wsub * ITS + j) * 16 + b, n_chunks - 1);  // a slot past the row reads the last chunk against x = 0
+    slot_at[j] = c * static_cast<uint32_t>(row_bytes) +
+                 min((wsub * ITS + j) * 16 + b, n_chunks - 1) * static_cast<uint32_t>(sizeof(chunk_t));  // a slot past the row reads the last chunk against x = 0
 
   // Codes and table entries of two stages (a stage = one projection of one row set) live in a
   // ring of registers: a slot is refilled, as soon as it has been used, with the same slot of
@@ -557,6 +570,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   // each slot from there (LDS reads cost no vector-memory issue slot,
   // which is what limits this kernel).
   chunk_t cw[2][ITS];
+  uint4 tbr[2];
   // (lanes past 8 * ITS fetch and store a copy nobody reads: no branch around the load)
   const uint32_t tb_lane = lane % (8 * ITS);
   const uint32_t tb_bias = tb_lane / (4 * ITS), tb_row = (tb_lane / ITS) & 3u, tb_piece = tb_lane % ITS;
@@ -566,8 +580,8 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   const uint32_t tb_drop = ANY && tb_g < ng ? tb_g - tb_group : 0u;
   uint16_t* my_tab = reinterpret_cast<uint16_t*>(s_quad + wsub * kWaveFloats);
   auto fetch = [&](int buf, int j, uint32_t set, int p) __attribute__((always_inline)) {
-    const size_t row = static_cast<size_t>(set) * 4 + c;
-    cw[buf][j] = *reinterpret_cast<const chunk_t*>(a.W[p] + row * row_bytes + static_cast<size_t>(chc[j]) * sizeof(chunk_t));
+    const uint8_t* rows = a.W[p] + static_cast<size_t>(set) * 4 * row_bytes;
+    cw[buf][j] = *reinterpret_cast<const chunk_t*>(rows + slot_at[j]);
   };
   auto fetch_tables = [&](uint32_t set, int p) __attribute__((always_inline)) {
     const uint16_t* piece = (tb_bias ? a.B[p] : a.S[p]) + (static_cast<size_t>(set) * 4 + tb_row) * ng + tb_group;
@@ -580,43 +594,40 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
     uint16_t* tab = my_tab + buf * (64 * 8);
     __builtin_amdgcn_wave_barrier();  // the wave reads back what its own lanes wrote (LDS keeps order)
-    uint4 tbn = make_uint4(0, 0, 0, 0);
+    tbr[buf] = fetch_tables(refill, p);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < ITS; ++j) {
       f32x4_t tmp = {0.0f, 0.0f, 0.0f, 0.0f};
+      auto eight = [&](int i, const uint4& e) __attribute__((always_inline)) {  // eight codes
+        tmp = mfma_quad(xa[j][2 * i], make_uint2(e.x, e.y), tmp);
+        tmp = mfma_quad(xa[j][2 * i + 1], make_uint2(e.z, e.w), tmp);
+      };
       if constexpr (BITS == kBits4) {
         const uint32_t w[4] = {cw[buf][j].x, cw[buf][j].y, cw[buf][j].z, cw[buf][j].w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint4 e = expand_q4(w[i]);
-          tmp = mfma_quad(xa[j][2 * i], make_uint2(e.x, e.y), tmp);
-          tmp = mfma_quad(xa[j][2 * i + 1], make_uint2(e.z, e.w), tmp);
-        }
+        for (int i = 0; i < 4; ++i) eight(i, subnormal_q4(w[i]));
       } else {
         const uint32_t w[2] = {cw[buf][j].x, cw[buf][j].y};
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           uint4 e, f;
-          expand_q2(w[i], e, f);
-          tmp = mfma_quad(xa[j][4 * i], make_uint2(e.x, e.y), tmp);
-          tmp = mfma_quad(xa[j][4 * i + 1], make_uint2(e.z, e.w), tmp);
-          tmp = mfma_quad(xa[j][4 * i + 2], make_uint2(f.x, f.y), tmp);
-          tmp = mfma_quad(xa[j][4 * i + 3], make_uint2(f.z, f.w), tmp);
+          subnormal_q2(w[i], e, f);
+          eight(2 * i, e);
+          eight(2 * i + 1, f);
         }
       }
       const uint32_t sb = tab[((c * ITS) + j) * 8 + (b >> 1)], bb = tab[(((4 + c) * ITS) + j) * 8 + (b >> 1)];
-      const uint32_t ms = ((sb + kScaleStep) ^ 0x8000u) & 0xFFFFu;  // -16 s (-4 s): exponent + 4 (2), sign flipped
-      acc = mfma_quad(sx[j], make_uint2(bb | (bb << 16), bb), acc);
-      acc = mfma_quad(sx[j], make_uint2(ms | (ms << 16), ms), acc);
-      const float s2 = (BITS == kBits4 ? 2.0f : 1.0f) * __uint_as_float(sb << 16);
+      const float s2 = kScaleMul * __uint_as_float(sb << 16);
       fetch(buf, j, refill, p);
-      if (j == 0) tbn = fetch_tables(refill, p);
+      acc = mfma_quad(sx[j], make_uint2(bb | (bb << 16), bb), acc);
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc[t] = __builtin_fmaf(s2, tmp[t], acc[t]);
+      __builtin_amdgcn_sched_barrier(0);  // a request stays where its registers fall free
     }
-    // every read of this ring slot's tables is issued: the refill stage's pieces take their place
+    // the next stage's pieces, requested a stage ago, to LDS
     __builtin_amdgcn_wave_barrier();
-    *reinterpret_cast<uint4*>(tab + lane * 8) = ANY ? drop_bf16(tbn, tb_drop) : tbn;
+    *reinterpret_cast<uint4*>(my_tab + (buf ^ 1) * (64 * 8) + lane * 8) = ANY ? drop_bf16(tbr[buf ^ 1], tb_drop) : tbr[buf ^ 1];
     float v[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -672,14 +683,12 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint4 v = make_uint4(0, 0, 0, 0);
-      if (live) v = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + chc[j] * 32 + 8 * i);
-      xa[j][2 * i] = make_uint2(__builtin_amdgcn_perm(v.z, v.x, 0x05040100u),   // (e0, e4)
-                                __builtin_amdgcn_perm(v.z, v.x, 0x07060302u));  // (e1, e5)
-      xa[j][2 * i + 1] = make_uint2(__builtin_amdgcn_perm(v.w, v.y, 0x05040100u),   // (e2, e6)
-                                    __builtin_amdgcn_perm(v.w, v.y, 0x07060302u));  // (e3, e7)
-      const uint32_t pr[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum = (sum + bf16_lo(pr[e])) + bf16_hi(pr[e]);
+      if (live) v = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + ch * 32 + 8 * i);
+      float part;
+      const uint4 o = matmul_row8(v, &part);
+      xa[j][2 * i] = make_uint2(o.x, o.y);
+      xa[j][2 * i + 1] = make_uint2(o.z, o.w);
+      sum += part;
     }
     const uint32_t hi = __float_as_uint(sum) & 0xFFFF0000u;
     const float r1 = sum - __uint_as_float(hi);
@@ -689,7 +698,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(const Row
   }
 
   *reinterpret_cast<uint4*>(my_tab + lane * 8) = ANY ? drop_bf16(t0, tb_drop) : t0;
-  *reinterpret_cast<uint4*>(my_tab + 64 * 8 + lane * 8) = ANY ? drop_bf16(t1, tb_drop) : t1;
+  tbr[1] = t1;
   if constexpr (NPROJ == 2) {
     for (; set < n_sets; set += G) {
       const uint32_t nxt = min(set + G, last);
@@ -949,20 +958,22 @@ QuadFit rows_quad_split(uint32_t m, uint32_t n, uint32_t& its, uint32_t& wpr) {
 
 template <int BITS, int NPROJ>
 hipError_t launch_rows_quad(hipStream_t s, const RowsQuadArgs& a, QuadFit fit, uint32_t its, uint32_t wpr, uint32_t num_cu) {
-  const uint32_t n_sets = a.M / 4;
-  const dim3 grid(std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / wpr))), block(wpr * 64);
+  const uint32_t n_sets = a.M / 4, blocks = (a.T + 3) / 4;
+  const dim3 grid(std::min<uint32_t>(n_sets, num_cu * std::max(1u, 8u / wpr) / blocks), blocks), block(wpr * 64);
   const uint32_t lds = wpr * quad_wave_bytes(NPROJ);
+#define MF_QUAD(I, A) rows_quad_kernel<BITS, NPROJ, I, A><<<grid, block, lds, s>>>(a)
   if (fit == QuadFit::kEven) {
-    if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, false><<<grid, block, lds, s>>>(a);
-    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, false><<<grid, block, lds, s>>>(a);
-    else rows_quad_kernel<BITS, NPROJ, 6, false><<<grid, block, lds, s>>>(a);
+    if (its == 4) MF_QUAD(4, false);
+    else if (its == 5) MF_QUAD(5, false);
+    else MF_QUAD(6, false);
   } else {
-    if (its == 2) rows_quad_kernel<BITS, NPROJ, 2, true><<<grid, block, lds, s>>>(a);
-    else if (its == 3) rows_quad_kernel<BITS, NPROJ, 3, true><<<grid, block, lds, s>>>(a);
-    else if (its == 4) rows_quad_kernel<BITS, NPROJ, 4, true><<<grid, block, lds, s>>>(a);
-    else if (its == 5) rows_quad_kernel<BITS, NPROJ, 5, true><<<grid, block, lds, s>>>(a);
-    else rows_quad_kernel<BITS, NPROJ, 6, true><<<grid, block, lds, s>>>(a);
+    if (its == 2) MF_QUAD(2, true);
+    else if (its == 3) MF_QUAD(3, true);
+    else if (its == 4) MF_QUAD(4, true);
+    else if (its == 5) MF_QUAD(5, true);
+    else MF_QUAD(6, true);
   }
+#undef MF_QUAD
   return hipGetLastError();
 }
 
@@ -991,11 +1002,13 @@ bool rows_lane_ordered(uint32_t m, uint32_t n, uint32_t num_cu) {
 //   gate / up 6.2 / 7.4; 19.9 / 8.7; 17408 x 4096: 10.1 / 12.2; 21.2 / 14.5, and eight 124 / 27; 2048 x 3136: 3.7 / 5.4;
 //   8.7 / 6.1);
 //   2-bit above, from 8 M weights on (6656 x 6592: 14.7 / 10.6; 34.0 / 12.1; 1024 x 6592: 4.9 / 5.1).
+// (What eight rows gain, since two blocks of rows share a launch, is more still: 2-bit 2048 x 2048 10.5 / 6.6, gate / up 13.4 / 7.7,
+// one row 3.2 / 4.9, 4.0 / 6.1: its share keeps the line where it is.)
 // Elsewhere the number of token rows decides (us per MLP, other kernels / this one): one row, where a step of
 // rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3; 3840 x 7680, a
-// sixteenth empty: 22.2 / 22.9); two to four (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25; 2048 x 6656:
-// 23.5 / 21.7); more: where the weights outweigh two launches (five rows, 2816 x 4096: 29.5 / 31.5; 3328 x 8192:
-// 46.5 / 42.8; 2-bit, 1088 x 2112: 18.9 / 19.9, 1984 x 5056: 33.6 / 28.0).
+// sixteenth empty: 22.2 / 22.9); two and more, from 4 M weights on (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25;
+// one projection, 4-bit 1088 x 4992, two, four, eight rows: 6.7 / 7.0, 13.5 / 8.0, 13.8 / 9.2; 2-bit 1024 x 6592: 7.2 / 6.1, 11.4 / 6.5,
+// 15.9 / 9.0).
 template <int BITS, int NPROJ>
 bool rows_quad_takes(QuadFit fit, uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu) {
   constexpr bool two = BITS == kBits2;
@@ -1007,27 +1020,24 @@ bool rows_quad_takes(QuadFit fit, uint32_t m, uint32_t n, uint32_t t, uint32_t n
   if (fit == QuadFit::kEven) return true;
   if (rows_lane_ordered<BITS, NPROJ>(m, n, num_cu)) return weights >= (two ? 8ull : 8ull * NPROJ) * 1000000;
   const uint32_t steps = (n + step - 1) / step;
-  const bool wide = weights >= (two ? 8ull : 24ull) * 1000000;
-  return t == 1 ? wide && n * 5ull < steps * static_cast<uint64_t>(step) * 4 : t <= 4 ? weights >= 4000000 : wide;
+  if (t > 1) return weights >= 4000000;
+  return weights >= (two ? 8ull : 24ull) * 1000000 && n * 5ull < steps * static_cast<uint64_t>(step) * 4;
 }
 
-// Up to four token rows in one launch.  Five to eight: two launches, rows 0..3 and the
-// rest.  The quad kernel runs the same instructions for a token whatever rides along, so every row
-// keeps the bits of a single-token call (MultiXKernelParityTests.swift:50-77); the weights stream
-// twice.  (y rows are M elements apart, 2 or 4 bytes each: 16-byte aligned since M % 4 == 0.)
+// Up to four token rows on one set of workgroups, five to eight on two, in one launch: half of the workgroups each, which read
+// the same weights at the same time (4-bit MLP of 5120 x 17408, five / eight rows: two launches 77.8 / 84.1 us, one 55.8 / 58.7;
+// 2048 x 6400 31.3 / 35.4, 24.4 / 27.7.  Both blocks' operands in one wave's registers, so that the codes are expanded once: 24.3 / 28.8
+// against 20.0 / 22.2 for 3136 x 4096, and five chunks a wave do not fit).
+// The quad kernel runs the same instructions for a token whatever rides along, so every row
+// keeps the bits of a single-token call (MultiXKernelParityTests.swift:50-77).
+// (y rows are M elements apart, 2 or 4 bytes each: 16-byte aligned since M % 4 == 0.)
 template <int BITS, int NPROJ>
 bool rows_quad_try(hipStream_t s, const RowsQuadArgs& a, uint32_t num_cu, hipError_t& err) {
   if (a.T < 1 || a.T > 8) return false;
   uint32_t its = 0, wpr = 0;
   const QuadFit fit = rows_quad_split(a.M, a.N, its, wpr);
   if (!rows_quad_takes<BITS, NPROJ>(fit, a.M, a.N, a.T, num_cu)) return false;
-  for (uint32_t t0 = 0; t0 < a.T && err == hipSuccess; t0 += 4) {
-    RowsQuadArgs q = a;
-    q.T = std::min(a.T - t0, 4u);
-    q.x = a.x + static_cast<size_t>(t0) * a.N;
-    q.y = static_cast<uint8_t*>(a.y) + static_cast<size_t>(t0) * a.M * (a.out_f32 ? 4 : 2);
-    err = launch_rows_quad<BITS, NPROJ>(s, q, fit, its, wpr, num_cu);
-  }
+  err = launch_rows_quad<BITS, NPROJ>(s, a, fit, its, wpr, num_cu);
   return true;
 }
 

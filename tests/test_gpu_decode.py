@@ -1191,8 +1191,8 @@ def test_int8_matmul_passes_infinities_on(gpu, d, f, t):
 
 @pytest.mark.parametrize("bits,m,n,t", [(4, 1024, 5120, 3), (4, 12800, 3136, 8), (2, 9408, 2560, 4), (2, 1216, 6592, 7)])
 def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
-    """an infinity or a NaN makes its own token's results NaN (the code offset is taken out as inf - inf, as in every row
-    kernel of these formats) and leaves the other tokens' bits alone"""
+    """an infinity or a NaN makes its own token's results NaN (as in every row kernel of these formats) and leaves the
+    other tokens' bits alone; rows times a power of two, of either block of four, give the results times it"""
     gen = torch.Generator(device="cuda")
     gen.manual_seed(n + t)
     table = lambda s: (s * (0.01 + 0.01 * torch.rand(m, n // 64, generator=gen, device="cuda"))).to(torch.bfloat16)
@@ -1200,10 +1200,11 @@ def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
     x, wild, at = _wild_rows(gen, t, n)
     g = ops.DequantInt4GEMVMultiX(gpu)
     out = []
-    for rows in (x, wild):
+    for rows in (x, wild, x * 2.0 ** 48, x * 2.0 ** -48):
         y = torch.zeros((t, m), dtype=torch.float32, device="cuda")
         g.encode(q, rows, y, m, n, t, output_float32=True)
         out.append(y)
+    assert torch.equal(out[2], out[0] * 2.0 ** 48) and torch.equal(out[3], out[0] * 2.0 ** -48)
     others = [i for i in range(t) if i not in at]
     assert torch.equal(out[0][others].view(torch.int32), out[1][others].view(torch.int32))
     assert torch.isnan(out[1][at]).all() and torch.isfinite(out[0]).all()
