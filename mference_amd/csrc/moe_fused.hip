@@ -9,10 +9,10 @@
 //   B  routed gate/up/activation rows of the K selected experts of every token
 //   C  the workgroups are split among the tokens, each owns output rows of one: the
 //      shared expert's down rows of those rows (-> gated h1, kept in LDS), then the
-//      routed down rows.  With one or two units of rows per workgroup K waves take the
-//      K slots of a unit, weight them, and one thread per row adds them to h1 in rank
-//      order; with three and more a wave takes all K slots of its units one after the
-//      other, four rows requested ahead.
+//      routed down rows.  A wave takes one slot of a unit of rows and weights its values; one
+//      thread per row adds a row's K values to h1 in rank order.  With one or two units per
+//      workgroup they go round by round, with three and more a wave takes its share of all
+//      (unit, slot) pairs, four requested ahead.
 //
 // Workgroups exchange three small vectors through HBM: logits, shared
 // activations, routed activations.  There is no grid barrier.  Every exchanged
@@ -67,31 +67,41 @@ constexpr uint32_t kMaxH1 = 2048;          // output rows of one token a workgro
 
 // A lane's step of a row: codes and the table entries of its group as they come from memory.  The entries become
 // numbers where they are used (scale(), bias()), behind an empty asm statement: converted next to their load they
-// would be waited for there, in front of everything that was to run while they are on their way.
+// would be waited for there, in front of everything that was to run while they are on their way.  They stay 16 bits
+// wide until then for the same reason: widened in front of a loop's branch back, they are waited for at that branch.
 template <int BITS> struct Chunk {
   uint4 codes;
-  uint32_t sraw, braw;
+  uint16_t sraw, braw;
   __device__ __forceinline__ float scale() const {
-    uint32_t r = sraw;
+    uint16_t r = sraw;
     asm volatile("" : "+v"(r));
-    return __uint_as_float(r << 16);
+    return bf16_to_f(r);
   }
   __device__ __forceinline__ float bias() const {
     if constexpr (BITS == kBitsTernary) return -scale();
-    uint32_t r = braw;
+    uint16_t r = braw;
     asm volatile("" : "+v"(r));
-    return __uint_as_float(r << 16);
+    return bf16_to_f(r);
   }
 };
+
+template <class T>
+__device__ __forceinline__ const __attribute__((address_space(1))) T* global_ptr(const void* p) {
+  return reinterpret_cast<const __attribute__((address_space(1))) T*>(reinterpret_cast<uint64_t>(p));
+}
 
 template <int BITS>
 __device__ __forceinline__ Chunk<BITS> load_chunk(const uint8_t* wrow, const uint16_t* srow,
                                                   const uint16_t* brow, uint32_t e0) {
   Chunk<BITS> c;
-  c.codes = load_codes16<true>(wrow + static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
-  c.sraw = srow[e0 / kGroup];
+  // (global loads by name: a base made of two readlanes is a flat address to the compiler, and a flat load in flight is
+  // waited for with every LDS read)
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const u32x4 q = *global_ptr<u32x4>(wrow + static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
+  c.codes = make_uint4(q.x, q.y, q.z, q.w);
+  c.sraw = *global_ptr<uint16_t>(srow + e0 / kGroup);
   if constexpr (BITS == kBitsTernary) c.braw = 0;
-  else c.braw = brow[e0 / kGroup];
+  else c.braw = *global_ptr<uint16_t>(brow + e0 / kGroup);
   return c;
 }
 
@@ -306,18 +316,21 @@ constexpr uint32_t fused_b_per_wg(uint32_t epl, uint32_t d, uint32_t f, uint32_t
 }
 
 // How stage C deals a token's output rows.  Rows form: a unit's K slots on K waves, their values meet in LDS -- all
-// waves work although a workgroup has only a unit or two.  Units form: a wave takes all K slots of a unit one after
-// the other with four rows requested ahead, no meeting -- from three units per workgroup on (large 2-bit layer, one
-// token: 8 units; most shapes at several tokens), while a row is one step of 64 lanes and the slices of the
-// activations are at most one a thread.
+// waves work although a workgroup has only a unit or two.  Units form: the (unit, slot) pairs of all units go to the
+// waves in turn with four requested ahead, and all values meet once -- from three units per workgroup on (large 2-bit
+// layer, one token: 8 units; most shapes at several tokens), while a row is one step of 64 lanes and the slices of the
+// activations are at most one a thread.  (With a unit's slots on one wave, one after the other, eleven waves of sixteen
+// worked at five tokens of the Qwen shape, and six of sixteen at one token of the 2816 x 704 layer.)  Launch, us, before
+// and now: Qwen shape 16.0 / 15.2 (two tokens), 26.7 / 26.2 (five), 32.2 / 31.1 (six); large 2-bit layer 52.3 / 50.2
+// (two), 145 / 138 (eight); ternary layer of 256 experts 18.4 / 17.3 (four).
 struct FusedSplit {
   bool by_units;
   uint32_t wgs, units, rounds;  // workgroups per token; units per workgroup (rows form: and round); rounds
 };
-constexpr FusedSplit fused_split(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg) {
+constexpr FusedSplit fused_split(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg, bool units_fit = true) {
   const uint32_t rpw = static_rows_per_wave(f, epl), rg = (d + rpw - 1) / rpw, wgs = n_wg / t;
   const uint32_t share = (rg + wgs - 1) / wgs;
-  const bool by_units = share >= 3 && f <= 64 * epl && k * (f / epl) <= kFusedThreads;
+  const bool by_units = units_fit && share >= 3 && f <= 64 * epl && k * (f / epl) <= kFusedThreads;
   const uint32_t per_round = kFusedWaves / k < share ? kFusedWaves / k : share;
   const uint32_t units = by_units ? share : per_round;
   return FusedSplit{by_units, wgs, units, by_units ? 1 : (rg + wgs * units - 1) / (wgs * units)};
@@ -710,7 +723,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   const uint32_t slpr = 1u << slpr_log2, srpw = 64u >> slpr_log2;
 
   // What the router decided is all a down row needs to be requested: the first codes leave before anything is
-  // waited for.  Rows form: slot wv % K of unit wv / K of the first round.  Units form: a wave walks
+  // waited for.  Rows form: slot wv % K of unit wv / K of the first round.  Units form: pair wv, wv + 16, ... of the
   // (unit, slot) pairs, slots fastest; four of them are in flight.
   constexpr uint32_t kEPLF = Fmt<BITS>::kElemsPer16B;
   constexpr int kRing = UNITS ? 4 : 1;
@@ -718,28 +731,34 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   const uint32_t e0 = sub * kEPLF;
   const bool lane_in = e0 < F;
   const uint32_t e0c = lane_in ? e0 : 0u;
-  // rows form
+  // (unit, slot) of the wave's first pair: of the round in the rows form, of all in the units form
   const uint32_t unit_local = S::K != kDyn ? wv / K : fdiv(wv, a.g.K), slot = wv - unit_local * K;
   // units form: the slots' blobs and weights, a slot per lane
   uint32_t base_lo = 0, base_hi = 0;
   float w_lane = 0.0f;
-  uint32_t f_unit = wv, f_slot = 0;               // the next (unit, slot) to request
   const uint32_t u_first = wl * ub, u_n = u_first < rg_per_tok ? (rg_per_tok - u_first < ub ? rg_per_tok - u_first : ub) : 0;
-  const uint32_t n_mine = UNITS ? (wv < u_n ? (u_n - wv + kFusedWaves - 1) / kFusedWaves : 0u) * K : 0u;
+  const uint32_t n_pairs = u_n * K, n_mine = UNITS && wv < n_pairs ? (n_pairs - wv + kFusedWaves - 1) / kFusedWaves : 0u;
+  const uint32_t step_units = S::K != kDyn ? kFusedWaves / K : fdiv(kFusedWaves, a.g.K), step_slots = kFusedWaves - step_units * K;
+  uint32_t f_unit = unit_local, f_slot = slot;    // the next (unit, slot) to request
   auto request = [&](const uint8_t* blob, uint32_t row) __attribute__((always_inline)) {
     const uint32_t rc = row < D ? row : 0u;
     return load_chunk<BITS>(blob + a.off.down_w + rc * rb,
                             reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + static_cast<size_t>(rc) * ng,
                             reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + static_cast<size_t>(rc) * ng, e0c);
   };
+  auto next_pair = [&](uint32_t& unit, uint32_t& sl) __attribute__((always_inline)) {
+    unit += step_units;
+    sl += step_slots;
+    if (sl >= K) {
+      sl -= K;
+      ++unit;
+    }
+  };
   auto fetch_unit = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
     const uint64_t base = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_hi), f_slot))) << 32) |
                           static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base_lo), f_slot));
     c = request(reinterpret_cast<const uint8_t*>(base), ((u_first + (f_unit < u_n ? f_unit : 0u)) << rpw_log2) + rloc);
-    if (++f_slot == K) {
-      f_slot = 0;
-      f_unit += kFusedWaves;
-    }
+    next_pair(f_unit, f_slot);
   };
   auto fetch_first = [&](Chunk<BITS>& c) __attribute__((always_inline)) {
     const uint32_t unit = wl * ub + unit_local;
@@ -1002,27 +1021,19 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       }
       __syncthreads();
       const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
-      const uint32_t my_expert = lane < K ? s_idx[tok * K + lane] : E;
+      const uint64_t live = __ballot((lane < K ? s_idx[tok * K + lane] : E) < E);
       w_lane = lane < K ? s_w[tok * K + lane] : 0.0f;
-      const unsigned long long live = __ballot(my_expert < E);
-      uint32_t c_unit = wv, c_slot = 0;  // the (unit, slot) at hand
-      float acc = 0.0f;
+      float* s_pv = reinterpret_cast<float*>(s_xq);  // [unit][slot][row of the unit]; the x slices have had their use
+      uint32_t c_unit = unit_local, c_slot = slot;   // the (unit, slot) at hand
       auto take = [&](const Chunk<BITS>& c) __attribute__((always_inline)) {
-        if (c_slot == 0) acc = Fs ? s_h1[(c_unit << rpw_log2) + rloc] : 0.0f;
         const XSlice<BITS> xs =
             load_xslice_lds<BITS>(reinterpret_cast<const uint4*>(s_acts), s_asum, 0, act_ld, c_slot * spl + (lane_in ? sub : 0u));
         float part = __builtin_fmaf(c.scale(), codes_dot<BITS>(c.codes, xs), 0.0f);  // the one step of row_partial
         part = __builtin_fmaf(c.bias(), xs.sum, part);
         const float v = group_sum(lane_in ? part : 0.0f, static_cast<int>(lpr));
-        // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first); sums in rank order
-        const float wgt = readlane_f(w_lane, static_cast<int>(c_slot));
-        if ((live >> c_slot) & 1ull) acc = acc + wgt * (maple ? round_bf16(v) : v);
-        if (++c_slot == K) {
-          const uint32_t row = ((u_first + c_unit) << rpw_log2) + rloc;
-          if (sub == 0 && row < D) store_row(row, acc, failed);
-          c_slot = 0;
-          c_unit += kFusedWaves;
-        }
+        // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first)
+        if (sub == 0) s_pv[((c_unit * K + c_slot) << rpw_log2) + rloc] = readlane_f(w_lane, static_cast<int>(c_slot)) * (maple ? round_bf16(v) : v);
+        next_pair(c_unit, c_slot);
       };
       uint32_t n = 0;
       for (; n + 2 * kRing <= n_mine; n += kRing) {
@@ -1032,12 +1043,31 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
           fetch_unit(ring[i]);
         }
       }
-      for (; n < n_mine; ++n) {
-        take(ring[0]);
-        ring[0] = ring[1];
-        ring[1] = ring[2];
-        ring[2] = ring[3];
-        if (n + kRing < n_mine) fetch_unit(ring[3]);
+      // what is left: up to four that are on their way and up to three that are not (no register with a request on its
+      // way is moved: that would wait for it)
+#pragma unroll
+      for (int i = 0; i < kRing; ++i) {
+        if (n + i < n_mine) take(ring[i]);
+        if (n + kRing + i < n_mine) fetch_unit(ring[i]);
+      }
+      n += kRing;
+#pragma unroll
+      for (int i = 0; i + 1 < kRing; ++i)
+        if (n + i < n_mine) take(ring[i]);
+      __syncthreads();
+      for (uint32_t i = threadIdx.x; i < u_n << rpw_log2; i += kFusedThreads) {  // sums in rank order, residual first
+        const uint32_t row = (u_first << rpw_log2) + i;
+        if (row < D) {
+          const float* pv = s_pv + (((i >> rpw_log2) * K) << rpw_log2) + (i & (rpw - 1));
+          float vk[MF_MAX_TOPK];
+#pragma unroll
+          for (uint32_t k = 0; k < MF_MAX_TOPK; ++k) vk[k] = pv[(k < K ? k : 0u) << rpw_log2];
+          float acc = Fs ? s_h1[i] : 0.0f;
+#pragma unroll
+          for (uint32_t k = 0; k < MF_MAX_TOPK; ++k)
+            if ((live >> k) & 1ull) acc = acc + vk[k];
+          store_row(row, acc, failed);
+        }
       }
     } else {
       for (uint32_t round = 0; round < rounds; ++round) {
@@ -1107,10 +1137,6 @@ static uint32_t fused_epl(const mf_moe_config& c) { return c.bits == MF_BITS_4 ?
 static uint32_t fused_b_per_wg(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
   return fused_b_per_wg(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
 }
-static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
-  return fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
-}
-
 static FusedGeo fused_geo(const mf_moe_config& c, uint32_t num_cu, uint32_t t, const FusedSplit& sp) {
   const uint32_t epl = fused_epl(c), sepl = c.shared_bits == MF_BITS_4 ? 32 : 64;
   FusedGeo g{};
@@ -1154,13 +1180,23 @@ static size_t fused_lds_base(const mf_moe_config& c, uint32_t num_cu, uint32_t t
          4 * (sact_words + acts_words + fused_stage_words(c, num_cu, t));
 }
 constexpr size_t kFusedLdsLimit = 150 * 1024;
+// units form of stage C: a value per slot and output row of a workgroup, where the x slices were
+static uint32_t fused_pv_words(const mf_moe_config& c, const FusedSplit& sp) {
+  return sp.by_units ? sp.units * (64u >> lanes_per_row_log2_dev(c.f, fused_epl(c))) * c.top_k : 0;
+}
+static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
+  FusedSplit sp = fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
+  if (fused_lds_base(c, num_cu, t) + 4 * static_cast<size_t>(fused_pv_words(c, sp)) > kFusedLdsLimit)
+    sp = fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu, false);
+  return sp;
+}
 // the x slices are kept in LDS when they fit beside everything else
 static bool fused_xprep(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
   return fused_lds_base(c, num_cu, t) + 4 * static_cast<size_t>(fused_xprep_words(c, t)) <= kFusedLdsLimit;
 }
 size_t fused_lds_bytes(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
-  const size_t base = fused_lds_base(c, num_cu, t);
-  return fused_xprep(c, num_cu, t) ? base + 4 * static_cast<size_t>(fused_xprep_words(c, t)) : base;
+  const size_t pv = fused_pv_words(c, fused_split(c, num_cu, t)), xs = fused_xprep(c, num_cu, t) ? fused_xprep_words(c, t) : 0;
+  return fused_lds_base(c, num_cu, t) + 4 * std::max(pv, xs);
 }
 
 bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void* x, const void* y,

@@ -389,6 +389,31 @@ def test_decode_layer_matches_oracle(gpu, oracle, bits, d, f, e, k, fs, t):
     assert np.array_equal(results[True], results[False])
 
 
+@pytest.mark.parametrize("bits,d,f,e,k,fs,t", [
+    (4, 512, 512, 16, 3, 0, 8),      # four units of rows a workgroup, twelve (unit, slot) pairs: four waves have none
+    (4, 1088, 320, 20, 5, 64, 8),    # nine units, the last workgroup of a token one short: two or three pairs a wave
+    (4, 832, 704, 16, 6, 0, 7),      # steps of K = 6 through sixteen waves
+    (4, 4096, 1024, 16, 8, 0, 8),    # 32 pairs a wave: the loop with requests in flight
+    (2, 1600, 1024, 12, 7, 128, 8),  # ten or eleven: the loop and a remainder of three
+    (1, 2048, 512, 32, 1, 0, 8),     # one slot
+])
+def test_down_rows_dealt_in_pairs(gpu, oracle, bits, d, f, e, k, fs, t):
+    """The fused launch deals a workgroup's (unit of output rows, slot) pairs to its waves and adds a row's values in
+    rank order; the chain of launches takes a row's slots one after the other.  Same products, same order: same bits."""
+    layer = oracle.synth_layer(ROOT_SEED + 0x9200 + bits, d, f, e, k, bits=bits, fs=fs)
+    x = ops.bf16_tensor(oracle.synth_x(ROOT_SEED + 0x9201, t, d))
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    out = []
+    for fused in (True, False):
+        moe.set_fused(fused)
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        moe.encode_decode_layer(wts, x, y, t=t)
+        moe.status()
+        out.append(ops.bf16_bits(y))
+    assert np.array_equal(*out)
+    assert np.isfinite(oracle.bf16_to_float(out[0])).all() and out[0].any()
+
+
 def test_decode_layer_residual_add_in_place(gpu, oracle):
     d, f, e, k, fs, t = 256, 128, 16, 4, 128, 2
     root = ROOT_SEED + 0x9100
