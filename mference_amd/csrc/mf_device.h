@@ -551,6 +551,8 @@ __device__ __forceinline__ uint4 load_bf16x8_guarded(const uint16_t* p, uint32_t
   return make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
 }
 
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
 // The activations one lane meets, permuted for the pairing above, plus their sum.
 template <int BITS> struct XSlice {
   static constexpr int kPairs = Fmt<BITS>::kElemsPer16B / 2;
@@ -669,6 +671,156 @@ __device__ __forceinline__ float codes_dot(const uint4& codes, const XSlice<BITS
     }
     return __builtin_fmaf(-4.0f, xs.sum, dot);  // sum((4 + q) x) -> sum(q x)
   }
+}
+
+// The rows of the routed experts meet a token's slice on the matrix core: codes are bf16 subnormals at the top of a byte
+// (above; the two-bit ones at two places with a sum each), four of them per v_mfma_f32_4x4x4_16b_bf16, whose blocks
+// multiply the codes of every lane of a quad with the values of every lane of it -- the lane's own share is on the diagonal.
+// Vector instructions are what the decode launch's routed stages wait for.  Per lane, 16 bytes and SIMD (four waves):
+// codes under an offset for the two-element dot product 96 / 173 ns (4 / 2 bits), subnormals for it 80 / 139, here 67 / 122;
+// error against 64 bits on normal values 2.1e-8 with the offset, 3.9e-9 / 3.4e-9 either way here (on SwiGLU outputs 5.4e-8, 1.1e-8).
+// An expert's slice holds its values times kRowScale, in the order of the codes, and their sum unscaled.  It is made in
+// four parts of a code word each (the words of raw numbers, the same number of words out; the part's sum, scaled), whose
+// sums are added (0 + 1) + (2 + 3).  SCALED: the raw words are at that scale already.
+template <int BITS> constexpr int kPartWords = Fmt<BITS>::kElemsPer16B / 8;
+template <int BITS, bool SCALED>
+__device__ __forceinline__ float expert_x_part(const uint32_t* raw, uint32_t* p) {
+  constexpr int kSpan = kPartWords<BITS> / 2;  // words between an element and the one in the other half of a code word
+#pragma unroll
+  for (int i = 0; i < kSpan; ++i) {
+    const uint32_t lo = raw[i], hi = raw[kSpan + i];
+    uint32_t even, odd;
+    if constexpr (SCALED) {
+      even = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+      odd = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+    } else {
+      even = upper_halves(bf16_lo(lo) * kRowScale, bf16_lo(hi) * kRowScale);
+      odd = upper_halves(bf16_hi(lo) * kRowScale, bf16_hi(hi) * kRowScale);
+    }
+    // 4 bits: codes 0..3 of a half word as they come; 2 bits: codes 0, 2, 4, 6 (lower place), then 1, 3, 5, 7
+    p[BITS == kBits4 ? 2 * i : i] = even;
+    p[BITS == kBits4 ? 2 * i + 1 : 4 + i] = odd;
+  }
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 2 * kSpan; ++i) sum = dot2_bf16(p[i], kOnes, sum);
+  return sum;
+}
+// n slices by the threads of a workgroup, four adjacent ones a slice, into the layout that load_xslice_lds reads:
+// src(i, at, sum_at) gives slice i's first element, where its blocks start and where its sum goes.  first_thread, threads: who
+// takes part (multiples of 64).  A thread's straight run of code is a quarter of a slice's: cold, it is fetched line by line.
+template <int BITS, bool ALIGNED, class Src>
+__device__ __forceinline__ void stage_expert_x(uint4* xq, float* xsum, uint32_t ld, uint32_t n, uint32_t first_thread, uint32_t threads, Src src) {
+  constexpr int kW = kPartWords<BITS>;
+  for (uint32_t i = threadIdx.x - first_thread; i < 4 * n; i += threads) {
+    const uint32_t sl = i >> 2, part = i & 3u;
+    uint32_t at, sum_at;
+    const uint16_t* x = src(sl, at, sum_at) + part * (2 * kW);
+    uint32_t raw[kW], p[kW];
+#pragma unroll
+    for (int q = 0; q < kW / 4; ++q) {
+      const uint4 v = load_x8<ALIGNED>(x + 8 * q);
+      raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
+    }
+    float sum = expert_x_part<BITS, false>(raw, p);
+    sum += dpp_f<0xB1>(sum);
+    sum += dpp_f<0x4E>(sum);
+#pragma unroll
+    for (int q = 0; q < kW / 4; ++q) xq[(part * (kW / 4) + q) * ld + at] = make_uint4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+    if (part == 0) xsum[sum_at] = sum * kRowUnscale;
+  }
+}
+template <int BITS, bool ALIGNED>
+__device__ __forceinline__ XSlice<BITS> load_expert_x(const uint16_t* x) {
+  constexpr int kQuads = Fmt<BITS>::kElemsPer16B / 8;
+  uint32_t raw[kQuads * 4];
+#pragma unroll
+  for (int q = 0; q < kQuads; ++q) {
+    const uint4 a = load_x8<ALIGNED>(x + 8 * q);
+    raw[4 * q] = a.x; raw[4 * q + 1] = a.y; raw[4 * q + 2] = a.z; raw[4 * q + 3] = a.w;
+  }
+  XSlice<BITS> xs;
+  float sum[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, false>(raw + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>);
+  xs.sum = ((sum[0] + sum[1]) + (sum[2] + sum[3])) * kRowUnscale;
+  return xs;
+}
+// a slice out of its numbers as they come, at the scale already
+template <int BITS>
+__device__ __forceinline__ XSlice<BITS> permuted_expert_x(const XSlice<BITS>& raw) {
+  XSlice<BITS> xs;
+  float sum[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, true>(raw.p + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>);
+  xs.sum = ((sum[0] + sum[1]) + (sum[2] + sum[3])) * kRowUnscale;
+  return xs;
+}
+// four codes of every lane against four of its values
+__device__ __forceinline__ f32x4_t lane_mfma(uint32_t a0, uint32_t a1, uint32_t x0, uint32_t x1, f32x4_t c) {
+  typedef __attribute__((ext_vector_type(4))) short s16x4;
+  return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(s16x4, make_uint2(a0, a1)),
+                                                __builtin_bit_cast(s16x4, make_uint2(x0, x1)), c, 0, 0, 0);
+}
+__device__ __forceinline__ float lane_diagonal(const f32x4_t& c) {
+  const uint32_t i = threadIdx.x;
+  const float lo = i & 1u ? c[1] : c[0], hi = i & 1u ? c[3] : c[2];
+  return i & 2u ? hi : lo;
+}
+// sum over the lane's share of q * x.  All lanes of the wave call it (the instruction knows no inactive lanes).
+template <int BITS>
+__device__ __forceinline__ float expert_dot(const uint4& codes, const XSlice<BITS>& xs) {
+  const uint32_t ws[4] = {codes.x, codes.y, codes.z, codes.w};
+  f32x4_t c = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (BITS == kBits4) {
+    constexpr uint32_t kMask = 0x00F000F0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w = ws[j];
+      c = lane_mfma((w << 4) & kMask, w & kMask, xs.p[4 * j], xs.p[4 * j + 1], c);
+      c = lane_mfma((w >> 4) & kMask, (w >> 8) & kMask, xs.p[4 * j + 2], xs.p[4 * j + 3], c);
+    }
+    return lane_diagonal(c) * 0x1p65f;  // q * 2^-129 met x * 2^64
+  } else {
+    constexpr uint32_t kHigh = 0x00C000C0u, kLow = 0x00300030u;
+    f32x4_t l = c;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t w = ws[j], up = w << 4, d4 = w >> 4, d8 = w >> 8;
+      l = lane_mfma(up & kLow, w & kLow, xs.p[8 * j], xs.p[8 * j + 1], l);
+      c = lane_mfma(up & kHigh, w & kHigh, xs.p[8 * j + 4], xs.p[8 * j + 5], c);
+      l = lane_mfma(d4 & kLow, d8 & kLow, xs.p[8 * j + 2], xs.p[8 * j + 3], l);
+      c = lane_mfma(d4 & kHigh, d8 & kHigh, xs.p[8 * j + 6], xs.p[8 * j + 7], c);
+    }
+    return __builtin_fmaf(lane_diagonal(l), 4.0f, lane_diagonal(c)) * 0x1p63f;  // q * 2^-129 and q * 2^-127 met x * 2^64
+  }
+}
+
+// The lane slices of x a routed row meets (XSlice: permuted pairs + their sum) depend on the token
+// only, so a workgroup builds them once in LDS instead of once per row: slice sl of token t keeps
+// its pairs as 16-byte blocks xq[(t * kQ + q) * n_sl + sl] (neighbouring lanes read neighbouring
+// blocks) and its sum at xsum[t * n_sl + sl].
+template <int BITS>
+__device__ __forceinline__ void store_xslice_lds(uint4* xq, float* xsum, uint32_t t, uint32_t n_sl, uint32_t sl,
+                                                 const XSlice<BITS>& xs) {
+  constexpr uint32_t kQ = XSlice<BITS>::kPairs / 4;
+#pragma unroll
+  for (uint32_t q = 0; q < kQ; ++q)
+    xq[(t * kQ + q) * n_sl + sl] = make_uint4(xs.p[4 * q], xs.p[4 * q + 1], xs.p[4 * q + 2], xs.p[4 * q + 3]);
+  xsum[t * n_sl + sl] = xs.sum;
+}
+template <int BITS>
+__device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, const float* xsum, uint32_t t, uint32_t n_sl,
+                                                        uint32_t sl) {
+  constexpr uint32_t kQ = XSlice<BITS>::kPairs / 4;
+  XSlice<BITS> xs;
+#pragma unroll
+  for (uint32_t q = 0; q < kQ; ++q) {
+    const uint4 v = xq[(t * kQ + q) * n_sl + sl];
+    xs.p[4 * q] = v.x; xs.p[4 * q + 1] = v.y; xs.p[4 * q + 2] = v.z; xs.p[4 * q + 3] = v.w;
+  }
+  xs.sum = xsum[t * n_sl + sl];
+  return xs;
 }
 
 // convenience form: one row against a slice loaded on the spot

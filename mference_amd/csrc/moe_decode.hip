@@ -1,6 +1,8 @@
 // Routed expert decode: phase 1 (gate/up/activation), phase 2 (down + weighted
 // rank-ordered reduce) as separate launches.  Experts are resident in HBM and
 // addressed on device as expert_base + idx * expert_stride.
+#include <algorithm>
+
 #include "mf_device.h"
 #include "mf_internal.h"
 
@@ -43,6 +45,13 @@ __device__ __forceinline__ BlobView view_blob(const uint8_t* blob, const mf_expe
 // maple_moe.metal:190-221; `maple` selects its bf16-stepped activation, :153-164).
 // G32 (2-bit experts only): the gate projection's tables hold an entry per 32 weights
 // (moe_int2_gate_up_rows_simd_dev_vec with gate_group_size 32, moe.metal:962-1060); up stays at 64.
+// Both phases: the four waves of a workgroup have rows of one route (one token) and share the slices of its x (its
+// routes' activations), at most kStageSlices of them at a time; a wave that made them for itself, once per row of 64 lanes, spent
+// more on that than on the products (2-bit layer 3200 x 1088, eight tokens: 163 us a layer with the codes under an offset, 195 with the
+// slices of expert_dot made by every wave, 99 here).
+constexpr uint32_t kStageSlices = 256;
+template <int BITS> constexpr size_t stage_bytes(uint32_t slices) { return slices * (XSlice<BITS>::kPairs * 4 + 4); }
+
 template <int BITS, bool ALIGNED, bool G32 = false>
 __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__ base,
                                                      size_t stride, mf_expert_offsets off,
@@ -55,19 +64,19 @@ __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__
                                                      uint32_t lpr_log2,
                                                      const uint32_t* __restrict__ subset,
                                                      uint32_t all_pairs, const SlotMap slots) {
-  constexpr int EPL = Fmt<BITS>::kElemsPer16B;
+  constexpr uint32_t EPL = Fmt<BITS>::kElemsPer16B;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t lpr = 1u << lpr_log2;
   const uint32_t rpw = 64u >> lpr_log2;
-  const uint32_t waves_per_pair = (F + rpw - 1) / rpw;
-  uint32_t pair = wave / waves_per_pair;
-  if (pair >= pairs) return;
+  const uint32_t waves_per_pair = (F + rpw - 1) / rpw, wgs_per_pair = (waves_per_pair + 3) / 4;
+  uint32_t pair = blockIdx.x / wgs_per_pair;
+  const uint32_t wave = (blockIdx.x % wgs_per_pair) * 4 + (threadIdx.x >> 6);
   if (subset) {  // moe_phase1_gate_up_act_subset_u16load (moe.metal:531-565): only the listed slots
     pair = subset[pair];
     if (pair >= all_pairs) return;  // a slot past the table does nothing (:551)
   }
-  const uint32_t row = (wave % waves_per_pair) * rpw + (lane >> lpr_log2);
+  const uint32_t row = wave * rpw + (lane >> lpr_log2);
   const uint32_t sub = lane & (lpr - 1);
   const bool row_ok = row < F;
   if (slots.all_hit && *slots.all_hit == 0u) return;  // guarded form: nothing unless every slot was found
@@ -88,14 +97,28 @@ __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__
   const size_t row_bytes = static_cast<size_t>(D) * Store<BITS>::kBits / 8;
   const size_t r = row_ok ? row : 0;
   float ga = 0.0f, ua = 0.0f;
-  for (uint32_t e0 = sub * EPL; e0 < D; e0 += lpr * EPL) {
-    if (!row_ok) break;
+  const uint32_t n_sl = D / EPL, staged = min(n_sl, kStageSlices);
+  uint4* xq = reinterpret_cast<uint4*>(smem);
+  float* xsum = reinterpret_cast<float*>(xq + XSlice<BITS>::kPairs / 4 * staged);
+  for (uint32_t first = 0; first < D; first += lpr * EPL) {  // all lanes take every step: one without a share drops its sums
+    const bool in = row_ok && first + sub * EPL < D;
+    const uint32_t e0 = in ? first + sub * EPL : first;
     const size_t boff = r * row_bytes + static_cast<size_t>(e0) * Store<BITS>::kBits / 8;
     const uint4 gc = load_codes16<ALIGNED>(bv.gw + boff);
     const uint4 uc = load_codes16<ALIGNED>(bv.uw + boff);
-    float gs, gb, us, ub, gd, ud, sum, sum2;
+    const uint32_t sl0 = first / EPL, at = sl0 % kStageSlices;  // (lpr divides kStageSlices)
+    if (at == 0) {  // the next slices
+      if (first) __syncthreads();
+      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, min(staged, n_sl - sl0), 0, 256, [&](uint32_t i, uint32_t& at, uint32_t& sum_at) {
+        at = sum_at = i;
+        return xt + static_cast<size_t>(sl0 + i) * EPL;
+      });
+      __syncthreads();
+    }
+    const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, xsum, 0, staged, at + (e0 - first) / EPL);
+    const float ud = expert_dot<BITS>(uc, xs);
+    float us, ub;
     load_scale_bias<BITS>(bv.us + r * n_groups, bv.ub + r * n_groups, e0, us, ub);
-    lane_dot<BITS, ALIGNED>(uc, xt + e0, ud, sum2);
     if constexpr (G32 && BITS == kBits2) {
       // the lane's 64 weights are two gate groups: entries e0 / 32 and e0 / 32 + 1 of a row of D / 32
       const uint16_t* gsr = bv.gs + r * (2 * n_groups) + e0 / 32;
@@ -104,18 +127,24 @@ __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__
       lane_dot_halves_q2<ALIGNED>(gc, xt + e0, hd, hs);
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        ga = __builtin_fmaf(bf16_to_f(gsr[half]), hd[half], ga);
-        ga = __builtin_fmaf(bf16_to_f(gbr[half]), hs[half], ga);
+        if (in) {
+          ga = __builtin_fmaf(bf16_to_f(gsr[half]), hd[half], ga);
+          ga = __builtin_fmaf(bf16_to_f(gbr[half]), hs[half], ga);
+        }
       }
-      (void)gs; (void)gb; (void)gd; (void)sum;
     } else {
+      float gs, gb;
       load_scale_bias<BITS>(bv.gs + r * n_groups, bv.gb + r * n_groups, e0, gs, gb);
-      lane_dot<BITS, ALIGNED>(gc, xt + e0, gd, sum);
-      ga = __builtin_fmaf(gs, gd, ga);
-      ga = __builtin_fmaf(gb, sum, ga);
+      const float gd = expert_dot<BITS>(gc, xs);
+      if (in) {
+        ga = __builtin_fmaf(gs, gd, ga);
+        ga = __builtin_fmaf(gb, xs.sum, ga);
+      }
     }
-    ua = __builtin_fmaf(us, ud, ua);
-    ua = __builtin_fmaf(ub, sum2, ua);
+    if (in) {
+      ua = __builtin_fmaf(us, ud, ua);
+      ua = __builtin_fmaf(ub, xs.sum, ua);
+    }
   }
   const float g = group_sum(ga, static_cast<int>(lpr));
   const float u = group_sum(ua, static_cast<int>(lpr));
@@ -137,48 +166,70 @@ __global__ __launch_bounds__(256) void phase2_kernel(const uint8_t* __restrict__
                                                      uint32_t F, uint32_t E, uint32_t T,
                                                      uint32_t K, int maple, uint32_t lpr_log2,
                                                      const SlotMap slots) {
-  constexpr int EPL = Fmt<BITS>::kElemsPer16B;
+  constexpr uint32_t EPL = Fmt<BITS>::kElemsPer16B;
   if (slots.all_hit && *slots.all_hit == 0u) return;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t lpr = 1u << lpr_log2;
   const uint32_t rpw = 64u >> lpr_log2;
-  const uint32_t waves_per_tok = (D + rpw - 1) / rpw;
-  const uint32_t tok = wave / waves_per_tok;
-  if (tok >= T) return;
-  const uint32_t row = (wave % waves_per_tok) * rpw + (lane >> lpr_log2);
+  const uint32_t waves_per_tok = (D + rpw - 1) / rpw, wgs_per_tok = (waves_per_tok + 3) / 4;
+  const uint32_t tok = blockIdx.x / wgs_per_tok;
+  const uint32_t row = ((blockIdx.x % wgs_per_tok) * 4 + (threadIdx.x >> 6)) * rpw + (lane >> lpr_log2);
   const uint32_t sub = lane & (lpr - 1);
   const bool row_ok = row < D;
   const size_t r = row_ok ? row : 0;
   const uint32_t n_groups = F / kGroup;
   const size_t row_bytes = static_cast<size_t>(F) * Store<BITS>::kBits / 8;
   float acc = residual ? bf16_to_f(residual[static_cast<size_t>(tok) * D + r]) : 0.0f;
-  for (uint32_t k = 0; k < K; ++k) {
-    const uint32_t pair = tok * K + k;
-    const uint8_t* blob;
-    if (slots.offsets) {
-      blob = base + slots.offsets[pair];
-    } else {
-      const uint32_t expert = idx[pair];
-      if (expert >= E) continue;
-      blob = base + static_cast<size_t>(expert) * stride;
+  // the slices of as many slots as fit at a time, of a slot longer than that piece by piece
+  const uint32_t spl = F / EPL, piece = min(spl, kStageSlices), slots_at_once = min(K, kStageSlices / piece), staged = slots_at_once * piece;
+  uint4* xq = reinterpret_cast<uint4*>(smem);
+  float* xsum = reinterpret_cast<float*>(xq + XSlice<BITS>::kPairs / 4 * staged);
+  float part = 0.0f;
+  for (uint32_t k0 = 0; k0 < K; k0 += slots_at_once) {
+    const uint32_t k1 = min(K, k0 + slots_at_once);
+    for (uint32_t s0 = 0; s0 < spl; s0 += piece) {
+      const uint32_t n = min(piece, spl - s0);
+      if (k0 || s0) __syncthreads();
+      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, (k1 - k0) * n, 0, 256, [&](uint32_t i, uint32_t& at, uint32_t& sum_at) {
+        const uint32_t k = i / n, sl = i - k * n;
+        at = sum_at = k * piece + sl;
+        return acts + static_cast<size_t>(tok * K + k0 + k) * F + static_cast<size_t>(s0 + sl) * EPL;
+      });
+      __syncthreads();
+      for (uint32_t k = k0; k < k1; ++k) {
+        const uint32_t pair = tok * K + k;
+        const uint8_t* blob;
+        if (slots.offsets) {
+          blob = base + slots.offsets[pair];
+        } else {
+          const uint32_t expert = idx[pair];
+          if (expert >= E) continue;
+          blob = base + static_cast<size_t>(expert) * stride;
+        }
+        const BlobView bv = view_blob(blob, off);
+        if (s0 == 0) part = 0.0f;
+        for (uint32_t first = 0; first < n; first += lpr) {
+          const bool in = row_ok && first + sub < n;
+          const uint32_t sl = in ? first + sub : first, e0 = (s0 + sl) * EPL;
+          const uint4 dc = load_codes16<ALIGNED>(bv.dw + r * row_bytes +
+                                                 static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
+          float s, b;
+          load_scale_bias<BITS>(bv.ds + r * n_groups, bv.db + r * n_groups, e0, s, b);
+          const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, xsum, 0, staged, (k - k0) * piece + sl);
+          const float dot = expert_dot<BITS>(dc, xs);
+          if (in) {
+            part = __builtin_fmaf(s, dot, part);
+            part = __builtin_fmaf(b, xs.sum, part);
+          }
+        }
+        if (s0 + piece >= spl) {
+          const float v = group_sum(part, static_cast<int>(lpr));
+          const float weighted = w[pair] * (maple ? round_bf16(v) : v);
+          acc = acc + weighted;
+        }
+      }
     }
-    const BlobView bv = view_blob(blob, off);
-    const uint16_t* a = acts + static_cast<size_t>(pair) * F;
-    float part = 0.0f;
-    for (uint32_t e0 = sub * EPL; e0 < F; e0 += lpr * EPL) {
-      if (!row_ok) break;
-      const uint4 dc = load_codes16<ALIGNED>(bv.dw + r * row_bytes +
-                                             static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
-      float s, b, dot, sum;
-      load_scale_bias<BITS>(bv.ds + r * n_groups, bv.db + r * n_groups, e0, s, b);
-      lane_dot<BITS, ALIGNED>(dc, a + e0, dot, sum);
-      part = __builtin_fmaf(s, dot, part);
-      part = __builtin_fmaf(b, sum, part);
-    }
-    const float v = group_sum(part, static_cast<int>(lpr));
-    const float weighted = w[pair] * (maple ? round_bf16(v) : v);
-    acc = acc + weighted;
   }
   if (row_ok && sub == 0) y[static_cast<size_t>(tok) * D + row] = f_to_bf16(acc);
 }
@@ -226,8 +277,9 @@ hipError_t launch_phase1(hipStream_t s, const mf_moe_config& cfg, const void* ba
   {                                                                                              \
     const uint32_t lpr_log2 = lanes_per_row_log2(cfg.d, Fmt<BITS>::kElemsPer16B);                \
     const uint32_t rpw = 64u >> lpr_log2;                                                        \
-    const uint32_t waves = pairs * ((cfg.f + rpw - 1) / rpw);                                    \
-    phase1_kernel<BITS, AL><<<dim3((waves + 3) / 4), dim3(256), 0, s>>>(                         \
+    const uint32_t waves = (cfg.f + rpw - 1) / rpw, slices = cfg.d / Fmt<BITS>::kElemsPer16B;    \
+    phase1_kernel<BITS, AL><<<dim3(pairs * ((waves + 3) / 4)), dim3(256),                        \
+                              stage_bytes<BITS>(std::min(slices, kStageSlices)), s>>>(           \
         b, stride, off, idx, x, x_stride, acts, cfg.d, cfg.f, cfg.num_experts, pairs, cfg.top_k, \
         cfg.swiglu_limit, static_cast<int>(cfg.maple_rounding), lpr_log2, subset, all_pairs,     \
         SlotMap{slot_offsets, all_hit});                                                         \
@@ -238,9 +290,10 @@ hipError_t launch_phase1(hipStream_t s, const mf_moe_config& cfg, const void* ba
       if (cfg.gate_group_size == 32) {
         const uint32_t lpr_log2 = lanes_per_row_log2(cfg.d, Fmt<kBits2>::kElemsPer16B);
         const uint32_t rpw = 64u >> lpr_log2;
-        const uint32_t waves = pairs * ((cfg.f + rpw - 1) / rpw);
+        const uint32_t waves = (cfg.f + rpw - 1) / rpw, slices = cfg.d / Fmt<kBits2>::kElemsPer16B;
 #define MF_P1G(AL)                                                                                  \
-  phase1_kernel<kBits2, AL, true><<<dim3((waves + 3) / 4), dim3(256), 0, s>>>(                      \
+  phase1_kernel<kBits2, AL, true><<<dim3(pairs * ((waves + 3) / 4)), dim3(256),                     \
+                                    stage_bytes<kBits2>(std::min(slices, kStageSlices)), s>>>(      \
       b, stride, off, idx, x, x_stride, acts, cfg.d, cfg.f, cfg.num_experts, pairs, cfg.top_k,      \
       cfg.swiglu_limit, static_cast<int>(cfg.maple_rounding), lpr_log2, subset, all_pairs,          \
       SlotMap{slot_offsets, all_hit})
@@ -277,8 +330,10 @@ hipError_t launch_phase2(hipStream_t s, const mf_moe_config& cfg, const void* ba
   {                                                                                          \
     const uint32_t lpr_log2 = lanes_per_row_log2(cfg.f, Fmt<BITS>::kElemsPer16B);            \
     const uint32_t rpw = 64u >> lpr_log2;                                                    \
-    const uint32_t waves = t * ((cfg.d + rpw - 1) / rpw);                                    \
-    phase2_kernel<BITS, AL><<<dim3((waves + 3) / 4), dim3(256), 0, s>>>(                     \
+    const uint32_t waves = (cfg.d + rpw - 1) / rpw, spl = cfg.f / Fmt<BITS>::kElemsPer16B;   \
+    const uint32_t piece = std::min(spl, kStageSlices);                                      \
+    phase2_kernel<BITS, AL><<<dim3(t * ((waves + 3) / 4)), dim3(256),                        \
+                              stage_bytes<BITS>(std::min(cfg.top_k, kStageSlices / piece) * piece), s>>>( \
         b, stride, off, idx, w, acts, residual, y, cfg.d, cfg.f, cfg.num_experts, t,         \
         cfg.top_k, static_cast<int>(cfg.maple_rounding), lpr_log2,                           \
         SlotMap{slot_offsets, all_hit});                                                     \

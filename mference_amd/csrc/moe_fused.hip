@@ -152,33 +152,6 @@ __device__ __forceinline__ void gate_up_partial(const uint8_t* gw, const uint16_
   }
 }
 
-// The lane slices of x a routed row meets (XSlice: permuted pairs + their sum) depend on the token
-// only, so a workgroup builds them once in LDS instead of once per row: slice sl of token t keeps
-// its pairs as 16-byte blocks xq[(t * kQ + q) * n_sl + sl] (neighbouring lanes read neighbouring
-// blocks) and its sum at xsum[t * n_sl + sl].
-template <int BITS>
-__device__ __forceinline__ void store_xslice_lds(uint4* xq, float* xsum, uint32_t t, uint32_t n_sl, uint32_t sl,
-                                                 const XSlice<BITS>& xs) {
-  constexpr uint32_t kQ = XSlice<BITS>::kPairs / 4;
-#pragma unroll
-  for (uint32_t q = 0; q < kQ; ++q)
-    xq[(t * kQ + q) * n_sl + sl] = make_uint4(xs.p[4 * q], xs.p[4 * q + 1], xs.p[4 * q + 2], xs.p[4 * q + 3]);
-  xsum[t * n_sl + sl] = xs.sum;
-}
-template <int BITS>
-__device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, const float* xsum, uint32_t t, uint32_t n_sl,
-                                                        uint32_t sl) {
-  constexpr uint32_t kQ = XSlice<BITS>::kPairs / 4;
-  XSlice<BITS> xs;
-#pragma unroll
-  for (uint32_t q = 0; q < kQ; ++q) {
-    const uint4 v = xq[(t * kQ + q) * n_sl + sl];
-    xs.p[4 * q] = v.x; xs.p[4 * q + 1] = v.y; xs.p[4 * q + 2] = v.z; xs.p[4 * q + 3] = v.w;
-  }
-  xs.sum = xsum[t * n_sl + sl];
-  return xs;
-}
-
 // n / d for n < 2^31 as a multiplication: the dimensions of most instances are launch arguments, a division by one
 // expands to some thirty instructions, and with sixteen waves on a CU an instruction that every wave executes costs 5 ns.
 struct FastDiv {
@@ -201,15 +174,6 @@ struct FusedGeo {
   uint8_t lpr_d, lpr_f, lpr_sd, lpr_sf;  // log2 of the lanes per row: rows of D and F (routed), of D and Fs (shared)
   FastDiv E, n_sl, rgf, K, srg, c_wgs_div, rpr;
 };
-
-// an activation slice out of its raw blocks in that layout
-template <int BITS>
-__device__ __forceinline__ XSlice<BITS> load_act_slice(const uint4* blocks, uint32_t ld, uint32_t sl) {
-  XRaw<BITS> r;
-#pragma unroll
-  for (int q = 0; q < Fmt<BITS>::kElemsPer16B / 8; ++q) r.q[q] = blocks[q * ld + sl];
-  return make_xslice<BITS>(r);
-}
 
 struct FusedArgs {
   const uint16_t* router_w;
@@ -318,8 +282,7 @@ constexpr uint32_t fused_b_per_wg(uint32_t epl, uint32_t d, uint32_t f, uint32_t
 // How stage C deals a token's output rows.  Rows form: a unit's K slots on K waves, their values meet in LDS -- all
 // waves work although a workgroup has only a unit or two.  Units form: the (unit, slot) pairs of all units go to the
 // waves in turn with four requested ahead, and all values meet once -- from three units per workgroup on (large 2-bit
-// layer, one token: 8 units; most shapes at several tokens), while a row is one step of 64 lanes and the slices of the
-// activations are at most one a thread.  (With a unit's slots on one wave, one after the other, eleven waves of sixteen
+// layer, one token: 8 units; most shapes at several tokens), while a row is one step of 64 lanes.  (With a unit's slots on one wave, one after the other, eleven waves of sixteen
 // worked at five tokens of the Qwen shape, and six of sixteen at one token of the 2816 x 704 layer.)  Launch, us, before
 // and now: Qwen shape 16.0 / 15.2 (two tokens), 26.7 / 26.2 (five), 32.2 / 31.1 (six); large 2-bit layer 52.3 / 50.2
 // (two), 145 / 138 (eight); ternary layer of 256 experts 18.4 / 17.3 (four).
@@ -330,7 +293,7 @@ struct FusedSplit {
 constexpr FusedSplit fused_split(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg, bool units_fit = true) {
   const uint32_t rpw = static_rows_per_wave(f, epl), rg = (d + rpw - 1) / rpw, wgs = n_wg / t;
   const uint32_t share = (rg + wgs - 1) / wgs;
-  const bool by_units = units_fit && share >= 3 && f <= 64 * epl && k * (f / epl) <= kFusedThreads;
+  const bool by_units = units_fit && share >= 3 && f <= 64 * epl;
   const uint32_t per_round = kFusedWaves / k < share ? kFusedWaves / k : share;
   const uint32_t units = by_units ? share : per_round;
   return FusedSplit{by_units, wgs, units, by_units ? 1 : (rg + wgs * units - 1) / (wgs * units)};
@@ -601,9 +564,8 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     // the x slices of the routed rows
     if (xprep && wv + n_poll + n_xw >= kFusedWaves && wv + n_poll < kFusedWaves) {
       for (uint32_t q = (wv + n_poll + n_xw - kFusedWaves) * kWave + lane; q < T * n_sl; q += n_xw * kWave) {
-        const uint32_t tok = S::D != kDyn ? q / n_sl : fdiv(q, a.g.n_sl), sl = q - tok * n_sl;
-        store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, sl,
-                               load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(tok) * D + sl * kEPL));
+        const uint32_t tok = S::T == 1 ? 0u : S::D != kDyn ? q / n_sl : fdiv(q, a.g.n_sl);
+        store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, q - tok * n_sl, load_expert_x<BITS, true>(xin + static_cast<size_t>(q) * kEPL));
       }
     }
   }
@@ -849,8 +811,8 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     float ga = 0.0f, ua = 0.0f;
     auto multiply = [&](uint32_t item, uint32_t step, const Step& c) __attribute__((always_inline)) {
       const XSlice<BITS> xs = xprep ? load_xslice_lds<BITS>(s_xq, s_xsum, c.tok, n_sl, c.e0 / kEPL)
-                                    : load_xslice<BITS, kXAligned>(xin + static_cast<size_t>(c.tok) * D + c.e0);
-      const float gd = codes_dot<BITS>(c.g.codes, xs), ud = codes_dot<BITS>(c.u.codes, xs);
+                                    : load_expert_x<BITS, true>(xin + static_cast<size_t>(c.tok) * D + c.e0);
+      const float gd = expert_dot<BITS>(c.g.codes, xs), ud = expert_dot<BITS>(c.u.codes, xs);
       if (c.ok) {
         ga = __builtin_fmaf(c.g.scale(), gd, ga);
         ga = __builtin_fmaf(c.g.bias(), xs.sum, ga);
@@ -897,9 +859,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     for (uint32_t i = threadIdx.x; i < n_words; i += kFusedThreads) {
       const uint32_t it = first + (i >> rpw_log2), pair = pair_of(it);
       const uint32_t row = ((it - pair * rgf) << rpw_log2) + (i & (rpw - 1));
-      // moe.metal:27-34, 528; maple_moe.metal:153-164
-      const uint32_t word =
-          static_cast<uint32_t>(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) | (tag16 << 16);
+      // moe.metal:27-34, 528; maple_moe.metal:153-164; exchanged at the scale that the slices of an expert have
+      const float act = bf16_to_f(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) * kRowScale;
+      const uint32_t word = (__float_as_uint(act) >> 16) | (tag16 << 16);
       if (row < F) store_u32_agent(&a.t_acts[static_cast<size_t>(pair) * F + row], word);
     }
   }
@@ -1007,19 +969,31 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       }
     };
 
-    if constexpr (UNITS) {
-      // The lane slices of the activations (permuted pairs and their sum) are the same for every unit: made once, in
-      // place, in the layout of the x slices.  (The launcher takes this form only when they are at most one a thread
-      // and a row is one step.)
-      const uint32_t spl = F / kEPLF, n_asl = K * spl;
-      float* s_asum = reinterpret_cast<float*>(s_stage);
-      {
-        if (threadIdx.x < n_asl) {  // a thread reads and writes the blocks of its own slice only
-          uint4* acts4 = reinterpret_cast<uint4*>(s_acts);
-          store_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, threadIdx.x, load_act_slice<BITS>(acts4, act_ld, threadIdx.x));
-        }
+    // The lane slices of the activations (permuted pairs and their sum) are the same for every output row: made once, in
+    // place, in the layout of the x slices.  A thread reads and writes the blocks of its own part of a slice only.
+    const uint32_t spl = F / kEPLF;
+    uint4* acts4 = reinterpret_cast<uint4*>(s_acts);
+    float* s_asum = reinterpret_cast<float*>(s_stage);
+    constexpr bool kStageActs = UNITS || BITS != kBits4;
+    for (uint32_t i = threadIdx.x; kStageActs && i < 4 * K * spl; i += kFusedThreads) {
+      constexpr int kW = kPartWords<BITS>;
+      const uint32_t sl = i >> 2, part = i & 3u;
+      uint32_t raw[kW], p[kW];
+#pragma unroll
+      for (int q = 0; q < kW / 4; ++q) {
+        const uint4 v = acts4[(part * (kW / 4) + q) * act_ld + sl];
+        raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
       }
-      __syncthreads();
+      float sum = expert_x_part<BITS, true>(raw, p);
+      sum += dpp_f<0xB1>(sum);
+      sum += dpp_f<0x4E>(sum);
+#pragma unroll
+      for (int q = 0; q < kW / 4; ++q) acts4[(part * (kW / 4) + q) * act_ld + sl] = make_uint4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+      if (part == 0) s_asum[sl] = sum * kRowUnscale;
+    }
+    if (kStageActs) __syncthreads();
+
+    if constexpr (UNITS) {
       const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
       const uint64_t live = __ballot((lane < K ? s_idx[tok * K + lane] : E) < E);
       w_lane = lane < K ? s_w[tok * K + lane] : 0.0f;
@@ -1027,8 +1001,8 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       uint32_t c_unit = unit_local, c_slot = slot;   // the (unit, slot) at hand
       auto take = [&](const Chunk<BITS>& c) __attribute__((always_inline)) {
         const XSlice<BITS> xs =
-            load_xslice_lds<BITS>(reinterpret_cast<const uint4*>(s_acts), s_asum, 0, act_ld, c_slot * spl + (lane_in ? sub : 0u));
-        float part = __builtin_fmaf(c.scale(), codes_dot<BITS>(c.codes, xs), 0.0f);  // the one step of row_partial
+            load_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, c_slot * spl + (lane_in ? sub : 0u));
+        float part = __builtin_fmaf(c.scale(), expert_dot<BITS>(c.codes, xs), 0.0f);  // the one step of a row
         part = __builtin_fmaf(c.bias(), xs.sum, part);
         const float v = group_sum(lane_in ? part : 0.0f, static_cast<int>(lpr));
         // moe.metal:1262; maple_moe.metal:258 (the down output is a bf16 number first)
@@ -1077,17 +1051,23 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
           const uint32_t pair = tok * K + slot;
           const uint32_t expert = __builtin_amdgcn_readfirstlane(s_idx[pair]);
           float part = 0.0f;
-          if (row < D && expert < E) {
+          if (expert < E) {  // (the same for all lanes)
             const uint8_t* blob = a.expert_base + static_cast<size_t>(expert) * a.expert_stride;
-            const uint8_t* wrow = blob + a.off.down_w + row * rb;
-            const uint16_t* srow = reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + row * ng;
-            const uint16_t* brow = reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + row * ng;
-            for (uint32_t e = e0; e < F; e += lpr * kEPLF) {  // the steps of row_partial
+            const uint32_t rc = row < D ? row : 0u;
+            const uint8_t* wrow = blob + a.off.down_w + rc * rb;
+            const uint16_t* srow = reinterpret_cast<const uint16_t*>(blob + a.off.down_s) + rc * ng;
+            const uint16_t* brow = reinterpret_cast<const uint16_t*>(blob + a.off.down_b) + rc * ng;
+            for (uint32_t first = 0; first < F; first += lpr * kEPLF) {  // the steps of a row
+              const uint32_t e = first + e0, ec = e < F ? e : 0u;
               Chunk<BITS> c = ring[0];
-              if (!(round == 0 && e == e0)) c = load_chunk<BITS>(wrow, srow, brow, e);
-              const XSlice<BITS> xs = load_act_slice<BITS>(reinterpret_cast<const uint4*>(s_acts), act_ld, (slot * F + e) / kEPLF);
-              part = __builtin_fmaf(c.scale(), codes_dot<BITS>(c.codes, xs), part);
-              part = __builtin_fmaf(c.bias(), xs.sum, part);
+              if (!(round == 0 && first == 0)) c = load_chunk<BITS>(wrow, srow, brow, ec);
+              XSlice<BITS> xs = load_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, slot * spl + ec / kEPLF);
+              if constexpr (!kStageActs) xs = permuted_expert_x<BITS>(xs);
+              const float dot = expert_dot<BITS>(c.codes, xs);
+              if (e < F) {
+                part = __builtin_fmaf(c.scale(), dot, part);
+                part = __builtin_fmaf(c.bias(), xs.sum, part);
+              }
             }
           }
           const float v = group_sum(part, static_cast<int>(lpr));
@@ -1161,7 +1141,7 @@ static FusedGeo fused_geo(const mf_moe_config& c, uint32_t num_cu, uint32_t t, c
 
 // words of the LDS staging area: a chunk of router logits in stage A, the (gate, up) sums of a
 // workgroup's run of routed rows in stage B
-// (and, in stage C's units form, the sums of the activation slices)
+// (and, in stage C, the sums of the activation slices)
 static uint32_t fused_stage_words(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
   const uint32_t epl = fused_epl(c), rpw = 64u >> lanes_per_row_log2_dev(c.d, epl);
   const uint32_t words = std::max(2 * fused_b_per_wg(c, num_cu, t) * rpw, c.top_k * (c.f / epl));

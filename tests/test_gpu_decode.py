@@ -414,6 +414,50 @@ def test_down_rows_dealt_in_pairs(gpu, oracle, bits, d, f, e, k, fs, t):
     assert np.isfinite(oracle.bf16_to_float(out[0])).all() and out[0].any()
 
 
+@pytest.mark.parametrize("bits,d,f,e,k,t", [
+    (4, 8256, 64, 4, 2, 2),     # x of 258 slices: staged in two pieces
+    (2, 16448, 64, 4, 2, 1),    # 257 slices
+    (4, 64, 8256, 4, 3, 2),     # a slot's activations longer than what is staged at a time
+    (2, 128, 6400, 8, 6, 1),    # 100 slices a slot: two slots at a time
+    (1, 320, 192, 8, 5, 3),     # five lanes of eight, three of four
+])
+def test_routed_phases_at_staging_edges(gpu, oracle, bits, d, f, e, k, t):
+    layer = oracle.synth_layer(ROOT_SEED + 0x9300 + bits, d, f, e, k, bits=bits, fs=0)
+    x = oracle.synth_x(ROOT_SEED + 0x9301, t, d)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    moe.set_fused(False)
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    moe.encode_decode_layer(wts, ops.bf16_tensor(x), y, t=t)
+    _sync()
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(oracle.moe_layer(layer, x)[0]),
+                       f"staged slices bits={bits} d={d} f={f}")
+
+
+@pytest.mark.parametrize("bits", [4, 2, 1])
+def test_routed_rows_of_any_magnitude(gpu, oracle, bits):
+    """A power of two on the activations of the down projection is one on its result, bit for bit (they are kept at a
+    scale of their own inside); an infinity stays with its token."""
+    d, f, e, k, t = 192, 320, 8, 3, 3
+    layer = oracle.synth_layer(ROOT_SEED + 0x9400 + bits, d, f, e, k, bits=bits, fs=0)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    g = torch.Generator().manual_seed(7)
+    acts = torch.randn((t, k, f), generator=g).to(torch.bfloat16)
+    idx = torch.tensor([[0, 3, 5], [1, 2, 7], [6, 4, 0]], dtype=torch.int32).cuda()
+    w = torch.rand((t, k), generator=g).cuda()
+
+    def down(a):
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        moe.encode_routed_phase2_reduce(wts.experts, wts.offsets, idx, w, a.cuda(), None, y, t=t)
+        _sync()
+        return y.float().cpu()
+    y0 = down(acts)
+    for p in (48, -48):
+        assert torch.equal(down((acts.float() * 2.0 ** p).to(torch.bfloat16)), y0 * 2.0 ** p)
+    acts[1, 2, 17] = float("inf")
+    y1 = down(acts)
+    assert torch.isnan(y1[1]).all() and torch.equal(y1[[0, 2]], y0[[0, 2]]) and (y0 != 0).float().mean() > 0.99
+
+
 def test_decode_layer_residual_add_in_place(gpu, oracle):
     d, f, e, k, fs, t = 256, 128, 16, 4, 128, 2
     root = ROOT_SEED + 0x9100
