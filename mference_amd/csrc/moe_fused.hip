@@ -240,9 +240,11 @@ __device__ __forceinline__ void trace_mark(const FusedArgs& a, uint32_t slot) {
 // has no router rows, no logits exchange and no top-k, and reads indices and weights instead of
 // writing them.  A compile-time property, so the kernels that route keep their code as it is.
 constexpr uint32_t kDyn = 0xFFFFFFFFu;  // a dimension read from the arguments
-template <bool GIVEN = false>
+// kAnyE: the number of experts need not be a multiple of four (an instance of its own: the few instructions more cost the
+// others 4 % of a small layer)
+template <bool GIVEN = false, bool ANYE = false>
 struct RuntimeShapeT {
-  static constexpr bool kStatic = false, kGiven = GIVEN;
+  static constexpr bool kStatic = false, kGiven = GIVEN, kAnyE = ANYE;
   static constexpr uint32_t D = kDyn, F = kDyn, E = kDyn, K = kDyn, T = kDyn, Fs = kDyn;
   static constexpr uint32_t Mode = kDyn, Maple = kDyn, NoLimit = 0, XPrep = kDyn;
 };
@@ -253,7 +255,7 @@ template <uint32_t D_, uint32_t F_, uint32_t E_, uint32_t K_, uint32_t T_, uint3
           uint32_t MODE_ = kDyn, uint32_t MAPLE_ = kDyn, uint32_t NOLIMIT_ = 0, uint32_t XPREP_ = kDyn>
 struct StaticShape {
   static constexpr bool kStatic = D_ != kDyn && F_ != kDyn && E_ != kDyn && K_ != kDyn && T_ != kDyn && Fs_ != kDyn;
-  static constexpr bool kGiven = GIVEN;
+  static constexpr bool kGiven = GIVEN, kAnyE = E_ != kDyn && E_ % 4 != 0;
   static constexpr uint32_t D = D_, F = F_, E = E_, K = K_, T = T_, Fs = Fs_;
   static constexpr uint32_t Mode = MODE_, Maple = MAPLE_, NoLimit = NOLIMIT_, XPrep = XPREP_;
 };
@@ -329,8 +331,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   float* s_h1 = reinterpret_cast<float*>(smem + 1024 + 4096);           // [kMaxH1]
   uint32_t* s_rank = reinterpret_cast<uint32_t*>(smem + 1024 + 4096 + kMaxH1 * 4);  // [kRankWords]
   uint8_t* dyn = smem + 1024 + 4096 + kMaxH1 * 4 + kRankWords * 4;
-  float* s_lg = reinterpret_cast<float*>(dyn);                          // [MF_MAX_TOKENS][E]
-  uint32_t* s_sact = reinterpret_cast<uint32_t*>(dyn + MF_MAX_TOKENS * E * 4);  // [(Fs+4)/2]
+  const uint32_t Ep = S::kAnyE ? (E + 3) & ~3u : E;  // logits per token in LDS: the selection reads them four at a time, -inf behind the last
+  float* s_lg = reinterpret_cast<float*>(dyn);                          // [MF_MAX_TOKENS][Ep]
+  uint32_t* s_sact = reinterpret_cast<uint32_t*>(dyn + MF_MAX_TOKENS * Ep * 4);  // [(Fs+4)/2]
   uint32_t* s_acts = s_sact + (((Fs + 4) / 2 + 3) & ~3u);               // [K*F/2], 16-byte aligned
   // the routed activations as 16-byte blocks in the order of the x slices: block q of slice sl at q * act_ld + sl (an
   // odd stride: the lanes that write a slice's blocks and those that read one block of many slices both spread over
@@ -469,10 +472,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     trace_mark(a, 7);
   }
   // rank counting selects the top-k when it is cheap enough, else one wave per token sorts
-  const bool rank_count = !S::kGiven && T * E * E <= kRankCountLimit && T * E <= kRankWords;
+  const bool rank_count = !S::kGiven && T * E * E <= kRankCountLimit && T * Ep <= kRankWords;
   // Who does what while the logits are on their way: the top waves poll for them (n_poll waves),
   // the waves below those build the x slices, the bottom waves have the rows of stage A.
-  const uint32_t n2 = S::kGiven ? 0 : T * E / 2;  // 16-byte pieces of tagged logits (E % 4 == 0)
+  const uint32_t n2 = S::kGiven ? 0 : (S::kAnyE ? T * E + 1 : T * E) / 2;  // 16-byte pieces of tagged logits
   const uint32_t n_poll = fused_poll_waves(n2), n_xw = fused_slice_waves(T * n_sl, n_poll);
 
   // ------------------------------------------------------------- stage A
@@ -577,6 +580,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     s_sc[threadIdx.x] = -__builtin_inff();
   }
   if (threadIdx.x < MF_MAX_TOKENS + 2) s_flag[threadIdx.x] = 0u;  // + s_fail and the selection's fallback flag behind it
+  if (S::kAnyE && threadIdx.x < T * 4) {
+    const uint32_t i = E + (threadIdx.x & 3u);
+    if (i < Ep) s_lg[(threadIdx.x >> 2) * Ep + i] = -__builtin_inff();
+  }
   {
     // keep every word of the activation buffers recently tagged (see the top)
     const uint32_t ts = epoch % MF_MAX_TOKENS;
@@ -600,7 +607,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         uint4 v = make_uint4(0, epoch, 0, epoch);
         for (uint32_t spins = 0;; ++spins) {
           if (in) v = load_u32x4_agent(a.t_logits + 2 * p);
-          if (__all(!in || (v.y == epoch && v.w == epoch))) break;
+          if (__all(!in || (v.y == epoch && (v.w == epoch || (S::kAnyE && 2 * p + 1 == T * E))))) break;  // (an odd number: half a piece)
           if (spins > kSpinLimit) {
             give_up(a.status, s_fail, lane);
             break;
@@ -609,8 +616,13 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         }
         if (in) {  // rank counting wants no NaN among the scores it compares
           const bool clean = rank_count && router_mode == 0;
-          s_lg[2 * p] = clean ? score_or_ninf(__uint_as_float(v.x)) : __uint_as_float(v.x);
-          s_lg[2 * p + 1] = clean ? score_or_ninf(__uint_as_float(v.z)) : __uint_as_float(v.z);
+          uint32_t at[2] = {2 * p, 2 * p + 1};
+          if constexpr (S::kAnyE) {
+            at[0] += fdiv(at[0], a.g.E) * (Ep - E);
+            at[1] += fdiv(at[1], a.g.E) * (Ep - E);
+          }
+          s_lg[at[0]] = clean ? score_or_ninf(__uint_as_float(v.x)) : __uint_as_float(v.x);
+          if (!S::kAnyE || 2 * p + 1 < T * E) s_lg[at[1]] = clean ? score_or_ninf(__uint_as_float(v.z)) : __uint_as_float(v.z);
         }
       }
     }
@@ -618,15 +630,15 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     trace_mark(a, 2);
     if (rank_count) {
       if (router_mode != 0) {  // full softmax first: the probabilities replace the logits
-        if (wv < T && !full_softmax_probs(s_lg + wv * E, s_lg + wv * E, E, lane)) {
+        if (wv < T && !full_softmax_probs(s_lg + wv * Ep, s_lg + wv * Ep, E, lane)) {
           if (lane == 0) s_flag[wv] = 1u;  // the token routes nowhere; its scores only have to be comparable
-          for (uint32_t i = lane; i < E; i += kWave) s_lg[wv * E + i] = 0.0f;
+          for (uint32_t i = lane; i < E; i += kWave) s_lg[wv * Ep + i] = 0.0f;
         }
         __syncthreads();
       }
       bool counted = false;
-      if (topk_prefilter_fits(T, E, K, kFusedWaves)) {
-        topk_prefilter(s_lg, s_rank, s_fail + 1, T, E, K, s_idx, s_sc, wv, lane);
+      if (topk_prefilter_fits(T, Ep, K, kFusedWaves)) {
+        topk_prefilter(s_lg, s_rank, s_fail + 1, T, Ep, K, s_idx, s_sc, wv, lane);
         counted = s_fail[1] == 0u;  // else too many experts passed the prefilter: rank everything
         if (!counted) {
           __syncthreads();
@@ -635,9 +647,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         }
       }
       if (!counted) {
-        topk_rank_count(s_lg, s_rank, T, E, wv, lane, kFusedWaves);
+        topk_rank_count(s_lg, s_rank, T, Ep, wv, lane, kFusedWaves);
         __syncthreads();
-        topk_rank_emit(s_lg, s_rank, T, E, K, s_idx, s_sc, threadIdx.x, kFusedThreads);
+        topk_rank_emit(s_lg, s_rank, T, Ep, K, s_idx, s_sc, threadIdx.x, kFusedThreads);
       }
       if (router_mode != 0) {  // a token with a non-finite logit routes nowhere (maple_moe.metal:62-119)
         __syncthreads();
@@ -645,8 +657,8 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       }
       // the routing weights follow after stage B: nothing needs them before stage C
     } else if (wv < T) {
-      if (router_mode == 0) topk_select_fast(s_lg + wv * E, E, K, s_idx + wv * K, s_w + wv * K, lane);
-      else topk_full_softmax_fast(s_lg + wv * E, s_lg + wv * E, E, K, s_idx + wv * K, s_w + wv * K, lane);
+      if (router_mode == 0) topk_select_fast(s_lg + wv * Ep, E, K, s_idx + wv * K, s_w + wv * K, lane);
+      else topk_full_softmax_fast(s_lg + wv * Ep, s_lg + wv * Ep, E, K, s_idx + wv * K, s_w + wv * K, lane);
     }
     __syncthreads();
   } else {  // routing written by an earlier launch on the stream (a family router): read, never written
@@ -1156,7 +1168,7 @@ static size_t fused_lds_base(const mf_moe_config& c, uint32_t num_cu, uint32_t t
   const size_t sact_words = ((c.shared_f + 4) / 2 + 3) & ~size_t(3);
   const uint32_t epl = fused_epl(c);
   const size_t acts_words = static_cast<size_t>(epl / 8 * 4) * ((c.top_k * c.f / epl) | 1u);
-  return 1024 + 4096 + kMaxH1 * 4 + kRankWords * 4 + static_cast<size_t>(MF_MAX_TOKENS) * c.num_experts * 4 +
+  return 1024 + 4096 + kMaxH1 * 4 + kRankWords * 4 + static_cast<size_t>(MF_MAX_TOKENS) * ((c.num_experts + 3) & ~3u) * 4 +
          4 * (sact_words + acts_words + fused_stage_words(c, num_cu, t));
 }
 constexpr size_t kFusedLdsLimit = 150 * 1024;
@@ -1182,7 +1194,6 @@ size_t fused_lds_bytes(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
 bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void* x, const void* y,
                      const void* hidden, uint32_t t) {
   const mf_moe_config& c = h.cfg;
-  if (c.num_experts % 4 != 0) return false;  // tagged logits are read two entries per lane
   if (c.gate_group_size == 32) return false;  // a gate projection at group 32 runs on the chain of launches
   const bool combo = (c.bits == MF_BITS_4 && (!c.shared_f || c.shared_bits == MF_BITS_4)) ||
                      (c.bits == MF_BITS_2 && (!c.shared_f || c.shared_bits == MF_BITS_4 ||
@@ -1335,9 +1346,15 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   const bool qwen_dims = c.bits == MF_BITS_4 && c.shared_bits == MF_BITS_4 && c.d == 2048 && c.f == 512 &&
                          c.num_experts == 256 && c.top_k == 8 && c.shared_f == 512;
   const bool lit = !h.generic_shape;  // shape instances allowed
+  using AnyE = RuntimeShapeT<false, true>;
+  const bool any_e = c.num_experts % 4 != 0;
   if (norm) {  // x made inside the launch: the Qwen shape's instances and the ones that read every dimension
     if (lit && qwen && one && !c.maple_rounding && no_limit && a.xprep) MF_FUSED_N(kBits4, kBits4, QwenT1);
     else if (lit && qwen) MF_FUSED_N(kBits4, kBits4, QwenTn);
+    else if (any_e && c.bits == MF_BITS_4) MF_FUSED_N(kBits4, kBits4, AnyE);
+    else if (any_e && c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits2, AnyE);
+    else if (any_e && c.bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits4, AnyE);
+    else if (any_e) MF_FUSED_N(kBitsTernary, kBits4, AnyE);
     else if (c.bits == MF_BITS_4) MF_FUSED_N(kBits4, kBits4, RuntimeShape);
     else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits2, RuntimeShape);
     else if (c.bits == MF_BITS_2) MF_FUSED_N(kBits2, kBits4, RuntimeShape);
@@ -1360,6 +1377,11 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
     else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED(kBits2, kBits2, Given);
     else if (c.bits == MF_BITS_2) MF_FUSED(kBits2, kBits4, Given);
     else MF_FUSED(kBitsTernary, kBits4, Given);
+  } else if (any_e) {
+    if (c.bits == MF_BITS_4) MF_FUSED(kBits4, kBits4, AnyE);
+    else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED(kBits2, kBits2, AnyE);
+    else if (c.bits == MF_BITS_2) MF_FUSED(kBits2, kBits4, AnyE);
+    else MF_FUSED(kBitsTernary, kBits4, AnyE);
   } else if (!lit) {
     if (c.bits == MF_BITS_4) MF_FUSED(kBits4, kBits4, RuntimeShape);
     else if (c.bits == MF_BITS_2 && c.shared_f && c.shared_bits == MF_BITS_2) MF_FUSED(kBits2, kBits2, RuntimeShape);

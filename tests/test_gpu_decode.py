@@ -1053,6 +1053,47 @@ def test_fused_topk_on_non_finite_logits(gpu, oracle, e):
         moe.set_fused(True)
 
 
+@pytest.mark.parametrize("bits,e,k,fs,t,norm", [
+    (4, 5, 5, 0, 1, False),      # an odd number of logits, every expert selected
+    (4, 21, 6, 128, 7, False),   # odd for all tokens together
+    (2, 30, 8, 128, 3, True),    # two short of a multiple of four, the norm inside the launch
+    (2, 62, 8, 0, 8, False),     # the padded count is a multiple of 64: selection through the prefilter
+    (4, 103, 8, 0, 4, True),
+    (4, 509, 4, 0, 6, False),    # too many for rank counting: a wave per token sorts
+])
+def test_fused_launch_at_any_number_of_experts(gpu, oracle, bits, e, k, fs, t, norm):
+    """Routing and rows of the fused launch where four does not divide the number of experts: the chain's and the
+    oracle's indices and weights, with ties (a token of zeros), a NaN logit, and the best expert at the very end."""
+    d, f = 256, 128
+    layer = oracle.synth_layer(ROOT_SEED + 0x9500 + e, d, f, e, k, bits=bits, fs=fs)
+    layer.router_w = layer.router_w.copy()
+    layer.router_w[e - 1, 0], layer.router_w[e // 2, 1] = 0x4120, 0x7FC0  # 10 x[0]; NaN
+    x = oracle.synth_x(ROOT_SEED + 0x9501, t, d)
+    x[:, 0] = 0x3F80
+    if t > 1 and not norm:
+        x[1, :] = 0
+    moe, wts, out = make_moe(gpu, layer), to_device_layer(layer), []
+    for fused in (True, False):
+        moe.set_fused(fused)
+        y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        idx = torch.zeros((t, k), dtype=torch.int32, device="cuda")
+        w = torch.zeros((t, k), dtype=torch.float32, device="cuda")
+        for _ in range(3):
+            if norm:
+                h = ops.bf16_tensor(x)
+                moe.encode_decode_layer_normed(wts, h, ops.bf16_tensor(np.full(d, 0x3F80, np.uint16)), y, t=t, out_indices=idx, out_weights=w)
+            else:
+                moe.encode_decode_layer(wts, ops.bf16_tensor(x), y, t=t, out_indices=idx, out_weights=w)
+        moe.status()
+        out.append((idx.cpu().numpy(), w.cpu().numpy().view(np.uint32), ops.bf16_bits(y)))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    if not norm:
+        _, ref_idx, ref_w = oracle.moe_layer(layer, x)
+        assert np.array_equal(out[0][0].astype(np.uint32), ref_idx) and np.array_equal(out[0][1], ref_w.view(np.uint32))
+    assert (out[0][0][t - 1] == e - 1).any()
+
+
 @pytest.mark.parametrize("m,n,t", [(1, 2048, 1), (1, 2048, 8), (64, 64, 3), (65, 192, 2), (130, 2816, 1), (8, 5120, 8)])
 def test_int8_gemv(gpu, oracle, m, n, t):
     """8-bit affine rows (DequantInt8GEMV.encode, Kernels/Quant/DequantInt8GEMV.swift:53; dequant_int8_gemv_simd,
