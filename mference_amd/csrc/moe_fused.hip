@@ -273,12 +273,16 @@ constexpr uint32_t static_rows_per_wave(uint32_t n, uint32_t elems_per_lane) {
 constexpr uint32_t kStaticWgs = 256;
 
 // Units of stage B one workgroup takes: an equal share, in whole 64-byte pieces of the exchanged activations (one
-// writer per memory line).
+// writer per memory line) while a wave then has one unit at most (1024 x 384, 48 experts, one token: 11.8 us, in 32-byte
+// pieces 11.9), else in 16-byte pieces: the 2816 x 704 layer would have 176 of 256 workgroups at work with 32 units each
+// (its router, layer and MLP 33.2 us, with 24 units on 235 workgroups 31.5; 1600 x 960, 100 experts, top 5: 19.6 / 18.1).
 constexpr uint32_t fused_b_per_wg(uint32_t epl, uint32_t d, uint32_t f, uint32_t k, uint32_t t, uint32_t n_wg) {
   const uint32_t rpw = static_rows_per_wave(d, epl);
   const uint32_t n = t * k * ((f + rpw - 1) / rpw), piece = rpw < 16 ? 16 / rpw : 1;
-  const uint32_t share = (n + n_wg - 1) / n_wg;
-  return (share + piece - 1) / piece * piece;
+  const uint32_t share = (n + n_wg - 1) / n_wg, whole = (share + piece - 1) / piece * piece;
+  if (whole <= kFusedWaves) return whole;
+  const uint32_t part = rpw < 4 ? 4 / rpw : 1;
+  return (share + part - 1) / part * part;
 }
 
 // How stage C deals a token's output rows.  Rows form: a unit's K slots on K waves, their values meet in LDS -- all
