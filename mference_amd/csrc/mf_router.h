@@ -108,7 +108,7 @@ constexpr uint32_t kNoWinner = 0xFFFFFFFFu;
 // All 64 lanes call it.
 // MODE 1: lg holds probabilities of the full softmax; the weights are p_r / (sum + 1e-20)
 // with the sum in rank order (maple_moe.metal:100-118).  MODE 2: lg holds selection scores of a
-// family router, only the indices are written.
+// family router, only the indices are written.  MODE 3: w receives the selected scores as they are.
 template <int PER, int MODE = 0>
 __device__ __forceinline__ void topk_select_sorted(const float* lg, uint32_t e, uint32_t k,
                                                    uint32_t* idx, float* w, uint32_t lane) {
@@ -161,8 +161,11 @@ __device__ __forceinline__ void topk_select_sorted(const float* lg, uint32_t e, 
       my_idx = widx;
     }
   }
-  if constexpr (MODE == 2) {  // indices only: the caller weighs them
-    if (lane < k) idx[lane] = my_idx;
+  if constexpr (MODE == 2 || MODE == 3) {  // the caller weighs them
+    if (lane < k) {
+      idx[lane] = my_idx;
+      if constexpr (MODE == 3) w[lane] = my_score;
+    }
     return;
   }
   if constexpr (MODE == 1) {

@@ -1053,6 +1053,17 @@ def test_fused_topk_on_non_finite_logits(gpu, oracle, e):
         moe.set_fused(True)
 
 
+@pytest.mark.parametrize("e", [32, 96, 128, 160])
+def test_selection_by_waves_on_non_finite_logits(gpu, oracle, e):
+    """the same at the edges of the selection that a wave makes by itself: top 8 of exactly 32 experts, two experts a
+    lane with the last lanes empty and full, and one block more (ranks are counted)"""
+    if e == 32:  # (its taps name experts up to 40)
+        for k in (8, 1):
+            test_fused_launch_at_any_number_of_experts(gpu, oracle, 4, e, k, 0, 5, False)
+    else:
+        test_fused_topk_on_non_finite_logits(gpu, oracle, e)
+
+
 @pytest.mark.parametrize("bits,e,k,fs,t,norm", [
     (4, 5, 5, 0, 1, False),      # an odd number of logits, every expert selected
     (4, 21, 6, 128, 7, False),   # odd for all tokens together
