@@ -238,19 +238,6 @@ __device__ __forceinline__ void issue_fence() { asm volatile("" ::: "memory"); }
 // every store this wave has issued is acknowledged at its scope
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// 32 bf16 (64 bytes) of exchanged activations
-__device__ __forceinline__ void load_x32_agent(const uint16_t* p, uint4 (&x)[4]) {
-  asm volatile(
-      "global_load_dwordx4 %0, %4, off sc1\n\t"
-      "global_load_dwordx4 %1, %4, off offset:16 sc1\n\t"
-      "global_load_dwordx4 %2, %4, off offset:32 sc1\n\t"
-      "global_load_dwordx4 %3, %4, off offset:48 sc1\n\t"
-      "s_waitcnt vmcnt(0)"
-      : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
-      : "v"(p)
-      : "memory");
-}
-
 // ------------------------------------------------------------- raw loads
 
 __device__ __forceinline__ uint32_t load_u32_bytes(const uint8_t* p) {
@@ -354,18 +341,6 @@ __device__ __forceinline__ f32x16_t mfma_bf16(const uint4& a, const uint4& b, co
 __device__ __forceinline__ uint4 expand_q4(uint32_t w) {
   return make_uint4(and_or(w << 3, 0x00780078u, kMagic8), and_or(w >> 1, 0x00780078u, kMagic8),
                     and_or(w >> 5, 0x00780078u, kMagic8), and_or(w >> 9, 0x00780078u, kMagic8));
-}
-
-// one packed word of sixteen 2-bit codes -> two MFMA operands in the same pairing: the byte swap
-// (B0, B2, B1, B3) puts code r and code r + 4 sixteen bits apart, and likewise 8 + r and 12 + r, so
-// a = (q0,q4),(q1,q5),(q2,q6),(q3,q7) and b = (q8,q12),...,(q11,q15) as the bf16 numbers 4 + q
-// (exponent 2^2, the code in mantissa bits 5..6): the x order of the 4-bit form serves both.
-__device__ __forceinline__ void expand_q2(uint32_t w, uint4& a, uint4& b) {
-  const uint32_t v = __builtin_amdgcn_perm(w, w, 0x03010200u);
-  a = make_uint4(and_or(v << 5, 0x00600060u, kMagic4), and_or(v << 3, 0x00600060u, kMagic4),
-                 and_or(v << 1, 0x00600060u, kMagic4), and_or(v >> 1, 0x00600060u, kMagic4));
-  b = make_uint4(and_or(v >> 3, 0x00600060u, kMagic4), and_or(v >> 5, 0x00600060u, kMagic4),
-                 and_or(v >> 7, 0x00600060u, kMagic4), and_or(v >> 9, 0x00600060u, kMagic4));
 }
 
 // ---- codes as bf16 subnormals: the operands of the quantized matmuls
@@ -591,30 +566,17 @@ __device__ __forceinline__ void permute_x(const uint32_t* raw, XSlice<BITS>& xs)
   }
 }
 
-enum XLoad : int { kXAligned = 0, kXUnaligned = 1, kXAgent = 2 };
+enum XLoad : int { kXAligned = 0, kXUnaligned = 1 };
 
 // loads and permutes the lane's slice of x starting at element pointer x
 template <int BITS, int MODE>
 __device__ __forceinline__ XSlice<BITS> load_xslice(const uint16_t* x) {
   constexpr int kQuads = Fmt<BITS>::kElemsPer16B / 8;
   uint32_t raw[kQuads * 4];
-  if constexpr (MODE == kXAgent) {
 #pragma unroll
-    for (int q = 0; q < kQuads; q += 4) {
-      uint4 a[4];
-      load_x32_agent(x + 8 * q, a);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        raw[4 * (q + i)] = a[i].x; raw[4 * (q + i) + 1] = a[i].y;
-        raw[4 * (q + i) + 2] = a[i].z; raw[4 * (q + i) + 3] = a[i].w;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < kQuads; ++q) {
-      const uint4 a = load_x8<MODE == kXAligned>(x + 8 * q);
-      raw[4 * q] = a.x; raw[4 * q + 1] = a.y; raw[4 * q + 2] = a.z; raw[4 * q + 3] = a.w;
-    }
+  for (int q = 0; q < kQuads; ++q) {
+    const uint4 a = load_x8<MODE == kXAligned>(x + 8 * q);
+    raw[4 * q] = a.x; raw[4 * q + 1] = a.y; raw[4 * q + 2] = a.z; raw[4 * q + 3] = a.w;
   }
   XSlice<BITS> xs;
   permute_x<BITS>(raw, xs);
