@@ -17,6 +17,9 @@
  *                                      is fp32 and the reference's narrowing points
  *                                      are kept, narrowing to bf16 instead of fp16
  *
+ * Activations that meet quantized weights may count as infinite from a magnitude of
+ * 2^63 on (most kernels keep them times 2^64); an infinity or a NaN stays with its row.
+ *
  * All pointers are DEVICE pointers unless a parameter says "host".  Activations
  * and scale/bias tables must be 2-byte aligned; packed weights may have any
  * alignment (16-byte aligned tensors take the fast 128-bit-load kernels).

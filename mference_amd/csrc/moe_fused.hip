@@ -763,7 +763,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // When the requests go out.  Rows form: behind stage B's first (and mostly only) ones, so that the codes are here when
   // the activations are and no poll for activations has to wait for them -- a wave's loads return in order (small 4-bit
   // layer 12.4 -> 11.5 us, ternary layer 12.6 -> 12.3).  Units form: behind stage B, whose own stream of rows they
-  // would sit in (Qwen shape, five tokens: 26.4 us, with the early requests 28.9).
+  // would sit in (Qwen shape, five tokens, as it was then: 26.4 us, with the early requests 28.9).
   auto request_down_rows = [&]() __attribute__((always_inline)) {
     if constexpr (UNITS) {
       const uint32_t expert = lane < K ? s_idx[tok * K + lane] : E;
