@@ -1000,7 +1000,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     const uint32_t spl = F / kEPLF;
     uint4* acts4 = reinterpret_cast<uint4*>(s_acts);
     float* s_asum = reinterpret_cast<float*>(s_stage);
-    constexpr bool kStageActs = UNITS || BITS != kBits4;
+    // (Rows form: a wave meets one slice or two and makes them itself for less than the barrier costs -- 2816 x 448, 2-bit,
+    // norm in front: 17.9 us staged, 17.4 -- except the 64-element slices of a literal shape: ternary layer 12.2 / 12.0.)
+    constexpr bool kStageActs = UNITS || (BITS != kBits4 && S::kStatic);
     for (uint32_t i = threadIdx.x; kStageActs && i < 4 * K * spl; i += kFusedThreads) {
       constexpr int kW = kPartWords<BITS>;
       const uint32_t sl = i >> 2, part = i & 3u;
