@@ -356,9 +356,20 @@ __device__ __forceinline__ uint4 expand_q4(uint32_t w) {
 // (Fields left where they are, at the bottom of the byte, would save half of the shifts: 292 / 167 / 147 ns.  The matrix core
 // aligns products by the operands' exponents, though, and the small ones then lose bits: 1.1e-7 on SwiGLU outputs.)
 // The rows that meet such codes are kept times 2^64 (kRowScale), so that products stay in the range of ordinary fp32
-// numbers; the group's scale takes the powers of two back.  Rows hold magnitudes up to 2^64 (beyond: infinity), and a sum keeps
-// all 24 bits down to 2^-61.  (The norm in front of a layer squares its rows in fp32, which ends at 2^64 as well.)
+// numbers; the group's scale takes the powers of two back.  A sum then keeps all 24 bits down to 2^-61, and values may reach
+// 2^57 (64 of them against codes of 15 stay finite).  What leaves that window takes another power of two, chosen by the largest
+// magnitude: 2^2 for large values, 2^126 for small ones.  So a bf16 number of any size has its product, as with numbers under an offset.
 constexpr float kRowScale = 0x1p64f, kRowUnscale = 0x1p-64f;
+// m: the largest magnitude, times kRowScale (infinite where that overflows)
+// (magnitudes compare as their bits do: where they are the same for a wave, on the scalar unit)
+__device__ __forceinline__ float scale_of_window(float m, float low, float high) {
+  const uint32_t b = __float_as_uint(m);
+  return b >= __float_as_uint(high) ? 0x1p2f : b - 1u < __float_as_uint(low) - 1u ? 0x1p126f : kRowScale;
+}
+__device__ __forceinline__ float row_scale(float m) { return scale_of_window(m, 0x1p5f, 0x1p121f); }
+// The activations between an MLP's products are scaled before the largest is known, by that of the token's x (m, as above): from
+// 2^-20 to 2^20 in x they are products of two sums of such numbers and stay within 2^-61 .. 2^62 unless the weights do not.
+__device__ __forceinline__ float act_scale(float m) { return scale_of_window(m, 0x1p44f, 0x1p84f); }
 
 // the upper halves of two fp32 numbers, (lo, hi) in the lower and the upper half
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
@@ -533,6 +544,7 @@ template <int BITS> struct XSlice {
   static constexpr int kPairs = Fmt<BITS>::kElemsPer16B / 2;
   uint32_t p[kPairs];
   float sum;
+  float unscale;  // (expert_dot's slices)
 };
 
 // raw: consecutive bf16 pairs (x0,x1),(x2,x3),... of the lane's slice
@@ -641,12 +653,24 @@ __device__ __forceinline__ float codes_dot(const uint4& codes, const XSlice<BITS
 // Vector instructions are what the decode launch's routed stages wait for.  Per lane, 16 bytes and SIMD (four waves):
 // codes under an offset for the two-element dot product 96 / 173 ns (4 / 2 bits), subnormals for it 80 / 139, here 67 / 122;
 // error against 64 bits on normal values 2.1e-8 with the offset, 3.9e-9 / 3.4e-9 either way here (on SwiGLU outputs 5.4e-8, 1.1e-8).
-// An expert's slice holds its values times kRowScale, in the order of the codes, and their sum unscaled.  It is made in
-// four parts of a code word each (the words of raw numbers, the same number of words out; the part's sum, scaled), whose
-// sums are added (0 + 1) + (2 + 3).  SCALED: the raw words are at that scale already.
+// An expert's slice holds its values times a power of two (row_scale, of the slice or of its token; act_scale), in the order of the
+// codes, their sum as it is, and what takes a dot product back to its own scale.  It is made in
+// four parts of a code word each (the words of raw numbers, the same number of words out), whose
+// sums are added (0 + 1) + (2 + 3).
 template <int BITS> constexpr int kPartWords = Fmt<BITS>::kElemsPer16B / 8;
+// 2^-k for scale 2^k, as a pair of bf16 numbers: against it a dot product gives the unscaled sum
+__device__ __forceinline__ uint32_t unscale_pair(float scale) {
+  const uint32_t b = (254u << 23) - __float_as_uint(scale);
+  return __builtin_amdgcn_perm(b, b, 0x03020302u);
+}
+// q * 2^-129 (2 bits: q * 2^-127) met x * scale
+template <int BITS>
+__device__ __forceinline__ float code_unscale(float scale) {
+  return __uint_as_float(((BITS == kBits4 ? 383u : 381u) << 23) - __float_as_uint(scale));
+}
+// SCALED: the raw words are at that scale already; else *largest is raised to the part's largest magnitude (at that scale)
 template <int BITS, bool SCALED>
-__device__ __forceinline__ float expert_x_part(const uint32_t* raw, uint32_t* p) {
+__device__ __forceinline__ float expert_x_part(const uint32_t* raw, uint32_t* p, float scale, float* largest) {
   constexpr int kSpan = kPartWords<BITS> / 2;  // words between an element and the one in the other half of a code word
 #pragma unroll
   for (int i = 0; i < kSpan; ++i) {
@@ -656,44 +680,72 @@ __device__ __forceinline__ float expert_x_part(const uint32_t* raw, uint32_t* p)
       even = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
       odd = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
     } else {
-      even = upper_halves(bf16_lo(lo) * kRowScale, bf16_lo(hi) * kRowScale);
-      odd = upper_halves(bf16_hi(lo) * kRowScale, bf16_hi(hi) * kRowScale);
+      const float e0 = bf16_lo(lo) * scale, e1 = bf16_lo(hi) * scale, o0 = bf16_hi(lo) * scale, o1 = bf16_hi(hi) * scale;
+      even = upper_halves(e0, e1);
+      odd = upper_halves(o0, o1);
+      *largest = fmaxf(*largest, fmaxf(fmaxf(fabsf(e0), fabsf(e1)), fmaxf(fabsf(o0), fabsf(o1))));
     }
     // 4 bits: codes 0..3 of a half word as they come; 2 bits: codes 0, 2, 4, 6 (lower place), then 1, 3, 5, 7
     p[BITS == kBits4 ? 2 * i : i] = even;
     p[BITS == kBits4 ? 2 * i + 1 : 4 + i] = odd;
   }
+  const uint32_t ones = unscale_pair(scale);
   float sum = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 2 * kSpan; ++i) sum = dot2_bf16(p[i], kOnes, sum);
+  for (int i = 0; i < 2 * kSpan; ++i) sum = dot2_bf16(p[i], ones, sum);
   return sum;
 }
-// n slices by the threads of a workgroup, four adjacent ones a slice, into the layout that load_xslice_lds reads:
-// src(i, at, sum_at) gives slice i's first element, where its blocks start and where its sum goes.  first_thread, threads: who
-// takes part (multiples of 64).  A thread's straight run of code is a quarter of a slice's: cold, it is fetched line by line.
-template <int BITS, bool ALIGNED, class Src>
-__device__ __forceinline__ void stage_expert_x(uint4* xq, float* xsum, uint32_t ld, uint32_t n, uint32_t first_thread, uint32_t threads, Src src) {
+// A quarter of a slice by a thread, four adjacent ones a slice: its numbers (x) to where its blocks start (xq, ld apart), the slice's sum
+// returned to all four.  scale 0: the slice's own, which is left there.  A thread's straight run of code is a quarter of a slice's:
+// cold, it is fetched line by line.
+template <int BITS, bool ALIGNED>
+__device__ __forceinline__ float stage_expert_x_part(uint4* xq, uint32_t ld, const uint16_t* x, uint32_t part, float& scale) {
   constexpr int kW = kPartWords<BITS>;
-  for (uint32_t i = threadIdx.x - first_thread; i < 4 * n; i += threads) {
-    const uint32_t sl = i >> 2, part = i & 3u;
-    uint32_t at, sum_at;
-    const uint16_t* x = src(sl, at, sum_at) + part * (2 * kW);
-    uint32_t raw[kW], p[kW];
+  uint32_t raw[kW], p[kW];
 #pragma unroll
-    for (int q = 0; q < kW / 4; ++q) {
-      const uint4 v = load_x8<ALIGNED>(x + 8 * q);
-      raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
-    }
-    float sum = expert_x_part<BITS, false>(raw, p);
-    sum += dpp_f<0xB1>(sum);
-    sum += dpp_f<0x4E>(sum);
+  for (int q = 0; q < kW / 4; ++q) {
+    const uint4 v = load_x8<ALIGNED>(x + part * (2 * kW) + 8 * q);
+    raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
+  }
+  float largest = 0.0f, sum;
+  if (scale == 0.0f) {
+    scale = kRowScale;
+    sum = expert_x_part<BITS, false>(raw, p, scale, &largest);
+    largest = fmaxf(largest, dpp_f<0xB1>(largest));
+    largest = fmaxf(largest, dpp_f<0x4E>(largest));
+    scale = row_scale(largest);
+  }
+  if (scale != kRowScale) sum = expert_x_part<BITS, false>(raw, p, scale, &largest);
+  sum += dpp_f<0xB1>(sum);
+  sum += dpp_f<0x4E>(sum);
 #pragma unroll
-    for (int q = 0; q < kW / 4; ++q) xq[(part * (kW / 4) + q) * ld + at] = make_uint4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
-    if (part == 0) xsum[sum_at] = sum * kRowUnscale;
+  for (int q = 0; q < kW / 4; ++q) xq[(part * (kW / 4) + q) * ld] = make_uint4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
+  return sum;
+}
+// n slices by the threads of a workgroup, into the layout that load_xslice_lds reads, each at a scale of its own:
+// src(i, at) gives slice i's first element and where its blocks, its sum and what takes a dot product back go.
+template <int BITS, bool ALIGNED, class Src>
+__device__ __forceinline__ void stage_expert_x(uint4* xq, float2* xsum, uint32_t ld, uint32_t n, Src src) {
+  for (uint32_t i = threadIdx.x; i < 4 * n; i += blockDim.x) {
+    uint32_t at;
+    const uint16_t* x = src(i >> 2, at);
+    float scale = 0.0f;
+    const float sum = stage_expert_x_part<BITS, ALIGNED>(xq + at, ld, x, i & 3u, scale);
+    if ((i & 3u) == 0) xsum[at] = make_float2(sum, code_unscale<BITS>(scale));
   }
 }
+// ... n consecutive ones at a scale that is not the ordinary one
+template <int BITS>
+__device__ __forceinline__ void stage_expert_x(uint4* xq, float* xsum, uint32_t ld, uint32_t n, float scale, const uint16_t* x) {
+  for (uint32_t i = threadIdx.x; i < 4 * n; i += blockDim.x) {
+    const uint32_t sl = i >> 2;
+    const float sum = stage_expert_x_part<BITS, true>(xq + sl, ld, x + sl * Fmt<BITS>::kElemsPer16B, i & 3u, scale);
+    if ((i & 3u) == 0) xsum[sl] = sum;
+  }
+}
+// *largest is raised to the slice's largest magnitude (at that scale)
 template <int BITS, bool ALIGNED>
-__device__ __forceinline__ XSlice<BITS> load_expert_x(const uint16_t* x) {
+__device__ __forceinline__ XSlice<BITS> load_expert_x(const uint16_t* x, float scale, float* largest) {
   constexpr int kQuads = Fmt<BITS>::kElemsPer16B / 8;
   uint32_t raw[kQuads * 4];
 #pragma unroll
@@ -704,18 +756,20 @@ __device__ __forceinline__ XSlice<BITS> load_expert_x(const uint16_t* x) {
   XSlice<BITS> xs;
   float sum[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, false>(raw + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>);
-  xs.sum = ((sum[0] + sum[1]) + (sum[2] + sum[3])) * kRowUnscale;
+  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, false>(raw + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>, scale, largest);
+  xs.sum = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+  xs.unscale = code_unscale<BITS>(scale);
   return xs;
 }
 // a slice out of its numbers as they come, at the scale already
 template <int BITS>
-__device__ __forceinline__ XSlice<BITS> permuted_expert_x(const XSlice<BITS>& raw) {
+__device__ __forceinline__ XSlice<BITS> permuted_expert_x(const XSlice<BITS>& raw, float scale) {
   XSlice<BITS> xs;
   float sum[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, true>(raw.p + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>);
-  xs.sum = ((sum[0] + sum[1]) + (sum[2] + sum[3])) * kRowUnscale;
+  for (int j = 0; j < 4; ++j) sum[j] = expert_x_part<BITS, true>(raw.p + j * kPartWords<BITS>, xs.p + j * kPartWords<BITS>, scale, nullptr);
+  xs.sum = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+  xs.unscale = code_unscale<BITS>(scale);
   return xs;
 }
 // four codes of every lane against four of its values
@@ -742,7 +796,7 @@ __device__ __forceinline__ float expert_dot(const uint4& codes, const XSlice<BIT
       c = lane_mfma((w << 4) & kMask, w & kMask, xs.p[4 * j], xs.p[4 * j + 1], c);
       c = lane_mfma((w >> 4) & kMask, (w >> 8) & kMask, xs.p[4 * j + 2], xs.p[4 * j + 3], c);
     }
-    return lane_diagonal(c) * 0x1p65f;  // q * 2^-129 met x * 2^64
+    return lane_diagonal(c) * xs.unscale;
   } else {
     constexpr uint32_t kHigh = 0x00C000C0u, kLow = 0x00300030u;
     f32x4_t l = c;
@@ -754,7 +808,7 @@ __device__ __forceinline__ float expert_dot(const uint4& codes, const XSlice<BIT
       l = lane_mfma(d4 & kLow, d8 & kLow, xs.p[8 * j + 2], xs.p[8 * j + 3], l);
       c = lane_mfma(d4 & kHigh, d8 & kHigh, xs.p[8 * j + 6], xs.p[8 * j + 7], c);
     }
-    return __builtin_fmaf(lane_diagonal(l), 4.0f, lane_diagonal(c)) * 0x1p63f;  // q * 2^-129 and q * 2^-127 met x * 2^64
+    return __builtin_fmaf(lane_diagonal(l), 4.0f, lane_diagonal(c)) * xs.unscale;  // (the lower place's products are q * 2^-129)
   }
 }
 
@@ -772,8 +826,7 @@ __device__ __forceinline__ void store_xslice_lds(uint4* xq, float* xsum, uint32_
   xsum[t * n_sl + sl] = xs.sum;
 }
 template <int BITS>
-__device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, const float* xsum, uint32_t t, uint32_t n_sl,
-                                                        uint32_t sl) {
+__device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, uint32_t t, uint32_t n_sl, uint32_t sl, float sum, float unscale) {
   constexpr uint32_t kQ = XSlice<BITS>::kPairs / 4;
   XSlice<BITS> xs;
 #pragma unroll
@@ -781,7 +834,8 @@ __device__ __forceinline__ XSlice<BITS> load_xslice_lds(const uint4* xq, const f
     const uint4 v = xq[(t * kQ + q) * n_sl + sl];
     xs.p[4 * q] = v.x; xs.p[4 * q + 1] = v.y; xs.p[4 * q + 2] = v.z; xs.p[4 * q + 3] = v.w;
   }
-  xs.sum = xsum[t * n_sl + sl];
+  xs.sum = sum;
+  xs.unscale = unscale;
   return xs;
 }
 

@@ -50,7 +50,7 @@ __device__ __forceinline__ BlobView view_blob(const uint8_t* blob, const mf_expe
 // more on that than on the products (2-bit layer 3200 x 1088, eight tokens: 163 us a layer with the codes under an offset, 195 with the
 // slices of expert_dot made by every wave, 99 here).
 constexpr uint32_t kStageSlices = 256;
-template <int BITS> constexpr size_t stage_bytes(uint32_t slices) { return slices * (XSlice<BITS>::kPairs * 4 + 4); }
+template <int BITS> constexpr size_t stage_bytes(uint32_t slices) { return slices * (XSlice<BITS>::kPairs * 4 + 8); }
 
 template <int BITS, bool ALIGNED, bool G32 = false>
 __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__ base,
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__
   float ga = 0.0f, ua = 0.0f;
   const uint32_t n_sl = D / EPL, staged = min(n_sl, kStageSlices);
   uint4* xq = reinterpret_cast<uint4*>(smem);
-  float* xsum = reinterpret_cast<float*>(xq + XSlice<BITS>::kPairs / 4 * staged);
+  float2* xsum = reinterpret_cast<float2*>(xq + XSlice<BITS>::kPairs / 4 * staged);
   for (uint32_t first = 0; first < D; first += lpr * EPL) {  // all lanes take every step: one without a share drops its sums
     const bool in = row_ok && first + sub * EPL < D;
     const uint32_t e0 = in ? first + sub * EPL : first;
@@ -109,13 +109,14 @@ __global__ __launch_bounds__(256) void phase1_kernel(const uint8_t* __restrict__
     const uint32_t sl0 = first / EPL, at = sl0 % kStageSlices;  // (lpr divides kStageSlices)
     if (at == 0) {  // the next slices
       if (first) __syncthreads();
-      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, min(staged, n_sl - sl0), 0, 256, [&](uint32_t i, uint32_t& at, uint32_t& sum_at) {
-        at = sum_at = i;
+      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, min(staged, n_sl - sl0), [&](uint32_t i, uint32_t& at) {
+        at = i;
         return xt + static_cast<size_t>(sl0 + i) * EPL;
       });
       __syncthreads();
     }
-    const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, xsum, 0, staged, at + (e0 - first) / EPL);
+    const float2 sum = xsum[at + (e0 - first) / EPL];
+    const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, 0, staged, at + (e0 - first) / EPL, sum.x, sum.y);
     const float ud = expert_dot<BITS>(uc, xs);
     float us, ub;
     load_scale_bias<BITS>(bv.us + r * n_groups, bv.ub + r * n_groups, e0, us, ub);
@@ -184,16 +185,16 @@ __global__ __launch_bounds__(256) void phase2_kernel(const uint8_t* __restrict__
   // the slices of as many slots as fit at a time, of a slot longer than that piece by piece
   const uint32_t spl = F / EPL, piece = min(spl, kStageSlices), slots_at_once = min(K, kStageSlices / piece), staged = slots_at_once * piece;
   uint4* xq = reinterpret_cast<uint4*>(smem);
-  float* xsum = reinterpret_cast<float*>(xq + XSlice<BITS>::kPairs / 4 * staged);
+  float2* xsum = reinterpret_cast<float2*>(xq + XSlice<BITS>::kPairs / 4 * staged);
   float part = 0.0f;
   for (uint32_t k0 = 0; k0 < K; k0 += slots_at_once) {
     const uint32_t k1 = min(K, k0 + slots_at_once);
     for (uint32_t s0 = 0; s0 < spl; s0 += piece) {
       const uint32_t n = min(piece, spl - s0);
       if (k0 || s0) __syncthreads();
-      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, (k1 - k0) * n, 0, 256, [&](uint32_t i, uint32_t& at, uint32_t& sum_at) {
+      stage_expert_x<BITS, ALIGNED>(xq, xsum, staged, (k1 - k0) * n, [&](uint32_t i, uint32_t& at) {
         const uint32_t k = i / n, sl = i - k * n;
-        at = sum_at = k * piece + sl;
+        at = k * piece + sl;
         return acts + static_cast<size_t>(tok * K + k0 + k) * F + static_cast<size_t>(s0 + sl) * EPL;
       });
       __syncthreads();
@@ -216,7 +217,8 @@ __global__ __launch_bounds__(256) void phase2_kernel(const uint8_t* __restrict__
                                                  static_cast<size_t>(e0) * Store<BITS>::kBits / 8);
           float s, b;
           load_scale_bias<BITS>(bv.ds + r * n_groups, bv.db + r * n_groups, e0, s, b);
-          const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, xsum, 0, staged, (k - k0) * piece + sl);
+          const float2 sum = xsum[(k - k0) * piece + sl];
+          const XSlice<BITS> xs = load_xslice_lds<BITS>(xq, 0, staged, (k - k0) * piece + sl, sum.x, sum.y);
           const float dot = expert_dot<BITS>(dc, xs);
           if (in) {
             part = __builtin_fmaf(s, dot, part);

@@ -483,6 +483,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   const uint32_t n2 = S::kGiven ? 0 : (S::kAnyE ? T * E + 1 : T * E) / 2;  // 16-byte pieces of tagged logits
   const uint32_t n_poll = fused_poll_waves(n2), n_xw = fused_slice_waves(T * n_sl, n_poll);
 
+  // The scales of a token's x and activations, at [token] and MF_MAX_TOKENS behind it.  One token: the largest magnitude, times kRowScale, that
+  // each of the waves that build slices met.  (s_v is free until stage C.)
+  float* s_scale = s_v;
+
   // ------------------------------------------------------------- stage A
   // Router rows are on the critical path and their logits are gathered by everybody: they go in
   // chunks of kRouterChunk consecutive rows to the first workgroups (a wave each; the chunk
@@ -569,11 +573,20 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         }
       }
     }
-    // the x slices of the routed rows
-    if (xprep && wv + n_poll + n_xw >= kFusedWaves && wv + n_poll < kFusedWaves) {
-      for (uint32_t q = (wv + n_poll + n_xw - kFusedWaves) * kWave + lane; q < T * n_sl; q += n_xw * kWave) {
-        const uint32_t tok = S::T == 1 ? 0u : S::D != kDyn ? q / n_sl : fdiv(q, a.g.n_sl);
-        store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, q - tok * n_sl, load_expert_x<BITS, true>(xin + static_cast<size_t>(q) * kEPL));
+    // the x slices of the routed rows, and every token's scales: a wave takes whole tokens (one token: a run of its slices)
+    if (wv + n_poll + n_xw >= kFusedWaves && wv + n_poll < kFusedWaves) {
+      const uint32_t xw = wv + n_poll + n_xw - kFusedWaves;
+      for (uint32_t tok = S::T == 1 ? 0u : xw; tok < T; tok += S::T == 1 ? 1u : n_xw) {
+        float largest = 0.0f;
+        for (uint32_t sl = S::T == 1 ? xw * kWave + lane : lane; sl < n_sl; sl += S::T == 1 ? n_xw * kWave : kWave) {
+          const XSlice<BITS> xs = load_expert_x<BITS, true>(xin + static_cast<size_t>(tok) * D + sl * kEPL, kRowScale, &largest);
+          if (xprep) store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, sl, xs);
+        }
+        largest = wave_max(largest);
+        if (lane == 0) {
+          s_scale[S::T == 1 ? xw : tok] = S::T == 1 ? largest : row_scale(largest);
+          if (S::T != 1) s_scale[MF_MAX_TOKENS + tok] = act_scale(largest);
+        }
       }
     }
   }
@@ -789,6 +802,10 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     }
   };
 
+  // lane t: the scale of token t's x (one token: the same in every lane); read behind the first requests of stage B
+  float x_scale = kRowScale, one_act_scale = kRowScale;
+  auto of_token = [&](float v, uint32_t token) __attribute__((always_inline)) { return S::T == 1 ? v : readlane_f(v, static_cast<int>(token)); };
+
   // ------------------------------------------------------------- stage B
   // Every workgroup takes a run of consecutive units (rpw rows of one routed slot), its waves
   // take them in turn; gate and up sums meet in LDS, the first threads turn them into
@@ -836,8 +853,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     };
     float ga = 0.0f, ua = 0.0f;
     auto multiply = [&](uint32_t item, uint32_t step, const Step& c) __attribute__((always_inline)) {
-      const XSlice<BITS> xs = xprep ? load_xslice_lds<BITS>(s_xq, s_xsum, c.tok, n_sl, c.e0 / kEPL)
-                                    : load_expert_x<BITS, true>(xin + static_cast<size_t>(c.tok) * D + c.e0);
+      float largest = 0.0f;
+      const XSlice<BITS> xs = xprep ? load_xslice_lds<BITS>(s_xq, c.tok, n_sl, c.e0 / kEPL, s_xsum[c.tok * n_sl + c.e0 / kEPL], code_unscale<BITS>(of_token(x_scale, c.tok)))
+                                    : load_expert_x<BITS, true>(xin + static_cast<size_t>(c.tok) * D + c.e0, of_token(x_scale, c.tok), &largest);
       const float gd = expert_dot<BITS>(c.g.codes, xs), ud = expert_dot<BITS>(c.u.codes, xs);
       if (c.ok) {
         ga = __builtin_fmaf(c.g.scale(), gd, ga);
@@ -861,6 +879,25 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     if (S::kStatic || item < last) fetch(item < n_items ? item : 0u, 0, cur);  // (literal shapes: no branch around the loads)
     if constexpr (!UNITS) request_down_rows();
     issue_fence();
+    if (S::T == 1) {
+      float most = s_scale[0];
+      for (uint32_t w = 1; w < n_xw; ++w) most = fmaxf(most, s_scale[w]);
+      most = readlane_f(most, 0);
+      x_scale = row_scale(most);
+      one_act_scale = act_scale(most);
+    } else {
+      x_scale = s_scale[lane & (MF_MAX_TOKENS - 1)];
+    }
+    // A token out of the ordinary window of magnitudes has its slices made again (the same for all waves)
+    const bool again = S::T == 1 ? x_scale != kRowScale : __any(lane < T && x_scale != kRowScale);
+    if (__builtin_expect(xprep && again, 0)) {
+      for (uint32_t t = 0; t < T; ++t) {
+        const float scale = of_token(x_scale, t);
+        if (scale == kRowScale) continue;
+        stage_expert_x<BITS>(s_xq + t * (XSlice<BITS>::kPairs / 4) * n_sl, s_xsum + t * n_sl, n_sl, n_sl, scale, xin + static_cast<size_t>(t) * D);
+      }
+      __syncthreads();
+    }
     if (item < last) {
       for (;;) {
         uint32_t nitem = item, nstep = step + 1;
@@ -885,8 +922,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     for (uint32_t i = threadIdx.x; i < n_words; i += kFusedThreads) {
       const uint32_t it = first + (i >> rpw_log2), pair = pair_of(it);
       const uint32_t row = ((it - pair * rgf) << rpw_log2) + (i & (rpw - 1));
-      // moe.metal:27-34, 528; maple_moe.metal:153-164; exchanged at the scale that the slices of an expert have
-      const float act = bf16_to_f(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) * kRowScale;
+      // moe.metal:27-34, 528; maple_moe.metal:153-164; exchanged at the scale that the slices of the token's activations have
+      const float scale = S::T == 1 ? one_act_scale : s_scale[MF_MAX_TOKENS + (S::K != kDyn ? pair / K : fdiv(pair, a.g.K))];
+      const float act = bf16_to_f(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) * scale;
       const uint32_t word = (__float_as_uint(act) >> 16) | (tag16 << 16);
       if (row < F) store_u32_agent(&a.t_acts[static_cast<size_t>(pair) * F + row], word);
     }
@@ -904,6 +942,9 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // ------------------------------------------------------------- stage C
   if (tok < T) {
     if constexpr (UNITS) request_down_rows();
+    // the scale of the token's activations, in a vector register: the scalar ones are all taken
+    float act_sc = S::T == 1 ? one_act_scale : s_scale[MF_MAX_TOKENS + tok];
+    asm volatile("" : "+v"(act_sc));
     // Gather what other workgroups produced: the routed activations [K*F] and the shared
     // activations (+ gate) [Fs (+4)], 256 words per wave step, two steps in flight.
     // The shared activations were written in stage A, long ago: when the routed words fit the
@@ -1012,14 +1053,19 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         const uint4 v = acts4[(part * (kW / 4) + q) * act_ld + sl];
         raw[4 * q] = v.x; raw[4 * q + 1] = v.y; raw[4 * q + 2] = v.z; raw[4 * q + 3] = v.w;
       }
-      float sum = expert_x_part<BITS, true>(raw, p);
+      float sum = expert_x_part<BITS, true>(raw, p, act_sc, nullptr);
       sum += dpp_f<0xB1>(sum);
       sum += dpp_f<0x4E>(sum);
 #pragma unroll
       for (int q = 0; q < kW / 4; ++q) acts4[(part * (kW / 4) + q) * act_ld + sl] = make_uint4(p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]);
-      if (part == 0) s_asum[sl] = sum * kRowUnscale;
+      if (part == 0) s_asum[sl] = sum;
     }
     if (kStageActs) __syncthreads();
+    auto act_slice = [&](uint32_t sl) __attribute__((always_inline)) {
+      const XSlice<BITS> xs = load_xslice_lds<BITS>(acts4, 0, act_ld, sl, kStageActs ? s_asum[sl] : 0.0f, code_unscale<BITS>(act_sc));
+      if constexpr (kStageActs) return xs;
+      else return permuted_expert_x<BITS>(xs, act_sc);
+    };
 
     if constexpr (UNITS) {
       const bool failed = *s_fail != 0u;  // a wait gave up: no result, and hidden stays as it is
@@ -1028,8 +1074,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       float* s_pv = reinterpret_cast<float*>(s_xq);  // [unit][slot][row of the unit]; the x slices have had their use
       uint32_t c_unit = unit_local, c_slot = slot;   // the (unit, slot) at hand
       auto take = [&](const Chunk<BITS>& c) __attribute__((always_inline)) {
-        const XSlice<BITS> xs =
-            load_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, c_slot * spl + (lane_in ? sub : 0u));
+        const XSlice<BITS> xs = act_slice(c_slot * spl + (lane_in ? sub : 0u));
         float part = __builtin_fmaf(c.scale(), expert_dot<BITS>(c.codes, xs), 0.0f);  // the one step of a row
         part = __builtin_fmaf(c.bias(), xs.sum, part);
         const float v = group_sum(lane_in ? part : 0.0f, static_cast<int>(lpr));
@@ -1089,8 +1134,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
               const uint32_t e = first + e0, ec = e < F ? e : 0u;
               Chunk<BITS> c = ring[0];
               if (!(round == 0 && first == 0)) c = load_chunk<BITS>(wrow, srow, brow, ec);
-              XSlice<BITS> xs = load_xslice_lds<BITS>(acts4, s_asum, 0, act_ld, slot * spl + ec / kEPLF);
-              if constexpr (!kStageActs) xs = permuted_expert_x<BITS>(xs);
+              const XSlice<BITS> xs = act_slice(slot * spl + ec / kEPLF);
               const float dot = expert_dot<BITS>(c.codes, xs);
               if (e < F) {
                 part = __builtin_fmaf(c.scale(), dot, part);
