@@ -683,8 +683,8 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
     for (int i = 0; i < 4; ++i) {
       uint4 v = make_uint4(0, 0, 0, 0);
       if (live) v = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + ch * 32 + 8 * i);
-      float part;
-      const uint4 o = matmul_row8(v, &part);
+      float part, largest = 0.0f;
+      const uint4 o = matmul_row8(v, kRowScale, &part, &largest);
       xa[j][2 * i] = make_uint2(o.x, o.y);
       xa[j][2 * i + 1] = make_uint2(o.z, o.w);
       sum += part;

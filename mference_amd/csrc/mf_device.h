@@ -375,16 +375,21 @@ __device__ __forceinline__ float act_scale(float m) { return scale_of_window(m, 
 __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
   return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
-// eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and at its scale; their sum in *sum (unscaled)
-__device__ __forceinline__ uint4 matmul_row8(const uint4& v, float* sum) {
+// what a result of rows at `scale` lacks: a factor that is 1 for ordinary rows (the matmuls' tables hold the powers of two of those)
+__device__ __forceinline__ float rel_of_scale(float scale) { return __uint_as_float(((2u * 127u + 64u) << 23) - __float_as_uint(scale)); }
+// eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and times `scale`; their sum in *sum (unscaled); *largest is
+// raised to the largest magnitude (at that scale)
+__device__ __forceinline__ uint4 matmul_row8(const uint4& v, float scale, float* sum, float* largest) {
   const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
   const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
   *sum = ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
-  return make_uint4(upper_halves(x0 * kRowScale, x4 * kRowScale), upper_halves(x1 * kRowScale, x5 * kRowScale),
-                    upper_halves(x2 * kRowScale, x6 * kRowScale), upper_halves(x3 * kRowScale, x7 * kRowScale));
+  const float y0 = x0 * scale, y1 = x1 * scale, y2 = x2 * scale, y3 = x3 * scale, y4 = x4 * scale, y5 = x5 * scale, y6 = x6 * scale, y7 = x7 * scale;
+  *largest = fmaxf(*largest, fmaxf(fmaxf(fmaxf(fabsf(y0), fabsf(y1)), fmaxf(fabsf(y2), fabsf(y3))),
+                                   fmaxf(fmaxf(fabsf(y4), fabsf(y5)), fmaxf(fabsf(y6), fabsf(y7)))));
+  return make_uint4(upper_halves(y0, y4), upper_halves(y1, y5), upper_halves(y2, y6), upper_halves(y3, y7));
 }
 
-// The fp32 sums of a row's groups of 64 values, as the matmuls read them for the bias term: three bf16 numbers each, which
+// The fp32 sums of a row's groups of 64 values (times 2^-64 and the row's scale: as they are for ordinary rows), as the matmuls read them for the bias term: three bf16 numbers each, which
 // hold all 24 bits.  Per eight groups the eight first parts, then the second, then the third ones (48 bytes); groups past the
 // row's last one are zeros.
 __host__ __device__ __forceinline__ size_t group_sum_words(uint32_t ng) { return static_cast<size_t>((ng + 7) / 8) * 24; }

@@ -37,6 +37,10 @@ struct QmmArgs {
   // activations: rows of kdim bf16 as matmul_row8 leaves them + their group sums (store_group_sum)
   const uint16_t* x;
   const uint16_t* sumx;
+  // largest magnitude of every token's row of the first product, times kRowScale (dense mode: of every row); the rows' scale follows
+  // from it (row_scale, or act_scale where act_rows is set), and so does that of the activations epilogue 0 leaves
+  const float* row_max;
+  int act_rows;
   uint32_t x_stride;
   int gather;           // 1: x row = sorted[pair].token, 0: x row = pair index
   const mf_pair* sorted;

@@ -33,7 +33,7 @@ __device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint3
 // loop runs (none inside it).  What that buys: 2816 x 704, 128 experts, 300 tokens, gate / up 70 -> 66 us and down
 // 70 -> 47 us under the tracer; Qwen shape, 93 tokens, gate / up 38.5 -> 31.7.
 // LDS (dynamic): x tile ring, 2 stages x 2 K groups x [TT / 32 nt][4 s][2 h][32 n] x 16 B,
-// scale tables [NPROJ][4 waves][ng][32 rows] fp32 or bf16, out slots [TT] u32.
+// scale tables [NPROJ][4 waves][ng][32 rows] fp32 or bf16, per route: out slot u32, what its results lack, scale of its activations.
 // One launch can carry two independent problems of the same instantiation (the routed experts
 // and the shared expert of the same phase): the second problem's work items follow the first's
 // on every XCD, so they fill the slots the first problem's last round leaves empty instead of
@@ -97,6 +97,8 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   using tab_t = std::conditional_t<TAB16, uint16_t, float>;
   tab_t* s_scale = reinterpret_cast<tab_t*>(smem + qmm_x_bytes(TT));  // [NPROJ][4][ng][32]
   uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT) + ((NPROJ * kQmmWaves * ng * 32 * sizeof(tab_t) + 15) & ~15u));
+  float* s_rel = reinterpret_cast<float*>(s_slot + TT);  // [TT]
+  float* s_act = s_rel + TT;                              // [TT]
 
   // weight pointers of this workgroup's projections
   const uint8_t* Wp[NPROJ];
@@ -177,6 +179,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     }
     if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
   }
+  const float row_max = a.row_max[a.dense_mode ? pair_start + min(threadIdx.x & 63u, count - 1) : pr.token];
   // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
   const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_c0 * 8;
   const uint32_t st_2nd = (st_c1 - st_c0) * 8;
@@ -305,6 +308,10 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     }
   }
   qmm_trace(a, work, 2);
+  if (threadIdx.x < TT) {  // (here, where the loads behind this one have been waited for)
+    s_rel[threadIdx.x] = rel_of_scale(a.act_rows ? act_scale(row_max) : row_scale(row_max));
+    s_act[threadIdx.x] = act_scale(row_max);
+  }
 
   // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
   const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
@@ -418,8 +425,22 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   qmm_trace(a, work, 3);
   // ---- epilogue: the lane holds weight row row_base[p] + m for tokens 8j + 4h + i of each 32-token block
   const uint32_t row_raw = (slice * kQmmWaves + wv) * wave_rows;  // past a.rows: this wave has no rows of its own
+  const bool far = __any(s_rel[lane & (TT - 1)] != 1.0f || s_act[lane & (TT - 1)] != kRowScale);  // a row out of the ordinary window
+  auto bring_back = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 rel = *reinterpret_cast<const float4*>(s_rel + nt * 32 + 8 * j + 4 * h);
+        const float r[4] = {rel.x, rel.y, rel.z, rel.w};
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[p][nt][4 * j + i] *= r[i];
+      }
+  };
   if (a.epi == 0) {
-    // SwiGLU, narrowed to bf16 (at the scale of the matmul's rows, kRowScale), transposed through the (now free) x ring so that a lane stores
+    // SwiGLU, narrowed to bf16 (at the scale of the token's activations), transposed through the (now free) x ring so that a lane stores
     // 16 bytes of one token: [token][32 rows] per wave, the rows of a run of 8 in the
     // (0,4,1,5,2,6,3,7) order phase 2 reads, i.e. rows r and r + 4 share a 32-bit word.
     __syncthreads();  // every wave is past its last read of the ring
@@ -431,7 +452,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     // 64 exponentials and reciprocals of a lane are one block of code the compiler can interleave (with
     // the three tests inside the loops every element was a block of its own).
     const bool clamp = a.limit > 0.0f, narrow = a.narrow != 0;
-    auto swiglu_block = [&](auto maple_tag) __attribute__((always_inline)) {
+    auto swiglu_block = [&](auto maple_tag, auto far_tag) __attribute__((always_inline)) {
       constexpr bool kMaple = decltype(maple_tag)::value;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
@@ -441,17 +462,22 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           if (j == 1 && count <= 8) break;
           if (NT == 1 && j == 2 && count <= 16) break;
           uint32_t bits[4];
+          float scale[4] = {kRowScale, kRowScale, kRowScale, kRowScale};
+          if constexpr (decltype(far_tag)::value) {
+            const float4 scales = *reinterpret_cast<const float4*>(s_act + nt * 32 + 8 * j + 4 * h);
+            scale[0] = scales.x; scale[1] = scales.y; scale[2] = scales.z; scale[3] = scales.w;
+          }
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             float gv = acc[0][nt][4 * j + i], uv = acc[NPROJ - 1][nt][4 * j + i];
             if constexpr (kMaple) {  // maple_moe.metal:153-164
-              bits[i] = f_to_bf16(maple_swiglu(gv, uv) * kRowScale);
+              bits[i] = f_to_bf16(maple_swiglu(gv, uv) * scale[i]);
             } else {
               const float gr = round_bf16(gv), ur = round_bf16(uv);
               const float g0 = narrow ? gr : gv, u0 = narrow ? ur : uv;
               gv = clamp ? fminf(g0, a.limit) : g0;  // (selects, so that a NaN stays one without a clamp)
               uv = clamp ? fminf(fmaxf(u0, -a.limit), a.limit) : u0;
-              bits[i] = f_to_bf16(fast_silu(gv) * uv * kRowScale);
+              bits[i] = f_to_bf16(fast_silu(gv) * uv * scale[i]);
             }
           }
           // lanes m and m ^ 4 trade halves: the lower lane ends with tokens i = 0, 1 of both rows,
@@ -467,8 +493,12 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
         }
       }
     };
-    if (a.maple) swiglu_block(std::true_type{});
-    else swiglu_block(std::false_type{});
+    if (__builtin_expect(far, 0)) {
+      bring_back();
+      if (a.maple) swiglu_block(std::true_type{}, std::true_type{});
+      else swiglu_block(std::false_type{}, std::true_type{});
+    } else if (a.maple) swiglu_block(std::true_type{}, std::false_type{});
+    else swiglu_block(std::false_type{}, std::false_type{});
     __syncthreads();
     // the sums of the slice's two groups: two waves' rows each, four threads a (token, group), 16 values of every thread
     {
@@ -479,14 +509,16 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
         const uint32_t task = it * 64 + (threadIdx.x >> 2), tok = task >> 1, gi = task & 1u, g = slice * 2 + gi;
         const uint32_t* half = reinterpret_cast<const uint32_t*>(s_x) + (2 * gi + (part >> 1)) * (TT * 16) + tok * 16 + (part & 1u) * 8;
         const uint4 v0 = *reinterpret_cast<const uint4*>(half), v1 = *reinterpret_cast<const uint4*>(half + 4);
-        float sum = (((bf16_lo(v0.x) + bf16_hi(v0.x)) + (bf16_lo(v0.y) + bf16_hi(v0.y))) +
-                     ((bf16_lo(v0.z) + bf16_hi(v0.z)) + (bf16_lo(v0.w) + bf16_hi(v0.w)))) +
-                    (((bf16_lo(v1.x) + bf16_hi(v1.x)) + (bf16_lo(v1.y) + bf16_hi(v1.y))) +
-                     ((bf16_lo(v1.z) + bf16_hi(v1.z)) + (bf16_lo(v1.w) + bf16_hi(v1.w))));
+        // (each times 2^-64 first: at their scale the sum of large ones would overflow)
+        const uint32_t pairs[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        float pair[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pair[i] = bf16_lo(pairs[i]) * kRowUnscale + bf16_hi(pairs[i]) * kRowUnscale;
+        float sum = ((pair[0] + pair[1]) + (pair[2] + pair[3])) + ((pair[4] + pair[5]) + (pair[6] + pair[7]));
         sum = group_sum(sum, 4);
         const uint32_t sl = s_slot[tok];
         if (part == 0 && sl != 0xFFFFFFFFu && g < ng_out)
-          store_group_sum(a.out_sums + sl * group_sum_words(ng_out), g, ng_out, sum * kRowUnscale);
+          store_group_sum(a.out_sums + sl * group_sum_words(ng_out), g, ng_out, sum);
       }
     }
     const uint32_t lane = threadIdx.x & 63u;
@@ -501,6 +533,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
                                   part * 8) = v;
     }
   } else {
+    if (__builtin_expect(far, 0)) bring_back();
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       if (nt == 1 && count <= 32) break;
@@ -685,14 +718,12 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
     b_term[nt][1] = *reinterpret_cast<const uint4*>(sp + 16);
     if (h) b_term[nt][1] = make_uint4(0, 0, 0, 0);
   }
-  uint32_t slot = 0;
-  if (threadIdx.x < TT) {
-    const uint32_t pi = pair_start + min(threadIdx.x, count - 1);
-    slot = pi;
-    if (!a.dense_mode && (a.epi == 1 || a.epi == 3)) {
-      const mf_pair pr = a.sorted[pi];
-      slot = pr.token * a.top_k + pr.rank;
-    }
+  // (every wave: lane i holds route i's slot and token)
+  uint32_t slot = pair_start + min(lane & (TT - 1), count - 1), token = slot;
+  if (!a.dense_mode) {
+    const mf_pair pr = a.sorted[slot];
+    token = pr.token;
+    if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
   }
   qmm_trace(a, work, 1);
 
@@ -718,6 +749,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + kres_turn<TT>(sidx + 4 * h)) & 31;
   __syncthreads();  // the only workgroup barrier: from here on the waves run on their own
   qmm_trace(a, work, 2);
+  const float row_max = a.row_max[token];  // (looked at in front of the first stores)
   // The sums of the lane's routes: K slots 8h..8h+7 of the bias product are groups 0..7 twice, the first parts for
   // h = 0 and the second ones for h = 1, then the third for h = 0 -- two products instead of three.
   // A tile of at most 32 routes fills only the first route block (NTA = 1): the second block, whose routes
@@ -808,6 +840,17 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
       }
     }
     if (w + 1 == n_walk) qmm_trace(a, work, 3);
+    const float rel = rel_of_scale(a.act_rows ? act_scale(row_max) : row_scale(row_max));
+    if (__builtin_expect(__any(rel != 1.0f), 0)) {  // a row out of the ordinary window among the tile's
+#pragma unroll
+      for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+        for (int r = 0; r < RES; ++r) {
+          const float v = __shfl(rel, static_cast<int>(nt * 32 + 8 * (r / 4) + 4 * h + r % 4));
+          acc[0][nt][r] *= v;
+          acc[1][nt][r] *= v;
+        }
+    }
     // ---- stores: the lane holds rows row + 32 p for routes 8j + 4h + i of each 32-route block
     const uint32_t row = row0 + w * 256;
     // byte offsets fit 32 bits (the launcher checks): one multiply-add per route, the base stays scalar
@@ -890,7 +933,7 @@ void qmm_kres_mixed_kernel(const KresLaunch launch) {
 inline size_t qmm_lds_bytes(uint32_t tile, uint32_t kdim, int nproj, bool tab16) {
   const uint32_t ng = kdim / kGroup;
   return qmm_x_bytes(tile) + ((static_cast<size_t>(nproj) * kQmmWaves * ng * 32 * (tab16 ? 2 : 4) + 15) & ~static_cast<size_t>(15)) +
-         tile * 4;
+         tile * 12;
 }
 // the scale tables as bf16 where fp32 tables would leave a CU (160 KB of LDS) room for one workgroup only
 inline bool qmm_tab16(uint32_t tile, uint32_t kdim, int nproj) {

@@ -52,11 +52,12 @@ struct RouterTail {
   uint32_t router_cols;  // workgroup columns that compute logits; the columns behind them prepare x
   const uint16_t* w_sg;  // null: no scalar gate
   uint16_t* sums;
+  float* row_max;
   uint16_t* gate;
 };
 
 __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ x, uint16_t* __restrict__ xp,
-                                           uint16_t* __restrict__ sums, const uint16_t* __restrict__ w_sg,
+                                           uint16_t* __restrict__ sums, float* __restrict__ row_max, const uint16_t* __restrict__ w_sg,
                                            uint16_t* __restrict__ gate, uint32_t row, uint32_t d, uint32_t lane);
 
 template <int CPL, int R>
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(256) void prefill_router_kernel(const uint16_t* __r
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (tail.xp && blockIdx.x >= tail.router_cols) {  // an x-preparation workgroup: one row per wave
     const uint32_t row = ((blockIdx.x - tail.router_cols) * gridDim.y + blockIdx.y) * 4 + wv;
-    if (row < T) prep_x_row(x + static_cast<size_t>(row) * x_stride, tail.xp, tail.sums, tail.w_sg, tail.gate, row, D, lane);
+    if (row < T) prep_x_row(x + static_cast<size_t>(row) * x_stride, tail.xp, tail.sums, tail.row_max, tail.w_sg, tail.gate, row, D, lane);
     return;
   }
   router_rows<CPL, R>(W, x, E, D, T, x_stride, logits, tokens_per_block, ld, lane, wv);
@@ -162,7 +163,7 @@ void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (tail.xp && blockIdx.y >= tail.router_cols) {  // an x-preparation workgroup (rows behind the expert blocks)
     const uint32_t row = ((blockIdx.y - tail.router_cols) * gridDim.x + blockIdx.x) * WAVES + wv;
-    if (row < T) prep_x_row(x + static_cast<size_t>(row) * x_stride, tail.xp, tail.sums, tail.w_sg, tail.gate, row, D, lane);
+    if (row < T) prep_x_row(x + static_cast<size_t>(row) * x_stride, tail.xp, tail.sums, tail.row_max, tail.w_sg, tail.gate, row, D, lane);
     return;
   }
   const uint32_t m = lane & 31, b = lane >> 5;
@@ -920,33 +921,57 @@ hipError_t launch_tile_experts(hipStream_t s, const mf_moe_config& c, const void
 // --------------------------------------------------------------- the matmul
 
 // Activation rows as the matmul wants them: inside every run of 8 K values the
-// order is (0,4,1,5,2,6,3,7) -- the pairing a packed code word expands to --, every value is times kRowScale,
-// and the fp32 sum of every 64-wide K group (of the values as they were) is kept beside them.  One lane per
-// run of 8.
-__global__ __launch_bounds__(256) void prep_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                        uint16_t* __restrict__ sums, uint32_t chunks, uint32_t ng) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-  uint4 v = make_uint4(0, 0, 0, 0);
-  if (c < chunks) v = *reinterpret_cast<const uint4*>(src + static_cast<size_t>(c) * 8);
+// order is (0,4,1,5,2,6,3,7) -- the pairing a packed code word expands to --, every value is times the row's scale,
+// and the fp32 sum of every 64-wide K group is kept beside them.  One lane per run of 8.
+__device__ __forceinline__ void prep_run(const uint4& v, float scale, uint32_t c, uint32_t chunks, bool live, uint16_t* __restrict__ dst,
+                                         uint16_t* __restrict__ sums, float* largest) {
   float sum;
-  const uint4 row = matmul_row8(v, &sum);
+  const uint4 prepared = matmul_row8(v, scale, &sum, largest);
   sum = group_sum(sum, 8);
-  if (c >= chunks) return;
-  *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) = row;
-  const uint32_t g = c >> 3, r = g / ng;
-  if ((c & 7) == 0) store_group_sum(sums + r * group_sum_words(ng), g - r * ng, ng, sum);
+  if (!live) return;
+  *reinterpret_cast<uint4*>(dst + static_cast<size_t>(c) * 8) = prepared;
+  if ((c & 7) == 0) store_group_sum(sums, c >> 3, chunks / 8, sum * (scale * kRowUnscale));
+}
+
+// A workgroup a row, a thread a run of 8 (of longer rows several): the row's largest magnitude first, so that nothing is written before
+// the barrier -- which would wait for it.  A thread's first run stays in registers.
+constexpr uint32_t kPrepThreads = 1024;
+__global__ __launch_bounds__(kPrepThreads) void prep_rows_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
+                                                                 uint16_t* __restrict__ sums, float* __restrict__ row_max, uint32_t chunks) {
+  __shared__ float s_max[kPrepThreads / kWave];
+  const size_t row = blockIdx.x;
+  src += row * chunks * 8;
+  dst += row * chunks * 8;
+  sums += row * group_sum_words(chunks / 8);
+  auto run = [&](uint32_t c) { return c < chunks ? *reinterpret_cast<const uint4*>(src + static_cast<size_t>(c) * 8) : make_uint4(0, 0, 0, 0); };
+  const uint4 first = run(threadIdx.x);
+  float largest = 0.0f, sum;
+  matmul_row8(first, kRowScale, &sum, &largest);
+  for (uint32_t c = threadIdx.x + blockDim.x; c < chunks; c += blockDim.x) matmul_row8(run(c), kRowScale, &sum, &largest);
+  largest = wave_max(largest);
+  if ((threadIdx.x & 63u) == 0) s_max[threadIdx.x >> 6] = largest;
+  __syncthreads();
+  for (uint32_t w = 0; w < blockDim.x / kWave; ++w) largest = fmaxf(largest, s_max[w]);
+  if (threadIdx.x == 0) row_max[row] = largest;
+  const float scale = row_scale(largest);
+  for (uint32_t c0 = 0; c0 < chunks; c0 += blockDim.x) {
+    const uint32_t c = c0 + threadIdx.x;
+    prep_run(c0 ? run(c) : first, scale, c, chunks, c < chunks, dst, sums, &largest);
+  }
 }
 
 // The same for the layer's input rows and, in the same pass, the scalar shared gate's logit
 // w_sg . x of every row (prefill_qwen_shared_scalar_gate, prefill.metal:42-80) in the router's lane
 // order (dot_bf16_row: lane l takes the chunks l, l+64, ... of a row, neighbour-first butterfly), so
-// the gate has the bits of the stand-alone router-row launch it replaces.  One wave per row.
+// the gate has the bits of the stand-alone router-row launch it replaces.  One wave per row, which is written at the ordinary
+// scale, and a second time where its largest magnitude asks for another.
 __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint16_t* __restrict__ xp,
-                                           uint16_t* __restrict__ sums, const uint16_t* __restrict__ w_sg,
+                                           uint16_t* __restrict__ sums, float* __restrict__ row_max, const uint16_t* __restrict__ w_sg,
                                            uint16_t* __restrict__ gate, uint32_t row, uint32_t d, uint32_t lane) {
   const uint32_t chunks = d / 8;  // a multiple of 8: the 8 lanes of a K group are live together
-  const size_t base = static_cast<size_t>(row) * chunks;
-  float acc = 0.0f;
+  xp += static_cast<size_t>(row) * d;
+  sums += row * group_sum_words(chunks / 8);
+  float acc = 0.0f, largest = 0.0f;
   for (uint32_t c0 = 0; c0 < chunks; c0 += kWave) {
     const uint32_t c = c0 + lane;
     const bool live = c < chunks;
@@ -955,12 +980,8 @@ __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint
       v = *reinterpret_cast<const uint4*>(xr + static_cast<size_t>(c) * 8);
       if (w_sg) wv = *reinterpret_cast<const uint4*>(w_sg + static_cast<size_t>(c) * 8);
     }
-    float sum;
-    const uint4 prepared = matmul_row8(v, &sum);
-    sum = group_sum(sum, 8);
+    prep_run(v, kRowScale, c, chunks, live, xp, sums, &largest);
     if (live) {
-      *reinterpret_cast<uint4*>(xp + (base + c) * 8) = prepared;
-      if ((c & 7) == 0) store_group_sum(sums + row * group_sum_words(chunks / 8), c >> 3, chunks / 8, sum);
       acc = __builtin_fmaf(bf16_lo(wv.x), bf16_lo(v.x), acc);
       acc = __builtin_fmaf(bf16_hi(wv.x), bf16_hi(v.x), acc);
       acc = __builtin_fmaf(bf16_lo(wv.y), bf16_lo(v.y), acc);
@@ -971,17 +992,28 @@ __device__ __forceinline__ void prep_x_row(const uint16_t* __restrict__ xr, uint
       acc = __builtin_fmaf(bf16_hi(wv.w), bf16_hi(v.w), acc);
     }
   }
+  largest = wave_max(largest);
+  if (lane == 0) row_max[row] = largest;
+  const float scale = row_scale(largest);
+  if (__builtin_expect(scale != kRowScale, 0)) {
+    for (uint32_t c0 = 0; c0 < chunks; c0 += kWave) {
+      const uint32_t c = c0 + lane;
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (c < chunks) v = *reinterpret_cast<const uint4*>(xr + static_cast<size_t>(c) * 8);
+      prep_run(v, scale, c, chunks, c < chunks, xp, sums, &largest);
+    }
+  }
   acc = wave_sum(acc);
   if (w_sg && lane == 0) gate[row] = f_to_bf16(acc);
 }
 
 __global__ __launch_bounds__(256) void prep_x_gate_kernel(const uint16_t* __restrict__ x,
                                                           uint16_t* __restrict__ xp, uint16_t* __restrict__ sums,
-                                                          const uint16_t* __restrict__ w_sg,
+                                                          float* __restrict__ row_max, const uint16_t* __restrict__ w_sg,
                                                           uint16_t* __restrict__ gate, uint32_t t, uint32_t d) {
   const uint32_t lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= t) return;
-  prep_x_row(x + static_cast<size_t>(row) * d, xp, sums, w_sg, gate, row, d, lane);
+  prep_x_row(x + static_cast<size_t>(row) * d, xp, sums, row_max, w_sg, gate, row, d, lane);
 }
 
 // y[t,d] = bf16(h1[t,d] + sum_r w[t,r] * partial[t*K+r, d]), residual first, rank
@@ -1221,10 +1253,10 @@ hipError_t launch_topk_group(hipStream_t s, const float* logits, uint32_t t, uin
 }
 
 // `rows` rows of k values
-hipError_t launch_prep_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, uint16_t* sums, uint32_t rows, uint32_t k) {
-  const uint32_t chunks = static_cast<uint32_t>(static_cast<size_t>(rows) * k / 8), blocks = (chunks + 255) / 256;
-  if (!blocks) return hipSuccess;
-  prep_rows_kernel<<<dim3(blocks), dim3(256), 0, s>>>(src, dst, sums, chunks, k / kGroup);
+hipError_t launch_prep_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, uint16_t* sums, float* row_max, uint32_t rows, uint32_t k) {
+  if (!rows || !k) return hipSuccess;
+  const uint32_t chunks = k / 8, threads = std::min((chunks + kWave - 1) / kWave * kWave, kPrepThreads);
+  prep_rows_kernel<<<dim3(rows), dim3(threads), 0, s>>>(src, dst, sums, row_max, chunks);
   return hipGetLastError();
 }
 
@@ -1362,7 +1394,7 @@ static size_t dense_gate_up_parts_bytes(uint32_t t, uint32_t f, uint32_t d) {
 __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* __restrict__ pg, const float* __restrict__ pu,
                                                                    uint32_t n_parts, size_t part_stride,
                                                                    uint16_t* __restrict__ act, uint16_t* __restrict__ sums,
-                                                                   size_t chunks, uint32_t ng, float limit) {
+                                                                   const float* __restrict__ row_max, size_t chunks, uint32_t ng, float limit) {
   const size_t c = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   float g[8], u[8];
 #pragma unroll
@@ -1384,6 +1416,8 @@ __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* 
   }
   uint32_t a[8];
   float v[8];
+  const size_t grp = c >> 3, r = grp / ng;
+  const float scale = act_scale(c < chunks ? row_max[r] : 0.0f);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     float gr = round_bf16(g[i]), ur = round_bf16(u[i]);
@@ -1391,7 +1425,7 @@ __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* 
       gr = fminf(gr, limit);
       ur = fminf(fmaxf(ur, -limit), limit);
     }
-    a[i] = f_to_bf16(fast_silu(gr) * ur * kRowScale);
+    a[i] = f_to_bf16(fast_silu(gr) * ur * scale);
     v[i] = bf16_to_f(static_cast<uint16_t>(a[i])) * kRowUnscale;
   }
   float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
@@ -1399,7 +1433,6 @@ __global__ __launch_bounds__(256) void dense_swiglu_combine_kernel(const float* 
   if (c >= chunks) return;
   *reinterpret_cast<uint4*>(act + c * 8) = make_uint4(a[0] | (a[4] << 16), a[1] | (a[5] << 16), a[2] | (a[6] << 16),
                                                       a[3] | (a[7] << 16));
-  const size_t grp = c >> 3, r = grp / ng;
   if ((c & 7) == 0) store_group_sum(sums + r * group_sum_words(ng), static_cast<uint32_t>(grp - r * ng), ng, sum);
 }
 
@@ -1413,16 +1446,16 @@ bool dense_qmm_takes(const mf_qtensor& w, int bits, const void* x, const void* y
 // bytes of the group sums of `rows` rows of k values
 static size_t sums_bytes(size_t rows, uint32_t k) { return sizeof(uint16_t) * rows * group_sum_words(k / kGroup); }
 static size_t dense_qmm_rows_bytes(uint32_t m, uint32_t k) {
-  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sums_bytes(m, k));
+  return up256(sizeof(uint16_t) * static_cast<size_t>(m) * k) + up256(sums_bytes(m, k)) + up256(sizeof(float) * m);
 }
 size_t dense_qmm_needs(uint32_t m, uint32_t n, uint32_t k) { return dense_qmm_rows_bytes(m, k) + dense_parts_bytes(m, n, dense_windows(m, n, k)); }
 size_t dense_qmm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k) {
   return dense_qmm_rows_bytes(m, k) + dense_parts_bytes_up_to(m, n, k);
 }
 
-// x_prepared: rows already in the matmul's order with their group sums in sumx (x is then ignored)
+// xp: rows in the matmul's order, their group sums in sumx; act_rows: activations, row_max is that of the x in front
 static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, const uint16_t* xp, const uint16_t* sumx,
-                                void* y, uint32_t m, uint32_t n, uint32_t k, uint32_t n_win, bool out_f32, void* parts) {
+                                const float* row_max, bool act_rows, void* y, uint32_t m, uint32_t n, uint32_t k, uint32_t n_win, bool out_f32, void* parts) {
   const uint32_t ng = k / kGroup;
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
   QmmArgs d{};
@@ -1432,7 +1465,7 @@ static hipError_t dense_project(hipStream_t s, const mf_qtensor& w, int bits, co
     d.ternary = 1;
     d.dense[0].biases = d.dense[1].biases = w.scales;
   }
-  d.x = xp; d.sumx = sumx; d.x_stride = k; d.rows = n;
+  d.x = xp; d.sumx = sumx; d.row_max = row_max; d.act_rows = act_rows; d.x_stride = k; d.rows = n;
   d.pair_rows = n % (2 * kQmmRows) == 0;
   const uint32_t tiles = (m + kTileTokens - 1) / kTileTokens;
   const size_t part_stride = up256(sizeof(float) * static_cast<size_t>(m) * n) / sizeof(float);
@@ -1460,10 +1493,11 @@ hipError_t launch_dense_qmm(hipStream_t s, const mf_qtensor& w, int bits, const 
   uint8_t* base = static_cast<uint8_t*>(workspace);
   uint16_t* xp = reinterpret_cast<uint16_t*>(base);
   uint16_t* sumx = reinterpret_cast<uint16_t*>(base + up256(sizeof(uint16_t) * static_cast<size_t>(m) * k));
-  void* parts = reinterpret_cast<uint8_t*>(sumx) + up256(sums_bytes(m, k));
-  const hipError_t e = launch_prep_rows(s, x, xp, sumx, m, k);
+  float* row_max = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(sumx) + up256(sums_bytes(m, k)));
+  void* parts = base + dense_qmm_rows_bytes(m, k);
+  const hipError_t e = launch_prep_rows(s, x, xp, sumx, row_max, m, k);
   if (e != hipSuccess) return e;
-  return dense_project(s, w, bits, xp, sumx, y, m, n, k, dense_windows(m, n, k), out_f32, parts);
+  return dense_project(s, w, bits, xp, sumx, row_max, false, y, m, n, k, dense_windows(m, n, k), out_f32, parts);
 }
 
 // The block form of the shared expert / dense SwiGLU MLP: gate and up in one launch with the SwiGLU epilogue
@@ -1477,7 +1511,7 @@ bool dense_mlp_takes(const mf_qtensor& gate, const mf_qtensor& up, const mf_qten
 
 static size_t dense_mlp_rows_bytes(uint32_t d, uint32_t f, uint32_t t) {
   return up256(sizeof(uint16_t) * static_cast<size_t>(t) * f) + up256(sizeof(uint16_t) * static_cast<size_t>(t) * d) +
-         up256(sums_bytes(t, d)) + up256(sums_bytes(t, f));
+         up256(sums_bytes(t, d)) + up256(sums_bytes(t, f)) + up256(sizeof(float) * t);
 }
 // (the window results of gate / up and of down follow one another in the same place)
 size_t dense_mlp_needs(uint32_t d, uint32_t f, uint32_t t, uint32_t down_windows) {
@@ -1499,7 +1533,9 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
   base += up256(sums_bytes(t, d));
   uint16_t* sum_act = reinterpret_cast<uint16_t*>(base);
   base += up256(sums_bytes(t, f));
-  hipError_t e = launch_prep_rows(s, x, xp, sumx, t, d);
+  float* row_max = reinterpret_cast<float*>(base);
+  base += up256(sizeof(float) * t);
+  hipError_t e = launch_prep_rows(s, x, xp, sumx, row_max, t, d);
   if (e != hipSuccess) return e;
   const int code_bits = bits == MF_BITS_4 ? 4 : 2;
   QmmArgs q{};
@@ -1510,7 +1546,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     q.dense[0].biases = gate.scales;
     q.dense[1].biases = up.scales;
   }
-  q.x = xp; q.sumx = sumx; q.x_stride = d; q.rows = f; q.kdim = d; q.epi = 0; q.out = act; q.out_sums = sum_act;
+  q.x = xp; q.sumx = sumx; q.row_max = row_max; q.x_stride = d; q.rows = f; q.kdim = d; q.epi = 0; q.out = act; q.out_sums = sum_act;
   const uint32_t gu_win = dense_gate_up_windows(d);
   if (gu_win > 1) {
     // few rows (or a K too long for one launch's scale tables): the contraction in windows, both projections as
@@ -1525,14 +1561,14 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     if (e != hipSuccess) return e;
     const size_t chunks = static_cast<size_t>(t) * f / 8;
     dense_swiglu_combine_kernel<<<dim3(static_cast<uint32_t>((chunks + 255) / 256)), dim3(256), 0, s>>>(
-        pg, pu, gu_win, part_stride, act, sum_act, chunks, f / kGroup, 0.0f);
+        pg, pu, gu_win, part_stride, act, sum_act, row_max, chunks, f / kGroup, 0.0f);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else {
     e = launch_qmm(s, kTileTokens, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
     if (e != hipSuccess) return e;
   }
-  return dense_project(s, down, bits, act, sum_act, y, t, d, f, down_windows, false, base);
+  return dense_project(s, down, bits, act, sum_act, row_max, true, y, t, d, f, down_windows, false, base);
 }
 
 // Routes of a tile of the layer call's two matmuls.  A tile of 32 leaves registers and LDS for three workgroups a CU where one
@@ -1566,7 +1602,7 @@ struct PrefillWs {
   float* logits; uint32_t* idx; float* w; uint32_t* counts; uint32_t* offsets; uint32_t* starts;
   uint32_t* status; Tile* tiles[2]; mf_pair* sorted; uint16_t* acts; float* partials;
   uint16_t* sact; uint16_t* hs; uint16_t* gate;
-  uint16_t* xp; uint16_t* sum_x; uint16_t* sum_acts; uint16_t* sum_sact;
+  uint16_t* xp; uint16_t* sum_x; uint16_t* sum_acts; uint16_t* sum_sact; float* row_max;
   size_t bytes;
 };
 
@@ -1598,6 +1634,7 @@ PrefillWs prefill_carve(const mf_moe_config& c, uint32_t t, void* base) {
   p.sum_x = static_cast<uint16_t*>(take(sums_bytes(t, c.d)));
   p.sum_acts = static_cast<uint16_t*>(take(sums_bytes(pairs, c.f)));
   p.sum_sact = static_cast<uint16_t*>(take(sums_bytes(t, std::max<uint32_t>(c.shared_f, 64))));
+  p.row_max = static_cast<float*>(take(sizeof(float) * t));
   p.bytes = pos;
   return p;
 }
@@ -1694,6 +1731,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
       tail.xp = ws.xp;
       tail.w_sg = c.shared_f && !w.w_sg_q8.weights ? w.w_sg : nullptr;  // (an 8-bit gate row: its own launch below)
       tail.sums = ws.sum_x;
+      tail.row_max = ws.row_max;
       tail.gate = ws.gate;
       MF_TRY(launch_prefill_router(s, w.router_w, x, c.num_experts, c.d, t, c.d, ws.logits, &tail));
       x_prepared = tail.xp != nullptr;
@@ -1714,10 +1752,10 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   if (x_prepared) {
     // the router launch has prepared x (and the gate's logits) on the side
   } else if (want_gate && !gate_q8) {  // one pass over x: matmul order, group sums and the shared gate's logits
-    prep_x_gate_kernel<<<dim3((t + 3) / 4), dim3(256), 0, s>>>(x, ws.xp, ws.sum_x, w.w_sg, ws.gate, t, c.d);
+    prep_x_gate_kernel<<<dim3((t + 3) / 4), dim3(256), 0, s>>>(x, ws.xp, ws.sum_x, ws.row_max, w.w_sg, ws.gate, t, c.d);
     MF_TRY(hipGetLastError());
   } else {
-    MF_TRY(launch_prep_rows(s, x, ws.xp, ws.sum_x, t, c.d));
+    MF_TRY(launch_prep_rows(s, x, ws.xp, ws.sum_x, ws.row_max, t, c.d));
   }
   // the scalar gate stored as an 8-bit row (RealForwardRunner.swift:2925-2941): one wave per token, the
   // bits of mf_gemv(MF_BITS_8) -- and of the decode launch
@@ -1752,6 +1790,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
     d.dense[0] = w.shared_gate; d.dense[1] = w.shared_up;
     d.x = ws.xp; d.sumx = ws.sum_x; d.x_stride = c.d; d.rows = c.shared_f; d.kdim = c.d; d.epi = 0; d.out = ws.sact;
     d.out_sums = ws.sum_sact;
+    d.row_max = ws.row_max;
   }
   // phase 1: routed gate/up -> acts [pair, F]; shared gate/up -> sact [token, Fs]
   q.w_off[0] = w.offsets.gate_w; q.s_off[0] = w.offsets.gate_s; q.b_off[0] = ternary ? w.offsets.gate_s : w.offsets.gate_b;
@@ -1759,6 +1798,7 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   q.x = ws.xp; q.sumx = ws.sum_x; q.x_stride = c.d; q.gather = 1; q.rows = c.f; q.kdim = c.d; q.epi = 0;
   q.out = ws.acts;
   q.out_sums = ws.sum_acts;
+  q.row_max = ws.row_max;
   // The shared expert's work items (whole 64-row tiles, the longest of the launch) go first: a short batch
   // leaves workgroup slots over, and up to about 4096 tokens the launch ends sooner with them out of the way
   // (Qwen shape, layer: 2048 tokens 280.5 -> 274.5 us, 1024 tokens 191 -> 187 us, 4096 tokens 506 -> 503 us;
@@ -1778,12 +1818,14 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   q.x = ws.acts; q.sumx = ws.sum_acts; q.x_stride = c.f; q.gather = 0; q.rows = c.d; q.kdim = c.f;
   q.epi = narrow_routes ? 3 : 1; q.out = ws.partials;
   q.limit = 0.0f;
+  q.act_rows = 1;
   q.trace = nullptr;
   q.pair_rows = c.d % (2 * kQmmRows) == 0;
   if (c.shared_f) {
     d.dense[0] = w.shared_down;
     d.x = ws.sact; d.sumx = ws.sum_sact; d.x_stride = c.shared_f; d.rows = c.d; d.kdim = c.shared_f; d.epi = 2; d.out = ws.hs;
     d.pair_rows = q.pair_rows;
+    d.act_rows = 1;
   }
   const bool kres_q = kres_takes(q, pairs), kres_d = c.shared_f && kres_takes(d, t);
   // Both parts in one launch of one kernel: the resident one when it takes both (their K has to be the same), else the
