@@ -554,6 +554,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
   // (a set's address is the same for all lanes: a request is this offset against a scalar base, no vector arithmetic)
   uint32_t slot_at[ITS];
   uint2 xa[ITS][8], sx[ITS];  // this lane's x operands and chunk sums (filled below)
+  float rel[4];               // what the four tokens' results lack (rel_of_scale)
 #pragma unroll
   for (int j = 0; j < ITS; ++j)
     slot_at[j] = c * static_cast<uint32_t>(row_bytes) +
@@ -632,6 +633,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
     for (int t = 0; t < 4; ++t) {
       v[t] = acc[t] + dpp_f<0x124>(acc[t]);  // + lane - 4 (rotation inside the 16-lane row)
       v[t] = v[t] + dpp_f<0x128>(v[t]);      // + lane - 8
+      v[t] *= rel[t];
     }
     if ((lane & 12u) == 0)
       *reinterpret_cast<float4*>(part_of(wsub, pb, p, lane >> 4, c)) = make_float4(v[0], v[1], v[2], v[3]);
@@ -674,21 +676,43 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
   }
   // ---- this lane's x: token c, chunks (wsub * ITS + j) * 16 + b.  The first two stages' weight
   // loads are already on their way: the x rows come from L2 behind them.
+  uint4 raw[ITS][4];
+  uint32_t most = 0;  // largest magnitudes of the even and of the odd elements
 #pragma unroll
   for (int j = 0; j < ITS; ++j) {
     const uint32_t ch = (wsub * ITS + j) * 16 + b;
     const bool live = ch < n_chunks && c < a.T;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      raw[j][i] = make_uint4(0, 0, 0, 0);
+      if (live) raw[j][i] = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + ch * 32 + 8 * i);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < ITS; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) most = max_magnitudes(max_magnitudes(most, raw[j][i].x, raw[j][i].y), raw[j][i].z, raw[j][i].w);
+  // the scale of a token's x follows from what this wave has of it: its partial sums are brought back before they meet the other waves'
+  float largest = fmaxf(bf16_lo(most), bf16_hi(most));
+  largest = fmaxf(largest, dpp_f<0x124>(largest));
+  largest = fmaxf(largest, dpp_f<0x128>(largest));
+  largest = fmaxf(largest, __shfl_xor(largest, 16));
+  largest = fmaxf(largest, __shfl_xor(largest, 32));
+  const float x_scale = row_scale(largest * kRowScale);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) rel[t] = readlane_f(rel_of_scale(x_scale), t);
+#pragma unroll
+  for (int j = 0; j < ITS; ++j) {
     float sum = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (live) v = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + ch * 32 + 8 * i);
-      float part, largest = 0.0f;
-      const uint4 o = matmul_row8(v, kRowScale, &part, &largest);
+      float part;
+      const uint4 o = matmul_row8(raw[j][i], x_scale, &part);
       xa[j][2 * i] = make_uint2(o.x, o.y);
       xa[j][2 * i + 1] = make_uint2(o.z, o.w);
       sum += part;
     }
+    sum *= x_scale * kRowUnscale;
     const uint32_t hi = __float_as_uint(sum) & 0xFFFF0000u;
     const float r1 = sum - __uint_as_float(hi);
     const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;

@@ -377,15 +377,21 @@ __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
 }
 // what a result of rows at `scale` lacks: a factor that is 1 for ordinary rows (the matmuls' tables hold the powers of two of those)
 __device__ __forceinline__ float rel_of_scale(float scale) { return __uint_as_float(((2u * 127u + 64u) << 23) - __float_as_uint(scale)); }
-// eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and times `scale`; their sum in *sum (unscaled); *largest is
-// raised to the largest magnitude (at that scale)
-__device__ __forceinline__ uint4 matmul_row8(const uint4& v, float scale, float* sum, float* largest) {
+// the larger magnitudes of pairs of bf16 numbers, element by element, as pairs of bits (which compare as the numbers do)
+__device__ __forceinline__ uint32_t max_magnitudes(uint32_t m, uint32_t a, uint32_t b) {
+  typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
+  auto pair = [](uint32_t w) { return __builtin_bit_cast(u16x2_t, w & 0x7FFF7FFFu); };
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, m), __builtin_elementwise_max(pair(a), pair(b))));
+}
+// eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and times `scale`; their sum in *sum (unscaled); *largest (where
+// given) is raised to the largest magnitude (at that scale)
+__device__ __forceinline__ uint4 matmul_row8(const uint4& v, float scale, float* sum, float* largest = nullptr) {
   const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
   const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
   *sum = ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
   const float y0 = x0 * scale, y1 = x1 * scale, y2 = x2 * scale, y3 = x3 * scale, y4 = x4 * scale, y5 = x5 * scale, y6 = x6 * scale, y7 = x7 * scale;
-  *largest = fmaxf(*largest, fmaxf(fmaxf(fmaxf(fabsf(y0), fabsf(y1)), fmaxf(fabsf(y2), fabsf(y3))),
-                                   fmaxf(fmaxf(fabsf(y4), fabsf(y5)), fmaxf(fabsf(y6), fabsf(y7)))));
+  if (largest) *largest = fmaxf(*largest, fmaxf(fmaxf(fmaxf(fabsf(y0), fabsf(y1)), fmaxf(fabsf(y2), fabsf(y3))),
+                                                fmaxf(fmaxf(fabsf(y4), fabsf(y5)), fmaxf(fabsf(y6), fabsf(y7)))));
   return make_uint4(upper_halves(y0, y4), upper_halves(y1, y5), upper_halves(y2, y6), upper_halves(y3, y7));
 }
 

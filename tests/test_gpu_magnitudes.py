@@ -155,3 +155,26 @@ def test_qmm_of_rows_far_from_one(gpu, bits, m, n, k):
         assert op.encode(q, (x.double() * factor).to(torch.bfloat16), y, m, n, k) == "affine-matrix-core-bf16"
         out.append(y.double() / factor)
     assert all(torch.equal(out[0], o) for o in out[1:])
+
+
+@pytest.mark.parametrize("bits", [4, 2, 1])
+@pytest.mark.parametrize("m,n,t", [(2048, 4096, 8), (1088, 4992, 4), (4672, 11392, 1), (6656, 2048, 3), (64, 256, 5), (130, 320, 2)])
+def test_few_rows_far_from_one(gpu, bits, m, n, t):
+    """as test_qmm_of_rows_far_from_one, through the kernels of one to eight rows (the larger sizes: quad matrix instructions)"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m + n + t + bits)
+    packed = torch.randint(0, 256, (m, n * (4 if bits == 4 else 2) // 8), generator=gen, device="cuda", dtype=torch.uint8)
+    if bits == 1:
+        packed &= 0x55
+    scales = (0.01 + 0.01 * torch.rand(m, n // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+    biases = -scales if bits == 1 else (-0.1 * torch.rand(m, n // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+    q = ops.QuantizedTensor(packed, scales, None if bits == 1 else biases, bits, m, n)
+    x = (1.0 + torch.rand(t, n, generator=gen, device="cuda")).to(torch.bfloat16)
+    op = ops.DequantInt4GEMVMultiX(gpu)
+    out = []
+    for shifts in (torch.zeros(t), 59.0 - torch.arange(t) % 2, 100.0 - torch.arange(t) % 3 * 90, -80.0 + torch.arange(t) % 4 * 20):
+        factor = (2.0 ** shifts.double()).cuda()[:, None]
+        y = torch.zeros((t, m), dtype=torch.float32, device="cuda")
+        op.encode(q, (x.double() * factor).to(torch.bfloat16), y, m, n, t, output_float32=True)
+        out.append(y.double() / factor)
+    assert all(torch.equal(out[0], o) for o in out[1:]) and (out[0] != 0).all()
