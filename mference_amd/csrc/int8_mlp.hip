@@ -107,12 +107,14 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
   }
 }
 
-// ---- many token rows, on the bf16 matrix cores.  A code byte in the low half of a 16-bit word is the bf16 number
-// q * 2^-133 (the subnormals, mf_device.h), so an operand is a mask, or a shift and a mask, of a packed word; rows meet it times
-// 2^64 and in the order the masks leave the codes in, and the scale takes the powers of two back.  A K group is
+// ---- many token rows, on the bf16 matrix cores.  Codes 0..255 are bf16 numbers as they are, so a K group is
 // sum(q x) from four 32x32x16 products, one fp32 multiply-add with the row's scale, and the biases enter as one more
 // product per two groups: sum(x) of a group as three bf16 terms (all 24 bits) against the bias in three K slots.
 // Tokens are the M side, weight rows the N side: a lane ends with one weight row, its scale is a per-lane scalar.
+// (A code byte masked into the low half of a 16-bit word is the bf16 number q * 2^-133, as in mf_device.h, for half of the vector
+// instructions; but codes below 128 then enter with the exponent of 128, the matrix core aligns products by the operands' exponents, and
+// small codes beside large values of x lost bits: rms error over the size of the terms 2.4e-8 -> 7.8e-8 at 2112 x 2816, 300 rows, nine
+// codes of ten below 16 and one value of 1000 in a row, 3.9e-8 -> 4.3e-7 at 256 x 128.  The 2- and 4-bit codes sit at the top of the byte.)
 //
 // A workgroup is 64 weight rows (of each projection) x 64 tokens, waves 2 x 2.  A stage is 128 K values: x rows and
 // code rows come in as whole 128-byte lines, three stages ahead of their use (two sets of registers and an LDS buffer: a stage's
@@ -123,11 +125,10 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
 // meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
 // loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens: gate/up 47.6 -> 37.9 us, down 23.8 -> 20.0).
-// The whole MLP of 2816 x 2112, us, with codes converted one by one and a stage requested one ahead / now: 16 rows 47.5 / 44.2,
-// 300 54.3 / 50.3, 600 89 / 76, 2048 223 / 203; 704 x 8192, 16 rows 66.4 / 57.4, 300 93 / 84.
+// The MLP, us, with a stage requested one ahead / now: 2816 x 2112, 16 rows 48.3 / 49.5, 300 53.2 / 53.6, 600 87.9 / 84.4,
+// 2048 223 / 220; 704 x 8192, 16 rows 67.4 / 64.5, 300 92.4 / 87.1; 2048 x 2048, 16 rows 43.7 / 39.1, 1024 76.7 / 68.9.
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
-constexpr float kByteScale = 0x1p69f;  // q * 2^-133 meets x * 2^64
 
 // LONG: a set walks more than three stages; a short walk is a plain loop (instructions that run once cost their fetch:
 // 128 x 192, 16 rows 12.8 us with the long form, 11.6 with this one; 10.1 before stages were requested three ahead).
@@ -199,12 +200,9 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const u32x4_t v = xs[i];
-      const float x0 = bf16_lo(v.x), x1 = bf16_hi(v.x), x2 = bf16_lo(v.y), x3 = bf16_hi(v.y);
-      const float x4 = bf16_lo(v.z), x5 = bf16_hi(v.z), x6 = bf16_lo(v.w), x7 = bf16_hi(v.w);
-      part += ((x0 + x1) + (x2 + x3)) + ((x4 + x5) + (x6 + x7));
-      reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] =
-          u32x4_t{upper_halves(x0 * kRowScale, x2 * kRowScale), upper_halves(x1 * kRowScale, x3 * kRowScale),
-                  upper_halves(x4 * kRowScale, x6 * kRowScale), upper_halves(x5 * kRowScale, x7 * kRowScale)};
+      reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] = v;
+      part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
+              ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
     }
     part = group_sum(part, 2);
     if ((xq & 1) == 0) s_sum[buf][xt][xq >> 1] = part;
@@ -253,11 +251,19 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const uint4 w = s_w[buf][p][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
-          constexpr uint32_t kMask = 0x00FF00FFu;
-          tmp = mfma_bf16(bx[2 * c], make_uint4(w.x & kMask, (w.x >> 8) & kMask, w.y & kMask, (w.y >> 8) & kMask), tmp);
-          tmp = mfma_bf16(bx[2 * c + 1], make_uint4(w.z & kMask, (w.z >> 8) & kMask, w.w & kMask, (w.w >> 8) & kMask), tmp);
+          const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {  // eight codes -> eight bf16 numbers (a byte as fp32 has its bits in the upper half)
+            uint32_t o[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              const uint32_t word = ww[2 * u + (k >> 1)] >> (16 * (k & 1));
+              o[k] = upper_halves(static_cast<float>(word & 0xFFu), static_cast<float>((word >> 8) & 0xFFu));
+            }
+            tmp = mfma_bf16(bx[2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp);
+          }
         }
-        const float s = kByteScale * (g ? bf16_hi(sw[p]) : bf16_lo(sw[p]));
+        const float s = g ? bf16_hi(sw[p]) : bf16_lo(sw[p]);
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[p][i] = __builtin_fmaf(s, tmp[i], acc[p][i]);
       }

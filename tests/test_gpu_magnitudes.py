@@ -178,3 +178,51 @@ def test_few_rows_far_from_one(gpu, bits, m, n, t):
         op.encode(q, (x.double() * factor).to(torch.bfloat16), y, m, n, t, output_float32=True)
         out.append(y.double() / factor)
     assert all(torch.equal(out[0], o) for o in out[1:]) and (out[0] != 0).all()
+
+
+@pytest.mark.parametrize("d,f,t,apart", [(128, 64, 16, 1), (576, 128, 70, 1), (192, 2112, 530, 3)])
+def test_int8_matmul_of_small_codes_beside_large_values(gpu, d, f, t, apart):
+    """every group holds A and -A against the same code and, elsewhere, numbers from 1 to 2 against codes of 1 to 3: gate is
+    the sum of the latter, to the last bit of an fp32 sum whose largest term is A = 2^13 (24 bits of it: 2^-10 a term, of 64
+    terms of at least 1).  up is one and down picks its row, so y is gate in bf16 (two roundings, 2^-8 of it)."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + f + t)
+    x = (1.0 + torch.rand(t, d, generator=gen, device="cuda")).to(torch.bfloat16)
+    x[:, ::64], x[:, apart::64], x[:, 5] = 2.0 ** 13, -2.0 ** 13, 1.0
+    gate = torch.randint(1, 4, (f, d), generator=gen, device="cuda", dtype=torch.uint8)
+    gate[:, ::64] = gate[:, apart::64] = 1
+    up = torch.zeros((f, d), dtype=torch.uint8, device="cuda")
+    up[:, 5] = 1
+    down = torch.zeros((d, f), dtype=torch.uint8, device="cuda")
+    pick = torch.arange(d, device="cuda") % f
+    down[torch.arange(d, device="cuda"), pick] = 1
+    one = lambda r, c: torch.ones((r, c // 64), dtype=torch.bfloat16, device="cuda")
+    q = [ops.QuantizedTensor(c, one(*c.shape), torch.zeros_like(one(*c.shape)), 8, *c.shape) for c in (gate, up, down)]
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    ops.SharedExpertInt8(gpu, silu_activation=True).encode(x, *q, y, torch.zeros((t, f), dtype=torch.bfloat16, device="cuda"), t=t)
+    want = (x.double() @ gate.double().T)[:, pick]
+    assert ((y.double() - want).abs() <= want * (2.0 ** -8 + 2.0 ** -10)).all()
+
+
+@pytest.mark.parametrize("t", [16, 70])
+def test_int8_matmul_of_rows_far_from_one(gpu, t):
+    """the values the row kernels give, for rows of any magnitude"""
+    d, f = 192, 320
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(t)
+    def q(rows, n):
+        table = lambda s: (s * (0.0005 + 0.0005 * torch.rand(rows, n // 64, generator=gen, device="cuda"))).to(torch.bfloat16)
+        return ops.QuantizedTensor(torch.randint(0, 256, (rows, n), dtype=torch.uint8, generator=gen, device="cuda"), table(1), table(-128), 8, rows, n)
+    qs = [q(f, d), q(f, d), q(d, f)]
+    powers = torch.tensor(_POWERS, dtype=torch.float64, device="cuda").repeat(t)[:t, None]
+    x = (torch.randn(t, d, generator=gen, device="cuda").double() * 2.0 ** powers).to(torch.bfloat16)
+    op = ops.SharedExpertInt8(gpu, silu_activation=True)
+    y, rows = torch.zeros((2, t, d), dtype=torch.bfloat16, device="cuda")
+    scratch = torch.zeros((t, f), dtype=torch.bfloat16, device="cuda")
+    op.encode(x, *qs, y, scratch, t=t)
+    for i in range(0, t, 8):
+        n = min(8, t - i)
+        op.encode(x[i:i + n], *qs, rows[i:i + n], scratch, t=n)
+    top = rows.double().abs().amax(dim=1, keepdim=True)
+    assert torch.isfinite(rows).all() and (top > 0).all()
+    assert (((y.double() - rows.double()) / top).norm(dim=1) <= 2.0 ** -8 * (rows.double() / top).norm(dim=1)).all()  # (_rows_close)
