@@ -130,8 +130,9 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
 
-// LONG: a set walks more than three stages; a short walk is a plain loop (instructions that run once cost their fetch:
-// 128 x 192, 16 rows 12.8 us with the long form, 11.6 with this one; 10.1 before stages were requested three ahead).
+// LONG: a set walks more than three stages.  A shorter walk ends before requests three ahead pay for themselves, and instructions that run
+// once cost their fetch: it requests one stage ahead, its table entries by themselves.  us, long form / short: 128 x 192, 16 rows
+// 13.9 / 10.0; 384 x 256, 64 rows 18.0 / 14.5; 768 x 384 (three stages a set), 200 rows 21.2 / 19.1; 1024 x 1024 (four), 16 rows 23.6 / 27.1.
 template <int NPROJ, int KS, bool LONG>
 __global__ __launch_bounds__(256 * KS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
@@ -221,8 +222,8 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[p][r] = 0.0f;
 
-  // one stage out of LDS; sw, bw: the words of the scales and biases of its two groups
-  auto multiply = [&](uint32_t buf, const uint32_t (&sw)[NPROJ], const uint32_t (&bw)[NPROJ]) __attribute__((always_inline)) {
+  // one stage out of LDS; scale(p, g): of projection p and the stage's group g; bias(p): the bits of that of group h
+  auto multiply = [&](uint32_t buf, auto scale, auto bias) __attribute__((always_inline)) {
     // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0)
     {
       const float v = s_sum[buf][tok_m][h];
@@ -233,7 +234,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
       const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);
 #pragma unroll
       for (int p = 0; p < NPROJ; ++p) {
-        const uint32_t b = h ? bw[p] >> 16 : bw[p] & 0xFFFFu;
+        const uint32_t b = bias(p);
         acc[p] = mfma_bf16(av, make_uint4(b | (b << 16), b, 0, 0), acc[p]);
       }
     }
@@ -263,7 +264,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
             tmp = mfma_bf16(bx[2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp);
           }
         }
-        const float s = g ? bf16_hi(sw[p]) : bf16_lo(sw[p]);
+        const float s = scale(p, g);
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[p][i] = __builtin_fmaf(s, tmp[i], acc[p][i]);
       }
@@ -293,27 +294,39 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
           sw[p] = s4[u4];
           bw[p] = b4[u4];
         }
-        multiply(buf, sw, bw);
+        multiply(buf, [&](int p, int g) { return g ? bf16_hi(sw[p]) : bf16_lo(sw[p]); }, [&](int p) { return h ? bw[p] >> 16 : bw[p] & 0xFFFFu; });
       }
     }
   } else {
-    fetch(st0, xr[0], wreg[0]);
-    Tab tab = fetch_tab(min(2 * st0, ng - 1));
-    put(0, xr[0], wreg[0]);
+    uint16_t sc[NPROJ][2], bi[NPROJ];  // a stage's table entries
+    auto fetch_entries = [&](uint32_t st) __attribute__((always_inline)) {
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p) {
+        const size_t at = static_cast<size_t>(row) * ng;
+        sc[p][0] = a.S[p][at + min(2 * st, ng - 1)];
+        sc[p][1] = a.S[p][at + min(2 * st + 1, ng - 1)];
+        bi[p] = a.B[p][at + min(2 * st + h, ng - 1)];
+      }
+    };
+    if (st0 < st1) {
+      fetch(st0, xr[0], wreg[0]);
+      fetch_entries(st0);
+      put(0, xr[0], wreg[0]);
+      if (st0 + 1 < st1) fetch(st0 + 1, xr[0], wreg[0]);
+    }
 #pragma unroll 1
     for (uint32_t i = 0; i < n_walk; ++i) {
       __syncthreads();
-      if (i + 1 < n_walk) fetch(st0 + i + 1, xr[0], wreg[0]);
-      uint32_t sw[NPROJ], bw[NPROJ];
+      if (st0 + i >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
+      uint16_t sv[NPROJ][2], bv[NPROJ];
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        sw[p] = tab.S[p].x;
-        bw[p] = tab.B[p].x;
-        tab.S[p] = make_uint4(tab.S[p].y, tab.S[p].z, tab.S[p].w, 0);
-        tab.B[p] = make_uint4(tab.B[p].y, tab.B[p].z, tab.B[p].w, 0);
+      for (int p = 0; p < NPROJ; ++p) sv[p][0] = sc[p][0], sv[p][1] = sc[p][1], bv[p] = bi[p];
+      if (st0 + i + 1 < st1) {
+        put((i + 1) & 1u, xr[0], wreg[0]);
+        fetch_entries(st0 + i + 1);
+        if (st0 + i + 2 < st1) fetch(st0 + i + 2, xr[0], wreg[0]);
       }
-      multiply(i & 1u, sw, bw);
-      if (i + 1 < n_walk) put((i + 1) & 1u, xr[0], wreg[0]);
+      multiply(i & 1u, [&](int p, int g) { return bf16_to_f(sv[p][g]); }, [&](int p) -> uint32_t { return bv[p]; });
     }
   }
   if constexpr (KS == 2) {  // the second set's sums to the first, over the x buffers
