@@ -1580,13 +1580,16 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
 // 347 / 322, 777 647 / 623, 2048 1194 / 1224; 64 ternary experts of 2048 x 1024: 400 tokens 136 / 111, 1600 267 / 259, 2048 310 / 312.
 // The resident kernel on 4-bit rows of 512 keeps tiles of 64: its three workgroups a CU have half the codes in flight each
 // (400 tokens, 2048 x 512: 24.1 / 30.0 us; 93 tokens 20.6 / 20.3).
+// resident: that kernel takes the down projections of the call.  Where it does not, the ring on tiles of 64 / 32, us a call: 2176 x 512,
+// 128 experts, 93 tokens 67.5 / 65.3; 2048 x 512 beside a shared expert of 1024, 40 67.7 / 65.0, 93 74.4 / 70.2, 300 109.5 / 104.8;
+// 1664 x 512, 64 experts, 93 56.6 / 54.1, 200 (25 routes an expert) 65.2 / 67.2.
 struct PrefillTiles { uint32_t up, down; };
-static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t) {
+static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t, bool resident) {
   const bool two_bit = c.bits != MF_BITS_4 && !c.shared_f;
   const uint64_t few = static_cast<uint64_t>(two_bit ? 128 : 32) * c.num_experts;
   PrefillTiles p;
   p.up = static_cast<uint64_t>(t) * c.top_k <= few ? kSmallTile : kTileTokens;
-  p.down = c.bits == MF_BITS_4 && c.f == 512 ? kTileTokens : p.up;
+  p.down = resident && c.bits == MF_BITS_4 && c.f == 512 ? kTileTokens : p.up;
   return p;
 }
 
@@ -1705,7 +1708,49 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   hipError_t e;
 #define MF_TRY(call) do { e = (call); if (e != hipSuccess) return e; } while (0)
   const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const PrefillTiles tile = prefill_tiles(c, t);
+  QmmArgs q{};
+  // the routed experts' blobs: the pool in the matmul's order when the caller built one (mf_moe_tile_experts)
+  q.expert_base = static_cast<const uint8_t*>(w.expert_tiled ? w.expert_tiled : w.expert_base);
+  q.tiled = w.expert_tiled != nullptr;
+  q.expert_stride = w.expert_stride;
+  q.top_k = c.top_k;
+  q.limit = c.swiglu_limit;
+  // ternary experts are 2-bit codes whose bias is -scale: the kernels take the scale table as bias table
+  const int code_bits = c.bits == MF_BITS_4 ? 4 : 2;
+  const bool ternary = c.bits == MF_BITS_TERNARY;
+  q.ternary = ternary;
+  q.maple = static_cast<int>(c.maple_rounding);
+  // phase 2: routed down -> fp32 partials [token*K+rank, D]; shared down -> hs [token, D].
+  // Per-route results as bf16 numbers where the rounding rule narrows them anyway before they meet their
+  // weights -- MapleMoE's (maple_moe.metal:258), or on request (mf_moe_set_prefill_route_rounding; the
+  // reference's prefill keeps 16-bit per-route results, prefill.metal:817-819, 644-651): half the bytes
+  // written here and read by the reduce.  The caller's buffer of a ragged call stays fp32.
+  const bool narrow_routes = !ragged && (c.maple_rounding || h.narrow_routes);
+  QmmArgs q2 = q, d2{};
+  q2.w_off[0] = w.offsets.down_w; q2.s_off[0] = w.offsets.down_s; q2.b_off[0] = ternary ? w.offsets.down_s : w.offsets.down_b;
+  q2.x_stride = c.f; q2.rows = c.d; q2.kdim = c.f;
+  q2.epi = narrow_routes ? 3 : 1;
+  q2.limit = 0.0f;
+  q2.act_rows = 1;
+  q2.pair_rows = c.d % (2 * kQmmRows) == 0;
+  if (c.shared_f) {
+    d2.dense_mode = 1; d2.dense_rows = t; d2.top_k = c.top_k; d2.narrow = 1;
+    d2.dense[0] = w.shared_down; d2.dense[1] = w.shared_up;
+    d2.x_stride = c.shared_f; d2.rows = c.d; d2.kdim = c.shared_f; d2.epi = 2;
+    d2.pair_rows = q2.pair_rows;
+    d2.act_rows = 1;
+  }
+  const bool kres_q = kres_takes(q2, pairs), kres_d = c.shared_f && kres_takes(d2, t);
+  // Both parts in one launch of one kernel: the resident one when it takes both (their K has to be the same), else the
+  // ring.  Routed experts the resident kernel takes beside a shared expert of another width get it in a launch of their
+  // own once its gain outweighs the shared expert's launch, whose few items are then alone on the chip (layer, us, one
+  // launch / two, same bits: 4096 x 256, shared 512, top 6: 40 tokens 98 / 93, 2048 tokens 369 / 296; 2048 x 128, shared
+  // 512, top 8: 150 tokens 72 / 74, 300 tokens 87 / 85, 2048 tokens 176 / 143; 2048 x 512, shared 1024, top 8: 300 tokens
+  // 102 / 111, 777 tokens 155 / 155, 2048 tokens 274 / 262; routed 1024 or 2048 beside a resident shared expert: one
+  // launch always, 375 / 385; 4-bit experts alike, 4096 x 256, 2048 tokens 362 / 297).
+  const bool kres_both = kres_q && (!c.shared_f || (kres_d && d2.kdim == q2.kdim));
+  const bool apart = c.shared_f && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
+  const PrefillTiles tile = prefill_tiles(c, t, c.shared_f && !apart ? kres_both : kres_q);
   TileLists lists{{ws.tiles[0], tile.down != tile.up ? ws.tiles[1] : nullptr},
                   {prefill_tile_slots(c, t, tile.up), prefill_tile_slots(c, t, tile.down)}, {tile.up, tile.down}};
   bool x_prepared = false, fused_group = false;
@@ -1761,20 +1806,8 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // bits of mf_gemv(MF_BITS_8) -- and of the decode launch
   if (gate_q8) MF_TRY(launch_gemv(s, w.w_sg_q8, MF_BITS_8, x, ws.gate, 1, c.d, t, false));
 
-  QmmArgs q{};
-  // the routed experts' blobs: the pool in the matmul's order when the caller built one (mf_moe_tile_experts)
-  q.expert_base = static_cast<const uint8_t*>(w.expert_tiled ? w.expert_tiled : w.expert_base);
-  q.tiled = w.expert_tiled != nullptr;
-  q.expert_stride = w.expert_stride;
   q.sorted = ws.sorted;
   q.tiles = lists.list[0];
-  q.top_k = c.top_k;
-  q.limit = c.swiglu_limit;
-  // ternary experts are 2-bit codes whose bias is -scale: the kernels take the scale table as bias table
-  const int code_bits = c.bits == MF_BITS_4 ? 4 : 2;
-  const bool ternary = c.bits == MF_BITS_TERNARY;
-  q.ternary = ternary;
-  q.maple = static_cast<int>(c.maple_rounding);
   // the (4-bit) shared expert rides in the routed launches of the same phase
   const bool shared_rides = c.shared_f != 0;
   const int launch_bits = c.shared_f && code_bits != 4 ? kMixedBits : code_bits;
@@ -1806,48 +1839,23 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   const bool dense_first = shared_rides && pairs <= 32768;
   if (dense_first) MF_TRY(launch_qmm(s, tile.up, launch_bits, d, 2, dense_up, &q, lists.slots[0]));
   else MF_TRY(launch_qmm(s, tile.up, launch_bits, q, 2, lists.slots[0], shared_rides ? &d : nullptr, dense_up));
-  // phase 2: routed down -> fp32 partials [token*K+rank, D]; shared down -> hs [token, D]
-  q.w_off[0] = w.offsets.down_w; q.s_off[0] = w.offsets.down_s; q.b_off[0] = ternary ? w.offsets.down_s : w.offsets.down_b;
-  q.w_off[1] = q.s_off[1] = q.b_off[1] = 0;
-  // Per-route results as bf16 numbers where the rounding rule narrows them anyway before they meet their
-  // weights -- MapleMoE's (maple_moe.metal:258), or on request (mf_moe_set_prefill_route_rounding; the
-  // reference's prefill keeps 16-bit per-route results, prefill.metal:817-819, 644-651): half the bytes
-  // written here and read by the reduce.  The caller's buffer of a ragged call stays fp32.
-  const bool narrow_routes = !ragged && (c.maple_rounding || h.narrow_routes);
   if (lists.list[1]) q.tiles = lists.list[1];
-  q.x = ws.acts; q.sumx = ws.sum_acts; q.x_stride = c.f; q.gather = 0; q.rows = c.d; q.kdim = c.f;
-  q.epi = narrow_routes ? 3 : 1; q.out = ws.partials;
-  q.limit = 0.0f;
-  q.act_rows = 1;
-  q.trace = nullptr;
-  q.pair_rows = c.d % (2 * kQmmRows) == 0;
+  q2.sorted = q.sorted; q2.tiles = q.tiles; q2.row_max = q.row_max;
+  q2.x = ws.acts; q2.sumx = ws.sum_acts; q2.out = ws.partials;
   if (c.shared_f) {
-    d.dense[0] = w.shared_down;
-    d.x = ws.sact; d.sumx = ws.sum_sact; d.x_stride = c.shared_f; d.rows = c.d; d.kdim = c.shared_f; d.epi = 2; d.out = ws.hs;
-    d.pair_rows = q.pair_rows;
-    d.act_rows = 1;
+    d2.x = ws.sact; d2.sumx = ws.sum_sact; d2.out = ws.hs; d2.row_max = d.row_max;
   }
-  const bool kres_q = kres_takes(q, pairs), kres_d = c.shared_f && kres_takes(d, t);
-  // Both parts in one launch of one kernel: the resident one when it takes both (their K has to be the same), else the
-  // ring.  Routed experts the resident kernel takes beside a shared expert of another width get it in a launch of their
-  // own once its gain outweighs the shared expert's launch, whose few items are then alone on the chip (layer, us, one
-  // launch / two, same bits: 4096 x 256, shared 512, top 6: 40 tokens 98 / 93, 2048 tokens 369 / 296; 2048 x 128, shared
-  // 512, top 8: 150 tokens 72 / 74, 300 tokens 87 / 85, 2048 tokens 176 / 143; 2048 x 512, shared 1024, top 8: 300 tokens
-  // 102 / 111, 777 tokens 155 / 155, 2048 tokens 274 / 262; routed 1024 or 2048 beside a resident shared expert: one
-  // launch always, 375 / 385; 4-bit experts alike, 4096 x 256, 2048 tokens 362 / 297).
-  const bool kres_both = kres_q && (!shared_rides || (kres_d && d.kdim == q.kdim));
-  const bool apart = shared_rides && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
-  const int down_proj = q.pair_rows ? 2 : 1;
+  const int down_proj = q2.pair_rows ? 2 : 1;
   if (!shared_rides || apart) {
-    if (kres_q) MF_TRY(launch_qmm_kres(s, tile.down, code_bits, q, lists.slots[1], nullptr, 0));
-    else MF_TRY(launch_qmm(s, tile.down, code_bits, q, down_proj, lists.slots[1], nullptr, 0));
-    if (apart && kres_d) MF_TRY(launch_qmm_kres(s, tile.down, 4, d, dense_down, nullptr, 0));
-    else if (apart) MF_TRY(launch_qmm(s, tile.down, 4, d, down_proj, dense_down, nullptr, 0));
+    if (kres_q) MF_TRY(launch_qmm_kres(s, tile.down, code_bits, q2, lists.slots[1], nullptr, 0));
+    else MF_TRY(launch_qmm(s, tile.down, code_bits, q2, down_proj, lists.slots[1], nullptr, 0));
+    if (apart && kres_d) MF_TRY(launch_qmm_kres(s, tile.down, 4, d2, dense_down, nullptr, 0));
+    else if (apart) MF_TRY(launch_qmm(s, tile.down, 4, d2, down_proj, dense_down, nullptr, 0));
   } else if (kres_both) {
-    if (dense_first) MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, d, dense_down, &q, lists.slots[1]));
-    else MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, q, lists.slots[1], &d, dense_down));
-  } else if (dense_first) MF_TRY(launch_qmm(s, tile.down, launch_bits, d, down_proj, dense_down, &q, lists.slots[1]));
-  else MF_TRY(launch_qmm(s, tile.down, launch_bits, q, down_proj, lists.slots[1], &d, dense_down));
+    if (dense_first) MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, d2, dense_down, &q2, lists.slots[1]));
+    else MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, q2, lists.slots[1], &d2, dense_down));
+  } else if (dense_first) MF_TRY(launch_qmm(s, tile.down, launch_bits, d2, down_proj, dense_down, &q2, lists.slots[1]));
+  else MF_TRY(launch_qmm(s, tile.down, launch_bits, q2, down_proj, lists.slots[1], &d2, dense_down));
   if (ragged) return hipSuccess;  // the per-route results are the caller's: mf_moe_unpermute reduces them
   const uint16_t* hs = nullptr;
   const uint16_t* gate = nullptr;

@@ -660,3 +660,16 @@ def test_prefill_from_the_tiled_pool_gives_the_same_bits(gpu, oracle, bits, d, f
     import ctypes as C
     assert lib.mf_moe_tile_experts(moe._h, None, wts.experts.data_ptr(), wts.experts.stride(0), C.byref(wts.offsets),
                                    wts.experts.data_ptr()) == -1
+
+
+@pytest.mark.parametrize("d,f,fs,t", [(640, 512, 0, 40), (256, 512, 1024, 33), (256, 512, 1024, 600)])
+def test_prefill_rows_of_512_beside_what_the_resident_kernel_refuses(gpu, oracle, d, f, fs, t):
+    """the down projections' tiles are chosen for the kernel that runs: not the resident one at d = 640 or in one launch with a
+    wider shared expert (few routes); two launches, one of them resident, from 8192 routes on are the last case's neighbours"""
+    layer = oracle.synth_layer(ROOT_SEED + 0xB500 + d + t, d, f, 16, 8, bits=4, fs=fs)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    x = oracle.synth_x(ROOT_SEED + t, t, d)
+    y = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    moe.encode_prefill_layer(wts, ops.bf16_tensor(x), y, t)
+    torch.cuda.synchronize()
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(oracle.moe_layer(layer, x)[0]), f"d={d} fs={fs} t={t}")
