@@ -1236,9 +1236,11 @@ constexpr size_t kFusedLdsLimit = 150 * 1024;
 static uint32_t fused_pv_words(const mf_moe_config& c, const FusedSplit& sp) {
   return sp.by_units ? sp.units * (64u >> lanes_per_row_log2_dev(c.f, fused_epl(c))) * c.top_k : 0;
 }
-static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
+// what the normalised rows of a launch that makes x itself take beside the rest
+static size_t fused_norm_bytes(const mf_moe_config& c, uint32_t t, bool norm) { return norm ? 16 + static_cast<size_t>(t) * c.d * 2 : 0; }
+static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t t, bool norm) {
   FusedSplit sp = fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu);
-  if (fused_lds_base(c, num_cu, t) + 4 * static_cast<size_t>(fused_pv_words(c, sp)) > kFusedLdsLimit)
+  if (fused_lds_base(c, num_cu, t) + 4 * static_cast<size_t>(fused_pv_words(c, sp)) + fused_norm_bytes(c, t, norm) > kFusedLdsLimit)
     sp = fused_split(fused_epl(c), c.d, c.f, c.top_k, t, num_cu, false);
   return sp;
 }
@@ -1246,9 +1248,15 @@ static FusedSplit fused_split(const mf_moe_config& c, uint32_t num_cu, uint32_t 
 static bool fused_xprep(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
   return fused_lds_base(c, num_cu, t) + 4 * static_cast<size_t>(fused_xprep_words(c, t)) <= kFusedLdsLimit;
 }
-size_t fused_lds_bytes(const mf_moe_config& c, uint32_t num_cu, uint32_t t) {
-  const size_t pv = fused_pv_words(c, fused_split(c, num_cu, t)), xs = fused_xprep(c, num_cu, t) ? fused_xprep_words(c, t) : 0;
+static size_t fused_lds_bytes(const mf_moe_config& c, uint32_t num_cu, uint32_t t, bool norm) {
+  const size_t pv = fused_pv_words(c, fused_split(c, num_cu, t, norm)), xs = fused_xprep(c, num_cu, t) ? fused_xprep_words(c, t) : 0;
   return fused_lds_base(c, num_cu, t) + 4 * std::max(pv, xs);
+}
+
+// whether the rows of one token that a workgroup owns fit the h1 array (every token needs a workgroup)
+static bool fused_rows_fit(const mf_moe_config& c, uint32_t num_cu, uint32_t t, bool norm) {
+  const FusedSplit sp = fused_split(c, num_cu, t, norm);
+  return sp.rounds * sp.units * (64u >> lanes_per_row_log2_dev(c.f, fused_epl(c))) <= kMaxH1;
 }
 
 bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void* x, const void* y,
@@ -1261,12 +1269,7 @@ bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void*
                      (c.bits == MF_BITS_TERNARY && (!c.shared_f || c.shared_bits == MF_BITS_4));
   if (!combo || c.d % 8 != 0) return false;
   if (fused_lds_base(c, static_cast<uint32_t>(h.ctx->num_cu), t) > kFusedLdsLimit) return false;
-  {  // rows of one token a workgroup owns must fit the h1 array, and every token needs a workgroup
-    const uint32_t num_cu = static_cast<uint32_t>(h.ctx->num_cu);
-    if (num_cu < t) return false;
-    const FusedSplit sp = fused_split(c, num_cu, t);
-    if (sp.rounds * sp.units * (64u >> lanes_per_row_log2_dev(c.f, fused_epl(c))) > kMaxH1) return false;
-  }
+  if (static_cast<uint32_t>(h.ctx->num_cu) < t || !fused_rows_fit(c, static_cast<uint32_t>(h.ctx->num_cu), t, false)) return false;
   const uint32_t offs = w.offsets.gate_w | w.offsets.up_w | w.offsets.down_w;
   if (!aligned16(w.expert_base) || w.expert_stride % 16 || offs % 16) return false;
   if (!aligned16(w.router_w) || !aligned16(x) || !aligned16(y)) return false;
@@ -1290,7 +1293,7 @@ bool fused_norm_supported(const mf_moe& h, const mf_moe_layer_weights& w, const 
   if (!aligned16(hidden) || !aligned16(norm_w) || (delta && !aligned16(delta))) return false;
   if (!fused_supported(h, w, hidden, y, hidden, t)) return false;  // (x stands in as an aligned pointer)
   const uint32_t num_cu = static_cast<uint32_t>(h.ctx->num_cu);
-  return fused_lds_bytes(c, num_cu, t) + 16 + static_cast<size_t>(t) * c.d * 2 <= kFusedLdsLimit;
+  return fused_rows_fit(c, num_cu, t, true) && fused_lds_bytes(c, num_cu, t, true) + fused_norm_bytes(c, t, true) <= kFusedLdsLimit;
 }
 
 // One instance in the form (rows or units of stage C) its shape takes; an instance with every dimension literal exists
@@ -1351,7 +1354,7 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
   a.maple = static_cast<int>(c.maple_rounding);
   const dim3 grid(static_cast<uint32_t>(h.ctx->num_cu)), block(kFusedThreads);
   const uint32_t num_cu = static_cast<uint32_t>(h.ctx->num_cu);
-  size_t lds = fused_lds_bytes(c, num_cu, t);
+  size_t lds = fused_lds_bytes(c, num_cu, t, norm != nullptr);
   a.stage_words = fused_stage_words(c, num_cu, t);
   a.xprep = fused_xprep(c, num_cu, t) ? 1 : 0;
   if (norm) {  // the normalised rows behind everything else in LDS
@@ -1361,7 +1364,7 @@ hipError_t launch_fused_decode(hipStream_t s, const mf_moe& h, const mf_moe_laye
     a.xn_off = static_cast<uint32_t>((lds + 15) & ~size_t(15));
     lds = a.xn_off + static_cast<size_t>(t) * c.d * 2;
   }
-  const FusedSplit sp = fused_split(c, num_cu, t);
+  const FusedSplit sp = fused_split(c, num_cu, t, norm != nullptr);
   a.g = fused_geo(c, num_cu, t, sp);
 #define MF_FUSED(B, SB, SHAPE) return launch_instance<B, SB, SHAPE, false>(sp.by_units, grid, block, lds, s, a)
 #define MF_FUSED_N(B, SB, SHAPE) return launch_instance<B, SB, SHAPE, true>(sp.by_units, grid, block, lds, s, a)

@@ -1415,3 +1415,35 @@ def test_a_layer_holds_no_tensor_it_does_not_name(gpu, oracle):
     lw.experts = lw.experts.cpu()
     with pytest.raises(ValueError):
         run()
+
+
+def test_norm_in_front_where_the_pair_values_do_not_fit(gpu):
+    """2-bit experts of 4096, top 8, six and more rows: the units form's values and the normalised rows do not fit the LDS together,
+    so the launch takes the rows form -- it still makes x itself (stage stamp 7), with the bits of the norm launch and the chain"""
+    d, f, e, k, t = 3520, 4096, 16, 8, 8
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(35)
+    off, _, stride = ops.expert_blob_layout(d, f, 2)
+    pool = torch.zeros((e, stride), dtype=torch.uint8, device="cuda")
+    for name, rows, n in (("gate", f, d), ("up", f, d), ("down", d, f)):
+        table = lambda s: (s * (0.01 + 0.01 * torch.rand(e, rows * n // 64, generator=gen, device="cuda"))).to(torch.bfloat16)
+        for part, v in (("w", torch.randint(0, 256, (e, rows * n // 4), generator=gen, device="cuda", dtype=torch.uint8)), ("s", table(1)), ("b", table(-1.5))):
+            at, v = getattr(off, f"{name}_{part}"), v.view(torch.uint8)
+            pool[:, at:at + v.shape[1]] = v
+    randn = lambda *s: torch.randn(s, generator=gen, device="cuda")
+    lw = ops.MoELayerWeights((randn(e, d) * 0.02).to(torch.bfloat16), pool, off, None, None)
+    hidden, norm = randn(t, d).to(torch.bfloat16), (1.0 + 0.1 * randn(d)).to(torch.bfloat16)
+    out = []
+    for fused in (True, False):
+        moe = ops.MoE(gpu, d, f, e, k, bits=2)
+        moe.set_fused(fused)
+        stamps = torch.zeros(256 * 8, dtype=torch.int64, device="cuda")
+        if fused:
+            moe.set_phase_trace(stamps)
+        h, y = hidden.clone(), torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        moe.encode_decode_layer_normed(lw, h, norm, y, t=t)
+        moe.status()
+        if fused:
+            assert bool((stamps.view(256, 8)[:, 7] > 0).all())
+        out.append((ops.bf16_bits(h), ops.bf16_bits(y)))
+    assert all(np.array_equal(a, b) for a, b in zip(*out)) and out[0][1].any()
