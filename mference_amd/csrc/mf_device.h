@@ -367,6 +367,8 @@ __device__ __forceinline__ float scale_of_window(float m, float low, float high)
   return b >= __float_as_uint(high) ? 0x1p2f : b - 1u < __float_as_uint(low) - 1u ? 0x1p126f : kRowScale;
 }
 __device__ __forceinline__ float row_scale(float m) { return scale_of_window(m, 0x1p5f, 0x1p121f); }
+// ... by the sum of the squares of up to 192 numbers (infinite, or zero, where that is what they come to)
+__device__ __forceinline__ float scale_of_squares(float s) { return s < 0x1p-110f ? 0x1p126f : s < 0x1p113f ? kRowScale : 0x1p2f; }
 // The activations between an MLP's products are scaled before the largest is known, by that of the token's x (m, as above): from
 // 2^-20 to 2^20 in x they are products of two sums of such numbers and stay within 2^-61 .. 2^62 unless the weights do not.
 __device__ __forceinline__ float act_scale(float m) { return scale_of_window(m, 0x1p44f, 0x1p84f); }
@@ -377,12 +379,6 @@ __device__ __forceinline__ uint32_t upper_halves(float lo, float hi) {
 }
 // what a result of rows at `scale` lacks: a factor that is 1 for ordinary rows (the matmuls' tables hold the powers of two of those)
 __device__ __forceinline__ float rel_of_scale(float scale) { return __uint_as_float(((2u * 127u + 64u) << 23) - __float_as_uint(scale)); }
-// the larger magnitudes of pairs of bf16 numbers, element by element, as pairs of bits (which compare as the numbers do)
-__device__ __forceinline__ uint32_t max_magnitudes(uint32_t m, uint32_t a, uint32_t b) {
-  typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
-  auto pair = [](uint32_t w) { return __builtin_bit_cast(u16x2_t, w & 0x7FFF7FFFu); };
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, m), __builtin_elementwise_max(pair(a), pair(b))));
-}
 // eight bf16 numbers of a row in the matmul's order (0,4,1,5,2,6,3,7) and times `scale`; their sum in *sum (unscaled); *largest (where
 // given) is raised to the largest magnitude (at that scale)
 __device__ __forceinline__ uint4 matmul_row8(const uint4& v, float scale, float* sum, float* largest = nullptr) {
