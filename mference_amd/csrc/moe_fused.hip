@@ -647,10 +647,12 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     __syncthreads();
     trace_mark(a, 2);
     if (rank_count && router_mode == 0 && E <= kWaveSelect && 4 * K <= E) {
-      // Few experts: a wave per token takes the best K times in registers, without a barrier before its result.  1024 x 384,
-      // 48 experts, top 4: 12.0 / 11.7 us (one token), 17.2 / 16.5 (eight); 2816 x 448, 64 experts, top 6, 2-bit: 15.7 / 14.9;
-      // 96 experts, top 8, four tokens: 18.6 / 17.5.  Counting ranks stays where there is little to count (30 experts, top 8,
-      // eight tokens: 38.5, by waves 40.2) and behind a full softmax, whose wave would do both (64 experts: 12.0, 12.6).
+      // Few experts: a wave per token takes the best K times in registers, without a barrier before its result.  Layer of 1024 x 384, us,
+      // counted / by waves, one and eight tokens: 48 experts, top 4 12.1 / 11.5, 17.5 / 15.5, top 8 12.7 / 12.6, 21.6 / 20.3; 96, top 4
+      // 12.7 / 11.6, 20.4 / 15.6; 128, top 4 12.5 / 11.6, 17.4 / 15.7, top 8 13.5 / 12.8, 21.9 / 20.4.  Counting stays where there is
+      // little to count (30 experts, top 8, eight tokens: 38.5, by waves 40.2) and behind a full softmax, whose wave would do
+      // both (64 experts: 12.0, 12.6).  The line is where two logits a lane end; four a lane (no instance has them) measured 160 experts, top 4
+      // 13.3 / 11.9, 26.4 / 16.4; 256, top 8, one, four and eight tokens 13.4 / 13.3, 17.1 / 16.4, 21.6 / 21.7.
       if (wv < T) {
         if (E <= kWave) topk_select_sorted<1, 3>(s_lg + wv * Ep, E, K, s_idx + wv * K, s_sc + wv * K, lane);
         else topk_select_sorted<2, 3>(s_lg + wv * Ep, E, K, s_idx + wv * K, s_sc + wv * K, lane);
