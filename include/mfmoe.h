@@ -17,8 +17,12 @@
  *                                      is fp32 and the reference's narrowing points
  *                                      are kept, narrowing to bf16 instead of fp16
  *
- * Activations that meet quantized weights may count as infinite from a magnitude of
- * 2^63 on (most kernels keep them times 2^64); an infinity or a NaN stays with its row.
+ * Activations that meet quantized weights may have any magnitude: the kernels keep a
+ * row (or a part of it) times a power of two that its largest magnitude decides.  The
+ * activations between the two products of an MLP take it from the token's x instead and
+ * may count as infinite from 2^64 on where the largest of x lies between 2^-20 and 2^20,
+ * from 2^2 on where it is smaller, from 2^126 on where it is larger.  Scales of quantized
+ * weights may overflow from a magnitude of 2^63 on.  An infinity or a NaN stays with its row.
  *
  * All pointers are DEVICE pointers unless a parameter says "host".  Activations
  * and scale/bias tables must be 2-byte aligned; packed weights may have any

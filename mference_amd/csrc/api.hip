@@ -782,11 +782,13 @@ mf_status mf_moe_prefill_layer(mf_moe* h, mf_stream stream, const mf_moe_layer_w
                   (!c.shared_f || (mf::aligned16(wts->shared_gate.weights) && mf::aligned16(wts->shared_up.weights) &&
                                    mf::aligned16(wts->shared_down.weights) &&
                                    !(wts->w_sg && !wts->w_sg_q8.weights && !mf::aligned16(wts->w_sg))));
-  // ... and up to one decode launch of rows always: six dependent launches do not pay there (us, decode / matmul:
-  // 2816 x 704, 128 experts, top 8: 1 row 18.5 / 56, 8 rows 58 / 98; 1088 x 576, 64 experts, top 4: 1 row 15 / 41,
-  // 8 rows 32 / 47).  Two of them where the routes rarely share an expert and no shared expert is read again (the first
-  // layer: 9 rows 78 / 99, 16 rows 113 / 135, 17 rows 132 / 137; 2-bit codes cost the decode launch more, 1472 x 1408,
-  // 92 experts, top 7: 12 rows 97 / 91).
+  // ... and up to one decode launch of rows always: six dependent launches do not pay there (us, decode / matmul at 1, 4
+  // and 8 rows: 2816 x 704, 128 experts, top 8 16 / 54, 33 / 68, 56 / 72; 1088 x 576, 64 experts, top 4, shared 576
+  // 14 / 37, 19 / 41, 27 / 42; 3136 x 1216, 64 experts, top 8, 2-bit 22 / 56, 48 / 70, 83 / 75).  Two of them where the routes
+  // rarely share an expert, no shared expert is read again and the codes are not 2-bit.  The two meet at about 9 rows since the
+  // matmuls' tiles hold 32 routes (first layer 9 rows 69 / 72, 12 rows 83 / 73, 16 rows 102 / 79, 17 rows 117 / 80; 2112 x 320, 96
+  // experts, top 6 48 / 52 at 12 and 71 / 53 at 17), before that at 17 (132 / 137): from 10 to 16 rows the second launch is kept for the
+  // decode launch's bits, not for its time.
   const bool few = t <= MF_MAX_TOKENS ||
                    (t <= 2 * MF_MAX_TOKENS && !c.shared_f && c.bits != MF_BITS_2 && t * c.top_k <= c.num_experts &&
                     h->fused && mf::fused_supported(*h, *wts, x, y, nullptr, MF_MAX_TOKENS));
