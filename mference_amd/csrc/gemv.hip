@@ -1018,21 +1018,21 @@ bool rows_lane_ordered(uint32_t m, uint32_t n, uint32_t num_cu) {
 // have to agree: where the other kernels give a row the same bits for every number of token rows, the quad kernel takes
 // all numbers or none.  The lines are where what four rows gain is more than what one row loses, the one row's share
 // counted twice (us, other kernels / this one; one row; four rows):
-//   4-bit of K below 2048, gate / up from 36 rows a CU on (9216 x 1536: 7.6 / 9.0; 19.9 / 10.1; 5120 x 1536: 5.4 / 7.2;
-//   13.7 / 8.2; one projection, 9216 x 1536: 4.9 / 6.8; 12.1 / 8.4);
-//   4-bit above, from 8 M weights a projection on (4096 x 3136: 6.5 / 7.0; 13.3 / 8.5, gate / up 9.4 / 8.8; 20.3 / 10.3;
-//   9216 x 3008: 8.0 / 9.7; 21.1 / 12.5; 2048 x 3136: 4.5 / 5.7; 10.7 / 6.3, and eight 10.5 / 12.1);
-//   2-bit of K up to 4096, from 16 rows a CU on (5120 x 1024: 3.7 / 4.4; 9.7 / 5.0; 4096 x 2560: 5.0 / 6.4; 13.5 / 7.9,
-//   gate / up 6.2 / 7.4; 19.9 / 8.7; 17408 x 4096: 10.1 / 12.2; 21.2 / 14.5, and eight 124 / 27; 2048 x 3136: 3.7 / 5.4;
-//   8.7 / 6.1);
-//   2-bit above, from 8 M weights on (6656 x 6592: 14.7 / 10.6; 34.0 / 12.1; 1024 x 6592: 4.9 / 5.1).
-// (What eight rows gain, since two blocks of rows share a launch, is more still: 2-bit 2048 x 2048 10.5 / 6.6, gate / up 13.4 / 7.7,
-// one row 3.2 / 4.9, 4.0 / 6.1: its share keeps the line where it is.)
+//   4-bit of K below 2048, gate / up from 36 rows a CU on (9216 x 1536: 7.6 / 8.7; 20.0 / 9.9; 5120 x 1536: 5.1 / 7.3;
+//   12.7 / 8.1; one projection, 9216 x 1536: 5.1 / 7.2; 12.1 / 8.5);
+//   4-bit above, from 8 M weights a projection on (4096 x 3136: 6.6 / 7.7; 13.3 / 8.8, gate / up 9.5 / 9.6; 20.4 / 10.5;
+//   9216 x 3008: 8.1 / 10.4; 21.1 / 12.9; 2048 x 3136: 4.5 / 6.3; 10.5 / 6.7, and eight 10.3 / 8.2);
+//   2-bit of K up to 4096, from 16 rows a CU on (5120 x 1024: 3.8 / 4.8; 9.7 / 5.3; 4096 x 2560: 4.8 / 6.3; 13.2 / 7.8,
+//   gate / up 5.9 / 7.5; 18.4 / 9.0; 17408 x 4096: 10.6 / 12.5; 21.3 / 14.2, and eight 124 / 19; 2048 x 3136: 3.7 / 6.2;
+//   8.7 / 6.6);
+//   2-bit above, from 8 M weights on (6656 x 6592: 14.9 / 11.5; 34.1 / 12.6; 1024 x 6592: 5.0 / 5.5).
+// (What eight rows gain, since two blocks of rows share a launch, is more still: 2-bit 2048 x 2048 10.5 / 6.7, gate / up 13.3 / 7.7,
+// one row 3.2 / 4.8, 4.0 / 5.6: its share keeps the line where it is.)
 // Elsewhere the number of token rows decides (us per MLP, other kernels / this one): one row, where a step of
-// rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 30.5 / 27.6, 2-bit 40.6 / 25.3; 3840 x 7680, a
-// sixteenth empty: 22.2 / 22.9); two and more, from 4 M weights on (3136 x 9664, four rows: 4-bit 72 / 27, 2-bit 71 / 25;
-// one projection, 4-bit 1088 x 4992, two, four, eight rows: 6.7 / 7.0, 13.5 / 8.0, 13.8 / 9.2; 2-bit 1024 x 6592: 7.2 / 6.1, 11.4 / 6.5,
-// 15.9 / 9.0).
+// rows_stream_kernel would be a fifth empty (4672 x 11392: 4-bit 34.0 / 31.2, 2-bit 43.8 / 28.8; 3840 x 7680, a
+// sixteenth empty: 23.6 / 25.5); two and more, from 4 M weights on (3136 x 9664, four rows: 4-bit 76 / 29, 2-bit 74 / 27;
+// one projection, 4-bit 1088 x 4992, two, four, eight rows: 6.7 / 7.3, 13.3 / 7.9, 13.7 / 9.0; 2-bit 1024 x 6592: 7.0 / 5.8, 11.3 / 6.5,
+// 15.8 / 8.9).
 template <int BITS, int NPROJ>
 bool rows_quad_takes(QuadFit fit, uint32_t m, uint32_t n, uint32_t t, uint32_t num_cu) {
   constexpr bool two = BITS == kBits2;
