@@ -165,14 +165,19 @@ __device__ __forceinline__ float group_sum(float v, int lanes) {
 __device__ __forceinline__ float wave_sum(float v) { return group_sum(v, kWave); }
 
 // maximum over the wave, returned in every lane (no NaN inputs)
-__device__ __forceinline__ float wave_max(float v) {
+// the largest of the lower and of the upper half of a wave
+__device__ __forceinline__ float2 half_wave_max(float v) {
   v = fmaxf(v, dpp_f<0xB1>(v));
   v = fmaxf(v, dpp_f<0x4E>(v));
   v = fmaxf(v, dpp_f<0x141>(v));
   v = fmaxf(v, dpp_f<0x140>(v));
   const float r0 = readlane_f(v, 0), r1 = readlane_f(v, 16);
   const float r2 = readlane_f(v, 32), r3 = readlane_f(v, 48);
-  return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
+  return make_float2(fmaxf(r0, r1), fmaxf(r2, r3));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  const float2 h = half_wave_max(v);
+  return fmaxf(h.x, h.y);
 }
 
 // ------------------------------------------- device-coherent accesses

@@ -173,7 +173,7 @@ struct FusedGeo {
   uint32_t c_units;    // output units of one workgroup: per round (rows form) or in all (units form)
   uint32_t c_rounds;   // rounds (rows form)
   uint8_t lpr_d, lpr_f, lpr_sd, lpr_sf;  // log2 of the lanes per row: rows of D and F (routed), of D and Fs (shared)
-  FastDiv E, n_sl, rgf, K, srg, c_wgs_div, rpr;
+  FastDiv E, n_sl, rgf, K, srg, c_wgs_div, rpr, x_runs;
 };
 
 struct FusedArgs {
@@ -311,8 +311,10 @@ __host__ __device__ __forceinline__ uint32_t fused_poll_waves(uint32_t n2) {
   const uint32_t w = (n2 + kWave - 1) / kWave;
   return w < 8 ? w : 8;
 }
-__host__ __device__ __forceinline__ uint32_t fused_slice_waves(uint32_t n, uint32_t n_poll) {
-  const uint32_t w = (n + kWave - 1) / kWave;
+// (a run: up to 64 slices of one token, on the lanes of a wave, or all of them on half a wave's where that holds them)
+__host__ __device__ __forceinline__ uint32_t fused_x_runs(uint32_t n_sl) { return (n_sl + kWave - 1) / kWave; }
+__host__ __device__ __forceinline__ uint32_t fused_slice_waves(uint32_t t, uint32_t n_sl, uint32_t n_poll) {
+  const uint32_t w = n_sl <= kWave / 2 ? (t + 1) / 2 : t * fused_x_runs(n_sl);
   return w < kFusedWaves - n_poll - 4 ? w : kFusedWaves - n_poll - 4;
 }
 
@@ -481,11 +483,14 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   // Who does what while the logits are on their way: the top waves poll for them (n_poll waves),
   // the waves below those build the x slices, the bottom waves have the rows of stage A.
   const uint32_t n2 = S::kGiven ? 0 : (S::kAnyE ? T * E + 1 : T * E) / 2;  // 16-byte pieces of tagged logits
-  const uint32_t n_poll = fused_poll_waves(n2), n_xw = fused_slice_waves(T * n_sl, n_poll);
+  const uint32_t n_poll = fused_poll_waves(n2), n_xw = fused_slice_waves(T, n_sl, n_poll);
+  const uint32_t x_runs = fused_x_runs(n_sl);
 
-  // The scales of a token's x and activations, at [token] and MF_MAX_TOKENS behind it.  One token: the largest magnitude, times kRowScale, that
-  // each of the waves that build slices met.  (s_v is free until stage C.)
+  // The scales of every token's activations and x.  Tokens of several runs: the runs' largest magnitudes, times kRowScale, first, and the
+  // scales behind the requests of stage B.  (s_v is free until stage C.)
   float* s_scale = s_v;
+  float* s_xscale = s_v + MF_MAX_TOKENS;
+  float* s_most = s_v + 2 * MF_MAX_TOKENS;
 
   // ------------------------------------------------------------- stage A
   // Router rows are on the critical path and their logits are gathered by everybody: they go in
@@ -573,19 +578,29 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
         }
       }
     }
-    // the x slices of the routed rows, and every token's scales: a wave takes whole tokens (one token: a run of its slices)
+    // the x slices of the routed rows, and the scales: a wave takes whole runs, two tokens' where half of its lanes hold one
+    // (us a layer, a wave a token before: 1024 x 384, two tokens 13.8 -> 13.1; 256 ternary experts of 512, eight 24.0 -> 22.9; large 2-bit layer, eight
+    // 122 -> 120.7; 2816 x 704, two 40.6 -> 40.1)
     if (wv + n_poll + n_xw >= kFusedWaves && wv + n_poll < kFusedWaves) {
-      const uint32_t xw = wv + n_poll + n_xw - kFusedWaves;
-      for (uint32_t tok = S::T == 1 ? 0u : xw; tok < T; tok += S::T == 1 ? 1u : n_xw) {
+      const uint32_t half = n_sl <= kWave / 2 ? 1u : 0u, run_lane = lane & ((kWave >> half) - 1), runs = T * x_runs;
+      for (uint32_t r0 = (wv + n_poll + n_xw - kFusedWaves) << half; r0 < runs; r0 += n_xw << half) {
+        const uint32_t run = r0 + (lane >> (6 - half));
+        const uint32_t tok = S::T == 1 ? 0u : S::D != kDyn ? run / x_runs : fdiv(run, a.g.x_runs);
+        const uint32_t sl = (run - tok * x_runs) * kWave + run_lane;
         float largest = 0.0f;
-        for (uint32_t sl = S::T == 1 ? xw * kWave + lane : lane; sl < n_sl; sl += S::T == 1 ? n_xw * kWave : kWave) {
+        if (run < runs && sl < n_sl) {
           const XSlice<BITS> xs = load_expert_x<BITS, true>(xin + static_cast<size_t>(tok) * D + sl * kEPL, kRowScale, &largest);
           if (xprep) store_xslice_lds<BITS>(s_xq, s_xsum, tok, n_sl, sl, xs);
         }
-        largest = wave_max(largest);
-        if (lane == 0) {
-          s_scale[S::T == 1 ? xw : tok] = S::T == 1 ? largest : row_scale(largest);
-          if (S::T != 1) s_scale[MF_MAX_TOKENS + tok] = act_scale(largest);
+        const float2 most = half_wave_max(largest);
+        largest = half ? (lane < kWave / 2 ? most.x : most.y) : fmaxf(most.x, most.y);
+        if (run < runs && run_lane == 0) {
+          if (x_runs == 1) {
+            s_scale[tok] = act_scale(largest);
+            s_xscale[tok] = row_scale(largest);
+          } else {
+            s_most[run] = largest;
+          }
         }
       }
     }
@@ -805,7 +820,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   };
 
   // lane t: the scale of token t's x (one token: the same in every lane); read behind the first requests of stage B
-  float x_scale = kRowScale, one_act_scale = kRowScale;
+  float x_scale = kRowScale;
   auto of_token = [&](float v, uint32_t token) __attribute__((always_inline)) { return S::T == 1 ? v : readlane_f(v, static_cast<int>(token)); };
 
   // ------------------------------------------------------------- stage B
@@ -881,17 +896,17 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
     if (S::kStatic || item < last) fetch(item < n_items ? item : 0u, 0, cur);  // (literal shapes: no branch around the loads)
     if constexpr (!UNITS) request_down_rows();
     issue_fence();
-    if (S::T == 1) {
-      float most = s_scale[0];
-      for (uint32_t w = 1; w < n_xw; ++w) most = fmaxf(most, s_scale[w]);
-      most = readlane_f(most, 0);
+    x_scale = s_xscale[S::T == 1 ? 0u : lane & (MF_MAX_TOKENS - 1)];
+    if (x_runs != 1) {
+      const float* of_lane = s_most + (lane < T ? lane * x_runs : 0u);
+      float most = of_lane[0];
+      for (uint32_t r = 1; r < x_runs; ++r) most = fmaxf(most, of_lane[r]);
+      if (S::T == 1) most = readlane_f(most, 0);
       x_scale = row_scale(most);
-      one_act_scale = act_scale(most);
-    } else {
-      x_scale = s_scale[lane & (MF_MAX_TOKENS - 1)];
+      if (threadIdx.x < T) s_scale[threadIdx.x] = act_scale(most);  // (read behind the barriers of stage B)
     }
     // A token out of the ordinary window of magnitudes has its slices made again (the same for all waves)
-    const bool again = S::T == 1 ? x_scale != kRowScale : __any(lane < T && x_scale != kRowScale);
+    const bool again = S::T == 1 ? __any(x_scale != kRowScale) : __any(lane < T && x_scale != kRowScale);
     if (__builtin_expect(xprep && again, 0)) {
       for (uint32_t t = 0; t < T; ++t) {
         const float scale = of_token(x_scale, t);
@@ -925,7 +940,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       const uint32_t it = first + (i >> rpw_log2), pair = pair_of(it);
       const uint32_t row = ((it - pair * rgf) << rpw_log2) + (i & (rpw - 1));
       // moe.metal:27-34, 528; maple_moe.metal:153-164; exchanged at the scale that the slices of the token's activations have
-      const float scale = S::T == 1 ? one_act_scale : s_scale[MF_MAX_TOKENS + (S::K != kDyn ? pair / K : fdiv(pair, a.g.K))];
+      const float scale = s_scale[S::T == 1 ? 0u : S::K != kDyn ? pair / K : fdiv(pair, a.g.K)];
       const float act = bf16_to_f(routed_activation(s_gu[2 * i], s_gu[2 * i + 1], limit, maple)) * scale;
       const uint32_t word = (__float_as_uint(act) >> 16) | (tag16 << 16);
       if (row < F) store_u32_agent(&a.t_acts[static_cast<size_t>(pair) * F + row], word);
@@ -945,7 +960,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
   if (tok < T) {
     if constexpr (UNITS) request_down_rows();
     // the scale of the token's activations, in a vector register: the scalar ones are all taken
-    float act_sc = S::T == 1 ? one_act_scale : s_scale[MF_MAX_TOKENS + tok];
+    float act_sc = s_scale[S::T == 1 ? 0u : tok];
     asm volatile("" : "+v"(act_sc));
     // Gather what other workgroups produced: the routed activations [K*F] and the shared
     // activations (+ gate) [Fs (+4)], 256 words per wave step, two steps in flight.
@@ -1207,6 +1222,7 @@ static FusedGeo fused_geo(const mf_moe_config& c, uint32_t num_cu, uint32_t t, c
   g.n_sl = make_fastdiv(c.d / epl);
   g.rgf = make_fastdiv((c.f + rpw_d - 1) / rpw_d);
   g.K = make_fastdiv(c.top_k);
+  g.x_runs = make_fastdiv(fused_x_runs(c.d / epl));
   g.srg = make_fastdiv((c.shared_f + rpw_sd - 1) / rpw_sd);
   g.c_wgs_div = make_fastdiv(sp.wgs);
   g.rpr = make_fastdiv(sp.units * rpw_f);
@@ -1270,6 +1286,7 @@ bool fused_supported(const mf_moe& h, const mf_moe_layer_weights& w, const void*
                                               c.shared_bits == MF_BITS_2)) ||
                      (c.bits == MF_BITS_TERNARY && (!c.shared_f || c.shared_bits == MF_BITS_4));
   if (!combo || c.d % 8 != 0) return false;
+  if (t * fused_x_runs(c.d / fused_epl(c)) > kFusedWaves * kWave - 2 * MF_MAX_TOKENS) return false;  // (hidden sizes from 260 000 on)
   if (fused_lds_base(c, static_cast<uint32_t>(h.ctx->num_cu), t) > kFusedLdsLimit) return false;
   if (static_cast<uint32_t>(h.ctx->num_cu) < t || !fused_rows_fit(c, static_cast<uint32_t>(h.ctx->num_cu), t, false)) return false;
   const uint32_t offs = w.offsets.gate_w | w.offsets.up_w | w.offsets.down_w;

@@ -34,6 +34,7 @@ _POWERS = [0, 50, -50, 23, -24, 12, 58, -30]
 @pytest.mark.parametrize("bits,d,f,e,k,t,form", [
     (4, 256, 128, 16, 4, 8, "fused"), (4, 2048, 512, 16, 8, 5, "fused"), (4, 704, 448, 12, 4, 1, "fused"), (2, 1024, 320, 16, 6, 8, "fused"),
     (2, 4096, 128, 16, 2, 1, "fused"), (1, 512, 256, 32, 8, 3, "fused"), (2, 128, 64, 16, 3, 7, "fused"), (4, 8192, 128, 4, 2, 8, "fused"),
+    (4, 2816, 128, 8, 2, 3, "fused"), (4, 1600, 128, 8, 2, 4, "fused"),
     (4, 256, 128, 16, 4, 8, "phases"), (2, 640, 320, 16, 3, 8, "phases"), (1, 512, 256, 32, 8, 5, "phases"),
 ])
 def test_decode_layer_of_rows_far_from_one(gpu, oracle, bits, d, f, e, k, t, form):
