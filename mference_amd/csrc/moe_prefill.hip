@@ -5,7 +5,8 @@
 // The matmul keeps the codes EXACT: a lane's packed uint32 is masked into bf16 subnormals (a 4-bit code in bits 4..7 of a
 // 16-bit half is the number q * 2^-129, mf_device.h), which are a matrix-core operand as they stand -- no LDS
 // staging of weights.  x rows are pre-permuted once per call to the same
-// (j, j+4) pairing, times 2^64, and staged through LDS per 64-wide K group.  Per K group the
+// (j, j+4) pairing, times a power of two that the row's largest magnitude decides (2^64 for ordinary rows; what another
+// lacks is made up for in the epilogue), and staged through LDS per 64-wide K group.  Per K group the
 // matrix core yields 2^-65 sum(q * x) (bf16 x bf16 products are exact in
 // fp32), and the group's bf16 scale is applied in fp32: acc += 2^65 s * tmp -- the
 // reference's own factoring s*sum(q*x) + b*sum(x)
