@@ -456,9 +456,10 @@ template <bool SWAPPED> struct QmmCodes<4, SWAPPED> {
     if (SWAPPED) return 16u * row_bytes;
     return tiled ? 1024u : 32u;
   }
-  // the part of the pair whose registers are free once group i of the pair before has been multiplied
-  __device__ __forceinline__ void load(int i, const uint8_t* p, size_t behind) {
-    const uint4 v = *reinterpret_cast<const uint4*>(i ? p + behind : p);
+  // the part of the pair whose registers are free once group i of the pair before has been multiplied (the second part lies
+  // second() behind the first)
+  __device__ __forceinline__ void load(int i, const uint8_t* p) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
     w[4 * i] = v.x; w[4 * i + 1] = v.y; w[4 * i + 2] = v.z; w[4 * i + 3] = v.w;
   }
   __device__ __forceinline__ void settle() {
@@ -479,7 +480,7 @@ template <bool SWAPPED> struct QmmCodes<2, SWAPPED> {  // (SWAPPED = false: only
     return SWAPPED ? (lane & 31u) * row_bytes + lane_group(lane) * 16u : lane * 16u;
   }
   static __device__ __forceinline__ size_t second(size_t, bool) { return 0; }
-  __device__ __forceinline__ void load(int i, const uint8_t* p, size_t) {
+  __device__ __forceinline__ void load(int i, const uint8_t* p) {  // (all of the pair with its second part)
     if (i == 0) return;
     const uint4 v = *reinterpret_cast<const uint4*>(p);
     w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;

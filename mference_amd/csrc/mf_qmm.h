@@ -15,10 +15,10 @@ constexpr uint32_t kQmmWaves = 4;      // waves per workgroup, 32 weight rows ea
 constexpr uint32_t kQmmRows = kQmmWaves * 32;
 
 struct Tile {
-  uint32_t expert, pair_start, count, pad;
+  uint32_t expert, pair_start, count, list_tiles;  // list_tiles: how many the list has
 };
-// What the grouping leaves for the two matmuls of a layer call: runs of at most `tokens` routes of one expert, `slots` entries
-// (a multiple of 8).  list[1] null: both read list[0].
+// What the grouping leaves for the two matmuls of a layer call: runs of at most `tokens` routes of one expert, in expert order, room for
+// `slots` (a multiple of 8).  A list of no tiles has a first record of zeros.  list[1] null: both read list[0].
 struct TileLists {
   Tile* list[2];
   uint32_t slots[2], tokens[2];
@@ -59,7 +59,6 @@ struct QmmArgs {
   int epi;              // 0 swiglu -> bf16 [pair, rows] as matmul_row8 leaves rows, group sums to out_sums; 1 fp32 [token*K+rank, rows]; 2 bf16 [pair, rows];
                         // 3 bf16 [token*K+rank, rows]
   int narrow;           // shared-expert rounding points (dequant_int4.metal:240-245)
-  int tab_aligned;      // scale / bias rows start on 16-byte boundaries (set by the launcher)
   int ternary;          // 2-bit codes {0,1,2} with bias = -scale: b_off / dense[].biases name the SCALE table
   int maple;            // MapleMoE's bf16-stepped activation in the SwiGLU epilogue
   void* out;

@@ -11,8 +11,23 @@
 
 namespace mf {
 
-// x tile ring: 2 stages of 2 K groups
+// LDS of qmm_kernel: x tile ring (2 stages of 2 K groups), the scales and the group sums of a step of 16 groups, 12 bytes a route
+constexpr uint32_t kTabStep = 16;
 __host__ __device__ constexpr uint32_t qmm_x_bytes(uint32_t tile) { return 2 * 2 * tile * 8 * 16; }
+__host__ __device__ constexpr uint32_t qmm_scale_bytes(int nproj) { return nproj * kQmmWaves * kTabStep * 32 * 4; }
+__host__ __device__ constexpr uint32_t qmm_sum_bytes(uint32_t tile) { return 3 * tile * 2 * 16; }
+__host__ __device__ constexpr uint32_t qmm_lds_bytes(uint32_t tile, int nproj) {
+  return qmm_x_bytes(tile) + qmm_scale_bytes(nproj) + qmm_sum_bytes(tile) + tile * 12;
+}
+
+// LDS[lds + 16 * lane ...] = the 16 bytes at p of every lane (lds: a byte address, uniform), without a register in between.  The
+// compiler does not know of the request: wait_loads and a barrier stand in front of the first read.
+__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+}
+// every load of this wave but its newest N has arrived
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
 // waves a SIMD (workgroups a CU) that the kernels' registers are budgeted for
 __host__ __device__ constexpr int qmm_waves(uint32_t tile, int nproj) { return tile == kSmallTile || nproj == 1 ? 3 : 2; }
 
@@ -20,20 +35,41 @@ __device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint3
   if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
 }
 
+// Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of one tile share its x rows, the
+// tiles of one expert share its weights) are laid on ONE XCD so that its L2 serves the re-reads.  Every XCD gets an eighth of the
+// routed part's live items, which are counted here (the first tile's record holds the number of tiles): with whole tiles dealt out
+// by eighths seven XCDs had 66 items for 64 slots and the eighth 48 (2816 x 704, 300 tokens, 85 tiles of 6 items).
+struct QmmPlace {
+  uint32_t xcd, slot, per_xcd;
+};
+constexpr uint32_t kNoWork = 0xFFFFFFFFu;
+__device__ __forceinline__ QmmPlace qmm_place(const uint32_t (&per_xcd)[2], bool& second) {
+  const uint32_t xcd_slot = blockIdx.x >> 3;
+  second = xcd_slot >= per_xcd[0];
+  return {blockIdx.x & 7u, xcd_slot - (second ? per_xcd[0] : 0u), per_xcd[second ? 1 : 0]};
+}
+__device__ __forceinline__ uint32_t qmm_work(const QmmArgs& a, const QmmPlace& at, uint32_t items_per_tile) {
+  if (a.dense_mode) return at.xcd * at.per_xcd + at.slot;
+  const uint32_t live = a.tiles->list_tiles * items_per_tile, per = (live + 7) / 8, work = at.xcd * per + at.slot;
+  return at.slot < per && work < live ? work : kNoWork;
+}
+
 // One workgroup: a tile of TT (64 or 32) routes of one expert x 128 weight rows (4 waves x 32) x
 // NPROJ projections, the whole K.  The matrix core computes the TRANSPOSED
 // product: the A operand is the x tile (tokens are the rows), the B operand is
 // the expanded codes, so a lane ends up holding ONE weight row (its column
 // m = lane % 32) for 16 tokens of each 32-token block, and the per-group scale
-// is one scalar per lane.  Tiles of 64: with two row blocks per wave two waves per SIMD stay
-// resident (the register budget of 256 keeps the matrix-core results in ordinary
-// registers, where the scale multiply reads them directly); with one row block the
-// kernel fits 168 registers and three waves stay resident.  Tiles of 32 fit 168 registers in both forms: the table words
-// are not requested a step ahead, units are kept apart in the loop, and a handful of values waits in scratch memory while a
-// loop runs (none inside it).  What that buys: 2816 x 704, 128 experts, 300 tokens, gate / up 70 -> 66 us and down
-// 70 -> 47 us under the tracer; Qwen shape, 93 tokens, gate / up 38.5 -> 31.7.
-// LDS (dynamic): x tile ring, 2 stages x 2 K groups x [TT / 32 nt][4 s][2 h][32 n] x 16 B,
-// scale tables [NPROJ][4 waves][ng][32 rows] fp32 or bf16, per route: out slot u32, what its results lack, scale of its activations.
+// is one scalar per lane.  Tiles of 64 keep two waves per SIMD (256 registers: the matrix-core results stay in ordinary
+// registers, where the scale multiply reads them directly), three with one row block; tiles of 32 fit 168 registers, three waves.
+// What bounds it: the vector and matrix instructions of the loop, at the clock that power leaves.  So whatever a work item waits
+// for in front of its loop is time the SIMD is not full, and the loop takes everything along: x goes straight to LDS, a pair of
+// groups ahead, and scales, biases and group sums come a step of 16 groups ahead (before, all of them in front of the loop, in
+// sequence for tiles of 32).  Stage stamps of a routed gate / up item, us, before -> now: Qwen shape, 2048 tokens, in front of the
+// loop 6.1 -> 3.5, whole item 33.1 -> 29.8, launch 136 -> 126 under the tracer; two 5120 x 17408 MLPs, 150 rows 303 -> 277; tiles of
+// 32: 2816 x 704, 300 tokens 64 -> 60, large 2-bit layer, 777 tokens 362 -> 345 (there the instructions of the loop are the bound).
+// LDS no longer grows with K, so every contraction keeps its two or three workgroups a CU.
+// LDS (dynamic): x tile ring, 2 stages x 2 K groups x [TT tokens][8 runs, turned] x 16 B; per wave the scales of a step
+// [NPROJ][16][32 rows] fp32; group sums of a step; per route: out slot u32, what its results lack, scale of its activations.
 // One launch can carry two independent problems of the same instantiation (the routed experts
 // and the shared expert of the same phase): the second problem's work items follow the first's
 // on every XCD, so they fill the slots the first problem's last round leaves empty instead of
@@ -45,15 +81,16 @@ struct QmmLaunch {
 
 // NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
 // of groups and rows.
-template <int TT, int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
-__device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_t* smem) {
+template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED>
+__device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place, uint8_t* smem) {
   constexpr int NT = TT / 32;             // token blocks of a tile
   constexpr uint32_t kXGroup = TT * 8;    // 16-byte pieces of one K group of the x tile
   constexpr uint32_t kGB = QmmCodes<BITS>::kGroupBytes;  // bytes of one K group of one weight row
-  const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t m = lane & 31, h = lane >> 5;
   const uint32_t wave_rows = a.pair_rows ? 32u * NPROJ : 32u;  // weight rows of one wave
   const uint32_t n_slices = NG8 ? a.rows / (kQmmWaves * wave_rows) : (a.rows + kQmmWaves * wave_rows - 1) / (kQmmWaves * wave_rows);
+  const uint32_t work = qmm_work(a, place, n_slices);
   uint32_t tile_id = work / n_slices, slice = work % n_slices, win = 0;
   if (a.dense_mode) {
     if (work >= a.dense_items) return;
@@ -80,25 +117,23 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
     pair_start = tile_id * TT;
     count = min(static_cast<uint32_t>(TT), a.dense_rows - pair_start);
   } else {
+    if (work == kNoWork) return;
     // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
     // fetched in a second round trip)
     const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
-    const Tile t{tv.x, tv.y, tv.z, tv.w};
-    if (t.count == 0) return;
-    expert = t.expert;
-    pair_start = t.pair_start;
-    count = t.count;
+    count = __builtin_amdgcn_readfirstlane(tv.z);
+    expert = __builtin_amdgcn_readfirstlane(tv.x);
+    pair_start = __builtin_amdgcn_readfirstlane(tv.y);
   }
 
   uint4* s_x = reinterpret_cast<uint4*>(smem);                      // 2 stages x 2 groups x kXGroup uint4
-  // The scale of every (row, group): fp32, or (TAB16, long contractions) a bf16 number -- a power of two times a bf16
-  // scale is one, so the upper half of the fp32 product is all of it.  That is half the LDS,
-  // which lets two workgroups share a CU up to 112 K groups (K = 7168), for one more instruction per read.
-  using tab_t = std::conditional_t<TAB16, uint16_t, float>;
-  tab_t* s_scale = reinterpret_cast<tab_t*>(smem + qmm_x_bytes(TT));  // [NPROJ][4][ng][32]
-  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT) + ((NPROJ * kQmmWaves * ng * 32 * sizeof(tab_t) + 15) & ~15u));
+  float* s_scale = reinterpret_cast<float*>(smem + qmm_x_bytes(TT)) + wv * (NPROJ * kTabStep * 32);  // this wave's [NPROJ][16 groups][32 rows]
+  uint4* s_sum = reinterpret_cast<uint4*>(smem + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ));  // [NT][3 parts][64 lanes]
+  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ) + qmm_sum_bytes(TT));
   float* s_rel = reinterpret_cast<float*>(s_slot + TT);  // [TT]
   float* s_act = s_rel + TT;                              // [TT]
+  const uint32_t lds_x = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) uint8_t*)smem));
+  const uint32_t lds_sum = lds_x + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ);
 
   // weight pointers of this workgroup's projections
   const uint8_t* Wp[NPROJ];
@@ -128,122 +163,109 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 
   // ---- everything the tile needs that depends only on the tile: issued back to back.
   // Routes past `count` read the tile's last route instead (finite data, results discarded).
-  // staging: a thread takes two runs of 8 K values of one token in every group, or one of a tile of at most 32 routes
-  const bool few = NT == 1 || (NPROJ == 2 && count <= 32);
-  const uint32_t st_i = few ? threadIdx.x >> 3 : threadIdx.x >> 2;
-  const uint32_t st_c0 = few ? threadIdx.x & 7 : (threadIdx.x & 3) * 2, st_c1 = few ? st_c0 : st_c0 + 1;
-  const uint32_t st_pair = pair_start + min(st_i, count - 1);
-  uint32_t st_row = st_pair, xrow[NT];
+  // x is requested straight into LDS, 8 tokens x 8 runs of 8 values an instruction: lane l brings a run of token l / 8 of the eight
+  const uint32_t st_n = 8 * wv + (lane >> 3);  // (and, of a tile of 64, token st_n + 32)
+  uint32_t xrow[NT], st_row[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) xrow[nt] = pair_start + min(32 * nt + m, count - 1);
+  for (int nt = 0; nt < NT; ++nt) {
+    xrow[nt] = pair_start + min(32 * nt + m, count - 1);
+    st_row[nt] = pair_start + min(32 * nt + st_n, count - 1);
+  }
   uint32_t slot = pair_start + min(threadIdx.x & 63u, count - 1);
   // the routes' records are requested here and looked at behind the code loads below, which do not depend on
   // them: the first codes are then on their way one memory round trip earlier
   mf_pair pr{};
-  uint32_t tok_st = 0, tok[NT] = {};
+  uint32_t tok_st[NT] = {}, tok[NT] = {};
   if (!a.dense_mode) {
     pr = a.sorted[slot];
     if (a.gather) {
-      tok_st = a.sorted[st_pair].token;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) tok[nt] = a.sorted[xrow[nt]].token;
+      for (int nt = 0; nt < NT; ++nt) {
+        tok_st[nt] = a.sorted[st_row[nt]].token;
+        tok[nt] = a.sorted[xrow[nt]].token;
+      }
     }
   }
-  const uint8_t* wrow[NPROJ];
+  // (addresses of codes and tables: a uniform base, which the scalar unit moves along, and the lane's 32-bit offset)
+  const uint8_t* wbase[NPROJ];
   using Codes = QmmCodes<BITS, SWAPPED>;
   const uint32_t gstride = a.tiled ? 32u * kGB : kGB;  // bytes from a group's codes to the next group's
-  const size_t second = Codes::second(row_bytes, a.tiled);
+  const uint32_t second = static_cast<uint32_t>(Codes::second(row_bytes, a.tiled));
+  const uint32_t lane_off = static_cast<uint32_t>(Codes::lane_offset(lane, row_bytes, a.tiled));
   const uint32_t last_pair = (ng - 1) & ~1u;
   // (the last pair of an odd number of groups is half a pair: the lanes that would ask for its second group ask for the first)
-  const uint32_t odd_back = !NG8 && (ng & 1u) ? Codes::lane_group(lane) * gstride : 0u;
-  auto pair_at = [&](uint32_t g) -> size_t {  // g: the pair's first group; past the end: the last pair again
+  const uint32_t last_off = lane_off - (!NG8 && (ng & 1u) ? Codes::lane_group(lane) * gstride : 0u);
+  // part i of the pair of groups from g on; past the end: the last pair again
+  auto codes_at = [&](int p, uint32_t g, int i) __attribute__((always_inline)) {
     const uint32_t gc = min(g, last_pair);
-    return static_cast<size_t>(gc) * gstride - (!NG8 && gc == last_pair ? odd_back : 0u);
+    return wbase[p] + (gc * gstride + (i ? second : 0u)) + (!NG8 && gc == last_pair ? last_off : lane_off);
   };
-  Codes cur[NPROJ][2];
+  // pairs of groups in flight: one for 4-bit codes on tiles of 32, whose registers do not hold a second (with it, 31 values went
+  // through scratch memory: 2816 x 704, 300 tokens, gate / up 60 -> 100 us; 93 tokens of the Qwen shape 31 -> 37)
+  constexpr int kRing = NT == 1 && BITS == 4 ? 1 : 2;
+  Codes cur[NPROJ][kRing];
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p) {
-    wrow[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride +
-              Codes::lane_offset(lane, row_bytes, a.tiled);
+    wbase[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride;
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < kRing; ++u)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow[p] + pair_at(2 * u), second);
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, codes_at(p, 2 * u, i));
   }
-  __builtin_amdgcn_sched_barrier(0);  // (keeps the look at the routes behind the code loads)
+  // Scale (what = 0) or bias words (1) of the lane's row of projection p in a step of 16 K groups: groups g0 + 8h .. + 7
+  auto tab_fetch = [&](int what, int p, uint32_t g0) __attribute__((always_inline)) -> uint4 {
+    const uint16_t* table = (what ? Bp[p] : Sp[p]) + static_cast<size_t>(row_base[p]) * ng_ld + g_off;
+    const uint32_t gl = g0 + 8 * h;
+    const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
+    // (whole 16-byte loads at any group and alignment; in the last step they end at the row's end and are moved down)
+    const uint32_t gb = NG8 ? gc : min(gc, ng - 8);
+    const uint4 v = load_16_bytes(table + (m * ng_ld + gb));
+    return !NG8 && g0 + kTabStep > ng ? drop_bf16(v, gc - gb) : v;
+  };
+  uint4 tab[2][NPROJ];  // of the next step
+#pragma unroll
+  for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+    for (int what = 0; what < 2; ++what)
+      tab[what][p] = NG8 || ng >= 8 ? tab_fetch(what, p, 0)
+                                    : load_bf16x8_guarded((what ? Bp[p] : Sp[p]) + static_cast<size_t>(row_base[p] + m) * ng_ld + g_off, h ? 0u : ng);
+  __builtin_amdgcn_sched_barrier(0);  // (keeps the look at the routes behind the loads that do not depend on them)
   if (!a.dense_mode) {
     if (a.gather) {
-      st_row = tok_st;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) xrow[nt] = tok[nt];
+      for (int nt = 0; nt < NT; ++nt) {
+        st_row[nt] = tok_st[nt];
+        xrow[nt] = tok[nt];
+      }
     }
     if (a.epi == 1 || a.epi == 3) slot = pr.token * a.top_k + pr.rank;
   }
   const float row_max = a.row_max[a.dense_mode ? pair_start + min(threadIdx.x & 63u, count - 1) : pr.token];
-  // x rows of groups 0..2 and, for the bias terms, the group sums of the lane's two routes
-  const uint16_t* st_src = a.x + static_cast<size_t>(st_row) * a.x_stride + static_cast<size_t>(g_off) * kGroup + st_c0 * 8;
-  const uint32_t st_2nd = (st_c1 - st_c0) * 8;
-  // K groups travel in pairs; a contraction of an odd number of groups ends in half a pair (its other half is read
-  // from the last group again and not multiplied)
-  // (arrays of a native vector type: arrays of the uint4 struct were kept in scratch memory)
-  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-  u32x4_t xs[2][2];  // the pair after the one in LDS, on its way there
-  u32x4_t x0[2][2];
+  // The place in the 128 bytes of a token's group where run c lies: c ^ (token / 2 % 8), so that the 16 lanes that read one run of
+  // as many tokens together meet all the banks.
+  const uint8_t* x_src[NT];
 #pragma unroll
-  for (int gi = 0; gi < 2; ++gi) {
-    const uint32_t ga = NG8 ? gi : min(static_cast<uint32_t>(gi), ng - 1), gb = NG8 ? 2u + gi : min(2u + gi, ng - 1);
-    x0[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup);
-    if (NT > 1) x0[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + ga * kGroup + st_2nd);
-    xs[gi][0] = xs[gi][1] = u32x4_t{0, 0, 0, 0};
-    if (NG8 || ng > 2) {
-      xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup);
-      if (NT > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gb * kGroup + st_2nd);
-    }
-  }
-  // Scale and bias words of the lane's row and the group sums of its two routes, 8 K groups at a time
-  // (groups gl = g0 + 8h .. gl + 7 for g0 = 0, 16, ...); the loads of the first step leave now, with the
-  // codes and the x rows, the loads of every later step one step ahead of their use.
-  auto sums_fetch = [&](int nt, uint32_t gc, uint4 (&sum)[3]) {
-    const uint16_t* sp = a.sumx + xrow[nt] * group_sum_words(ng_ld) + (g_off + gc) / 8 * 24;
+  for (int nt = 0; nt < NT; ++nt)
+    x_src[nt] = reinterpret_cast<const uint8_t*>(a.x + static_cast<size_t>(st_row[nt]) * a.x_stride + static_cast<size_t>(g_off) * kGroup) +
+                ((lane & 7u) ^ ((st_n >> 1) & 7u)) * 16u;
+  // K groups g and g + 1 of the tile's first `blocks` blocks of 32 tokens into a stage of the ring (an odd number of groups: the
+  // last pair's second group is the last one again, and not multiplied)
+  auto x_request = [&](uint32_t g, uint32_t stage, int blocks) __attribute__((always_inline)) {
 #pragma unroll
-    for (int part = 0; part < 3; ++part) sum[part] = *reinterpret_cast<const uint4*>(sp + 8 * part);
+    for (int gi = 0; gi < 2; ++gi)
+#pragma unroll
+      for (int nt = 0; nt < blocks; ++nt)
+        load_to_lds(x_src[nt] + (NG8 ? g + gi : min(g + gi, ng - 1)) * 128u,
+                    lds_x + ((stage * 2 + gi) * TT + nt * 32 + wv * 8) * 128);
   };
-  struct TabStep {
-    uint4 S[NPROJ], B[NPROJ];
-    uint4 sum[3];  // of the first token block (the second block's are requested at the top of their step: registers)
-  };
-  auto tab_fetch = [&](uint32_t g0) {
-    TabStep t;
-    const uint32_t gl = g0 + 8 * h;
-    const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
-    sums_fetch(0, gc, t.sum);
-    if (!NG8 && ng >= 8) {  // whole 16-byte loads at any group; in the last step they end at the row's end and are moved down
-      const uint32_t gb = min(gc, ng - 8), sh = gc - gb;
-      const bool last = g0 + 16 > ng;  // (uniform)
+  // the group sums of a step, for the bias terms: three bf16 parts of 8 groups by half, token by lane
+  auto sums_request = [&](uint32_t g0, int blocks) __attribute__((always_inline)) {
+    const uint32_t gl = g0 + 8 * h, gc = gl < ng ? gl : 0;
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gb;
-        t.B[p] = load_16_bytes(Bp[p] + at);
-        t.S[p] = load_16_bytes(Sp[p] + at);
-        if (last) {
-          t.B[p] = drop_bf16(t.B[p], sh);
-          t.S[p] = drop_bf16(t.S[p], sh);
-        }
-      }
-      return t;
-    }
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p) {
-      const size_t at = static_cast<size_t>(row_base[p] + m) * ng_ld + g_off + gc;
-      t.B[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Bp[p] + at) : load_x8<false>(Bp[p] + at))
-                   : load_bf16x8_guarded(Bp[p] + at, ng - gc);
-      t.S[p] = NG8 ? (a.tab_aligned ? load_x8<true>(Sp[p] + at) : load_x8<false>(Sp[p] + at))
-                   : load_bf16x8_guarded(Sp[p] + at, ng - gc);
-    }
-    return t;
+    for (int i = 0; i < 3 * blocks; ++i)
+      if (wv == i % kQmmWaves)
+        load_to_lds(a.sumx + xrow[i / 3] * group_sum_words(ng_ld) + (g_off + gc) / 8 * 24 + 8 * (i % 3), lds_sum + i * 1024);
   };
-  TabStep tab_cur;
-  if constexpr (NT > 1) tab_cur = tab_fetch(0);
   qmm_trace(a, work, 1);
 
   if (threadIdx.x < TT) s_slot[threadIdx.x] = threadIdx.x < count ? slot : 0xFFFFFFFFu;
@@ -256,144 +278,117 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[p][nt][r] = 0.0f;
 
-  // ---- per step: the scales of the wave's rows, times the powers of two that codes and rows carry, into the
-  // [g][row] table, and the bias term: acc[token, row] += sumx[token, g] * B[row, g].
   // A tile of at most 32 routes fills only the first token block: the second block's matrix
   // instructions and scale multiplies are left out (NTA = 1); its accumulators stay zero and its
   // output slots are empty.  Of a tile of at most 8 routes (most tiles of a short prompt) a lane's first four results are all
   // there is: only those are scaled (RES), 4 of 16 multiply-adds per group and row block.
   auto tile_body = [&](auto nta_c, auto res_c) {
   constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
-  for (uint32_t g0 = 0; g0 < ng; g0 += 16) {
-    TabStep t;
-    if constexpr (NT > 1) {
-      t = tab_cur;
-      tab_cur = tab_fetch(g0 + 16 < ng ? g0 + 16 : g0);  // past the end: the same step again, unused
-    } else {
-      t = tab_fetch(g0);  // (three waves a SIMD hide its round trip, and their registers do not hold a second step)
-    }
-    const uint32_t gl = g0 + 8 * h;
-    const bool have = gl < ng;
-    uint4 sum[NTA][3];
-#pragma unroll
-    for (int part = 0; part < 3; ++part) sum[0][part] = t.sum[part];
-    if constexpr (NTA > 1) sums_fetch(1, have ? gl : 0, sum[1]);
-    uint4 ab[NPROJ];
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p) {
-      tab_t* tab = s_scale + (p * kQmmWaves + wv) * ng * 32;
-      auto entry = [](float v) -> tab_t {
-        if constexpr (TAB16) return static_cast<uint16_t>(__float_as_uint(v) >> 16);
-        else return v;
-      };
-      const uint32_t pr[4] = {t.S[p].x, t.S[p].y, t.S[p].z, t.S[p].w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (have && (NG8 || gl + 2 * i < ng)) tab[(gl + 2 * i) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_lo(pr[i]));
-        if (have && (NG8 || gl + 2 * i + 1 < ng)) tab[(gl + 2 * i + 1) * 32 + m] = entry(QmmCodes<BITS>::kScaleMul * bf16_hi(pr[i]));
-      }
-      // ternary rows store no biases: the bias is -scale (the table pointer is the scale table then)
-      ab[p] = a.ternary ? make_uint4(t.B[p].x ^ 0x80008000u, t.B[p].y ^ 0x80008000u, t.B[p].z ^ 0x80008000u,
-                                     t.B[p].w ^ 0x80008000u)
-                        : t.B[p];
-      if (!have) ab[p] = make_uint4(0, 0, 0, 0);
-    }
-#pragma unroll
-    for (int nt = 0; nt < NTA; ++nt) {
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-#pragma unroll
-        for (int part = 0; part < 3; ++part) acc[p][nt] = mfma_bf16(sum[nt][part], ab[p], acc[p][nt]);
-      }
-    }
-  }
-  qmm_trace(a, work, 2);
-  if (threadIdx.x < TT) {  // (here, where the loads behind this one have been waited for)
+  sums_request(0, NTA);
+  x_request(0, 0, NTA);
+  if (threadIdx.x < TT) {
     s_rel[threadIdx.x] = rel_of_scale(a.act_rows ? act_scale(row_max) : row_scale(row_max));
     s_act[threadIdx.x] = act_scale(row_max);
   }
-
-  // run c = 2q (+1): K 8c..8c+7 -> slot (h = c / 4, s = c % 4)
-  const uint32_t st_nt = st_i >> 5, st_n = st_i & 31, c0 = st_c0, c1 = st_c1;
-  // inside a 32-token block the column is rotated by 2 * (s + 4h): the 16 lanes that store together -- four runs
-  // of four tokens, or eight of two -- hit sixteen different bank groups
-  const uint32_t st_slot0 = ((st_nt * 4 + (c0 & 3)) * 2 + (c0 >> 2)) * 32 + ((st_n + 2 * c0) & 31);
-  const uint32_t st_slot1 = ((st_nt * 4 + (c1 & 3)) * 2 + (c1 >> 2)) * 32 + ((st_n + 2 * c1) & 31);
   uint32_t rd_col[4];
 #pragma unroll
-  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = (m + 2 * sidx + 8 * h) & 31;
+  for (int sidx = 0; sidx < 4; ++sidx) rd_col[sidx] = m * 8 + ((4 * h + sidx) ^ ((m >> 1) & 7u));
+  // Per step of 16 groups: the scales of the wave's rows, times the powers of two that codes and rows carry, into the
+  // [g][row] table, and the bias term: acc[token, row] += sumx[token, g] * B[row, g].
+  auto tab_step = [&](uint32_t g0) __attribute__((always_inline)) {
+    const bool have = g0 + 8 * h < ng;
+    uint4 ab[NPROJ];
 #pragma unroll
-  for (int gi = 0; gi < 2; ++gi) {
-    *reinterpret_cast<u32x4_t*>(s_x + gi * kXGroup + st_slot0) = x0[gi][0];
-    if (NTA > 1) *reinterpret_cast<u32x4_t*>(s_x + gi * kXGroup + st_slot1) = x0[gi][1];
-  }
+    for (int p = 0; p < NPROJ; ++p) {
+      const uint4 S = tab[0][p], B = tab[1][p];
+      float* to = s_scale + p * (kTabStep * 32) + 8 * h * 32 + m;
+      const uint32_t w[4] = {S.x, S.y, S.z, S.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        to[2 * i * 32] = QmmCodes<BITS>::kScaleMul * bf16_lo(w[i]);
+        to[(2 * i + 1) * 32] = QmmCodes<BITS>::kScaleMul * bf16_hi(w[i]);
+      }
+      // ternary rows store no biases: the bias is -scale (the table pointer is the scale table then)
+      ab[p] = a.ternary ? make_uint4(B.x ^ 0x80008000u, B.y ^ 0x80008000u, B.z ^ 0x80008000u, B.w ^ 0x80008000u) : B;
+      if (!have) ab[p] = make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int nt = 0; nt < NTA; ++nt)
+#pragma unroll
+      for (int part = 0; part < 3; ++part) {
+        const uint4 sum = s_sum[(nt * 3 + part) * 64 + lane];
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) acc[p][nt] = mfma_bf16(sum, ab[p], acc[p][nt]);
+      }
+  };
+  wait_loads<0>();
+  qmm_trace(a, work, 2);
 
-  // Weight codes run four K groups ahead in a ring of registers (the expert's bytes come
-  // from HBM); x rows come from L2 in pairs of groups, one pair in registers behind
-  // the pair in the LDS stage that is not being read.
-
+  // Weight codes run up to four K groups ahead in a ring of registers (the expert's bytes come from HBM); x rows come from L2 a pair
+  // of groups ahead, into the stage that is not being read.  kCodeLoads: what a wave requests behind a pair's x until that pair's turn.
+  constexpr int kCodeLoads = NPROJ * (BITS == 4 ? 2 : 1);
   Codes now[NPROJ];
   for (uint32_t g0 = 0; g0 < ng; g0 += 4) {
 #pragma unroll
     for (int uu = 0; uu < 2; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
       const uint32_t gu = g0 + 2 * uu;
       if (!NG8 && gu >= ng) break;
-      __syncthreads();  // stage uu is complete, stage uu ^ 1 is no longer read
-      // ---- the next pair into the other stage, fetch the pair after it into the freed registers.
-      // With whole steps of 8 groups the body has no branch (past the end the last pair is fetched
-      // again and the write goes to the stage nobody reads any more): every pass issues the same
-      // loads in the same order, so a wait for the codes of this pass never covers the x rows
-      // requested a moment before it.
-      if (NG8 || gu + 2 < ng) {
-        uint4* wbuf = s_x + (uu ^ 1) * 2 * kXGroup;
+      wait_loads<kCodeLoads>();  // this wave's part of stage uu is there
+      __syncthreads();           // stage uu is complete, stage uu ^ 1 is no longer read
+      // The pair's codes are taken up in front of the request for x: the compiler counts the loads it knows, so behind
+      // that request its wait for them would be one for x, too.
 #pragma unroll
-        for (int gi = 0; gi < 2; ++gi) {
-          *reinterpret_cast<u32x4_t*>(wbuf + gi * kXGroup + st_slot0) = xs[gi][0];
-          if (NTA > 1) *reinterpret_cast<u32x4_t*>(wbuf + gi * kXGroup + st_slot1) = xs[gi][1];
-        }
-        if (NG8 || gu + 4 < ng) {
-          const uint32_t gx = NG8 ? min(gu + 4, ng - 2) : gu + 4;
+      for (int p = 0; p < NPROJ; ++p) {
+        if constexpr (BITS == 2) now[p] = cur[p][uu % kRing];  // (all four registers of the pair are one load, which leaves below)
+        Codes& codes = BITS == 2 ? now[p] : cur[p][uu % kRing];
+        codes.settle();
 #pragma unroll
-          for (int gi = 0; gi < 2; ++gi) {
-            const uint32_t gy = NG8 ? gx + gi : min(gx + gi, ng - 1);
-            xs[gi][0] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup);
-            if (NTA > 1) xs[gi][1] = *reinterpret_cast<const u32x4_t*>(st_src + gy * kGroup + st_2nd);
-          }
-        }
+        for (auto& w : codes.w) asm volatile("" : "+v"(w));
+      }
+      if (gu + 2 < ng) x_request(gu + 2, uu ^ 1, NTA);
+      if constexpr (BITS == 2) {
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p) cur[p][uu % kRing].load(1, codes_at(p, gu + 2 * kRing, 1));
+      }
+      // tables: a step's sums are requested when everybody has read the step's before, its scales and biases a pair ahead
+      if (uu == 0 && g0 % kTabStep == 0) tab_step(g0);
+      if (uu == 1 && g0 % kTabStep == 0 && g0 + kTabStep < ng) sums_request(g0 + kTabStep, NTA);
+      if (uu == 1 && g0 % kTabStep == kTabStep - 4 && g0 + 4 < ng) {
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+          for (int what = 0; what < 2; ++what) tab[what][p] = tab_fetch(what, p, g0 + 4);
       }
 #pragma unroll
       for (int gi = 0; gi < 2; ++gi) {
         const uint32_t g = gu + gi;
-        if (!NG8 && g >= ng) break;  // the half pair at the end of an odd number of groups
+        if (!NG8 && g >= ng) {  // the half pair at the end of an odd number of groups; its loads leave on either way, which keeps the compiler's count of them
+          if constexpr (BITS != 2) {
+#pragma unroll
+            for (int p = 0; p < NPROJ; ++p) cur[p][uu % kRing].load(gi, codes_at(p, gu + 2 * kRing, gi));
+          }
+          break;
+        }
         // ---- matrix core: tmp[token, row] = sum over the group of x * q, times the powers of two kScaleMul takes back
         const uint4* buf = s_x + (2 * uu + gi) * kXGroup;
         uint4 bx[2][4];
 #pragma unroll
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
-          for (int s = 0; s < 4; ++s) bx[nt][s] = buf[((nt * 4 + s) * 2 + h) * 32 + rd_col[s]];
+          for (int s = 0; s < 4; ++s) bx[nt][s] = buf[nt * 256 + rd_col[s]];
 #pragma unroll
         for (int p = 0; p < NPROJ; ++p) {
-          float sc;
-          if constexpr (TAB16) sc = bf16_to_f(s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m]);
-          else sc = s_scale[((p * kQmmWaves + wv) * ng + g) * 32 + m];
+          const float sc = s_scale[(p * kTabStep + g % kTabStep) * 32 + m];
           f32x16_t tmp[2];
 #pragma unroll
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) tmp[nt][r] = 0.0f;
-          if (gi == 0) {
-            if constexpr (BITS == 2) {  // (all four registers of the pair are one load: it leaves at once, from a copy)
-              now[p] = cur[p][uu];
-              cur[p][uu].load(1, wrow[p] + pair_at(gu + 4), second);
-              now[p].settle();
-            } else cur[p][uu].settle();
-          }
           if constexpr (BITS == 2) group_products<BITS, NTA>(now[p], gi, bx, tmp, [](int) {});
-          else group_products<BITS, NTA>(cur[p][uu], gi, bx, tmp, [](int) {});
+          else group_products<BITS, NTA>(cur[p][uu % kRing], gi, bx, tmp, [](int) {});
           // the registers that held this group's codes take their part of the pair two ahead
           // (past the end the last pair is read again: no branch inside the unrolled body)
-          if constexpr (BITS != 2) cur[p][uu].load(gi, wrow[p] + pair_at(gu + 4), second);
+          if constexpr (BITS != 2) cur[p][uu % kRing].load(gi, codes_at(p, gu + 2 * kRing, gi));
 #pragma unroll
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -401,6 +396,11 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
           if constexpr (NT == 1) __builtin_amdgcn_sched_barrier(0);  // one unit at a time: the registers of three waves
         }
       }
+      // (the sums are wanted here: without this a pair's products are kept beyond the branches behind it)
+#pragma unroll
+      for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+        for (int nt = 0; nt < NTA; ++nt) asm volatile("" : "+v"(acc[p][nt]));
     }
   }
   // (results that do not exist: not kept through the loop)
@@ -562,40 +562,30 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, uint32_t work, uint8_
   qmm_trace(a, work, 4);
 }
 
-// Workgroups go to the 8 XCDs round-robin by blockIdx; consecutive work items (the row slices of
-// one tile share its x rows, the tiles of one expert share its weights) are laid on ONE XCD so
-// that its L2 serves the re-reads.  The tile list is laid out by group_scan_kernel so that every
-// eighth of it holds an eighth of the live tiles.
-__device__ __forceinline__ uint32_t qmm_work(const uint32_t (&per_xcd)[2], bool& second) {
-  const uint32_t xcd_slot = blockIdx.x >> 3;
-  second = xcd_slot >= per_xcd[0];
-  return (blockIdx.x & 7u) * per_xcd[second ? 1 : 0] + (xcd_slot - (second ? per_xcd[0] : 0u));
-}
-
 // (Both parts of a launch read their codes in the form SWAPPED names; without it 2-bit codes have to be tiled.  The dense
 // problem beside 2-bit experts is 4-bit and goes through qmm_mixed_kernel: the launchers refuse a 2-bit one beside a tiled pool.)
-template <int TT, int BITS, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
+template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
 void qmm_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmPlace at = qmm_place(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  qmm_item<TT, BITS, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
+  qmm_item<TT, BITS, NPROJ, NG8, SWAPPED>(a, at, smem);
 }
 
 // 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
 // expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
 // tokens: 53 + 33 beside 388 + 207).
-template <int TT, int NPROJ, bool NG8, bool TAB16, bool SWAPPED>
+template <int TT, int NPROJ, bool NG8, bool SWAPPED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
 void qmm_mixed_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmPlace at = qmm_place(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_item<TT, 4, NPROJ, NG8, TAB16, true>(a, work, smem);
-  else qmm_item<TT, 2, NPROJ, NG8, TAB16, SWAPPED>(a, work, smem);
+  if (a.dense_mode) qmm_item<TT, 4, NPROJ, NG8, true>(a, at, smem);
+  else qmm_item<TT, 2, NPROJ, NG8, SWAPPED>(a, at, smem);
 }
 
 // ---- the same product for a short contraction (K <= 512: the down projections) ----
@@ -629,7 +619,7 @@ template <int NG> __device__ __forceinline__ uint4 load_groups_bf16(const uint16
 }
 
 template <int TT, int BITS, int NG, bool SWAPPED>
-__device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, uint32_t n_walk, uint8_t* smem) {
+__device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, const QmmPlace& place, uint32_t n_walk, uint8_t* smem) {
   static_assert(NG == 2 || NG == 4 || NG == 8, "K is 128, 256 or 512");
   constexpr int NT = TT / 32;           // token blocks of a tile
   constexpr uint32_t kXGroup = TT * 8;  // 16-byte pieces of one K group of the x tile
@@ -639,6 +629,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t m = lane & 31, h = lane >> 5;
   const uint32_t items_per_tile = a.rows / (256u * n_walk);
+  const uint32_t work = qmm_work(a, place, items_per_tile);
   uint32_t tile_id = work / items_per_tile, slice0 = (work % items_per_tile) * n_walk;
   if (a.dense_mode) {
     if (work >= a.dense_items) return;
@@ -653,11 +644,9 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
     pair_start = tile_id * TT;
     count = min(static_cast<uint32_t>(TT), a.dense_rows - pair_start);
   } else {
-    // (the whole 16-byte record in one load: read field by field, the count was fetched, tested, and the rest
-    // fetched in a second round trip)
+    if (work == kNoWork) return;
     const uint4 tv = *reinterpret_cast<const uint4*>(a.tiles + tile_id);
     const Tile t{tv.x, tv.y, tv.z, tv.w};
-    if (t.count == 0) return;
     expert = t.expert;
     pair_start = t.pair_start;
     count = t.count;
@@ -692,9 +681,9 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int u = 0; u < kRing; ++u)
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride, second);
+      for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride + (i ? second : 0));
   uint4 nS[2], nB[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -816,7 +805,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
         if (g % 2 == 0) {
           if constexpr (BITS == 2) {
             now[p] = codes;
-            codes.load(1, next_pair, second);
+            codes.load(1, next_pair);
             now[p].settle();
           } else codes.settle();
         }
@@ -827,7 +816,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, uint32_t work, u
           }
         });
         // the registers take the codes kRing pairs on: of this slice, or of the next one
-        if constexpr (BITS != 2) codes.load(g % 2, next_pair, second);
+        if constexpr (BITS != 2) codes.load(g % 2, next_pair + (g % 2 ? second : 0));
 #pragma unroll
         for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
@@ -911,10 +900,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(T
 void qmm_kres_kernel(const KresLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second);
+  const QmmPlace at = qmm_place(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
   const uint32_t walk = launch.slices[second ? 1 : 0];
-  qmm_kres_item<TT, BITS, NG, SWAPPED>(a, work, walk, smem);
+  qmm_kres_item<TT, BITS, NG, SWAPPED>(a, at, walk, smem);
 }
 
 template <int TT, int NG, bool SWAPPED>  // as qmm_mixed_kernel
@@ -922,23 +911,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(T
 void qmm_kres_mixed_kernel(const KresLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
-  const uint32_t work = qmm_work(launch.per_xcd, second), walk = launch.slices[second ? 1 : 0];
+  const QmmPlace at = qmm_place(launch.per_xcd, second);
+  const uint32_t walk = launch.slices[second ? 1 : 0];
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_kres_item<TT, 4, NG, true>(a, work, walk, smem);
-  else qmm_kres_item<TT, 2, NG, SWAPPED>(a, work, walk, smem);
+  if (a.dense_mode) qmm_kres_item<TT, 4, NG, true>(a, at, walk, smem);
+  else qmm_kres_item<TT, 2, NG, SWAPPED>(a, at, walk, smem);
 }
 
 // ------------------------------------------------------------------ launches
-
-inline size_t qmm_lds_bytes(uint32_t tile, uint32_t kdim, int nproj, bool tab16) {
-  const uint32_t ng = kdim / kGroup;
-  return qmm_x_bytes(tile) + ((static_cast<size_t>(nproj) * kQmmWaves * ng * 32 * (tab16 ? 2 : 4) + 15) & ~static_cast<size_t>(15)) +
-         tile * 12;
-}
-// the scale tables as bf16 where fp32 tables would leave a CU (160 KB of LDS) room for one workgroup only
-inline bool qmm_tab16(uint32_t tile, uint32_t kdim, int nproj) {
-  return static_cast<size_t>(qmm_waves(tile, nproj)) * qmm_lds_bytes(tile, kdim, nproj, false) > kMaxLds;
-}
 
 // Work items of a dense problem that one XCD gets: an eighth, but at least 4 while there are any -- a handful
 // of items (the shared expert beside the routed experts of a short batch) runs faster on few XCDs, whose L2
@@ -1006,8 +986,7 @@ hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj
   QmmLaunch launch{};
   const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
   if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
-  size_t lds = 0;
-  bool ng8 = true, tab16 = false;
+  bool ng8 = true;
   for (int part = 0; part < (b ? 2 : 1); ++part) {
     QmmArgs& q = launch.part[part];
     q = part ? *b : a;
@@ -1021,15 +1000,9 @@ hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj
     } else {
       launch.per_xcd[part] = slots / 8 * n_slices;
     }
-    q.tab_aligned = q.dense_mode
-        ? aligned16(q.dense[0].scales) && aligned16(q.dense[0].biases) && aligned16(q.dense[1].scales) &&
-              aligned16(q.dense[1].biases)
-        : aligned16(q.expert_base) && q.expert_stride % 16 == 0 &&
-              (q.s_off[0] | q.b_off[0] | q.s_off[1] | q.b_off[1]) % 16 == 0;
-    tab16 = tab16 || qmm_tab16(TT, q.kdim, nproj);  // with windows: kdim is the longest window
     ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0 && q.rows % slice_rows == 0;
   }
-  for (int part = 0; part < (b ? 2 : 1); ++part) lds = std::max(lds, qmm_lds_bytes(TT, launch.part[part].kdim, nproj, tab16));
+  const size_t lds = qmm_lds_bytes(TT, nproj);
   const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
   if (grid.x == 0) return hipSuccess;
 #define MF_QMM_L(...)                                                                                  \
@@ -1038,22 +1011,17 @@ hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj
     if (e != hipSuccess) return e;                                                                     \
     __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
   } while (0)
-#define MF_QMM(P, G, T)                                                                                \
+#define MF_QMM(P, G)                                                                                   \
   do {                                                                                                 \
-    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<TT, P, G, T, false>);                       \
-    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<TT, P, G, T, true>);                            \
-    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<TT, 4, P, G, T, false>);                              \
-    else if (bits == 4) MF_QMM_L(qmm_kernel<TT, 4, P, G, T, true>);                                        \
-    else if (tiled) MF_QMM_L(qmm_kernel<TT, 2, P, G, T, false>);                                           \
-    else MF_QMM_L(qmm_kernel<TT, 2, P, G, T, true>);                                                       \
+    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<TT, P, G, false>);                          \
+    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<TT, P, G, true>);                               \
+    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<TT, 4, P, G, false>);                                 \
+    else if (bits == 4) MF_QMM_L(qmm_kernel<TT, 4, P, G, true>);                                           \
+    else if (tiled) MF_QMM_L(qmm_kernel<TT, 2, P, G, false>);                                              \
+    else MF_QMM_L(qmm_kernel<TT, 2, P, G, true>);                                                          \
   } while (0)
-#define MF_QMM_G(P, G)                                         \
-  do {                                                         \
-    if (tab16) MF_QMM(P, G, true); else MF_QMM(P, G, false);   \
-  } while (0)
-  if (nproj == 2) { if (ng8) MF_QMM_G(2, true); else MF_QMM_G(2, false); }
-  else { if (ng8) MF_QMM_G(1, true); else MF_QMM_G(1, false); }
-#undef MF_QMM_G
+  if (nproj == 2) { if (ng8) MF_QMM(2, true); else MF_QMM(2, false); }
+  else { if (ng8) MF_QMM(1, true); else MF_QMM(1, false); }
 #undef MF_QMM
 #undef MF_QMM_L
   return hipGetLastError();

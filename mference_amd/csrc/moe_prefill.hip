@@ -460,15 +460,6 @@ __device__ __forceinline__ void group_layout(uint32_t c, uint32_t E, uint32_t* _
     s_total[0] = run_t[0];
     s_total[1] = run_t[1];
   }
-  // A list has `slots` entries (a multiple of 8).  The matmul sends the workgroups of
-  // slot range k * slots/8 .. to XCD k, so every eighth of the list gets an eighth of the
-  // live tiles, in expert order; the rest of each eighth stays empty (count 0).
-  if (publish) {
-#pragma unroll
-    for (int l = 0; l < 2; ++l)
-      if (tiles.list[l])
-        for (uint32_t i = e; i < tiles.slots[l]; i += blockDim.x) tiles.list[l][i] = Tile{0, 0, 0, 0};
-  }
   __syncthreads();
   if (publish && e < E) {
     const uint32_t start = run_c - c;
@@ -477,11 +468,10 @@ __device__ __forceinline__ void group_layout(uint32_t c, uint32_t E, uint32_t* _
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
       if (!tiles.list[l]) continue;
-      const uint32_t per_live = (s_total[l] + 7) / 8, per_slot = tiles.slots[l] / 8, tokens = tiles.tokens[l];
-      for (uint32_t j = 0; j < mine[l]; ++j) {
-        const uint32_t id = run_t[l] - mine[l] + j;
-        tiles.list[l][(id / per_live) * per_slot + id % per_live] = Tile{e, start + j * tokens, min(tokens, c - j * tokens), 0};
-      }
+      const uint32_t tokens = tiles.tokens[l], first = run_t[l] - mine[l], total = s_total[l];
+      if (e == 0 && total == 0) tiles.list[l][0] = Tile{0, 0, 0, 0};
+      for (uint32_t j = 0; j < mine[l]; ++j)
+        tiles.list[l][first + j] = Tile{e, start + j * tokens, min(tokens, c - j * tokens), total};
     }
   }
 }

@@ -673,3 +673,20 @@ def test_prefill_rows_of_512_beside_what_the_resident_kernel_refuses(gpu, oracle
     moe.encode_prefill_layer(wts, ops.bf16_tensor(x), y, t)
     torch.cuda.synchronize()
     assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y)), oracle.bf16_to_float(oracle.moe_layer(layer, x)[0]), f"d={d} fs={fs} t={t}")
+
+
+@pytest.mark.parametrize("bits,d,f,e,k,fs,t", [
+    (4, 960, 128, 4, 2, 0, 70), (4, 1024, 192, 4, 2, 128, 70), (4, 1088, 1024, 8, 2, 0, 40), (4, 1152, 128, 8, 4, 128, 33),
+    (4, 2112, 1088, 4, 2, 0, 90), (2, 960, 1088, 4, 2, 0, 300), (2, 1088, 128, 8, 2, 1024, 50), (2, 1024, 2112, 4, 2, 128, 300),
+    (1, 2112, 1024, 32, 8, 0, 20), (4, 128, 128, 2, 1, 0, 17), (2, 2048, 128, 2, 1, 0, 9),
+])
+def test_prefill_contractions_around_the_steps_of_the_tables(gpu, oracle, bits, d, f, e, k, fs, t):
+    """the tiled matmuls take scales, biases and group sums in steps of 16 K groups: one group less, a whole step, one more, two
+    steps and a half pair; tiles of 64 and of 32 routes; lists of one or two tiles, which leave most XCDs without work"""
+    layer = oracle.synth_layer(ROOT_SEED + 0x57E9 + d + f + t, d, f, e, k, bits=bits, fs=fs, router_mode=1 if bits == 1 else 0)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    x = oracle.synth_x(ROOT_SEED + 0x57 + t, t, d)
+    y, idx, _ = _run_prefill(moe, wts, x, t, d, k)
+    ref, ref_idx, _ = oracle.moe_layer(layer, x)
+    assert np.array_equal(idx, ref_idx)
+    assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref), f"bits={bits} d={d} f={f}")
