@@ -499,11 +499,16 @@ __global__ __launch_bounds__(KS * 64) void rows_mfma_kernel(const RowsMfmaArgs a
 // the L2.  The waves of a workgroup split the chunks of a row
 // set (4 rows); partial sums meet in LDS in a fixed order.
 //
-// Bound by how long a stage waits for its loads: codes are requested two stages ahead into the registers that the stage has just
+// Bound by how long a stage waits for its loads, and by what stands in front of the first and between two stages: codes are requested two stages ahead into the registers that the stage has just
 // read (an empty scheduling barrier keeps every request there: left alone the compiler gathers them behind the last product), a
 // stage's table pieces two stages ahead into registers and to LDS one stage ahead -- written in the stage that requested
-// them they made it wait out a whole round trip -- and a request is a scalar base and a constant offset per lane.  4-bit MLP of 5120 x 17408,
-// one / four rows: 43.4 / 47.3 -> 39.5 / 43.5 us; 2-bit 40.8 / 45.2 -> 35.3 / 40.1; 4-bit 4096 x 12800 30.5 / 33.2 -> 26.6 / 29.4.
+// them they made it wait out a whole round trip -- and a request is a scalar base and a constant offset per lane.  x: of the 20 us of a
+// 5120 x 17408 projection over four rows every wave spent 3.7 on making its operands, when both its stages were there and nothing was on its way,
+// and one wave 0.45 a stage on adding up totals the others wait for; now an integer addition and a permutation per two numbers, sums of x and of
+// the wave's blocks by the matrix core and row swaps.  MLPs, one / four / eight rows, us, before -> now: 4-bit 5120 x 17408
+// 41.0 / 45.8 / 58.9 -> 39.6 / 43.2 / 56.2, 4096 x 12800 27.5 / 31.0 / 41.3 -> 24.9 / 29.1 / 40.3, 2048 x 6400 16.2 / 20.7 / 24.7 ->
+// 15.5 / 20.1 / 24.4; 2-bit 5120 x 17408 37.9 / 42.6 / 60.9 -> 32.5 / 40.1 / 54.6.  (More stages ahead, by loads straight to LDS, gained
+// nothing: such a load takes 40 ns of a CU per KB, 6.5 TB/s over the chip, and x waits behind what is requested in front of it.)
 struct RowsQuadArgs {
   const uint8_t* W[2];
   const uint16_t* S[2];
@@ -524,7 +529,18 @@ __device__ __forceinline__ f32x4_t mfma_quad(uint2 a, uint2 b, f32x4_t c) {
 constexpr uint32_t kQuadMaxWaves = 8;
 // LDS of one wave: table pieces of two stages, partial sums of two buffers
 constexpr uint32_t kQuadTabBytes = 2 * 64 * 8 * sizeof(uint16_t);
-__host__ __device__ constexpr uint32_t quad_wave_bytes(int nproj) { return kQuadTabBytes + 2u * nproj * 4 * 4 * 4 * sizeof(float); }
+__host__ __device__ constexpr uint32_t quad_wave_bytes(int nproj) { return kQuadTabBytes + 2u * nproj * 4 * 4 * sizeof(float); }
+
+// u + v over pairs of 16-lane rows: rows 0 and 2 of the result hold u's sums of rows 0 + 1 and 2 + 3, rows 1 and 3 v's; over the
+// halves of the wave: the lower half holds u's sums, the upper one v's
+__device__ __forceinline__ float swap_rows_sum(float u, float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float swap_halves_sum(float u, float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(u), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 
 // BITS 4, or 2: the chunk is then 8 bytes -- again 32 K values, half a group.
 // ANY: K is any multiple of 64; otherwise of 512, so that the table pieces are whole and aligned.
@@ -542,10 +558,10 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
   // [buffer][projection][16-lane row][weight row][token]
   constexpr uint32_t kWaveFloats = quad_wave_bytes(NPROJ) / sizeof(float), kTabFloats = kQuadTabBytes / sizeof(float);
   extern __shared__ __attribute__((aligned(16))) float s_quad[];
-  const uint32_t lane = threadIdx.x & 63, wsub = threadIdx.x >> 6, wpr = blockDim.x >> 6;
+  const uint32_t lane = threadIdx.x & 63, wsub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wpr = blockDim.x >> 6;
   const uint32_t b = lane >> 2, c = lane & 3;
-  auto part_of = [&](uint32_t w, uint32_t pb, int p, uint32_t r, uint32_t row) __attribute__((always_inline)) {
-    return s_quad + w * kWaveFloats + kTabFloats + (((pb * NPROJ + p) * 4 + r) * 4 + row) * 4;
+  auto part_of = [&](uint32_t w, uint32_t pb, int p) __attribute__((always_inline)) {
+    return s_quad + w * kWaveFloats + kTabFloats + (pb * NPROJ + p) * 16;
   };
   const uint32_t n_chunks = a.N / 32, ng = a.N / kGroup, n_sets = a.M / 4;
   const size_t row_bytes = static_cast<size_t>(a.N) * BITS / 8;
@@ -587,8 +603,7 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
     const uint16_t* piece = (tb_bias ? a.B[p] : a.S[p]) + (static_cast<size_t>(set) * 4 + tb_row) * ng + tb_group;
     return ANY ? load_16_bytes(piece) : *reinterpret_cast<const uint4*>(piece);
   };
-  // the wave's part of D[token, row] for one row set; then the four blocks of each 16-lane row
-  // are added and lanes 0..3 of the row leave [weight row][token] in LDS.  `refill` is the row
+  // the wave's part of D[token, row] for one row set; then the sixteen blocks are added and leave [token][weight row] in LDS.  `refill` is the row
   // set whose stage takes over the ring slots.
   auto compute = [&](int buf, int p, uint32_t pb, uint32_t refill) __attribute__((always_inline)) {
     f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -628,28 +643,28 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
     // the next stage's pieces, requested a stage ago, to LDS
     __builtin_amdgcn_wave_barrier();
     *reinterpret_cast<uint4*>(my_tab + (buf ^ 1) * (64 * 8) + lane * 8) = ANY ? drop_bf16(tbr[buf ^ 1], tb_drop) : tbr[buf ^ 1];
-    float v[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       // (back at their own scale first: token t's x is lane t's of the quad)
       acc[t] *= t == 0 ? dpp_f<0x00>(rel) : t == 1 ? dpp_f<0x55>(rel) : t == 2 ? dpp_f<0xAA>(rel) : dpp_f<0xFF>(rel);
-      v[t] = acc[t] + dpp_f<0x124>(acc[t]);  // + lane - 4 (rotation inside the 16-lane row)
-      v[t] = v[t] + dpp_f<0x128>(v[t]);      // + lane - 8
+      acc[t] = acc[t] + dpp_f<0x124>(acc[t]);  // + lane - 4 (rotation inside the 16-lane row)
+      acc[t] = acc[t] + dpp_f<0x128>(acc[t]);  // + lane - 8
     }
-    if ((lane & 12u) == 0)
-      *reinterpret_cast<float4*>(part_of(wsub, pb, p, lane >> 4, c)) = make_float4(v[0], v[1], v[2], v[3]);
+    // the four 16-lane rows: tokens 0 and 1 (2 and 3) trade odd for even rows, then the pairs the halves of the wave, so that row t
+    // ends with token t's total
+    const float total = swap_halves_sum(swap_rows_sum(acc[0], acc[1]), swap_rows_sum(acc[2], acc[3]));
+    if ((lane & 12u) == 0) part_of(wsub, pb, p)[(lane >> 4) * 4 + c] = total;
   };
-  // threads 0..15: (weight row, token) totals in wave then row order
+  // threads 0..15: (token, weight row) totals in the waves' order
   auto combine = [&](uint32_t set, uint32_t pb) __attribute__((always_inline)) {
     if (threadIdx.x >= 16) return;
     const uint32_t cc = threadIdx.x & 3, t = threadIdx.x >> 2;
     float v[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
-      v[p] = 0.0f;
-      for (uint32_t w = 0; w < wpr; ++w)
+      v[p] = part_of(0, pb, p)[threadIdx.x];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[p] = v[p] + part_of(w, pb, p, r, cc)[t];
+      for (uint32_t w = 1; w < kQuadMaxWaves; ++w) v[p] = v[p] + (w < wpr ? part_of(w, pb, p)[threadIdx.x] : 0.0f);
     }
     if (t >= a.T) return;
     const size_t at = static_cast<size_t>(t) * a.M + set * 4 + cc;
@@ -677,15 +692,20 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
   }
   // ---- this lane's x: token c, chunks (wsub * ITS + j) * 16 + b.  The first two stages' weight
   // loads are already on their way: the x rows come from L2 behind them.
+  // (a lane without a token or a chunk loads another's and drops it: no branch between the loads)
   uint4 raw[ITS][4];
 #pragma unroll
   for (int j = 0; j < ITS; ++j) {
-    const uint32_t ch = (wsub * ITS + j) * 16 + b;
-    const bool live = ch < n_chunks && c < a.T;
+    const uint16_t* from = a.x + static_cast<size_t>(min(c, a.T - 1)) * a.N + min((wsub * ITS + j) * 16 + b, n_chunks - 1) * 32;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      raw[j][i] = make_uint4(0, 0, 0, 0);
-      if (live) raw[j][i] = *reinterpret_cast<const uint4*>(a.x + static_cast<size_t>(c) * a.N + ch * 32 + 8 * i);
+    for (int i = 0; i < 4; ++i) raw[j][i] = *reinterpret_cast<const uint4*>(from + 8 * i);
+  }
+  if (a.T < 4 || (wsub + 1) * ITS * 16 > n_chunks) {
+#pragma unroll
+    for (int j = 0; j < ITS; ++j) {
+      const bool live = (wsub * ITS + j) * 16 + b < n_chunks && c < a.T;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) raw[j][i] = live ? raw[j][i] : make_uint4(0, 0, 0, 0);
     }
   }
   // A lane's x has the scale that its own squares ask for: the blocks of a wave are separate products, whose results are brought back
@@ -700,25 +720,49 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
       squares[2] = dot2_bf16(raw[j][i].z, raw[j][i].z, squares[2]);
       squares[3] = dot2_bf16(raw[j][i].w, raw[j][i].w, squares[3]);
     }
-  const float x_scale = scale_of_squares((squares[0] + squares[1]) + (squares[2] + squares[3]));
+  // (a lane without a token or a chunk: zeros, at any scale)
+  const float x_scale = c >= a.T || wsub * ITS * 16 + b >= n_chunks ? kRowScale : scale_of_squares((squares[0] + squares[1]) + (squares[2] + squares[3]));
   rel = rel_of_scale(x_scale);
+  // the chunks' sums from the matrix core, 32 numbers against ones; three bf16 terms each
 #pragma unroll
   for (int j = 0; j < ITS; ++j) {
-    float sum = 0.0f;
+    f32x4_t sums = {0.0f, 0.0f, 0.0f, 0.0f};
+    const uint2 ones = make_uint2(0x3F803F80u, 0x3F803F80u);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float part;
-      const uint4 o = matmul_row8(raw[j][i], x_scale, &part);
-      xa[j][2 * i] = make_uint2(o.x, o.y);
-      xa[j][2 * i + 1] = make_uint2(o.z, o.w);
-      sum += part;
+      sums = mfma_quad(make_uint2(raw[j][i].x, raw[j][i].y), ones, sums);
+      sums = mfma_quad(make_uint2(raw[j][i].z, raw[j][i].w), ones, sums);
     }
-    sum *= x_scale * kRowUnscale;
+    const float sum = (c == 0 ? sums[0] : c == 1 ? sums[1] : c == 2 ? sums[2] : sums[3]) * (x_scale * kRowUnscale);
     const uint32_t hi = __float_as_uint(sum) & 0xFFFF0000u;
     const float r1 = sum - __uint_as_float(hi);
     const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
     const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
     sx[j] = make_uint2((hi >> 16) | mid, lo >> 16);  // K slots: hi, mid, lo, 0
+  }
+  // Ordinary lanes: 2^64 is 64 more in every exponent field, which neither overflows nor carries (a zero becomes 2^-63, whose products
+  // with codes of at most 2^-125 are zero in fp32 as its own are; so is the product of a number below 2^-126, whose field is zero).
+  if (__builtin_expect(__all(x_scale == kRowScale), 1)) {
+#pragma unroll
+    for (int j = 0; j < ITS; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        constexpr uint32_t kMore = 0x20002000u;
+        const uint32_t v[4] = {raw[j][i].x + kMore, raw[j][i].y + kMore, raw[j][i].z + kMore, raw[j][i].w + kMore};
+        // (0, 4), (1, 5), (2, 6), (3, 7)
+        xa[j][2 * i] = make_uint2(__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u));
+        xa[j][2 * i + 1] = make_uint2(__builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u));
+      }
+  } else {
+#pragma unroll
+    for (int j = 0; j < ITS; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float part;
+        const uint4 o = matmul_row8(raw[j][i], x_scale, &part);
+        xa[j][2 * i] = make_uint2(o.x, o.y);
+        xa[j][2 * i + 1] = make_uint2(o.z, o.w);
+      }
   }
 
   *reinterpret_cast<uint4*>(my_tab + lane * 8) = ANY ? drop_bf16(t0, tb_drop) : t0;

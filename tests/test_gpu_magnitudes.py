@@ -181,6 +181,37 @@ def test_few_rows_far_from_one(gpu, bits, m, n, t):
     assert all(torch.equal(out[0], o) for o in out[1:]) and (out[0] != 0).all()
 
 
+@pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("m,n,t", [(4096, 4096, 4), (4096, 3136, 3), (5120, 17408, 7)])
+def test_few_rows_of_zeros_and_numbers_too_small_for_a_product(gpu, bits, m, n, t):
+    """rows of zeros, single zeros and bf16 subnormals beside ordinary rows, whose lanes take the power of two by an addition to the
+    exponent fields: a zero has no product and no part in a sum, a row has the bits it has alone"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m + n + t + bits)
+    q = ops.Quantization(gpu).quantize_affine(torch.randn((m, n), generator=gen, device="cuda") * 0.02 + 0.01, bits)
+    x = torch.randn((t, n), generator=gen, device="cuda").to(torch.bfloat16)
+    x[0] = 0.0
+    x[1, ::3] = 0.0
+    x[1, 1::3] = -0.0
+    x[2, 5:200] = 2.0 ** -130
+    op = ops.DequantInt4GEMVMultiX(gpu)
+    y, one = torch.full((t, m), 9.0, device="cuda"), torch.full((1, m), 9.0, device="cuda")
+    op.encode(q, x, y, m, n, t, output_float32=True)
+    for r in range(t):
+        op.encode(q, x[r:r + 1].contiguous(), one, m, n, 1, output_float32=True)
+        torch.cuda.synchronize()
+        assert torch.equal(one[0], y[r]), r
+    assert (y[0] == 0).all()
+    without = x.clone()
+    without[2, 5:200] = 0.0
+    z = torch.zeros_like(y)
+    op.encode(q, without, z, m, n, t, output_float32=True)
+    torch.cuda.synchronize()
+    # 195 numbers of 2^-130 against weights below 1 are under 2^-122: none of it is left in a sum of ordinary ones, which may only be
+    # rounded elsewhere on its way (each of the up to 9 sums a lane makes per group, 2^-24 of what it has: under 1e-6 of the whole)
+    assert torch.linalg.norm(z[2].double() - y[2].double()) <= 1e-6 * torch.linalg.norm(z[2].double())
+
+
 @pytest.mark.parametrize("d,f,t,apart", [(128, 64, 16, 1), (576, 128, 70, 1), (192, 2112, 530, 3)])
 def test_int8_matmul_of_small_codes_beside_large_values(gpu, d, f, t, apart):
     """every group holds A and -A against the same code and, elsewhere, numbers from 1 to 2 against codes of 1 to 3: gate is
