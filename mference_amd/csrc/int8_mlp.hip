@@ -116,7 +116,9 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // small codes beside large values of x lost bits: rms error over the size of the terms 2.4e-8 -> 7.8e-8 at 2112 x 2816, 300 rows, nine
 // codes of ten below 16 and one value of 1000 in a row, 3.9e-8 -> 4.3e-7 at 256 x 128.  The 2- and 4-bit codes sit at the top of the byte.)
 //
-// A workgroup is 64 weight rows (of each projection) x 64 tokens, waves 2 x 2.  A stage is 128 K values: x rows and
+// A workgroup is 64 weight rows (of each projection) x 64 tokens.  Its four waves are 2 row blocks x 2 projections, or with one projection x
+// the 2 groups of a stage, and each takes all 64 tokens: what bounds the kernel is vector instructions, above all those that make numbers of
+// the codes, and so every code is converted once in a workgroup (waves of 2 row blocks x 2 token blocks did it twice).  A stage is 128 K values: x rows and
 // code rows come in as whole 128-byte lines, three stages ahead of their use (two sets of registers and an LDS buffer: a stage's
 // arithmetic is 0.5 us, a round trip to memory 1 to 2), and are handed out through LDS (16-byte
 // pieces, XOR-swizzled so that 16 lanes reading one piece of 16 rows cover all banks): read straight from memory a
@@ -124,9 +126,10 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // core, would set the pace.  Scales and biases come 8 groups (four stages) to a load.
 // KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
 // meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
-// loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens: gate/up 47.6 -> 37.9 us, down 23.8 -> 20.0).
-// The MLP, us, with a stage requested one ahead / now: 2816 x 2112, 16 rows 48.3 / 49.5, 300 53.2 / 53.6, 600 87.9 / 84.4,
-// 2048 223 / 220; 704 x 8192, 16 rows 67.4 / 64.5, 300 92.4 / 87.1; 2048 x 2048, 16 rows 43.7 / 39.1, 1024 76.7 / 68.9.
+// loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens, waves of two token blocks: gate/up 47.6 -> 37.9 us).
+// The MLP, us, waves of two token blocks with results stored by their lanes / now: 2816 x 2112, 16 rows 49.8 / 43.3, 300 53.8 / 46.8, 600
+// 84.3 / 73.6, 2048 220.7 / 199.5; 704 x 8192, 16 rows 63.2 / 57.3, 300 87.3 / 79.2, 2048 240 / 204; 2048 x 2048, 16 rows 39.2 / 34.3, 1024
+// 70.3 / 61.0; 192 x 128, 64 rows 12.3 / 10.4.
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
 
@@ -148,8 +151,8 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   const uint32_t per = (n_work + 7) / 8, work = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   if ((blockIdx.x >> 3) >= per || work >= n_work) return;
   const uint32_t t0 = (work % n_tiles) * kTok, r0 = (work / n_tiles) * 64;
-  const uint32_t lane = tid & 63, wv = tid >> 6, m = lane & 31, h = lane >> 5;
-  const uint32_t rb = wv & 1, tb = wv >> 1;
+  const uint32_t lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), m = lane & 31, h = lane >> 5;
+  const uint32_t rb = wv & 1, z = wv >> 1;
   const uint32_t ng = a.N / kGroup, n_st = (ng + 1) / 2;
   const uint32_t n_walk = (n_st + KS - 1) / KS, st0 = kh * n_walk, st1 = min(n_st, st0 + n_walk);  // this set's stages
 
@@ -176,23 +179,23 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
         ws[p][i] = *reinterpret_cast<const u32x4_t*>(a.W[p] + static_cast<size_t>(min(r0 + wr + 32 * i, a.M - 1)) * a.N + k0);
     }
   };
-  // scales and biases of the eight groups from g (a group of the row) on; groups past the row's last one are zeros
-  struct Tab { uint4 S[NPROJ], B[NPROJ]; };
+  // scales and biases of the wave's projection
+  const uint16_t* tab_s = a.S[NPROJ == 2 ? z : 0];
+  const uint16_t* tab_b = a.B[NPROJ == 2 ? z : 0];
+  // those of the eight groups from g (a group of the row) on; groups past the row's last one are zeros
+  struct Tab { uint4 S, B; };
   auto fetch_tab = [&](uint32_t g) __attribute__((always_inline)) {
     Tab t;
     // (a load past the row's last group reads on into the next row, the table's last loads end with the table: what is not the row's is taken off)
     const uint32_t at = row * ng + g, base = min(at, a.M * ng - 8);
+    t.S = drop_bf16(load_16_bytes(tab_s + base), at - base);
+    t.B = drop_bf16(load_16_bytes(tab_b + base), at - base);
+    if (g + 8 > ng) {
+      uint32_t keep[4];
 #pragma unroll
-    for (int p = 0; p < NPROJ; ++p) {
-      t.S[p] = drop_bf16(load_16_bytes(a.S[p] + base), at - base);
-      t.B[p] = drop_bf16(load_16_bytes(a.B[p] + base), at - base);
-      if (g + 8 > ng) {
-        uint32_t keep[4];
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) keep[i] = g + 2 * i + 1 < ng ? 0xFFFFFFFFu : g + 2 * i < ng ? 0xFFFFu : 0u;
-        t.S[p] = make_uint4(t.S[p].x & keep[0], t.S[p].y & keep[1], t.S[p].z & keep[2], t.S[p].w & keep[3]);
-        t.B[p] = make_uint4(t.B[p].x & keep[0], t.B[p].y & keep[1], t.B[p].z & keep[2], t.B[p].w & keep[3]);
-      }
+      for (uint32_t i = 0; i < 4; ++i) keep[i] = g + 2 * i + 1 < ng ? 0xFFFFFFFFu : g + 2 * i < ng ? 0xFFFFu : 0u;
+      t.S = make_uint4(t.S.x & keep[0], t.S.y & keep[1], t.S.z & keep[2], t.S.w & keep[3]);
+      t.B = make_uint4(t.B.x & keep[0], t.B.y & keep[1], t.B.z & keep[2], t.B.w & keep[3]);
     }
     return t;
   };
@@ -215,59 +218,62 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
         reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = ws[p][i];
       }
   };
-  f32x16_t acc[NPROJ];
-  const uint32_t tok_m = tb * 32 + m;  // the token whose x operands this lane reads
+  // acc[j]: tokens of block j ^ z (with one projection, the bias term of wave z's own block is its first accumulator's)
+  f32x16_t acc[2];
 #pragma unroll
-  for (int p = 0; p < NPROJ; ++p)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[p][r] = 0.0f;
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+  const uint32_t tok_of[2] = {z * 32 + m, (z ^ 1u) * 32 + m};  // the tokens whose x operands this lane reads
 
-  // one stage out of LDS; scale(p, g): of projection p and the stage's group g; bias(p): the bits of that of group h
-  auto multiply = [&](uint32_t buf, auto scale, auto bias) __attribute__((always_inline)) {
-    // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0)
-    {
-      const float v = s_sum[buf][tok_m][h];
+  // one stage out of LDS; scale(g): of the stage's group g; bias: the bits of that of group h
+  auto multiply = [&](uint32_t buf, auto scale, uint32_t bias) __attribute__((always_inline)) {
+    // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0).  Two projections:
+    // each wave its own, for both blocks; one: the two waves of a row block share both groups, and each takes one block.
+#pragma unroll
+    for (int j = 0; j < NPROJ; ++j) {
+      const float v = s_sum[buf][tok_of[j]][h];
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
       const float r1 = __builtin_isinf(v) ? 0.0f : v - __uint_as_float(hi);  // (an infinite sum has no rest: inf - inf would be NaN)
       const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
       const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
-      const uint4 av = make_uint4((hi >> 16) | mid, lo >> 16, 0, 0);
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        const uint32_t b = bias(p);
-        acc[p] = mfma_bf16(av, make_uint4(b | (b << 16), b, 0, 0), acc[p]);
-      }
+      acc[j] = mfma_bf16(make_uint4((hi >> 16) | mid, lo >> 16, 0, 0), make_uint4(bias | (bias << 16), bias, 0, 0), acc[j]);
     }
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      uint4 bx[4];
+    for (int gi = 0; gi < NPROJ; ++gi) {
+      const uint32_t g = NPROJ == 2 ? gi : z;
+      uint4 bx[2][4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) bx[s] = s_x[buf][tok_m * 16 + ((8 * g + 4 * h + s) ^ (tok_m & 15u))];
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        const uint32_t r = rb * 32 + m;
-        f32x16_t tmp;
+        for (int s = 0; s < 4; ++s) bx[j][s] = s_x[buf][tok_of[j] * 16 + ((8 * g + 4 * h + s) ^ (tok_of[j] & 15u))];
+      const uint32_t r = rb * 32 + m;
+      f32x16_t tmp[2];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) tmp[i] = 0.0f;
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const uint4 w = s_w[buf][p][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
-          const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+        for (int i = 0; i < 16; ++i) tmp[j][i] = 0.0f;
 #pragma unroll
-          for (int u = 0; u < 2; ++u) {  // eight codes -> eight bf16 numbers (a byte as fp32 has its bits in the upper half)
-            uint32_t o[4];
+      for (int c = 0; c < 2; ++c) {
+        const uint4 w = s_w[buf][NPROJ == 2 ? z : 0][r * 8 + ((4 * g + 2 * h + c) ^ ((r >> 1) & 7u))];
+        const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const uint32_t word = ww[2 * u + (k >> 1)] >> (16 * (k & 1));
-              o[k] = upper_halves(static_cast<float>(word & 0xFFu), static_cast<float>((word >> 8) & 0xFFu));
-            }
-            tmp = mfma_bf16(bx[2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp);
+        for (int u = 0; u < 2; ++u) {  // eight codes -> eight bf16 numbers (a byte as fp32 has its bits in the upper half)
+          uint32_t o[4];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const uint32_t word = ww[2 * u + (k >> 1)] >> (16 * (k & 1));
+            o[k] = upper_halves(static_cast<float>(word & 0xFFu), static_cast<float>((word >> 8) & 0xFFu));
           }
-        }
-        const float s = scale(p, g);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[p][i] = __builtin_fmaf(s, tmp[i], acc[p][i]);
+          for (int j = 0; j < 2; ++j) tmp[j] = mfma_bf16(bx[j][2 * c + u], make_uint4(o[0], o[1], o[2], o[3]), tmp[j]);
+        }
       }
+      const float s = scale(g);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[j][i] = __builtin_fmaf(s, tmp[j][i], acc[j][i]);
     }
   };
   if constexpr (LONG) {
@@ -287,26 +293,17 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
         const int buf = u4 & 1, other = buf ^ 1;
         if (i0 + u4 + 1 < n_walk) put(other, xr[other], wreg[other]);
         fetch(st0 + i0 + u4 + 3, xr[other], wreg[other]);
-        uint32_t sw[NPROJ], bw[NPROJ];
-#pragma unroll
-        for (int p = 0; p < NPROJ; ++p) {
-          const uint32_t s4[4] = {tab.S[p].x, tab.S[p].y, tab.S[p].z, tab.S[p].w}, b4[4] = {tab.B[p].x, tab.B[p].y, tab.B[p].z, tab.B[p].w};
-          sw[p] = s4[u4];
-          bw[p] = b4[u4];
-        }
-        multiply(buf, [&](int p, int g) { return g ? bf16_hi(sw[p]) : bf16_lo(sw[p]); }, [&](int p) { return h ? bw[p] >> 16 : bw[p] & 0xFFFFu; });
+        const uint32_t s4[4] = {tab.S.x, tab.S.y, tab.S.z, tab.S.w}, b4[4] = {tab.B.x, tab.B.y, tab.B.z, tab.B.w};
+        multiply(buf, [&](uint32_t g) { return g ? bf16_hi(s4[u4]) : bf16_lo(s4[u4]); }, h ? b4[u4] >> 16 : b4[u4] & 0xFFFFu);
       }
     }
   } else {
-    uint16_t sc[NPROJ][2], bi[NPROJ];  // a stage's table entries
+    uint16_t sc[2], bi;  // a stage's table entries
     auto fetch_entries = [&](uint32_t st) __attribute__((always_inline)) {
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) {
-        const size_t at = static_cast<size_t>(row) * ng;
-        sc[p][0] = a.S[p][at + min(2 * st, ng - 1)];
-        sc[p][1] = a.S[p][at + min(2 * st + 1, ng - 1)];
-        bi[p] = a.B[p][at + min(2 * st + h, ng - 1)];
-      }
+      const size_t at = static_cast<size_t>(row) * ng;
+      sc[0] = tab_s[at + min(2 * st, ng - 1)];
+      sc[1] = tab_s[at + min(2 * st + 1, ng - 1)];
+      bi = tab_b[at + min(2 * st + h, ng - 1)];
     };
     if (st0 < st1) {
       fetch(st0, xr[0], wreg[0]);
@@ -318,49 +315,46 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     for (uint32_t i = 0; i < n_walk; ++i) {
       __syncthreads();
       if (st0 + i >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
-      uint16_t sv[NPROJ][2], bv[NPROJ];
-#pragma unroll
-      for (int p = 0; p < NPROJ; ++p) sv[p][0] = sc[p][0], sv[p][1] = sc[p][1], bv[p] = bi[p];
+      const uint16_t sv[2] = {sc[0], sc[1]}, bv = bi;
       if (st0 + i + 1 < st1) {
         put((i + 1) & 1u, xr[0], wreg[0]);
         fetch_entries(st0 + i + 1);
         if (st0 + i + 2 < st1) fetch(st0 + i + 2, xr[0], wreg[0]);
       }
-      multiply(i & 1u, [&](int p, int g) { return bf16_to_f(sv[p][g]); }, [&](int p) -> uint32_t { return bv[p]; });
+      multiply(i & 1u, [&](uint32_t g) { return bf16_to_f(g ? sv[1] : sv[0]); }, bv);
     }
   }
-  if constexpr (KS == 2) {  // the second set's sums to the first, over the x buffers
-    static_assert(sizeof(s_x_all) >= 4u * 64 * NPROJ * 16 * sizeof(float), "the sums fit the x buffers");
-    float* s_acc = reinterpret_cast<float*>(&s_x_all[0][0][0]);
-    __syncthreads();
-    if (kh == 1) {
+  // All sums go through LDS, over the x buffers, [set][part = wave's z][token][row], and the whole workgroup stores: 64 rows of a token per
+  // wave and step, in a loop that stays short (straight-line code that runs once costs its fetch: with 16 results a lane of the first set's
+  // waves it was 2400 instructions).
+  static_assert(sizeof(s_x_all) >= KS * 2u * 64 * 64 * sizeof(float), "the sums fit the x buffers");
+  float* s_acc = reinterpret_cast<float*>(&s_x_all[0][0][0]);
+  __syncthreads();
 #pragma unroll
-      for (int p = 0; p < NPROJ; ++p)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s_acc[(p * 16 + i) * 256 + tid] = acc[p][i];
-    }
-    __syncthreads();
-    if (kh == 1) return;
-#pragma unroll
-    for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[p][i] = acc[p][i] + s_acc[(p * 16 + i) * 256 + tid];
-  }
-  // the lane holds weight row r0 + 32 rb + m for tokens 8j + 4h + i of each 32-token block
-  const uint32_t out_row = r0 + rb * 32 + m;
+    for (int i = 0; i < 16; ++i)  // the lane holds weight row r0 + 32 rb + m for tokens 8 (i / 4) + 4h + i % 4 of a 32-token block
+      s_acc[((kh * 2 + z) * 64 + (z ^ j) * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 64 + rb * 32 + m] = acc[j][i];
+  __syncthreads();
+  const uint32_t out_row = r0 + lane, n_tok = min(kTok, a.T - t0);
   if (out_row >= a.M) return;
+#pragma unroll 2
+  for (uint32_t tok = kh * 4 + wv; tok < n_tok; tok += 4 * KS) {
+    float v[2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t tok = t0 + tb * 32 + 8 * j + 4 * h + i;
-      if (tok >= a.T) continue;
-      const size_t at = static_cast<size_t>(tok) * a.M + out_row;
-      const float v = acc[0][4 * j + i];
-      if constexpr (NPROJ == 2) static_cast<uint16_t*>(a.y)[at] = q8_activation(v, acc[NPROJ - 1][4 * j + i], a.silu != 0);
-      else if (a.out_f32) static_cast<float*>(a.y)[at] = v;
-      else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(v);
+    for (uint32_t p = 0; p < 2; ++p) {
+      v[p] = s_acc[(p * 64 + tok) * 64 + lane];
+      if constexpr (KS == 2) v[p] = v[p] + s_acc[((2 + p) * 64 + tok) * 64 + lane];
     }
+    const size_t at = static_cast<size_t>(t0 + tok) * a.M + out_row;
+    if constexpr (NPROJ == 2) {
+      static_cast<uint16_t*>(a.y)[at] = q8_activation(v[0], v[1], a.silu != 0);
+    } else {
+      const float sum = v[0] + v[1];
+      if (a.out_f32) static_cast<float*>(a.y)[at] = sum;
+      else static_cast<uint16_t*>(a.y)[at] = f_to_bf16(sum);
+    }
+  }
 }
 
 // Which kernel: from 16 token rows on the matmul (its workgroups take 64 tokens at the price of one), below that the row
