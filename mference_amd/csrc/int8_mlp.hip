@@ -127,9 +127,9 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // KS = 2: two such sets of four waves share the workgroup, each walks half of K in buffers of its own, and their sums
 // meet in LDS at the end -- for problems of at most a workgroup per CU, where one wave to a SIMD neither hides its
 // loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens, waves of two token blocks: gate/up 47.6 -> 37.9 us).
-// The MLP, us, waves of two token blocks with results stored by their lanes / now: 2816 x 2112, 16 rows 49.8 / 43.3, 300 53.8 / 46.8, 600
-// 84.3 / 73.6, 2048 220.7 / 199.5; 704 x 8192, 16 rows 63.2 / 57.3, 300 87.3 / 79.2, 2048 240 / 204; 2048 x 2048, 16 rows 39.2 / 34.3, 1024
-// 70.3 / 61.0; 192 x 128, 64 rows 12.3 / 10.4.
+// The MLP, us, waves of two token blocks with results stored by their lanes / now: 2816 x 2112, 16 rows 49.8 / 43.1, 300 53.8 / 47.1, 600
+// 84.3 / 75.1, 2048 220.7 / 199.8; 704 x 8192, 16 rows 63.2 / 59.8, 300 87.3 / 81.5, 2048 240 / 220; 2048 x 2048, 16 rows 39.2 / 34.6, 1024
+// 70.3 / 64.1; 192 x 128, 64 rows 12.3 / 10.6.
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
 
@@ -218,21 +218,21 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
         reinterpret_cast<u32x4_t*>(s_w[buf][p])[r * 8 + (wc ^ ((r >> 1) & 7u))] = ws[p][i];
       }
   };
-  // acc[j]: tokens of block j ^ z (with one projection, the bias term of wave z's own block is its first accumulator's)
-  f32x16_t acc[2];
+  f32x16_t acc[2];  // of the two blocks of 32 tokens
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
-  const uint32_t tok_of[2] = {z * 32 + m, (z ^ 1u) * 32 + m};  // the tokens whose x operands this lane reads
+  const uint32_t tok_of[2] = {m, 32 + m};  // the tokens whose x operands this lane reads
 
   // one stage out of LDS; scale(g): of the stage's group g; bias: the bits of that of group h
   auto multiply = [&](uint32_t buf, auto scale, uint32_t bias) __attribute__((always_inline)) {
-    // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0).  Two projections:
-    // each wave its own, for both blocks; one: the two waves of a row block share both groups, and each takes one block.
+    // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0).  With one projection a
+    // wave takes its own group's alone: q x and the bias term mostly cancel, so they belong into one sum (both groups' biases in one of
+    // the two waves' sums: error against 64 bits 1.6e-7 -> 2.5e-7 at 2112 x 2816).
 #pragma unroll
-    for (int j = 0; j < NPROJ; ++j) {
-      const float v = s_sum[buf][tok_of[j]][h];
+    for (int j = 0; j < 2; ++j) {
+      const float v = NPROJ == 2 || h == z ? s_sum[buf][tok_of[j]][h] : 0.0f;
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
       const float r1 = __builtin_isinf(v) ? 0.0f : v - __uint_as_float(hi);  // (an infinite sum has no rest: inf - inf would be NaN)
       const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
@@ -334,7 +334,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i)  // the lane holds weight row r0 + 32 rb + m for tokens 8 (i / 4) + 4h + i % 4 of a 32-token block
-      s_acc[((kh * 2 + z) * 64 + (z ^ j) * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 64 + rb * 32 + m] = acc[j][i];
+      s_acc[((kh * 2 + z) * 64 + j * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 64 + rb * 32 + m] = acc[j][i];
   __syncthreads();
   const uint32_t out_row = r0 + lane, n_tok = min(kTok, a.T - t0);
   if (out_row >= a.M) return;
