@@ -243,6 +243,14 @@ __device__ __forceinline__ void issue_fence() { asm volatile("" ::: "memory"); }
 // every store this wave has issued is acknowledged at its scope
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// LDS[lds + 16 * lane ...] = the 16 bytes at p of every lane (lds: a byte address, uniform), without a register in between.  The
+// compiler does not know of the request: wait_loads and a barrier stand in front of the first read.
+__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+}
+// every load of this wave but its newest N has arrived
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
 // ------------------------------------------------------------- raw loads
 
 __device__ __forceinline__ uint32_t load_u32_bytes(const uint8_t* p) {

@@ -20,14 +20,6 @@ __host__ __device__ constexpr uint32_t qmm_lds_bytes(uint32_t tile, int nproj) {
   return qmm_x_bytes(tile) + qmm_scale_bytes(nproj) + qmm_sum_bytes(tile) + tile * 12;
 }
 
-// LDS[lds + 16 * lane ...] = the 16 bytes at p of every lane (lds: a byte address, uniform), without a register in between.  The
-// compiler does not know of the request: wait_loads and a barrier stand in front of the first read.
-__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
-}
-// every load of this wave but its newest N has arrived
-template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 // waves a SIMD (workgroups a CU) that the kernels' registers are budgeted for
 __host__ __device__ constexpr int qmm_waves(uint32_t tile, int nproj) { return tile == kSmallTile || nproj == 1 ? 3 : 2; }
 

@@ -142,16 +142,16 @@ __device__ __forceinline__ void router_rows(const uint16_t* __restrict__ W, cons
 // Needs D % 512 == 0 (all 64 chains the same length) and E % 32 == 0.
 typedef __attribute__((ext_vector_type(32))) float f32x32_t;
 
-// N_I = D / 512 as a compile-time constant unrolls the whole walk (a wave's 8 chain pairs x N_I runs): the
+// N_I = D / 512, 2 or 4, as a compile-time constant unrolls the whole walk (a wave's 8 chain pairs x N_I runs): the
 // operand offsets, the ring slots and the levels of the binary counter are then literals, the operand ring
 // needs no register moves and a chain's first instruction takes the constant 0 as its accumulator -- 3.9
-// vector instructions per matrix instruction where the loop for any width (N_I = 0) issues 10.6, and the
+// vector instructions per matrix instruction where a loop with operands in registers issued 10.6, and the
 // matrix instructions of a SIMD wait for its vector instructions (T=2048: 38.6 -> 34.1 us, T=512: 18.5 ->
 // 14.8 us).  (The unrolled form needs 123 registers; eight waves of 8 chains per block, four to a SIMD,
 // measured no faster than these four of 16 chains: 34.7 / 15.8 us.)  Three waves per SIMD: the x-preparation
 // workgroups behind the router's then share the CUs with them instead of waiting for a second round (-1.3 us).
 template <int N_I>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(N_I > 0 ? 3 : 2, N_I > 0 ? 3 : 2)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
                                                                   const uint16_t* __restrict__ x,
                                                                   uint32_t E, uint32_t D, uint32_t T,
@@ -160,7 +160,7 @@ void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
                                                                   const RouterTail tail) {
   constexpr int WAVES = 4, kPairs = 32 / WAVES;  // waves of a workgroup, chain pairs of one wave
   __shared__ float s_part[WAVES - 1][16 * 64];
-  __shared__ uint4 s_stage[N_I > 0 ? WAVES : 1][2][N_I > 0 ? 2 * 128 : 1];  // per wave: x and w, two buffers of 32 rows x 64 B
+  __shared__ uint4 s_stage[WAVES][2][2 * 128];  // per wave: x and w, two buffers of 32 rows x 64 B
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (tail.xp && blockIdx.y >= tail.router_cols) {  // an x-preparation workgroup (rows behind the expert blocks)
     const uint32_t row = ((blockIdx.y - tail.router_cols) * gridDim.x + blockIdx.x) * WAVES + wv;
@@ -171,42 +171,38 @@ void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
   // token tiles vary fastest: workgroups go to the XCDs round-robin, so each XCD's L2 sees an
   // eighth of the token rows (and all of the small router matrix)
   const uint32_t t0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
-  const uint32_t n_i = D / 512;
-  const uint16_t* xrow = x + static_cast<size_t>(min(t0 + m, T - 1)) * x_stride + 8 * (2 * kPairs * wv + b);
-  const uint16_t* wrow = W + static_cast<size_t>(e0 + m) * D + 8 * (2 * kPairs * wv + b);
 
   float lev0[16], lev1[16], lev2[16], total[16];
 #pragma unroll
   for (int r = 0; r < 16; ++r) lev0[r] = lev1[r] = lev2[r] = total[r] = 0.0f;
-  if constexpr (N_I > 0) {
-    // A lane needs 16 bytes of its token row and of its expert row per step -- read straight from memory
-    // that is 32 rows, 32 cache lines, per load instruction, and the L1's line rate, not the matrix core,
-    // sets the pace.  So the wave fetches 64 contiguous bytes of every row at a time (the operands of two
-    // chain pairs: four lanes side by side, 16 lines per instruction) and hands them to itself through a
-    // wave-private LDS buffer.  A stage is (pair group pg, K run i): 2 steps, 16 matrix instructions.  The
-    // two chain pairs of a group keep an accumulator each across the runs.
-    constexpr int kGroups = kPairs / 2, kStages = kGroups * N_I;
-    const uint32_t ld_row = lane >> 2, ld_chunk = lane & 3;  // fetch: rows ld_row, ld_row + 16; 16-byte chunk
-    const uint16_t* xsrc[2];
-    const uint16_t* wsrc[2];
+  // A lane needs 16 bytes of its token row and of its expert row per step -- read straight from memory
+  // that is 32 rows, 32 cache lines, per load instruction, and the L1's line rate, not the matrix core,
+  // sets the pace.  So the wave fetches 64 contiguous bytes of every row at a time (the operands of two
+  // chain pairs: four lanes side by side, 16 lines per instruction) and hands them to itself through a
+  // wave-private LDS buffer.  A stage is (pair group pg, K run i): 2 steps, 16 matrix instructions.  The
+  // two chain pairs of a group keep an accumulator each across the runs.
+  constexpr int kGroups = kPairs / 2, kStages = kGroups * N_I;
+  const uint32_t ld_row = lane >> 2, ld_chunk = lane & 3;  // fetch: rows ld_row, ld_row + 16; 16-byte chunk
+  const uint16_t* xsrc[2];
+  const uint16_t* wsrc[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      xsrc[j] = x + static_cast<size_t>(min(t0 + ld_row + 16 * j, T - 1)) * x_stride + 8 * (2 * kPairs * wv + ld_chunk);
-      wsrc[j] = W + static_cast<size_t>(e0 + ld_row + 16 * j) * D + 8 * (2 * kPairs * wv + ld_chunk);
-    }
-    // LDS rows of 64 bytes; chunk c of row r sits in slot c ^ ((r >> 2) & 3): 16 lanes that read the same
-    // chunk of 16 consecutive rows then cover 256 bytes of distinct banks
-    uint4* stage_x = s_stage[wv][0];
-    uint4* stage_w = s_stage[wv][1];
-    uint32_t st_at[2], rd_at[2];
+  for (int j = 0; j < 2; ++j) {
+    xsrc[j] = x + static_cast<size_t>(min(t0 + ld_row + 16 * j, T - 1)) * x_stride + 8 * (2 * kPairs * wv + ld_chunk);
+    wsrc[j] = W + static_cast<size_t>(e0 + ld_row + 16 * j) * D + 8 * (2 * kPairs * wv + ld_chunk);
+  }
+  // LDS rows of 64 bytes; chunk c of row r sits in slot c ^ ((r >> 2) & 3): 16 lanes that read the same
+  // chunk of 16 consecutive rows then cover 256 bytes of distinct banks
+  uint4* stage_x = s_stage[wv][0];
+  uint4* stage_w = s_stage[wv][1];
+  uint32_t st_at[2], rd_at[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const uint32_t r = ld_row + 16 * j;
-      st_at[j] = r * 4 + (ld_chunk ^ ((r >> 2) & 3));
-      rd_at[j] = m * 4 + ((2 * j + b) ^ ((m >> 2) & 3));  // pair j of the group, block b
-    }
-    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-    u32x4_t fx0, fx1, fw0, fw1;  // the stage on its way from memory to LDS
+  for (int j = 0; j < 2; ++j) {
+    const uint32_t r = ld_row + 16 * j;
+    st_at[j] = r * 4 + (ld_chunk ^ ((r >> 2) & 3));
+    rd_at[j] = m * 4 + ((2 * j + b) ^ ((m >> 2) & 3));  // pair j of the group, block b
+  }
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  u32x4_t fx0, fx1, fw0, fw1;  // the stage on its way from memory to LDS
 #define MF_ROUTER_FETCH(ST)                                                                          \
   do {                                                                                               \
     const int f_off = 32 * ((ST) / N_I) + 512 * ((ST) % N_I);                                        \
@@ -222,141 +218,64 @@ void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
     *reinterpret_cast<u32x4_t*>(stage_w + (BUF) * 128 + st_at[0]) = fw0;                             \
     *reinterpret_cast<u32x4_t*>(stage_w + (BUF) * 128 + st_at[1]) = fw1;                             \
   } while (0)
-    MF_ROUTER_FETCH(0);
-    MF_ROUTER_PUT(0);
-    if (kStages > 1) MF_ROUTER_FETCH(1);
-    f32x32_t acc[2];
+  MF_ROUTER_FETCH(0);
+  MF_ROUTER_PUT(0);
+  if (kStages > 1) MF_ROUTER_FETCH(1);
+  f32x32_t acc[2];
 #pragma unroll
-    for (int st = 0; st < kStages; ++st) {
-      const int pg = st / N_I, i = st % N_I;
+  for (int st = 0; st < kStages; ++st) {
+    const int pg = st / N_I, i = st % N_I;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint4 cxq = stage_x[(st & 1) * 128 + rd_at[j]], cwq = stage_w[(st & 1) * 128 + rd_at[j]];
-        const uint32_t xw[4] = {cxq.x, cxq.y, cxq.z, cxq.w}, ww[4] = {cwq.x, cwq.y, cwq.z, cwq.w};
-        float xa[8], wa[8];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          xa[2 * u] = bf16_lo(xw[u]); xa[2 * u + 1] = bf16_hi(xw[u]);
-          wa[2 * u] = bf16_lo(ww[u]); wa[2 * u + 1] = bf16_hi(ww[u]);
-        }
-        // all 16 operands in registers of their own before the step's first matrix instruction (see below)
-        asm volatile("" : "+v"(xa[0]), "+v"(xa[1]), "+v"(xa[2]), "+v"(xa[3]), "+v"(xa[4]), "+v"(xa[5]), "+v"(xa[6]), "+v"(xa[7]),
-                          "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7]));
-        if (i == 0) {  // a chain's first product lands on 0
-          f32x32_t zero;
-#pragma unroll
-          for (int r = 0; r < 32; ++r) zero[r] = 0.0f;
-          acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[0], wa[0], zero, 0, 0, 0);
-        } else {
-          acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[0], wa[0], acc[j], 0, 0, 0);
-        }
-#pragma unroll
-        for (int u = 1; u < 8; ++u) acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[u], wa[u], acc[j], 0, 0, 0);
-      }
-      if (st + 1 < kStages) {  // the next stage into the other buffer (read last a stage ago), the one after it on its way
-        MF_ROUTER_PUT((st + 1) & 1);
-        if (st + 2 < kStages) MF_ROUTER_FETCH(st + 2);
-      }
-      if (i == N_I - 1) {  // two pairs of chains are complete: stride-1 level, then the binary counter
-        constexpr int kLevels = kPairs == 8 ? 3 : 2;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const int pp = 2 * pg + j;
-          float carry[16];
-#pragma unroll
-          for (int r = 0; r < 16; ++r) carry[r] = acc[j][r] + acc[j][16 + r];
-          int level = 0;
-#pragma unroll
-          for (; level < kLevels && ((pp >> level) & 1); ++level) {
-            float* lv = level == 0 ? lev0 : level == 1 ? lev1 : lev2;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) carry[r] = lv[r] + carry[r];
-          }
-          float* dst = level == kLevels ? total : level == 0 ? lev0 : level == 1 ? lev1 : lev2;
-#pragma unroll
-          for (int r = 0; r < 16; ++r) dst[r] = carry[r];
-        }
-      }
-    }
-#undef MF_ROUTER_FETCH
-#undef MF_ROUTER_PUT
-  } else {
-  // step q = pp * n_i + i: chain pair pp (chains 16 wv + 2 pp + b), K run i; operands run 4 steps ahead
-  const uint32_t steps = 8 * n_i;
-  uint4 cx[4], cw[4], nx[4], nw[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const uint32_t q = min(static_cast<uint32_t>(u), steps - 1), off = 16 * (q / n_i) + 512 * (q % n_i);
-    cx[u] = *reinterpret_cast<const uint4*>(xrow + off);
-    cw[u] = *reinterpret_cast<const uint4*>(wrow + off);
-  }
-  f32x32_t acc;
-#pragma unroll
-  for (int r = 0; r < 32; ++r) acc[r] = 0.0f;
-  uint32_t pp = 0, i = 0;
-  for (uint32_t q0 = 0; q0 < steps; q0 += 4) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const uint32_t q = min(q0 + 4 + u, steps - 1), off = 16 * (q / n_i) + 512 * (q % n_i);
-      nx[u] = *reinterpret_cast<const uint4*>(xrow + off);
-      nw[u] = *reinterpret_cast<const uint4*>(wrow + off);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (q0 + u >= steps) break;
-      // The 16 operands of the step's 8 matrix instructions, each in a register of its own, before the
-      // first of them issues: a vector instruction that writes a register an MFMA in flight still reads
-      // as A or B waits until that MFMA is done (64 cycles here), so operands made one at a time in a
-      // recycled register pair cost 89 instead of 65 cycles per instruction.
-      const uint32_t xw[4] = {cx[u].x, cx[u].y, cx[u].z, cx[u].w}, ww[4] = {cw[u].x, cw[u].y, cw[u].z, cw[u].w};
+    for (int j = 0; j < 2; ++j) {
+      const uint4 cxq = stage_x[(st & 1) * 128 + rd_at[j]], cwq = stage_w[(st & 1) * 128 + rd_at[j]];
+      const uint32_t xw[4] = {cxq.x, cxq.y, cxq.z, cxq.w}, ww[4] = {cwq.x, cwq.y, cwq.z, cwq.w};
       float xa[8], wa[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        xa[2 * j] = bf16_lo(xw[j]); xa[2 * j + 1] = bf16_hi(xw[j]);
-        wa[2 * j] = bf16_lo(ww[j]); wa[2 * j + 1] = bf16_hi(ww[j]);
+      for (int u = 0; u < 4; ++u) {
+        xa[2 * u] = bf16_lo(xw[u]); xa[2 * u + 1] = bf16_hi(xw[u]);
+        wa[2 * u] = bf16_lo(ww[u]); wa[2 * u + 1] = bf16_hi(ww[u]);
       }
+      // all 16 operands in registers of their own before the step's first matrix instruction
       asm volatile("" : "+v"(xa[0]), "+v"(xa[1]), "+v"(xa[2]), "+v"(xa[3]), "+v"(xa[4]), "+v"(xa[5]), "+v"(xa[6]), "+v"(xa[7]),
                         "+v"(wa[0]), "+v"(wa[1]), "+v"(wa[2]), "+v"(wa[3]), "+v"(wa[4]), "+v"(wa[5]), "+v"(wa[6]), "+v"(wa[7]));
+      if (i == 0) {  // a chain's first product lands on 0
+        f32x32_t zero;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[j], wa[j], acc, 0, 0, 0);
-      if (++i == n_i) {  // the pair of chains is complete: stride-1 level, then the binary counter
+        for (int r = 0; r < 32; ++r) zero[r] = 0.0f;
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[0], wa[0], zero, 0, 0, 0);
+      } else {
+        acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[0], wa[0], acc[j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int u = 1; u < 8; ++u) acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(xa[u], wa[u], acc[j], 0, 0, 0);
+    }
+    if (st + 1 < kStages) {  // the next stage into the other buffer (read last a stage ago), the one after it on its way
+      MF_ROUTER_PUT((st + 1) & 1);
+      if (st + 2 < kStages) MF_ROUTER_FETCH(st + 2);
+    }
+    if (i == N_I - 1) {  // two pairs of chains are complete: stride-1 level, then the binary counter
+      constexpr int kLevels = kPairs == 8 ? 3 : 2;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int pp = 2 * pg + j;
         float carry[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) carry[r] = acc[r] + acc[16 + r];
+        for (int r = 0; r < 16; ++r) carry[r] = acc[j][r] + acc[j][16 + r];
+        int level = 0;
 #pragma unroll
-        for (int r = 0; r < 32; ++r) acc[r] = 0.0f;
-        if (pp & 1) {
+        for (; level < kLevels && ((pp >> level) & 1); ++level) {
+          float* lv = level == 0 ? lev0 : level == 1 ? lev1 : lev2;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) carry[r] = lev0[r] + carry[r];
-          if (pp & 2) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) carry[r] = lev1[r] + carry[r];
-            if (pp & 4) {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) total[r] = lev2[r] + carry[r];
-            } else {
-#pragma unroll
-              for (int r = 0; r < 16; ++r) lev2[r] = carry[r];
-            }
-          } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) lev1[r] = carry[r];
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) lev0[r] = carry[r];
+          for (int r = 0; r < 16; ++r) carry[r] = lv[r] + carry[r];
         }
-        i = 0;
-        ++pp;
+        float* dst = level == kLevels ? total : level == 0 ? lev0 : level == 1 ? lev1 : lev2;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dst[r] = carry[r];
       }
     }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      cx[u] = nx[u];
-      cw[u] = nw[u];
-    }
   }
-  }  // the loop for any width
+#undef MF_ROUTER_FETCH
+#undef MF_ROUTER_PUT
   if (wv > 0) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) s_part[wv - 1][r * 64 + lane] = total[r];
@@ -376,6 +295,139 @@ void prefill_router_mfma_kernel(const uint16_t* __restrict__ W,
       const uint32_t t = t0 + 8 * (r / 4) + 4 * b + (r % 4);
       if (t < T) logits[static_cast<size_t>(t) * ld + e0 + m] = v[0];
     }
+  }
+}
+
+// The same for rows of any number of runs of 512, in a loop of one stage (two chain pairs in one run).  What bounds it: a wave's matrix
+// instructions, 64 cycles each, as long as everything else stays out of their way: rows go straight to LDS, three stages ahead.  Unrolled
+// like the kernel above, the 32 stages of a row of 4096 are 32 KB of instructions that a wave runs once and, with a wave to a SIMD,
+// waits for.  Router and selection, us, unrolled / as a loop: 256 rows of 4096, 200 tokens 30.0 / 26.8, 777 tokens 41.0 / 30.5, 2048
+// 60.9 / 52.1, 4096 100.1 / 99.5; of 2048, 777 tokens 19.4 / 20.1, 4096 50.7 / 62.4; of 1024, 777 tokens 14.4 / 15.2.  A loop with operands
+// four steps ahead in registers (16 bytes of a row a lane): 128 rows of 2560, 777 tokens 23.5 / 20.7, 64 rows of 5120 35.1 / 31.5.
+constexpr int kRouterRing = 3;  // stages on their way
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+void prefill_router_loop_kernel(const uint16_t* W, const uint16_t* x, uint32_t E, uint32_t D, uint32_t T, uint32_t x_stride,
+                                float* logits, uint32_t ld, const RouterTail tail) {
+  constexpr int WAVES = 4, kGroups = 4;  // waves of a workgroup; groups of two chain pairs of a wave
+  __shared__ uint4 s_stage[WAVES][kRouterRing][2][128];  // per wave: a ring of stages of x and w, 32 rows x 64 bytes each
+  const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (tail.xp && blockIdx.y >= tail.router_cols) {  // an x-preparation workgroup (rows behind the expert blocks)
+    const uint32_t row = ((blockIdx.y - tail.router_cols) * gridDim.x + blockIdx.x) * WAVES + wv;
+    if (row < T) prep_x_row(x + static_cast<size_t>(row) * x_stride, tail.xp, tail.sums, tail.row_max, tail.w_sg, tail.gate, row, D, lane);
+    return;
+  }
+  const uint32_t m = lane & 31, b = lane >> 5;
+  // token tiles vary fastest: workgroups go to the XCDs round-robin, so each XCD's L2 sees an
+  // eighth of the token rows (and all of the small router matrix)
+  const uint32_t t0 = blockIdx.x * 32, e0 = blockIdx.y * 32;
+  const uint32_t n_i = D / 512, n_st = kGroups * n_i;
+  // fetch: 16 rows an instruction, four lanes to a row; piece c of row r lies in place c ^ (r / 4 % 4), so that 16 lanes that read the
+  // same piece of 16 consecutive rows cover 256 bytes of distinct banks
+  const uint32_t ld_row = lane >> 2, ld_chunk = (lane & 3) ^ ((lane >> 4) & 3);
+  const uint16_t* src[4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    src[j] = x + static_cast<size_t>(min(t0 + ld_row + 16 * j, T - 1)) * x_stride + 8 * (16 * wv + ld_chunk);
+    src[2 + j] = W + static_cast<size_t>(e0 + ld_row + 16 * j) * D + 8 * (16 * wv + ld_chunk);
+  }
+  const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) uint4*)&s_stage[wv][0][0][0]));
+  uint32_t rq_off = 0, rq_i = 0, rq = 0;  // the next stage to request: its first value, its run, its number
+  auto request = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) load_to_lds(src[j] + rq_off, lds + (rq % kRouterRing) * 4096 + j * 1024);
+    ++rq;
+    rq_off += 512;
+    if (++rq_i == n_i) {  // the next group's first run; behind the last stage: the first group's again, which nobody uses
+      rq_i = 0;
+      rq_off = rq < n_st ? 32 * (rq / n_i) : 0;
+    }
+  };
+  uint32_t rd_at[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) rd_at[j] = m * 4 + ((2 * j + b) ^ ((m >> 2) & 3));  // pair j of the group, block b
+  uint4 raw[2][2];  // [pair][x, w] of the stage at hand
+  auto take = [&](uint32_t st) __attribute__((always_inline)) {
+    const uint4* buf = &s_stage[wv][st % kRouterRing][0][0];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int o = 0; o < 2; ++o) raw[j][o] = buf[o * 128 + rd_at[j]];
+  };
+#pragma unroll
+  for (int u = 0; u < kRouterRing; ++u) request();
+  wait_loads<4 * (kRouterRing - 1)>();
+  take(0);
+
+  float lev1[16], lev2[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) lev1[r] = lev2[r] = 0.0f;
+  uint32_t st = 0;
+#pragma unroll 1
+  for (uint32_t pg = 0; pg < kGroups; ++pg) {
+    f32x32_t acc[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 32; ++r) acc[j][r] = 0.0f;
+#pragma unroll 1
+    for (uint32_t i = 0; i < n_i; ++i, ++st) {
+      // All operands of the stage in registers of their own before its first matrix instruction: a vector instruction that writes a
+      // register an MFMA in flight still reads as A or B waits until that MFMA is done (64 cycles here), so operands made one at a
+      // time in a recycled register pair cost 89 instead of 65 cycles per instruction.
+      float op[2][2][8];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+          const uint32_t v[4] = {raw[j][o].x, raw[j][o].y, raw[j][o].z, raw[j][o].w};
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            op[j][o][2 * u] = bf16_lo(v[u]);
+            op[j][o][2 * u + 1] = bf16_hi(v[u]);
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(op[j][o][u]));
+        }
+      request();  // into the stage just taken up
+      wait_loads<4 * (kRouterRing - 1)>();
+      take(st + 1);
+      __builtin_amdgcn_sched_barrier(0);  // (left to itself the compiler reads them behind most of the matrix instructions)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc[j] = __builtin_amdgcn_mfma_f32_32x32x1f32(op[j][0][u], op[j][1][u], acc[j], 0, 0, 0);
+    }
+    // two pairs of chains are complete: the stride-1 level, the pairs' sum, then the binary counter
+    float carry[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) carry[r] = (acc[0][r] + acc[0][16 + r]) + (acc[1][r] + acc[1][16 + r]);
+    if (pg == 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lev1[r] = carry[r];
+    } else if (pg == 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lev2[r] = lev1[r] + carry[r];
+    } else if (pg == 2) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lev1[r] = carry[r];
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lev1[r] = lev2[r] + (lev1[r] + carry[r]);
+    }
+  }
+  // the last levels of the tree, over the ring: neighbouring waves first
+  wait_loads<0>();
+  __syncthreads();
+  float* s_part = reinterpret_cast<float*>(&s_stage[0][0][0][0]);  // [wave][16][64]
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s_part[(wv * 16 + r) * 64 + lane] = lev1[r];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t q = 0; q < 4; ++q) {  // a wave stores a quarter: tokens 8 wv + 4b + q
+    const uint32_t r = 4 * wv + q, t = t0 + 8 * wv + 4 * b + q;
+    const float* v = s_part + r * 64 + lane;
+    const float sum = (v[0] + v[1024]) + (v[2048] + v[3072]);
+    if (t < T) logits[static_cast<size_t>(t) * ld + e0 + m] = sum;
   }
 }
 
@@ -1138,10 +1190,10 @@ hipError_t launch_prefill_router(hipStream_t s, const uint16_t* W, const uint16_
     }
     if (tail_ok) prep_rows = ((T + 3) / 4 + (T + 31) / 32 - 1) / ((T + 31) / 32);
     const dim3 grid((T + 31) / 32, e32 / 32 + prep_rows);
+    // (rows of 1024 and 2048 unrolled, all others as a loop: the times of both stand at the kernels)
     if (D == 1024) prefill_router_mfma_kernel<2><<<grid, dim3(256), 0, s>>>(W, x, e32, D, T, x_stride, logits, E, mt);
     else if (D == 2048) prefill_router_mfma_kernel<4><<<grid, dim3(256), 0, s>>>(W, x, e32, D, T, x_stride, logits, E, mt);
-    else if (D == 4096) prefill_router_mfma_kernel<8><<<grid, dim3(256), 0, s>>>(W, x, e32, D, T, x_stride, logits, E, mt);
-    else prefill_router_mfma_kernel<0><<<grid, dim3(256), 0, s>>>(W, x, e32, D, T, x_stride, logits, E, mt);
+    else prefill_router_loop_kernel<<<grid, dim3(256), 0, s>>>(W, x, e32, D, T, x_stride, logits, E, mt);
     if (e32 == E) return hipGetLastError();
   }
   const uint32_t rest = E - e32;

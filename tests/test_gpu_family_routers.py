@@ -82,8 +82,8 @@ def test_sqrtsoftplus_router_bit_exact(gpu, oracle, e, d, k, t):
 @pytest.mark.parametrize("seed", range(14))
 def test_router_logits_sweep(gpu, oracle, seed):
     """drawn (experts, width, tokens) across the batched router's kernels: the register-tiled one (up to 256
-    tokens, widths that are no multiple of 512), the matrix-core walk as a loop (1536, 2560, 3072) and unrolled
-    (1024, 2048, 4096), expert counts that leave rows over after the blocks of 32 (100, 258) -- logits bit for
+    tokens, widths that are no multiple of 512), the matrix-core walk as a loop (512, 1536, 2560, 3072, 4096) and unrolled
+    (1024, 2048), expert counts that leave rows over after the blocks of 32 (100, 258) -- logits bit for
     bit against the one-row order of the oracle on sampled tokens, and the selection on top of them"""
     rng0 = np.random.default_rng(0x60A7 + seed)
     e = int(rng0.choice([32, 64, 100, 128, 256, 258, 512]))
@@ -107,6 +107,23 @@ def test_router_logits_sweep(gpu, oracle, seed):
         ri, rw = oracle.router_sqrtsoftplus(ref_lg, bias, k, 1.5)
         assert np.array_equal(idx_h[i], ri), (what, i)
         assert np.array_equal(_bits(w_h[i]), _bits(rw)), (what, i)
+
+
+@pytest.mark.parametrize("e,d,t", [(32, 512, 193), (64, 512, 225), (32, 4608, 194), (32, 7680, 17)])
+def test_router_logits_of_few_and_many_runs(gpu, oracle, e, d, t):
+    """the matrix-core walk as a loop at one run of 512 (every request past the end goes round the ring) and at 9 and 15 runs,
+    with token tiles of 1, 1, 2 and 17 rows: each token's logits as its own one-row call gives them"""
+    _, wr, x = _draw(oracle, f"runs-{e}-{d}-{t}", e, d, t, 0.05)
+    fam, w_d, x_d = ops.FamilyRouters(gpu), ops.bf16_tensor(wr), ops.bf16_tensor(x)
+    def logits(rows):
+        n = rows.shape[0]
+        lg = torch.zeros((n, e), dtype=torch.float32, device="cuda")
+        fam.encode_router_top_k(w_d, rows, torch.zeros(e, device="cuda"), torch.zeros((n, 4), dtype=torch.int32, device="cuda"),
+                                torch.zeros((n, 4), device="cuda"), e, d, 1.0, lg, top_k=4, t=n)
+        return lg
+    got = logits(x_d)
+    want = torch.cat([logits(x_d[i:i + 8].contiguous()) for i in range(0, t, 8)])
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
 
 
 @pytest.mark.parametrize("e", [8, 16, 24, 33, 100, 128, 168, 255, 256])
