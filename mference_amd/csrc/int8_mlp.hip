@@ -137,7 +137,9 @@ __global__ __launch_bounds__(256) void rows_q8_kernel(const Q8Args a) {
 // loads nor overlaps vector and matrix instructions (2816 x 2112, 300 tokens, waves of two token blocks: gate/up 47.6 -> 37.9 us).
 // The MLP, us, waves of two token blocks with results stored by their lanes / now: 2816 x 2112, 16 rows 49.8 / 43.1, 300 53.8 / 47.1, 600
 // 84.3 / 75.1, 2048 220.7 / 199.8; 704 x 8192, 16 rows 63.2 / 59.8, 300 87.3 / 81.5, 2048 240 / 220; 2048 x 2048, 16 rows 39.2 / 34.6, 1024
-// 70.3 / 64.1; 192 x 128, 64 rows 12.3 / 10.6.
+// 70.3 / 64.1; 192 x 128, 64 rows 12.3 / 10.6.  Nothing looks at a register where it is requested (the zeros for what lies past the row
+// were put in there, and every stage waited for its own request, tables for all of them): 2816 x 2112, 16 rows 43.1 / 38.3, 300 47.1 / 43.5,
+// 2048 199.8 / 179.9; 704 x 8192, 16 rows 59.8 / 51.0, 2048 220 / 192; 2048 x 2048, 16 rows 34.6 / 30.5.
 // (128 tokens per workgroup, two accumulators a wave to one set of codes, lost at every size: 2816 x 2112, 2048 tokens 302
 // against 224 us, 16384 tokens 1895 against 1492; 704 x 8192, 1500 tokens 227 against 195.)
 
@@ -171,14 +173,10 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   u32x4_t xr[2][4], wreg[2][NPROJ][2];                  // stage st waits in set st & 1 (counted from st0)
   const uint32_t row = min(r0 + rb * 32 + m, a.M - 1);  // the lane's weight row (past the end: the last one, not stored)
   auto fetch = [&](uint32_t st, u32x4_t (&xs)[4], u32x4_t (&ws)[NPROJ][2]) __attribute__((always_inline)) {
-    const uint32_t g = 2 * st + (xq >> 1);
-    const bool in = g < ng && st < st1;  // half a stage behind an odd number of groups, stages past this set's last: zeros
-    const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt, a.T - 1)) * a.N + (in ? g : ng - 1) * kGroup + (xq & 1) * 32;
+    const uint32_t g = min(2 * st + (xq >> 1), ng - 1);  // (past the row: its last group, which `put` makes zeros of)
+    const uint16_t* src = a.x + static_cast<size_t>(min(t0 + xt, a.T - 1)) * a.N + g * kGroup + (xq & 1) * 32;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      xs[i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
-      if (!in) xs[i] = u32x4_t{0, 0, 0, 0};
-    }
+    for (int i = 0; i < 4; ++i) xs[i] = *reinterpret_cast<const u32x4_t*>(src + 8 * i);
     const uint32_t k0 = min(st * 128 + wc * 16, a.N - 16);  // (codes past the row, or of a stage past the last, meet x = 0)
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
@@ -190,28 +188,34 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   // scales and biases of the wave's projection
   const uint16_t* tab_s = a.S[NPROJ == 2 ? z : 0];
   const uint16_t* tab_b = a.B[NPROJ == 2 ? z : 0];
-  // those of the eight groups from g (a group of the row) on; groups past the row's last one are zeros
+  // Those of the eight groups from g (a group of the row) on.  A load past the row's last group reads on into the next row, the table's
+  // last loads end with the table; what is not the row's is taken off, and groups past its last one become zeros, when the four stages
+  // that use them begin.
   struct Tab { uint4 S, B; };
   auto fetch_tab = [&](uint32_t g) __attribute__((always_inline)) {
-    Tab t;
-    // (a load past the row's last group reads on into the next row, the table's last loads end with the table: what is not the row's is taken off)
-    const uint32_t at = row * ng + g, base = min(at, a.M * ng - 8);
-    t.S = drop_bf16(load_16_bytes(tab_s + base), at - base);
-    t.B = drop_bf16(load_16_bytes(tab_b + base), at - base);
+    const uint32_t base = min(row * ng + g, a.M * ng - 8);
+    return Tab{load_16_bytes(tab_s + base), load_16_bytes(tab_b + base)};
+  };
+  auto settle_tab = [&](const Tab& t, uint32_t g) __attribute__((always_inline)) {
+    const uint32_t at = row * ng + g, skip = at - min(at, a.M * ng - 8);
+    uint4 S = drop_bf16(t.S, skip), B = drop_bf16(t.B, skip);
     if (g + 8 > ng) {
       uint32_t keep[4];
 #pragma unroll
       for (uint32_t i = 0; i < 4; ++i) keep[i] = g + 2 * i + 1 < ng ? 0xFFFFFFFFu : g + 2 * i < ng ? 0xFFFFu : 0u;
-      t.S = make_uint4(t.S.x & keep[0], t.S.y & keep[1], t.S.z & keep[2], t.S.w & keep[3]);
-      t.B = make_uint4(t.B.x & keep[0], t.B.y & keep[1], t.B.z & keep[2], t.B.w & keep[3]);
+      S = make_uint4(S.x & keep[0], S.y & keep[1], S.z & keep[2], S.w & keep[3]);
+      B = make_uint4(B.x & keep[0], B.y & keep[1], B.z & keep[2], B.w & keep[3]);
     }
-    return t;
+    return Tab{S, B};
   };
-  auto put = [&](uint32_t buf, const u32x4_t (&xs)[4], const u32x4_t (&ws)[NPROJ][2]) __attribute__((always_inline)) {
+  // stage st into a buffer.  Half a stage behind an odd number of groups and a stage past this set's last are zeros, and become so here:
+  // a look at the registers where they are requested would wait for them.
+  auto put = [&](uint32_t buf, uint32_t st, const u32x4_t (&xs)[4], const u32x4_t (&ws)[NPROJ][2]) __attribute__((always_inline)) {
+    const bool in = 2 * st + (xq >> 1) < ng && st < st1;
     float part = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const u32x4_t v = xs[i];
+      const u32x4_t v = in ? xs[i] : u32x4_t{0, 0, 0, 0};
       reinterpret_cast<u32x4_t*>(s_x[buf])[xt * 16 + ((4 * xq + i) ^ (xt & 15u))] = v;
       part += ((bf16_lo(v.x) + bf16_hi(v.x)) + (bf16_lo(v.y) + bf16_hi(v.y))) +
               ((bf16_lo(v.z) + bf16_hi(v.z)) + (bf16_lo(v.w) + bf16_hi(v.w)));
@@ -288,18 +292,19 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     // (no branch around a request: a wait for one stage's registers would cover the later stages' as well)
     fetch(st0, xr[0], wreg[0]);
     Tab next = fetch_tab(min(2 * st0, ng - 1));
+    issue_fence();  // (in front of the stages' loads: the wait for the first table is not one for those)
     fetch(st0 + 1, xr[1], wreg[1]);
-    put(0, xr[0], wreg[0]);
+    put(0, st0, xr[0], wreg[0]);
     fetch(st0 + 2, xr[0], wreg[0]);
     for (uint32_t i0 = 0; i0 < n_walk; i0 += 4) {
-      const Tab tab = next;
+      const Tab tab = settle_tab(next, min(2 * (st0 + i0), ng - 1));
       next = fetch_tab(min(2 * (st0 + i0 + 4), ng - 1));
 #pragma unroll
       for (int u4 = 0; u4 < 4; ++u4) {  // stage i0 + u4, in buffer u4 & 1
         if (i0 + u4 >= n_walk) break;
         __syncthreads();  // its buffer is complete, the other one is no longer read
         const int buf = u4 & 1, other = buf ^ 1;
-        if (i0 + u4 + 1 < n_walk) put(other, xr[other], wreg[other]);
+        if (i0 + u4 + 1 < n_walk) put(other, st0 + i0 + u4 + 1, xr[other], wreg[other]);
         fetch(st0 + i0 + u4 + 3, xr[other], wreg[other]);
         const uint32_t s4[4] = {tab.S.x, tab.S.y, tab.S.z, tab.S.w}, b4[4] = {tab.B.x, tab.B.y, tab.B.z, tab.B.w};
         multiply(buf, [&](uint32_t g) { return g ? bf16_hi(s4[u4]) : bf16_lo(s4[u4]); }, h ? b4[u4] >> 16 : b4[u4] & 0xFFFFu);
@@ -316,7 +321,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     if (st0 < st1) {
       fetch(st0, xr[0], wreg[0]);
       fetch_entries(st0);
-      put(0, xr[0], wreg[0]);
+      put(0, st0, xr[0], wreg[0]);
       if (st0 + 1 < st1) fetch(st0 + 1, xr[0], wreg[0]);
     }
 #pragma unroll 1
@@ -325,7 +330,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
       if (st0 + i >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
       const uint16_t sv[2] = {sc[0], sc[1]}, bv = bi;
       if (st0 + i + 1 < st1) {
-        put((i + 1) & 1u, xr[0], wreg[0]);
+        put((i + 1) & 1u, st0 + i + 1, xr[0], wreg[0]);
         fetch_entries(st0 + i + 1);
         if (st0 + i + 2 < st1) fetch(st0 + i + 2, xr[0], wreg[0]);
       }
