@@ -708,6 +708,9 @@ __host__ __device__ __forceinline__ size_t group_one_lds_bytes(uint32_t t, uint3
   return (bits > serial ? bits : serial) + 16;
 }
 
+// Workgroups behind the first prepare x, a row per wave (the layer call with a router of its own has that done beside the router): one
+// workgroup groups for 8 to 12 us while the chip is idle otherwise.  Given routing, us: 777 tokens of 4096 with the scalar gate, grouping
+// 11.5 and a launch of 9.0 behind it -> 11.8; 300 tokens of 2816, 8.1 and 4.8 -> 8.3.
 __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restrict__ idx,
                                                          const float* __restrict__ w, uint32_t n_pairs,
                                                          uint32_t K, uint32_t E, uint32_t tpe_log2,
@@ -715,10 +718,16 @@ __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restr
                                                          uint32_t* __restrict__ offsets,
                                                          uint32_t* __restrict__ starts,
                                                          mf_pair* __restrict__ sorted, const TileLists tiles,
-                                                         uint32_t* __restrict__ status) {
+                                                         uint32_t* __restrict__ status, const uint16_t* __restrict__ x,
+                                                         uint32_t D, const RouterTail prep) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ uint32_t s_cnt[MF_MAX_EXPERTS], s_row[MF_MAX_EXPERTS];
   const uint32_t T = n_pairs / K, W = group_one_row_words(T);
+  if (blockIdx.x) {
+    const uint32_t r = (blockIdx.x - 1) * 16 + (threadIdx.x >> 6);
+    if (r < T) prep_x_row(x + static_cast<size_t>(r) * D, prep.xp, prep.sums, prep.row_max, prep.w_sg, prep.gate, r, D, threadIdx.x & 63);
+    return;
+  }
   uint32_t* bm = reinterpret_cast<uint32_t*>(smem);                 // [E][W] bits: token t of row e
   uint16_t* pref = reinterpret_cast<uint16_t*>(smem + static_cast<size_t>(E) * W * 4);  // [E][W] set bits before word
   // a thread's routes (at most kGroupOnePairs / 1024 = 8) stay in registers from the marking pass to the
@@ -1229,10 +1238,11 @@ hipError_t launch_prefill_router(hipStream_t s, const uint16_t* W, const uint16_
   return launch_prefill_router(s, W, x, E, D, T, x_stride, logits, nullptr);
 }
 
+// `prep` (optional): the x preparation of rows of d values, for the grouping launch to take along; its xp is null on return when it did
 hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint32_t t, uint32_t K,
                         uint32_t E, uint32_t* counts, uint32_t* offsets, uint32_t* starts,
                         mf_pair* sorted, const TileLists& tiles,
-                        uint32_t* status, uint32_t* chunk_hist) {
+                        uint32_t* status, uint32_t* chunk_hist, const uint16_t* x, uint32_t d, RouterTail* prep) {
   const uint32_t n_pairs = t * K;
   if (n_pairs && n_pairs <= kGroupOnePairs && group_one_lds_bytes(t, E) <= kGroupOneMaxBytes) {
     const size_t lds = group_one_lds_bytes(t, E);
@@ -1240,8 +1250,10 @@ hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint
     while (tpe_log2 < 4 && (E << (tpe_log2 + 1)) <= 1024) ++tpe_log2;
     const hipError_t e = allow_lds<group_one_kernel>(lds, static_cast<int>(kGroupOneMaxBytes));
     if (e != hipSuccess) return e;
-    group_one_kernel<<<dim3(1), dim3(1024), lds, s>>>(idx, w, n_pairs, K, E, tpe_log2, counts, offsets, starts, sorted,
-                                                      tiles, status);
+    const bool take = prep && prep->xp;
+    group_one_kernel<<<dim3(take ? 1 + (t + 15) / 16 : 1), dim3(1024), lds, s>>>(idx, w, n_pairs, K, E, tpe_log2, counts, offsets, starts,
+                                                                                sorted, tiles, status, x, d, take ? *prep : RouterTail{});
+    if (take) prep->xp = nullptr;
     return hipGetLastError();
   }
   if (n_pairs == 0) {  // no routes: the scan over no chunks writes empty experts and a clean status word
@@ -1262,6 +1274,13 @@ hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint
   group_emit_kernel<<<dim3(n_chunks), dim3(256), 0, s>>>(idx, w, n_pairs, K, E, chunk_pairs, chunk_hist, starts,
                                                          sorted);
   return hipGetLastError();
+}
+
+hipError_t launch_group(hipStream_t s, const uint32_t* idx, const float* w, uint32_t t, uint32_t K,
+                        uint32_t E, uint32_t* counts, uint32_t* offsets, uint32_t* starts,
+                        mf_pair* sorted, const TileLists& tiles,
+                        uint32_t* status, uint32_t* chunk_hist) {
+  return launch_group(s, idx, w, t, K, E, counts, offsets, starts, sorted, tiles, status, chunk_hist, nullptr, 0, nullptr);
 }
 
 // words of the handle's grouping scratch: 2048 of small tables, the per-chunk counts and flags of the
@@ -1797,6 +1816,12 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   TileLists lists{{ws.tiles[0], tile.down != tile.up ? ws.tiles[1] : nullptr},
                   {prefill_tile_slots(c, t, tile.up), prefill_tile_slots(c, t, tile.down)}, {tile.up, tile.down}};
   bool x_prepared = false, fused_group = false;
+  RouterTail tail{};  // what the router launch, or else the grouping launch, prepares on the side
+  tail.xp = ws.xp;
+  tail.w_sg = c.shared_f && !w.w_sg_q8.weights ? w.w_sg : nullptr;  // (an 8-bit gate row: its own launch below)
+  tail.sums = ws.sum_x;
+  tail.row_max = ws.row_max;
+  tail.gate = ws.gate;
   if (ragged) {
     // the caller's grouping: its per-expert counts are a one-chunk histogram for the scan that lays
     // out the tile list (the runs start at 0 in expert order, as mf_moe_group writes them)
@@ -1815,14 +1840,9 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
     ws.partials = ragged->partials;
   } else {
     if (w.router_w) {  // else the routing in out_idx / out_w is the caller's
-      RouterTail tail{};
-      tail.xp = ws.xp;
-      tail.w_sg = c.shared_f && !w.w_sg_q8.weights ? w.w_sg : nullptr;  // (an 8-bit gate row: its own launch below)
-      tail.sums = ws.sum_x;
-      tail.row_max = ws.row_max;
-      tail.gate = ws.gate;
-      MF_TRY(launch_prefill_router(s, w.router_w, x, c.num_experts, c.d, t, c.d, ws.logits, &tail));
-      x_prepared = tail.xp != nullptr;
+      RouterTail routed = tail;
+      MF_TRY(launch_prefill_router(s, w.router_w, x, c.num_experts, c.d, t, c.d, ws.logits, &routed));
+      x_prepared = routed.xp != nullptr;
       fused_group = topk_group_takes(t) && pairs > kGroupOnePairs;
       if (fused_group)
         MF_TRY(launch_topk_group(s, ws.logits, t, c.top_k, c.num_experts, c.router_mode, ws.idx, ws.w, ws.counts,
@@ -1830,15 +1850,18 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
                                  h.ws.group_tmp));
       else MF_TRY(launch_topk(s, ws.logits, c.num_experts, c.top_k, t, c.router_mode, ws.idx, ws.w));
     }
-    if (!fused_group)
+    if (!fused_group) {
+      RouterTail grouped = tail;
       MF_TRY(launch_group(s, ws.idx, ws.w, t, c.top_k, c.num_experts, ws.counts, ws.offsets, ws.starts,
-                          ws.sorted, lists, ws.status, h.ws.group_tmp + 2048));
+                          ws.sorted, lists, ws.status, h.ws.group_tmp + 2048, x, c.d, x_prepared ? nullptr : &grouped));
+      x_prepared |= !x_prepared && !grouped.xp;
+    }
   }
 
   const bool gate_q8 = c.shared_f && w.w_sg_q8.weights;
   const bool want_gate = c.shared_f && (w.w_sg || gate_q8);
   if (x_prepared) {
-    // the router launch has prepared x (and the gate's logits) on the side
+    // done on the side (the gate's logits, too)
   } else if (want_gate && !gate_q8) {  // one pass over x: matmul order, group sums and the shared gate's logits
     prep_x_gate_kernel<<<dim3((t + 3) / 4), dim3(256), 0, s>>>(x, ws.xp, ws.sum_x, ws.row_max, w.w_sg, ws.gate, t, c.d);
     MF_TRY(hipGetLastError());
