@@ -209,10 +209,9 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
     const uint16_t* table = (what ? Bp[p] : Sp[p]) + static_cast<size_t>(row_base[p]) * ng_ld + g_off;
     const uint32_t gl = g0 + 8 * h;
     const uint32_t gc = gl < ng ? gl : 0;  // a lane without groups reads group 0 and drops it
-    // (whole 16-byte loads at any group and alignment; in the last step they end at the row's end and are moved down)
-    const uint32_t gb = NG8 ? gc : min(gc, ng - 8);
-    const uint4 v = load_16_bytes(table + (m * ng_ld + gb));
-    return !NG8 && g0 + kTabStep > ng ? drop_bf16(v, gc - gb) : v;
+    // (whole 16-byte loads at any group and alignment; in the last step they end at the row's end and tab_step moves them down: done
+    // here, it would wait for them and for every request in front of them)
+    return load_16_bytes(table + (m * ng_ld + (NG8 ? gc : min(gc, ng - 8))));
   };
   uint4 tab[2][NPROJ];  // of the next step
 #pragma unroll
@@ -292,7 +291,12 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
     uint4 ab[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p) {
-      const uint4 S = tab[0][p], B = tab[1][p];
+      uint4 S = tab[0][p], B = tab[1][p];
+      if (!NG8 && ng >= 8 && g0 + kTabStep > ng) {
+        const uint32_t gc = have ? g0 + 8 * h : 0, skip = gc - min(gc, ng - 8);
+        S = drop_bf16(S, skip);
+        B = drop_bf16(B, skip);
+      }
       float* to = s_scale + p * (kTabStep * 32) + 8 * h * 32 + m;
       const uint32_t w[4] = {S.x, S.y, S.z, S.w};
 #pragma unroll

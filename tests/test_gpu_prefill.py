@@ -443,6 +443,25 @@ def test_prefill_rows_wider_than_4096(gpu, oracle, d, e, t):
     assert_layer_close(oracle.bf16_to_float(y[rows]), oracle.bf16_to_float(ref_y), f"prefill d={d} e={e} t={t}")
 
 
+@pytest.mark.parametrize("d,fs", [(192, 0), (640, 128)])
+@pytest.mark.parametrize("t", [17, 32, 33, 2049])
+def test_given_routing_has_the_bits_of_the_layers_own(gpu, oracle, d, fs, t):
+    """With the routing given, x is prepared by workgroups of 16 rows beside the grouping (beyond 8192 routes by a launch of its
+    own); without, beside the router: the same result, rows at another power of two among them."""
+    f, e, k = 128, 32, 4
+    layer = oracle.synth_layer(ROOT_SEED + 0xB700 + d, d, f, e, k, bits=4, fs=fs)
+    x = oracle.synth_x(ROOT_SEED + t, t, d)
+    x[t - 1] = oracle.bf16_bits(oracle.bf16_to_float(x[t - 1]) * np.float32(2.0 ** 50))
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    y, idx, w = _run_prefill(moe, wts, x, t, d, k)
+    given = ops.MoELayerWeights(None, wts.experts, wts.offsets, wts.shared, wts.w_sg)
+    out = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+    moe.encode_prefill_layer(given, ops.bf16_tensor(x), out, t, out_indices=torch.from_numpy(idx.astype(np.int32)).cuda(),
+                             out_weights=torch.from_numpy(w).cuda())
+    torch.cuda.synchronize()
+    assert np.array_equal(ops.bf16_bits(out), y)
+
+
 @pytest.mark.parametrize("workload,t", [("dsv4-2bit", 300), ("maple-ternary", 300)])
 def test_prefill_other_formats_full_size(gpu, oracle, workload, t):
     """the large 2-bit layer (D 4096, F 2048, E 256, K 6, 4-bit shared 2048) and the ternary layer
