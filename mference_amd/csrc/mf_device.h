@@ -243,6 +243,17 @@ __device__ __forceinline__ void issue_fence() { asm volatile("" ::: "memory"); }
 // every store this wave has issued is acknowledged at its scope
 __device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// An array kept in registers: every index is a literal once the loops are unrolled.  A call of index_past_the_end that is left then is an
+// error of the build, so a loop that runs past the array does not compile (clang has no warning for it).
+__device__ void index_past_the_end() __attribute__((error("index past the end of a register array")));
+template <typename T, int N> struct RegArray {
+  T v[N];
+  __device__ __forceinline__ T& operator[](int i) {
+    if (i >= N) index_past_the_end();
+    return v[i];
+  }
+};
+
 // LDS[lds + 16 * lane ...] = the 16 bytes at p of every lane (lds: a byte address, uniform), without a register in between.  The
 // compiler does not know of the request: wait_loads and a barrier stand in front of the first read.
 __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {

@@ -195,7 +195,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
   // pairs of groups in flight: one for 4-bit codes on tiles of 32, whose registers do not hold a second (with it, 31 values went
   // through scratch memory: 2816 x 704, 300 tokens, gate / up 60 -> 100 us; 93 tokens of the Qwen shape 31 -> 37)
   constexpr int kRing = NT == 1 && BITS == 4 ? 1 : 2;
-  Codes cur[NPROJ][kRing];
+  RegArray<Codes, kRing> cur[NPROJ];
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p) {
     wbase[p] = Wp[p] + row_base[p] * row_bytes + static_cast<size_t>(g_off) * gstride;
@@ -673,11 +673,11 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, const QmmPlace& 
   const uint16_t* brow = Bp + static_cast<size_t>(row0) * NG;
 
   // ---- everything issued back to back: codes of the first slice, its scale / bias words, the x tile
-  Codes cur[2][kRing];
+  RegArray<Codes, kRing> cur[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < kRing; ++u)
 #pragma unroll
       for (int i = 0; i < 2; ++i) cur[p][u].load(i, wrow + p * 32 * kRowBytes + u * pair_stride + (i ? second : 0));
   uint4 nS[2], nB[2];

@@ -257,3 +257,32 @@ def test_a_workspace_for_many_rows_serves_every_smaller_block(n, k):
         for m in range(1, min(most, 700) + 1):
             assert lib.mf_qmm_path(w, 4, 4096, 4096, m, n, k, 4096, have) == 1, (most, m)
         assert lib.mf_qmm_path(w, 4, 4096, 4096, most, n, k, 4096, 256) == 2
+
+
+def test_a_loop_past_a_register_array_does_not_build(tmp_path):
+    """RegArray (mf_device.h), which holds the matmuls' codes in flight: a loop over its elements compiles, one step more is an
+    error of the build"""
+    import subprocess
+    from mference_amd import build
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("needs hipcc")
+    src = tmp_path / "regs.hip"
+    src.write_text("""#include "mf_device.h"
+__global__ void probe(const float* x, float* y) {
+  mf::RegArray<float, SIZE> r;
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) r[i] = x[threadIdx.x + 64 * i];
+  float sum = 0.0f;
+#pragma unroll
+  for (int i = 0; i < SIZE; ++i) sum += r[i];
+  y[threadIdx.x] = sum;
+}
+""")
+    def compiles(n, to):
+        cmd = [hipcc, *build.FLAGS, f"-DSIZE={n}", f"-DSTEPS={to}", "-I", build.CSRC, "-c", "-o", str(tmp_path / "regs.o"), str(src)]
+        return subprocess.run(cmd, capture_output=True, text=True)
+    for n in (1, 2):
+        ok, past = compiles(n, n), compiles(n, n + 1)
+        assert ok.returncode == 0, ok.stderr
+        assert past.returncode != 0 and "index past the end of a register array" in past.stderr
