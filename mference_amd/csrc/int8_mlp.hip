@@ -197,7 +197,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     return Tab{load_16_bytes(tab_s + base), load_16_bytes(tab_b + base)};
   };
   auto settle_tab = [&](const Tab& t, uint32_t g) __attribute__((always_inline)) {
-    const uint32_t at = row * ng + g, skip = at - min(at, a.M * ng - 8);
+    const uint32_t at = row * ng + min(g, ng - 1), skip = at - min(at, a.M * ng - 8);
     uint4 S = drop_bf16(t.S, skip), B = drop_bf16(t.B, skip);
     if (g + 8 > ng) {
       uint32_t keep[4];
@@ -241,15 +241,18 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
   auto multiply = [&](uint32_t buf, auto scale, uint32_t bias) __attribute__((always_inline)) {
     // biases: K slots of half h = (hi, mid, lo) of sum(x) over the stage's group h (a group past the end sums to 0).  With one projection a
     // wave takes its own group's alone: q x and the bias term mostly cancel, so they belong into one sum (both groups' biases in one of
-    // the two waves' sums: error against 64 bits 1.6e-7 -> 2.5e-7 at 2112 x 2816).
+    // the two waves' sums: error against 64 bits 1.6e-7 -> 2.5e-7 at 2112 x 2816).  An infinite bias meets hi alone: mid, lo and what a
+    // wave leaves to the other are zeros, and 0 times it would be NaN.
+    const bool own = NPROJ == 2 || h == z;
+    const uint32_t b_hi = own ? bias : 0u, b_rest = (b_hi & 0x7F80u) == 0x7F80u ? 0u : b_hi;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const float v = NPROJ == 2 || h == z ? s_sum[buf][tok_of[j]][h] : 0.0f;
+      const float v = own ? s_sum[buf][tok_of[j]][h] : 0.0f;
       const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
       const float r1 = __builtin_isinf(v) ? 0.0f : v - __uint_as_float(hi);  // (an infinite sum has no rest: inf - inf would be NaN)
       const uint32_t mid = __float_as_uint(r1) & 0xFFFF0000u;
       const uint32_t lo = __float_as_uint(r1 - __uint_as_float(mid));
-      acc[j] = mfma_bf16(make_uint4((hi >> 16) | mid, lo >> 16, 0, 0), make_uint4(bias | (bias << 16), bias, 0, 0), acc[j]);
+      acc[j] = mfma_bf16(make_uint4((hi >> 16) | mid, lo >> 16, 0, 0), make_uint4(b_hi | (b_rest << 16), b_rest, 0, 0), acc[j]);
     }
 #pragma unroll
     for (int gi = 0; gi < NPROJ; ++gi) {
@@ -297,7 +300,7 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     put(0, st0, xr[0], wreg[0]);
     fetch(st0 + 2, xr[0], wreg[0]);
     for (uint32_t i0 = 0; i0 < n_walk; i0 += 4) {
-      const Tab tab = settle_tab(next, min(2 * (st0 + i0), ng - 1));
+      const Tab tab = settle_tab(next, 2 * (st0 + i0));
       next = fetch_tab(min(2 * (st0 + i0 + 4), ng - 1));
 #pragma unroll
       for (int u4 = 0; u4 < 4; ++u4) {  // stage i0 + u4, in buffer u4 & 1
@@ -328,7 +331,9 @@ void qmm8_kernel(const Q8Args a, uint32_t n_tiles, uint32_t n_work) {
     for (uint32_t i = 0; i < n_walk; ++i) {
       __syncthreads();
       if (st0 + i >= st1) continue;  // (the second set may have a stage less: it keeps the barriers company)
-      const uint16_t sv[2] = {sc[0], sc[1]}, bv = bi;
+      // (half a stage behind an odd number of groups: zeros, like its x; the entry that came is the last group's)
+      const bool whole = 2 * (st0 + i) + 1 < ng;
+      const uint16_t sv[2] = {sc[0], whole ? sc[1] : uint16_t{0}}, bv = whole || h == 0 ? bi : uint16_t{0};
       if (st0 + i + 1 < st1) {
         put((i + 1) & 1u, st0 + i + 1, xr[0], wreg[0]);
         fetch_entries(st0 + i + 1);

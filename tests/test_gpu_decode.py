@@ -1310,6 +1310,42 @@ def test_int8_matmul_passes_infinities_on(gpu, d, f, t):
     assert torch.equal(torch.sign(got[1].float()), torch.sign(want[1].float()))
 
 
+@pytest.mark.parametrize("d,f,t", [(192, 128, 16), (128, 192, 70), (704, 320, 70), (192, 1088, 16), (64, 4096, 70), (4096, 192, 300), (4096, 1088, 300)])
+def test_int8_matmul_of_infinite_table_entries(gpu, d, f, t):
+    """an infinite bias or scale in the first, a middle and the last group of some weight rows, everything else above zero: those results
+    are infinite (0 times an infinity does not enter a row's sum), as in the row kernels, and the other rows keep their bits.  Short and long
+    walks, by one set of waves and halved among two, with whole and half last stages"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + f + t)
+    def q(rows, n):
+        table = lambda: (0.01 + 0.01 * torch.rand(rows, n // 64, generator=gen, device="cuda")).to(torch.bfloat16)
+        return ops.QuantizedTensor(torch.randint(1, 256, (rows, n), dtype=torch.uint8, generator=gen, device="cuda"), table(), table(), 8, rows, n)
+    qs = [q(f, d), q(f, d), q(d, f)]
+    # (x of the size of 1 / d: activations of the order of one; sums of 64 equal numbers are one bf16 number, others have three parts)
+    x = ((0.5 + torch.rand(t, d, generator=gen, device="cuda")) / d).to(torch.bfloat16)
+    x[3] = 2.0 ** -8
+    op = ops.SharedExpertInt8(gpu)
+
+    def run(tensors, step):
+        y, act = (torch.zeros((t, n), dtype=torch.bfloat16, device="cuda") for n in (d, f))
+        for t0 in range(0, t, step):
+            op.encode(x[t0:t0 + step], *tensors, y[t0:t0 + step], act[t0:t0 + step], t=min(step, t - t0))
+        return y
+
+    finite = run(qs, t)
+    assert torch.isfinite(finite).all()
+    groups = sorted({0, f // 128, f // 64 - 1})
+    for name in ("biases", "scales"):
+        down = ops.QuantizedTensor(qs[2].packed, qs[2].scales.clone(), qs[2].biases.clone(), 8, d, f)
+        at = [7 + 11 * i for i in range(len(groups))]
+        for r, g in zip(at, groups):
+            getattr(down, name)[r, g] = float("inf")
+        got, rows = run([*qs[:2], down], t), run([*qs[:2], down], 8)
+        others = [r for r in range(d) if r not in at]
+        assert torch.equal(got[:, others].view(torch.int16), finite[:, others].view(torch.int16)), name
+        assert (rows[:, at] == float("inf")).all() and (got[:, at] == float("inf")).all(), (name, at, got[:4, at])
+
+
 @pytest.mark.parametrize("bits,m,n,t", [(4, 1024, 5120, 3), (4, 12800, 3136, 8), (2, 9408, 2560, 4), (2, 1216, 6592, 7)])
 def test_quad_rows_kernel_keeps_infinities_to_their_row(gpu, bits, m, n, t):
     """an infinity or a NaN makes its own token's results NaN (as in every row kernel of these formats) and leaves the
