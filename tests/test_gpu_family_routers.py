@@ -126,6 +126,24 @@ def test_router_logits_of_few_and_many_runs(gpu, oracle, e, d, t):
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
 
 
+@pytest.mark.parametrize("e,d,t,off", [(2, 64, 256, 1), (2, 64, 257, 1), (32, 576, 16, 1), (32, 576, 17, 1), (128, 2816, 32, 1), (128, 2816, 33, 1),
+                                       (256, 4096, 16, 1), (256, 4096, 17, 1), (64, 5184, 16, 0), (64, 5184, 17, 0), (64, 5184, 17, 1)])
+def test_router_logits_on_both_sides_of_the_few_waves(gpu, oracle, e, d, t, off):
+    """a wave per (token, row) with the row's loads asked for together and, one token further, only those inside the row: rows of part
+    of a trip, whole trips and two, x on a 16-byte boundary and one element behind it, bit for bit the oracle's rows"""
+    _, wr, x = _draw(oracle, f"few-{e}-{d}", e, d, t, 0.05)
+    fam = ops.FamilyRouters(gpu)
+    rows = torch.empty(t * d + 8, dtype=torch.bfloat16, device="cuda")[off:off + t * d].view(t, d)
+    rows.copy_(ops.bf16_tensor(x))
+    lg = torch.zeros((t, e), dtype=torch.float32, device="cuda")
+    fam.encode_router_top_k(ops.bf16_tensor(wr), rows, torch.zeros(e, device="cuda"), torch.zeros((t, 2), dtype=torch.int32, device="cuda"),
+                            torch.zeros((t, 2), device="cuda"), e, d, 1.0, lg, top_k=2, t=t)
+    torch.cuda.synchronize()
+    got = lg.cpu().numpy()
+    for i in sorted({0, 1, t // 2, t - 1}):
+        assert np.array_equal(_bits(got[i]), _bits(oracle.router_logits(wr, x[i]))), i
+
+
 @pytest.mark.parametrize("e", [8, 16, 24, 33, 100, 128, 168, 255, 256])
 def test_sqrtsoftplus_ties_match_serial(gpu, oracle, e):
     """RouterTopKParityTests.swift:52-77: tie-heavy logits and duplicated correction biases"""
