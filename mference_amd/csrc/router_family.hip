@@ -20,9 +20,9 @@ namespace {
 // x' = x * effective_scale is exact in fp32 for bf16 factors.  A lane's first CPL chunks are requested together
 // (a row of 2816 is six chunks a lane: six trips to memory one after the other took 2 us of a one-token call), and the
 // scales and biases of their groups come a group to a lane: two requests for all of them instead of two per chunk
-// (128 rows of 2816, one token, with a wave to a workgroup: 3.9 -> 3.5 us).
+// (128 rows of 2816, one token, with a wave to a workgroup: 3.9 -> 3.5 us).  FEW: as in router_logits_kernel.
 // (The pointers are not declared restrict: loads of memory that is never written may be moved behind the fence, next to their use.)
-template <int CPL, bool ALIGNED>
+template <int CPL, bool ALIGNED, bool FEW>
 __global__ __launch_bounds__(256) void router_logits_int8_kernel(
     const uint8_t* codes, const uint16_t* scales,
     const uint16_t* biases, const uint16_t* x,
@@ -45,7 +45,8 @@ __global__ __launch_bounds__(256) void router_logits_int8_kernel(
     uint4 xv[CPL], ev[CPL];
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
-      const uint32_t c = min(c0 + i * kWave, chunks - 1);  // past the row: the last chunk again, dropped below
+      const uint32_t c = FEW ? min(c0 + i * kWave, chunks - 1) : c0 + i * kWave;  // past the row: the last chunk again, dropped below
+      if (!FEW && c >= chunks) continue;
       if constexpr (ALIGNED) q[i] = *reinterpret_cast<const uint2*>(q_row + c * 8);
       else q[i] = make_uint2(load_u32_bytes(q_row + c * 8), load_u32_bytes(q_row + c * 8 + 4));
       xv[i] = load_x8<ALIGNED>(x_row + c * 8);
@@ -320,11 +321,18 @@ hipError_t launch_router_logits_int8(hipStream_t s, const uint8_t* codes, const 
 #undef MF_R8
     return hipGetLastError();
   }
-  // a wave to a workgroup while that is at most four a CU: its loads have a CU's paths to themselves
-  const uint32_t block = waves <= 4 * device_cu_count() ? 64u : 256u;
+  // A wave to a workgroup while that is at most four a CU: its loads have a CU's paths to themselves.  Few waves: nothing branches between
+  // a row's loads; beyond, nothing past the row is asked for.  us with the selection, without / with branches: aligned, 128 rows of 2816, 15
+  // tokens 6.83 / 7.04; of 5120, 16, 64, 300 tokens 7.8 / 7.95, 14.4 / 13.6, 46.1 / 40.8; unaligned (two chunks a trip), 64 rows of 1088, 15, 32,
+  // 300 tokens 6.01 / 6.02, 6.48 / 6.28, 18.7 / 14.4.
+  const uint32_t cus = device_cu_count(), block = waves <= 4 * cus ? 64u : 256u;
+  const bool few = waves <= (al ? 8 : 4) * cus;
   const dim3 grid((waves + block / 64 - 1) / (block / 64));
-#define MF_R8(CPL, AL) \
-  router_logits_int8_kernel<CPL, AL><<<grid, dim3(block), 0, s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits)
+#define MF_R8(CPL, AL)                                                                                                                   \
+  do {                                                                                                                                   \
+    if (few) router_logits_int8_kernel<CPL, AL, true><<<grid, dim3(block), 0, s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits); \
+    else router_logits_int8_kernel<CPL, AL, false><<<grid, dim3(block), 0, s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits);    \
+  } while (0)
   if (!al) MF_R8(2, false);
   else if (cpl <= 2) MF_R8(2, true);
   else if (cpl <= 4) MF_R8(4, true);
