@@ -255,9 +255,10 @@ template <typename T, int N> struct RegArray {
 };
 
 // LDS[lds + 16 * lane ...] = the 16 bytes at p of every lane (lds: a byte address, uniform), without a register in between.  The
-// compiler does not know of the request: wait_loads and a barrier stand in front of the first read.
+// compiler does not know of the request: wait_loads stands in front of the first read, and a barrier behind it where another wave reads.
+// (The address is an input in m0, so that the compiler writes that register and knows that it does; the wait state between is this asm's.)
 __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 // every load of this wave but its newest N has arrived
 template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
