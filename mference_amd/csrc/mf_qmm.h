@@ -89,10 +89,11 @@ constexpr int kMixedBits = 24;
 inline int part_bits(int bits, const QmmArgs& q) { return bits != kMixedBits ? bits : q.dense_mode ? 4 : 2; }
 
 // tile_slots: entries of the tile list (routed; a multiple of 8) or number of tiles (dense), tiles of TT rows (kTileTokens or
-// kSmallTile) in both.  `b` (optional) is a second problem for the same instantiation, run behind `a` in the same launch.
+// kSmallTile) in both.  `b` (optional) is a second problem for the same instantiation, run behind `a` in the same launch.  few: the
+// form for few work items (tiles of 32 only).
 template <int TT>
 hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj, uint32_t tile_slots, const QmmArgs* b,
-                            uint32_t b_tile_slots);
+                            uint32_t b_tile_slots, bool few);
 template <int TT>
 hipError_t launch_kres_tiles(hipStream_t s, int bits, const QmmArgs& a, uint32_t tile_slots, const QmmArgs* b,
                              uint32_t b_tile_slots);

@@ -11,17 +11,20 @@
 
 namespace mf {
 
-// LDS of qmm_kernel: x tile ring (2 stages of 2 K groups), the scales and the group sums of a step of 16 groups, 12 bytes a route
+// LDS of qmm_kernel: x tile ring (2 stages of 2 K groups, 4 of the form for few work items), the scales and the group sums of a step of 16 groups, 12 bytes a route
 constexpr uint32_t kTabStep = 16;
-__host__ __device__ constexpr uint32_t qmm_x_bytes(uint32_t tile) { return 2 * 2 * tile * 8 * 16; }
+__host__ __device__ constexpr uint32_t qmm_stages(bool few) { return few ? 4 : 2; }
+__host__ __device__ constexpr uint32_t qmm_x_bytes(uint32_t tile, bool few) { return qmm_stages(few) * 2 * tile * 8 * 16; }
 __host__ __device__ constexpr uint32_t qmm_scale_bytes(int nproj) { return nproj * kQmmWaves * kTabStep * 32 * 4; }
 __host__ __device__ constexpr uint32_t qmm_sum_bytes(uint32_t tile) { return 3 * tile * 2 * 16; }
-__host__ __device__ constexpr uint32_t qmm_lds_bytes(uint32_t tile, int nproj) {
-  return qmm_x_bytes(tile) + qmm_scale_bytes(nproj) + qmm_sum_bytes(tile) + tile * 12;
+__host__ __device__ constexpr uint32_t qmm_lds_bytes(uint32_t tile, int nproj, bool few) {
+  return qmm_x_bytes(tile, few) + qmm_scale_bytes(nproj) + qmm_sum_bytes(tile) + tile * 12;
 }
 
-// waves a SIMD (workgroups a CU) that the kernels' registers are budgeted for
-__host__ __device__ constexpr int qmm_waves(uint32_t tile, int nproj) { return tile == kSmallTile || nproj == 1 ? 3 : 2; }
+// waves a SIMD (workgroups a CU) that the kernels' registers are budgeted for; few: the form for few work items
+__host__ __device__ constexpr int qmm_waves(uint32_t tile, int nproj, bool few = false) {
+  return !few && (tile == kSmallTile || nproj == 1) ? 3 : 2;
+}
 
 __device__ __forceinline__ void qmm_trace(const QmmArgs& a, uint32_t work, uint32_t k) {
   if (a.trace && threadIdx.x == 0 && work < a.trace_items) a.trace[work * 8 + k] = wall_clock64();
@@ -60,7 +63,11 @@ __device__ __forceinline__ uint32_t qmm_work(const QmmArgs& a, const QmmPlace& a
 // loop 6.1 -> 3.5, whole item 33.1 -> 29.8, launch 136 -> 126 under the tracer; two 5120 x 17408 MLPs, 150 rows 303 -> 277; tiles of
 // 32: 2816 x 704, 300 tokens 64 -> 60, large 2-bit layer, 777 tokens 362 -> 345 (there the instructions of the loop are the bound).
 // LDS no longer grows with K, so every contraction keeps its two or three workgroups a CU.
-// LDS (dynamic): x tile ring, 2 stages x 2 K groups x [TT tokens][8 runs, turned] x 16 B; per wave the scales of a step
+// FEW (tiles of 32): a launch that leaves a CU at most two workgroups is bound by what each waits for, codes from HBM above all.  It has
+// the registers of two waves and their LDS: codes run four pairs of groups ahead, x three, and units are not kept apart.  The layer call,
+// us, x in registers and two pairs of codes (the kernel before) / one pair / this: 16 experts of 8192 x 512, top 2, 17 tokens 81.3 / 91.4 /
+// 75.8, 150 tokens 95.6 / 100.9 / 86.5; 32 of 5120 x 1536, top 1, 17 tokens 66.3 / 70.5 / 61.2; Qwen shape, 9 tokens 53.2 / 55.6 / 52.6.
+// LDS (dynamic): x tile ring, 2 stages (FEW: 4) x 2 K groups x [TT tokens][8 runs, turned] x 16 B; per wave the scales of a step
 // [NPROJ][16][32 rows] fp32; group sums of a step; per route: out slot u32, what its results lack, scale of its activations.
 // One launch can carry two independent problems of the same instantiation (the routed experts
 // and the shared expert of the same phase): the second problem's work items follow the first's
@@ -73,7 +80,7 @@ struct QmmLaunch {
 
 // NG8: K is a whole number of steps of 8 groups and the rows a whole number of slices; the other form takes any number
 // of groups and rows.
-template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED>
+template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED, bool FEW>
 __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place, uint8_t* smem) {
   constexpr int NT = TT / 32;             // token blocks of a tile
   constexpr uint32_t kXGroup = TT * 8;    // 16-byte pieces of one K group of the x tile
@@ -119,13 +126,13 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
   }
 
   uint4* s_x = reinterpret_cast<uint4*>(smem);                      // 2 stages x 2 groups x kXGroup uint4
-  float* s_scale = reinterpret_cast<float*>(smem + qmm_x_bytes(TT)) + wv * (NPROJ * kTabStep * 32);  // this wave's [NPROJ][16 groups][32 rows]
-  uint4* s_sum = reinterpret_cast<uint4*>(smem + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ));  // [NT][3 parts][64 lanes]
-  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ) + qmm_sum_bytes(TT));
+  float* s_scale = reinterpret_cast<float*>(smem + qmm_x_bytes(TT, FEW)) + wv * (NPROJ * kTabStep * 32);  // this wave's [NPROJ][16 groups][32 rows]
+  uint4* s_sum = reinterpret_cast<uint4*>(smem + qmm_x_bytes(TT, FEW) + qmm_scale_bytes(NPROJ));  // [NT][3 parts][64 lanes]
+  uint32_t* s_slot = reinterpret_cast<uint32_t*>(smem + qmm_x_bytes(TT, FEW) + qmm_scale_bytes(NPROJ) + qmm_sum_bytes(TT));
   float* s_rel = reinterpret_cast<float*>(s_slot + TT);  // [TT]
   float* s_act = s_rel + TT;                              // [TT]
   const uint32_t lds_x = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) uint8_t*)smem));
-  const uint32_t lds_sum = lds_x + qmm_x_bytes(TT) + qmm_scale_bytes(NPROJ);
+  const uint32_t lds_sum = lds_x + qmm_x_bytes(TT, FEW) + qmm_scale_bytes(NPROJ);
 
   // weight pointers of this workgroup's projections
   const uint8_t* Wp[NPROJ];
@@ -192,9 +199,9 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
     const uint32_t gc = min(g, last_pair);
     return wbase[p] + (gc * gstride + (i ? second : 0u)) + (!NG8 && gc == last_pair ? last_off : lane_off);
   };
-  // pairs of groups in flight: one for 4-bit codes on tiles of 32, whose registers do not hold a second (with it, 31 values went
+  // pairs of groups in flight: one for 4-bit codes on tiles of 32, whose 168 registers do not hold a second (with it, 31 values went
   // through scratch memory: 2816 x 704, 300 tokens, gate / up 60 -> 100 us; 93 tokens of the Qwen shape 31 -> 37)
-  constexpr int kRing = NT == 1 && BITS == 4 ? 1 : 2;
+  constexpr int kRing = FEW ? 4 : NT == 1 && BITS == 4 ? 1 : 2;
   RegArray<Codes, kRing> cur[NPROJ];
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p) {
@@ -275,8 +282,16 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
   // there is: only those are scaled (RES), 4 of 16 multiply-adds per group and row block.
   auto tile_body = [&](auto nta_c, auto res_c) {
   constexpr int NTA = decltype(nta_c)::value, RES = decltype(res_c)::value;
+  // Behind a pair's x a wave requests kCodeLoads loads of codes, and before that pair's turn the x of every further stage and as many
+  // codes again: kBehind, of which none may be left out.
+  constexpr int kStages = qmm_stages(FEW), kCodeLoads = NPROJ * (BITS == 4 ? 2 : 1);
+  constexpr int kBehind = (kStages - 2) * (kCodeLoads + 2 * NTA) + kCodeLoads;
   sums_request(0, NTA);
   x_request(0, 0, NTA);
+  if constexpr (FEW) {
+#pragma unroll
+    for (int u = 1; u < kStages - 1; ++u) x_request(min(2u * u, last_pair), u, NTA);
+  }
   if (threadIdx.x < TT) {
     s_rel[threadIdx.x] = rel_of_scale(a.act_rows ? act_scale(row_max) : row_scale(row_max));
     s_act[threadIdx.x] = act_scale(row_max);
@@ -320,17 +335,16 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
   wait_loads<0>();
   qmm_trace(a, work, 2);
 
-  // Weight codes run up to four K groups ahead in a ring of registers (the expert's bytes come from HBM); x rows come from L2 a pair
-  // of groups ahead, into the stage that is not being read.  kCodeLoads: what a wave requests behind a pair's x until that pair's turn.
-  constexpr int kCodeLoads = NPROJ * (BITS == 4 ? 2 : 1);
+  // Weight codes run kRing pairs of K groups ahead in a ring of registers (the expert's bytes come from HBM); x rows come from L2
+  // kStages - 1 pairs ahead, into the stage that was read last.
   Codes now[NPROJ];
-  for (uint32_t g0 = 0; g0 < ng; g0 += 4) {
+  for (uint32_t g0 = 0; g0 < ng; g0 += 2 * kStages) {
 #pragma unroll
-    for (int uu = 0; uu < 2; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
+    for (int uu = 0; uu < kStages; ++uu) {  // pair of K groups g0 + 2uu, g0 + 2uu + 1 in stage uu
       const uint32_t gu = g0 + 2 * uu;
       if (!NG8 && gu >= ng) break;
-      wait_loads<kCodeLoads>();  // this wave's part of stage uu is there
-      __syncthreads();           // stage uu is complete, stage uu ^ 1 is no longer read
+      wait_loads<kBehind>();  // this wave's part of stage uu is there
+      __syncthreads();        // stage uu is complete, the stage before it is no longer read
       // The pair's codes are taken up in front of the request for x: the compiler counts the loads it knows, so behind
       // that request its wait for them would be one for x, too.
 #pragma unroll
@@ -341,7 +355,8 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
 #pragma unroll
         for (auto& w : codes.w) asm volatile("" : "+v"(w));
       }
-      if (gu + 2 < ng) x_request(gu + 2, uu ^ 1, NTA);
+      if constexpr (FEW) x_request(min(gu + 2 * (kStages - 1), last_pair), (uu + kStages - 1) % kStages, NTA);
+      else if (gu + 2 < ng) x_request(gu + 2, uu ^ 1, NTA);
       if constexpr (BITS == 2) {
 #pragma unroll
         for (int p = 0; p < NPROJ; ++p) cur[p][uu % kRing].load(1, codes_at(p, gu + 2 * kRing, 1));
@@ -349,11 +364,11 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
       // tables: a step's sums are requested when everybody has read the step's before, its scales and biases a pair ahead
       if (uu == 0 && g0 % kTabStep == 0) tab_step(g0);
       if (uu == 1 && g0 % kTabStep == 0 && g0 + kTabStep < ng) sums_request(g0 + kTabStep, NTA);
-      if (uu == 1 && g0 % kTabStep == kTabStep - 4 && g0 + 4 < ng) {
+      if (uu == kStages - 1 && g0 % kTabStep == kTabStep - 2 * kStages && g0 + 2 * kStages < ng) {
 #pragma unroll
         for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
-          for (int what = 0; what < 2; ++what) tab[what][p] = tab_fetch(what, p, g0 + 4);
+          for (int what = 0; what < 2; ++what) tab[what][p] = tab_fetch(what, p, g0 + 2 * kStages);
       }
 #pragma unroll
       for (int gi = 0; gi < 2; ++gi) {
@@ -389,7 +404,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
           for (int nt = 0; nt < NTA; ++nt)
 #pragma unroll
             for (int r = 0; r < RES; ++r) acc[p][nt][r] = __builtin_fmaf(sc, tmp[nt][r], acc[p][nt][r]);
-          if constexpr (NT == 1) __builtin_amdgcn_sched_barrier(0);  // one unit at a time: the registers of three waves
+          if constexpr (NT == 1 && !FEW) __builtin_amdgcn_sched_barrier(0);  // one unit at a time: the registers of three waves
         }
       }
       // (the sums are wanted here: without this a pair's products are kept beyond the branches behind it)
@@ -399,6 +414,7 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
         for (int nt = 0; nt < NTA; ++nt) asm volatile("" : "+v"(acc[p][nt]));
     }
   }
+  if constexpr (FEW) wait_loads<0>();  // (what was requested past the end: the ring is used again, and LDS is given back)
   // (results that do not exist: not kept through the loop)
 #pragma unroll
   for (int p = 0; p < NPROJ; ++p)
@@ -560,28 +576,28 @@ __device__ __forceinline__ void qmm_item(const QmmArgs& a, const QmmPlace& place
 
 // (Both parts of a launch read their codes in the form SWAPPED names; without it 2-bit codes have to be tiled.  The dense
 // problem beside 2-bit experts is 4-bit and goes through qmm_mixed_kernel: the launchers refuse a 2-bit one beside a tiled pool.)
-template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
+template <int TT, int BITS, int NPROJ, bool NG8, bool SWAPPED, bool FEW = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ, FEW), qmm_waves(TT, NPROJ, FEW))))
 void qmm_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const QmmPlace at = qmm_place(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  qmm_item<TT, BITS, NPROJ, NG8, SWAPPED>(a, at, smem);
+  qmm_item<TT, BITS, NPROJ, NG8, SWAPPED, FEW>(a, at, smem);
 }
 
 // 2-bit (or ternary) routed experts and a 4-bit shared expert in one launch: a launch of its own leaves the shared
 // expert's few, long work items on a handful of CUs (large 2-bit layer, 32 tokens: 39 + 25 us beside 127 + 69; 777
 // tokens: 53 + 33 beside 388 + 207).
-template <int TT, int NPROJ, bool NG8, bool SWAPPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ), qmm_waves(TT, NPROJ))))
+template <int TT, int NPROJ, bool NG8, bool SWAPPED, bool FEW = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qmm_waves(TT, NPROJ, FEW), qmm_waves(TT, NPROJ, FEW))))
 void qmm_mixed_kernel(const QmmLaunch launch) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   bool second;
   const QmmPlace at = qmm_place(launch.per_xcd, second);
   const QmmArgs& a = launch.part[second ? 1 : 0];
-  if (a.dense_mode) qmm_item<TT, 4, NPROJ, NG8, true>(a, at, smem);
-  else qmm_item<TT, 2, NPROJ, NG8, SWAPPED>(a, at, smem);
+  if (a.dense_mode) qmm_item<TT, 4, NPROJ, NG8, true, FEW>(a, at, smem);
+  else qmm_item<TT, 2, NPROJ, NG8, SWAPPED, FEW>(a, at, smem);
 }
 
 // ---- the same product for a short contraction (K <= 512: the down projections) ----
@@ -978,7 +994,7 @@ hipError_t launch_kres_tiles(hipStream_t s, int bits, const QmmArgs& a, uint32_t
 
 template <int TT>
 hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj, uint32_t tile_slots, const QmmArgs* b,
-                            uint32_t b_tile_slots) {
+                            uint32_t b_tile_slots, bool few) {
   QmmLaunch launch{};
   const bool tiled = a.tiled || (b && b->tiled);  // which form of the code loads: QmmCodes
   if (bits == 2 && tiled && !(a.tiled && (!b || b->tiled))) return hipErrorInvalidValue;
@@ -998,8 +1014,8 @@ hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj
     }
     ng8 = ng8 && (q.n_win > 1 ? q.ng_ld : q.kdim / kGroup) % 8 == 0 && q.rows % slice_rows == 0;
   }
-  const size_t lds = qmm_lds_bytes(TT, nproj);
   const dim3 grid(8 * (launch.per_xcd[0] + launch.per_xcd[1])), block(256);
+  const size_t lds = qmm_lds_bytes(TT, nproj, TT == kSmallTile && few);
   if (grid.x == 0) return hipSuccess;
 #define MF_QMM_L(...)                                                                                  \
   do {                                                                                                 \
@@ -1007,18 +1023,26 @@ hipError_t launch_qmm_tiles(hipStream_t s, int bits, const QmmArgs& a, int nproj
     if (e != hipSuccess) return e;                                                                     \
     __VA_ARGS__<<<grid, block, lds, s>>>(launch);                                                      \
   } while (0)
+#define MF_QMM_FORM(KERNEL, ...)                                                                       \
+  do {                                                                                                 \
+    if constexpr (TT == kSmallTile) {                                                                  \
+      if (few) { MF_QMM_L(KERNEL<__VA_ARGS__, true>); break; }                                         \
+    }                                                                                                  \
+    MF_QMM_L(KERNEL<__VA_ARGS__, false>);                                                              \
+  } while (0)
 #define MF_QMM(P, G)                                                                                   \
   do {                                                                                                 \
-    if (bits == kMixedBits && tiled) MF_QMM_L(qmm_mixed_kernel<TT, P, G, false>);                          \
-    else if (bits == kMixedBits) MF_QMM_L(qmm_mixed_kernel<TT, P, G, true>);                               \
-    else if (bits == 4 && tiled) MF_QMM_L(qmm_kernel<TT, 4, P, G, false>);                                 \
-    else if (bits == 4) MF_QMM_L(qmm_kernel<TT, 4, P, G, true>);                                           \
-    else if (tiled) MF_QMM_L(qmm_kernel<TT, 2, P, G, false>);                                              \
-    else MF_QMM_L(qmm_kernel<TT, 2, P, G, true>);                                                          \
+    if (bits == kMixedBits && tiled) MF_QMM_FORM(qmm_mixed_kernel, TT, P, G, false);                       \
+    else if (bits == kMixedBits) MF_QMM_FORM(qmm_mixed_kernel, TT, P, G, true);                            \
+    else if (bits == 4 && tiled) MF_QMM_FORM(qmm_kernel, TT, 4, P, G, false);                              \
+    else if (bits == 4) MF_QMM_FORM(qmm_kernel, TT, 4, P, G, true);                                        \
+    else if (tiled) MF_QMM_FORM(qmm_kernel, TT, 2, P, G, false);                                           \
+    else MF_QMM_FORM(qmm_kernel, TT, 2, P, G, true);                                                       \
   } while (0)
   if (nproj == 2) { if (ng8) MF_QMM(2, true); else MF_QMM(2, false); }
   else { if (ng8) MF_QMM(1, true); else MF_QMM(1, false); }
 #undef MF_QMM
+#undef MF_QMM_FORM
 #undef MF_QMM_L
   return hipGetLastError();
 }

@@ -1323,9 +1323,9 @@ hipError_t launch_prep_rows(hipStream_t s, const uint16_t* src, uint16_t* dst, u
 }
 
 static hipError_t launch_qmm(hipStream_t s, uint32_t tile, int bits, const QmmArgs& a, int nproj, uint32_t tile_slots,
-                             const QmmArgs* b, uint32_t b_tile_slots) {
-  return tile == kSmallTile ? launch_qmm_tiles<kSmallTile>(s, bits, a, nproj, tile_slots, b, b_tile_slots)
-                            : launch_qmm_tiles<kTileTokens>(s, bits, a, nproj, tile_slots, b, b_tile_slots);
+                             const QmmArgs* b, uint32_t b_tile_slots, bool few = false) {
+  return tile == kSmallTile ? launch_qmm_tiles<kSmallTile>(s, bits, a, nproj, tile_slots, b, b_tile_slots, few)
+                            : launch_qmm_tiles<kTileTokens>(s, bits, a, nproj, tile_slots, b, b_tile_slots, few);
 }
 static hipError_t launch_qmm_kres(hipStream_t s, uint32_t tile, int bits, const QmmArgs& a, uint32_t tile_slots,
                                   const QmmArgs* b, uint32_t b_tile_slots) {
@@ -1610,6 +1610,9 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
   }
   q.x = xp; q.sumx = sumx; q.row_max = row_max; q.x_stride = d; q.rows = f; q.kdim = d; q.epi = 0; q.out = act; q.out_sums = sum_act;
   const uint32_t gu_win = dense_gate_up_windows(d);
+  // At most 32 rows over a long K: tiles of 32 in the form for few work items.  The MLP, us, tiles of 64 / this: 5120 x 17408, 9 rows
+  // 77.3 / 74.5, 32 rows 79.5 / 77.8; 7168 x 2048, 9 rows 63.6 / 58.1; 4096 x 12800, 9 rows 53.3 / 50.7; at d of 2048 and less no gain.
+  const uint32_t tile = t <= kSmallTile && d > 2048 && gu_win * ((f + kQmmRows - 1) / kQmmRows) <= 2 * device_cu_count() ? kSmallTile : kTileTokens;
   if (gu_win > 1) {
     // few rows (or a K too long for one launch's scale tables): the contraction in windows, both projections as
     // fp32 per window, then one pass that adds the windows, activates and sums the groups
@@ -1619,7 +1622,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     float* pu = pg + part_stride * gu_win;
     q.ng_ld = ng; q.kdim = dense_longest_window(ng, gu_win) * kGroup; q.n_win = gu_win; q.out_win_stride = part_stride;
     q.epi = 1; q.out = pg; q.out2 = pu;
-    e = launch_qmm(s, kTileTokens, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
+    e = launch_qmm(s, tile, code_bits, q, 2, (t + tile - 1) / tile, nullptr, 0, tile == kSmallTile);
     if (e != hipSuccess) return e;
     const size_t chunks = static_cast<size_t>(t) * f / 8;
     dense_swiglu_combine_kernel<<<dim3(static_cast<uint32_t>((chunks + 255) / 256)), dim3(256), 0, s>>>(
@@ -1627,7 +1630,7 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   } else {
-    e = launch_qmm(s, kTileTokens, code_bits, q, 2, (t + kTileTokens - 1) / kTileTokens, nullptr, 0);
+    e = launch_qmm(s, tile, code_bits, q, 2, (t + tile - 1) / tile, nullptr, 0, tile == kSmallTile);
     if (e != hipSuccess) return e;
   }
   return dense_project(s, down, bits, act, sum_act, row_max, true, y, t, d, f, down_windows, false, base);
@@ -1646,6 +1649,15 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
 // 128 experts, 93 tokens 67.5 / 65.3; 2048 x 512 beside a shared expert of 1024, 40 67.7 / 65.0, 93 74.4 / 70.2, 300 109.5 / 104.8;
 // 1664 x 512, 64 experts, 93 56.6 / 54.1, 200 (25 routes an expert) 65.2 / 67.2.
 struct PrefillTiles { uint32_t up, down; };
+// Whether a matmul launch on tiles of 32 has few work items (`items`, at most) over a long contraction: the kernel's form for that, which
+// keeps two workgroups on a CU.  Layer call, us, the form of three workgroups / that form.  Length: 1024 x 384, 48 experts, top 4, 64
+// tokens 34.3 / 35.6; ternary 1536 x 128, 64 tokens 46.3 / 44.7; Qwen shape (2048), 9 tokens 44.5 / 42.6.  Items: 64 experts of 2048 x 1024,
+// top 2, 300 tokens, 640 items 59.0 / 65.3; 32 of 5120 x 1536, top 1, 480 items, 193 tokens (6 routes an expert) 83.9 / 75.2, but
+// 300 tokens (9), whose tiles have twice the results to scale, 105.8 / 109.3; 16 of 8192 x 512, top 2, 108 items, 193 tokens (24) 104.9 / 90.3.
+static bool prefill_few(const mf_moe_config& c, uint32_t t, uint64_t items, uint32_t kdim) {
+  return kdim > 1024 && (items <= device_cu_count() ||
+                         (items <= 2 * device_cu_count() && static_cast<uint64_t>(t) * c.top_k <= 8ull * c.num_experts));
+}
 static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t, bool resident) {
   const bool two_bit = c.bits != MF_BITS_4 && !c.shared_f;
   const uint64_t few = static_cast<uint64_t>(two_bit ? 128 : 32) * c.num_experts;
@@ -1655,10 +1667,10 @@ static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t, bool resid
   return p;
 }
 
-// entries of the tile list: every live expert may end in a partial tile; a multiple of 8
+// entries of the tile list, a multiple of 8: an expert of c routes has ceil(c / tile) tiles, and at most min(experts, routes) have any
 uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t, uint32_t tile) {
   const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const size_t n = std::min<size_t>(c.num_experts, pairs) + pairs / tile + 1;
+  const size_t n = std::max<size_t>((pairs + (tile - 1) * std::min<size_t>(c.num_experts, pairs)) / tile, 1);
   return static_cast<uint32_t>((n + 7) / 8 * 8);
 }
 
@@ -1903,8 +1915,10 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   // (Qwen shape, layer: 2048 tokens 280.5 -> 274.5 us, 1024 tokens 191 -> 187 us, 4096 tokens 506 -> 503 us;
   // at 16 384 tokens they are better last, 1763 against 1776 us, where they fill the holes of the last round).
   const bool dense_first = shared_rides && pairs <= 32768;
-  if (dense_first) MF_TRY(launch_qmm(s, tile.up, launch_bits, d, 2, dense_up, &q, lists.slots[0]));
-  else MF_TRY(launch_qmm(s, tile.up, launch_bits, q, 2, lists.slots[0], shared_rides ? &d : nullptr, dense_up));
+  const auto slices = [](uint32_t rows, uint32_t rows_per_item) -> uint64_t { return (rows + rows_per_item - 1) / rows_per_item; };
+  const bool few_up = prefill_few(c, t, lists.slots[0] * slices(c.f, kQmmRows) + dense_up * slices(c.shared_f, kQmmRows), c.d);
+  if (dense_first) MF_TRY(launch_qmm(s, tile.up, launch_bits, d, 2, dense_up, &q, lists.slots[0], few_up));
+  else MF_TRY(launch_qmm(s, tile.up, launch_bits, q, 2, lists.slots[0], shared_rides ? &d : nullptr, dense_up, few_up));
   if (lists.list[1]) q.tiles = lists.list[1];
   q2.sorted = q.sorted; q2.tiles = q.tiles; q2.row_max = q.row_max;
   q2.x = ws.acts; q2.sumx = ws.sum_acts; q2.out = ws.partials;
@@ -1912,16 +1926,18 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
     d2.x = ws.sact; d2.sumx = ws.sum_sact; d2.out = ws.hs; d2.row_max = d.row_max;
   }
   const int down_proj = q2.pair_rows ? 2 : 1;
+  const uint64_t down_slices = slices(c.d, kQmmRows * down_proj);
+  const bool few_down = prefill_few(c, t, (lists.slots[1] + (apart ? 0 : dense_down)) * down_slices, c.f);
   if (!shared_rides || apart) {
     if (kres_q) MF_TRY(launch_qmm_kres(s, tile.down, code_bits, q2, lists.slots[1], nullptr, 0));
-    else MF_TRY(launch_qmm(s, tile.down, code_bits, q2, down_proj, lists.slots[1], nullptr, 0));
+    else MF_TRY(launch_qmm(s, tile.down, code_bits, q2, down_proj, lists.slots[1], nullptr, 0, few_down));
     if (apart && kres_d) MF_TRY(launch_qmm_kres(s, tile.down, 4, d2, dense_down, nullptr, 0));
-    else if (apart) MF_TRY(launch_qmm(s, tile.down, 4, d2, down_proj, dense_down, nullptr, 0));
+    else if (apart) MF_TRY(launch_qmm(s, tile.down, 4, d2, down_proj, dense_down, nullptr, 0, prefill_few(c, t, dense_down * down_slices, c.shared_f)));
   } else if (kres_both) {
     if (dense_first) MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, d2, dense_down, &q2, lists.slots[1]));
     else MF_TRY(launch_qmm_kres(s, tile.down, launch_bits, q2, lists.slots[1], &d2, dense_down));
-  } else if (dense_first) MF_TRY(launch_qmm(s, tile.down, launch_bits, d2, down_proj, dense_down, &q2, lists.slots[1]));
-  else MF_TRY(launch_qmm(s, tile.down, launch_bits, q2, down_proj, lists.slots[1], &d2, dense_down));
+  } else if (dense_first) MF_TRY(launch_qmm(s, tile.down, launch_bits, d2, down_proj, dense_down, &q2, lists.slots[1], few_down));
+  else MF_TRY(launch_qmm(s, tile.down, launch_bits, q2, down_proj, lists.slots[1], &d2, dense_down, few_down));
   if (ragged) return hipSuccess;  // the per-route results are the caller's: mf_moe_unpermute reduces them
   const uint16_t* hs = nullptr;
   const uint16_t* gate = nullptr;

@@ -709,3 +709,25 @@ def test_prefill_contractions_around_the_steps_of_the_tables(gpu, oracle, bits, 
     ref, ref_idx, _ = oracle.moe_layer(layer, x)
     assert np.array_equal(idx, ref_idx)
     assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref), f"bits={bits} d={d} f={f}")
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+@pytest.mark.parametrize("bits,d,f,e,k,fs,t", [
+    (4, 1088, 128, 16, 1, 0, 17), (4, 1152, 192, 8, 2, 128, 20), (4, 1216, 128, 4, 4, 0, 29), (4, 1280, 1088, 8, 2, 0, 33), (4, 1984, 128, 8, 1, 0, 24),
+    (4, 2048, 128, 16, 2, 128, 64), (4, 3072, 256, 8, 2, 0, 40), (2, 1088, 128, 8, 2, 128, 17), (2, 1280, 128, 4, 2, 0, 40), (2, 1536, 1152, 8, 2, 0, 33),
+    (2, 1984, 192, 8, 1, 192, 30), (1, 2112, 128, 32, 8, 0, 20), (4, 8192, 128, 4, 2, 0, 40),
+])
+def test_prefill_of_few_work_items(gpu, oracle, bits, d, f, e, k, fs, t, tiled):
+    """contractions longer than 1024 whose launches leave most of the chip idle: rings of four pairs of K groups at 17 to 20 groups (a last
+    pass of one half pair to two pairs), 31, whole passes, and 128; tiles of at most 8, 16 and 32 routes; the shared expert beside them"""
+    if tiled and (d % 128 or f % 128 or fs % 128):
+        pytest.skip("a tiled pool needs whole 128-row widths")
+    layer = oracle.synth_layer(ROOT_SEED + 0xFE3 + d + f + t, d, f, e, k, bits=bits, fs=fs, router_mode=1 if bits == 1 else 0)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    if tiled:
+        wts.experts_tiled = moe.tile_experts(wts.experts, wts.offsets)
+    x = oracle.synth_x(ROOT_SEED + 0xFE + t, t, d)
+    y, idx, _ = _run_prefill(moe, wts, x, t, d, k)
+    ref, ref_idx, _ = oracle.moe_layer(layer, x)
+    assert np.array_equal(idx, ref_idx)
+    assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref), f"bits={bits} d={d} f={f}")

@@ -246,6 +246,27 @@ def test_mlp_block_of_few_rows(gpu, oracle, bits, d, f, t):
 
 
 @pytest.mark.parametrize("bits", [4, 2])
+@pytest.mark.parametrize("d,f", [(2112, 192), (2176, 448), (2240, 128), (2304, 128), (2560, 1024), (7296, 128)])
+def test_mlp_block_of_few_rows_over_a_long_contraction(gpu, bits, d, f):
+    """gate and up of at most 32 rows over more than 2048 values go in tiles of 32 with rings of four pairs of K groups: a row has the bits
+    it has among 33, which go in tiles of 64 (33 to 36 groups, 40, and two windows of 57; down keeps its windows up to 64 rows)"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + f + bits)
+    mk = lambda r, c: ops.Quantization(gpu).quantize_affine(torch.randn((r, c), generator=gen, device="cuda") * 0.02, bits)
+    qs = [mk(f, d), mk(f, d), mk(d, f)]
+    x = torch.randn((33, d), generator=gen, device="cuda").to(torch.bfloat16)
+    op = ops.SharedExpertInt4(gpu)
+    scratch = torch.zeros(op.scratch_bytes(d, f, 33), dtype=torch.uint8, device="cuda")
+    out = {}
+    for t in (33, 32, 24, 17, 16):
+        out[t] = torch.zeros((t, d), dtype=torch.bfloat16, device="cuda")
+        op.encode(x[:t].contiguous(), *qs, out[t], scratch, t=t)
+    torch.cuda.synchronize()
+    for t in (32, 24, 17, 16):
+        assert torch.equal(out[t], out[33][:t]), t
+
+
+@pytest.mark.parametrize("bits", [4, 2])
 @pytest.mark.parametrize("d,f,t", [(1152, 640, 20), (256, 3200, 70)])
 def test_mlp_block_keeps_infinities_to_their_row(gpu, bits, d, f, t):
     """rows with an infinity or a NaN come out NaN (an infinity meets codes of zero, and biases below zero) and
