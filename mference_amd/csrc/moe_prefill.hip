@@ -1636,15 +1636,29 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
   return dense_project(s, down, bits, act, sum_act, row_max, true, y, t, d, f, down_windows, false, base);
 }
 
+// entries of the tile list, a multiple of 8: an expert of c routes has ceil(c / tile) tiles, and at most min(experts, routes) have any
+uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t, uint32_t tile) {
+  const size_t pairs = static_cast<size_t>(t) * c.top_k;
+  const size_t n = std::max<size_t>((pairs + (tile - 1) * std::min<size_t>(c.num_experts, pairs)) / tile, 1);
+  return static_cast<uint32_t>((n + 7) / 8 * 8);
+}
+
 // Routes of a tile of the layer call's two matmuls.  A tile of 32 leaves registers and LDS for three workgroups a CU where one
 // of 64 leaves them for two, and wastes less where few tokens meet an expert; past 32 routes an expert (on average, over the
 // layer's experts) more and more tiles of 64 are full, and expand a weight for 64 tokens at a time.  2-bit codes without a
-// 4-bit shared expert beside them are read and expanded faster: past 128.  Layer call, tiles of 64 / 32, us: 256 4-bit experts
-// 2048 x 512, shared 512: 93 tokens 81.4 / 73.8, 256 95.3 / 88.7, 512 118.6 / 117.8, 2048 243 / 262; 128 experts of
-// 2816 x 704: 300 tokens 235 / 210, 500 302 / 299, 800 358 / 377; 256 2-bit experts of 4096 x 2048, shared 2048: 200 tokens
-// 347 / 322, 777 647 / 623, 2048 1194 / 1224; 64 ternary experts of 2048 x 1024: 400 tokens 136 / 111, 1600 267 / 259, 2048 310 / 312.
-// The resident kernel on 4-bit rows of 512 keeps tiles of 64: its three workgroups a CU have half the codes in flight each
-// (400 tokens, 2048 x 512: 24.1 / 30.0 us; 93 tokens 20.6 / 20.3).
+// 4-bit shared expert beside them are read and expanded faster: past 128.  Layer call, tiles of 64 / 32 in both matmuls, us, pool as loaded
+// (and tiled): 256 4-bit experts of 2048 x 512, shared 512: 93 tokens 79.5 / 68.9, 512 122.7 / 117.9, 1024 161 / 171 (153 / 153), 2048 244 / 277;
+// 128 experts of 2816 x 704: 300 tokens 185 / 172, 500 216 / 225, 800 252 / 286; 256 2-bit experts of 4096 x 2048, shared 2048: 200 tokens
+// 654 / 653 (587 / 551), 777 775 / 769 (698 / 672), 1365 987 / 1059 (916 / 955), 2048 1203 / 1368; 64 ternary experts of 2048 x 1024: 400 tokens
+// 128 / 121, 1024 194 / 195 (193 / 185), 2048 303 / 328; 256 of 2048 x 512: 1500 tokens 185 / 182 (180 / 172), 3000 293 / 304, 4096 363 / 392.
+// Around the lines no one number is right for every shape: the fewer work items a launch has, the longer tiles of 32 win.  At 32 routes an
+// expert 128 2-bit experts of 4096 x 256, shared 512, 158 / 134; 64 of 2048 x 768 92.5 / 89.5; 128 of 4096 x 1024 294 / 312 (274 / 263); 32 of
+// 5120 x 1536 199 / 224 (182 / 181).  At 64 of 2-bit codes 64 of 1536 x 128 71 / 63, 64 of 4096 x 2048 363 / 379 (348 / 349).
+// The resident kernel on 4-bit rows of 512 has half the codes in flight each in its three workgroups a CU: tiles of 32 from a route
+// an expert on and while their work items make up to five a CU.  Layer call, us, 64 / 32: 2048 x 512, 256 experts, top 8, shared 512, 16, 32, 64, 96, 192, 256,
+// 384, 768 tokens 54.2 / 55.2, 58.6 / 59.5, 71.2 / 69.3, 72.6 / 70.4, 81.6 / 77.5, 91.6 / 91.0, 96.7 / 99.9, 144.4 / 149.0; 1024 x 512, 128 experts, 64, 192, 384 tokens
+// 49.9 / 47.1, 55.7 / 53.6, 61.5 / 58.2; 4096 x 512, 64 experts, top 4, 96, 256, 384 tokens 72.4 / 69.5, 101.3 / 97.6, 120.0 / 120.8; 5120 x 512,
+// 128 experts, shared 512, 9, 32, 96, 256 tokens 93.2 / 93.4, 114.3 / 116.7, 157.6 / 163.7, 211.6 / 218.4.
 // resident: that kernel takes the down projections of the call.  Where it does not, the ring on tiles of 64 / 32, us a call: 2176 x 512,
 // 128 experts, 93 tokens 67.5 / 65.3; 2048 x 512 beside a shared expert of 1024, 40 67.7 / 65.0, 93 74.4 / 70.2, 300 109.5 / 104.8;
 // 1664 x 512, 64 experts, 93 56.6 / 54.1, 200 (25 routes an expert) 65.2 / 67.2.
@@ -1663,15 +1677,10 @@ static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t, bool resid
   const uint64_t few = static_cast<uint64_t>(two_bit ? 128 : 32) * c.num_experts;
   PrefillTiles p;
   p.up = static_cast<uint64_t>(t) * c.top_k <= few ? kSmallTile : kTileTokens;
-  p.down = resident && c.bits == MF_BITS_4 && c.f == 512 ? kTileTokens : p.up;
+  const bool few_or_many = static_cast<uint64_t>(t) * c.top_k <= c.num_experts ||
+                           static_cast<uint64_t>(prefill_tile_slots(c, t, kSmallTile)) * c.d > 5ull * 512 * device_cu_count();  // (an item: 512 rows)
+  p.down = resident && c.bits == MF_BITS_4 && c.f == 512 && few_or_many ? kTileTokens : p.up;
   return p;
-}
-
-// entries of the tile list, a multiple of 8: an expert of c routes has ceil(c / tile) tiles, and at most min(experts, routes) have any
-uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t, uint32_t tile) {
-  const size_t pairs = static_cast<size_t>(t) * c.top_k;
-  const size_t n = std::max<size_t>((pairs + (tile - 1) * std::min<size_t>(c.num_experts, pairs)) / tile, 1);
-  return static_cast<uint32_t>((n + 7) / 8 * 8);
 }
 
 // workspace carve-up of one prefill layer call

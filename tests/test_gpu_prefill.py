@@ -564,6 +564,26 @@ def test_prefill_full_size_rows_do_not_depend_on_their_neighbours(gpu, oracle):
                            oracle.bf16_to_float(ops.bf16_bits(yd)), f"prefill row {i} vs decode")
 
 
+def test_prefill_rows_on_both_sides_of_the_resident_tiles(gpu):
+    """256 experts of 2048 x 512: the resident down projections take tiles of 32 from 33 to 288 tokens and of 64 on either side, beside gate / up
+    on tiles of 32 and, in the long prompt, of 64: a token's row has the same bits in all"""
+    import bench
+    w = dict(bench.QWEN)
+    lw = bench.build_stack(gpu, w, 1, torch.device("cuda", 0))[0]
+    moe = ops.MoE(gpu, w["d"], w["f"], w["e"], w["k"], bits=4, shared_f=w["fs"], shared_bits=4)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    x = torch.randn((1100, w["d"]), generator=gen, device="cuda").to(torch.bfloat16)
+    def rows(t):
+        y = torch.zeros((t, w["d"]), dtype=torch.bfloat16, device="cuda")
+        moe.encode_prefill_layer(lw, x[:t].contiguous(), y, t)
+        torch.cuda.synchronize()
+        return y.view(torch.int16)
+    want = rows(1100)
+    for t in (20, 33, 288, 289, 1024):
+        assert torch.equal(rows(t), want[:t]), t
+
+
 def test_prefill_16k_tokens_repeat_the_2048_token_rows(gpu):
     """16 384 tokens (131 072 routes, 2 000+ tiles, 1 GiB of per-route partial rows -- byte offsets
     of the down projection's stores reach 2^30): the batch is the 2048-token batch eight times
