@@ -1826,13 +1826,16 @@ hipError_t launch_prefill_layer(hipStream_t s, const mf_moe& h, const mf_moe_lay
   const bool kres_q = kres_takes(q2, pairs), kres_d = c.shared_f && kres_takes(d2, t);
   // Both parts in one launch of one kernel: the resident one when it takes both (their K has to be the same), else the
   // ring.  Routed experts the resident kernel takes beside a shared expert of another width get it in a launch of their
-  // own once its gain outweighs the shared expert's launch, whose few items are then alone on the chip (layer, us, one
-  // launch / two, same bits: 4096 x 256, shared 512, top 6: 40 tokens 98 / 93, 2048 tokens 369 / 296; 2048 x 128, shared
-  // 512, top 8: 150 tokens 72 / 74, 300 tokens 87 / 85, 2048 tokens 176 / 143; 2048 x 512, shared 1024, top 8: 300 tokens
-  // 102 / 111, 777 tokens 155 / 155, 2048 tokens 274 / 262; routed 1024 or 2048 beside a resident shared expert: one
-  // launch always, 375 / 385; 4-bit experts alike, 4096 x 256, 2048 tokens 362 / 297).
+  // own once its gain, which grows with the results it writes, outweighs the shared expert's launch, whose few items are then
+  // alone on the chip: from 6 M results on, and of rows of 512, where the ring is nearly as good, from 24 M (2-bit layer, us, one launch /
+  // two, same bits: 4096 x 256, shared 512, top 6: 100 tokens 93.5 / 93.0, 300 127.6 / 121.5, 2048 361 / 298; 2048 x 128, shared 512, top 8: 150
+  // tokens 63.3 / 65.9, 400 79.3 / 79.4, 1000 111 / 103; 1024 x 128, shared 384, top 4: 1000 tokens 66.9 / 74.7, 2000 82.6 / 82.2, 4000 113 / 108;
+  // 2048 x 256, shared 768, top 4: 600 tokens 86.5 / 89.0, 1000 105 / 106, 1500 123 / 114; 6144 x 256, shared 1536, top 2: 400 tokens 135 / 137,
+  // 600 157 / 151.  Rows of 512: 2048, shared 1024, top 8: 300 tokens 93.5 / 103.3, 1024 162.1 / 162.3, 2048 263 / 261; shared 192, 1000 153 / 157,
+  // 1500 194 / 186; 4096, shared 1024, top 4: 600 tokens 160 / 167, 2048 300 / 299, 3000 400 / 384.  4-bit experts alike: 2048 x 512, shared 1024,
+  // 300 tokens 94 / 111; 1024 x 128, 1000 tokens 66 / 74.  Routed 1024 or 2048 beside a resident shared expert: one launch always, 375 / 385).
   const bool kres_both = kres_q && (!c.shared_f || (kres_d && d2.kdim == q2.kdim));
-  const bool apart = c.shared_f && kres_q && !kres_both && pairs >= (c.shared_f <= 512 ? 1024u : 8192u);
+  const bool apart = c.shared_f && kres_q && !kres_both && pairs * c.d >= (c.f <= 256 ? 6u : 24u) << 20;
   const PrefillTiles tile = prefill_tiles(c, t, c.shared_f && !apart ? kres_both : kres_q);
   TileLists lists{{ws.tiles[0], tile.down != tile.up ? ws.tiles[1] : nullptr},
                   {prefill_tile_slots(c, t, tile.up), prefill_tile_slots(c, t, tile.down)}, {tile.up, tile.down}};

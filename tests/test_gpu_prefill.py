@@ -704,7 +704,7 @@ def test_prefill_from_the_tiled_pool_gives_the_same_bits(gpu, oracle, bits, d, f
 @pytest.mark.parametrize("d,f,fs,t", [(640, 512, 0, 40), (256, 512, 1024, 33), (256, 512, 1024, 600)])
 def test_prefill_rows_of_512_beside_what_the_resident_kernel_refuses(gpu, oracle, d, f, fs, t):
     """the down projections' tiles are chosen for the kernel that runs: not the resident one at d = 640 or in one launch with a
-    wider shared expert (few routes); two launches, one of them resident, from 8192 routes on are the last case's neighbours"""
+    wider shared expert (few routes); two launches, one of them resident, have a test of their own below"""
     layer = oracle.synth_layer(ROOT_SEED + 0xB500 + d + t, d, f, 16, 8, bits=4, fs=fs)
     moe, wts = make_moe(gpu, layer), to_device_layer(layer)
     x = oracle.synth_x(ROOT_SEED + t, t, d)
@@ -751,3 +751,23 @@ def test_prefill_of_few_work_items(gpu, oracle, bits, d, f, e, k, fs, t, tiled):
     ref, ref_idx, _ = oracle.moe_layer(layer, x)
     assert np.array_equal(idx, ref_idx)
     assert_layer_close(oracle.bf16_to_float(y), oracle.bf16_to_float(ref), f"bits={bits} d={d} f={f}")
+
+
+@pytest.mark.parametrize("bits,d,f,fs,t", [(4, 1024, 128, 384, 1536), (2, 512, 256, 192, 3072), (4, 768, 512, 192, 8192)])
+def test_prefill_with_the_shared_expert_in_a_launch_of_its_own(gpu, oracle, bits, d, f, fs, t):
+    """Routed rows that the resident kernel takes beside a shared expert of another width: one launch up to a line in the results written
+    (6 M, and 24 M for rows of 512), two from there on.  The longest prompt below the line, the one at it, and a row more have the same bits."""
+    e, k = 8, 4
+    layer = oracle.synth_layer(ROOT_SEED + 0xA9A7 + d + f, d, f, e, k, bits=bits, fs=fs, router_mode=0)
+    moe, wts = make_moe(gpu, layer), to_device_layer(layer)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(d + f)
+    x = torch.randn((t + 1, d), generator=gen, device="cuda").to(torch.bfloat16)
+    out = []
+    for n in (t - 1, t, t + 1):
+        y = torch.zeros((n, d), dtype=torch.bfloat16, device="cuda")
+        moe.encode_prefill_layer(wts, x[:n].contiguous(), y, n)
+        out.append(y.view(torch.int16))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1][:t - 1]) and torch.equal(out[1], out[2][:t])
+    assert_layer_close(oracle.bf16_to_float(ops.bf16_bits(y[:2])), oracle.bf16_to_float(oracle.moe_layer(layer, ops.bf16_bits(x[:2]))[0]), f"d={d} f={f} t={t}")
