@@ -323,8 +323,9 @@ hipError_t launch_router_logits_int8(hipStream_t s, const uint8_t* codes, const 
   }
   // A wave to a workgroup while that is at most four a CU: its loads have a CU's paths to themselves.  Few waves: nothing branches between
   // a row's loads; beyond, nothing past the row is asked for.  us with the selection, without / with branches: aligned, 128 rows of 2816, 15
-  // tokens 6.83 / 7.04; of 5120, 16, 64, 300 tokens 7.8 / 7.95, 14.4 / 13.6, 46.1 / 40.8; unaligned (two chunks a trip), 64 rows of 1088, 15, 32,
-  // 300 tokens 6.01 / 6.02, 6.48 / 6.28, 18.7 / 14.4.
+  // tokens 6.83 / 7.04; of 5120, 16, 64, 300 tokens 7.8 / 7.95, 14.4 / 13.6, 46.1 / 40.8; unaligned, 64 rows of 1088, 15, 32, 300 tokens
+  // 6.01 / 6.02, 6.48 / 6.28, 18.7 / 14.4.  Unaligned rows take two chunks a trip up to 2048 elements and six beyond (128 rows of 2816, 1, 64
+  // tokens, two / six: 6.65 / 6.2, 14.3 / 13.4).
   const uint32_t cus = device_cu_count(), block = waves <= 4 * cus ? 64u : 256u;
   const bool few = waves <= (al ? 8 : 4) * cus;
   const dim3 grid((waves + block / 64 - 1) / (block / 64));
@@ -333,7 +334,8 @@ hipError_t launch_router_logits_int8(hipStream_t s, const uint8_t* codes, const 
     if (few) router_logits_int8_kernel<CPL, AL, true><<<grid, dim3(block), 0, s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits); \
     else router_logits_int8_kernel<CPL, AL, false><<<grid, dim3(block), 0, s>>>(codes, scales, biases, x, eff, e, d, t, x_stride, logits);    \
   } while (0)
-  if (!al) MF_R8(2, false);
+  if (!al && cpl <= 4) MF_R8(2, false);
+  else if (!al) MF_R8(6, false);
   else if (cpl <= 2) MF_R8(2, true);
   else if (cpl <= 4) MF_R8(4, true);
   else MF_R8(6, true);

@@ -266,7 +266,7 @@ def test_inkling_ties(gpu, oracle):
                                            (128, 2816, 8, 2, 1), (256, 1024, 4, 150, 0), (128, 2816, 8, 40, 0),
                                            (66, 4096, 8, 33, 0), (24, 256, 8, 20, 0), (128, 2816, 8, 20, 1),
                                            # on both sides of the few waves: unaligned rows of part of a trip and of two, aligned rows of two
-                                           (32, 576, 8, 32, 1), (32, 576, 8, 33, 1), (32, 1088, 8, 33, 1), (64, 5184, 8, 32, 0), (64, 5184, 8, 33, 0)])
+                                           (32, 576, 8, 32, 1), (32, 576, 8, 33, 1), (32, 1088, 8, 33, 1), (64, 5184, 8, 32, 0), (64, 5184, 8, 33, 0), (64, 5184, 8, 33, 1)])
 def test_gemma4_router_bit_exact(gpu, oracle, e, d, k, t, shift):
     """8-bit affine router rows; shift = 1 hands over pointers that are only 1- / 2-byte aligned"""
     rng = oracle.Rng.key(ROOT_SEED + 0xFA32, f"gemma4-{e}-{d}-{k}-{t}")
