@@ -15,9 +15,19 @@ namespace mf {
 // order with fmaf into one fp32 accumulator; lanes are combined by an xor
 // butterfly with strides 1..32 (neighbours first).  Replaces router_gemv_bf16_r4
 // (moe.metal:162-185) / maple_router_bf16_gemv (maple_moe.metal:25-60).
+__device__ __forceinline__ float fma_chunk_bf16(const uint4& w, const uint4& x, float acc) {
+  const uint32_t ws[4] = {w.x, w.y, w.z, w.w}, xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    acc = __builtin_fmaf(bf16_lo(ws[j]), bf16_lo(xs[j]), acc);
+    acc = __builtin_fmaf(bf16_hi(ws[j]), bf16_hi(xs[j]), acc);
+  }
+  return acc;
+}
+// (w and x on 16-byte boundaries)
 __device__ __forceinline__ float dot_bf16_row(const uint16_t* __restrict__ w,
                                               const uint16_t* __restrict__ x, uint32_t d,
-                                              uint32_t lane, bool aligned) {
+                                              uint32_t lane) {
   float acc = 0.0f;
   const uint32_t chunks = d / 8;
   // four steps' loads are requested before the first product is taken: a lane's chunks are one
@@ -28,28 +38,13 @@ __device__ __forceinline__ float dot_bf16_row(const uint16_t* __restrict__ w,
     for (int s = 0; s < 4; ++s) {
       const uint32_t c = c0 + s * kWave;
       if (c < chunks) {
-        if (aligned) {
-          wv[s] = load_x8<true>(w + c * 8);
-          xv[s] = load_x8<true>(x + c * 8);
-        } else {
-          wv[s] = load_x8<false>(w + c * 8);
-          xv[s] = load_x8<false>(x + c * 8);
-        }
+        wv[s] = load_x8<true>(w + c * 8);
+        xv[s] = load_x8<true>(x + c * 8);
       }
     }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (c0 + s * kWave < chunks) {
-        acc = __builtin_fmaf(bf16_lo(wv[s].x), bf16_lo(xv[s].x), acc);
-        acc = __builtin_fmaf(bf16_hi(wv[s].x), bf16_hi(xv[s].x), acc);
-        acc = __builtin_fmaf(bf16_lo(wv[s].y), bf16_lo(xv[s].y), acc);
-        acc = __builtin_fmaf(bf16_hi(wv[s].y), bf16_hi(xv[s].y), acc);
-        acc = __builtin_fmaf(bf16_lo(wv[s].z), bf16_lo(xv[s].z), acc);
-        acc = __builtin_fmaf(bf16_hi(wv[s].z), bf16_hi(xv[s].z), acc);
-        acc = __builtin_fmaf(bf16_lo(wv[s].w), bf16_lo(xv[s].w), acc);
-        acc = __builtin_fmaf(bf16_hi(wv[s].w), bf16_hi(xv[s].w), acc);
-      }
-    }
+    for (int s = 0; s < 4; ++s)
+      if (c0 + s * kWave < chunks) acc = fma_chunk_bf16(wv[s], xv[s], acc);
   }
   return wave_sum(acc);
 }

@@ -515,21 +515,11 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
 #pragma unroll
           for (int sidx = 0; sidx < 4; ++sidx) {
             const uint32_t c = lane + sidx * kWave;
-            if (c < D / 8) {
-              const uint4 xv = load_x8<true>(xr + c * 8), wq = pre_w[sidx];
-              acc = __builtin_fmaf(bf16_lo(wq.x), bf16_lo(xv.x), acc);
-              acc = __builtin_fmaf(bf16_hi(wq.x), bf16_hi(xv.x), acc);
-              acc = __builtin_fmaf(bf16_lo(wq.y), bf16_lo(xv.y), acc);
-              acc = __builtin_fmaf(bf16_hi(wq.y), bf16_hi(xv.y), acc);
-              acc = __builtin_fmaf(bf16_lo(wq.z), bf16_lo(xv.z), acc);
-              acc = __builtin_fmaf(bf16_hi(wq.z), bf16_hi(xv.z), acc);
-              acc = __builtin_fmaf(bf16_lo(wq.w), bf16_lo(xv.w), acc);
-              acc = __builtin_fmaf(bf16_hi(wq.w), bf16_hi(xv.w), acc);
-            }
+            if (c < D / 8) acc = fma_chunk_bf16(pre_w[sidx], load_x8<true>(xr + c * 8), acc);
           }
           v = wave_sum(acc);
         } else {
-          v = dot_bf16_row(a.router_w + static_cast<size_t>(e) * D, xin + static_cast<size_t>(tok) * D, D, lane, true);
+          v = dot_bf16_row(a.router_w + static_cast<size_t>(e) * D, xin + static_cast<size_t>(tok) * D, D, lane);
         }
         if (lane == 0) s_stage64[wv] = (static_cast<unsigned long long>(epoch_now()) << 32) | __float_as_uint(v);
       }
@@ -547,7 +537,7 @@ __global__ __launch_bounds__(kFusedThreads) void fused_decode_kernel(const Fused
       if (item < n_gate) {
         const uint32_t tok = item;
         const float v = a.gq_w ? dot_q8_row(a.gq_w, a.gq_s, a.gq_b, xin + static_cast<size_t>(tok) * D, D, lane, true)
-                               : dot_bf16_row(a.w_sg, xin + static_cast<size_t>(tok) * D, D, lane, true);
+                               : dot_bf16_row(a.w_sg, xin + static_cast<size_t>(tok) * D, D, lane);
         if (lane < 4)  // the gate rides behind the token's shared activations
           store_u32_agent(&a.t_sact[static_cast<size_t>(tok) * sact_stride + Fs + lane],
                           (lane == 0 ? static_cast<uint32_t>(f_to_bf16(v)) : 0u) | (epoch_now() << 16));

@@ -41,12 +41,7 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint16_t* w, c
 #pragma unroll
     for (int i = 0; i < CPL; ++i) {
       if (c0 + i * kWave >= chunks) break;
-      const uint32_t ws[4] = {wv[i].x, wv[i].y, wv[i].z, wv[i].w}, xs[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc = __builtin_fmaf(bf16_lo(ws[j]), bf16_lo(xs[j]), acc);
-        acc = __builtin_fmaf(bf16_hi(ws[j]), bf16_hi(xs[j]), acc);
-      }
+      acc = fma_chunk_bf16(wv[i], xv[i], acc);
     }
   }
   const float v = wave_sum(acc);
