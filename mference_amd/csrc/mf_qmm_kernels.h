@@ -728,7 +728,7 @@ __device__ __forceinline__ void qmm_kres_item(const QmmArgs& a, const QmmPlace& 
   }
   qmm_trace(a, work, 1);
 
-  // ---- x tile into LDS (the layout qmm_kernel's ring uses for one group, NG times)
+  // ---- x tile into LDS: [group][block of 32 routes][s][h][32 routes, turned by kres_turn] x 16 B, run c = s + 4 h of a group
   {
     // (the 16 lanes that store together hold four runs of 8 of four routes each, or eight of two: the column is rotated so
     // that they hit different bank groups)

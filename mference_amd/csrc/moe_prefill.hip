@@ -710,7 +710,10 @@ __host__ __device__ __forceinline__ size_t group_one_lds_bytes(uint32_t t, uint3
 
 // Workgroups behind the first prepare x, a row per wave (the layer call with a router of its own has that done beside the router): one
 // workgroup groups for 8 to 12 us while the chip is idle otherwise.  Given routing, us: 777 tokens of 4096 with the scalar gate, grouping
-// 11.5 and a launch of 9.0 behind it -> 11.8; 300 tokens of 2816, 8.1 and 4.8 -> 8.3.
+// 11.5 and a launch of 9.0 behind it -> 11.8; 300 tokens of 2816, 8.1 and 4.8 -> 8.3.  They carry the first one's threads and LDS, one or
+// two to a CU, and gain where they are most, too.  The layer call, experts of 128, top 1, us, behind / beside: 16 experts of 2048, 8192 tokens
+// 90.8 / 79.9; 64 experts of 2048, 512 tokens 38.0 / 34.7, 8192 90.0 / 79.4; of 4096, 8192 tokens 162.1 / 157.6 (shared expert of 128:
+// 234.8 / 226.7); top 2, 128 experts of 5120, 4096 tokens 170.6 / 162.6.
 __global__ __launch_bounds__(1024) void group_one_kernel(const uint32_t* __restrict__ idx,
                                                          const float* __restrict__ w, uint32_t n_pairs,
                                                          uint32_t K, uint32_t E, uint32_t tpe_log2,
@@ -1350,14 +1353,18 @@ size_t up256(size_t v) { return (v + 255) / 256 * 256; }
 // ---- dense projections over many rows: MPPPrefillInt4QMM.encode (MPPPrefillInt4QMM.swift:34-78) and the
 // block form of the shared expert / dense MLP (PrefillSharedExpert.encodeBlock, PrefillSharedExpert.swift:81-172)
 //
-// y[m, n] = x[m, k] . W[n, k]^T through qmm_kernel in dense mode.  The kernel keeps the scales of a
-// workgroup's rows for the whole contraction in LDS, so a long K is cut into windows of at most
-// kDenseWindow groups (multiples of 8 groups, the last takes the rest): every window is a launch that
-// writes fp32 [m, n], and dense_combine_kernel adds the windows in order and narrows the sum.
-// A gate / up pair whose K does not fit one launch's tables (kDenseFusedMax groups) goes the same way:
-// both projections as fp32 per window, then dense_swiglu_combine_kernel.
-constexpr uint32_t kDenseWindow = 64;   // K groups per launch (4096 values)
-constexpr uint32_t kDenseFusedMax = 112;  // K groups a gate/up + SwiGLU launch can hold (both projections' scales in LDS)
+// y[m, n] = x[m, k] . W[n, k]^T through qmm_kernel in dense mode.  A long K is cut into windows (multiples of 8 groups, the last
+// takes the rest), which one launch computes side by side: each writes fp32 [m, n], and dense_combine_kernel adds the windows in
+// order and narrows the sum.  A window is at most kDenseWindow groups, because a result's sum is one fp32 accumulator over its groups:
+// error of the fp32 results against 64 bits, 512 x 17408, N(0, 1) and quantized N(0, 0.02): one window 3.9e-7, two 3.2e-7, five 2.6e-7;
+// 512 x 8192: 3.1e-7, two 2.6e-7.  That bound has a price where the work items fill the chip without it (us, chosen / fewer windows:
+// 5120 x 17408, 512 rows 134 / 122 (6, 3 windows); 17408 x 5120, 800 rows 200 / 173 (2, 1); 4096 x 12800, 1024 rows 156 / 138 (4, 2)).
+// A gate / up pair is one launch up to kDenseFusedMax groups.  Beyond, both projections go in windows as fp32, which
+// dense_swiglu_combine_kernel adds: again the shorter sums, and faster until a launch has a full round of work items.  The MLP, us,
+// one launch / two windows: 7296 x 2048, 9 rows 77.3 / 54.3, 150 98.0 / 71.7, 1024 145 / 140, 2048 229 / 252; 8192 x 8192, 64 rows
+// 107 / 83, 150 128 / 124, 1024 443 / 477; 12288 x 4096, 32 rows 111 / 76, 512 196 / 195, 2048 661 / 701.
+constexpr uint32_t kDenseWindow = 64;   // K groups of a window (4096 values)
+constexpr uint32_t kDenseFusedMax = 112;  // K groups of a gate/up + SwiGLU launch (7168 values)
 __global__ __launch_bounds__(256) void dense_combine_kernel(const float* __restrict__ parts, uint32_t n_parts,
                                                             size_t part_stride, void* __restrict__ y, size_t count,
                                                             int out_f32) {
@@ -1369,14 +1376,14 @@ __global__ __launch_bounds__(256) void dense_combine_kernel(const float* __restr
   else static_cast<uint16_t*>(y)[i] = f_to_bf16(acc);
 }
 
-// Windows of a contraction of length k for m rows of n results.  At least as many as the scale tables ask for; more where
+// Windows of a contraction of length k for m rows of n results.  At least as many as kDenseWindow asks for; more where
 // the work items (64 rows of x, 128 or 256 weight rows, one window) would leave the chip idle or its last round nearly
 // empty.  A round is two items a CU, whose time follows the longest window: 4 us per 8 groups and 1.5; a last round of at
 // most one item a CU has the CU to itself, 3 us per 8 groups and 1 less.  The windows' sums cost their bytes, written and read at 8 TB/s,
-// and 2 us.  (Fitted to 13 shapes, n 1024 .. 5120, k 1024 .. 17408, 9 .. 2048 rows, every count of windows timed: 0.5 % from
-// the best on average, 10 % at worst; the fewest windows 35 % and 126 %.  us for the projection, fewest / chosen:
-// 5120 x 17408, 9 rows 38.2 / 28.2 (5, 9 windows), 150 rows 79.1 / 65.5 (7), 512 rows 164 / 149 (6); 1152 x 3200, 32 rows
-// 31.8 / 16.5 (1, 6); 2048 x 8192, 64 rows 54.1 / 26.1 (2, 16); 4096 x 14336, 32 rows 39.2 / 25.8 (4, 15).)
+// and 2 us.  (16 shapes, n 1024 .. 17408, k 1024 .. 17408, 9 .. 2048 rows, up to 26 windows timed: 0.6 % from the best of those allowed
+// on average, 9 % at worst (1024 x 17408, 64 rows: 34 windows 31.9, 17 29.3); the fewest windows 33 % and 113 %.  us for the projection, fewest /
+// chosen: 5120 x 17408, 9 rows 41.7 / 30.3 (5, 12 windows), 150 rows 71.4 / 60.6 (7), 512 rows 144 / 134 (6); 1152 x 3200, 32 rows
+// 28.6 / 15.4 (1, 6); 2048 x 8192, 64 rows 46.4 / 25.6 (2, 16); 4096 x 14336, 32 rows 40.8 / 27.7 (4, 14).)
 // The choice follows the number of 64-row tiles, not m: a row's sums come out the same in every block of that many tiles.
 // From kWholeRounds rounds of the fewest windows on an emptier last round is no longer worth the windows' bytes.
 constexpr uint32_t kWholeRounds = 8;
@@ -1614,8 +1621,8 @@ hipError_t launch_dense_mlp(hipStream_t s, const mf_qtensor& gate, const mf_qten
   // 77.3 / 74.5, 32 rows 79.5 / 77.8; 7168 x 2048, 9 rows 63.6 / 58.1; 4096 x 12800, 9 rows 53.3 / 50.7; at d of 2048 and less no gain.
   const uint32_t tile = t <= kSmallTile && d > 2048 && gu_win * ((f + kQmmRows - 1) / kQmmRows) <= 2 * device_cu_count() ? kSmallTile : kTileTokens;
   if (gu_win > 1) {
-    // few rows (or a K too long for one launch's scale tables): the contraction in windows, both projections as
-    // fp32 per window, then one pass that adds the windows, activates and sums the groups
+    // past kDenseFusedMax: the contraction in windows, both projections as fp32 per window, then one pass that adds the
+    // windows, activates and sums the groups
     const uint32_t ng = d / kGroup;
     const size_t part_stride = up256(sizeof(float) * static_cast<size_t>(t) * f) / sizeof(float);
     float* pg = reinterpret_cast<float*>(base);

@@ -167,7 +167,7 @@ def _close_or_one_step(oracle, got_bits, ref_bits, what):
     assert rel_l2 <= 1e-3 and max_abs <= max(2e-2, step + 1e-9), (what, rel_l2, max_abs, step)
 
 
-# (d = 7680: 120 K groups, more than one gate/up launch holds tables for -- the contraction goes in two windows
+# (d = 7680: 120 K groups, more than a gate/up launch takes -- the contraction goes in two windows
 # that meet in the SwiGLU combine pass)
 @pytest.mark.parametrize("d,f,t", [(2048, 512, 40), (1024, 1536, 128), (5120, 1536, 33), (7680, 256, 70)])
 def test_shared_expert_block_form(gpu, oracle, d, f, t):
