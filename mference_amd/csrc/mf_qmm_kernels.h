@@ -60,8 +60,9 @@ __device__ __forceinline__ uint32_t qmm_work(const QmmArgs& a, const QmmPlace& a
 // for in front of its loop is time the SIMD is not full, and the loop takes everything along: x goes straight to LDS, a pair of
 // groups ahead, and scales, biases and group sums come a step of 16 groups ahead (before, all of them in front of the loop, in
 // sequence for tiles of 32).  Stage stamps of a routed gate / up item, us, before -> now: Qwen shape, 2048 tokens, in front of the
-// loop 6.1 -> 3.5, whole item 33.1 -> 29.8, launch 136 -> 126 under the tracer; two 5120 x 17408 MLPs, 150 rows 303 -> 277; tiles of
-// 32: 2816 x 704, 300 tokens 64 -> 60, large 2-bit layer, 777 tokens 362 -> 345 (there the instructions of the loop are the bound).
+// loop 6.1 -> 3.5, whole item 33.1 -> 29.8.  Launches of both forms traced on one card, us: that one 127.5 -> 115; a 5120 x 17408 MLP of 150
+// rows, gate / up 98.9 -> 89.6, down in windows 59.6 -> 54.5; tiles of 32, where the instructions of the loop are the bound: large 2-bit layer,
+// 777 tokens, gate / up 354 -> 345, down 179 -> 181; 2816 x 704, 300 tokens, gate / up 67.2 -> 68.3, down (11 groups) 50.9 -> 44.5.
 // LDS no longer grows with K, so every contraction keeps its two or three workgroups a CU.
 // FEW (tiles of 32): a launch that leaves a CU at most two workgroups is bound by what each waits for, codes from HBM above all.  It has
 // the registers of two waves and their LDS: codes run four pairs of groups ahead, x three, and units are not kept apart.  The layer call,
