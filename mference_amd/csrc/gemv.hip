@@ -742,12 +742,30 @@ __global__ __launch_bounds__(kQuadMaxWaves * 64) void rows_quad_kernel(RowsQuadA
   }
   // Ordinary lanes: 2^64 is 64 more in every exponent field, which neither overflows nor carries (a zero becomes 2^-63, whose products
   // with codes of at most 2^-125 are zero in fp32 as its own are; so is the product of a number below 2^-126, whose field is zero).
-  if (__builtin_expect(__all(x_scale == kRowScale), 1)) {
+  // Six chunks a lane (IN_PLACE): the operands of two branches stand in registers beside x, 16 for each chunk, and with six of them 34
+  // values went through scratch memory.  There other lanes' numbers take x's place with 2^64 taken off, and one form makes the operands.
+  // 4-bit launches, us, two branches / this: gate / up 6144 x 2688, five rows 18.4 / 14.8, 6144 x 3072, four rows 15.2 / 12.7, one
+  // projection 1536 x 11136, three rows 15.6 / 10.2.  (At fewer chunks two branches are faster, the MLP of one row: 4-bit 3968 x 6272
+  // 18.2 / 19.6, 2-bit 3840 x 6592 18.6 / 20.3.)
+  constexpr bool IN_PLACE = ITS == 6;
+  constexpr uint32_t kMore = 0x20002000u;
+  const bool ordinary = __all(x_scale == kRowScale);
+  if (IN_PLACE && __builtin_expect(!ordinary, 0)) {
 #pragma unroll
     for (int j = 0; j < ITS; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        constexpr uint32_t kMore = 0x20002000u;
+        float part;
+        const uint4 o = matmul_row8(raw[j][i], x_scale, &part);  // (0, 4), (1, 5), (2, 6), (3, 7)
+        raw[j][i] = make_uint4(__builtin_amdgcn_perm(o.y, o.x, 0x05040100u) - kMore, __builtin_amdgcn_perm(o.w, o.z, 0x05040100u) - kMore,
+                               __builtin_amdgcn_perm(o.y, o.x, 0x07060302u) - kMore, __builtin_amdgcn_perm(o.w, o.z, 0x07060302u) - kMore);
+      }
+  }
+  if (IN_PLACE || __builtin_expect(ordinary, 1)) {
+#pragma unroll
+    for (int j = 0; j < ITS; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
         const uint32_t v[4] = {raw[j][i].x + kMore, raw[j][i].y + kMore, raw[j][i].z + kMore, raw[j][i].w + kMore};
         // (0, 4), (1, 5), (2, 6), (3, 7)
         xa[j][2 * i] = make_uint2(__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u));

@@ -286,3 +286,17 @@ __global__ void probe(const float* x, float* y) {
         ok, past = compiles(n, n), compiles(n, n + 1)
         assert ok.returncode == 0, ok.stderr
         assert past.returncode != 0 and "index past the end of a register array" in past.stderr
+
+
+def test_the_quad_row_kernels_keep_to_their_registers():
+    """rows_quad_kernel (gemv.hip) holds a row set's x in registers: no instance goes through scratch memory"""
+    import re, subprocess
+    from mference_amd import build
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    if not os.path.exists(hipcc):
+        pytest.skip("needs hipcc")
+    cmd = [hipcc, *build.FLAGS, "--offload-device-only", "-Rpass-analysis=kernel-resource-usage", "-c", "-o", os.devnull, os.path.join(build.CSRC, "gemv.hip")]
+    done = subprocess.run(cmd, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+    scratch = re.findall(r"Function Name: (\S*rows_quad_kernel\S*).*?ScratchSize \[bytes/lane\]: (\d+)", done.stderr, re.S)
+    assert len(scratch) == 32 and all(size == "0" for _, size in scratch), scratch

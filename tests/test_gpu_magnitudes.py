@@ -181,6 +181,13 @@ def test_few_rows_far_from_one(gpu, bits, m, n, t):
     assert all(torch.equal(out[0], o) for o in out[1:]) and (out[0] != 0).all()
 
 
+@pytest.mark.parametrize("bits", [4, 2, 1])
+@pytest.mark.parametrize("m,n,t", [(4096, 3072, 4), (4096, 2688, 7), (6144, 6144, 3), (4096, 11136, 5)])
+def test_few_rows_far_from_one_in_six_chunks_a_lane(gpu, bits, m, n, t):
+    """as above where a lane of the quad kernel takes six chunks of a row: their operands are made in the place of x"""
+    test_few_rows_far_from_one(gpu, bits, m, n, t)
+
+
 @pytest.mark.parametrize("bits", [4, 2])
 @pytest.mark.parametrize("m,n,t", [(4096, 4096, 4), (4096, 3136, 3), (5120, 17408, 7)])
 def test_few_rows_of_zeros_and_numbers_too_small_for_a_product(gpu, bits, m, n, t):
