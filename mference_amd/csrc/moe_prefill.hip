@@ -1662,8 +1662,8 @@ uint32_t prefill_tile_slots(const mf_moe_config& c, uint32_t t, uint32_t tile) {
 // expert 128 2-bit experts of 4096 x 256, shared 512, 158 / 134; 64 of 2048 x 768 92.5 / 89.5; 128 of 4096 x 1024 294 / 312 (274 / 263); 32 of
 // 5120 x 1536 199 / 224 (182 / 181).  At 64 of 2-bit codes 64 of 1536 x 128 71 / 63, 64 of 4096 x 2048 363 / 379 (348 / 349).
 // The resident kernel on 4-bit rows of 512 has half the codes in flight each in its three workgroups a CU: tiles of 32 from a route
-// an expert on and while their work items make up to five a CU.  Layer call, us, 64 / 32: 2048 x 512, 256 experts, top 8, shared 512, 16, 32, 64, 96, 192, 256,
-// 384, 768 tokens 54.2 / 55.2, 58.6 / 59.5, 71.2 / 69.3, 72.6 / 70.4, 81.6 / 77.5, 91.6 / 91.0, 96.7 / 99.9, 144.4 / 149.0; 1024 x 512, 128 experts, 64, 192, 384 tokens
+// an expert on and while their work items make up to 4.75 a CU.  Layer call, us, 64 / 32: 2048 x 512, 256 experts, top 8, shared 512, 16, 32, 64, 96, 192, 258, 280,
+// 384, 768 tokens 54.2 / 55.2, 58.6 / 59.5, 71.2 / 69.3, 72.6 / 70.4, 81.6 / 77.5, 92.9 / 95.1, 93.6 / 95.1, 96.7 / 99.9, 144.4 / 149.0; 1024 x 512, 128 experts, 64, 192, 384 tokens
 // 49.9 / 47.1, 55.7 / 53.6, 61.5 / 58.2; 4096 x 512, 64 experts, top 4, 96, 256, 384 tokens 72.4 / 69.5, 101.3 / 97.6, 120.0 / 120.8; 5120 x 512,
 // 128 experts, shared 512, 9, 32, 96, 256 tokens 93.2 / 93.4, 114.3 / 116.7, 157.6 / 163.7, 211.6 / 218.4.
 // resident: that kernel takes the down projections of the call.  Where it does not, the ring on tiles of 64 / 32, us a call: 2176 x 512,
@@ -1685,7 +1685,7 @@ static PrefillTiles prefill_tiles(const mf_moe_config& c, uint32_t t, bool resid
   PrefillTiles p;
   p.up = static_cast<uint64_t>(t) * c.top_k <= few ? kSmallTile : kTileTokens;
   const bool few_or_many = static_cast<uint64_t>(t) * c.top_k <= c.num_experts ||
-                           static_cast<uint64_t>(prefill_tile_slots(c, t, kSmallTile)) * c.d > 5ull * 512 * device_cu_count();  // (an item: 512 rows)
+                           static_cast<uint64_t>(prefill_tile_slots(c, t, kSmallTile)) * c.d > 19ull * 128 * device_cu_count();  // (4.75 items of 512 rows)
   p.down = resident && c.bits == MF_BITS_4 && c.f == 512 && few_or_many ? kTileTokens : p.up;
   return p;
 }
